@@ -132,7 +132,7 @@ int pkv_update_cache_cnt_legacy(const int32_t *sorted_ids, const int32_t *topk_c
  * chunk_suf uint16 [R][n_chunks][128] for each `chunk_keys`-key chunk
  * (n_chunks = ceil(n_keys / chunk_keys)) and row_suf uint32 [R][128], which is
  * ADDED to with atomics and must be zero on entry.
- * chunk_keys must be a multiple of 2048 and at most 32768. */
+ * chunk_keys must be a multiple of 256 and at most 32768. */
 int pkv_collision_scan(const uint8_t *codes, int64_t cs_b, int64_t cs_h, int64_t cs_key, int64_t cs_sub,
                        int bs, int n_kv_heads, int64_t n_keys, const uint8_t *lut,
                        uint8_t *cnt_u8, int32_t *cnt_i32, uint32_t *row_suf, uint16_t *chunk_suf,
@@ -626,7 +626,7 @@ int pkv_adaptive_decode_step(const pkv_retrieve_args *retrieve, void *ws, size_t
  * chunk_suffix_hist, row_suffix_hist, cand, scores, cand_record_word, handover_status.  Returns PKV_EINVAL for an
  * unknown name.  chunk_suffix_hist holds uint16 counts of the keys of a chunk with at least `bin` votes:
  * [row][chunk][128 bins] for rows scanned one chunk per workgroup, and [row][128 bins][chunk][4 pieces] where the
- * chunk size (the smallest power of two from 2048 that keeps a launch within 1024 workgroups) is 8192 keys or more and
+ * chunk size (a power of two from 256 on, larger where a launch would exceed 1024 workgroups) is 8192 keys or more and
  * a row has at most 128 chunks: a workgroup then scans four pieces of chunk_keys / 4 keys that lie n_chunks pieces
  * apart, and piece p of the row, in key order, is entry [p % n_chunks][p / n_chunks]. */
 int pkv_retrieve_ws_view(void *ws, int rows, int64_t n_keys, int64_t n_cand, int64_t k,

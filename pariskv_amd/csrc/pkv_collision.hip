@@ -93,8 +93,10 @@ __global__ __launch_bounds__(kScanThreads) void pkv_scan_keymajor_kernel(
     const int64_t k0 = piece * piece_keys < n_keys ? piece * piece_keys : n_keys;
     const int64_t k1 = (k0 + piece_keys < n_keys) ? k0 + piece_keys : n_keys;
     int64_t kc = k0;
-    if (out8 && !out32 && chunk_suf) {  // uniform: the retrieval's form; whole runs of 1024 keys first
+    if (out8 && !out32 && chunk_suf) {  // uniform: the retrieval's form; whole runs of 1024, then 512 and 256 keys first
       for (; kc + 4 * kScanThreads <= k1; kc += 4 * kScanThreads) scan_whole_keys<4>(base, kc, l8, out8, s_hist, copy);
+      if (kc + 2 * kScanThreads <= k1) scan_whole_keys<2>(base, kc, l8, out8, s_hist, copy), kc += 2 * kScanThreads;
+      if (kc + kScanThreads <= k1) scan_whole_keys<1>(base, kc, l8, out8, s_hist, copy), kc += kScanThreads;
     }
     for (int64_t i0 = kc + tid; i0 < k1; i0 += 4 * kScanThreads) {
       pkv_u32x4 v[4];
@@ -232,14 +234,14 @@ static int launch_scan_impl(const uint8_t *codes, int64_t cs_b, int64_t cs_h, in
                             int n_kv_heads, int64_t n_keys, const uint8_t *lut, uint8_t *cnt_u8,
                             int64_t cnt_u8_stride, int32_t *cnt_i32, uint32_t *row_suf, uint16_t *chunk_suf,
                             int chunk_keys, hipStream_t s, hipEvent_t ev_start, hipEvent_t ev_stop, int sub_blocks = 1) {
-  PKV_REQUIRE(chunk_keys >= 2048 && chunk_keys % 2048 == 0 && chunk_keys <= 32768,
-              "chunk_keys must be a multiple of 2048 in [2048,32768], got %d", chunk_keys);
+  PKV_REQUIRE(chunk_keys >= 256 && chunk_keys % 256 == 0 && chunk_keys <= 32768,
+              "chunk_keys must be a multiple of 256 in [256,32768], got %d", chunk_keys);
   const int64_t n_chunks = (n_keys + chunk_keys - 1) / chunk_keys;
   PKV_REQUIRE(n_chunks >= 1 && n_chunks <= 65535 * 16, "too many chunks (%lld)", (long long)n_chunks);
   PKV_REQUIRE(pkv_aligned(lut, 4), "lut must be 4-byte aligned");
   dim3 grid((unsigned)n_chunks, (unsigned)(bs * n_kv_heads));
   const bool keymajor = cs_sub == 1 && cs_key == 16 && pkv_aligned(codes, 16) && cs_b % 16 == 0 && cs_h % 16 == 0;
-  PKV_REQUIRE((sub_blocks == 1 || (sub_blocks == 4 && keymajor && chunk_suf)) && chunk_keys % (sub_blocks * 1024) == 0,
+  PKV_REQUIRE((sub_blocks == 1 || (sub_blocks == 4 && keymajor && chunk_suf)) && (sub_blocks == 1 || chunk_keys % (sub_blocks * 1024) == 0),
               "a chunk of %d keys cannot be scanned as %d strided pieces", chunk_keys, sub_blocks);
   if (keymajor) {
     // the ext launch ties the two events to this dispatch's own begin/end timestamps

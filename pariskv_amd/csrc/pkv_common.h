@@ -50,14 +50,22 @@ struct PkvTiers {
   int n;
 };
 
-// Keys per workgroup-chunk of the collision scan / candidate select, chosen so
-// that rows * n_chunks is about a thousand workgroups (4 per CU, the measured
-// optimum at 32 rows x 128K keys) while the per-row chunk histograms (uint16 [n_chunks][128]) stay small.  Always a
-// multiple of 2048 and at most 32768 (a chunk's histogram bins are uint16).
+// Keys per workgroup-chunk of the collision scan / candidate select.
+// Large rows: rows * n_chunks is about a thousand workgroups (4 per CU, the measured optimum at 32 rows x 128K keys)
+// while the per-row chunk histograms (uint16 [n_chunks][128]) stay small.
+// Small rows: chunks below 2048 keys, because there the launches are as long as their fullest workgroup (up to half of
+// the keys are candidates: 1024 per workgroup of 256 threads at 8 rows x 3.5K keys) and most of the chip is idle; at
+// most 32 chunks to a row, or 128 workgroups in all, since every chunk adds to the same 128 words of the row and reads
+// the histograms of the chunks before it.  us per decode step with chunks of 256 / 512 / 1024 / 2048 keys:
+//   8 rows x 3.5K 32.2 / 34.1 / - / 39.5,  8 x 7.6K 32.8 / 33.1 / - / 38.0,  8 x 16K 34.8 / 33.9 / - / 37.5,
+//   8 x 32K - / 37.2 / 36.5 / 38.0,  32 x 11K - / 35.8 / 37.0 / 37.9,  32 x 32K - / - / 40.0 / 40.8.
+// Always a power of two of 256 .. 32768 (a chunk's histogram bins are uint16).
 static inline int pkv_pick_chunk_keys(int rows, int64_t n_keys) {
-  int64_t chunk = 2048;
-  while (chunk < 16384 && (int64_t)rows * ((n_keys + chunk - 1) / chunk) > 1024) chunk *= 2;
-  while (chunk < 32768 && (n_keys + chunk - 1) / chunk > 512) chunk *= 2;
+  int64_t chunk = 256;
+  auto n_chunks = [&] { return (n_keys + chunk - 1) / chunk; };
+  while (chunk < 2048 && ((int64_t)rows * n_chunks() > 1024 || (n_chunks() > 32 && (int64_t)rows * n_chunks() > 128))) chunk *= 2;
+  while (chunk < 16384 && (int64_t)rows * n_chunks() > 1024) chunk *= 2;
+  while (chunk < 32768 && n_chunks() > 512) chunk *= 2;
   return (int)chunk;
 }
 #define PKV_MAX_KEYS_PER_ROW ((int64_t)1 << 24)  // 512 chunks of 32768 keys

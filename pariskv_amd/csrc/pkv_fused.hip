@@ -371,7 +371,7 @@ int pkv_launch_fused_retrieve(const void *q, int dtype, int bs, int n_kv_heads, 
                               uint32_t *range_slots, int64_t range_row_stride, hipStream_t s) {
   const int rows = bs * n_kv_heads;
   const int64_t n_chunks = (n_keys + chunk_keys - 1) / chunk_keys;
-  PKV_REQUIRE(chunk_keys >= 2048 && chunk_keys % 2048 == 0 && chunk_keys <= kFusedMaxChunkKeys && n_chunks <= 256,
+  PKV_REQUIRE(chunk_keys >= 256 && chunk_keys % 256 == 0 && chunk_keys <= kFusedMaxChunkKeys && n_chunks <= 256,
               "fused retrieval: chunk of %d keys, %lld chunks per row not supported", chunk_keys, (long long)n_chunks);
   PKV_REQUIRE(!extra_out || (extra_off >= 0 && extra_off % 4 == 0 && extra_off + 4 <= ns_key),
               "the extra word must lie inside the key's record (offset %lld, record %lld bytes)", (long long)extra_off,

@@ -724,6 +724,29 @@ def test_retrieve_fused_matches_oracle(ops, request, wl_name):
         assert np.array_equal(out[b, h].cpu().numpy(), whole)
 
 
+@pytest.mark.parametrize("H,N,C", [(2, 255, 254), (2, 257, 100), (8, 769, 385), (8, 8192, 4096), (8, 8193, 900), (8, 16385, 1639),
+                                   (1, 32769, 1500)])
+def test_retrieve_short_rows_chunk_edges(ops, H, N, C):
+    """Rows scanned in chunks of 256, 512 and 1024 keys, at and beside the sizes where the chunk size changes and with
+    ragged last chunks: vote counts, histograms, candidate list and final ids against the oracle."""
+    w = W.make_workload(f"short{N}", 1, H, 4, N, C, min(100, C), O.BF16, 0.3, seed0=N, with_values=False)
+    _say(f"retrieve short rows H={H} N={N} C={C}")
+    plan, out, scores = _run_fused(ops, w)
+    cnt = plan.view("cnt_u8", w.N, w.C, w.K, torch.uint8).view(w.R, (N + 15) // 16 * 16)[:, :N].cpu().numpy()
+    cand = plan.view("cand", w.N, w.C, w.K, torch.int64).view(w.R, w.C).cpu().numpy()
+    suf = plan.view("chunk_suffix_hist", w.N, w.C, w.K, torch.int16).view(w.R, -1, 128).cpu().numpy().astype(np.int64) & 0xFFFF
+    for r in range(w.R):
+        st = W.oracle_stages(w, r)
+        assert np.array_equal(cnt[r], st["cnt"].astype(np.uint8))
+        chunk = 256 << next(i for i in range(4) if -(-N // (256 << i)) == suf.shape[1])   # the chunk size that was taken
+        for c in range(suf.shape[1]):
+            hist = np.bincount(st["cnt"][c * chunk:(c + 1) * chunk], minlength=128)
+            assert np.array_equal(suf[r, c], np.cumsum(hist[::-1])[::-1])
+        assert np.array_equal(cand[r], st["cand"])
+        assert np.array_equal(out[0, r].cpu().numpy(), st["final"])
+        assert np.array_equal(scores[0, r].cpu().numpy(), st["final_scores"])
+
+
 @pytest.mark.parametrize("wl_name", ["wl_cfg1", "wl_cfg2", "wl_small_bf16"])
 def test_one_launch_plan_equals_three_launches(ops, request, wl_name):
     """pkv_retrieve_args.launch_plan = PKV_PLAN_ONE_LAUNCH (query prep, scan and select + rerank as one launch whose
