@@ -50,7 +50,7 @@ int pkv_version(void);
 const char *pkv_last_error(void);
 /* sizeof of the argument structs as this library was compiled, for a binding to
  * compare with its own mirror: 0 pkv_attn_segment, 1 pkv_attn_args,
- * 2 pkv_retrieve_args, 3 pkv_adaptive_args (0 for any other number).
+ * 2 pkv_retrieve_args, 3 pkv_adaptive_args, 5 pkv_prefill_args (0 for any other number).
  * No counterpart in the reference. */
 size_t pkv_struct_bytes(int which);
 
@@ -76,6 +76,52 @@ int pkv_encode_append(const void *keys, int dtype, int bs, int n_kv_heads, int64
                       uint16_t *weight, int64_t ws_b, int64_t ws_h, int64_t ws_key, int64_t ws_sub,
                       int32_t *cluster_counts, int64_t cc_b, int64_t cc_h,
                       void *stream);
+
+/* A prompt's K and V rows into the cache and the index of its retrieval zone in
+ * one launch: replaces the slice copies of prefill_update_kv_cache, the staging
+ * copies before the offload and batch_encode + _count_cluster_keys
+ * (cache_hub/polar_cache.py:430-504, :513-611), in the adaptive caches also the
+ * value norms (cache_hub/polar_cache_adaptivek_varlen.py:680-756).  Also used for
+ * the tokens that leave the local window at an index refresh (:743-799).
+ * Tokens [0, n_sink) and [n_sink + n_encode, + n_tail) of k / v go to rows
+ * 0 .. n_sink-1 and tail_row0 .. of dense_k / dense_v; the n_encode tokens
+ * between them go to rows 0 .. of zone_k / zone_v and are encoded as by
+ * pkv_encode_append (all outputs; cluster_counts +=).  Value norms (||v|| in
+ * dtype, widened; summation order of pkv_append_kv): dense_vnorm of the dense
+ * rows by destination row, zone_vnorm (any key stride) and zone_vnorm2
+ * (contiguous) of the encoded tokens; each may be NULL.  Where nib / weight are
+ * the two parts of 128-byte key records (weight = nib + 64 bytes, key stride 128
+ * bytes, aligned) and zone_vnorm is NULL or the records' word at byte 96, the
+ * records are written whole: bytes 100..127, and 96..99 without norms, become
+ * zero.  Source rows: 128
+ * contiguous elements, strides in elements (16-byte multiples); destination rows
+ * contiguous.  Strides in elements throughout. */
+typedef struct pkv_prefill_args {
+  const void *k, *v;
+  int dtype, bs, n_kv_heads;
+  int64_t k_stride_b, k_stride_h, k_stride_key, v_stride_b, v_stride_h, v_stride_key;
+  int64_t n_sink, n_encode, n_tail, tail_row0;
+  void *dense_k, *dense_v;
+  int64_t dense_stride_b, dense_stride_h;
+  void *zone_k, *zone_v;
+  int64_t zone_stride_b, zone_stride_h;
+  float *dense_vnorm;
+  int64_t dn_b, dn_h;
+  float *zone_vnorm;
+  int64_t zn_b, zn_h, zn_key;
+  float *zone_vnorm2;
+  int64_t zn2_b, zn2_h;
+  const float *signs;
+  uint8_t *codes;
+  int64_t cs_b, cs_h, cs_key, cs_sub;
+  uint8_t *nib;
+  int64_t ns_b, ns_h, ns_key, ns_sub;
+  uint16_t *weight;
+  int64_t ws_b, ws_h, ws_key, ws_sub;
+  int32_t *cluster_counts;
+  int64_t cc_b, cc_h;
+} pkv_prefill_args;
+int pkv_prefill_store(const pkv_prefill_args *args, void *stream);
 
 /* polar_cache._count_cluster_keys on its own (cache_hub/polar_cache.py:980-996):
  * cluster_counts[b][h][s][code] += 1 for every key and subspace. */

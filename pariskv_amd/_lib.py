@@ -78,6 +78,26 @@ class AdaptiveArgs(C.Structure):
     ]
 
 
+class PrefillArgs(C.Structure):
+    """Mirror of ``pkv_prefill_args``."""
+
+    _fields_ = [
+        ("k", _vp), ("v", _vp), ("dtype", _i), ("bs", _i), ("n_kv_heads", _i),
+        ("k_stride_b", _i64), ("k_stride_h", _i64), ("k_stride_key", _i64),
+        ("v_stride_b", _i64), ("v_stride_h", _i64), ("v_stride_key", _i64),
+        ("n_sink", _i64), ("n_encode", _i64), ("n_tail", _i64), ("tail_row0", _i64),
+        ("dense_k", _vp), ("dense_v", _vp), ("dense_stride_b", _i64), ("dense_stride_h", _i64),
+        ("zone_k", _vp), ("zone_v", _vp), ("zone_stride_b", _i64), ("zone_stride_h", _i64),
+        ("dense_vnorm", _vp), ("dn_b", _i64), ("dn_h", _i64),
+        ("zone_vnorm", _vp), ("zn_b", _i64), ("zn_h", _i64), ("zn_key", _i64),
+        ("zone_vnorm2", _vp), ("zn2_b", _i64), ("zn2_h", _i64),
+        ("signs", _vp), ("codes", _vp), ("cs_b", _i64), ("cs_h", _i64), ("cs_key", _i64), ("cs_sub", _i64),
+        ("nib", _vp), ("ns_b", _i64), ("ns_h", _i64), ("ns_key", _i64), ("ns_sub", _i64),
+        ("weight", _vp), ("ws_b", _i64), ("ws_h", _i64), ("ws_key", _i64), ("ws_sub", _i64),
+        ("cluster_counts", _vp), ("cc_b", _i64), ("cc_h", _i64),
+    ]
+
+
 # name -> (restype, argtypes); one entry per declaration in include/pariskv_hip.h
 PROTOTYPES = {
     "pkv_version": (_i, []),
@@ -88,6 +108,7 @@ PROTOTYPES = {
                                _vp, _i64, _i64, _i64, _i64,
                                _vp, _i64, _i64, _i64, _i64,
                                _vp, _i64, _i64, _vp]),
+    "pkv_prefill_store": (_i, [C.POINTER(PrefillArgs), _vp]),
     "pkv_count_cluster_keys": (_i, [_vp, _i64, _i64, _i64, _i64, _i, _i, _i64, _vp, _i64, _i64, _vp]),
     "pkv_query_prep_lut": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _i64, _i64, _vp, _i, _vp, _vp, _vp, _vp, _vp]),
     "pkv_update_cache_cnt": (_i, [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _i64,
@@ -168,7 +189,9 @@ def lib():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
-        for which, mirror in enumerate((AttnSegment, AttnArgs, RetrieveArgs, AdaptiveArgs)):
+        for which, mirror in ((0, AttnSegment), (1, AttnArgs), (2, RetrieveArgs), (3, AdaptiveArgs), (5, PrefillArgs)):
+            if os.environ.get("PARISKV_HIP_SO") and handle.pkv_struct_bytes(which) == 0:
+                continue
             if handle.pkv_struct_bytes(which) != C.sizeof(mirror):
                 raise RuntimeError(f"{SO_PATH} was built from another header: {mirror.__name__} is "
                                    f"{handle.pkv_struct_bytes(which)} bytes there, {C.sizeof(mirror)} here; rebuild it")

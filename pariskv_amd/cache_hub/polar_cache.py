@@ -234,24 +234,21 @@ class polar_cache(KV_Cache):
         self._offload_inflight[layer_idx] = True
         return self._copy_events[layer_idx]
 
-    def _stage_prefill_rows(self, k: torch.Tensor, v: torch.Tensor):
-        """Private contiguous copies of the [bsz,H,n,D] views k, v in one of the two staging pairs (the reference's
-        ``.contiguous()`` copies, polar_cache.py:457-458): the caller may rewrite its tensors as soon as this call
-        returns, and the copy engines get whole blocks.  Returns (slot, staged k, staged v)."""
+    def _prefill_stage_rows(self, shape):
+        """One of the two staging pairs, [bsz,H,n,D], for the prompt rows that leave for the host (the reference's
+        ``.contiguous()`` copies, polar_cache.py:457-458): the caller may rewrite its tensors as soon as the prefill
+        call returns, and the copy engines get whole blocks.  Returns (slot, staged k, staged v)."""
         slot = self._prefill_stage_next
         self._prefill_stage_next ^= 1
         if self._prefill_stage_event[slot] is not None:   # the copy that last read this pair must be over
             torch.cuda.current_stream(self.device).wait_event(self._prefill_stage_event[slot])
-        need = k.shape[0] * k.shape[1] * k.shape[2] * k.shape[3]
+        need = math.prod(shape)
         pair = self._prefill_stage[slot]
         if pair is None or pair[0].numel() < need:
             self._prefill_stage[slot] = None
             pair = (torch.empty(need, dtype=self.dtype, device=self.device), torch.empty(need, dtype=self.dtype, device=self.device))
             self._prefill_stage[slot] = pair
-        sk, sv = pair[0][:need].view(k.shape), pair[1][:need].view(v.shape)
-        sk.copy_(k)
-        sv.copy_(v)
-        return slot, sk, sv
+        return slot, pair[0][:need].view(shape), pair[1][:need].view(shape)
 
     def release_prefill_staging(self) -> None:
         """Free the prefill staging pairs (two layers' worth of retrieval-zone K/V in HBM) once prefill is over; they
@@ -261,16 +258,22 @@ class polar_cache(KV_Cache):
             self._prefill_stage = [None, None]
             self._prefill_stage_event = [None, None]
 
-    def _encode(self, layer_idx: int, keys_bhsd: torch.Tensor, b0: int, b1: int, abs0: int) -> None:
-        """Encode keys [b1-b0, H, n, D] (any strides) into metadata positions [abs0, abs0+n) and add to the cluster sizes."""
-        n = keys_bhsd.shape[2]
-        if n == 0:
-            return
-        sl = slice(abs0, abs0 + n)
+    def _store_rows(self, layer_idx, k, v, b0, b1, n_sink, n_encode, dense, tail_row0, zone, abs0) -> None:
+        """K/V rows [b1-b0, H, n, D] (any strides) into the cache, their middle n_encode tokens also encoded into metadata
+        positions [abs0, abs0 + n_encode) and added to the cluster sizes: one launch (``ops.prefill_store``)."""
+        if k.dtype != self.dtype or v.dtype != self.dtype:
+            k, v = k.to(self.dtype), v.to(self.dtype)
+        vec = 16 // k.element_size()
+        if any(t.stride(3) != 1 or t.data_ptr() % 16 or any(x % vec for x in t.stride()[:3]) for t in (k, v)):
+            k, v = k.contiguous(), v.contiguous()
+        index = zone_norms = None
+        if n_encode > 0:
+            sl = slice(abs0, abs0 + n_encode)
+            index = (self.codebook_gpu[layer_idx][b0:b1, :, :, sl], self.key_4bit_packed_gpu[layer_idx][b0:b1, :, :, sl],
+                     self.key_block_weight_gpu[layer_idx][b0:b1, :, :, sl], self.cluster_key_counts_gpu[layer_idx][b0:b1])
         ranges.push("batch_encode+cluster_count")  # the reference's prefill_step1_batch_encode / prefill_step3_cluster_count
-        ops.encode_append(keys_bhsd, self._srht_signs, self.codebook_gpu[layer_idx][b0:b1, :, :, sl],
-                          self.key_4bit_packed_gpu[layer_idx][b0:b1, :, :, sl], self.key_block_weight_gpu[layer_idx][b0:b1, :, :, sl],
-                          self.cluster_key_counts_gpu[layer_idx][b0:b1])
+        ops.prefill_store(k, v, n_sink, n_encode, self._srht_signs, dense, tail_row0, zone, index,
+                          **self._norm_targets(layer_idx, b0, b1, abs0, n_encode))
         ranges.pop()
 
     # ------------------------------------------------------------- prefill
@@ -298,32 +301,23 @@ class polar_cache(KV_Cache):
         v = value_states[:, vs:].permute(0, 2, 1, 3)
         kg, vg = self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx]
         last = (layer_idx == self.layer_num - 1) and (b1 == self.batch_size)
+        dense = kg[b0:b1], vg[b0:b1]
         if retrieval == 0:  # short prompt: everything stays dense on the GPU (:430-440)
             n = min(n_tok, self._gpu_rows[layer_idx])
-            kg[b0:b1, :, :n] = k[:, :, :n].to(self.dtype)
-            vg[b0:b1, :, :n] = v[:, :, :n].to(self.dtype)
-            self._on_prefill(layer_idx, b0, b1, v, 0, n)
+            self._store_rows(layer_idx, k[:, :, :n], v[:, :, :n], b0, b1, n, 0, dense, 0, None, 0)
             if last:
                 self.context += n
             return key_states[:, vs:], value_states[:, vs:]
         S0, r_end = self.sink_size, self.sink_size + retrieval
+        self.cluster_key_counts_gpu[layer_idx][b0:b1].zero_()  # prefill assigns, refresh accumulates (:493, :775)
         if self._layer_offload[layer_idx]:
-            kg[b0:b1, :, :S0] = k[:, :, :S0].to(self.dtype)
-            vg[b0:b1, :, :S0] = v[:, :, :S0].to(self.dtype)
-            kg[b0:b1, :, S0:S0 + local_len] = k[:, :, r_end:].to(self.dtype)
-            vg[b0:b1, :, S0:S0 + local_len] = v[:, :, r_end:].to(self.dtype)
             self._wait_offload(layer_idx)
-            slot, stage_k, stage_v = self._stage_prefill_rows(k[:, :, S0:r_end], v[:, :, S0:r_end])
+            slot, stage_k, stage_v = self._prefill_stage_rows((bsz, self.kv_head, retrieval, self.head_dim))
+            self._store_rows(layer_idx, k, v, b0, b1, S0, retrieval, dense, S0, (stage_k, stage_v), S0)
             self._prefill_stage_event[slot] = self._offload_rows(layer_idx, b0, b1, stage_k, stage_v, 0)
             self.cpu_valid_end[layer_idx] = retrieval
-            enc_src = stage_k
         else:
-            kg[b0:b1, :, :n_tok] = k.to(self.dtype)
-            vg[b0:b1, :, :n_tok] = v.to(self.dtype)
-            enc_src = kg[b0:b1, :, S0:r_end]
-        self.cluster_key_counts_gpu[layer_idx][b0:b1].zero_()  # prefill assigns, refresh accumulates (:493, :775)
-        self._encode(layer_idx, enc_src, b0, b1, S0)
-        self._on_prefill(layer_idx, b0, b1, v, retrieval, local_len)
+            self._store_rows(layer_idx, k, v, b0, b1, S0, retrieval, dense, r_end, (dense[0][:, :, S0:], dense[1][:, :, S0:]), S0)
         if last:
             self.context += n_tok
         return key_states[:, vs:], value_states[:, vs:]
@@ -362,14 +356,18 @@ class polar_cache(KV_Cache):
         kg, vg = self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx]
         n, S0 = r.n_new, self.sink_size
         bs = self.batch_size
-        self._encode(layer_idx, kg[:, :, r.gpu_row0:r.gpu_row0 + n], 0, bs, r.encode_abs0)
-        self._on_refresh(layer_idx, r)
-        if not self._layer_offload[layer_idx]:
+        if not self._layer_offload[layer_idx]:  # the rows stay where they are
+            sl = slice(r.encode_abs0, r.encode_abs0 + n)
+            with ranges.span("batch_encode+cluster_count"):
+                ops.encode_append(kg[:, :, r.gpu_row0:r.gpu_row0 + n], self._srht_signs, self.codebook_gpu[layer_idx][:, :, :, sl],
+                                  self.key_4bit_packed_gpu[layer_idx][:, :, :, sl], self.key_block_weight_gpu[layer_idx][:, :, :, sl],
+                                  self.cluster_key_counts_gpu[layer_idx])
+            self._on_refresh(layer_idx, r)
             return
         self._wait_offload(layer_idx)  # staging buffers are free again
         sk, sv = self._offload_keys_buffer[layer_idx][:, :, :n], self._offload_values_buffer[layer_idx][:, :, :n]
-        sk.copy_(kg[:, :, S0:S0 + n])
-        sv.copy_(vg[:, :, S0:S0 + n])
+        self._store_rows(layer_idx, kg[:, :, S0:S0 + n], vg[:, :, S0:S0 + n], 0, bs, 0, n, None, 0, (sk, sv), r.encode_abs0)
+        self._on_refresh(layer_idx, r)
         self._offload_rows(layer_idx, 0, bs, sk, sv, r.cpu_row0)
         self.cpu_valid_end[layer_idx] = r.cpu_row0 + n
         # slide the window: rows [sink+n, sink+local+n) -> [sink, sink+local)
@@ -382,8 +380,9 @@ class polar_cache(KV_Cache):
             vg[:, :, S0:S0 + L] = vg[:, :, S0 + n:S0 + n + L]
 
     # hooks for subclasses that keep more per-token state (value norms of the adaptive-k variant)
-    def _on_prefill(self, layer_idx, b0, b1, values_bhsd, retrieval, local_len):
-        pass
+    def _norm_targets(self, layer_idx, b0, b1, abs0, n_encode):
+        """Where the launch that stores rows leaves their value norms (keyword arguments of ``ops.prefill_store``)."""
+        return {}
 
     def _append(self, layer_idx, slot, key_states, value_states):
         ops.append_kv(key_states, value_states, self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx], slot)

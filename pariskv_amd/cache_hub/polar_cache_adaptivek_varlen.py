@@ -95,20 +95,11 @@ class polar_cache(_polar_cache_base):
         return 0.05, 0.2
 
     # ------------------------------------------------ value-norm bookkeeping
-    def _vnorm(self, values):
-        """||v||_2 per token as the reference computes it: in the tensor's dtype, then widened (:680, :756, :1179)."""
-        return torch.linalg.vector_norm(values.to(self.dtype), dim=-1).to(torch.float32)
-
-    def _on_prefill(self, layer_idx, b0, b1, values_bhsd, retrieval, local_len):
-        S0 = self.sink_size
-        sl = self._sl_vnorm_cache[layer_idx]
-        if retrieval == 0:  # short prompt: all tokens are dense GPU rows (:680)
-            sl[b0:b1, :, :local_len] = self._vnorm(values_bhsd[:, :, :local_len])
-            return
-        r_end = S0 + retrieval
-        sl[b0:b1, :, :S0] = self._vnorm(values_bhsd[:, :, :S0])                              # :704
-        sl[b0:b1, :, S0:S0 + local_len] = self._vnorm(values_bhsd[:, :, r_end:r_end + local_len])  # :706
-        self.value_norm_gpu[layer_idx][b0:b1, :, S0:r_end] = self._vnorm(values_bhsd[:, :, S0:r_end])  # :753-756
+    def _norm_targets(self, layer_idx, b0, b1, abs0, n_encode):
+        """||v||_2 per token in the cache's dtype, then widened (:680, :704-706, :753-756, :1075-1078), by the launch that
+        stores the rows: dense rows by GPU slot, the retrieval zone by absolute position."""
+        zone = self.value_norm_gpu[layer_idx][b0:b1, :, abs0:abs0 + n_encode] if n_encode > 0 else None
+        return dict(dense_vnorm=self._sl_vnorm_cache[layer_idx][b0:b1], zone_vnorm=zone)
 
     def _append(self, layer_idx, slot, key_states, value_states):
         """K/V rows and the value norm of the new token (:1179) in one launch."""
@@ -118,7 +109,6 @@ class polar_cache(_polar_cache_base):
     def _on_refresh(self, layer_idx, r):
         S0, n, L = self.sink_size, r.n_new, self.local_size
         sl = self._sl_vnorm_cache[layer_idx]
-        self.value_norm_gpu[layer_idx][:, :, r.encode_abs0:r.encode_abs0 + n] = sl[:, :, S0:S0 + n]  # :1075-1078
         sl[:, :, S0:S0 + L] = sl[:, :, S0 + n:S0 + n + L].clone()                                 # :1130-1133
 
     # ---------------------------------------------------------------- compute

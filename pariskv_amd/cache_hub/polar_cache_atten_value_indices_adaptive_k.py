@@ -50,15 +50,12 @@ class polar_cache(_adaptive_base):
         return cap, 1, cap
 
     # ------------------------------------------------ value-norm bookkeeping
-    def _on_prefill(self, layer_idx, b0, b1, values_bhsd, retrieval, local_len):
-        if self.enable_offload:
-            return super()._on_prefill(layer_idx, b0, b1, values_bhsd, retrieval, local_len)
-        # every token at its absolute position (:611-614); the retrieval zone's norms also by position (:634-637)
-        S0, n = self.sink_size, values_bhsd.shape[2]
-        vn = self._vnorm(values_bhsd)
-        self._sl_vnorm_cache[layer_idx][b0:b1, :, :n] = vn
-        if retrieval > 0:
-            self.value_norm_gpu[layer_idx][b0:b1, :, S0:S0 + retrieval] = vn[:, :, S0:S0 + retrieval]
+    def _norm_targets(self, layer_idx, b0, b1, abs0, n_encode):
+        targets = super()._norm_targets(layer_idx, b0, b1, abs0, n_encode)
+        if not self.enable_offload and n_encode > 0:
+            # every token at its absolute position (:611-614); the retrieval zone's norms also by position (:634-637)
+            targets["zone_vnorm2"] = self._sl_vnorm_cache[layer_idx][b0:b1, :, abs0:abs0 + n_encode]
+        return targets
 
     def _on_refresh(self, layer_idx, r):
         if self.enable_offload:

@@ -456,20 +456,130 @@ __device__ __forceinline__ bool enc_key_fast_f32(const float (&xr)[8], const flo
   return bad;
 }
 
+// ---- the rows of a prompt stored in the same launch as its keys are encoded ----------------------------------
+//
+// A STORE launch, grid (blocks, kv heads, batch): an encode workgroup first copies the value rows of its keys to their
+// place in the zone (taking their norms), then encodes the keys and writes each key row from the registers it is
+// encoded from (no second read of K); behind the encode workgroups of a head, dense workgroups copy K and V rows of 64
+// sink or local-window tokens each.  Bound by HBM: 1136 bytes per key in bf16, in 478 us for 4 x 8 heads x 65536 keys =
+// 5.0 TB/s, what a plain copy reaches (762 us as two copies and the encoder alone).  Value rows by workgroups of their
+// own between the encoding ones: 555 us with the records' tails left out, 485 us with whole records; heads instead of
+// blocks fastest over the grid 595 us; 128 / 512 keys per workgroup 479 / 504 us.
+enum EncStoreMode {
+  kEncNoStore = 0,
+  kEncStoreRows = 1,
+  kEncStoreRecords = 2,  // as kEncStoreRows; the 128-byte key records are written whole: the tail behind the weights
+                         // takes the value norm, or zeros (where 32 bytes of a line are left out, memory reads it back)
+};
+struct EncStore {
+  const char *v;                        // value rows of the encoded tokens; strides in bytes
+  int64_t v_b, v_h, v_key;
+  char *zk, *zv;                        // where the encoded tokens' rows go (rows contiguous)
+  int64_t z_b, z_h;
+  float *zn, *zn2;                      // value norms of the encoded tokens (either may be null; zn is null where they go into whole records)
+  int64_t zn_b, zn_h, zn_key, zn2_b, zn2_h;
+  int record_norm;                      // kEncStoreRecords: the record's word behind the weights takes the value norm
+  const char *dk_src, *dv_src;          // token 0 of the prompt
+  int64_t k_b, k_h, k_key;              // key strides in bytes (values: v_b, v_h, v_key)
+  char *dk, *dv;                        // dense rows: token t < n_sink to row t, token tail_src0 + i to row tail_row0 + i
+  int64_t d_b, d_h;
+  float *dn;                            // their value norms (may be null), rows contiguous
+  int64_t dn_b, dn_h;
+  int n_sink, n_tail;
+  int64_t tail_src0, tail_row0;
+  int n_blocks;                         // encode workgroups per head
+};
+constexpr int kEncDenseRows = 64;
+
+// n_rows rows of 128 elements from src (src_step bytes apart) to consecutive rows at dst, by one workgroup; norm /
+// norm2 / s_norm (may be null): the rows' 2-norms in the rows' type, summed in the order of the append kernel (squares of a
+// lane's 16 bytes left to right, then a pairwise tree over the row's lanes).
+template <bool BF16>
+__device__ __forceinline__ void enc_copy_rows(const char *src, int64_t src_step, char *dst, int n_rows, float *norm,
+                                              int64_t norm_step, float *norm2, float *s_norm = nullptr) {
+  constexpr int kVec = BF16 ? 16 : 32;             // 16-byte words per row
+  constexpr int kRowsPerStep = kEncThreads / kVec;
+  constexpr int kAhead = 8;                        // loads of a thread in flight
+  const int lane = threadIdx.x % kVec, r0 = threadIdx.x / kVec;
+  for (int base = 0; base < n_rows; base += kAhead * kRowsPerStep) {
+    pkv_u32x4 val[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int row = base + u * kRowsPerStep + r0;
+      val[u] = *(const pkv_u32x4 *)(src + (int64_t)(row < n_rows ? row : n_rows - 1) * src_step + 16 * lane);
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int row = base + u * kRowsPerStep + r0;
+      if (row < n_rows) __builtin_nontemporal_store(val[u], (pkv_u32x4 *)(dst + (int64_t)row * (16 * kVec) + 16 * lane));
+    }
+    if (norm || norm2 || s_norm) {  // uniform
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int row = base + u * kRowsPerStep + r0;
+        const uint32_t w[4] = {val[u].x, val[u].y, val[u].z, val[u].w};
+        float acc;
+        if (BF16) {
+          float e[8];
+#pragma unroll
+          for (int p = 0; p < 4; ++p) e[2 * p] = __uint_as_float(w[p] << 16), e[2 * p + 1] = __uint_as_float(w[p] & 0xffff0000u);
+          acc = e[0] * e[0];
+#pragma unroll
+          for (int j = 1; j < 8; ++j) acc = acc + e[j] * e[j];
+        } else {
+          acc = __uint_as_float(w[0]) * __uint_as_float(w[0]);
+#pragma unroll
+          for (int j = 1; j < 4; ++j) acc = acc + __uint_as_float(w[j]) * __uint_as_float(w[j]);
+        }
+        acc = acc + pkv_lane_xor_f<1>(acc);
+        acc = acc + pkv_lane_xor_f<2>(acc);
+        acc = acc + pkv_lane_xor_f<4>(acc);
+        acc = acc + pkv_lane_xor_f<8>(acc);
+        if (!BF16) acc = acc + pkv_lane_xor_f<16>(acc);
+        if (lane == 0 && row < n_rows) {
+          const float n = BF16 ? pkv_bf16_round(sqrtf(acc)) : sqrtf(acc);
+          if (norm) norm[(int64_t)row * norm_step] = n;
+          if (norm2) norm2[row] = n;
+          if (s_norm) s_norm[row] = n;
+        }
+      }
+    }
+  }
+}
+
+// A dense workgroup of a STORE launch: sink or local-window rows, no encoding.
+template <bool BF16>
+__device__ __forceinline__ void enc_store_dense(const EncStore &st, int b, int h, int blk) {
+  constexpr int row_bytes = BF16 ? 256 : 512;
+  const int sink_blocks = (st.n_sink + kEncDenseRows - 1) / kEncDenseRows;
+  const bool tail = blk >= sink_blocks;
+  const int i0 = (tail ? blk - sink_blocks : blk) * kEncDenseRows, all = tail ? st.n_tail : st.n_sink;
+  const int n = all - i0 < kEncDenseRows ? all - i0 : kEncDenseRows;
+  const int64_t src0 = (tail ? st.tail_src0 : 0) + i0, dst0 = (tail ? st.tail_row0 : 0) + i0;
+  const int64_t dst = b * st.d_b + h * st.d_h + dst0 * row_bytes;
+  enc_copy_rows<BF16>(st.dk_src + b * st.k_b + h * st.k_h + src0 * st.k_key, st.k_key, st.dk + dst, n, nullptr, 0, nullptr);
+  enc_copy_rows<BF16>(st.dv_src + b * st.v_b + h * st.v_h + src0 * st.v_key, st.v_key, st.dv + dst, n, nullptr, 0,
+                      st.dn ? st.dn + b * st.dn_b + h * st.dn_h + dst0 : nullptr);
+}
+
 // ALL: codes, 4-bit records, weights and cluster sizes are all written (the caller's pointers are all set), so the
 // loop body has no branch around a store.  Loads and stores retire through one in-order counter; with a store that
 // may or may not have been issued after the load of the next key, the only safe wait for that key is "everything
 // outstanding", stores included.  Without the branches the wait names the exact count and the stores stay in flight.
-template <bool BF16, bool ALL>
+// STORE (with ALL): the launch also stores the prompt's rows, see EncStore.
+template <bool BF16, bool ALL, int STORE>
 __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEncWavesPerSimd, kEncWavesPerSimd))) void pkv_encode_kernel(
     const void *__restrict__ keys, int n_kv_heads, int64_t n_keys, int64_t k_stride_b, int64_t k_stride_h,
     int64_t k_stride_key, const float *__restrict__ signs, uint8_t *__restrict__ codes, int64_t cs_b, int64_t cs_h,
     int64_t cs_key, int64_t cs_sub, uint8_t *__restrict__ nib, int64_t ns_b, int64_t ns_h, int64_t ns_key,
     int64_t ns_sub, uint16_t *__restrict__ weight, int64_t ws_b, int64_t ws_h, int64_t ws_key, int64_t ws_sub,
-    int32_t *__restrict__ cluster_counts, int64_t cc_b, int64_t cc_h, int keys_per_wg) {
+    int32_t *__restrict__ cluster_counts, int64_t cc_b, int64_t cc_h, int keys_per_wg, EncStore st) {
   const bool has_nib = ALL || nib, has_weight = ALL || weight, has_hist = ALL || cluster_counts;
-  const int row = blockIdx.y;
-  const int b = row / n_kv_heads, h = row % n_kv_heads;
+  const int b = STORE ? (int)blockIdx.z : (int)blockIdx.y / n_kv_heads, h = STORE ? (int)blockIdx.y : (int)blockIdx.y % n_kv_heads;
+  if (STORE && (int)blockIdx.x >= st.n_blocks) {
+    enc_store_dense<BF16>(st, b, h, (int)blockIdx.x - st.n_blocks);
+    return;
+  }
   const int tid = threadIdx.x;
   const int s = enc_block_of_lane(tid & 15);  // block (subspace) owned by this lane
   const int kq = tid >> 4;  // key slot inside the iteration
@@ -478,6 +588,7 @@ __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEn
   __shared__ __align__(16) uint2 s_mag[BF16 ? kMagEntries : 2];
   __shared__ float s_centers[8];  // magnitude centres, looked up by code (an LDS read instead of a load from constant memory)
   __shared__ uint32_t s_spread[256];
+  __shared__ float s_norm[STORE == kEncStoreRecords ? kEncKeysPerWg : 1];
   __shared__ __align__(16) pkv_u32x4 s_band[BF16 ? 1 : kMagBands];
   if (tid < 8) s_centers[tid] = c_centers[tid];
   if (!BF16 && tid < kMagBands) s_band[tid] = ((const pkv_u32x4 *)g_enc_tables.band)[tid];
@@ -490,6 +601,15 @@ __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEn
   }
   if (has_hist)
     for (int i = tid; i < 16 * 256; i += kEncThreads) s_hist[i] = 0;
+  if (STORE) {
+    constexpr int row_bytes = BF16 ? 256 : 512;
+    const int64_t i0 = (int64_t)blockIdx.x * keys_per_wg;
+    enc_copy_rows<BF16>(st.v + b * st.v_b + h * st.v_h + i0 * st.v_key, st.v_key, st.zv + b * st.z_b + h * st.z_h + i0 * row_bytes,
+                        (int)(n_keys - i0 < keys_per_wg ? n_keys - i0 : keys_per_wg),
+                        st.zn ? st.zn + b * st.zn_b + h * st.zn_h + i0 * st.zn_key : nullptr, st.zn_key,
+                        st.zn2 ? st.zn2 + b * st.zn2_b + h * st.zn2_h + i0 : nullptr,
+                        STORE == kEncStoreRecords && st.record_norm ? s_norm : nullptr);
+  }
   __syncthreads();
 
   float sg[8];
@@ -517,7 +637,10 @@ __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEn
   const uint32_t key_bytes = (uint32_t)(k_stride_key * esize), blk_off = (uint32_t)(8 * s * esize);
   const uint32_t k_lane = (uint32_t)kq * key_bytes + blk_off;
   const uint32_t c_lane = (uint32_t)(kq * cs_key + s * cs_sub), n_lane = (uint32_t)(kq * ns_key + s * ns_sub),
-                 w_lane = (uint32_t)(2 * (kq * ws_key + s * ws_sub));
+                 w_blk = STORE == kEncStoreRecords ? (uint32_t)(4 * (s >> 1) + (s & 1) * 32) : (uint32_t)(2 * s * ws_sub),
+                 w_lane = (uint32_t)(2 * kq * ws_key) + w_blk;
+  char *z_base = STORE ? st.zk + b * st.z_b + h * st.z_h + key_begin * (128 * esize) : nullptr;
+  const uint32_t z_lane = (uint32_t)kq * (128 * esize) + blk_off;
   const int64_t k_step = (int64_t)kEncKeysPerIter * k_stride_key * esize, c_step = (int64_t)kEncKeysPerIter * cs_key,
                 n_step = (int64_t)kEncKeysPerIter * ns_key, w_step = (int64_t)kEncKeysPerIter * ws_key * 2;
   // A wave keeps the keys of its next kEncAhead iterations in flight, each in a register set of its own: set j holds
@@ -545,6 +668,14 @@ __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEn
 #pragma unroll
     for (int q = 0; q < kW; ++q) cur[q] = reg[q];
     load_iter(it + kEncAhead, reg);
+    if (STORE) {  // lanes past a ragged end hold the block's last key and store that row once more
+      char *zb = z_base + (int64_t)it * (kEncKeysPerIter * 128 * esize);
+      uint32_t z_off = z_lane;
+      if (last - first < kEncKeysPerIter - 1) z_off = (uint32_t)(kq < last - first ? kq : last - first) * (128 * esize) + blk_off;
+      asm volatile("" : "+v"(z_off));
+#pragma unroll
+      for (int q = 0; q < kW; ++q) __builtin_nontemporal_store(cur[q], (pkv_u32x4 *)(zb + z_off) + q);
+    }
     EncOut o;
     bool exact = true;
     float x[8];
@@ -586,13 +717,21 @@ __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEn
         const uint32_t kk = (uint32_t)(kq < last - first ? kq : last - first);
         c_off = kk * (uint32_t)cs_key + (uint32_t)(s * cs_sub);
         n_off = kk * (uint32_t)ns_key + (uint32_t)(s * ns_sub);
-        w_off = 2 * (kk * (uint32_t)ws_key + (uint32_t)(s * ws_sub));
+        w_off = 2 * kk * (uint32_t)ws_key + w_blk;
       }
       asm volatile("" : "+v"(c_off), "+v"(n_off), "+v"(w_off));
       // written once and not read again by this launch: streaming stores (5 - 8 % on two of three shapes)
       __builtin_nontemporal_store((uint8_t)o.code, cb + c_off);
       __builtin_nontemporal_store(o.packed, (uint32_t *)(nb + n_off));
-      __builtin_nontemporal_store((uint16_t)o.wbits, (uint16_t *)(wb + w_off));
+      if (STORE == kEncStoreRecords) {
+        // the second half of the record as sixteen words: even blocks hold two weights, block 1 the value norm
+        const uint32_t pair = o.wbits | (pkv_lane_xor<1>(o.wbits) << 16);
+        const float norm = st.record_norm ? s_norm[first + (kq < last - first ? kq : last - first)] : 0.f;
+        const uint32_t word = (s & 1) ? (s == 1 ? __float_as_uint(norm) : 0u) : pair;
+        __builtin_nontemporal_store(word, (uint32_t *)(wb + w_off));
+      } else {
+        __builtin_nontemporal_store((uint16_t)o.wbits, (uint16_t *)(wb + w_off));
+      }
       if (active) atomicAdd(&s_hist[s * 256 + o.code], 1u);
     } else if (active) {
       asm volatile("" : "+v"(c_off), "+v"(n_off), "+v"(w_off));
@@ -673,9 +812,9 @@ extern "C" int pkv_encode_append(const void *keys, int dtype, int bs, int n_kv_h
   const int64_t per_wg = kEncKeysPerWg;
   dim3 grid((unsigned)((n_keys + per_wg - 1) / per_wg), (unsigned)rows);
 #define PKV_ENC(BF, ALL)                                                                                               \
-  hipLaunchKernelGGL((pkv_encode_kernel<BF, ALL>), grid, dim3(kEncThreads), 0, (hipStream_t)stream, keys, n_kv_heads,  \
+  hipLaunchKernelGGL((pkv_encode_kernel<BF, ALL, kEncNoStore>), grid, dim3(kEncThreads), 0, (hipStream_t)stream, keys, n_kv_heads,  \
                      n_keys, k_stride_b, k_stride_h, k_stride_key, signs, codes, cs_b, cs_h, cs_key, cs_sub, nib, ns_b, \
-                     ns_h, ns_key, ns_sub, weight, ws_b, ws_h, ws_key, ws_sub, cluster_counts, cc_b, cc_h, (int)per_wg)
+                     ns_h, ns_key, ns_sub, weight, ws_b, ws_h, ws_key, ws_sub, cluster_counts, cc_b, cc_h, (int)per_wg, EncStore())
   const bool all = nib && weight && cluster_counts;
   if (dtype == PKV_DTYPE_BF16) {
     if (all) PKV_ENC(true, true); else PKV_ENC(true, false);
@@ -683,6 +822,81 @@ extern "C" int pkv_encode_append(const void *keys, int dtype, int bs, int n_kv_h
     if (all) PKV_ENC(false, true); else PKV_ENC(false, false);
   }
 #undef PKV_ENC
+  PKV_LAUNCH_CHECK("pkv_encode_kernel");
+  return PKV_OK;
+}
+
+extern "C" int pkv_prefill_store(const pkv_prefill_args *a, void *stream) {
+  PKV_REQUIRE(a != nullptr, "pkv_prefill_store: null args");
+  PKV_REQUIRE(a->dtype == PKV_DTYPE_F32 || a->dtype == PKV_DTYPE_BF16, "unknown dtype %d", a->dtype);
+  PKV_REQUIRE(a->bs > 0 && a->bs <= 65535 && a->n_kv_heads > 0 && (int64_t)a->bs * a->n_kv_heads <= 65535,
+              "bad shape bs=%d kv_heads=%d", a->bs, a->n_kv_heads);
+  PKV_REQUIRE(a->n_sink >= 0 && a->n_encode >= 0 && a->n_tail >= 0 && a->tail_row0 >= a->n_sink &&
+                  a->n_sink + a->n_encode + a->n_tail < ((int64_t)1 << 23),
+              "pkv_prefill_store: bad token counts %lld + %lld + %lld", (long long)a->n_sink, (long long)a->n_encode,
+              (long long)a->n_tail);
+  if (a->n_sink + a->n_encode + a->n_tail == 0) return PKV_OK;
+  const bool bf = a->dtype == PKV_DTYPE_BF16;
+  const int64_t vec = bf ? 8 : 4, es = bf ? 2 : 4;
+  PKV_REQUIRE(a->k && a->v && pkv_aligned(a->k, 16) && pkv_aligned(a->v, 16) && a->k_stride_b % vec == 0 &&
+                  a->k_stride_h % vec == 0 && a->k_stride_key % vec == 0 && a->v_stride_b % vec == 0 &&
+                  a->v_stride_h % vec == 0 && a->v_stride_key % vec == 0 && a->k_stride_key >= 0 && a->v_stride_key >= 0,
+              "pkv_prefill_store: K/V must be 16-byte aligned with 16-byte-multiple strides");
+  PKV_REQUIRE(a->n_sink + a->n_tail == 0 ||
+                  (a->dense_k && a->dense_v && pkv_aligned(a->dense_k, 16) && pkv_aligned(a->dense_v, 16) &&
+                   a->dense_stride_b % vec == 0 && a->dense_stride_h % vec == 0),
+              "pkv_prefill_store: the dense rows need a 16-byte aligned destination");
+  if (a->n_encode > 0) {
+    PKV_REQUIRE(a->zone_k && a->zone_v && pkv_aligned(a->zone_k, 16) && pkv_aligned(a->zone_v, 16) &&
+                    a->zone_stride_b % vec == 0 && a->zone_stride_h % vec == 0,
+                "pkv_prefill_store: the encoded tokens' rows need a 16-byte aligned destination");
+    PKV_REQUIRE(a->signs && a->codes && a->nib && a->weight && a->cluster_counts, "pkv_prefill_store: null index pointer");
+    PKV_REQUIRE(pkv_aligned(a->nib, 4) && a->ns_b % 4 == 0 && a->ns_h % 4 == 0 && a->ns_key % 4 == 0 && a->ns_sub % 4 == 0,
+                "packed 4-bit blocks must be 4-byte aligned");
+    const int64_t lim = (int64_t)1 << 31;  // a lane's byte offsets inside one iteration's keys are kept in 32 bits
+    PKV_REQUIRE(a->cs_key >= 0 && a->cs_sub >= 0 && a->ns_key >= 0 && a->ns_sub >= 0 && a->ws_key >= 0 && a->ws_sub >= 0 &&
+                    kEncKeysPerIter * a->k_stride_key * 4 + 512 < lim && kEncKeysPerIter * a->cs_key + 16 * a->cs_sub < lim &&
+                    kEncKeysPerIter * a->ns_key + 16 * a->ns_sub < lim && 2 * (kEncKeysPerIter * a->ws_key + 16 * a->ws_sub) < lim,
+                "pkv_prefill_store: key or block strides out of range");
+  }
+  EncStore st;
+  memset(&st, 0, sizeof st);
+  const char *k = (const char *)a->k, *v = (const char *)a->v;
+  st.dk_src = k, st.dv_src = v;
+  st.k_b = a->k_stride_b * es, st.k_h = a->k_stride_h * es, st.k_key = a->k_stride_key * es;
+  st.v_b = a->v_stride_b * es, st.v_h = a->v_stride_h * es, st.v_key = a->v_stride_key * es;
+  st.v = v + a->n_sink * st.v_key;
+  st.zk = (char *)a->zone_k, st.zv = (char *)a->zone_v, st.z_b = a->zone_stride_b * es, st.z_h = a->zone_stride_h * es;
+  st.zn = a->zone_vnorm, st.zn_b = a->zn_b, st.zn_h = a->zn_h, st.zn_key = a->zn_key;
+  st.zn2 = a->zone_vnorm2, st.zn2_b = a->zn2_b, st.zn2_h = a->zn2_h;
+  st.dk = (char *)a->dense_k, st.dv = (char *)a->dense_v, st.d_b = a->dense_stride_b * es, st.d_h = a->dense_stride_h * es;
+  st.dn = a->dense_vnorm, st.dn_b = a->dn_b, st.dn_h = a->dn_h;
+  st.n_sink = (int)a->n_sink, st.n_tail = (int)a->n_tail;
+  st.tail_src0 = a->n_sink + a->n_encode, st.tail_row0 = a->tail_row0;
+  st.n_blocks = (int)((a->n_encode + kEncKeysPerWg - 1) / kEncKeysPerWg);
+  // key records (64 nibble bytes, 32 weight bytes, a tail of 32): written whole where the tail belongs to this call,
+  // i.e. where the value norms, if wanted, go to its first word
+  const bool norm_in_record = a->zone_vnorm && (const uint8_t *)a->zone_vnorm == a->nib + 96 && a->zn_key == 32 &&
+                              a->zn_b * 4 == a->ns_b && a->zn_h * 4 == a->ns_h;
+  const bool records = a->n_encode > 0 && pkv_aligned(a->nib, 128) && a->ns_key == 128 && a->ns_sub == 4 &&
+                       a->ns_b % 128 == 0 && a->ns_h % 128 == 0 && (const uint8_t *)a->weight == a->nib + 64 &&
+                       a->ws_key == 64 && a->ws_sub == 1 && a->ws_b * 2 == a->ns_b && a->ws_h * 2 == a->ns_h &&
+                       (!a->zone_vnorm || norm_in_record);
+  if (records && norm_in_record) st.record_norm = 1, st.zn = nullptr;
+  const int dense_blocks = (st.n_sink + kEncDenseRows - 1) / kEncDenseRows + (st.n_tail + kEncDenseRows - 1) / kEncDenseRows;
+  const dim3 grid((unsigned)(st.n_blocks + dense_blocks), (unsigned)a->n_kv_heads, (unsigned)a->bs);
+#define PKV_ENC_ST(BF, MODE)                                                                                           \
+  hipLaunchKernelGGL((pkv_encode_kernel<BF, true, MODE>), grid, dim3(kEncThreads), 0, (hipStream_t)stream,              \
+                     k + a->n_sink * st.k_key, a->n_kv_heads, a->n_encode, a->k_stride_b, a->k_stride_h, a->k_stride_key, \
+                     a->signs, a->codes, a->cs_b, a->cs_h, a->cs_key, a->cs_sub, a->nib, a->ns_b, a->ns_h, a->ns_key,   \
+                     a->ns_sub, a->weight, a->ws_b, a->ws_h, a->ws_key, a->ws_sub, a->cluster_counts, a->cc_b, a->cc_h, \
+                     kEncKeysPerWg, st)
+  if (bf) {
+    if (records) PKV_ENC_ST(true, kEncStoreRecords); else PKV_ENC_ST(true, kEncStoreRows);
+  } else {
+    if (records) PKV_ENC_ST(false, kEncStoreRecords); else PKV_ENC_ST(false, kEncStoreRows);
+  }
+#undef PKV_ENC_ST
   PKV_LAUNCH_CHECK("pkv_encode_kernel");
   return PKV_OK;
 }

@@ -146,6 +146,71 @@ def encode_append(keys: torch.Tensor, signs: torch.Tensor, codebook: torch.Tenso
         _p(key_4bit), *ns, _p(key_block_weight), *ws, _p(cluster_counts), *cc, _stream(keys)))
 
 
+def prefill_store(k: torch.Tensor, v: torch.Tensor, n_sink: int, n_encode: int, signs: torch.Tensor, dense=None, tail_row0: int = 0,
+                  zone=None, index=None, dense_vnorm: Optional[torch.Tensor] = None,
+                  zone_vnorm: Optional[torch.Tensor] = None, zone_vnorm2: Optional[torch.Tensor] = None) -> None:
+    """Rows of a prompt into the cache and the index of its retrieval zone in one launch (cache_hub/polar_cache.py:430-504).
+
+    k, v [bs,H,S,128] (any strides, contiguous rows): tokens [0, n_sink) and the tail behind the n_encode encoded ones are
+    copied to rows 0.. and tail_row0.. of ``dense`` = (dk, dv) [bs,H,rows,128]; the n_encode tokens from n_sink on are
+    copied to rows 0.. of ``zone`` = (zk, zv) and encoded into ``index`` = (codebook, key_4bit, key_block_weight,
+    cluster_counts), shaped for them as in :func:`encode_append`.  fp32 value norms: ``dense_vnorm`` [bs,H,rows] by dense
+    row, ``zone_vnorm`` / ``zone_vnorm2`` [bs,H,n_encode]."""
+    bs, H, S, D = k.shape
+    n_tail = S - n_sink - n_encode
+    _cuda(k, v)
+    _need(D == HEAD_DIM and v.shape == k.shape and v.dtype == k.dtype and n_sink >= 0 and n_encode >= 0 and n_tail >= 0,
+          "k, v: [bs,H,S,128] of one dtype, n_sink + n_encode <= S")
+    _need(k.stride(3) == 1 and v.stride(3) == 1, "k, v: contiguous rows")
+    a = _lib.PrefillArgs()
+    a.k, a.v, a.dtype, a.bs, a.n_kv_heads = k.data_ptr(), v.data_ptr(), _dt(k.dtype), bs, H
+    a.k_stride_b, a.k_stride_h, a.k_stride_key = k.stride()[:3]
+    a.v_stride_b, a.v_stride_h, a.v_stride_key = v.stride()[:3]
+    a.n_sink, a.n_encode, a.n_tail, a.tail_row0 = n_sink, n_encode, n_tail, tail_row0 if n_tail else n_sink
+
+    def rows_of(pair, need):
+        dk, dv = pair
+        _cuda(dk, dv)
+        _need(dk.dtype == k.dtype and dv.dtype == k.dtype and dk.shape == dv.shape and dk.stride() == dv.stride() and
+              tuple(dk.shape[:2]) == (bs, H) and dk.shape[3] == D and dk.stride(3) == 1 and dk.stride(2) == D and
+              dk.shape[2] >= need, f"destination: [bs,H,>={need},128] of the source dtype with contiguous rows")
+        return dk.data_ptr(), dv.data_ptr(), dk.stride(0), dk.stride(1)
+
+    def norms_of(t, need, unit):
+        _cuda(t)
+        _need(t.dtype == torch.float32 and tuple(t.shape[:2]) == (bs, H) and t.shape[2] >= need and
+              (not unit or t.stride(2) == 1), f"value norms: fp32 [bs,H,>={need}]")
+        return t.data_ptr(), t.stride(0), t.stride(1)
+
+    if n_sink + n_tail > 0:
+        need = max(n_sink, tail_row0 + n_tail if n_tail else 0)
+        a.dense_k, a.dense_v, a.dense_stride_b, a.dense_stride_h = rows_of(dense, need)
+        if dense_vnorm is not None:
+            a.dense_vnorm, a.dn_b, a.dn_h = norms_of(dense_vnorm, need, True)
+    if n_encode > 0:
+        a.zone_k, a.zone_v, a.zone_stride_b, a.zone_stride_h = rows_of(zone, n_encode)
+        cb, k4, kw, cc = index
+        _cuda(cb, k4, kw, cc)
+        _need(signs.is_cuda and signs.dtype == torch.float32 and signs.numel() == HEAD_DIM and signs.is_contiguous(), "signs: float32[128]")
+        _need(cb.dtype == torch.uint8 and tuple(cb.shape) == (bs, H, B_SUB, n_encode), "codebook must be u8 [bs,H,16,n_encode]")
+        _need(k4.dtype == torch.uint8 and tuple(k4.shape) == (bs, H, B_SUB, n_encode, 4) and k4.stride(4) == 1,
+              "key_4bit must be u8 [bs,H,16,n_encode,4] with a contiguous last dim")
+        _need(kw.dtype == torch.bfloat16 and tuple(kw.shape) == (bs, H, B_SUB, n_encode), "key_block_weight must be bf16 [bs,H,16,n_encode]")
+        _need(cc.dtype == torch.int32 and tuple(cc.shape) == (bs, H, B_SUB, K_CLUSTERS) and cc.stride(3) == 1 and
+              cc.stride(2) == K_CLUSTERS, "cluster_counts must be int32 [bs,H,16,256] with contiguous [16,256] blocks")
+        a.signs = signs.data_ptr()
+        a.codes, a.cs_b, a.cs_h, a.cs_sub, a.cs_key = (cb.data_ptr(),) + cb.stride()
+        a.nib, a.ns_b, a.ns_h, a.ns_sub, a.ns_key = (k4.data_ptr(),) + k4.stride()[:4]
+        a.weight, a.ws_b, a.ws_h, a.ws_sub, a.ws_key = (kw.data_ptr(),) + kw.stride()
+        a.cluster_counts, a.cc_b, a.cc_h = cc.data_ptr(), cc.stride(0), cc.stride(1)
+        if zone_vnorm is not None:
+            a.zone_vnorm, a.zn_b, a.zn_h = norms_of(zone_vnorm, n_encode, False)
+            a.zn_key = zone_vnorm.stride(2)
+        if zone_vnorm2 is not None:
+            a.zone_vnorm2, a.zn2_b, a.zn2_h = norms_of(zone_vnorm2, n_encode, True)
+    _lib.check(_lib.lib().pkv_prefill_store(C.byref(a), _stream(k)))
+
+
 def count_cluster_keys(codebook: torch.Tensor, cluster_counts: torch.Tensor) -> None:
     """cluster_counts[bs,H,16,256] += per-subspace histogram of codebook [bs,H,16,N]."""
     _cuda(codebook, cluster_counts)

@@ -1654,3 +1654,50 @@ def test_offload_rows_equals_sliced_copy(ops, engine):
         ops.offload_rows(stage_k, stage_v, kc[:bs], vc[:bs], cap - 9, **kw)
     with pytest.raises(RuntimeError):
         ops.offload_rows(stage_k, stage_v, kc[:bs].clone(), vc[:bs], 0, **kw)   # not pinned
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n_sink,n_enc,n_tail", [(0, 1, 0), (4, 255, 3), (64, 256, 64), (65, 2049, 129), (70, 0, 0), (3, 4097, 1)])
+def test_prefill_store_rows_index_and_norms(ops, dtype, n_sink, n_enc, n_tail):
+    """pkv_prefill_store at and beside its workgroup sizes (256 encoded, 64 dense tokens): rows copied bit for bit to
+    their places and nowhere else, the index equal to pkv_encode_append's on the same keys, value norms equal to the
+    oracle's restatement."""
+    bs, H, S = 2, 3, n_sink + n_enc + n_tail
+    odt = O.BF16 if dtype == torch.bfloat16 else O.F32
+    _say(f"prefill_store {dtype} {n_sink}+{n_enc}+{n_tail}")
+    gen = torch.Generator().manual_seed(S)
+    k = torch.randn(bs, S, H, 128, generator=gen).to(dtype).to(DEV)
+    v = torch.randn(bs, S, H, 128, generator=gen).to(dtype).to(DEV)
+    kp, vp = k.permute(0, 2, 1, 3), v.permute(0, 2, 1, 3)
+    signs = ops.srht_signs(DEV)
+    gap, cap = 2, n_enc + 5                                # rows between the sink and the tail, spare rows behind
+    tail0 = n_sink + gap
+    dk = torch.full((bs, H, tail0 + n_tail + 3, 128), 7.0, dtype=dtype, device=DEV)
+    zk = torch.full((bs, H, cap, 128), 7.0, dtype=dtype, device=DEV)
+    dv, zv = dk.clone(), zk.clone()
+    dn = torch.full(dk.shape[:3], 7.0, device=DEV)
+    zn2 = torch.full((bs, H, cap), 7.0, device=DEV)
+    codes, nib, w, cb, k4, kw = ops.alloc_keymajor(bs, H, cap, DEV)
+    zn = ops.record_value_norm_view(nib)
+    cc = torch.ones(bs, H, 16, 256, dtype=torch.int32, device=DEV)
+    sl = slice(0, n_enc)
+    ops.prefill_store(kp, vp, n_sink, n_enc, signs, (dk, dv), tail0, (zk, zv),
+                      (cb[..., sl], k4[:, :, :, sl], kw[..., sl], cc) if n_enc else None, dense_vnorm=dn,
+                      zone_vnorm=zn[..., sl], zone_vnorm2=zn2)
+    norm = torch.from_numpy(O.value_norm(vp.float().cpu().contiguous().view(-1, 128).numpy(), odt)).view(bs, H, S).to(DEV)
+    for src, dense, zone in ((kp, dk, zk), (vp, dv, zv)):
+        want_d, want_z = torch.full_like(dense, 7.0), torch.full_like(zone, 7.0)
+        want_d[:, :, :n_sink], want_d[:, :, tail0:tail0 + n_tail] = src[:, :, :n_sink], src[:, :, n_sink + n_enc:]
+        want_z[:, :, :n_enc] = src[:, :, n_sink:n_sink + n_enc]
+        assert torch.equal(dense, want_d) and torch.equal(zone, want_z)
+    want = torch.full_like(dn, 7.0)
+    want[:, :, :n_sink], want[:, :, tail0:tail0 + n_tail] = norm[:, :, :n_sink], norm[:, :, n_sink + n_enc:]
+    assert torch.equal(dn, want)
+    if n_enc:
+        codes2, nib2, w2, cb2, k42, kw2 = ops.alloc_keymajor(bs, H, cap, DEV)
+        cc2 = torch.ones_like(cc)
+        ops.encode_append(kp[:, :, n_sink:n_sink + n_enc], signs, cb2[..., sl], k42[:, :, :, sl], kw2[..., sl], cc2)
+        assert torch.equal(codes, codes2) and torch.equal(nib, nib2) and torch.equal(w.view(torch.int16), w2.view(torch.int16))
+        assert torch.equal(cc, cc2)
+        assert torch.equal(zn[..., sl], norm[:, :, n_sink:n_sink + n_enc]) and torch.equal(zn2[..., sl], norm[:, :, n_sink:n_sink + n_enc])
+        assert torch.all(zn[..., n_enc:] == 0) and torch.all(zn2[..., n_enc:] == 7.0)
