@@ -30,6 +30,9 @@ from .cache import KV_Cache
 from .zones import LayerZones
 
 USE_RABITQ_RERANK = True
+# Offloading layers attend to every token while the sequence is below the dense-attention threshold; up to this threshold
+# the rows such a step needs also stay in HBM (see polar_cache._short_rows)
+SHORT_ROWS_MAX = 4096
 DEFAULT_SRHT_ROUNDS = 1
 
 
@@ -114,6 +117,7 @@ class polar_cache(KV_Cache):
         self.unified_values_cpu = [None] * layer_num if enable_offload else None
         self.cpu_valid_end = [0] * layer_num if enable_offload else None
         self._layer_offload = [False] * layer_num
+        self._short_kv = [None] * layer_num  # (k, v, samples present), see _short_rows
         self._offload_keys_buffer = [None] * layer_num
         self._offload_values_buffer = [None] * layer_num
         if enable_offload:
@@ -250,6 +254,29 @@ class polar_cache(KV_Cache):
             self._prefill_stage[slot] = pair
         return slot, pair[0][:need].view(shape), pair[1][:need].view(shape)
 
+    def _min_total(self) -> int:
+        """Sequence length from which a step retrieves instead of attending to every token (:1008-1013)."""
+        return max(self.FULL_ATTENTION_THRESHOLD, self.sink_size + self.local_size + self.final_topk * 2)
+
+    def _short_rows(self, layer_idx: int, b0: int, b1: int, n_tok: int):
+        """Where the prefill of samples b0..b1-1 puts the retrieval-zone rows of a prompt that is still below the
+        dense-attention threshold: K/V [b1-b0,H,rows,D] in HBM, beside the host store.  Every step of such a sequence
+        attends to all of its tokens; read from the host they cost a wait for the copy stream and two strided copies over
+        PCIe per layer and token (235 us for 924 rows x 8 heads), from HBM 7 us.  At most SHORT_ROWS_MAX rows a head;
+        given back by the first step that retrieves.  None for longer prompts or a threshold too high for that."""
+        rows = self._min_total() - self.sink_size - self.local_size
+        if n_tok >= self._min_total() or rows > SHORT_ROWS_MAX:
+            self._short_kv[layer_idx] = None
+            return None
+        kv = self._short_kv[layer_idx]
+        if kv is None or kv[0].shape[2] < rows:
+            shape = (self.batch_size, self.kv_head, rows, self.head_dim)
+            kv = (torch.empty(shape, dtype=self.dtype, device=self.device),
+                  torch.empty(shape, dtype=self.dtype, device=self.device), [False] * self.batch_size)
+            self._short_kv[layer_idx] = kv
+        kv[2][b0:b1] = [True] * (b1 - b0)   # samples whose rows are here: prompts may arrive one by one
+        return kv[0][b0:b1], kv[1][b0:b1]
+
     def release_prefill_staging(self) -> None:
         """Free the prefill staging pairs (two layers' worth of retrieval-zone K/V in HBM) once prefill is over; they
         are allocated again on demand."""
@@ -312,9 +339,15 @@ class polar_cache(KV_Cache):
         self.cluster_key_counts_gpu[layer_idx][b0:b1].zero_()  # prefill assigns, refresh accumulates (:493, :775)
         if self._layer_offload[layer_idx]:
             self._wait_offload(layer_idx)
-            slot, stage_k, stage_v = self._prefill_stage_rows((bsz, self.kv_head, retrieval, self.head_dim))
+            short = self._short_rows(layer_idx, b0, b1, n_tok)
+            if short is not None:  # the rows stay in HBM as well, and leave for the host from there
+                stage_k, stage_v = (t[:, :, :retrieval] for t in short)
+            else:
+                slot, stage_k, stage_v = self._prefill_stage_rows((bsz, self.kv_head, retrieval, self.head_dim))
             self._store_rows(layer_idx, k, v, b0, b1, S0, retrieval, dense, S0, (stage_k, stage_v), S0)
-            self._prefill_stage_event[slot] = self._offload_rows(layer_idx, b0, b1, stage_k, stage_v, 0)
+            event = self._offload_rows(layer_idx, b0, b1, stage_k, stage_v, 0)
+            if short is None:
+                self._prefill_stage_event[slot] = event
             self.cpu_valid_end[layer_idx] = retrieval
         else:
             self._store_rows(layer_idx, k, v, b0, b1, S0, retrieval, dense, r_end, (dense[0][:, :, S0:], dense[1][:, :, S0:]), S0)
@@ -365,7 +398,14 @@ class polar_cache(KV_Cache):
             self._on_refresh(layer_idx, r)
             return
         self._wait_offload(layer_idx)  # staging buffers are free again
-        sk, sv = self._offload_keys_buffer[layer_idx][:, :, :n], self._offload_values_buffer[layer_idx][:, :, :n]
+        if r.cpu_row0 == 0:  # the first tokens of the zone: a prompt without one, or none yet
+            self._short_rows(layer_idx, 0, bs, self.current_seq_len[layer_idx])
+        short = self._short_kv[layer_idx]
+        if short is not None and self.current_seq_len[layer_idx] < self._min_total() and r.cpu_row0 + n <= short[0].shape[2]:
+            sk, sv = (t[:, :, r.cpu_row0:r.cpu_row0 + n] for t in short[:2])
+        else:
+            self._short_kv[layer_idx] = None
+            sk, sv = self._offload_keys_buffer[layer_idx][:, :, :n], self._offload_values_buffer[layer_idx][:, :, :n]
         self._store_rows(layer_idx, kg[:, :, S0:S0 + n], vg[:, :, S0:S0 + n], 0, bs, 0, n, None, 0, (sk, sv), r.encode_abs0)
         self._on_refresh(layer_idx, r)
         self._offload_rows(layer_idx, 0, bs, sk, sv, r.cpu_row0)
@@ -414,19 +454,22 @@ class polar_cache(KV_Cache):
         return self._attention.run(queries, [s for s in segments if s[3] > 0])
 
     def _full_kv(self, layer_idx):
-        """Dense fallback: every stored token (reference _get_full_kv_for_attention :701-737)."""
+        """Dense fallback: every stored token (reference _get_full_kv_for_attention :701-737), as attention segments."""
         z = self._zones[layer_idx]
         kg, vg = self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx]
         if not self._layer_offload[layer_idx]:
-            return kg[:, :, :z.seq_len], vg[:, :, :z.seq_len]
+            return [(kg, vg, 0, z.seq_len)]
         n = z.gpu_prefix_rows
         if z.encoded == 0:
-            return kg[:, :, :n], vg[:, :, :n]
+            return [(kg, vg, 0, n)]
+        short = self._short_kv[layer_idx]
+        if short is not None and z.encoded <= short[0].shape[2] and all(short[2]):
+            return [(kg, vg, 0, n), (short[0], short[1], 0, z.encoded)]
         self._copy_stream.synchronize()  # the host reads below must see what the copy stream wrote (:707)
         self._offload_inflight[layer_idx] = False
         rk = self.unified_keys_cpu[layer_idx][:, :, :z.encoded].to(self.device, non_blocking=True)
         rv = self.unified_values_cpu[layer_idx][:, :, :z.encoded].to(self.device, non_blocking=True)
-        return torch.cat([kg[:, :, :n], rk], dim=2), torch.cat([vg[:, :, :n], rv], dim=2)
+        return [(kg, vg, 0, n), (rk, rv, 0, z.encoded)]
 
     def retrieval_shape(self, layer_idx):
         """(n_keys, n_cand, k, tier_counts) the next retrieval of this layer will use."""
@@ -451,8 +494,7 @@ class polar_cache(KV_Cache):
         n_keys = self.cpu_valid_end[layer_idx] if self._layer_offload[layer_idx] else z.encoded
         if step[0] != n_keys or z.next_append_refreshes():
             return None
-        min_total = max(self.FULL_ATTENTION_THRESHOLD, self.sink_size + self.local_size + self.final_topk * 2)
-        return step[1] if z.seq_len + 1 >= min_total and n_keys > 0 else None
+        return step[1] if z.seq_len + 1 >= self._min_total() and n_keys > 0 else None
 
     def _bound_step_of(self, layer_idx):
         return self._bound[layer_idx]
@@ -463,12 +505,9 @@ class polar_cache(KV_Cache):
         total = z.seq_len
         offload = self._layer_offload[layer_idx]
         n_keys = self.cpu_valid_end[layer_idx] if offload else z.encoded
-        min_total = max(self.FULL_ATTENTION_THRESHOLD, self.sink_size + self.local_size + self.final_topk * 2)
-        if total < min_total or n_keys <= 0:
-            k, v = self._full_kv(layer_idx)
-            if not (k.stride(3) == 1 and k.stride(2) == self.head_dim and v.stride() == k.stride()):
-                k, v = k.contiguous(), v.contiguous()
-            return self._attend(queries.contiguous(), [(k, v, 0, k.shape[2])])
+        if total < self._min_total() or n_keys <= 0:
+            return self._attend(queries.contiguous(), self._full_kv(layer_idx))
+        self._short_kv[layer_idx] = None   # the sequence has outgrown the dense branch
         q = queries if queries.is_contiguous() else queries.contiguous()
         step = self._bound[layer_idx]
         if step is None or step[0] != n_keys:

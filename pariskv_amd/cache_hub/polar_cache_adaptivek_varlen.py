@@ -153,9 +153,9 @@ class polar_cache(_polar_cache_base):
         z = self._zones[layer_idx]
         total = z.seq_len
         n_keys = self.cpu_valid_end[layer_idx]
-        min_total = max(self.FULL_ATTENTION_THRESHOLD, self.sink_size + self.local_size + self.final_topk * 2)
-        if total < min_total or n_keys <= 0:
+        if total < self._min_total() or n_keys <= 0:
             return super().compute(queries, layer_idx)  # dense branch
+        self._short_kv[layer_idx] = None   # the sequence has outgrown it
         q = queries if queries.is_contiguous() else queries.contiguous()
         step = self._adaptive_bound[layer_idx]
         if step is None or step[0] != n_keys:

@@ -79,8 +79,7 @@ class polar_cache(_adaptive_base):
             return super().compute(queries, layer_idx)  # the fused step, with the broadcast of max k switched on
         z = self._zones[layer_idx]
         total, n_keys = z.seq_len, z.encoded
-        min_total = max(self.FULL_ATTENTION_THRESHOLD, self.sink_size + self.local_size + self.final_topk * 2)
-        if total < min_total or n_keys <= 0:
+        if total < self._min_total() or n_keys <= 0:
             return _polar_cache_base.compute(self, queries, layer_idx)  # dense branch
         q = queries if queries.is_contiguous() else queries.contiguous()
         bs, H, S0 = self.batch_size, self.kv_head, self.sink_size

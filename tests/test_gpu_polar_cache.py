@@ -874,3 +874,46 @@ def test_fp32_cache_decode_steps(offload):
                                                         hv[b].permute(1, 0, 2)[h:h + 1, sel], G=G * 10)
             err = (out[b, 0].cpu() - ref).abs().max().item()
             assert err < 1e-3, f"step {step}: attention differs by {err}"
+
+
+@pytest.mark.parametrize("S,thr,per_sample", [(40, 260, False), (150, 260, True), (150, 5000, False), (259, 260, False)])
+def test_short_context_offload_equals_hbm(S, thr, per_sample):
+    """Sequences below the dense-attention threshold with K/V on the host: every step attends to all tokens, read from the
+    rows kept in HBM beside the host store (threshold 260: from the first refresh on, from the prompt on, prompt just
+    below the threshold; two prompts in turn in the same cache) or from the host (threshold above SHORT_ROWS_MAX).
+    Attention equals a cache that holds everything in HBM, across refreshes and the change to retrieval; the
+    kept rows are given back there; the host store holds the same rows as before."""
+    bs, Hkv, Hq, layers, steps = 2, 2, 8, 2, 150
+    sink, local, interval, topk = 4, 64, 16, 50
+    caches = [_make_cache(off, bs, Hkv, Hq, layers, S, steps + 4, sink, local, interval, topk, thr=thr) for off in (True, False)]
+    gen = torch.Generator().manual_seed(S)
+    for prompt in range(2):
+        hist = []
+        for l in range(layers):
+            k, v = (t.to(DEV) for t in _synth_kv(gen, bs, S, Hkv))
+            hist.append([k, v])
+            for c in caches:
+                if per_sample:
+                    for b in (1, 0):
+                        c.prefill_update_kv_cache(None, k[b:b + 1], v[b:b + 1], l, b)
+                else:
+                    c.prefill_update_kv_cache(None, k, v, l, 0)
+        for step in range(steps):
+            for l in range(layers):
+                k1, v1 = (t.to(DEV) for t in _synth_kv(gen, bs, 1, Hkv))
+                q = torch.randn(bs, 1, Hq, 128, generator=gen).to(torch.bfloat16).to(DEV)
+                hist[l] = [torch.cat([a, b_], dim=1) for a, b_ in zip(hist[l], (k1, v1))]
+                out = []
+                for c in caches:
+                    c.decode_update_kv_cache(k1, v1, l)
+                    out.append(c.compute(q, l).float())
+                assert (out[0] - out[1]).abs().max().item() < 2e-2, f"prompt {prompt} step {step} layer {l}"
+                short = caches[0]._short_kv[l]
+                z = caches[0]._zones[l]
+                if z.encoded > 0:
+                    assert (short is not None) == (z.seq_len < caches[0]._min_total() and thr <= 4096)
+        torch.cuda.synchronize()
+        for l in range(layers):
+            n = caches[0].cpu_valid_end[l]
+            for host, h in zip((caches[0].unified_keys_cpu[l], caches[0].unified_values_cpu[l]), hist[l]):
+                assert torch.equal(host[:, :, :n], h[:, sink:sink + n].permute(0, 2, 1, 3).cpu())
