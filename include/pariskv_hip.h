@@ -87,7 +87,8 @@ int pkv_encode_append(const void *keys, int dtype, int bs, int n_kv_heads, int64
  * 0 .. n_sink-1 and tail_row0 .. of dense_k / dense_v; the n_encode tokens
  * between them go to rows 0 .. of zone_k / zone_v and are encoded as by
  * pkv_encode_append (all outputs; cluster_counts +=).  Value norms (||v|| in
- * dtype, widened; summation order of pkv_append_kv): dense_vnorm of the dense
+ * dtype, widened; four consecutive squares left to right, then a pairwise tree
+ * over the 32 groups): dense_vnorm of the dense
  * rows by destination row, zone_vnorm (any key stride) and zone_vnorm2
  * (contiguous) of the encoded tokens; each may be NULL.  Where nib / weight are
  * the two parts of 128-byte key records (weight = nib + 64 bytes, key stride 128

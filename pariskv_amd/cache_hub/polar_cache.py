@@ -299,8 +299,9 @@ class polar_cache(KV_Cache):
             index = (self.codebook_gpu[layer_idx][b0:b1, :, :, sl], self.key_4bit_packed_gpu[layer_idx][b0:b1, :, :, sl],
                      self.key_block_weight_gpu[layer_idx][b0:b1, :, :, sl], self.cluster_key_counts_gpu[layer_idx][b0:b1])
         ranges.push("batch_encode+cluster_count")  # the reference's prefill_step1_batch_encode / prefill_step3_cluster_count
-        ops.prefill_store(k, v, n_sink, n_encode, self._srht_signs, dense, tail_row0, zone, index,
-                          **self._norm_targets(layer_idx, b0, b1, abs0, n_encode))
+        # a refresh (no dense rows) moves rows whose norms are known since they were appended: _on_refresh takes those over
+        norms = self._norm_targets(layer_idx, b0, b1, abs0, n_encode) if dense is not None else {}
+        ops.prefill_store(k, v, n_sink, n_encode, self._srht_signs, dense, tail_row0, zone, index, **norms)
         ranges.pop()
 
     # ------------------------------------------------------------- prefill

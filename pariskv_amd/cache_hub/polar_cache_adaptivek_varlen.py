@@ -96,8 +96,8 @@ class polar_cache(_polar_cache_base):
 
     # ------------------------------------------------ value-norm bookkeeping
     def _norm_targets(self, layer_idx, b0, b1, abs0, n_encode):
-        """||v||_2 per token in the cache's dtype, then widened (:680, :704-706, :753-756, :1075-1078), by the launch that
-        stores the rows: dense rows by GPU slot, the retrieval zone by absolute position."""
+        """||v||_2 per token in the cache's dtype, then widened (:680, :704-706, :753-756), by the launch that stores a
+        prompt's rows: dense rows by GPU slot, the retrieval zone by absolute position."""
         zone = self.value_norm_gpu[layer_idx][b0:b1, :, abs0:abs0 + n_encode] if n_encode > 0 else None
         return dict(dense_vnorm=self._sl_vnorm_cache[layer_idx][b0:b1], zone_vnorm=zone)
 
@@ -109,6 +109,7 @@ class polar_cache(_polar_cache_base):
     def _on_refresh(self, layer_idx, r):
         S0, n, L = self.sink_size, r.n_new, self.local_size
         sl = self._sl_vnorm_cache[layer_idx]
+        self.value_norm_gpu[layer_idx][:, :, r.encode_abs0:r.encode_abs0 + n] = sl[:, :, S0:S0 + n]  # :1075-1078
         sl[:, :, S0:S0 + L] = sl[:, :, S0 + n:S0 + n + L].clone()                                 # :1130-1133
 
     # ---------------------------------------------------------------- compute

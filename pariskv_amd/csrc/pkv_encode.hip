@@ -492,8 +492,9 @@ struct EncStore {
 constexpr int kEncDenseRows = 64;
 
 // n_rows rows of 128 elements from src (src_step bytes apart) to consecutive rows at dst, by one workgroup; norm /
-// norm2 / s_norm (may be null): the rows' 2-norms in the rows' type, summed in the order of the append kernel (squares of a
-// lane's 16 bytes left to right, then a pairwise tree over the row's lanes).
+// norm2 / s_norm (may be null): the rows' 2-norms in the rows' type: four consecutive squares left to right, then a
+// pairwise tree over the row's 32 groups, which is the order of torch.linalg.vector_norm over the last dimension (its fp32
+// bits; an order of one's own moves about one norm in a million to the neighbouring bf16 value).
 template <bool BF16>
 __device__ __forceinline__ void enc_copy_rows(const char *src, int64_t src_step, char *dst, int n_rows, float *norm,
                                               int64_t norm_step, float *norm2, float *s_norm = nullptr) {
@@ -524,8 +525,10 @@ __device__ __forceinline__ void enc_copy_rows(const char *src, int64_t src_step,
 #pragma unroll
           for (int p = 0; p < 4; ++p) e[2 * p] = __uint_as_float(w[p] << 16), e[2 * p + 1] = __uint_as_float(w[p] & 0xffff0000u);
           acc = e[0] * e[0];
+          float hi = e[4] * e[4];
 #pragma unroll
-          for (int j = 1; j < 8; ++j) acc = acc + e[j] * e[j];
+          for (int j = 1; j < 4; ++j) acc = acc + e[j] * e[j], hi = hi + e[4 + j] * e[4 + j];
+          acc = acc + hi;
         } else {
           acc = __uint_as_float(w[0]) * __uint_as_float(w[0]);
 #pragma unroll

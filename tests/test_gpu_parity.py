@@ -1660,10 +1660,9 @@ def test_offload_rows_equals_sliced_copy(ops, engine):
 @pytest.mark.parametrize("n_sink,n_enc,n_tail", [(0, 1, 0), (4, 255, 3), (64, 256, 64), (65, 2049, 129), (70, 0, 0), (3, 4097, 1)])
 def test_prefill_store_rows_index_and_norms(ops, dtype, n_sink, n_enc, n_tail):
     """pkv_prefill_store at and beside its workgroup sizes (256 encoded, 64 dense tokens): rows copied bit for bit to
-    their places and nowhere else, the index equal to pkv_encode_append's on the same keys, value norms equal to the
-    oracle's restatement."""
+    their places and nowhere else, the index equal to pkv_encode_append's on the same keys, value norms equal to a
+    restatement of their summation order."""
     bs, H, S = 2, 3, n_sink + n_enc + n_tail
-    odt = O.BF16 if dtype == torch.bfloat16 else O.F32
     _say(f"prefill_store {dtype} {n_sink}+{n_enc}+{n_tail}")
     gen = torch.Generator().manual_seed(S)
     k = torch.randn(bs, S, H, 128, generator=gen).to(dtype).to(DEV)
@@ -1684,7 +1683,11 @@ def test_prefill_store_rows_index_and_norms(ops, dtype, n_sink, n_enc, n_tail):
     ops.prefill_store(kp, vp, n_sink, n_enc, signs, (dk, dv), tail0, (zk, zv),
                       (cb[..., sl], k4[:, :, :, sl], kw[..., sl], cc) if n_enc else None, dense_vnorm=dn,
                       zone_vnorm=zn[..., sl], zone_vnorm2=zn2)
-    norm = torch.from_numpy(O.value_norm(vp.float().cpu().contiguous().view(-1, 128).numpy(), odt)).view(bs, H, S).to(DEV)
+    quads = vp.float().cpu().contiguous().view(bs, H, S, 32, 4) ** 2
+    norm = ((quads[..., 0] + quads[..., 1]) + quads[..., 2]) + quads[..., 3]
+    while norm.shape[-1] > 1:
+        norm = norm[..., 0::2] + norm[..., 1::2]
+    norm = torch.from_numpy(np.sqrt(norm[..., 0].numpy())).to(dtype).float().to(DEV)   # correctly rounded, as torch's CPU root is not
     for src, dense, zone in ((kp, dk, zk), (vp, dv, zv)):
         want_d, want_z = torch.full_like(dense, 7.0), torch.full_like(zone, 7.0)
         want_d[:, :, :n_sink], want_d[:, :, tail0:tail0 + n_tail] = src[:, :, :n_sink], src[:, :, n_sink + n_enc:]

@@ -917,3 +917,32 @@ def test_short_context_offload_equals_hbm(S, thr, per_sample):
             n = caches[0].cpu_valid_end[l]
             for host, h in zip((caches[0].unified_keys_cpu[l], caches[0].unified_values_cpu[l]), hist[l]):
                 assert torch.equal(host[:, :, :n], h[:, sink:sink + n].permute(0, 2, 1, 3).cpu())
+
+
+@pytest.mark.parametrize("form,offload", [("varlen", True), ("dense", True), ("dense", False)])
+def test_refresh_keeps_the_value_norms_of_the_rows_it_moves(form, offload):
+    """At an index refresh the moved tokens' value norms are the ones they had as dense rows, bit for bit: of the prompt's
+    rows in torch's summation order, of appended rows in the append kernel's."""
+    if form == "varlen":
+        from pariskv_amd.cache_hub.polar_cache_adaptivek_varlen import polar_cache as cls
+    else:
+        from pariskv_amd.cache_hub.polar_cache_atten_value_indices_adaptive_k import polar_cache as cls
+    bs, H, S, sink, local, interval, steps = 2, 2, 700, 4, 24, 16, 50
+    cache = cls(valid_start=[0] * bs, layer_num=1, batch_size=bs, max_length=S + steps, num_key_value_heads=H, num_heads=2 * H,
+                head_dim=128, dtype=torch.bfloat16, layer_mapping={0: DEV}, max_new_length=steps, sink_size=sink,
+                local_size=local, num_gpus=1, model_size=8, dynamic_update_interval=interval, full_attention_threshold=100,
+                enable_offload=offload)
+    gen = torch.Generator().manual_seed(5)
+    k, v = (t.to(DEV) for t in _synth_kv(gen, bs, S, H))
+    cache.prefill_update_kv_cache(None, k, v, 0, 0)
+    want = [torch.linalg.vector_norm(v, dim=-1).float().permute(0, 2, 1)]     # by absolute position
+    for step in range(steps):
+        k1, v1 = (t.to(DEV) for t in _synth_kv(gen, bs, 1, H))
+        slot = cache._zones[0].append_slot()
+        moved = cache._zones[0].next_append_refreshes()
+        cache.decode_update_kv_cache(k1, v1, 0)
+        at = slot - interval if offload and moved else slot   # the refresh slid the window
+        want.append(cache._sl_vnorm_cache[0][:, :, at:at + 1].clone())
+    n = cache._zones[0].encoded
+    assert n == S - sink - local + steps // interval * interval
+    assert torch.equal(cache.value_norm_gpu[0][:, :, sink:sink + n], torch.cat(want, dim=2)[:, :, sink:sink + n])
