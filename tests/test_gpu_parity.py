@@ -1318,6 +1318,23 @@ def test_decode_attention_indexed_segment_equals_gathered(ops, dtype, group, K):
         att.run(q, [(kk, vv, sink, K, idx.to(torch.int32))])
 
 
+@pytest.mark.parametrize("group", [3, 4, 5, 7, 8])
+def test_decode_attention_fp32_head_groups(ops, group):
+    """fp32 query heads in workgroups of four side by side: every head count around that limit, ragged rows, against the
+    oracle (fp32 sums of at most 333 keys: 1e-4, as in the segment test)."""
+    bs, H, n = 2, 2, 333
+    g = torch.Generator(device=DEV).manual_seed(group)
+    q = torch.randn(bs, 1, H * group, 128, generator=g, device=DEV) * 1.5
+    k, v = (torch.randn(bs, H, n, 128, generator=g, device=DEV) for _ in range(2))
+    row_keys = torch.tensor([[n, 1], [33, n - 1]], dtype=torch.int32, device=DEV)
+    out = ops.DecodeAttention(bs, H, group, n, DEV).run(q, [(k, v, 0, n)], row_keys=row_keys).cpu().numpy().reshape(bs, H, group, 128)
+    for b in range(bs):
+        for h in range(H):
+            rk = int(row_keys[b, h])
+            ref = O.attention(q.cpu().numpy().reshape(bs, H, group, 128)[b, h], k[b, h, :rk].cpu().numpy(), v[b, h, :rk].cpu().numpy())
+            assert np.abs(out[b, h] - ref).max() <= 1e-4, (b, h)
+
+
 def test_decode_attention_argument_errors(ops):
     att = ops.DecodeAttention(1, 2, 4, 64, DEV)
     q = torch.zeros(1, 1, 8, 128, dtype=torch.bfloat16, device=DEV)
