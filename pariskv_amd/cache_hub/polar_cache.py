@@ -180,7 +180,6 @@ class polar_cache(KV_Cache):
         max_cand = max(1, math.ceil(max_keys * 0.5))
         self._plan = ops.RetrievePlan(bs, H, self.group_size, cap, dev, max_keys, max_cand, max(1, min(final_topk, max_cand)))
         self._plan.skip_vote_counts = True  # the cache never looks at the per-key vote counts of a step
-        self._attn_k = self._attn_v = None  # no-offload mode with few rows: staging buffer of the selected rows
         self._bound = [None] * layer_num  # per layer: (n_keys, ops.BoundStep, topk, out_ids, index of the local segment)
         self._out_ids = torch.empty((bs, H, max(1, final_topk)), dtype=torch.int64, device=dev)
         self._attention = ops.DecodeAttention(bs, H, self.group_size, self.unified_kv_capacity, dev)
@@ -548,23 +547,13 @@ class polar_cache(KV_Cache):
         if not out_ids.is_contiguous():
             out_ids = torch.empty((self.batch_size, self.kv_head, topk), dtype=torch.int64, device=self.device)
         if not offload:
-            # The reference gathers sink ++ top-k ++ local rows into a new tensor (:1089-1095).  Sink and local window
-            # are always attended in place here.  The selected rows are either a segment addressed through the index
-            # list the retrieval just wrote (nothing is copied, one launch fewer) or gathered into a small buffer
-            # first: with few (batch, kv-head) rows the extra dependent index load inside the attention kernel costs
-            # more than the gather launch (65.2 vs 62.8 us per layer-step at 8 rows x 32K keys; 111.9 vs 113.2 us at
-            # 32 rows x 128K keys).
-            if self.batch_groups >= 16:
-                gather = None
-                selected = (kg, vg, self.sink_size, topk, out_ids)
-            else:
-                if self._attn_k is None or self._attn_k.shape[2] < topk:
-                    shape = (self.batch_size, self.kv_head, max(topk, self.final_topk), self.head_dim)
-                    self._attn_k = torch.zeros(shape, dtype=self.dtype, device=self.device)
-                    self._attn_v = torch.zeros(shape, dtype=self.dtype, device=self.device)
-                gather = dict(src_k=kg, src_v=vg, from_host=False, idx_offset=self.sink_size, dst_k=self._attn_k,
-                              dst_v=self._attn_v, dst_row0=0)
-                selected = (self._attn_k, self._attn_v, 0, topk)
+            # The reference gathers sink ++ top-k ++ local rows into a new tensor (:1089-1095).  Here nothing is copied:
+            # sink and local window are attended in place, the selected rows through the index list the retrieval just
+            # wrote.  A gather launch into a small buffer instead costs more than the index load at every row count
+            # (us per layer, gather / in place: 8 rows x 32K keys, top 512, 37.0 / 33.9; 2 rows x 20K, top 1024,
+            # 38.9 / 33.7; 12 rows x 9001 fp32, top 256, 47 / 38).
+            gather = None
+            selected = (kg, vg, self.sink_size, topk, out_ids)
             segments = [(kg, vg, 0, self.sink_size), selected, (kg, vg, z.local_start, z.dense_tail_len)]
             segments = [s for s in segments if s[3] > 0]
             local_seg = len(segments) - 1
