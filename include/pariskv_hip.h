@@ -638,7 +638,7 @@ int pkv_decode_step(const pkv_retrieve_args *retrieve, void *ws, size_t ws_bytes
  * pkv_decode_attention with row_keys = row_keys_base + k.  Every field has the
  * meaning of the same-named argument of those entry points. */
 typedef struct pkv_adaptive_args {
-  const void *dense_k;            /* GPU K store; rows 0 .. dense_rows-1 of each (b, h) are the dense tokens */
+  const void *dense_k;            /* GPU K store; rows 0 .. dense_rows-1 of each (b, h) are the dense tokens (see dense_split) */
   int64_t dense_stride_b, dense_stride_h;  /* elements */
   int64_t dense_rows;
   const float *dense_vnorm;       /* [bs*n_kv_heads][dense_vnorm_stride] */
@@ -658,11 +658,15 @@ typedef struct pkv_adaptive_args {
                                      gather and row_keys use max(adaptive_k) for every row (the dense form) */
   void *ws;                       /* pkv_adaptive_topk_ws_bytes(rows, n_cand, k_out) */
   size_t ws_bytes;
-  const void *src_k, *src_v;      /* pinned host K/V stores [bs][h][src_len] rows */
+  const void *src_k, *src_v;      /* pinned host K/V stores [bs][h][src_len] rows; src_k NULL: no gather, the attention's
+                                     segments name the selected rows by topk_ids */
   int64_t src_len, idx_offset;
   void *dst_k, *dst_v;            /* GPU [bs][h][dst_len] rows; row (b, h) receives its k rows from dst_row0 on */
   int64_t dst_len, dst_row0;
   int row_bytes;
+  int64_t dense_split, dense_row1; /* with dense_vnorm_run: dense tokens from dense_split on are rows dense_row1, .. of
+                                     dense_k and dense_vnorm (sink and local rows at absolute positions) */
+  float *dense_vnorm_run;         /* NULL, or scratch [bs*n_kv_heads][dense_logits_stride]: the dense tokens' norms side by side */
 } pkv_adaptive_args;
 
 int pkv_adaptive_decode_step(const pkv_retrieve_args *retrieve, void *ws, size_t ws_bytes,

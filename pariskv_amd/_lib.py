@@ -75,6 +75,7 @@ class AdaptiveArgs(C.Structure):
         ("uniform_k", _vp), ("ws", _vp), ("ws_bytes", _sz),
         ("src_k", _vp), ("src_v", _vp), ("src_len", _i64), ("idx_offset", _i64),
         ("dst_k", _vp), ("dst_v", _vp), ("dst_len", _i64), ("dst_row0", _i64), ("row_bytes", _i),
+        ("dense_split", _i64), ("dense_row1", _i64), ("dense_vnorm_run", _vp),
     ]
 
 

@@ -555,8 +555,7 @@ class polar_cache(KV_Cache):
             gather = None
             selected = (kg, vg, self.sink_size, topk, out_ids)
             segments = [(kg, vg, 0, self.sink_size), selected, (kg, vg, z.local_start, z.dense_tail_len)]
-            segments = [s for s in segments if s[3] > 0]
-            local_seg = len(segments) - 1
+            local_seg = 2  # empty where the window is, until a token is appended
         bound = self._plan.bind(q, self._srht_signs, self._mag_centers, self.cluster_key_counts_gpu[layer_idx],
                                 self._codes_km[layer_idx], self._nib_km[layer_idx], self._w_km[layer_idx], self.sink_size,
                                 n_keys, tiers, n_cand, topk, out_ids, gather, self._attention, segments, any_order=True)

@@ -71,12 +71,14 @@ class polar_cache(_polar_cache_base):
         # norm is in the HBM line the rerank fetches anyway (the reference keeps a separate [bs,H,cap] tensor)
         self.value_norm_gpu = [ops.record_value_norm_view(self._nib_km[l]) for l in range(layer_num)]
         cap = max(1, buffer_cap)
-        self._dense_logits = torch.empty((bs, H, self.gpu_kv_capacity), dtype=torch.float32, device=dev)
+        dense_cap = min(self.gpu_kv_capacity, self.sink_size + self.local_size + self.dynamic_update_interval)
+        self._dense_logits = torch.empty((bs, H, dense_cap), dtype=torch.float32, device=dev)
         self._adaptive_k = torch.zeros((bs, H), dtype=torch.int64, device=dev)
         self._uniform_k = torch.zeros((bs, H), dtype=torch.int64, device=dev) if uniform_k else None
         self._topk_ids = torch.zeros((bs * H * cap,), dtype=torch.int64, device=dev)
         self._row_keys = torch.zeros((bs, H), dtype=torch.int32, device=dev)
         self._adk_ws = None
+        self._dense_vnorm_run = None  # HBM form: the dense tokens' norms side by side
         self._adaptive_bound = [None] * layer_num  # per layer: (n_keys, ops.BoundAdaptiveStep, topk_cap)
         self.last_adaptive_k = None  # [bs, H] int64 of the most recent retrieval step
         if self.enable_offload:

@@ -19,7 +19,7 @@ from __future__ import annotations
 
 import torch
 
-from .. import ops
+from .. import ops, ranges
 from .polar_cache import polar_cache as _polar_cache_base
 from .polar_cache_adaptivek_varlen import polar_cache as _adaptive_base
 
@@ -82,29 +82,49 @@ class polar_cache(_adaptive_base):
         if total < self._min_total() or n_keys <= 0:
             return _polar_cache_base.compute(self, queries, layer_idx)  # dense branch
         q = queries if queries.is_contiguous() else queries.contiguous()
-        bs, H, S0 = self.batch_size, self.kv_head, self.sink_size
+        step = self._adaptive_bound[layer_idx]
+        if step is None or step[0] != n_keys:
+            step = self._bind_adaptive_step(layer_idx, q, n_keys)
+        _, bound, local_seg = step
+        # what moves with every token: the local window grows by one; k goes to a tensor of its own, as the caller may keep it
+        dense = z.gpu_prefix_rows
+        bound.ad.dense_rows = bound.ad.row_keys_base = dense
+        bound.segs[local_seg].n_rows = z.dense_tail_len
+        self.last_adaptive_k = torch.empty_like(self._adaptive_k)
+        bound.ad.adaptive_k = self.last_adaptive_k.data_ptr()
+        # one host call, as in the offloading form; the dense rows (two runs: sink, local) and the selected ones are read
+        # where they lie
+        if ranges.enabled:
+            with ranges.span("collision_topk+adaptive_k+attention_varlen"):
+                return bound.launch(q)
+        return bound.launch(q)
+
+    def _bind_adaptive_step(self, layer_idx, q, n_keys):
+        if self.enable_offload:
+            return super()._bind_adaptive_step(layer_idx, q, n_keys)
+        z, S0 = self._zones[layer_idx], self.sink_size
         n_keys, n_cand, _, tiers = self.retrieval_shape(layer_idx)
-        cand, scores = self._plan.run_candidates(q, self._srht_signs, self._mag_centers, self.cluster_key_counts_gpu[layer_idx],
-                                                 self._codes_km[layer_idx], self._nib_km[layer_idx], self._w_km[layer_idx],
-                                                 S0, n_keys, tiers, n_cand)
-        kg, vg = self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx]
-        local0, local_len = z.local_start, z.dense_tail_len
-        sl = S0 + local_len
-        # dense tokens = sink rows ++ local rows, where they lie (:1421-1434 index_selects copies of them)
-        logits = self._dense_logits[:, :, :sl]
-        ops.dense_logits(q, kg, S0, self._attn_scale, out=logits)
-        if local_len > 0:
-            ops.dense_logits(q, kg[:, :, local0:], local_len, self._attn_scale, out=logits[:, :, S0:])
-        norms = self._sl_vnorm_cache[layer_idx]
-        sl_vnorm = torch.cat([norms[:, :, :S0], norms[:, :, local0:local0 + local_len]], dim=2)
         topk_cap, k_min, k_max = self._caps(n_cand)
-        adaptive_k, topk_ids = ops.adaptive_topk(logits, sl_vnorm, scores, self._attn_scale, cand,
-                                                 float(self.adaptive_topk_threshold), topk_cap,
-                                                 value_norm=self.value_norm_gpu[layer_idx], vn_offset=S0, k_min=k_min,
-                                                 k_max=k_max)
-        self.last_adaptive_k = adaptive_k
-        _, row_keys = ops.uniform_k(adaptive_k, row_keys_base=sl)
-        # the selected rows are read in place through the index list (the reference gathers copies, :1481-1488); they
-        # come last so that the per-row key count cuts inside them
-        segments = [(kg, vg, 0, S0), (kg, vg, local0, local_len), (kg, vg, S0, topk_cap, topk_ids)]
-        return self._attention.run(q, [s for s in segments if s[3] > 0], row_keys=row_keys)
+        kg, vg = self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx]
+        bs, H = self.batch_size, self.kv_head
+        need = ops.adaptive_topk_ws_bytes(self.batch_groups, n_cand, topk_cap)
+        if self._adk_ws is None or self._adk_ws.numel() < need:
+            self._adk_ws = torch.empty(need, dtype=torch.uint8, device=self.device)
+        if self._dense_vnorm_run is None:
+            self._dense_vnorm_run = torch.empty_like(self._dense_logits)
+        local0, dense = z.local_start, z.gpu_prefix_rows
+        adaptive = dict(dense_k=kg, dense_rows=dense, dense_split=S0, dense_row1=local0, dense_vnorm=self._sl_vnorm_cache[layer_idx],
+                        dense_vnorm_run=self._dense_vnorm_run, dense_logits=self._dense_logits, scale=self._attn_scale,
+                        value_norm=self.value_norm_gpu[layer_idx], vn_offset=S0, record_word_offset=ops.RECORD_VALUE_NORM_OFFSET,
+                        threshold=self.adaptive_topk_threshold, k_out=topk_cap, k_min=k_min, k_max=k_max,
+                        adaptive_k=self._adaptive_k, topk_ids=self._topk_ids, row_keys=self._row_keys, row_keys_base=dense,
+                        uniform_k=self._uniform_k, ws=self._adk_ws, src_k=None, src_v=None, dst_k=None, dst_v=None)
+        ids = self._topk_ids[:bs * H * topk_cap].view(bs, H, topk_cap)
+        # the selected rows come last so that the per-row key count cuts inside them (the reference gathers copies, :1481-1488)
+        segments = [(kg, vg, 0, S0), (kg, vg, local0, z.dense_tail_len), (kg, vg, S0, topk_cap, ids)]  # runs may be empty
+        bound = self._plan.bind_adaptive(q, self._srht_signs, self._mag_centers, self.cluster_key_counts_gpu[layer_idx],
+                                         self._codes_km[layer_idx], self._nib_km[layer_idx], self._w_km[layer_idx], S0,
+                                         n_keys, tiers, n_cand, adaptive, self._attention, segments)
+        step = (n_keys, bound, 1)
+        self._adaptive_bound[layer_idx] = step
+        return step

@@ -73,11 +73,31 @@ static inline int pkv_pick_chunk_keys(int rows, int64_t n_keys) {
 // Internal launchers shared between translation units (not exported).
 #define PKV_INTERNAL __attribute__((visibility("hidden")))
 
+// Dense (sink / local / buffer) tokens of the adaptive-k step: token i of row (b, h) is row i of k for i < split and row
+// i + shift from there on (split = n_rows: one run).  vn_out (or null): the tokens' value norms, taken from vn_in by the
+// same row numbers, side by side.
+struct PkvDenseLogits {
+  const void *k;
+  int64_t k_stride_b, k_stride_h, n_rows, split, shift;
+  float scale;
+  float *out;
+  int64_t out_stride;
+  const float *vn_in;
+  int64_t vn_in_stride;
+  float *vn_out;
+};
+constexpr int kDenseLogitThreads = 256;
+constexpr int kDenseLogitRows = kDenseLogitThreads / 16;  // tokens per workgroup
+
+PKV_INTERNAL int pkv_launch_dense_logits(const void *q, int dtype, int bs, int n_kv_heads, int group, const PkvDenseLogits &d,
+                                         hipStream_t s);
+
 PKV_INTERNAL int pkv_launch_query_prep_lut(const void *q, int dtype, int bs, int n_kv_heads, int group,
                                            const float *signs, const int32_t *cc, int64_t cc_b, int64_t cc_h,
                                            const PkvTiers &tiers, float *qhat, float *qnorm, uint8_t *lut,
                                            int64_t *sorted_ids, uint32_t *row_suf_to_zero, hipStream_t s,
-                                           uint32_t *zero_ptr = nullptr, int64_t zero_words = 0);
+                                           uint32_t *zero_ptr = nullptr, int64_t zero_words = 0,
+                                           const PkvDenseLogits *dense = nullptr);
 PKV_INTERNAL int pkv_launch_scan(const uint8_t *codes, int64_t cs_b, int64_t cs_h, int64_t cs_key, int64_t cs_sub,
                                  int bs, int n_kv_heads, int64_t n_keys, const uint8_t *lut, uint8_t *cnt_u8,
                                  int64_t cnt_u8_stride, int32_t *cnt_i32, uint32_t *row_suf, uint16_t *chunk_suf,
@@ -298,6 +318,52 @@ __device__ __forceinline__ void pkv_query_group_mean_t(const void *__restrict__ 
 #pragma unroll
     for (int j = 0; j < 8; ++j) x[j] = pkv_rdt(acc[j] / (float)group, dtype);
   }
+}
+
+// Logits of kDenseLogitRows dense tokens (workgroup `part` of row bh) against the group-mean query
+// (polar_cache_adaptivek_varlen.py:1418-1419, :1731): out[bh][i] = dtype(mean_g q . K[i]) widened to fp32, times scale.
+// 16 lanes per key row, 8 dims per lane: a lane adds its 8 products in order, the 16 partial sums meet in a pairwise
+// tree (lane ^ 1, 2, 4, 8).  kDenseLogitThreads threads.
+template <bool BF16>
+__device__ __forceinline__ void pkv_dense_logits_rows(const void *__restrict__ q, int n_kv_heads, int group,
+                                                      const PkvDenseLogits &d, int part, int bh) {
+  const int b = bh / n_kv_heads, h = bh % n_kv_heads;
+  const int s = threadIdx.x & 15;
+  const int64_t i = (int64_t)part * kDenseLogitRows + (threadIdx.x >> 4);
+  const int64_t ii = i < d.n_rows ? i : d.n_rows - 1;
+  const int64_t row = ii < d.split ? ii : ii + d.shift;
+  const int64_t at = (int64_t)b * d.k_stride_b + (int64_t)h * d.k_stride_h + row * 128 + 8 * s;
+  pkv_u32x4 lo, hi = {0u, 0u, 0u, 0u};
+  if (BF16) {
+    lo = *(const pkv_u32x4 *)((const uint16_t *)d.k + at);
+  } else {
+    lo = *(const pkv_u32x4 *)((const float *)d.k + at);
+    hi = *(const pkv_u32x4 *)((const float *)d.k + at + 4);
+  }
+  if (d.vn_out && s == 0 && i < d.n_rows) d.vn_out[(int64_t)bh * d.out_stride + i] = d.vn_in[(int64_t)bh * d.vn_in_stride + row];
+  float qa[8];
+  pkv_query_group_mean_t<BF16>(q, b, h, n_kv_heads, group, qa);
+  float kv[8];
+  if (BF16) {
+    const uint32_t ww[4] = {lo.x, lo.y, lo.z, lo.w};
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      kv[2 * p] = __uint_as_float(ww[p] << 16);
+      kv[2 * p + 1] = __uint_as_float(ww[p] & 0xffff0000u);
+    }
+  } else {
+    kv[0] = __uint_as_float(lo.x), kv[1] = __uint_as_float(lo.y), kv[2] = __uint_as_float(lo.z), kv[3] = __uint_as_float(lo.w);
+    kv[4] = __uint_as_float(hi.x), kv[5] = __uint_as_float(hi.y), kv[6] = __uint_as_float(hi.z), kv[7] = __uint_as_float(hi.w);
+  }
+  float acc = qa[0] * kv[0];
+#pragma unroll
+  for (int j = 1; j < 8; ++j) acc = acc + qa[j] * kv[j];
+  acc = acc + pkv_lane_xor_f<1>(acc);
+  acc = acc + pkv_lane_xor_f<2>(acc);
+  acc = acc + pkv_lane_xor_f<4>(acc);
+  acc = acc + pkv_lane_xor_f<8>(acc);
+  if (s == 0 && i < d.n_rows)
+    d.out[(int64_t)bh * d.out_stride + i] = pkv_rdt(acc, BF16 ? PKV_DTYPE_BF16 : PKV_DTYPE_F32) * d.scale;
 }
 
 // The normalisation and rotation of pkv_normalize_rotate_16 with the 128-vector spread over the 64 lanes of ONE wave: lane l holds dims

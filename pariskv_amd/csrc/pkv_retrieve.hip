@@ -118,7 +118,8 @@ extern "C" int pkv_retrieve_ws_view(void *ws, int rows, int64_t n_keys, int64_t 
   return PKV_OK;
 }
 
-static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, void *stream) {
+// dense (or null): the adaptive-k step's dense tokens, whose logits ride with the query prep where that is a launch of its own
+static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, void *stream, const PkvDenseLogits *dense = nullptr) {
   PKV_REQUIRE(a != nullptr, "pkv_retrieve: null args");
   PKV_REQUIRE(a->q && a->signs && a->centers && a->cluster_counts && a->codes && a->nib && a->weight,
               "pkv_retrieve: null pointer");
@@ -191,8 +192,9 @@ static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, 
     rc = a->table_ready ? PKV_OK
                         : pkv_launch_query_prep_lut(a->q, a->dtype, a->bs, H, a->group, a->signs, a->cluster_counts,
                                                     (int64_t)H * 4096, 4096, t, qhat, qnorm, lut, nullptr, rowsuf, s, topk_ctl,
-                                                    ctl_words);
+                                                    ctl_words, dense);
     if (rc) return rc;
+    if (!a->table_ready) dense = nullptr;  // done
     if (a->n_cand == a->n_keys) {
       rc = pkv_launch_identity_fill(cand, a->n_keys, a->n_cand, rows, s);
       if (rc) return rc;
@@ -211,6 +213,10 @@ static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, 
     }
   }
   if (rc) return rc;
+  if (dense) {
+    rc = pkv_launch_dense_logits(a->q, a->dtype, a->bs, H, a->group, *dense, s);
+    if (rc) return rc;
+  }
   if (!a->out_ids) return PKV_OK;  // candidates only: the caller reads them out of the workspace
   rc = pkv_launch_topk_f32(scores, a->n_cand, cand, a->n_cand, rows, a->n_cand, a->k, a->out_ids, a->out_scores,
                            (char *)ws + w.topk, w.topk_bytes, s, a->any_order != 0, topk_ctl != nullptr);
@@ -356,7 +362,20 @@ extern "C" int pkv_adaptive_decode_step(const pkv_retrieve_args *retrieve, void 
   PKV_REQUIRE(ad->dense_rows > 0 && ad->dense_rows <= ad->dense_vnorm_stride && ad->dense_rows <= ad->dense_logits_stride,
               "pkv_adaptive_decode_step: %lld dense rows exceed the norm / logit rows (%lld, %lld)",
               (long long)ad->dense_rows, (long long)ad->dense_vnorm_stride, (long long)ad->dense_logits_stride);
-  int rc = pkv_retrieve(retrieve, ws, ws_bytes, stream);
+  PKV_REQUIRE(ad->dense_k && ad->dense_logits && ad->dense_vnorm && pkv_aligned(ad->dense_k, 16) && ad->dense_stride_b % 8 == 0 &&
+                  ad->dense_stride_h % 8 == 0,
+              "pkv_adaptive_decode_step: the dense rows must be 16-byte aligned");
+  // the dense tokens: one run of rows, or two (sink rows, then local rows further on) with their norms brought together
+  const bool two_runs = ad->dense_vnorm_run && ad->dense_split < ad->dense_rows;
+  PKV_REQUIRE(!two_runs || (ad->dense_split >= 0 && ad->dense_row1 >= ad->dense_split &&
+                            ad->dense_row1 + (ad->dense_rows - ad->dense_split) <= ad->dense_vnorm_stride),
+              "pkv_adaptive_decode_step: second run of dense rows [%lld, +%lld) outside the norm rows (%lld)",
+              (long long)ad->dense_row1, (long long)(ad->dense_rows - ad->dense_split), (long long)ad->dense_vnorm_stride);
+  const PkvDenseLogits dense{ad->dense_k, ad->dense_stride_b, ad->dense_stride_h, ad->dense_rows,
+                             two_runs ? ad->dense_split : ad->dense_rows, two_runs ? ad->dense_row1 - ad->dense_split : 0, ad->scale,
+                             ad->dense_logits, ad->dense_logits_stride, ad->dense_vnorm, ad->dense_vnorm_stride,
+                             two_runs ? ad->dense_vnorm_run : nullptr};
+  int rc = retrieve_impl(retrieve, ws, ws_bytes, stream, &dense);
   if (rc) return rc;
   const int rows = retrieve->bs * retrieve->n_kv_heads;
   const WsLayout w = layout(rows, retrieve->n_keys, retrieve->n_cand, retrieve->k);
@@ -366,11 +385,8 @@ extern "C" int pkv_adaptive_decode_step(const pkv_retrieve_args *retrieve, void 
   // records (not on the all-keys-are-candidates path, which reranks without the fused kernel)
   const bool norms_emitted = retrieve->record_word_offset > 0 && retrieve->n_cand != retrieve->n_keys;
   const float *cand_vnorm = norms_emitted ? (const float *)((char *)ws + w.cand_extra) : nullptr;
-  rc = pkv_dense_logits(retrieve->q, retrieve->dtype, retrieve->bs, retrieve->n_kv_heads, retrieve->group, ad->dense_k,
-                        ad->dense_stride_b, ad->dense_stride_h, ad->dense_rows, ad->scale, ad->dense_logits,
-                        ad->dense_logits_stride, stream);
-  if (rc) return rc;
-  rc = pkv_adaptive_topk(ad->dense_logits, ad->dense_logits_stride, ad->dense_vnorm, ad->dense_vnorm_stride,
+  rc = pkv_adaptive_topk(ad->dense_logits, ad->dense_logits_stride, two_runs ? ad->dense_vnorm_run : ad->dense_vnorm,
+                         two_runs ? ad->dense_logits_stride : ad->dense_vnorm_stride,
                          ad->dense_rows, scores, PKV_DTYPE_F32, ad->scale, cand_vnorm, ad->value_norm, ad->vn_stride,
                          ad->vn_offset, ad->vn_pos_stride, cand, retrieve->n_cand, ad->threshold, ad->k_out, rows, ad->adaptive_k,
                          ad->topk_ids, ad->k_min, ad->k_max, ad->row_keys, ad->row_keys_base, ad->ws, ad->ws_bytes, stream);
@@ -379,11 +395,13 @@ extern "C" int pkv_adaptive_decode_step(const pkv_retrieve_args *retrieve, void 
     rc = pkv_uniform_k(ad->adaptive_k, rows, ad->uniform_k, ad->row_keys, ad->row_keys_base, stream);
     if (rc) return rc;
   }
-  rc = pkv_gather_uva_ragged(ad->src_k, ad->src_v, ad->src_len, ad->topk_ids, ad->k_out,
-                             ad->uniform_k ? ad->uniform_k : ad->adaptive_k, ad->idx_offset,
-                             ad->dst_k, ad->dst_v, ad->dst_len, ad->dst_row0, retrieve->bs, retrieve->n_kv_heads,
-                             ad->row_bytes, stream);
-  if (rc) return rc;
+  if (ad->src_k) {  // else: the attention reads the selected rows where they lie, through topk_ids
+    rc = pkv_gather_uva_ragged(ad->src_k, ad->src_v, ad->src_len, ad->topk_ids, ad->k_out,
+                               ad->uniform_k ? ad->uniform_k : ad->adaptive_k, ad->idx_offset,
+                               ad->dst_k, ad->dst_v, ad->dst_len, ad->dst_row0, retrieve->bs, retrieve->n_kv_heads,
+                               ad->row_bytes, stream);
+    if (rc) return rc;
+  }
   return pkv_decode_attention(retrieve->q, retrieve->dtype, retrieve->bs, retrieve->n_kv_heads, retrieve->group,
                               attention->segments, attention->n_segments, attention->row_keys, attention->scale,
                               attention->out, attention->ws, attention->ws_bytes, stream);

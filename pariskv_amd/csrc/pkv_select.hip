@@ -2099,45 +2099,11 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_uniform_k_kernel(const int64
   }
 }
 
-// Logits of the dense (sink / local / buffer) rows against the group-mean query
-// (polar_cache_adaptivek_varlen.py:1418-1419, :1731): out[(b,h)][r] = dtype(mean_g q . K[r]) widened to fp32,
-// times scale.  16 lanes per key row, 8 dims per lane: a lane adds its 8 products in order, the 16 partial
-// sums meet in a pairwise tree (lane ^ 1, 2, 4, 8).  grid (ceil(n_rows / 16), bs * H) x 256 threads.
-constexpr int kDenseLogitThreads = 256;
-
+// Logits of the dense tokens on their own: grid (ceil(n_rows / kDenseLogitRows), bs * H).
 template <bool BF16>
-__global__ __launch_bounds__(kDenseLogitThreads) void pkv_dense_logits_kernel(
-    const void *__restrict__ q, int n_kv_heads, int group, const void *__restrict__ k, int64_t k_stride_b,
-    int64_t k_stride_h, int64_t n_rows, float scale, float *__restrict__ out, int64_t out_stride) {
-  const int bh = blockIdx.y, b = bh / n_kv_heads, h = bh % n_kv_heads;
-  const int s = threadIdx.x & 15;
-  const int64_t row = (int64_t)blockIdx.x * (kDenseLogitThreads / 16) + (threadIdx.x >> 4);
-  float qa[8];
-  pkv_query_group_mean_t<BF16>(q, b, h, n_kv_heads, group, qa);
-  const int64_t r = row < n_rows ? row : n_rows - 1;
-  const int64_t at = (int64_t)b * k_stride_b + (int64_t)h * k_stride_h + r * 128 + 8 * s;
-  float kv[8];
-  if (BF16) {
-    const pkv_u32x4 w = *(const pkv_u32x4 *)((const uint16_t *)k + at);
-    const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      kv[2 * p] = __uint_as_float(ww[p] << 16);
-      kv[2 * p + 1] = __uint_as_float(ww[p] & 0xffff0000u);
-    }
-  } else {
-    const float4 lo = *(const float4 *)((const float *)k + at), hi = *(const float4 *)((const float *)k + at + 4);
-    kv[0] = lo.x, kv[1] = lo.y, kv[2] = lo.z, kv[3] = lo.w, kv[4] = hi.x, kv[5] = hi.y, kv[6] = hi.z, kv[7] = hi.w;
-  }
-  float acc = qa[0] * kv[0];
-#pragma unroll
-  for (int j = 1; j < 8; ++j) acc = acc + qa[j] * kv[j];
-  acc = acc + pkv_lane_xor_f<1>(acc);
-  acc = acc + pkv_lane_xor_f<2>(acc);
-  acc = acc + pkv_lane_xor_f<4>(acc);
-  acc = acc + pkv_lane_xor_f<8>(acc);
-  if (s == 0 && row < n_rows)
-    out[(int64_t)bh * out_stride + row] = pkv_rdt(acc, BF16 ? PKV_DTYPE_BF16 : PKV_DTYPE_F32) * scale;
+__global__ __launch_bounds__(kDenseLogitThreads) void pkv_dense_logits_kernel(const void *__restrict__ q, int n_kv_heads, int group,
+                                                                             PkvDenseLogits d) {
+  pkv_dense_logits_rows<BF16>(q, n_kv_heads, group, d, blockIdx.x, blockIdx.y);
 }
 
 static size_t lds_bytes(int P) { return (size_t)(P < 1024 ? 1024 : P) * 8; }
@@ -2478,14 +2444,16 @@ extern "C" int pkv_dense_logits(const void *q, int dtype, int bs, int n_kv_heads
               "pkv_dense_logits: bad shape bs=%d heads=%d group=%d rows=%lld", bs, n_kv_heads, group, (long long)n_rows);
   PKV_REQUIRE(k_stride_b % 8 == 0 && k_stride_h % 8 == 0 && pkv_aligned(q, 16) && pkv_aligned(k, 16),
               "pkv_dense_logits: rows must be 16-byte aligned");
-  constexpr int rows_per_wg = kDenseLogitThreads / 16;
-  const dim3 grid((unsigned)((n_rows + rows_per_wg - 1) / rows_per_wg), (unsigned)(bs * n_kv_heads));
+  const PkvDenseLogits d{k, k_stride_b, k_stride_h, n_rows, n_rows, 0, scale, out, out_stride, nullptr, 0, nullptr};
+  return pkv_launch_dense_logits(q, dtype, bs, n_kv_heads, group, d, (hipStream_t)stream);
+}
+
+int pkv_launch_dense_logits(const void *q, int dtype, int bs, int n_kv_heads, int group, const PkvDenseLogits &d, hipStream_t s) {
+  const dim3 grid((unsigned)((d.n_rows + kDenseLogitRows - 1) / kDenseLogitRows), (unsigned)(bs * n_kv_heads));
   if (dtype == PKV_DTYPE_BF16)
-    hipLaunchKernelGGL(pkv_dense_logits_kernel<true>, grid, dim3(kDenseLogitThreads), 0, (hipStream_t)stream, q,
-                       n_kv_heads, group, k, k_stride_b, k_stride_h, n_rows, scale, out, out_stride);
+    hipLaunchKernelGGL(pkv_dense_logits_kernel<true>, grid, dim3(kDenseLogitThreads), 0, s, q, n_kv_heads, group, d);
   else
-    hipLaunchKernelGGL(pkv_dense_logits_kernel<false>, grid, dim3(kDenseLogitThreads), 0, (hipStream_t)stream, q,
-                       n_kv_heads, group, k, k_stride_b, k_stride_h, n_rows, scale, out, out_stride);
+    hipLaunchKernelGGL(pkv_dense_logits_kernel<false>, grid, dim3(kDenseLogitThreads), 0, s, q, n_kv_heads, group, d);
   PKV_LAUNCH_CHECK("pkv_dense_logits_kernel");
   return PKV_OK;
 }

@@ -972,7 +972,9 @@ class RetrievePlan:
         rerank then hands the candidates' norms over and no second gather runs), vn_offset, threshold, k_out, k_min, k_max, adaptive_k int64 [bs,H], topk_ids int64 (>= bs*H*k_out
         elements), row_keys int32 [bs,H], row_keys_base, optional uniform_k int64 [bs,H] (then every row gathers and
         attends to max(adaptive_k) ids), ws uint8 (pkv_adaptive_topk_ws_bytes), src_k / src_v pinned
-        CPU [bs,H,len,128], dst_k / dst_v GPU [bs,H,>=k_out,128].  ``segments`` are the attention's; its per-row key
+        CPU [bs,H,len,128], dst_k / dst_v GPU [bs,H,>=k_out,128] (all four None: no gather, ``segments`` name the selected
+        rows by topk_ids); optional dense_vnorm_run (like dense_logits) with dense_split and dense_row1: dense tokens from
+        dense_split on are the rows from dense_row1 on.  ``segments`` are the attention's; its per-row key
         count is ``row_keys``."""
         d = adaptive
         a = self._fill(queries, signs, centers, cluster_counts, codes_km, nib_km, w_km, key0, n_keys, tier_counts, n_cand, 1,
@@ -1003,11 +1005,12 @@ class RetrievePlan:
               rk.numel() == bs * H, "adaptive_k / topk_ids / row_keys: contiguous int64 / int64 / int32 of the step's size")
         need = _lib.lib().pkv_adaptive_topk_ws_bytes(self.rows, n_cand, k_out)
         _need(ws.dtype == torch.uint8 and ws.is_contiguous() and ws.numel() >= need, "adaptive workspace too small")
-        _need(sk.is_cpu and sv.is_cpu and sk.is_pinned() and sv.is_pinned() and sk.is_contiguous() and sv.is_contiguous() and
-              sk.shape == sv.shape and tuple(sk.shape[:2]) == (bs, H) and sk.dtype == queries.dtype,
+        _need((sk is None) == (tk is None), "src and dst of the gather come together")
+        _need(sk is None or (sk.is_cpu and sv.is_cpu and sk.is_pinned() and sv.is_pinned() and sk.is_contiguous() and sv.is_contiguous() and
+              sk.shape == sv.shape and tuple(sk.shape[:2]) == (bs, H) and sk.dtype == queries.dtype),
               "src_k / src_v: contiguous pinned CPU [bs,H,len,128] of the query dtype")
-        _need(tk.is_contiguous() and tv.is_contiguous() and tk.shape == tv.shape and tuple(tk.shape[:2]) == (bs, H) and
-              tk.shape[2] >= k_out and tk.dtype == queries.dtype, "dst_k / dst_v: contiguous GPU [bs,H,>=k_out,128]")
+        _need(tk is None or (tk.is_contiguous() and tv.is_contiguous() and tk.shape == tv.shape and tuple(tk.shape[:2]) == (bs, H) and
+              tk.shape[2] >= k_out and tk.dtype == queries.dtype), "dst_k / dst_v: contiguous GPU [bs,H,>=k_out,128]")
         ad = _lib.AdaptiveArgs()
         ad.dense_k, ad.dense_stride_b, ad.dense_stride_h, ad.dense_rows = dk.data_ptr(), dk.stride(0), dk.stride(1), int(d["dense_rows"])
         ad.dense_vnorm, ad.dense_vnorm_stride = dvn.data_ptr(), dvn.shape[2]
@@ -1022,9 +1025,17 @@ class RetrievePlan:
             _need(uk.dtype == torch.int64 and uk.is_contiguous() and uk.numel() == bs * H, "uniform_k: contiguous int64 [bs,H]")
             ad.uniform_k = uk.data_ptr()
         ad.ws, ad.ws_bytes = ws.data_ptr(), ws.numel()
-        ad.src_k, ad.src_v, ad.src_len, ad.idx_offset = sk.data_ptr(), sv.data_ptr(), sk.shape[2], int(d.get("idx_offset", 0))
-        ad.dst_k, ad.dst_v, ad.dst_len, ad.dst_row0 = tk.data_ptr(), tv.data_ptr(), tk.shape[2], 0
-        ad.row_bytes = HEAD_DIM * sk.element_size()
+        if sk is not None:
+            ad.src_k, ad.src_v, ad.src_len, ad.idx_offset = sk.data_ptr(), sv.data_ptr(), sk.shape[2], int(d.get("idx_offset", 0))
+            ad.dst_k, ad.dst_v, ad.dst_len, ad.dst_row0 = tk.data_ptr(), tv.data_ptr(), tk.shape[2], 0
+            ad.row_bytes = HEAD_DIM * sk.element_size()
+        split, row1, run = int(d.get("dense_split", 0)), int(d.get("dense_row1", 0)), d.get("dense_vnorm_run")
+        if run is not None:
+            _cuda(run)
+            _need(run.dtype == torch.float32 and run.is_contiguous() and run.shape == dl.shape, "dense_vnorm_run: like dense_logits")
+            _need(0 <= split <= row1 and row1 + int(d["dense_rows"]) - split <= min(dvn.shape[2], dk.shape[2]),
+                  "the second run of dense rows exceeds dense_k / dense_vnorm")
+            ad.dense_split, ad.dense_row1, ad.dense_vnorm_run = split, row1, run.data_ptr()
         aa, _ = att.c_args(queries, segments, out=queries, row_keys=rk)  # out is patched at every launch
         keep = (signs, centers, cluster_counts, codes_km, nib_km, w_km, d, att, segments, self.ws)
         return BoundAdaptiveStep(self, a, ad, aa, keep, queries)

@@ -946,3 +946,50 @@ def test_refresh_keeps_the_value_norms_of_the_rows_it_moves(form, offload):
     n = cache._zones[0].encoded
     assert n == S - sink - local + steps // interval * interval
     assert torch.equal(cache.value_norm_gpu[0][:, :, sink:sink + n], torch.cat(want, dim=2)[:, :, sink:sink + n])
+
+
+@pytest.mark.parametrize("sink,S,dtype,bs,group", [(0, 700, torch.bfloat16, 1, 4), (3, 1513, torch.float32, 2, 5),
+                                                   (64, 2600, torch.bfloat16, 2, 1)])
+def test_dense_adaptive_step_with_two_runs_of_dense_rows(sink, S, dtype, bs, group):
+    """K/V in HBM: sink and local rows are two runs of the store, and their logits ride with the query prep.  Logits, k and
+    ids equal the stand-alone operators' on copies of the rows side by side, from an empty update buffer to a full one."""
+    from pariskv_amd import ops
+    from pariskv_amd.cache_hub.polar_cache_atten_value_indices_adaptive_k import polar_cache as dense_adaptive_cache
+
+    H, local, I, steps = 2, 33, 16, 20
+    cache = dense_adaptive_cache(valid_start=[0] * bs, layer_num=1, batch_size=bs, max_length=S + steps + 2,
+                                 num_key_value_heads=H, num_heads=H * group, head_dim=128, dtype=dtype, layer_mapping={0: DEV},
+                                 max_new_length=steps + 2, sink_size=sink, local_size=local, final_topk=50,
+                                 dynamic_update_interval=I, full_attention_threshold=100, enable_offload=False,
+                                 adaptive_topk_max_k=300)
+    g = torch.Generator(device=DEV).manual_seed(S)
+
+    def rows(n):
+        return torch.randn(bs, n, H, 128, generator=g, device=DEV).to(dtype)
+
+    cache.prefill_update_kv_cache(None, rows(S), rows(S), 0, 0)
+    for step in range(steps):
+        if step:
+            cache.decode_update_kv_cache(rows(1), rows(1), 0)
+        q = torch.randn(bs, 1, H * group, 128, generator=g, device=DEV).to(dtype)
+        out = cache.compute(q, 0)
+        k_got, z = cache.last_adaptive_k.clone(), cache._zones[0]
+        n_keys, n_cand, _, tiers = cache.retrieval_shape(0)
+        cap = cache._caps(n_cand)[0]
+        ids_got = cache._topk_ids[:bs * H * cap].view(bs, H, cap).clone()
+        pos = torch.cat([torch.arange(sink), torch.arange(z.local_start, z.seq_len)]).to(DEV)
+        logits_got = cache._dense_logits[:, :, :len(pos)].clone()
+        cand, scores = cache._plan.run_candidates(q, cache._srht_signs, cache._mag_centers, cache.cluster_key_counts_gpu[0],
+                                                  cache._codes_km[0], cache._nib_km[0], cache._w_km[0], sink, n_keys, tiers, n_cand)
+        logits = ops.dense_logits(q, cache.unified_keys_gpu[0][:, :, pos].contiguous(), len(pos), cache._attn_scale)
+        k_ref, ids_ref = ops.adaptive_topk(logits, cache._sl_vnorm_cache[0][:, :, pos].contiguous(), scores, cache._attn_scale, cand,
+                                           cache.adaptive_topk_threshold, cap, value_norm=cache.value_norm_gpu[0],
+                                           vn_offset=sink, k_min=1, k_max=cap)
+        assert torch.equal(logits_got, logits) and torch.equal(k_got, k_ref) and torch.equal(ids_got, ids_ref), step
+        kmax = int(k_ref.max())
+        ids = torch.cat([pos.expand(bs, H, -1), ids_ref[:, :, :kmax] + sink], dim=2)[..., None].expand(-1, -1, -1, 128)
+        K, V = (t[0].double().gather(2, ids) for t in (cache.unified_keys_gpu, cache.unified_values_gpu))
+        p = torch.softmax(q.double().view(bs, H, group, 128) @ K.transpose(2, 3).contiguous() * cache._attn_scale, dim=-1)
+        ref = (p @ V).view(bs, 1, H * group, 128)
+        # bf16: probabilities and result rounded to 8 bits; fp32: sums of a few hundred terms
+        assert (out.double() - ref).abs().max().item() < (2e-2 if dtype == torch.bfloat16 else 1e-5)
