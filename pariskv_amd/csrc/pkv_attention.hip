@@ -285,12 +285,75 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 
 constexpr int kMfmaWaves = 4;  // waves per workgroup: each takes a quarter of the split, merged through LDS
 
+// Segments that share one K and one V tensor (the cache's rows in HBM: sink, selected rows, local window), at most one of
+// them indexed: a key is a 32-bit byte offset into the (b, h) slab.  Half of a launch over a few hundred keys used to go
+// into finding addresses (1.2 us to pick a 64-bit pointer out of four for each of a lane's ten rows, after 1 us for a
+// 300-byte argument block); here that is one lane exchange per row.
+struct AttOne {
+  const char *k, *v;
+  int64_t stride_b, stride_h;           // bytes
+  uint32_t end[PKV_ATTN_MAX_SEGMENTS];  // exclusive ends in the concatenated key order; unused: 2^32 - 1
+  int32_t delta[PKV_ATTN_MAX_SEGMENTS]; // row - concatenated key
+  const int64_t *idx;                   // of the indexed segment, keys [idx_lo, idx_hi)
+  int64_t idx_stride, idx_limit;
+  uint32_t idx_lo, idx_hi, idx_row0;
+};
+
+// One key's place: a byte offset into the slab (AttOne), or the addresses of its K and V rows.
+template <bool ONE>
+struct AttPlace {
+  uint32_t off;
+  __device__ __forceinline__ AttPlace from(int lane) const { return {(uint32_t)__shfl((int)off, lane, PKV_WAVE)}; }
+};
+template <>
+struct AttPlace<false> {
+  uint64_t k, v;
+  __device__ __forceinline__ const char *k_from(int lane) const { return (const char *)pull(k, lane); }
+  __device__ __forceinline__ const char *v_from(int lane) const { return (const char *)pull(v, lane); }
+  static __device__ __forceinline__ uint64_t pull(uint64_t x, int lane) {
+    return ((uint64_t)(uint32_t)__shfl((int)(x >> 32), lane, PKV_WAVE) << 32) | (uint32_t)__shfl((int)(uint32_t)x, lane, PKV_WAVE);
+  }
+};
+
 template <bool INDEXED>
+__device__ __forceinline__ AttPlace<true> att_place(const AttOne &a, int row, int, int, uint32_t jj) {
+  int32_t d = a.delta[0];
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t) d = jj >= a.end[t - 1] ? a.delta[t] : d;
+  uint32_t r = jj + (uint32_t)d;
+  if (INDEXED && jj >= a.idx_lo && jj < a.idx_hi) {
+    const int64_t x = a.idx[(int64_t)row * a.idx_stride + (jj - a.idx_lo)];
+    r = a.idx_row0 + (uint32_t)(x < 0 ? 0 : (x >= a.idx_limit ? a.idx_limit - 1 : x));
+  }
+  return {r * 256u};
+}
+
+template <bool INDEXED>
+__device__ __forceinline__ AttPlace<false> att_place(const AttSegs &a, int row, int b, int h, uint32_t jj) {
+  int s = 0;
+  uint32_t first = 0;
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (t < a.n && jj >= (uint32_t)a.end[t - 1]) s = t, first = (uint32_t)a.end[t - 1];
+  const char *k = (const char *)a.k[0], *v = (const char *)a.v[0];
+  int64_t sb = a.stride_b[0], sh = a.stride_h[0], row0 = a.row0[0];
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (s == t) k = (const char *)a.k[t], v = (const char *)a.v[t], sb = a.stride_b[t], sh = a.stride_h[t], row0 = a.row0[t];
+  const int64_t r = INDEXED ? (int64_t)(att_resolve_row(a, row, jj) & 0x1fffffffu) : row0 + (int64_t)(jj - first);
+  const int64_t off = ((int64_t)b * sb + (int64_t)h * sh) * 2 + r * 256;
+  return {(uint64_t)(k + off), (uint64_t)(v + off)};
+}
+
+// grid (splits, KV heads, batch).  Decode step, us, with four-way pointer selection per row / with places by lane exchange:
+// 8 rows x 693 attended keys 30.2 / 27.7, 8 x 1188 (4 layers) 136.5 / 124.2, 64 x 887 (2 layers) 133.4 / 122.8.
+template <bool INDEXED, typename SEGS>
 __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_kernel(
-    const void *__restrict__ q, int n_kv_heads, int group, AttSegs segs, int64_t total,
-    const int32_t *__restrict__ row_keys, int64_t per_split, float scale_log2e, float *__restrict__ ws) {
-  const int split = blockIdx.x, row = blockIdx.y;
-  const int b = row / n_kv_heads, h = row % n_kv_heads;
+    const void *__restrict__ q, int group, SEGS segs, int64_t total, const int32_t *__restrict__ row_keys, int64_t per_split,
+    float scale_log2e, float *__restrict__ ws) {
+  constexpr bool ONE = __is_same(SEGS, AttOne);
+  const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
+  const int row = b * (int)gridDim.y + h;
   const int lane = threadIdx.x & (PKV_WAVE - 1), wave = threadIdx.x / PKV_WAVE;
   const int n = lane & 15, j = lane >> 4;
   if (row_keys) {
@@ -301,35 +364,19 @@ __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_k
   const int64_t j0 = (int64_t)split * per_split + (int64_t)wave * per_wave;
   const int64_t j1 = (j0 + per_wave < total) ? j0 + per_wave : total;  // j1 <= j0: nothing left for this wave
 
-  // per segment: byte address of "concatenated key 0" for this (b, h); with indexed segments: of row 0 of the slab
-  const char *kb[PKV_ATTN_MAX_SEGMENTS], *vb[PKV_ATTN_MAX_SEGMENTS];
-#pragma unroll
-  for (int s = 0; s < PKV_ATTN_MAX_SEGMENTS; ++s) {
-    const int64_t first = s == 0 ? 0 : segs.end[s - 1];
-    const int64_t off = ((int64_t)b * segs.stride_b[s] + (int64_t)h * segs.stride_h[s] +
-                         (INDEXED ? 0 : (segs.row0[s] - first) * 128)) * 2;
-    kb[s] = (const char *)segs.k[s] + off;
-    vb[s] = (const char *)segs.v[s] + off;
+  // Lane l holds the place of key blk0 + l of the current block of 64 keys (two steps; keys past j1 repeat the last one);
+  // the lanes that read a row get it from there, so that a place is found once per key and wave.
+  AttPlace<ONE> mine;
+  const char *kbase = nullptr, *vbase = nullptr;
+  if constexpr (ONE) {
+    const int64_t slab = (int64_t)b * segs.stride_b + (int64_t)h * segs.stride_h;
+    kbase = segs.k + slab, vbase = segs.v + slab;
   }
-  // INDEXED: lane l holds the resolved row of key blk0 + l for the current block of 64 keys (two steps);
-  // the rows a lane needs are then fetched from the owning lanes, so the index loads are one per key.
-  uint32_t my_row = 0;
-  int64_t blk0 = j0;
-  auto row_ptr = [&](const char *const (&base)[PKV_ATTN_MAX_SEGMENTS], int64_t key) {
-    const uint32_t jj = (uint32_t)(key < j1 ? key : j1 - 1);
-    const char *p = base[0];
-    if (INDEXED) {
-      const uint32_t packed = (uint32_t)__shfl((int)my_row, (int)(jj - (uint32_t)blk0), PKV_WAVE);
-#pragma unroll
-      for (int s = 1; s < PKV_ATTN_MAX_SEGMENTS; ++s)
-        if ((packed >> 29) == (uint32_t)s) p = base[s];
-      return p + (uint64_t)(packed & 0x1fffffffu) * 256u;
-    }
-#pragma unroll
-    for (int s = 1; s < PKV_ATTN_MAX_SEGMENTS; ++s)
-      if (s < segs.n && jj >= (uint32_t)segs.end[s - 1]) p = base[s];
-    return p + jj * 256u;
+  auto place_block = [&](int64_t jb) {
+    const int64_t key = jb + lane;
+    mine = att_place<INDEXED>(segs, row, b, h, (uint32_t)(key < j1 ? key : j1 - 1));
   };
+  if (j0 < j1) place_block(j0);  // before the queries: the indices' latency is the longer one
 
   const pkv_u32x4 zero4 = {0u, 0u, 0u, 0u};
   pkv_u32x4 qb[4];
@@ -343,23 +390,27 @@ __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_k
   for (int m = 0; m < 8; ++m) o[m] = pkv_f32x4{0.f, 0.f, 0.f, 0.f};
 
   for (int64_t jb = j0; jb < j1; jb += kMfmaStepKeys) {
-    if (INDEXED && ((jb - j0) & (PKV_WAVE - 1)) == 0) {
-      blk0 = jb;
-      const int64_t key = jb + lane;
-      my_row = att_resolve_row(segs, row, (uint32_t)(key < j1 ? key : j1 - 1));
-    }
+    const int in_block = (int)(jb - j0) & (PKV_WAVE - 1);
+    if (in_block == 0 && jb != j0) place_block(jb);
     // K: two tiles of 16 keys, lane (n, j) reads dims 32c + 8j .. +7 of key jb + 16t + n
     pkv_u32x4 ka[2][4], vr[8];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const char *kp = row_ptr(kb, jb + 16 * t + n) + 16 * j;
+      const char *kp;
+      if constexpr (ONE) kp = kbase + (uint64_t)(mine.from(in_block + 16 * t + n).off + 16u * (uint32_t)j);
+      else kp = mine.k_from(in_block + 16 * t + n) + 16 * j;
 #pragma unroll
       for (int c = 0; c < 4; ++c) ka[t][c] = __builtin_nontemporal_load((const pkv_u32x4 *)(kp + 64 * c));
     }
     // V: dims 8n .. 8n+7 of the 8 keys whose probabilities this lane will hold
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      vr[e] = __builtin_nontemporal_load((const pkv_u32x4 *)(row_ptr(vb, jb + 16 * (e >> 2) + 4 * j + (e & 3)) + 16 * n));
+    for (int e = 0; e < 8; ++e) {
+      const int at = in_block + 16 * (e >> 2) + 4 * j + (e & 3);
+      const char *vp;
+      if constexpr (ONE) vp = vbase + (uint64_t)(mine.from(at).off + 16u * (uint32_t)n);
+      else vp = mine.v_from(at) + 16 * n;
+      vr[e] = __builtin_nontemporal_load((const pkv_u32x4 *)vp);
+    }
 
     pkv_f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -381,12 +432,12 @@ __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_k
     mx = fmaxf(mx, __shfl_xor(mx, 16, PKV_WAVE));
     mx = fmaxf(mx, __shfl_xor(mx, 32, PKV_WAVE));
     const float m_new = fmaxf(m_run, mx);
-    const float corr = exp2f(m_run - m_new);
+    const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
     m_run = m_new;
     float p[8], psum = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      p[e] = valid[e] ? exp2f(sc[e] - m_new) : 0.f;
+      p[e] = valid[e] ? __builtin_amdgcn_exp2f(sc[e] - m_new) : 0.f;
       psum += p[e];
     }
     l_part = l_part * corr + psum;
@@ -507,6 +558,31 @@ int pick_splits_mfma(int rows, int64_t total) {
   return (int)s;
 }
 
+// The segments as offsets into one (b, h) slab: false where they lie in different tensors, more than one is indexed or a
+// row's byte offset would not fit 32 bits (2^24 rows of 256 bytes).
+bool as_one_tensor(const AttSegs &sg, AttOne &one) {
+  memset(&one, 0, sizeof one);
+  one.k = (const char *)sg.k[0], one.v = (const char *)sg.v[0];
+  one.stride_b = sg.stride_b[0] * 2, one.stride_h = sg.stride_h[0] * 2;
+  for (int i = 0; i < PKV_ATTN_MAX_SEGMENTS; ++i) one.end[i] = 0xffffffffu;
+  int64_t first = 0;
+  for (int i = 0; i < sg.n; ++i) {
+    if (sg.k[i] != sg.k[0] || sg.v[i] != sg.v[0] || sg.stride_b[i] != sg.stride_b[0] || sg.stride_h[i] != sg.stride_h[0])
+      return false;
+    const int64_t n = sg.end[i] - first, rows = sg.row0[i] + (sg.idx[i] ? sg.idx_limit[i] : n);
+    if (rows > ((int64_t)1 << 24)) return false;
+    one.end[i] = (uint32_t)sg.end[i];
+    one.delta[i] = (int32_t)(sg.row0[i] - first);
+    if (sg.idx[i]) {
+      if (one.idx) return false;
+      one.idx = sg.idx[i], one.idx_stride = sg.idx_stride[i], one.idx_limit = sg.idx_limit[i];
+      one.idx_lo = (uint32_t)first, one.idx_hi = (uint32_t)sg.end[i], one.idx_row0 = (uint32_t)sg.row0[i];
+    }
+    first = sg.end[i];
+  }
+  return true;
+}
+
 }  // namespace
 
 extern "C" size_t pkv_decode_attention_ws_bytes(int bs, int n_kv_heads, int group, int64_t total_keys) {
@@ -568,12 +644,17 @@ extern "C" int pkv_decode_attention(const void *q, int dtype, int bs, int n_kv_h
   hipStream_t s = (hipStream_t)stream;
   dim3 grid((unsigned)n_splits, (unsigned)rows);
   if (bf) {
-    if (indexed)
-      hipLaunchKernelGGL(pkv_attn_partial_mfma_kernel<true>, grid, dim3(kMfmaWaves * PKV_WAVE), 0, s, q, n_kv_heads, group, sg, total,
-                         row_keys, per_split, scale_log2e, (float *)ws);
-    else
-      hipLaunchKernelGGL(pkv_attn_partial_mfma_kernel<false>, grid, dim3(kMfmaWaves * PKV_WAVE), 0, s, q, n_kv_heads, group, sg, total,
-                         row_keys, per_split, scale_log2e, (float *)ws);
+    const dim3 grid3((unsigned)n_splits, (unsigned)n_kv_heads, (unsigned)bs);
+    AttOne one;
+#define PKV_ATT_MFMA(IDX, S)                                                                                                    \
+  hipLaunchKernelGGL((pkv_attn_partial_mfma_kernel<IDX, decltype(S)>), grid3, dim3(kMfmaWaves * PKV_WAVE), 0, s, q, group, S, total, \
+                     row_keys, per_split, scale_log2e, (float *)ws)
+    if (as_one_tensor(sg, one)) {
+      if (indexed) PKV_ATT_MFMA(true, one); else PKV_ATT_MFMA(false, one);
+    } else {
+      if (indexed) PKV_ATT_MFMA(true, sg); else PKV_ATT_MFMA(false, sg);
+    }
+#undef PKV_ATT_MFMA
   } else {
     // The KV head's other query heads in workgroups beside the first four's, in one launch: 12 rows x 865 keys, seven
     // heads, 2 x 8.0 us as two launches one after the other; the decode step around it (9001 keys) 48.3 -> 43 us.

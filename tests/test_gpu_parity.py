@@ -1721,3 +1721,34 @@ def test_prefill_store_rows_index_and_norms(ops, dtype, n_sink, n_enc, n_tail):
         assert torch.equal(cc, cc2)
         assert torch.equal(zn[..., sl], norm[:, :, n_sink:n_sink + n_enc]) and torch.equal(zn2[..., sl], norm[:, :, n_sink:n_sink + n_enc])
         assert torch.all(zn[..., n_enc:] == 0) and torch.all(zn2[..., n_enc:] == 7.0)
+
+
+@pytest.mark.parametrize("same_tensor", [True, False])
+@pytest.mark.parametrize("lens,indexed", [((1,), ()), ((1, 31, 1), (1,)), ((5, 64, 33), (1,)), ((127, 130), (0,)), ((63, 1, 64, 3), (3,)),
+                                          ((20, 40, 17), (0, 2)), ((9000,), ()), ((40, 8300), (1,))])
+def test_decode_attention_places_of_keys(ops, same_tensor, lens, indexed):
+    """Segments of one K/V tensor (places as 32-bit offsets), of several tensors, with no, one and two indexed segments, at the
+    edges of waves and splits: against attention over the same rows in 64 bits."""
+    bs, H, group = 2, 3, 5
+    g = torch.Generator(device=DEV).manual_seed(sum(lens) + 2 * len(indexed) + same_tensor)
+    rows = max(lens) + 50
+    pool = [[torch.randn(bs, H, rows, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2)] for _ in lens]
+    q = torch.randn(bs, 1, H * group, 128, generator=g, device=DEV).to(torch.bfloat16)
+    segs, K, V = [], [], []
+    for i, n in enumerate(lens):
+        k, v = pool[0 if same_tensor else i]
+        row0 = 7 + 3 * i
+        if i in indexed:
+            idx = torch.randint(0, rows - row0, (bs, H, n + 2), generator=g, device=DEV)
+            segs.append((k, v, row0, n, idx))
+            at = (idx[:, :, :n] + row0)[..., None].expand(-1, -1, -1, 128)
+            K.append(k.gather(2, at)), V.append(v.gather(2, at))
+        else:
+            segs.append((k, v, row0, n))
+            K.append(k[:, :, row0:row0 + n]), V.append(v[:, :, row0:row0 + n])
+    out = ops.DecodeAttention(bs, H, group, sum(lens), DEV).run(q, segs)
+    K, V = torch.cat(K, dim=2).double(), torch.cat(V, dim=2).double()
+    p = torch.softmax(q.double().view(bs, H, group, 128) @ K.transpose(2, 3).contiguous() / math.sqrt(128), dim=-1)
+    ref = (p @ V).view(bs, 1, H * group, 128)
+    # probabilities and the result are rounded to bf16 (2^-9 relative each); values up to ~4.5
+    assert (out.double() - ref).abs().max().item() < 2e-2
