@@ -50,7 +50,7 @@ int pkv_version(void);
 const char *pkv_last_error(void);
 /* sizeof of the argument structs as this library was compiled, for a binding to
  * compare with its own mirror: 0 pkv_attn_segment, 1 pkv_attn_args,
- * 2 pkv_retrieve_args, 3 pkv_adaptive_args, 5 pkv_prefill_args (0 for any other number).
+ * 2 pkv_retrieve_args, 3 pkv_adaptive_args, 5 pkv_prefill_args, 6 pkv_append_args (0 for any other number).
  * No counterpart in the reference. */
 size_t pkv_struct_bytes(int which);
 
@@ -272,6 +272,17 @@ int pkv_append_kv(const void *k_new, int64_t k_stride_b, int64_t k_stride_h,
                   void *dst_k, void *dst_v, int64_t dst_stride_b, int64_t dst_stride_h, int64_t dst_len,
                   int64_t slot, int bs, int n_kv_heads, int row_bytes,
                   float *vnorm, int64_t vn_stride_b, int64_t vn_stride_h, void *stream);
+/* The same with the destination in a block that a caller fills once per layer. */
+typedef struct pkv_append_args {
+  void *dst_k, *dst_v;
+  int64_t dst_stride_b, dst_stride_h, dst_len; /* bytes, bytes, rows */
+  int bs, n_kv_heads, row_bytes;
+  float *vnorm;
+  int64_t vn_stride_b, vn_stride_h;
+} pkv_append_args;
+int pkv_append_kv_run(const pkv_append_args *args, const void *k_new, int64_t k_stride_b, int64_t k_stride_h,
+                      const void *v_new, int64_t v_stride_b, int64_t v_stride_h, int64_t slot, void *stream);
+
 
 /* The oldest tokens of a layer leave the GPU: replaces the copy_() of staged
  * [bs][h][n][d] tensors into slices of the pinned host tensors on the side
@@ -624,6 +635,10 @@ typedef struct pkv_attn_args {
   void *ws;
   size_t ws_bytes;          /* pkv_decode_attention_ws_bytes(...) */
 } pkv_attn_args;
+
+/* pkv_decode_attention with its arguments in a block. */
+int pkv_decode_attention_run(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_args *args,
+                             void *stream);
 
 int pkv_decode_step(const pkv_retrieve_args *retrieve, void *ws, size_t ws_bytes,
                     const pkv_attn_args *attention, void *stream);

@@ -35,6 +35,13 @@ class AttnArgs(C.Structure):
                 ("out", _vp), ("ws", _vp), ("ws_bytes", _sz)]
 
 
+class AppendArgs(C.Structure):
+    """Mirror of ``pkv_append_args``."""
+
+    _fields_ = [("dst_k", _vp), ("dst_v", _vp), ("dst_stride_b", _i64), ("dst_stride_h", _i64), ("dst_len", _i64),
+                ("bs", _i), ("n_kv_heads", _i), ("row_bytes", _i), ("vnorm", _vp), ("vn_stride_b", _i64), ("vn_stride_h", _i64)]
+
+
 class KvAppend(C.Structure):
     """Mirror of ``pkv_kv_append``."""
 
@@ -144,6 +151,8 @@ PROTOTYPES = {
     "pkv_uniform_k": (_i, [_vp, _i, _vp, _vp, _i64, _vp]),
     "pkv_dense_logits": (_i, [_vp, _i, _i, _i, _i, _vp, _i64, _i64, _i64, C.c_float, _vp, _i64, _vp]),
     "pkv_decode_attention_ws_bytes": (_sz, [_i, _i, _i, _i64]),
+    "pkv_decode_attention_run": (_i, [_vp, _i, _i, _i, _i, C.POINTER(AttnArgs), _vp]),
+    "pkv_append_kv_run": (_i, [C.POINTER(AppendArgs), _vp, _i64, _i64, _vp, _i64, _i64, _i64, _vp]),
     "pkv_decode_attention": (_i, [_vp, _i, _i, _i, _i, C.POINTER(AttnSegment), _i, _vp, C.c_float, _vp, _vp, _sz, _vp]),
     "pkv_qk_norm_rope": (_i, [_vp, _i64, _i, _i, _i, _vp, _vp, C.c_float, _vp, _vp, _vp, _vp, _vp]),
     "pkv_add_rmsnorm": (_i, [_vp, _vp, _vp, C.c_float, _i, _i, _vp, _vp, _vp]),
@@ -190,7 +199,8 @@ def lib():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
-        for which, mirror in ((0, AttnSegment), (1, AttnArgs), (2, RetrieveArgs), (3, AdaptiveArgs), (5, PrefillArgs)):
+        for which, mirror in ((0, AttnSegment), (1, AttnArgs), (2, RetrieveArgs), (3, AdaptiveArgs), (5, PrefillArgs),
+                              (6, AppendArgs)):
             if os.environ.get("PARISKV_HIP_SO") and handle.pkv_struct_bytes(which) == 0:
                 continue
             if handle.pkv_struct_bytes(which) != C.sizeof(mirror):

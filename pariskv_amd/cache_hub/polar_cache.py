@@ -181,6 +181,9 @@ class polar_cache(KV_Cache):
         self._plan = ops.RetrievePlan(bs, H, self.group_size, cap, dev, max_keys, max_cand, max(1, min(final_topk, max_cand)))
         self._plan.skip_vote_counts = True  # the cache never looks at the per-key vote counts of a step
         self._bound = [None] * layer_num  # per layer: (n_keys, ops.BoundStep, topk, out_ids, index of the local segment)
+        # per layer: the append's destination, and the dense branch's attention as (encoded tokens, ops.BoundAttention)
+        self._append_bound = [None] * layer_num
+        self._dense_bound = [None] * layer_num
         self._out_ids = torch.empty((bs, H, max(1, final_topk)), dtype=torch.int64, device=dev)
         self._attention = ops.DecodeAttention(bs, H, self.group_size, self.unified_kv_capacity, dev)
         self.last_topk_indices = None  # [bs, H, K] of the most recent retrieval (zone-relative), for inspection
@@ -264,6 +267,7 @@ class polar_cache(KV_Cache):
         PCIe per layer and token (235 us for 924 rows x 8 heads), from HBM 7 us.  At most SHORT_ROWS_MAX rows a head;
         given back by the first step that retrieves.  None for longer prompts or a threshold too high for that."""
         rows = self._min_total() - self.sink_size - self.local_size
+        self._dense_bound[layer_idx] = None
         if n_tok >= self._min_total() or rows > SHORT_ROWS_MAX:
             self._short_kv[layer_idx] = None
             return None
@@ -275,6 +279,11 @@ class polar_cache(KV_Cache):
             self._short_kv[layer_idx] = kv
         kv[2][b0:b1] = [True] * (b1 - b0)   # samples whose rows are here: prompts may arrive one by one
         return kv[0][b0:b1], kv[1][b0:b1]
+
+    def _drop_short_rows(self, layer_idx: int) -> None:
+        """The sequence has outgrown the dense branch: its retrieval-zone rows in HBM go back to the allocator."""
+        if self._short_kv[layer_idx] is not None:
+            self._short_kv[layer_idx] = self._dense_bound[layer_idx] = None
 
     def release_prefill_staging(self) -> None:
         """Free the prefill staging pairs (two layers' worth of retrieval-zone K/V in HBM) once prefill is over; they
@@ -404,7 +413,7 @@ class polar_cache(KV_Cache):
         if short is not None and self.current_seq_len[layer_idx] < self._min_total() and r.cpu_row0 + n <= short[0].shape[2]:
             sk, sv = (t[:, :, r.cpu_row0:r.cpu_row0 + n] for t in short[:2])
         else:
-            self._short_kv[layer_idx] = None
+            self._drop_short_rows(layer_idx)
             sk, sv = self._offload_keys_buffer[layer_idx][:, :, :n], self._offload_values_buffer[layer_idx][:, :, :n]
         self._store_rows(layer_idx, kg[:, :, S0:S0 + n], vg[:, :, S0:S0 + n], 0, bs, 0, n, None, 0, (sk, sv), r.encode_abs0)
         self._on_refresh(layer_idx, r)
@@ -425,7 +434,13 @@ class polar_cache(KV_Cache):
         return {}
 
     def _append(self, layer_idx, slot, key_states, value_states):
-        ops.append_kv(key_states, value_states, self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx], slot)
+        bound = self._append_bound[layer_idx]
+        if bound is None:
+            bound = self._append_bound[layer_idx] = self._bind_append(layer_idx)
+        bound.launch(key_states, value_states, slot)
+
+    def _bind_append(self, layer_idx):
+        return ops.BoundAppend(self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx])
 
     def _on_refresh(self, layer_idx, r):
         pass
@@ -452,6 +467,19 @@ class polar_cache(KV_Cache):
         """softmax(q k^T / sqrt(D)) v over the attended set (:1097-1105).  queries [bs,1,Hq,D]; segments: list of
         (k, v, row0, n_rows) runs of [bs,Hkv,rows,D] tensors, read in place by the HIP decode-attention kernel."""
         return self._attention.run(queries, [s for s in segments if s[3] > 0])
+
+    def _attend_all(self, q, layer_idx, z):
+        """The dense branch.  Its argument block holds until the retrieval zone or its rows in HBM change; filling and
+        checking it anew for every token took the host longer than the two launches take the GPU (20 against 9 us)."""
+        bound = self._dense_bound[layer_idx]
+        if bound is None or bound[0] != z.encoded:
+            segments = self._full_kv(layer_idx)
+            kg, short = self.unified_keys_gpu[layer_idx], self._short_kv[layer_idx]
+            if not all(s[0] is kg or (short is not None and s[0] is short[0]) for s in segments):
+                return self._attend(q, segments)   # copies of host rows: this step's only
+            bound = self._dense_bound[layer_idx] = (z.encoded, ops.BoundAttention(self._attention, q, segments))
+        bound[1].segs[0].n_rows = z.gpu_prefix_rows if self._layer_offload[layer_idx] else z.seq_len
+        return bound[1].launch(q)
 
     def _full_kv(self, layer_idx):
         """Dense fallback: every stored token (reference _get_full_kv_for_attention :701-737), as attention segments."""
@@ -506,8 +534,8 @@ class polar_cache(KV_Cache):
         offload = self._layer_offload[layer_idx]
         n_keys = self.cpu_valid_end[layer_idx] if offload else z.encoded
         if total < self._min_total() or n_keys <= 0:
-            return self._attend(queries.contiguous(), self._full_kv(layer_idx))
-        self._short_kv[layer_idx] = None   # the sequence has outgrown the dense branch
+            return self._attend_all(queries if queries.is_contiguous() else queries.contiguous(), layer_idx, z)
+        self._drop_short_rows(layer_idx)
         q = queries if queries.is_contiguous() else queries.contiguous()
         step = self._bound[layer_idx]
         if step is None or step[0] != n_keys:

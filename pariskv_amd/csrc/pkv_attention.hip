@@ -683,3 +683,10 @@ extern "C" int pkv_decode_attention(const void *q, int dtype, int bs, int n_kv_h
   PKV_LAUNCH_CHECK("pkv_attn_merge_kernel");
   return PKV_OK;
 }
+
+extern "C" int pkv_decode_attention_run(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_args *a,
+                                        void *stream) {
+  PKV_REQUIRE(a != nullptr, "pkv_decode_attention: null args");
+  return pkv_decode_attention(q, dtype, bs, n_kv_heads, group, a->segments, a->n_segments, a->row_keys, a->scale, a->out, a->ws,
+                              a->ws_bytes, stream);
+}

@@ -265,6 +265,14 @@ extern "C" int pkv_append_kv(const void *k_new, int64_t k_stride_b, int64_t k_st
   return PKV_OK;
 }
 
+extern "C" int pkv_append_kv_run(const pkv_append_args *a, const void *k_new, int64_t k_stride_b, int64_t k_stride_h,
+                                 const void *v_new, int64_t v_stride_b, int64_t v_stride_h, int64_t slot, void *stream) {
+  PKV_REQUIRE(a != nullptr, "append: null args");
+  return pkv_append_kv(k_new, k_stride_b, k_stride_h, v_new, v_stride_b, v_stride_h, a->dst_k, a->dst_v, a->dst_stride_b,
+                       a->dst_stride_h, a->dst_len, slot, a->bs, a->n_kv_heads, a->row_bytes, a->vnorm, a->vn_stride_b,
+                       a->vn_stride_h, stream);
+}
+
 extern "C" int pkv_offload_rows(const void *src_k, const void *src_v, int64_t src_stride_b, int64_t src_stride_h,
                                 int64_t src_stride_row, void *dst_k_host, void *dst_v_host, int64_t dst_len,
                                 int64_t dst_row0, int64_t n_rows, int bs, int n_kv_heads, int row_bytes, void *stream) {

@@ -31,6 +31,7 @@ extern "C" size_t pkv_struct_bytes(int which) {
     case 2: return sizeof(pkv_retrieve_args);
     case 3: return sizeof(pkv_adaptive_args);
     case 5: return sizeof(pkv_prefill_args);
+    case 6: return sizeof(pkv_append_args);
     default: return 0;
   }
 }

@@ -28,11 +28,11 @@ MAG_CENTERS = (0.0419921875, 0.126953125, 0.212890625, 0.302734375, 0.396484375,
 
 
 def _p(t: Optional[torch.Tensor]):
-    return C.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _stream(t: torch.Tensor):
-    return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _dt(dtype: torch.dtype) -> int:
@@ -527,6 +527,37 @@ def gather_hbm(src_k, src_v, idx, dst_k, dst_v, idx_offset: int = 0, dst_row0: i
     _gather(_lib.lib().pkv_gather_hbm, src_k, src_v, idx, dst_k, dst_v, idx_offset, dst_row0)
 
 
+class BoundAppend:
+    """The destination of one layer's :func:`append_kv`, validated once: a token costs the checks of its own rows."""
+
+    __slots__ = ("_a", "_ra", "keep", "_shape", "_dtype", "_es", "_fn", "_device")
+
+    def __init__(self, dst_k, dst_v, vnorm: Optional[torch.Tensor] = None):
+        bs, H, rows, D = dst_k.shape
+        _need(dst_k.is_cuda and dst_v.is_cuda and dst_k.dtype == dst_v.dtype and dst_k.shape == dst_v.shape and
+              dst_k.stride() == dst_v.stride() and dst_k.stride(3) == 1 and dst_k.stride(2) == D,
+              "dst_k, dst_v: [bs,Hkv,rows,D] with contiguous rows")
+        _need(vnorm is None or (vnorm.is_cuda and vnorm.dtype == torch.float32 and tuple(vnorm.shape[:2]) == (bs, H) and
+                                vnorm.is_contiguous()), "vnorm: contiguous fp32 [bs,Hkv,rows]")
+        es = dst_k.element_size()
+        self._a = _lib.AppendArgs(dst_k.data_ptr(), dst_v.data_ptr(), dst_k.stride(0) * es, dst_k.stride(1) * es, rows, bs, H,
+                                  D * es, _p(vnorm), *(vnorm.stride()[:2] if vnorm is not None else (0, 0)))
+        self._ra, self.keep = C.byref(self._a), (dst_k, dst_v, vnorm)
+        self._shape, self._dtype, self._es, self._device = (bs, 1, H, D), dst_k.dtype, es, dst_k.device
+        self._fn = _lib.lib().pkv_append_kv_run
+
+    def launch(self, k, v, slot: int) -> None:
+        """k, v: [bs,1,Hkv,D] of the destination's dtype with contiguous rows, on the GPU."""
+        ks, vs, es = k.stride(), v.stride(), self._es
+        _need(k.shape == self._shape and v.shape == self._shape and ks[3] == 1 and vs[3] == 1 and k.is_cuda and v.is_cuda,
+              "key_states, value_states: [bs,1,Hkv,D] on the GPU with contiguous rows")
+        _need(k.dtype == self._dtype and v.dtype == self._dtype, "append: dtypes differ")
+        rc = self._fn(self._ra, k.data_ptr(), ks[0] * es, ks[2] * es, v.data_ptr(), vs[0] * es, vs[2] * es, slot,
+                      torch.cuda.current_stream(self._device).cuda_stream)
+        if rc != 0:
+            _lib.check(rc)
+
+
 def append_kv(key_states, value_states, dst_k, dst_v, slot: int, vnorm: Optional[torch.Tensor] = None) -> None:
     """dst_k[:, :, slot, :] = key_states[:, 0] and the same for values, in one launch
     (decode_update_kv_cache, cache_hub/polar_cache.py:848-856).  key_states/value_states [bs,1,Hkv,D];
@@ -781,6 +812,30 @@ def gather_cpu(src: torch.Tensor, index: torch.Tensor, out: torch.Tensor, n_thre
 
 
 # ------------------------------------------------------- fused decode step
+
+
+class BoundAttention:
+    """The argument block of one layer's pkv_decode_attention, validated once; the caller patches ``segs[i].n_rows``."""
+
+    __slots__ = ("aa", "segs", "keep", "_raa", "_dims", "_fn", "_numel", "_dtype")
+
+    def __init__(self, att, q, segments):
+        self.aa, _ = att.c_args(q, segments, out=q)  # out is patched at every launch
+        self.segs, self._raa, self.keep = self.aa.segments, C.byref(self.aa), (att, segments)
+        self._dims = (_dt(q.dtype), att.bs, att.H, att.G)
+        self._fn = _lib.lib().pkv_decode_attention_run
+        self._numel, self._dtype = q.numel(), q.dtype
+
+    def launch(self, q: torch.Tensor) -> torch.Tensor:
+        """q: contiguous [bs,1,Hq,128] of the bound dtype.  Returns the attention output, shaped like q."""
+        _need(q.is_cuda and q.is_contiguous() and q.numel() == self._numel and q.dtype == self._dtype and q.shape[-1] == HEAD_DIM,
+              "queries must be contiguous [bs,1,Hq,128] of the cache dtype")
+        out = torch.empty_like(q)
+        self.aa.out = out.data_ptr()
+        rc = self._fn(q.data_ptr(), *self._dims, self._raa, torch.cuda.current_stream(q.device).cuda_stream)
+        if rc != 0:
+            _lib.check(rc)
+        return out
 
 
 class BoundStep:

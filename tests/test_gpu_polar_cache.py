@@ -993,3 +993,31 @@ def test_dense_adaptive_step_with_two_runs_of_dense_rows(sink, S, dtype, bs, gro
         ref = (p @ V).view(bs, 1, H * group, 128)
         # bf16: probabilities and result rounded to 8 bits; fp32: sums of a few hundred terms
         assert (out.double() - ref).abs().max().item() < (2e-2 if dtype == torch.bfloat16 else 1e-5)
+
+
+@pytest.mark.parametrize("host", [True, False])
+def test_dense_branch_over_refreshes_and_new_prompts(host):
+    """Below the retrieval threshold the attention's argument block is kept between tokens: over index refreshes, a second
+    and a third prompt in the same cache (shorter than sink + local, then long again) every step attends to all tokens."""
+    from pariskv_amd.cache_hub.polar_cache import polar_cache
+
+    bs, H, group, I = 1, 2, 4, 16
+    cache = polar_cache(valid_start=[0], layer_num=1, batch_size=bs, max_length=700, num_key_value_heads=H, num_heads=H * group,
+                        head_dim=128, dtype=torch.bfloat16, layer_mapping={0: DEV}, max_new_length=60, sink_size=8, local_size=32,
+                        final_topk=20, dynamic_update_interval=I, full_attention_threshold=2000, enable_offload=host)
+    g = torch.Generator(device=DEV).manual_seed(11)
+    for S in (300, 30, 500):
+        K, V = (torch.randn(bs, S, H, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+        cache.context = 0
+        cache.prefill_update_kv_cache(None, K, V, 0, 0)
+        for t in range(2 * I + 3):
+            k, v = (torch.randn(bs, 1, H, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+            q = torch.randn(bs, 1, H * group, 128, generator=g, device=DEV).to(torch.bfloat16)
+            K, V = torch.cat([K, k], dim=1), torch.cat([V, v], dim=1)
+            cache.decode_update_kv_cache(k, v, 0)
+            out = cache.compute(q, 0)
+            Kd, Vd = K.permute(0, 2, 1, 3).double().contiguous(), V.permute(0, 2, 1, 3).double().contiguous()
+            p = torch.softmax(q.double().view(bs, H, group, 128) @ Kd.transpose(2, 3).contiguous() / math.sqrt(128), dim=-1)
+            ref = (p @ Vd).view(bs, 1, H * group, 128)
+            # probabilities and the result are rounded to bf16; values up to ~4.5
+            assert (out.double() - ref).abs().max().item() < 2e-2, (S, t)
