@@ -13,16 +13,16 @@ constexpr int kSelThreads = 256;
 constexpr int kSelKeysPerThread = 16;                             // one 128-bit load of counts
 constexpr int kSelKeysPerIter = kSelThreads * kSelKeysPerThread;  // 4096
 
-// 16 one-byte counts (all <= 127) against the threshold, four at a time: adding 127 - theta
+// 4 * ND one-byte counts (all <= 127) against the threshold, four at a time: adding 127 - theta
 // (128 - theta) to a byte sets its top bit exactly when the count is above (at or above) theta, and no
 // byte overflows into its neighbour.  Bit 8b + 7 of gt[d] / eq[d] stands for key 4d + b; only the
 // first n_valid keys count.
-__device__ __forceinline__ void count_masks16(const pkv_u32x4 w, uint32_t theta, int64_t n_valid, uint32_t (&gt)[4],
-                                              uint32_t (&eq)[4]) {
+template <int ND>
+__device__ __forceinline__ void count_masks(const uint32_t (&ww)[ND], uint32_t theta, int64_t n_valid, uint32_t (&gt)[ND],
+                                            uint32_t (&eq)[ND]) {
   const uint32_t kgt = (127u - theta) * 0x01010101u, kge = (128u - theta) * 0x01010101u;
-  const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-  for (int d = 0; d < 4; ++d) {
+  for (int d = 0; d < ND; ++d) {
     const int64_t left = n_valid - 4 * d;
     const uint32_t vm = left >= 4 ? 0x80808080u : (left <= 0 ? 0u : (0x80808080u >> (8 * (4 - (int)left))));
     const uint32_t v7 = ww[d] & 0x7f7f7f7fu;
@@ -33,9 +33,20 @@ __device__ __forceinline__ void count_masks16(const pkv_u32x4 w, uint32_t theta,
   }
 }
 
-__device__ __forceinline__ int popc4(const uint32_t (&m)[4]) {
-  return __popc(m[0]) + __popc(m[1]) + __popc(m[2]) + __popc(m[3]);
+__device__ __forceinline__ void count_masks16(const pkv_u32x4 w, uint32_t theta, int64_t n_valid, uint32_t (&gt)[4],
+                                              uint32_t (&eq)[4]) {
+  const uint32_t ww[4] = {w.x, w.y, w.z, w.w};
+  count_masks<4>(ww, theta, n_valid, gt, eq);
 }
+
+template <int ND>
+__device__ __forceinline__ int popc_all(const uint32_t (&m)[ND]) {
+  int n = 0;
+#pragma unroll
+  for (int d = 0; d < ND; ++d) n += __popc(m[d]);
+  return n;
+}
+__device__ __forceinline__ int popc4(const uint32_t (&m)[4]) { return popc_all<4>(m); }
 
 // Threshold and output offsets of one workgroup from the suffix histograms the collision scan leaves
 // behind: row_suf[row][t] = keys of the row with count >= t (summed over chunks with atomics),
@@ -79,12 +90,10 @@ __device__ __forceinline__ void select_prologue(uint32_t rs_mine, const uint16_t
     gt += g;
     eq += ge - g;
   }
-#pragma unroll
-  for (int m = 1; m < PKV_WAVE; m <<= 1) {
-    gt += __shfl_xor(gt, m, PKV_WAVE);
-    eq += __shfl_xor(eq, m, PKV_WAVE);
-  }
-  if (pkv_lane() == 0) {
+  // wave sums in the last lane, without a trip through the LDS crossbar (twelve dependent ones took 0.4 us here)
+  gt = (uint32_t)pkv_wave_incl_scan((int)gt);
+  eq = (uint32_t)pkv_wave_incl_scan((int)eq);
+  if (pkv_lane() == PKV_WAVE - 1) {
     s_red[0][tid / PKV_WAVE] = gt;
     s_red[1][tid / PKV_WAVE] = eq;
   }

@@ -91,6 +91,9 @@ __global__ __launch_bounds__(kSelThreads) void pkv_select_kernel(const uint8_t *
 // out/scores: [rows][k]; position p of a row holds the candidate's key index and its score.
 // extra_out (optional, [rows][k]): the fp32 word at byte extra_off of the candidate's record, e.g. the value
 // norm the adaptive-k stage weighs it with.
+// KPT: counts per thread and pass.  With 16 a 256-key chunk's candidates (half of its keys on short rows) were listed by 16
+// threads one after the other, 1.4 us of a 5.7 us launch.
+template <int KPT>
 __global__ __launch_bounds__(kSelThreads) void pkv_select_rerank_kernel(
     const uint8_t *__restrict__ cnt, int64_t cnt_stride, const uint32_t *__restrict__ row_suf,
     const uint16_t *__restrict__ chunk_suf, int chunk_keys, int n_kv_heads, int64_t n_keys, int64_t k,
@@ -106,15 +109,32 @@ __global__ __launch_bounds__(kSelThreads) void pkv_select_rerank_kernel(
 
   __shared__ int s_scan[2][kSelThreads / PKV_WAVE];
   __shared__ float s_prod[128 * 16];
-  __shared__ uint16_t s_list_key[kSelKeysPerIter];  // offset of the key inside the iteration's 4096-key block
+  constexpr int kKeysPerIter = kSelThreads * KPT;
+  constexpr int ND = KPT < 4 ? 1 : KPT / 4;
+  __shared__ uint16_t s_list_key[kKeysPerIter];  // offset of the key inside the iteration's block of keys
 
   const uint8_t *crow = cnt + (int64_t)row * cnt_stride;
   const int64_t chunk_begin = (int64_t)chunk * chunk_keys;
   const int64_t chunk_end = (chunk_begin + chunk_keys < n_keys) ? chunk_begin + chunk_keys : n_keys;
-  const pkv_u32x4 zero4 = {0u, 0u, 0u, 0u};
-  int64_t i0 = chunk_begin + (int64_t)tid * kSelKeysPerThread;
+  // count rows are 16-byte aligned and padded to 16: whole loads stay in bounds
+  auto load_counts = [&](int64_t at, uint32_t (&ww)[ND]) {
+    const bool live = at < chunk_end;
+    if constexpr (KPT == 16) {
+      const pkv_u32x4 x = live ? *(const pkv_u32x4 *)(crow + at) : pkv_u32x4{0u, 0u, 0u, 0u};
+      ww[0] = x.x, ww[1] = x.y, ww[2] = x.z, ww[3] = x.w;
+    } else if constexpr (KPT == 8) {
+      const pkv_u32x2 x = live ? *(const pkv_u32x2 *)(crow + at) : pkv_u32x2{0u, 0u};
+      ww[0] = x.x, ww[1] = x.y;
+    } else if constexpr (KPT == 4) {
+      ww[0] = live ? *(const uint32_t *)(crow + at) : 0u;
+    } else {
+      ww[0] = live ? crow[at] : 0u;
+    }
+  };
+  int64_t i0 = chunk_begin + (int64_t)tid * KPT;
   const uint32_t rs_mine = tid < 128 ? row_suf[(int64_t)row * 128 + tid] : 0u;  // both before the threshold is known
-  pkv_u32x4 w = i0 < chunk_end ? *(const pkv_u32x4 *)(crow + i0) : zero4;
+  uint32_t w[ND];
+  load_counts(i0, w);
   const float qn = qnorm[row];
 
   pkv_build_prod_table<kSelThreads>(s_prod, qhat + (int64_t)row * 128, centers);
@@ -127,12 +147,13 @@ __global__ __launch_bounds__(kSelThreads) void pkv_select_rerank_kernel(
   const uint16_t *wrow = weight + (int64_t)b * ws_b + (int64_t)h * ws_h;
 
   int it = 0;
-  for (int64_t blk0 = chunk_begin; blk0 < chunk_end; blk0 += kSelKeysPerIter, ++it) {
-    uint32_t gt[4], eq[4];
-    count_masks16(w, theta, chunk_end - i0, gt, eq);
-    i0 += kSelKeysPerIter;
-    if (blk0 + kSelKeysPerIter < chunk_end) w = i0 < chunk_end ? *(const pkv_u32x4 *)(crow + i0) : zero4;
-    const int packed = popc4(gt) | (popc4(eq) << 16);
+  for (int64_t blk0 = chunk_begin; blk0 < chunk_end; blk0 += kKeysPerIter, ++it) {
+    uint32_t gt[ND], eq[ND];
+    const int64_t left = chunk_end - i0;
+    count_masks<ND>(w, theta, left < KPT ? left : KPT, gt, eq);
+    i0 += kKeysPerIter;
+    if (blk0 + kKeysPerIter < chunk_end) load_counts(i0, w);
+    const int packed = popc_all<ND>(gt) | (popc_all<ND>(eq) << 16);
     int total;
     const int excl = pkv_block_excl_scan<kSelThreads>(packed, s_scan[it & 1], total);
     const int n_gt_it = total & 0xffff, n_sel_it = n_gt_it + (total >> 16);
@@ -142,17 +163,17 @@ __global__ __launch_bounds__(kSelThreads) void pkv_select_rerank_kernel(
     int lg = excl & 0xffff;
     int le = n_gt_it + (excl >> 16);
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
+    for (int d = 0; d < ND; ++d) {
       uint32_t g = gt[d], e = eq[d];
       while (g) {
         const int bit = __ffs((int)g) - 1;
         g &= g - 1;
-        s_list_key[lg++] = (uint16_t)(tid * kSelKeysPerThread + 4 * d + (bit >> 3));
+        s_list_key[lg++] = (uint16_t)(tid * KPT + 4 * d + (bit >> 3));
       }
       while (e) {
         const int bit = __ffs((int)e) - 1;
         e &= e - 1;
-        s_list_key[le++] = (uint16_t)(tid * kSelKeysPerThread + 4 * d + (bit >> 3));
+        s_list_key[le++] = (uint16_t)(tid * KPT + 4 * d + (bit >> 3));
       }
     }
     const int64_t pos_gt0 = base_gt, pos_eq0 = base_eq - n_gt_it, eq_room = k - base_eq;
@@ -2166,11 +2187,16 @@ int pkv_launch_select_rerank(const uint8_t *cnt_u8, int64_t cnt_stride, const ui
     PKV_LAUNCH_CHECK("pkv_select_rerank_pieces_kernel");
     return PKV_OK;
   }
-  hipLaunchKernelGGL(pkv_select_rerank_kernel, grid, dim3(kSelThreads), 0, s, cnt_u8, cnt_stride, row_suf, chunk_suf,
-                     chunk_keys,
-                     n_kv_heads, n_keys, k, nib, ns_b, ns_h, (int)ns_key, weight, ws_b, ws_h, (int)ws_key, qhat, qnorm,
-                     centers, cand, scores, (int)extra_off, extra_out,
-                     range_slots, range_row_stride);
+  // as many counts per thread as make one pass of the chunk (chunks are powers of two from 256 keys on)
+#define PKV_SR(KPT)                                                                                                           \
+  hipLaunchKernelGGL(pkv_select_rerank_kernel<KPT>, grid, dim3(kSelThreads), 0, s, cnt_u8, cnt_stride, row_suf, chunk_suf,    \
+                     chunk_keys, n_kv_heads, n_keys, k, nib, ns_b, ns_h, (int)ns_key, weight, ws_b, ws_h, (int)ws_key, qhat,  \
+                     qnorm, centers, cand, scores, (int)extra_off, extra_out, range_slots, range_row_stride)
+  if (chunk_keys <= 256) PKV_SR(1);
+  else if (chunk_keys <= 1024) PKV_SR(4);
+  else if (chunk_keys <= 2048) PKV_SR(8);
+  else PKV_SR(16);
+#undef PKV_SR
   PKV_LAUNCH_CHECK("pkv_select_rerank_kernel");
   return PKV_OK;
 }

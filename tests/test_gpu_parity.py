@@ -1752,3 +1752,29 @@ def test_decode_attention_places_of_keys(ops, same_tensor, lens, indexed):
     ref = (p @ V).view(bs, 1, H * group, 128)
     # probabilities and the result are rounded to bf16 (2^-9 relative each); values up to ~4.5
     assert (out.double() - ref).abs().max().item() < 2e-2
+
+
+@pytest.mark.parametrize("rows,n,k", [(1, 300, 150), (8, 3520, 1760), (8, 6000, 3), (8, 32000, 3200), (16, 20001, 4001),
+                                      (64, 40000, 4000), (32, 70001, 7000)])
+def test_select_rerank_at_every_chunk_size(ops, rows, n, k):
+    """Candidates and scores of the fused select + rerank for chunks of 256, 1024, 2048 and 4096 keys (one to sixteen counts per
+    thread), with a ragged last chunk: the candidate list is the stand-alone select's, the scores the stand-alone rerank's."""
+    bs, H, G = (rows // 8, 8, 2) if rows >= 8 else (1, rows, 2)
+    g = torch.Generator(device=DEV).manual_seed(n + k)
+    keys = torch.randn(bs, H, n, 128, generator=g, device=DEV).to(torch.bfloat16)
+    signs, centers = ops.srht_signs(DEV), ops.mag_centers(DEV)
+    codes_km, nib_km, w_km, cb, k4, kw = ops.alloc_keymajor(bs, H, n, DEV)
+    cc = torch.zeros(bs, H, 16, 256, dtype=torch.int32, device=DEV)
+    ops.encode_append(keys, signs, cb, k4, kw, cc)
+    q = torch.randn(bs, 1, H * G, 128, generator=g, device=DEV).to(torch.bfloat16)
+    tiers = [int(math.ceil(n * 0.3 * r)) for r in ops.TIER_RATIOS]
+    plan = ops.RetrievePlan(bs, H, G, n, DEV, n, k, 1)
+    cand, scores = plan.run_candidates(q, signs, centers, cc, codes_km, nib_km, w_km, 0, n, tiers, k)
+    qhat, qnorm, lut, _ = ops.query_prep_lut(q, H, signs, cc, tiers)
+    cnt = ops.collision_scan(cb, lut)
+    cnt = cnt[0] if isinstance(cnt, tuple) else cnt
+    want = ops.bucket_topk(cnt.view(bs * H, n), k).view(bs, H, k)
+    assert torch.equal(cand.view(bs, H, k), want)
+    ref = ops.rerank4(want, k4, kw, qhat.view(bs, H, 16, 8), qnorm.view(bs, H, 1), centers)
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    assert torch.equal(scores.view(bs, H, k), ref.view(bs, H, k))
