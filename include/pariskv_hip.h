@@ -634,6 +634,7 @@ typedef struct pkv_attn_args {
   void *out;                /* [bs][n_kv_heads*group][128] in the query dtype */
   void *ws;
   size_t ws_bytes;          /* pkv_decode_attention_ws_bytes(...) */
+  int row_keys_uniform;     /* 1: every row attends to the largest of row_keys[0 .. bs*n_kv_heads) keys */
 } pkv_attn_args;
 
 /* pkv_decode_attention with its arguments in a block. */

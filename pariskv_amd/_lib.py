@@ -32,7 +32,7 @@ class AttnArgs(C.Structure):
     """Mirror of ``pkv_attn_args``."""
 
     _fields_ = [("segments", AttnSegment * 4), ("n_segments", _i), ("row_keys", _vp), ("scale", C.c_float),
-                ("out", _vp), ("ws", _vp), ("ws_bytes", _sz)]
+                ("out", _vp), ("ws", _vp), ("ws_bytes", _sz), ("row_keys_uniform", _i)]
 
 
 class AppendArgs(C.Structure):

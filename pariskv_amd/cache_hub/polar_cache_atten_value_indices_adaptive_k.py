@@ -9,8 +9,9 @@ Like :mod:`polar_cache_adaptivek_varlen`, every decode step ranks the candidates
   clamp (``:1564-1577``);
 * the attended set is dense: every row keeps ``global_k = max over rows of k`` ids of its own benefit order
   (``:1585-1589``, ``:1462-1499``), so rows with a small k still attend to the next-best candidates of their list.
-  The reference reads ``global_k`` back to the host to size its tensors; here a one-workgroup kernel broadcasts the
-  maximum on the device and the gather and the attention take it from there, so the step has no host synchronisation;
+  The reference reads ``global_k`` back to the host to size its tensors; here the attention takes the maximum over the
+  rows on the device (with K/V on the host a one-workgroup kernel broadcasts it, for the gather too), so the step has no
+  host synchronisation;
 * both storage modes are supported: with ``enable_offload=False`` the K/V rows and the value norms live at their
   absolute positions on the GPU (``:377-381``, ``:1086``, ``:967``) and the selected rows are attended in place through
   the index list.
@@ -118,7 +119,7 @@ class polar_cache(_adaptive_base):
                         value_norm=self.value_norm_gpu[layer_idx], vn_offset=S0, record_word_offset=ops.RECORD_VALUE_NORM_OFFSET,
                         threshold=self.adaptive_topk_threshold, k_out=topk_cap, k_min=k_min, k_max=k_max,
                         adaptive_k=self._adaptive_k, topk_ids=self._topk_ids, row_keys=self._row_keys, row_keys_base=dense,
-                        uniform_k=self._uniform_k, ws=self._adk_ws, src_k=None, src_v=None, dst_k=None, dst_v=None)
+                        row_keys_uniform=True, ws=self._adk_ws, src_k=None, src_v=None, dst_k=None, dst_v=None)
         ids = self._topk_ids[:bs * H * topk_cap].view(bs, H, topk_cap)
         # the selected rows come last so that the per-row key count cuts inside them (the reference gathers copies, :1481-1488)
         segments = [(kg, vg, 0, S0), (kg, vg, local0, z.dense_tail_len), (kg, vg, S0, topk_cap, ids)]  # runs may be empty

@@ -105,13 +105,31 @@ __device__ __forceinline__ void load8(const void *base, int64_t elem_off, float 
   expand8<BF16>(r, x);
 }
 
+// Keys row `row` attends to: all `total`, its own row_keys[row], or with uniform > 0 the largest of row_keys[0 .. uniform)
+// (the dense form of the adaptive-k step, where a launch of its own for the maximum took 4.5 us at 24 rows).
+__device__ __forceinline__ int64_t att_row_total(int64_t total, const int32_t *__restrict__ row_keys, int row, int uniform) {
+  if (!row_keys) return total;
+  int64_t rk;
+  if (uniform > 0) {
+    int m = 0;
+    for (int r = pkv_lane(); r < uniform; r += PKV_WAVE) m = max(m, row_keys[r]);
+#define PKV_ATT_MAX(M) { const int o = (int)pkv_lane_xor<M>((uint32_t)m); m = max(m, o); }
+    PKV_ATT_MAX(1) PKV_ATT_MAX(2) PKV_ATT_MAX(4) PKV_ATT_MAX(8) PKV_ATT_MAX(16) PKV_ATT_MAX(32)
+#undef PKV_ATT_MAX
+    rk = __builtin_amdgcn_readfirstlane(m);
+  } else {
+    rk = row_keys[row];
+  }
+  return rk < total ? (rk > 0 ? rk : 1) : total;
+}
+
 // Partial results layout: ws[((row * n_splits + split) * G + g) * 130 + {0: max, 1: sum, 2..129: output}].
 constexpr int kPartStride = 130;
 
 template <bool BF16, int G, bool INDEXED>
 __global__ __launch_bounds__(kAttThreads) void pkv_attn_partial_kernel(const void *__restrict__ q, int n_kv_heads,
                                                                        int group, AttSegs segs, int64_t total,
-                                                                       const int32_t *__restrict__ row_keys,
+                                                                       const int32_t *__restrict__ row_keys, int uniform,
                                                                        int64_t per_split, float scale_log2e,
                                                                        float *__restrict__ ws) {
   // blockIdx.z: query heads g0 .. g0 + g_count - 1 of the KV head (more than four would not fit the registers)
@@ -122,10 +140,7 @@ __global__ __launch_bounds__(kAttThreads) void pkv_attn_partial_kernel(const voi
   const int lane16 = tid & 15;        // owns dims 8*lane16 .. +7
   const int grp = tid >> 4;           // 16 key slots per workgroup step
 
-  if (row_keys) {  // ragged rows: this (b, h) attends to its first row_keys[row] keys only
-    const int64_t rk = row_keys[row];
-    total = rk < total ? (rk > 0 ? rk : 1) : total;
-  }
+  total = att_row_total(total, row_keys, row, uniform);  // ragged rows
   const int64_t j0 = (int64_t)split * per_split;
   const int64_t j1 = (j0 + per_split < total) ? j0 + per_split : total;
   // per segment: byte address of this lane's 16 bytes of "concatenated key 0" (may lie before the tensor);
@@ -349,17 +364,14 @@ __device__ __forceinline__ AttPlace<false> att_place(const AttSegs &a, int row, 
 // 8 rows x 693 attended keys 30.2 / 27.7, 8 x 1188 (4 layers) 136.5 / 124.2, 64 x 887 (2 layers) 133.4 / 122.8.
 template <bool INDEXED, typename SEGS>
 __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_kernel(
-    const void *__restrict__ q, int group, SEGS segs, int64_t total, const int32_t *__restrict__ row_keys, int64_t per_split,
-    float scale_log2e, float *__restrict__ ws) {
+    const void *__restrict__ q, int group, SEGS segs, int64_t total, const int32_t *__restrict__ row_keys, int uniform,
+    int64_t per_split, float scale_log2e, float *__restrict__ ws) {
   constexpr bool ONE = __is_same(SEGS, AttOne);
   const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int row = b * (int)gridDim.y + h;
   const int lane = threadIdx.x & (PKV_WAVE - 1), wave = threadIdx.x / PKV_WAVE;
   const int n = lane & 15, j = lane >> 4;
-  if (row_keys) {
-    const int64_t rk = row_keys[row];
-    total = rk < total ? (rk > 0 ? rk : 1) : total;
-  }
+  total = att_row_total(total, row_keys, row, uniform);
   const int64_t per_wave = per_split / kMfmaWaves;  // a multiple of the 32 keys of one step
   const int64_t j0 = (int64_t)split * per_split + (int64_t)wave * per_wave;
   const int64_t j1 = (j0 + per_wave < total) ? j0 + per_wave : total;  // j1 <= j0: nothing left for this wave
@@ -591,9 +603,9 @@ extern "C" size_t pkv_decode_attention_ws_bytes(int bs, int n_kv_heads, int grou
   return pkv_align_up((size_t)bs * n_kv_heads * 64 * group * kPartStride * sizeof(float), 256);
 }
 
-extern "C" int pkv_decode_attention(const void *q, int dtype, int bs, int n_kv_heads, int group,
-                                    const pkv_attn_segment *segments, int n_segments, const int32_t *row_keys,
-                                    float scale, void *out, void *ws, size_t ws_bytes, void *stream) {
+static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_segment *segments,
+                            int n_segments, const int32_t *row_keys, int uniform, float scale, void *out, void *ws,
+                            size_t ws_bytes, void *stream) {
   PKV_REQUIRE(q && segments && out && ws, "pkv_decode_attention: null pointer");
   PKV_REQUIRE(dtype == PKV_DTYPE_F32 || dtype == PKV_DTYPE_BF16, "unknown dtype %d", dtype);
   PKV_REQUIRE(bs > 0 && n_kv_heads > 0 && (int64_t)bs * n_kv_heads <= 65535, "bad shape bs=%d kv_heads=%d", bs,
@@ -648,7 +660,7 @@ extern "C" int pkv_decode_attention(const void *q, int dtype, int bs, int n_kv_h
     AttOne one;
 #define PKV_ATT_MFMA(IDX, S)                                                                                                    \
   hipLaunchKernelGGL((pkv_attn_partial_mfma_kernel<IDX, decltype(S)>), grid3, dim3(kMfmaWaves * PKV_WAVE), 0, s, q, group, S, total, \
-                     row_keys, per_split, scale_log2e, (float *)ws)
+                     row_keys, uniform, per_split, scale_log2e, (float *)ws)
     if (as_one_tensor(sg, one)) {
       if (indexed) PKV_ATT_MFMA(true, one); else PKV_ATT_MFMA(false, one);
     } else {
@@ -662,7 +674,7 @@ extern "C" int pkv_decode_attention(const void *q, int dtype, int bs, int n_kv_h
     grid.z = (unsigned)((group + per_wg - 1) / per_wg);
 #define PKV_ATT(GG, IDX)                                                                                                  \
   hipLaunchKernelGGL((pkv_attn_partial_kernel<false, GG, IDX>), grid, dim3(kAttThreads), 0, s, q, n_kv_heads, group, sg, \
-                     total, row_keys, per_split, scale_log2e, (float *)ws)
+                     total, row_keys, uniform, per_split, scale_log2e, (float *)ws)
 #define PKV_ATT_G(IDX)                     \
   do {                                     \
     if (per_wg == 1) PKV_ATT(1, IDX);      \
@@ -684,9 +696,15 @@ extern "C" int pkv_decode_attention(const void *q, int dtype, int bs, int n_kv_h
   return PKV_OK;
 }
 
+extern "C" int pkv_decode_attention(const void *q, int dtype, int bs, int n_kv_heads, int group,
+                                    const pkv_attn_segment *segments, int n_segments, const int32_t *row_keys,
+                                    float scale, void *out, void *ws, size_t ws_bytes, void *stream) {
+  return decode_attention(q, dtype, bs, n_kv_heads, group, segments, n_segments, row_keys, 0, scale, out, ws, ws_bytes, stream);
+}
+
 extern "C" int pkv_decode_attention_run(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_args *a,
                                         void *stream) {
   PKV_REQUIRE(a != nullptr, "pkv_decode_attention: null args");
-  return pkv_decode_attention(q, dtype, bs, n_kv_heads, group, a->segments, a->n_segments, a->row_keys, a->scale, a->out, a->ws,
-                              a->ws_bytes, stream);
+  return decode_attention(q, dtype, bs, n_kv_heads, group, a->segments, a->n_segments, a->row_keys,
+                          a->row_keys_uniform ? bs * n_kv_heads : 0, a->scale, a->out, a->ws, a->ws_bytes, stream);
 }

@@ -94,13 +94,13 @@ __device__ __forceinline__ void pkv_lut_rank_subspace(int dtype, const int32_t *
   {
     const int c = tid & 127, half = tid >> 7;
     const uint32_t mine = sm.key[c];
-    int part = 0;
+    int part = 0, part1 = 0, part2 = 0, part3 = 0;  // four chains of dependent adds (one: +0.3 us per launch)
     const pkv_u32x4 *k4 = (const pkv_u32x4 *)sm.key + half * 32;
     if (dtype == PKV_DTYPE_BF16) {
 #pragma unroll 8
       for (int c4 = 0; c4 < 32; ++c4) {
         const pkv_u32x4 k = k4[c4];
-        part += (k.x > mine) + (k.y > mine) + (k.z > mine) + (k.w > mine);
+        part += (k.x > mine), part1 += (k.y > mine), part2 += (k.z > mine), part3 += (k.w > mine);
       }
     } else {
 #pragma unroll 8
@@ -108,11 +108,12 @@ __device__ __forceinline__ void pkv_lut_rank_subspace(int dtype, const int32_t *
         const pkv_u32x4 k = k4[c4];
         const int o = half * 128 + 4 * c4;
         part += (k.x > mine || (k.x == mine && o + 0 < c)) ? 1 : 0;
-        part += (k.y > mine || (k.y == mine && o + 1 < c)) ? 1 : 0;
-        part += (k.z > mine || (k.z == mine && o + 2 < c)) ? 1 : 0;
-        part += (k.w > mine || (k.w == mine && o + 3 < c)) ? 1 : 0;
+        part1 += (k.y > mine || (k.y == mine && o + 1 < c)) ? 1 : 0;
+        part2 += (k.z > mine || (k.z == mine && o + 2 < c)) ? 1 : 0;
+        part3 += (k.w > mine || (k.w == mine && o + 3 < c)) ? 1 : 0;
       }
     }
+    part += part1 + part2 + part3;
     if (half) sm.part[c] = part;
     __syncthreads();
     if (!half) {

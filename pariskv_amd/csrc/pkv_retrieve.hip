@@ -347,9 +347,8 @@ extern "C" int pkv_decode_step(const pkv_retrieve_args *retrieve, void *ws, size
   PKV_REQUIRE(retrieve && attention, "pkv_decode_step: null args");
   int rc = pkv_retrieve(retrieve, ws, ws_bytes, stream);
   if (rc) return rc;
-  return pkv_decode_attention(retrieve->q, retrieve->dtype, retrieve->bs, retrieve->n_kv_heads, retrieve->group,
-                              attention->segments, attention->n_segments, attention->row_keys, attention->scale,
-                              attention->out, attention->ws, attention->ws_bytes, stream);
+  return pkv_decode_attention_run(retrieve->q, retrieve->dtype, retrieve->bs, retrieve->n_kv_heads, retrieve->group, attention,
+                                  stream);
 }
 
 extern "C" int pkv_adaptive_decode_step(const pkv_retrieve_args *retrieve, void *ws, size_t ws_bytes,
@@ -402,7 +401,6 @@ extern "C" int pkv_adaptive_decode_step(const pkv_retrieve_args *retrieve, void 
                                ad->row_bytes, stream);
     if (rc) return rc;
   }
-  return pkv_decode_attention(retrieve->q, retrieve->dtype, retrieve->bs, retrieve->n_kv_heads, retrieve->group,
-                              attention->segments, attention->n_segments, attention->row_keys, attention->scale,
-                              attention->out, attention->ws, attention->ws_bytes, stream);
+  return pkv_decode_attention_run(retrieve->q, retrieve->dtype, retrieve->bs, retrieve->n_kv_heads, retrieve->group, attention,
+                                  stream);
 }

@@ -1028,7 +1028,8 @@ class RetrievePlan:
         elements), row_keys int32 [bs,H], row_keys_base, optional uniform_k int64 [bs,H] (then every row gathers and
         attends to max(adaptive_k) ids), ws uint8 (pkv_adaptive_topk_ws_bytes), src_k / src_v pinned
         CPU [bs,H,len,128], dst_k / dst_v GPU [bs,H,>=k_out,128] (all four None: no gather, ``segments`` name the selected
-        rows by topk_ids); optional dense_vnorm_run (like dense_logits) with dense_split and dense_row1: dense tokens from
+        rows by topk_ids); row_keys_uniform: the attention (without a gather) takes
+        the largest row's count for all rows; optional dense_vnorm_run (like dense_logits) with dense_split and dense_row1: dense tokens from
         dense_split on are the rows from dense_row1 on.  ``segments`` are the attention's; its per-row key
         count is ``row_keys``."""
         d = adaptive
@@ -1092,6 +1093,7 @@ class RetrievePlan:
                   "the second run of dense rows exceeds dense_k / dense_vnorm")
             ad.dense_split, ad.dense_row1, ad.dense_vnorm_run = split, row1, run.data_ptr()
         aa, _ = att.c_args(queries, segments, out=queries, row_keys=rk)  # out is patched at every launch
+        aa.row_keys_uniform = int(bool(d.get("row_keys_uniform", False)))
         keep = (signs, centers, cluster_counts, codes_km, nib_km, w_km, d, att, segments, self.ws)
         return BoundAdaptiveStep(self, a, ad, aa, keep, queries)
 
