@@ -68,7 +68,10 @@ __global__ __launch_bounds__(kScanThreads) void pkv_scan_keymajor_kernel(
     int32_t *__restrict__ cnt_i32, uint32_t *__restrict__ row_suf, uint16_t *__restrict__ chunk_suf, int chunk_keys,
     int sub_blocks) {
   const int row = blockIdx.y;
-  const int chunk = blockIdx.x;
+  // Workgroups go to the eight dies in turn.  Rows start at another chunk each, so that the chunks that hold most of the
+  // candidates (the ones near the queries, the same in every row) do not all meet on one die: 64 rows x 16 chunks, two layers,
+  // 115.8 -> 114.6 us with the select + rerank doing the same.
+  const int chunk = (int)((blockIdx.x + blockIdx.y) % gridDim.x);
   const int n_chunks = gridDim.x;
   const int b = row / n_kv_heads, h = row % n_kv_heads;
   const int tid = threadIdx.x;

@@ -102,7 +102,7 @@ __global__ __launch_bounds__(kSelThreads) void pkv_select_rerank_kernel(
     const float *__restrict__ centers, int64_t *__restrict__ out, float *__restrict__ scores, int extra_off,
     float *__restrict__ extra_out, uint32_t *__restrict__ range_slots, int64_t range_row_stride) {
   const int row = blockIdx.y;
-  const int chunk = blockIdx.x;
+  const int chunk = (int)((blockIdx.x + blockIdx.y) % gridDim.x);  // see pkv_scan_keymajor_kernel
   const int tid = threadIdx.x;
   const int b = row / n_kv_heads, h = row % n_kv_heads;
   uint32_t smax = 0u, smin = 0xffffffffu;  // ordered bits of the largest / smallest score this thread wrote
@@ -1064,12 +1064,23 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_sort_kernel(
   const int tid = threadIdx.x;
   const float *xr = x + (int64_t)row * x_stride;
   const int64_t *ir = ids ? ids + (int64_t)row * ids_stride : nullptr;
+  // The ids are two thirds of the bytes and needed only once the bins are known: they stay in flight until then (waiting
+  // for them with the scores: +0.6 us a launch at 8 rows x 3220 candidates, +0.85 at 64 x 6497).  v: score bits over a one, zero past the row's end.
   uint64_t v[EIN];
+  uint32_t id[EIN], score[EIN];
 #pragma unroll
   for (int e = 0; e < EIN; ++e) {
     const int i = tid + e * kTopkThreads;
-    v[e] = i < len ? make_key(xr, ir, i) : 0ull;
+    score[e] = __float_as_uint(xr[i < len ? i : len - 1]);
   }
+#pragma unroll
+  for (int e = 0; e < EIN; ++e) {
+    const int i = tid + e * kTopkThreads;
+    id[e] = ir ? (uint32_t)ir[i < len ? i : len - 1] : (uint32_t)i;
+  }
+#pragma unroll
+  for (int e = 0; e < EIN; ++e)
+    v[e] = tid + e * kTopkThreads < len ? ((uint64_t)pkv_ordered_u32(__uint_as_float(score[e])) << 32) | 1ull : 0ull;
   if (tid == 0) s_counter = 0;
   if (SORTED)
     for (int i = tid; i < (P < 1024 ? 1024 : P); i += kTopkThreads) s_keys[i] = 0ull;
@@ -1077,6 +1088,9 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_sort_kernel(
   uint32_t bin[EIN];
   LinSel L;
   const bool lin = linear_bins<EIN>(v, (uint32_t)k, s_hist, s_cnt, s_bcast, bin, L);  // uniform over the workgroup
+#pragma unroll
+  for (int e = 0; e < EIN; ++e)  // the whole keys
+    if (v[e] != 0ull) v[e] = (v[e] & 0xffffffff00000000ull) | (uint64_t)(uint32_t)~id[e];
   int64_t *oi = out_ids + (int64_t)row * k;
   float *ov = out_vals ? out_vals + (int64_t)row * k : nullptr;
   if (SORTED && lin && L.max_winners <= kLinRankMax) {
