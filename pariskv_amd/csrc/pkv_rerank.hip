@@ -80,13 +80,19 @@ __global__ __launch_bounds__(kRerankThreads) void pkv_rerank_kernel(
       if (V4B) store_v4b(v4b, row, n_cand, i, blk, s_val, words[blk]);
     }
   } else {
-#pragma unroll 4
+    // all 32 loads in flight before the first product: 16 rows x 4003 of 20011 keys 16.0 -> 14.3 us; bound by the lines it
+    // touches (every line of the index at one key in five) and the unpacked values, 47 MB
+    uint32_t words[16], wbits[16];
+#pragma unroll
+    for (int blk = 0; blk < 16; ++blk) words[blk] = *(const uint32_t *)(nrow + key * ns_key + (int64_t)blk * ns_sub);
+#pragma unroll
+    for (int blk = 0; blk < 16; ++blk) wbits[blk] = wrow[key * ws_key + (int64_t)blk * ws_sub];
+#pragma unroll
     for (int blk = 0; blk < 16; ++blk) {
-      const uint32_t word = *(const uint32_t *)(nrow + key * ns_key + (int64_t)blk * ns_sub);
-      const float t = pkv_block_dot(s_prod, blk, word);
-      const float tw = t * pkv_bf16_bits_to_f32(wrow[key * ws_key + (int64_t)blk * ws_sub]);
+      const float t = pkv_block_dot(s_prod, blk, words[blk]);
+      const float tw = t * pkv_bf16_bits_to_f32(wbits[blk]);
       s = (blk == 0) ? tw : s + tw;
-      if (V4B) store_v4b(v4b, row, n_cand, i, blk, s_val, word);
+      if (V4B) store_v4b(v4b, row, n_cand, i, blk, s_val, words[blk]);
     }
   }
   *out = s * qnorm[row];

@@ -373,6 +373,23 @@ def test_bucket_and_radix_topk_on_counts(ops, rows, L, k):
         assert np.array_equal(np.sort(x[r][out_b[r]]), np.sort(tv))
 
 
+@pytest.mark.parametrize("rows,N,k", [(1, 3, 1), (1, 255, 128), (2, 1026, 500), (8, 9001, 4000), (8, 20005, 20004), (33, 70003, 7000)])
+def test_subspace_major_votes_and_coarse_filter_at_every_chunk_size(ops, rows, N, k):
+    """Votes of a subspace-major codebook, four keys to a thread (rows of odd length: unaligned runs, one to three keys
+    left over), and the coarse filter with 1, 4, 8 and 16 counts to a thread: whole numbers, exact."""
+    from pariskv_amd.cache_hub.collision_fused import update_cache_cnt_cuda_interface
+
+    _say(f"submajor votes rows={rows} N={N} k={k}")
+    ids, counts, codebook = _collision_recipe(1, rows, N)
+    tiers = O.tier_counts(N, 0.3)
+    cnt = update_cache_cnt_cuda_interface(ids.to(DEV), counts.to(DEV), codebook.to(DEV), tiers)
+    out = ops.bucket_topk(cnt.view(rows, N), k).cpu().numpy()
+    for r in range(rows):
+        ref = O.collision_count(np.ascontiguousarray(codebook[0, r].numpy().T), O.tier_lut(ids[0, r].numpy(), counts[0, r].numpy(), tiers))
+        assert np.array_equal(cnt[0, r].cpu().numpy(), ref)
+        assert np.array_equal(out[r], O.select_candidates(ref, k)[0])
+
+
 def test_bucket_topk_all_equal_and_clamp(ops):
     x = torch.full((2, 3000), 7, dtype=torch.int32, device=DEV)
     assert torch.equal(ops.bucket_topk(x, 50).cpu(), torch.arange(50).expand(2, 50))
