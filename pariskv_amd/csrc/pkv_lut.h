@@ -103,14 +103,35 @@ __device__ __forceinline__ void pkv_lut_rank_subspace(int dtype, const int32_t *
         part += (k.x > mine), part1 += (k.y > mine), part2 += (k.z > mine), part3 += (k.w > mine);
       }
     } else {
+      // "ahead" is k > mine, and from smaller ids also k == mine.  A wave's 64 centroids lie in one block of 64 ids, so of
+      // the two blocks a thread counts over, only the wave's own needs the ids compared key by key (all of them: +0.6 us a launch
+      // at 12 rows, 7.7 against 7.1).
+      const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), c0 = (wave & 1) * 64, o_half = (wave >> 1) * 128;
+      for (int o0 = o_half; o0 < o_half + 128; o0 += 64) {
+        const pkv_u32x4 *kb = (const pkv_u32x4 *)sm.key + o0 / 4;
+        if (o0 > c0) {
+#pragma unroll
+          for (int c4 = 0; c4 < 16; ++c4) {
+            const pkv_u32x4 k = kb[c4];
+            part += (k.x > mine), part1 += (k.y > mine), part2 += (k.z > mine), part3 += (k.w > mine);
+          }
+        } else if (o0 < c0) {
+#pragma unroll
+          for (int c4 = 0; c4 < 16; ++c4) {
+            const pkv_u32x4 k = kb[c4];
+            part += (k.x >= mine), part1 += (k.y >= mine), part2 += (k.z >= mine), part3 += (k.w >= mine);
+          }
+        } else {
 #pragma unroll 8
-      for (int c4 = 0; c4 < 32; ++c4) {
-        const pkv_u32x4 k = k4[c4];
-        const int o = half * 128 + 4 * c4;
-        part += (k.x > mine || (k.x == mine && o + 0 < c)) ? 1 : 0;
-        part1 += (k.y > mine || (k.y == mine && o + 1 < c)) ? 1 : 0;
-        part2 += (k.z > mine || (k.z == mine && o + 2 < c)) ? 1 : 0;
-        part3 += (k.w > mine || (k.w == mine && o + 3 < c)) ? 1 : 0;
+          for (int c4 = 0; c4 < 16; ++c4) {
+            const pkv_u32x4 k = kb[c4];
+            const int o = o0 + 4 * c4;
+            part += (k.x > mine || (k.x == mine && o + 0 < c)) ? 1 : 0;
+            part1 += (k.y > mine || (k.y == mine && o + 1 < c)) ? 1 : 0;
+            part2 += (k.z > mine || (k.z == mine && o + 2 < c)) ? 1 : 0;
+            part3 += (k.w > mine || (k.w == mine && o + 3 < c)) ? 1 : 0;
+          }
+        }
       }
     }
     part += part1 + part2 + part3;

@@ -220,6 +220,23 @@ def test_query_prep_lut_bit_exact(ops, request, wl_name):
         assert np.array_equal(lut[b, h].cpu().numpy(), st["lut"])
 
 
+def test_query_prep_fp32_ranks_of_equal_scores(ops, wl_cfg1):
+    """One-hot fp32 queries rotate into components of one magnitude, so that the 256 centroids of a subspace share nine scores:
+    the ranks are decided by the ids, inside a wave's block of 64 ids and across blocks."""
+    w = wl_cfg1
+    signs = torch.from_numpy(np.ascontiguousarray(w.signs)).to(DEV)
+    q = torch.zeros(1, 8, 128)
+    for h in range(6):
+        q[0, h, 23 * h] = 1.0 if h % 2 else -3.0
+    q[0, 6] = torch.arange(128).remainder(4) - 1.5
+    q[0, 7] = torch.randn(128, generator=torch.Generator().manual_seed(5))
+    counts = torch.ones(1, 8, 16, 256, dtype=torch.int32, device=DEV)
+    ids = ops.query_prep_lut(q.to(DEV), 8, signs, counts, [100], True)[3].cpu().numpy()
+    for h in range(8):
+        qh, _ = O.query_prep(q[0, h].numpy(), w.signs, O.F32)
+        assert np.array_equal(ids[0, h], O.rank_centroids(qh, O.F32))
+
+
 def test_query_prep_single_tier_and_group1(ops, wl_cfg1):
     w = wl_cfg1
     d = W.to_device(w, DEV, torch)
