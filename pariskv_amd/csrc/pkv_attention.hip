@@ -123,12 +123,77 @@ __device__ __forceinline__ int64_t att_row_total(int64_t total, const int32_t *_
   return rk < total ? (rk > 0 ? rk : 1) : total;
 }
 
+// Segments that share one K and one V tensor (the cache's rows in HBM: sink, selected rows, local window), at most one of
+// them indexed: a key is a 32-bit byte offset into the (b, h) slab.  Half of a launch over a few hundred keys used to go
+// into finding addresses (1.2 us to pick a 64-bit pointer out of four for each of a lane's ten rows, after 1 us for a
+// 300-byte argument block); here that is one lane exchange per row.
+struct AttOne {
+  const char *k, *v;
+  int64_t stride_b, stride_h;           // bytes
+  uint32_t end[PKV_ATTN_MAX_SEGMENTS];  // exclusive ends in the concatenated key order; unused: 2^32 - 1
+  int32_t delta[PKV_ATTN_MAX_SEGMENTS]; // row - concatenated key
+  const int64_t *idx;                   // of the indexed segment, keys [idx_lo, idx_hi)
+  int64_t idx_stride, idx_limit;
+  uint32_t idx_lo, idx_hi, idx_row0;
+};
+
+// One key's place: a byte offset into the slab (AttOne), or the addresses of its K and V rows.
+template <bool ONE>
+struct AttPlace {
+  uint32_t off;
+  __device__ __forceinline__ AttPlace from(int lane) const { return {(uint32_t)__shfl((int)off, lane, PKV_WAVE)}; }
+};
+template <>
+struct AttPlace<false> {
+  uint64_t k, v;
+  __device__ __forceinline__ const char *k_from(int lane) const { return (const char *)pull(k, lane); }
+  __device__ __forceinline__ const char *v_from(int lane) const { return (const char *)pull(v, lane); }
+  static __device__ __forceinline__ uint64_t pull(uint64_t x, int lane) {
+    return ((uint64_t)(uint32_t)__shfl((int)(x >> 32), lane, PKV_WAVE) << 32) | (uint32_t)__shfl((int)(uint32_t)x, lane, PKV_WAVE);
+  }
+};
+
+// ROW: bytes of a row.
+template <bool INDEXED, uint32_t ROW>
+__device__ __forceinline__ AttPlace<true> att_place(const AttOne &a, int row, int, int, uint32_t jj) {
+  int32_t d = a.delta[0];
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t) d = jj >= a.end[t - 1] ? a.delta[t] : d;
+  uint32_t r = jj + (uint32_t)d;
+  if (INDEXED && jj >= a.idx_lo && jj < a.idx_hi) {
+    const int64_t x = a.idx[(int64_t)row * a.idx_stride + (jj - a.idx_lo)];
+    r = a.idx_row0 + (uint32_t)(x < 0 ? 0 : (x >= a.idx_limit ? a.idx_limit - 1 : x));
+  }
+  return {r * ROW};
+}
+
+template <bool INDEXED, uint32_t ROW>
+__device__ __forceinline__ AttPlace<false> att_place(const AttSegs &a, int row, int b, int h, uint32_t jj) {
+  int s = 0;
+  uint32_t first = 0;
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (t < a.n && jj >= (uint32_t)a.end[t - 1]) s = t, first = (uint32_t)a.end[t - 1];
+  const char *k = (const char *)a.k[0], *v = (const char *)a.v[0];
+  int64_t sb = a.stride_b[0], sh = a.stride_h[0], row0 = a.row0[0];
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (s == t) k = (const char *)a.k[t], v = (const char *)a.v[t], sb = a.stride_b[t], sh = a.stride_h[t], row0 = a.row0[t];
+  const int64_t r = INDEXED ? (int64_t)(att_resolve_row(a, row, jj) & 0x1fffffffu) : row0 + (int64_t)(jj - first);
+  const int64_t off = ((int64_t)b * sb + (int64_t)h * sh) * (ROW / 128) + r * ROW;
+  return {(uint64_t)(k + off), (uint64_t)(v + off)};
+}
+
 // Partial results layout: ws[((row * n_splits + split) * G + g) * 130 + {0: max, 1: sum, 2..129: output}].
 constexpr int kPartStride = 130;
 
-template <bool BF16, int G, bool INDEXED>
+// Splits are of 64 keys while the key set allows: a launch is one chain of dependent loads with some 1000 instructions behind
+// it, not bandwidth.  Places of keys as in the bf16 kernel below.  Decode step, us, with a 64-bit pointer picked out of four for
+// each row / with places: 12 rows x 865 attended keys, 7 heads (2 layers) 74.6 / 70.0, 8 rows x 696 (2 layers) 66.5 / 61.0,
+// 32 rows x 896 48.6 / 45.2.
+template <bool BF16, int G, bool INDEXED, typename SEGS>
 __global__ __launch_bounds__(kAttThreads) void pkv_attn_partial_kernel(const void *__restrict__ q, int n_kv_heads,
-                                                                       int group, AttSegs segs, int64_t total,
+                                                                       int group, SEGS segs, int64_t total,
                                                                        const int32_t *__restrict__ row_keys, int uniform,
                                                                        int64_t per_split, float scale_log2e,
                                                                        float *__restrict__ ws) {
@@ -143,42 +208,39 @@ __global__ __launch_bounds__(kAttThreads) void pkv_attn_partial_kernel(const voi
   total = att_row_total(total, row_keys, row, uniform);  // ragged rows
   const int64_t j0 = (int64_t)split * per_split;
   const int64_t j1 = (j0 + per_split < total) ? j0 + per_split : total;
-  // per segment: byte address of this lane's 16 bytes of "concatenated key 0" (may lie before the tensor);
-  // with indexed segments: of row 0 of the (b, h) slab
-  const int esz = BF16 ? 2 : 4;
-  const char *kb[PKV_ATTN_MAX_SEGMENTS], *vb[PKV_ATTN_MAX_SEGMENTS];
-#pragma unroll
-  for (int s = 0; s < PKV_ATTN_MAX_SEGMENTS; ++s) {
-    const int64_t first = s == 0 ? 0 : segs.end[s - 1];
-    const int64_t off = ((int64_t)b * segs.stride_b[s] + (int64_t)h * segs.stride_h[s] +
-                         (INDEXED ? 0 : (segs.row0[s] - first) * 128) + 8 * lane16) * esz;
-    kb[s] = (const char *)segs.k[s] + off;
-    vb[s] = (const char *)segs.v[s] + off;
+  constexpr bool ONE = __is_same(SEGS, AttOne);
+  constexpr uint32_t kRow = BF16 ? 256 : 512;
+  const int lane = tid & (PKV_WAVE - 1), wave = tid / PKV_WAVE;
+  const char *kbase = nullptr, *vbase = nullptr;
+  if constexpr (ONE) {
+    const int64_t slab = (int64_t)b * segs.stride_b + (int64_t)h * segs.stride_h;
+    kbase = segs.k + slab, vbase = segs.v + slab;
   }
   // K/V rows of the step after the current one are requested before the current one is consumed
   float kx[kAttUnroll][8], vx[kAttUnroll][8];
   Raw8<BF16> kn[kAttUnroll], vn[kAttUnroll];
+  AttPlace<ONE> mine;
   auto fetch = [&](int64_t jb, Raw8<BF16> (&kd)[kAttUnroll], Raw8<BF16> (&vd)[kAttUnroll]) {
+    // four turns (64 keys) at a time: lane 4 t + i (mod 16) finds the place of the key that the wave's lanes 16 i .. 16 i + 15
+    // read in turn t
+    static_assert(4 % kAttUnroll == 0 && kAttKeysPerIter == 16, "a wave reads four keys in a turn");
+    const int turn = ((int)(jb - j0) / kAttKeysPerIter) & 3;
+    if (turn == 0) {
+      const int64_t key = jb + ((lane >> 2) & 3) * kAttKeysPerIter + 4 * wave + (lane & 3);
+      mine = att_place<INDEXED, kRow>(segs, row, b, h, (uint32_t)(key < j1 ? key : j1 - 1));  // fewer than 2^24 keys
+    }
 #pragma unroll
     for (int u = 0; u < kAttUnroll; ++u) {
-      const int64_t j = jb + u * kAttKeysPerIter + grp;
-      const uint32_t jj = (uint32_t)(j < j1 ? j : j1 - 1);  // fewer than 2^24 keys
-      const char *kp = kb[0], *vp = vb[0];
-      uint32_t rownum = jj;
-      if (INDEXED) {
-        const uint32_t packed = att_resolve_row(segs, row, jj);
-        rownum = packed & 0x1fffffffu;
-#pragma unroll
-        for (int s = 1; s < PKV_ATTN_MAX_SEGMENTS; ++s)
-          if ((packed >> 29) == (uint32_t)s) kp = kb[s], vp = vb[s];
+      const int at = 4 * (turn + u) + (lane >> 4);
+      const char *kp, *vp;
+      if constexpr (ONE) {
+        const uint64_t off = mine.from(at).off + (kRow / 16) * (uint32_t)lane16;
+        kp = kbase + off, vp = vbase + off;
       } else {
-#pragma unroll
-        for (int s = 1; s < PKV_ATTN_MAX_SEGMENTS; ++s)
-          if (s < segs.n && jj >= (uint32_t)segs.end[s - 1]) kp = kb[s], vp = vb[s];
+        kp = mine.k_from(at) + (kRow / 16) * lane16, vp = mine.v_from(at) + (kRow / 16) * lane16;
       }
-      const uint64_t boff = (uint64_t)rownum * (uint32_t)(128 * esz);
-      load_raw8<BF16>(kp + boff, 0, kd[u]);
-      load_raw8<BF16>(vp + boff, 0, vd[u]);
+      load_raw8<BF16>(kp, 0, kd[u]);
+      load_raw8<BF16>(vp, 0, vd[u]);
     }
   };
   if (j0 < j1) fetch(j0, kn, vn);  // before the queries: nothing here waits for them
@@ -300,66 +362,6 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
 
 constexpr int kMfmaWaves = 4;  // waves per workgroup: each takes a quarter of the split, merged through LDS
 
-// Segments that share one K and one V tensor (the cache's rows in HBM: sink, selected rows, local window), at most one of
-// them indexed: a key is a 32-bit byte offset into the (b, h) slab.  Half of a launch over a few hundred keys used to go
-// into finding addresses (1.2 us to pick a 64-bit pointer out of four for each of a lane's ten rows, after 1 us for a
-// 300-byte argument block); here that is one lane exchange per row.
-struct AttOne {
-  const char *k, *v;
-  int64_t stride_b, stride_h;           // bytes
-  uint32_t end[PKV_ATTN_MAX_SEGMENTS];  // exclusive ends in the concatenated key order; unused: 2^32 - 1
-  int32_t delta[PKV_ATTN_MAX_SEGMENTS]; // row - concatenated key
-  const int64_t *idx;                   // of the indexed segment, keys [idx_lo, idx_hi)
-  int64_t idx_stride, idx_limit;
-  uint32_t idx_lo, idx_hi, idx_row0;
-};
-
-// One key's place: a byte offset into the slab (AttOne), or the addresses of its K and V rows.
-template <bool ONE>
-struct AttPlace {
-  uint32_t off;
-  __device__ __forceinline__ AttPlace from(int lane) const { return {(uint32_t)__shfl((int)off, lane, PKV_WAVE)}; }
-};
-template <>
-struct AttPlace<false> {
-  uint64_t k, v;
-  __device__ __forceinline__ const char *k_from(int lane) const { return (const char *)pull(k, lane); }
-  __device__ __forceinline__ const char *v_from(int lane) const { return (const char *)pull(v, lane); }
-  static __device__ __forceinline__ uint64_t pull(uint64_t x, int lane) {
-    return ((uint64_t)(uint32_t)__shfl((int)(x >> 32), lane, PKV_WAVE) << 32) | (uint32_t)__shfl((int)(uint32_t)x, lane, PKV_WAVE);
-  }
-};
-
-template <bool INDEXED>
-__device__ __forceinline__ AttPlace<true> att_place(const AttOne &a, int row, int, int, uint32_t jj) {
-  int32_t d = a.delta[0];
-#pragma unroll
-  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t) d = jj >= a.end[t - 1] ? a.delta[t] : d;
-  uint32_t r = jj + (uint32_t)d;
-  if (INDEXED && jj >= a.idx_lo && jj < a.idx_hi) {
-    const int64_t x = a.idx[(int64_t)row * a.idx_stride + (jj - a.idx_lo)];
-    r = a.idx_row0 + (uint32_t)(x < 0 ? 0 : (x >= a.idx_limit ? a.idx_limit - 1 : x));
-  }
-  return {r * 256u};
-}
-
-template <bool INDEXED>
-__device__ __forceinline__ AttPlace<false> att_place(const AttSegs &a, int row, int b, int h, uint32_t jj) {
-  int s = 0;
-  uint32_t first = 0;
-#pragma unroll
-  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
-    if (t < a.n && jj >= (uint32_t)a.end[t - 1]) s = t, first = (uint32_t)a.end[t - 1];
-  const char *k = (const char *)a.k[0], *v = (const char *)a.v[0];
-  int64_t sb = a.stride_b[0], sh = a.stride_h[0], row0 = a.row0[0];
-#pragma unroll
-  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
-    if (s == t) k = (const char *)a.k[t], v = (const char *)a.v[t], sb = a.stride_b[t], sh = a.stride_h[t], row0 = a.row0[t];
-  const int64_t r = INDEXED ? (int64_t)(att_resolve_row(a, row, jj) & 0x1fffffffu) : row0 + (int64_t)(jj - first);
-  const int64_t off = ((int64_t)b * sb + (int64_t)h * sh) * 2 + r * 256;
-  return {(uint64_t)(k + off), (uint64_t)(v + off)};
-}
-
 // grid (splits, KV heads, batch).  Decode step, us, with four-way pointer selection per row / with places by lane exchange:
 // 8 rows x 693 attended keys 30.2 / 27.7, 8 x 1188 (4 layers) 136.5 / 124.2, 64 x 887 (2 layers) 133.4 / 122.8.
 template <bool INDEXED, typename SEGS>
@@ -386,7 +388,7 @@ __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_k
   }
   auto place_block = [&](int64_t jb) {
     const int64_t key = jb + lane;
-    mine = att_place<INDEXED>(segs, row, b, h, (uint32_t)(key < j1 ? key : j1 - 1));
+    mine = att_place<INDEXED, 256>(segs, row, b, h, (uint32_t)(key < j1 ? key : j1 - 1));
   };
   if (j0 < j1) place_block(j0);  // before the queries: the indices' latency is the longer one
 
@@ -571,18 +573,18 @@ int pick_splits_mfma(int rows, int64_t total) {
 }
 
 // The segments as offsets into one (b, h) slab: false where they lie in different tensors, more than one is indexed or a
-// row's byte offset would not fit 32 bits (2^24 rows of 256 bytes).
-bool as_one_tensor(const AttSegs &sg, AttOne &one) {
+// row's byte offset would not fit 32 bits (2^24 rows of 256 bytes, 2^23 of 512).
+bool as_one_tensor(const AttSegs &sg, int es, AttOne &one) {
   memset(&one, 0, sizeof one);
   one.k = (const char *)sg.k[0], one.v = (const char *)sg.v[0];
-  one.stride_b = sg.stride_b[0] * 2, one.stride_h = sg.stride_h[0] * 2;
+  one.stride_b = sg.stride_b[0] * es, one.stride_h = sg.stride_h[0] * es;
   for (int i = 0; i < PKV_ATTN_MAX_SEGMENTS; ++i) one.end[i] = 0xffffffffu;
   int64_t first = 0;
   for (int i = 0; i < sg.n; ++i) {
     if (sg.k[i] != sg.k[0] || sg.v[i] != sg.v[0] || sg.stride_b[i] != sg.stride_b[0] || sg.stride_h[i] != sg.stride_h[0])
       return false;
     const int64_t n = sg.end[i] - first, rows = sg.row0[i] + (sg.idx[i] ? sg.idx_limit[i] : n);
-    if (rows > ((int64_t)1 << 24)) return false;
+    if (rows > ((int64_t)1 << 32) / (128 * es)) return false;
     one.end[i] = (uint32_t)sg.end[i];
     one.delta[i] = (int32_t)(sg.row0[i] - first);
     if (sg.idx[i]) {
@@ -655,13 +657,14 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
   const float scale_log2e = scale * 1.4426950408889634f;
   hipStream_t s = (hipStream_t)stream;
   dim3 grid((unsigned)n_splits, (unsigned)rows);
+  AttOne one;
+  const bool is_one = as_one_tensor(sg, bf ? 2 : 4, one);
   if (bf) {
     const dim3 grid3((unsigned)n_splits, (unsigned)n_kv_heads, (unsigned)bs);
-    AttOne one;
 #define PKV_ATT_MFMA(IDX, S)                                                                                                    \
   hipLaunchKernelGGL((pkv_attn_partial_mfma_kernel<IDX, decltype(S)>), grid3, dim3(kMfmaWaves * PKV_WAVE), 0, s, q, group, S, total, \
                      row_keys, uniform, per_split, scale_log2e, (float *)ws)
-    if (as_one_tensor(sg, one)) {
+    if (is_one) {
       if (indexed) PKV_ATT_MFMA(true, one); else PKV_ATT_MFMA(false, one);
     } else {
       if (indexed) PKV_ATT_MFMA(true, sg); else PKV_ATT_MFMA(false, sg);
@@ -672,16 +675,20 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
     // heads, 2 x 8.0 us as two launches one after the other; the decode step around it (9001 keys) 48.3 -> 43 us.
     const int per_wg = group == 1 ? 1 : group == 2 ? 2 : 4;
     grid.z = (unsigned)((group + per_wg - 1) / per_wg);
-#define PKV_ATT(GG, IDX)                                                                                                  \
-  hipLaunchKernelGGL((pkv_attn_partial_kernel<false, GG, IDX>), grid, dim3(kAttThreads), 0, s, q, n_kv_heads, group, sg, \
-                     total, row_keys, uniform, per_split, scale_log2e, (float *)ws)
-#define PKV_ATT_G(IDX)                     \
-  do {                                     \
-    if (per_wg == 1) PKV_ATT(1, IDX);      \
-    else if (per_wg == 2) PKV_ATT(2, IDX); \
-    else PKV_ATT(4, IDX);                  \
+#define PKV_ATT(GG, IDX, S)                                                                                               \
+  hipLaunchKernelGGL((pkv_attn_partial_kernel<false, GG, IDX, decltype(S)>), grid, dim3(kAttThreads), 0, s, q, n_kv_heads, group, \
+                     S, total, row_keys, uniform, per_split, scale_log2e, (float *)ws)
+#define PKV_ATT_G(IDX, S)                     \
+  do {                                        \
+    if (per_wg == 1) PKV_ATT(1, IDX, S);      \
+    else if (per_wg == 2) PKV_ATT(2, IDX, S); \
+    else PKV_ATT(4, IDX, S);                  \
   } while (0)
-    if (indexed) PKV_ATT_G(true); else PKV_ATT_G(false);
+    if (is_one) {
+      if (indexed) PKV_ATT_G(true, one); else PKV_ATT_G(false, one);
+    } else {
+      if (indexed) PKV_ATT_G(true, sg); else PKV_ATT_G(false, sg);
+    }
 #undef PKV_ATT_G
 #undef PKV_ATT
   }

@@ -1788,6 +1788,36 @@ def test_decode_attention_places_of_keys(ops, same_tensor, lens, indexed):
     assert (out.double() - ref).abs().max().item() < 2e-2
 
 
+@pytest.mark.parametrize("same_tensor", [True, False])
+@pytest.mark.parametrize("lens,indexed", [((1,), ()), ((1, 31, 1), (1,)), ((5, 64, 33), (1,)), ((63, 1, 64, 3), (3,)), ((20, 40, 17), (0, 2)),
+                                          ((9000,), ()), ((40, 8300), (1,))])
+def test_decode_attention_fp32_places_of_keys(ops, same_tensor, lens, indexed):
+    """The same for fp32 rows, whose places are found for 64 keys of a workgroup at a time."""
+    bs, H, group = 2, 3, 5
+    g = torch.Generator(device=DEV).manual_seed(sum(lens) + 2 * len(indexed) + same_tensor)
+    rows = max(lens) + 50
+    pool = [[torch.randn(bs, H, rows, 128, generator=g, device=DEV) for _ in range(2)] for _ in lens]
+    q = torch.randn(bs, 1, H * group, 128, generator=g, device=DEV)
+    segs, K, V = [], [], []
+    for i, n in enumerate(lens):
+        k, v = pool[0 if same_tensor else i]
+        row0 = 7 + 3 * i
+        if i in indexed:
+            idx = torch.randint(0, rows - row0, (bs, H, n + 2), generator=g, device=DEV)
+            segs.append((k, v, row0, n, idx))
+            at = (idx[:, :, :n] + row0)[..., None].expand(-1, -1, -1, 128)
+            K.append(k.gather(2, at)), V.append(v.gather(2, at))
+        else:
+            segs.append((k, v, row0, n))
+            K.append(k[:, :, row0:row0 + n]), V.append(v[:, :, row0:row0 + n])
+    out = ops.DecodeAttention(bs, H, group, sum(lens), DEV).run(q, segs)
+    K, V = torch.cat(K, dim=2).double(), torch.cat(V, dim=2).double()
+    p = torch.softmax(q.double().view(bs, H, group, 128) @ K.transpose(2, 3).contiguous() / math.sqrt(128), dim=-1)
+    ref = (p @ V).view(bs, 1, H * group, 128)
+    # a score's 128 products and a result's weighted mean, each rounded at 2^-24: a few 1e-6 of values up to ~4.5
+    assert (out.double() - ref).abs().max().item() < 2e-5
+
+
 @pytest.mark.parametrize("rows,n,k", [(1, 300, 150), (8, 3520, 1760), (8, 6000, 3), (8, 32000, 3200), (16, 20001, 4001),
                                       (64, 40000, 4000), (32, 70001, 7000)])
 def test_select_rerank_at_every_chunk_size(ops, rows, n, k):
