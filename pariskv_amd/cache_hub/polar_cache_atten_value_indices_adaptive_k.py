@@ -84,11 +84,13 @@ class polar_cache(_adaptive_base):
             return _polar_cache_base.compute(self, queries, layer_idx)  # dense branch
         q = queries if queries.is_contiguous() else queries.contiguous()
         step = self._adaptive_bound[layer_idx]
-        if step is None or step[0] != n_keys:
+        if step is None or step[0] != n_keys or step[3] != self.adaptive_topk_max_k:
             step = self._bind_adaptive_step(layer_idx, q, n_keys)
-        _, bound, local_seg = step
-        # what moves with every token: the local window grows by one; k goes to a tensor of its own, as the caller may keep it
+        _, bound, local_seg, _ = step
+        # what moves with every token: the local window grows by one; k goes to a tensor of its own, as the caller may keep it.
+        # adaptive_topk_threshold and adaptive_topk_max_k hold for the next step, whenever they are set.
         dense = z.gpu_prefix_rows
+        bound.ad.threshold = float(self.adaptive_topk_threshold)
         bound.ad.dense_rows = bound.ad.row_keys_base = dense
         bound.segs[local_seg].n_rows = z.dense_tail_len
         self.last_adaptive_k = torch.empty_like(self._adaptive_k)
@@ -113,6 +115,8 @@ class polar_cache(_adaptive_base):
             self._adk_ws = torch.empty(need, dtype=torch.uint8, device=self.device)
         if self._dense_vnorm_run is None:
             self._dense_vnorm_run = torch.empty_like(self._dense_logits)
+        if self._topk_ids.numel() < bs * H * topk_cap:   # adaptive_topk_max_k was raised; bound steps keep the tensor they name
+            self._topk_ids = torch.empty(bs * H * topk_cap, dtype=torch.int64, device=self.device)
         local0, dense = z.local_start, z.gpu_prefix_rows
         adaptive = dict(dense_k=kg, dense_rows=dense, dense_split=S0, dense_row1=local0, dense_vnorm=self._sl_vnorm_cache[layer_idx],
                         dense_vnorm_run=self._dense_vnorm_run, dense_logits=self._dense_logits, scale=self._attn_scale,
@@ -126,6 +130,6 @@ class polar_cache(_adaptive_base):
         bound = self._plan.bind_adaptive(q, self._srht_signs, self._mag_centers, self.cluster_key_counts_gpu[layer_idx],
                                          self._codes_km[layer_idx], self._nib_km[layer_idx], self._w_km[layer_idx], S0,
                                          n_keys, tiers, n_cand, adaptive, self._attention, segments)
-        step = (n_keys, bound, 1)
+        step = (n_keys, bound, 1, self.adaptive_topk_max_k)
         self._adaptive_bound[layer_idx] = step
         return step

@@ -1021,3 +1021,49 @@ def test_dense_branch_over_refreshes_and_new_prompts(host):
             ref = (p @ Vd).view(bs, 1, H * group, 128)
             # probabilities and the result are rounded to bf16; values up to ~4.5
             assert (out.double() - ref).abs().max().item() < 2e-2, (S, t)
+
+
+def _cache_of(form, offload, bs, H, group, S, new, sink, local, interval, topk, thr, dtype=torch.bfloat16, layers=1, **kw):
+    """A cache of one of the three classes ("fixed", "varlen", "dense")."""
+    if form == "varlen":
+        from pariskv_amd.cache_hub.polar_cache_adaptivek_varlen import polar_cache as cls
+    elif form == "dense":
+        from pariskv_amd.cache_hub.polar_cache_atten_value_indices_adaptive_k import polar_cache as cls
+    else:
+        from pariskv_amd.cache_hub.polar_cache import polar_cache as cls
+    return cls(valid_start=[0] * bs, layer_num=layers, batch_size=bs, max_length=S + new, num_key_value_heads=H,
+               num_heads=H * group, head_dim=128, dtype=dtype, layer_mapping={i: DEV for i in range(layers)}, max_new_length=new,
+               sink_size=sink, local_size=local, num_gpus=1, model_size=8, final_topk=topk, dynamic_update_interval=interval,
+               full_attention_threshold=thr, enable_offload=offload, **kw)
+
+
+
+def test_dense_adaptive_step_follows_its_threshold_and_cap():
+    """K/V in HBM: adaptive_topk_threshold and adaptive_topk_max_k hold for the next step, between two tokens of one index and
+    with a cap above the one the cache was made with: k and ids equal the stand-alone operator's."""
+    from pariskv_amd import ops
+
+    bs, H, group, S, sink, local = 2, 2, 4, 2600, 4, 64
+    cache = _cache_of("dense", False, bs, H, group, S, 16, sink, local, 32, 50, 100, adaptive_topk_max_k=300)
+    gen = torch.Generator().manual_seed(9)
+    k, v = (t.to(DEV) for t in _synth_kv(gen, bs, S, H))
+    cache.prefill_update_kv_cache(None, k, v, 0, 0)
+    seen = []
+    for thr, cap in ((0.9, 300), (0.2, 300), (0.9, 40), (0.999, 1000), (0.9, 300)):
+        cache.adaptive_topk_threshold, cache.adaptive_topk_max_k = thr, cap
+        k1, v1 = (t.to(DEV) for t in _synth_kv(gen, bs, 1, H))
+        cache.decode_update_kv_cache(k1, v1, 0)
+        q = (torch.randn(bs, 1, H * group, 128, generator=gen) * 0.2).to(torch.bfloat16).to(DEV)
+        cache.compute(q, 0)
+        k_got, z = cache.last_adaptive_k.clone(), cache._zones[0]
+        n_keys, n_cand, _, tiers = cache.retrieval_shape(0)
+        ids_got = cache._topk_ids[:bs * H * cap].view(bs, H, cap).clone()
+        pos = torch.cat([torch.arange(sink), torch.arange(z.local_start, z.seq_len)]).to(DEV)
+        cand, scores = cache._plan.run_candidates(q, cache._srht_signs, cache._mag_centers, cache.cluster_key_counts_gpu[0],
+                                                  cache._codes_km[0], cache._nib_km[0], cache._w_km[0], sink, n_keys, tiers, n_cand)
+        logits = ops.dense_logits(q, cache.unified_keys_gpu[0][:, :, pos].contiguous(), len(pos), cache._attn_scale)
+        k_ref, ids_ref = ops.adaptive_topk(logits, cache._sl_vnorm_cache[0][:, :, pos].contiguous(), scores, cache._attn_scale, cand,
+                                           thr, cap, value_norm=cache.value_norm_gpu[0], vn_offset=sink, k_min=1, k_max=cap)
+        assert torch.equal(k_got, k_ref) and torch.equal(ids_got, ids_ref), (thr, cap)
+        seen.append(int(k_got.max()))
+    assert seen[1] < seen[0] and seen[2] <= 40 and seen[3] > 300   # the settings make a difference here
