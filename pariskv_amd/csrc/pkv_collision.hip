@@ -202,8 +202,8 @@ __global__ __launch_bounds__(kScanThreads) void pkv_scan_strided_kernel(
       for (int s = 0; s < 16; ++s)
 #pragma unroll
         for (int e = 0; e < 4; ++e) c[e] += l8[s * 256 + ((w[s] >> (8 * e)) & 255u)];
-      if (out8) {
-        const uint32_t c8 = c[0] | c[1] << 8 | c[2] << 16 | c[3] << 24;
+      if (out8) {  // low bytes: a caller's table may hold entries that add up to more than the retrieval's 127 votes
+        const uint32_t c8 = (c[0] & 255u) | (c[1] & 255u) << 8 | (c[2] & 255u) << 16 | c[3] << 24;
         __builtin_memcpy(out8 + i, &c8, 4);
       }
       if (out32) __builtin_memcpy(out32 + i, c, 16);

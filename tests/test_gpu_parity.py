@@ -1842,3 +1842,17 @@ def test_select_rerank_at_every_chunk_size(ops, rows, n, k):
     ref = ops.rerank4(want, k4, kw, qhat.view(bs, H, 16, 8), qnorm.view(bs, H, 1), centers)
     ref = ref[0] if isinstance(ref, tuple) else ref
     assert torch.equal(scores.view(bs, H, k), ref.view(bs, H, k))
+
+
+@pytest.mark.parametrize("N", [1, 7, 1027, 5000])
+def test_scan_counts_of_any_table(ops, N):
+    """Votes of a table with any entries (the retrieval's hold at most 127 in all): int32 counts are the sums, byte counts
+    their low eight bits, in every code layout."""
+    bs, H = 1, 3
+    g = torch.Generator(device=DEV).manual_seed(N)
+    lut = torch.randint(0, 256, (bs, H, 16, 256), generator=g, device=DEV).to(torch.uint8)
+    code = torch.randint(0, 256, (bs, H, 16, N), generator=g, device=DEV).to(torch.uint8)
+    want = lut.int().gather(3, code.long()).sum(dim=2)
+    for layout in (code, code.permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2)):   # subspace-major, key-major
+        assert torch.equal(ops.collision_scan(layout, lut, torch.int32)[0], want.int())
+        assert torch.equal(ops.collision_scan(layout, lut, torch.uint8)[0], (want & 255).to(torch.uint8))
