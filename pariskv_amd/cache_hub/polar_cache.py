@@ -294,10 +294,10 @@ class polar_cache(KV_Cache):
             self._prefill_stage_event = [None, None]
 
     def _store_rows(self, layer_idx, k, v, b0, b1, n_sink, n_encode, dense, tail_row0, zone, abs0) -> None:
-        """K/V rows [b1-b0, H, n, D] (any strides) into the cache, their middle n_encode tokens also encoded into metadata
+        """K/V rows [b1-b0, H, n, D] (any strides; on any device, as a slice copy takes them) into the cache, their middle n_encode tokens also encoded into metadata
         positions [abs0, abs0 + n_encode) and added to the cluster sizes: one launch (``ops.prefill_store``)."""
-        if k.dtype != self.dtype or v.dtype != self.dtype:
-            k, v = k.to(self.dtype), v.to(self.dtype)
+        if k.dtype != self.dtype or v.dtype != self.dtype or k.device != self.device or v.device != self.device:
+            k, v = k.to(self.device, self.dtype), v.to(self.device, self.dtype)
         vec = 16 // k.element_size()
         if any(t.stride(3) != 1 or t.data_ptr() % 16 or any(x % vec for x in t.stride()[:3]) for t in (k, v)):
             k, v = k.contiguous(), v.contiguous()

@@ -54,6 +54,14 @@ def _cuda(*ts):
             _need(t.is_cuda, "tensor must be on the GPU")
 
 
+def _one_device(*ts):
+    first = None
+    for t in ts:
+        if t is not None:
+            first = t if first is None else first
+            _need(t.device == first.device, f"tensors of one launch are on {first.device} and {t.device}")
+
+
 def _philox4x32_10(ctr, key):
     """One block of the Philox4x32-10 counter-based generator (Salmon et al., SC'11): 4 x uint32 out."""
     m0, m1, w0, w1, mask = 0xD2511F53, 0xCD9E8D57, 0x9E3779B9, 0xBB67AE85, 0xFFFFFFFF
@@ -162,6 +170,8 @@ def prefill_store(k: torch.Tensor, v: torch.Tensor, n_sink: int, n_encode: int, 
     _need(D == HEAD_DIM and v.shape == k.shape and v.dtype == k.dtype and n_sink >= 0 and n_encode >= 0 and n_tail >= 0,
           "k, v: [bs,H,S,128] of one dtype, n_sink + n_encode <= S")
     _need(k.stride(3) == 1 and v.stride(3) == 1, "k, v: contiguous rows")
+    _one_device(k, v, signs if n_encode else None, *(dense or ()), *(zone or ()), *(index or ()), dense_vnorm, zone_vnorm,
+                zone_vnorm2)
     a = _lib.PrefillArgs()
     a.k, a.v, a.dtype, a.bs, a.n_kv_heads = k.data_ptr(), v.data_ptr(), _dt(k.dtype), bs, H
     a.k_stride_b, a.k_stride_h, a.k_stride_key = k.stride()[:3]

@@ -140,3 +140,32 @@ def test_gather_cpu_equals_the_reference_build():
         ref.gather_kv_out_cpu(src_t, idx, big_w[:, :, 4:13])
     with pytest.raises(RuntimeError, match="out of bounds"):
         ext.gather_kv_out_cpu(src_t, idx, big_g[:, :, 4:13])
+
+
+def test_prefill_store_refuses_operands_of_several_devices():
+    """The launch goes to the stream of k's device: rows, index or norms on another one are refused before it (host tensors
+    that say they are on a GPU stand in for two cards)."""
+    import torch
+
+    from pariskv_amd import ops
+
+    class On:
+        def __init__(self, device, t):
+            self._t, self.device, self.is_cuda = t, torch.device(device), True
+
+        def __getattr__(self, name):
+            return getattr(self._t, name)
+
+    def operands(**elsewhere):
+        t = dict(k=torch.zeros(1, 2, 8, 128), v=torch.zeros(1, 2, 8, 128), signs=torch.ones(128), dk=torch.zeros(1, 2, 4, 128),
+                 dv=torch.zeros(1, 2, 4, 128), zk=torch.zeros(1, 2, 5, 128), zv=torch.zeros(1, 2, 5, 128),
+                 cb=torch.zeros(1, 2, 16, 5, dtype=torch.uint8), k4=torch.zeros(1, 2, 16, 5, 4, dtype=torch.uint8),
+                 kw=torch.zeros(1, 2, 16, 5, dtype=torch.bfloat16), cc=torch.zeros(1, 2, 16, 256, dtype=torch.int32),
+                 dn=torch.zeros(1, 2, 4), zn=torch.zeros(1, 2, 5), zn2=torch.zeros(1, 2, 5))
+        return {n: On(elsewhere.get(n, "cuda:0"), x) for n, x in t.items()}
+
+    for name in operands():
+        o = operands(**{name: "cuda:1"})
+        with pytest.raises(RuntimeError, match="tensors of one launch"):
+            ops.prefill_store(o["k"], o["v"], 2, 5, o["signs"], (o["dk"], o["dv"]), 3, (o["zk"], o["zv"]),
+                              (o["cb"], o["k4"], o["kw"], o["cc"]), dense_vnorm=o["dn"], zone_vnorm=o["zn"], zone_vnorm2=o["zn2"])

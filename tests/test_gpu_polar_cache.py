@@ -1067,3 +1067,27 @@ def test_dense_adaptive_step_follows_its_threshold_and_cap():
         assert torch.equal(k_got, k_ref) and torch.equal(ids_got, ids_ref), (thr, cap)
         seen.append(int(k_got.max()))
     assert seen[1] < seen[0] and seen[2] <= 40 and seen[3] > 300   # the settings make a difference here
+
+
+@pytest.mark.parametrize("form,offload", [("fixed", True), ("fixed", False), ("varlen", True), ("dense", False)])
+@pytest.mark.parametrize("S", [30, 700])
+def test_prompt_in_host_memory(form, offload, S):
+    """prefill_update_kv_cache takes K/V from host memory too, in the cache's type or another: cache, index, value norms and
+    host store equal those of the same prompt on the GPU."""
+    bs, H = 2, 2
+    gen = torch.Generator().manual_seed(S)
+    k, v = (torch.randn(bs, S, H, 128, generator=gen) for _ in range(2))
+    caches = []
+    for prompt in ((k.to(torch.bfloat16).to(DEV), v.to(torch.bfloat16).to(DEV)), (k.to(torch.bfloat16), v.to(torch.bfloat16)), (k, v)):
+        caches.append(_cache_of(form, offload, bs, H, 4, S, 16, 4, 64, 16, 50, 100))
+        kr, vr = caches[-1].prefill_update_kv_cache(None, *prompt, 0, 0)
+        assert kr.device == prompt[0].device and torch.equal(vr, prompt[1])   # handed back as they came
+    torch.cuda.synchronize()
+    for c in caches[1:]:
+        for name in ("unified_keys_gpu", "unified_values_gpu", "_codes_km", "_nib_km", "_w_km", "cluster_key_counts_gpu",
+                     "value_norm_gpu", "_sl_vnorm_cache") + (("unified_keys_cpu", "unified_values_cpu") if offload else ()):
+            if hasattr(c, name):
+                a, b = getattr(caches[0], name)[0], getattr(c, name)[0]
+                if name.endswith("_cpu"):
+                    a, b = a[:, :, :c.cpu_valid_end[0]], b[:, :, :c.cpu_valid_end[0]]
+                assert torch.equal(a, b), name
