@@ -300,7 +300,8 @@ class polar_cache(KV_Cache):
             k, v = k.to(self.device, self.dtype), v.to(self.device, self.dtype)
         vec = 16 // k.element_size()
         if any(t.stride(3) != 1 or t.data_ptr() % 16 or any(x % vec for x in t.stride()[:3]) for t in (k, v)):
-            k, v = k.contiguous(), v.contiguous()
+            # a clone, as contiguous() hands a tensor that is contiguous but misaligned back as it is
+            k, v = (t.clone(memory_format=torch.contiguous_format) for t in (k, v))
         index = zone_norms = None
         if n_encode > 0:
             sl = slice(abs0, abs0 + n_encode)

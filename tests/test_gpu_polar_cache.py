@@ -1091,3 +1091,19 @@ def test_prompt_in_host_memory(form, offload, S):
                 if name.endswith("_cpu"):
                     a, b = a[:, :, :c.cpu_valid_end[0]], b[:, :, :c.cpu_valid_end[0]]
                 assert torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("S", [1, 30, 700])
+def test_prompt_that_is_contiguous_but_not_aligned(dtype, S):
+    """One KV head: the head-major view of a prompt is contiguous as it stands, also where it starts at an odd element of
+    its storage and its rows are not 16-byte aligned."""
+    gen = torch.Generator(device=DEV).manual_seed(S)
+    k, v = (torch.randn(S * 128 + 1, generator=gen, device=DEV).to(dtype)[1:].view(1, S, 1, 128) for _ in range(2))
+    caches = []
+    for prompt in ((k.clone(), v.clone()), (k, v)):
+        caches.append(_cache_of("fixed", False, 1, 1, 4, S, 16, 4, 64, 16, 50, 100, dtype=dtype))
+        caches[-1].prefill_update_kv_cache(None, *prompt, 0, 0)
+    for name in ("unified_keys_gpu", "unified_values_gpu", "_codes_km", "_nib_km", "_w_km", "cluster_key_counts_gpu"):
+        assert torch.equal(getattr(caches[0], name)[0], getattr(caches[1], name)[0]), name
+    assert torch.equal(caches[1].unified_keys_gpu[0][:, :, :S], k.permute(0, 2, 1, 3))
