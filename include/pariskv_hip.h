@@ -86,7 +86,8 @@ int pkv_encode_append(const void *keys, int dtype, int bs, int n_kv_heads, int64
  * Tokens [0, n_sink) and [n_sink + n_encode, + n_tail) of k / v go to rows
  * 0 .. n_sink-1 and tail_row0 .. of dense_k / dense_v; the n_encode tokens
  * between them go to rows 0 .. of zone_k / zone_v and are encoded as by
- * pkv_encode_append (all outputs; cluster_counts +=).  Value norms (||v|| in
+ * pkv_encode_append (all outputs; cluster_counts +=).  Fewer than 2^29 tokens in
+ * all.  Value norms (||v|| in
  * dtype, widened; four consecutive squares left to right, then a pairwise tree
  * over the 32 groups): dense_vnorm of the dense
  * rows by destination row, zone_vnorm (any key stride) and zone_vnorm2

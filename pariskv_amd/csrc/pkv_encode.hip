@@ -834,8 +834,11 @@ extern "C" int pkv_prefill_store(const pkv_prefill_args *a, void *stream) {
   PKV_REQUIRE(a->dtype == PKV_DTYPE_F32 || a->dtype == PKV_DTYPE_BF16, "unknown dtype %d", a->dtype);
   PKV_REQUIRE(a->bs > 0 && a->bs <= 65535 && a->n_kv_heads > 0 && (int64_t)a->bs * a->n_kv_heads <= 65535,
               "bad shape bs=%d kv_heads=%d", a->bs, a->n_kv_heads);
-  PKV_REQUIRE(a->n_sink >= 0 && a->n_encode >= 0 && a->n_tail >= 0 && a->tail_row0 >= a->n_sink &&
-                  a->n_sink + a->n_encode + a->n_tail < ((int64_t)1 << 23),
+  // A launch has fewer than 2^32 threads, four for each dense row; block counts and rows inside a run are ints, addresses 64 bits
+  // wide.  (Each count first: their sum cannot overflow then.)
+  const int64_t most = (int64_t)1 << 29;
+  PKV_REQUIRE(a->n_sink >= 0 && a->n_encode >= 0 && a->n_tail >= 0 && a->n_sink < most && a->n_encode < most && a->n_tail < most &&
+                  a->n_sink + a->n_encode + a->n_tail < most && a->tail_row0 >= a->n_sink,
               "pkv_prefill_store: bad token counts %lld + %lld + %lld", (long long)a->n_sink, (long long)a->n_encode,
               (long long)a->n_tail);
   if (a->n_sink + a->n_encode + a->n_tail == 0) return PKV_OK;

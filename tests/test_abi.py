@@ -169,3 +169,17 @@ def test_prefill_store_refuses_operands_of_several_devices():
         with pytest.raises(RuntimeError, match="tensors of one launch"):
             ops.prefill_store(o["k"], o["v"], 2, 5, o["signs"], (o["dk"], o["dv"]), 3, (o["zk"], o["zv"]),
                               (o["cb"], o["k4"], o["kw"], o["cc"]), dense_vnorm=o["dn"], zone_vnorm=o["zn"], zone_vnorm2=o["zn2"])
+
+
+def test_prefill_store_has_room_for_the_longest_rows():
+    """Token counts up to 2^29 pass the check of pkv_prefill_store (the index itself takes 2^24 keys a row); no kernel is
+    launched, as there is no K/V to copy."""
+    from pariskv_amd import _lib
+
+    L = _lib.lib()
+    a = _lib.PrefillArgs()
+    a.dtype, a.bs, a.n_kv_heads, a.n_sink, a.n_tail, a.tail_row0 = _lib.DTYPE_BF16, 1, 1, 64, 512, 64
+    for n, ok in ((1 << 23, True), ((1 << 24) + 5, True), ((1 << 29) - 577, True), ((1 << 29) - 576, False), (1 << 40, False), (-1, False)):
+        a.n_encode = n
+        assert L.pkv_prefill_store(a, None) == _lib.EINVAL
+        assert (b"token counts" not in L.pkv_last_error()) == ok, (n, L.pkv_last_error())

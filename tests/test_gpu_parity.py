@@ -1856,3 +1856,27 @@ def test_scan_counts_of_any_table(ops, N):
     for layout in (code, code.permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2)):   # subspace-major, key-major
         assert torch.equal(ops.collision_scan(layout, lut, torch.int32)[0], want.int())
         assert torch.equal(ops.collision_scan(layout, lut, torch.uint8)[0], (want & 255).to(torch.uint8))
+
+
+def test_prefill_store_beyond_2_to_the_23_tokens(ops):
+    """One head with more than 2^23 tokens: all rows in their places, the index of the last keys equal to pkv_encode_append's,
+    every key counted once."""
+    n_sink, n_tail, last = 5, 70, 1000
+    n = (1 << 23) + 301
+    S = n_sink + n + n_tail
+    g = torch.Generator(device=DEV).manual_seed(8)
+    k, v = (torch.randn(1, 1, S, 128, generator=g, device=DEV, dtype=torch.bfloat16) for _ in range(2))
+    signs = ops.srht_signs(DEV)
+    dk, zk = torch.zeros(1, 1, n_sink + n_tail, 128, dtype=k.dtype, device=DEV), torch.zeros(1, 1, n, 128, dtype=k.dtype, device=DEV)
+    dv, zv = torch.zeros_like(dk), torch.zeros_like(zk)
+    codes, nib, w, cb, k4, kw = ops.alloc_keymajor(1, 1, n, DEV)
+    cc = torch.zeros(1, 1, 16, 256, dtype=torch.int32, device=DEV)
+    ops.prefill_store(k, v, n_sink, n, signs, (dk, dv), n_sink, (zk, zv), (cb, k4, kw, cc))
+    for src, dense, zone in ((k, dk, zk), (v, dv, zv)):
+        assert torch.equal(zone, src[:, :, n_sink:n_sink + n])
+        assert torch.equal(dense, torch.cat([src[:, :, :n_sink], src[:, :, n_sink + n:]], dim=2))
+    assert torch.all(cc.sum(dim=3) == n)
+    codes2, nib2, w2, cb2, k42, kw2 = ops.alloc_keymajor(1, 1, last, DEV)
+    ops.encode_append(k[:, :, n_sink + n - last:n_sink + n], signs, cb2, k42, kw2, torch.zeros_like(cc))
+    assert torch.equal(codes[:, :, -last:], codes2) and torch.equal(nib[:, :, -last:], nib2)
+    assert torch.equal(w[:, :, -last:].view(torch.int16), w2.view(torch.int16))
