@@ -281,9 +281,9 @@ class polar_cache(KV_Cache):
         return kv[0][b0:b1], kv[1][b0:b1]
 
     def _drop_short_rows(self, layer_idx: int) -> None:
-        """The sequence has outgrown the dense branch: its retrieval-zone rows in HBM go back to the allocator."""
-        if self._short_kv[layer_idx] is not None:
-            self._short_kv[layer_idx] = self._dense_bound[layer_idx] = None
+        """The sequence has outgrown the dense branch: its retrieval-zone rows in HBM go back to the allocator, and with them
+        the argument block that holds them."""
+        self._short_kv[layer_idx] = self._dense_bound[layer_idx] = None
 
     def release_prefill_staging(self) -> None:
         """Free the prefill staging pairs (two layers' worth of retrieval-zone K/V in HBM) once prefill is over; they

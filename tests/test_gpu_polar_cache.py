@@ -1107,3 +1107,28 @@ def test_prompt_that_is_contiguous_but_not_aligned(dtype, S):
     for name in ("unified_keys_gpu", "unified_values_gpu", "_codes_km", "_nib_km", "_w_km", "cluster_key_counts_gpu"):
         assert torch.equal(getattr(caches[0], name)[0], getattr(caches[1], name)[0]), name
     assert torch.equal(caches[1].unified_keys_gpu[0][:, :, :S], k.permute(0, 2, 1, 3))
+
+
+@pytest.mark.parametrize("form", ["fixed", "varlen", "dense"])
+def test_first_retrieving_step_gives_the_short_rows_back(form):
+    """The zone rows that a short sequence keeps in HBM are freed by the first step that retrieves, in every class that
+    offloads: no argument block holds them any longer."""
+    import gc
+    import weakref
+
+    bs, H, group, S, thr, steps = 2, 2, 4, 250, 260, 30
+    cache = _cache_of(form, True, bs, H, group, S, steps, 4, 64, 16, 50, thr)
+    gen = torch.Generator().manual_seed(3)
+    k, v = (t.to(DEV) for t in _synth_kv(gen, bs, S, H))
+    cache.prefill_update_kv_cache(None, k, v, 0, 0)
+    refs = []
+    for step in range(steps):
+        k1, v1 = (t.to(DEV) for t in _synth_kv(gen, bs, 1, H))
+        cache.decode_update_kv_cache(k1, v1, 0)
+        cache.compute(torch.randn(bs, 1, H * group, 128, generator=gen).to(torch.bfloat16).to(DEV), 0)
+        if not refs:
+            refs = [weakref.ref(t) for t in cache._short_kv[0][:2]]
+        gc.collect()
+        dense = cache._zones[0].seq_len < cache._min_total()
+        assert [r() is not None for r in refs] == [dense, dense], step
+    assert not dense
