@@ -265,7 +265,8 @@ class polar_cache(KV_Cache):
         dense-attention threshold: K/V [b1-b0,H,rows,D] in HBM, beside the host store.  Every step of such a sequence
         attends to all of its tokens; read from the host they cost a wait for the copy stream and two strided copies over
         PCIe per layer and token (235 us for 924 rows x 8 heads), from HBM 7 us.  At most SHORT_ROWS_MAX rows a head;
-        given back by the first step that retrieves.  None for longer prompts or a threshold too high for that."""
+        given back by the first step that retrieves; every stream that works on them is told to the allocator (a decode on
+        another stream than the prefill's may still have attention over them queued then).  None for longer prompts or a threshold too high for that."""
         rows = self._min_total() - self.sink_size - self.local_size
         self._dense_bound[layer_idx] = None
         if n_tok >= self._min_total() or rows > SHORT_ROWS_MAX:
@@ -277,8 +278,14 @@ class polar_cache(KV_Cache):
             kv = (torch.empty(shape, dtype=self.dtype, device=self.device),
                   torch.empty(shape, dtype=self.dtype, device=self.device), [False] * self.batch_size)
             self._short_kv[layer_idx] = kv
+        self._record_short_rows(kv)
         kv[2][b0:b1] = [True] * (b1 - b0)   # samples whose rows are here: prompts may arrive one by one
         return kv[0][b0:b1], kv[1][b0:b1]
+
+    def _record_short_rows(self, kv) -> None:
+        stream = torch.cuda.current_stream(self.device)
+        for t in kv[:2]:
+            t.record_stream(stream)
 
     def _drop_short_rows(self, layer_idx: int) -> None:
         """The sequence has outgrown the dense branch: its retrieval-zone rows in HBM go back to the allocator, and with them
@@ -412,6 +419,7 @@ class polar_cache(KV_Cache):
             self._short_rows(layer_idx, 0, bs, self.current_seq_len[layer_idx])
         short = self._short_kv[layer_idx]
         if short is not None and self.current_seq_len[layer_idx] < self._min_total() and r.cpu_row0 + n <= short[0].shape[2]:
+            self._record_short_rows(short)
             sk, sv = (t[:, :, r.cpu_row0:r.cpu_row0 + n] for t in short[:2])
         else:
             self._drop_short_rows(layer_idx)
@@ -478,7 +486,8 @@ class polar_cache(KV_Cache):
             kg, short = self.unified_keys_gpu[layer_idx], self._short_kv[layer_idx]
             if not all(s[0] is kg or (short is not None and s[0] is short[0]) for s in segments):
                 return self._attend(q, segments)   # copies of host rows: this step's only
-            bound = self._dense_bound[layer_idx] = (z.encoded, ops.BoundAttention(self._attention, q, segments))
+            lent = short[:2] if short is not None else ()
+            bound = self._dense_bound[layer_idx] = (z.encoded, ops.BoundAttention(self._attention, q, segments, lent))
         bound[1].segs[0].n_rows = z.gpu_prefix_rows if self._layer_offload[layer_idx] else z.seq_len
         return bound[1].launch(q)
 

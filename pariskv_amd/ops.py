@@ -825,16 +825,19 @@ def gather_cpu(src: torch.Tensor, index: torch.Tensor, out: torch.Tensor, n_thre
 
 
 class BoundAttention:
-    """The argument block of one layer's pkv_decode_attention, validated once; the caller patches ``segs[i].n_rows``."""
+    """The argument block of one layer's pkv_decode_attention, validated once; the caller patches ``segs[i].n_rows``.
+    ``lent``: tensors of the segments that the caller may let go while a launch is queued; every stream that launches is
+    told to the allocator once, so that their memory waits for it."""
 
-    __slots__ = ("aa", "segs", "keep", "_raa", "_dims", "_fn", "_numel", "_dtype")
+    __slots__ = ("aa", "segs", "keep", "_raa", "_dims", "_fn", "_numel", "_dtype", "_lent", "_streams")
 
-    def __init__(self, att, q, segments):
+    def __init__(self, att, q, segments, lent=()):
         self.aa, _ = att.c_args(q, segments, out=q)  # out is patched at every launch
         self.segs, self._raa, self.keep = self.aa.segments, C.byref(self.aa), (att, segments)
         self._dims = (_dt(q.dtype), att.bs, att.H, att.G)
         self._fn = _lib.lib().pkv_decode_attention_run
         self._numel, self._dtype = q.numel(), q.dtype
+        self._lent, self._streams = lent, set()
 
     def launch(self, q: torch.Tensor) -> torch.Tensor:
         """q: contiguous [bs,1,Hq,128] of the bound dtype.  Returns the attention output, shaped like q."""
@@ -842,7 +845,13 @@ class BoundAttention:
               "queries must be contiguous [bs,1,Hq,128] of the cache dtype")
         out = torch.empty_like(q)
         self.aa.out = out.data_ptr()
-        rc = self._fn(q.data_ptr(), *self._dims, self._raa, torch.cuda.current_stream(q.device).cuda_stream)
+        stream = torch.cuda.current_stream(q.device)
+        handle = stream.cuda_stream
+        if self._lent and handle not in self._streams:
+            for t in self._lent:
+                t.record_stream(stream)
+            self._streams.add(handle)
+        rc = self._fn(q.data_ptr(), *self._dims, self._raa, handle)
         if rc != 0:
             _lib.check(rc)
         return out

@@ -1132,3 +1132,38 @@ def test_first_retrieving_step_gives_the_short_rows_back(form):
         dense = cache._zones[0].seq_len < cache._min_total()
         assert [r() is not None for r in refs] == [dense, dense], step
     assert not dense
+
+
+@pytest.mark.parametrize("form", ["fixed", "varlen"])
+def test_short_rows_outlive_the_stream_that_reads_them(form):
+    """Decode on another stream than the prefill: the zone rows of a short sequence come from the prefill's stream.  Given
+    back while the decode stream still has attention over them queued, their memory goes to nobody until that stream is done
+    (the decode stream is held up by a spinning kernel meanwhile; nothing reads or writes what is allocated here)."""
+    bs, H, group, S, thr, steps = 2, 8, 2, 1990, 2000, 12
+    cache = _cache_of(form, True, bs, H, group, S, steps + 4, 4, 64, 512, 50, thr)
+    gen = torch.Generator().manual_seed(4)
+    k, v = (t.to(DEV) for t in _synth_kv(gen, bs, S, H))
+    new = [[t.to(DEV) for t in _synth_kv(gen, bs, 1, H)] for _ in range(steps)]
+    q = torch.randn(bs, 1, H * group, 128, generator=gen).to(torch.bfloat16).to(DEV)
+    pre, dec = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for turn in range(2):   # the first turn loads every kernel
+        with torch.cuda.stream(pre):
+            cache.prefill_update_kv_cache(None, k, v, 0, 0)
+        torch.cuda.synchronize()
+        rows = {t.data_ptr() for t in cache._short_kv[0][:2]}
+        shape = cache._short_kv[0][0].shape
+        with torch.cuda.stream(dec):
+            if turn:
+                torch.cuda._sleep(1 << 29)
+            for k1, v1 in new:
+                cache.decode_update_kv_cache(k1, v1, 0)
+                cache.compute(q, 0)
+        assert cache._short_kv[0] is None
+        if turn:
+            with torch.cuda.stream(pre):
+                taken = [torch.empty(shape, dtype=torch.bfloat16, device=DEV) for _ in range(6)]
+            if dec.query():
+                pytest.skip("the decode stream was done before the check")
+            assert not rows & {t.data_ptr() for t in taken}
+        torch.cuda.synchronize()
