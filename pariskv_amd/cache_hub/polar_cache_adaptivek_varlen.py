@@ -185,6 +185,13 @@ class polar_cache(_polar_cache_base):
                 return bound.launch(q)
         return bound.launch(q)
 
+    def _larger(self, scratch, n, dtype):
+        """Scratch of n elements in the place of a smaller one, whose memory waits for what this stream has queued on it (it
+        may come from another stream's pool)."""
+        if scratch is not None:
+            scratch.record_stream(torch.cuda.current_stream(self.device))
+        return torch.empty(n, dtype=dtype, device=self.device)
+
     def _bind_adaptive_step(self, layer_idx, q, n_keys):
         """Argument blocks of this layer's step, valid until the next index refresh changes ``n_keys``."""
         z = self._zones[layer_idx]
@@ -194,7 +201,7 @@ class polar_cache(_polar_cache_base):
         sl_end = z.gpu_prefix_rows
         need = ops.adaptive_topk_ws_bytes(self.batch_groups, n_cand, topk_cap)
         if self._adk_ws is None or self._adk_ws.numel() < need:
-            self._adk_ws = torch.empty(need, dtype=torch.uint8, device=self.device)
+            self._adk_ws = self._larger(self._adk_ws, need, torch.uint8)
         adaptive = dict(dense_k=kg, dense_rows=sl_end, dense_vnorm=self._sl_vnorm_cache[layer_idx],
                         dense_logits=self._dense_logits, scale=self._attn_scale, value_norm=self.value_norm_gpu[layer_idx],
                         vn_offset=self.sink_size, record_word_offset=ops.RECORD_VALUE_NORM_OFFSET, threshold=self.adaptive_topk_threshold, k_out=topk_cap, k_min=k_min,

@@ -112,11 +112,11 @@ class polar_cache(_adaptive_base):
         bs, H = self.batch_size, self.kv_head
         need = ops.adaptive_topk_ws_bytes(self.batch_groups, n_cand, topk_cap)
         if self._adk_ws is None or self._adk_ws.numel() < need:
-            self._adk_ws = torch.empty(need, dtype=torch.uint8, device=self.device)
+            self._adk_ws = self._larger(self._adk_ws, need, torch.uint8)
         if self._dense_vnorm_run is None:
             self._dense_vnorm_run = torch.empty_like(self._dense_logits)
         if self._topk_ids.numel() < bs * H * topk_cap:   # adaptive_topk_max_k was raised; bound steps keep the tensor they name
-            self._topk_ids = torch.empty(bs * H * topk_cap, dtype=torch.int64, device=self.device)
+            self._topk_ids = self._larger(self._topk_ids, bs * H * topk_cap, torch.int64)
         local0, dense = z.local_start, z.gpu_prefix_rows
         adaptive = dict(dense_k=kg, dense_rows=dense, dense_split=S0, dense_row1=local0, dense_vnorm=self._sl_vnorm_cache[layer_idx],
                         dense_vnorm_run=self._dense_vnorm_run, dense_logits=self._dense_logits, scale=self._attn_scale,

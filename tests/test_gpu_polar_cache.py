@@ -1167,3 +1167,36 @@ def test_short_rows_outlive_the_stream_that_reads_them(form):
                 pytest.skip("the decode stream was done before the check")
             assert not rows & {t.data_ptr() for t in taken}
         torch.cuda.synchronize()
+
+
+def test_outgrown_adaptive_scratch_outlives_the_stream_that_uses_it():
+    """Dense adaptive form in HBM, decoded on another stream than the one its scratch comes from: scratch that a larger cap
+    replaces goes to nobody while steps that use it are queued (behind a spinning kernel; nothing reads or writes what is
+    allocated here)."""
+    bs, H, group, S = 2, 2, 4, 30000
+    first, dec = torch.cuda.Stream(), torch.cuda.Stream()
+    gen = torch.Generator().manual_seed(2)
+    k, v = (t.to(DEV) for t in _synth_kv(gen, bs, S, H))
+    q = torch.randn(bs, 1, H * group, 128, generator=gen).to(torch.bfloat16).to(DEV)
+    for turn in range(2):   # the first turn loads every kernel
+        with torch.cuda.stream(first):
+            cache = _cache_of("dense", False, bs, H, group, S, 8, 4, 64, 32, 50, 100, adaptive_topk_max_k=300)
+            cache.prefill_update_kv_cache(None, k, v, 0, 0)
+            cache.compute(q, 0)
+        torch.cuda.synchronize()
+        old = {n: (getattr(cache, n).data_ptr(), getattr(cache, n).numel(), getattr(cache, n).dtype) for n in ("_topk_ids", "_adk_ws")}
+        with torch.cuda.stream(dec):
+            if turn:
+                torch.cuda._sleep(1 << 28)
+            cache.compute(q, 0)
+            cache.adaptive_topk_max_k = 1200
+            cache.compute(q, 0)
+        gone = [o for n, o in old.items() if getattr(cache, n).data_ptr() != o[0]]
+        assert gone
+        if turn:
+            with torch.cuda.stream(first):
+                taken = {torch.empty(numel, dtype=dt, device=DEV) for _, numel, dt in gone for _ in range(6)}
+            if dec.query():
+                pytest.skip("the decode stream was done before the check")
+            assert not {o[0] for o in gone} & {t.data_ptr() for t in taken}
+        torch.cuda.synchronize()
