@@ -540,7 +540,7 @@ def gather_hbm(src_k, src_v, idx, dst_k, dst_v, idx_offset: int = 0, dst_row0: i
 class BoundAppend:
     """The destination of one layer's :func:`append_kv`, validated once: a token costs the checks of its own rows."""
 
-    __slots__ = ("_a", "_ra", "keep", "_shape", "_dtype", "_es", "_fn", "_device")
+    __slots__ = ("_a", "_ra", "keep", "_shape", "_dtype", "_es", "_fn", "_device", "_slots")
 
     def __init__(self, dst_k, dst_v, vnorm: Optional[torch.Tensor] = None):
         bs, H, rows, D = dst_k.shape
@@ -555,6 +555,7 @@ class BoundAppend:
         self._ra, self.keep = C.byref(self._a), (dst_k, dst_v, vnorm)
         self._shape, self._dtype, self._es, self._device = (bs, 1, H, D), dst_k.dtype, es, dst_k.device
         self._fn = _lib.lib().pkv_append_kv_run
+        self._slots = rows if vnorm is None else min(rows, vnorm.shape[2])  # the kernel checks nothing: rows and norms have these
 
     def launch(self, k, v, slot: int) -> None:
         """k, v: [bs,1,Hkv,D] of the destination's dtype with contiguous rows, on the GPU."""
@@ -562,6 +563,7 @@ class BoundAppend:
         _need(k.shape == self._shape and v.shape == self._shape and ks[3] == 1 and vs[3] == 1 and k.is_cuda and v.is_cuda,
               "key_states, value_states: [bs,1,Hkv,D] on the GPU with contiguous rows")
         _need(k.dtype == self._dtype and v.dtype == self._dtype, "append: dtypes differ")
+        _need(0 <= slot < self._slots, "append: the slot lies outside the K/V rows or the value norms")
         rc = self._fn(self._ra, k.data_ptr(), ks[0] * es, ks[2] * es, v.data_ptr(), vs[0] * es, vs[2] * es, slot,
                       torch.cuda.current_stream(self._device).cuda_stream)
         if rc != 0:

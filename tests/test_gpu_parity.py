@@ -1880,3 +1880,23 @@ def test_prefill_store_beyond_2_to_the_23_tokens(ops):
     ops.encode_append(k[:, :, n_sink + n - last:n_sink + n], signs, cb2, k42, kw2, torch.zeros_like(cc))
     assert torch.equal(codes[:, :, -last:], codes2) and torch.equal(nib[:, :, -last:], nib2)
     assert torch.equal(w[:, :, -last:].view(torch.int16), w2.view(torch.int16))
+
+
+def test_bound_append_refuses_a_slot_behind_the_norms(ops):
+    """The kept append refuses what append_kv refuses: a slot that the K/V rows have and the value norms have not."""
+    dk, dv = (torch.zeros(1, 2, 8, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    k, v = (torch.ones(1, 1, 2, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    vn = torch.zeros(1, 2, 5, device=DEV)
+    bound = ops.BoundAppend(dk, dv, vnorm=vn)
+    bound.launch(k, v, 4)
+    assert torch.equal(vn[:, :, 4], torch.full((1, 2), float(torch.tensor(128.0).sqrt().to(torch.bfloat16)), device=DEV))
+    for slot in (5, 7, 8, -1):
+        with pytest.raises(RuntimeError):
+            bound.launch(k, v, slot)
+    bound = ops.BoundAppend(dk, dv)
+    bound.launch(k, v, 7)
+    for slot in (8, -1):
+        with pytest.raises(RuntimeError):
+            bound.launch(k, v, slot)
+    torch.cuda.synchronize()
+    assert torch.all(dk[:, :, [4, 7]] == 1) and torch.all(dk[:, :, [0, 1, 2, 3, 5, 6]] == 0)
