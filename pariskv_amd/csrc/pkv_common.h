@@ -60,8 +60,9 @@ struct PkvTiers {
 //   8 rows x 3.5K 32.2 / 34.1 / - / 39.5,  8 x 7.6K 32.8 / 33.1 / - / 38.0,  8 x 16K 34.8 / 33.9 / - / 37.5,
 //   8 x 32K - / 37.2 / 36.5 / 38.0,  32 x 11K - / 35.8 / 37.0 / 37.9,  32 x 32K - / - / 40.0 / 40.8.
 // Always a power of two of 256 .. 32768 (a chunk's histogram bins are uint16).
-static inline int pkv_pick_chunk_keys(int rows, int64_t n_keys) {
-  int64_t chunk = 256;
+// least: the smallest chunk to consider (a power of two of 256 .. 2048).
+static inline int pkv_pick_chunk_keys(int rows, int64_t n_keys, int least = 256) {
+  int64_t chunk = least;
   auto n_chunks = [&] { return (n_keys + chunk - 1) / chunk; };
   while (chunk < 2048 && ((int64_t)rows * n_chunks() > 1024 || (n_chunks() > 32 && (int64_t)rows * n_chunks() > 128))) chunk *= 2;
   while (chunk < 16384 && (int64_t)rows * n_chunks() > 1024) chunk *= 2;

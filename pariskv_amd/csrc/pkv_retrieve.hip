@@ -38,7 +38,7 @@ struct WsLayout {
   int sub_blocks;  // pieces per chunk of the scan -> select + rerank pair (one suffix histogram each)
 };
 
-WsLayout layout(int rows, int64_t n_keys, int64_t n_cand, int64_t k) {
+WsLayout layout(int rows, int64_t n_keys, int64_t n_cand, int64_t k, int least_chunk = 256) {
   WsLayout w;
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -46,7 +46,7 @@ WsLayout layout(int rows, int64_t n_keys, int64_t n_cand, int64_t k) {
     off += pkv_align_up(bytes, 256);
     return o;
   };
-  w.chunk_keys = pkv_pick_chunk_keys(rows, n_keys);
+  w.chunk_keys = pkv_pick_chunk_keys(rows, n_keys, least_chunk);
   w.n_chunks = (n_keys + w.chunk_keys - 1) / w.chunk_keys;
   w.cnt_stride = (int64_t)pkv_align_up((size_t)n_keys, 16);
   w.qhat = take((size_t)rows * 128 * sizeof(float));
@@ -119,7 +119,8 @@ extern "C" int pkv_retrieve_ws_view(void *ws, int rows, int64_t n_keys, int64_t 
 }
 
 // dense (or null): the adaptive-k step's dense tokens, whose logits ride with the query prep where that is a launch of its own
-static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, void *stream, const PkvDenseLogits *dense = nullptr) {
+static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, void *stream, const PkvDenseLogits *dense = nullptr,
+                         int least_chunk = 256) {
   PKV_REQUIRE(a != nullptr, "pkv_retrieve: null args");
   PKV_REQUIRE(a->q && a->signs && a->centers && a->cluster_counts && a->codes && a->nib && a->weight,
               "pkv_retrieve: null pointer");
@@ -136,7 +137,7 @@ static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, 
   PKV_REQUIRE(pkv_aligned(a->codes, 16) && pkv_aligned(a->nib, 16) && pkv_aligned(a->weight, 16) &&
                   pkv_aligned(a->q, 16),
               "queries / codes / nib / weight must be 16-byte aligned");
-  const WsLayout w = layout(rows, a->n_keys, a->n_cand, a->k);
+  const WsLayout w = layout(rows, a->n_keys, a->n_cand, a->k, least_chunk);
   if (!ws || ws_bytes < w.total || !pkv_aligned(ws, 256)) {
     pkv_set_error("pkv_retrieve: workspace of %zu bytes (256-aligned) required, got %zu", w.total, ws_bytes);
     return PKV_ENOMEM;
@@ -318,7 +319,14 @@ extern "C" int pkv_retrieve_noalloc(const pkv_retrieve_args *a, void *stream) {
   PKV_REQUIRE(a->bs > 0 && a->n_kv_heads > 0 && shape_ok(rows, a->n_keys, a->n_cand, a->k),
               "need 0 < k <= n_cand <= n_keys <= 2^24 (k=%lld n_cand=%lld n_keys=%lld rows=%d)", (long long)a->k,
               (long long)a->n_cand, (long long)a->n_keys, rows);
-  const size_t need = layout(rows, a->n_keys, a->n_cand, a->k).total;
+  // Short rows' chunks below 2048 keys take up to 256 KB more for their histograms: a shape that fits without them is scanned
+  // in larger chunks rather than refused.
+  int least_chunk = 256;
+  size_t need = layout(rows, a->n_keys, a->n_cand, a->k).total;
+  if (need > (size_t)PKV_NOALLOC_SCRATCH_BYTES) {
+    least_chunk = 2048;
+    need = layout(rows, a->n_keys, a->n_cand, a->k, least_chunk).total;
+  }
   if (need > (size_t)PKV_NOALLOC_SCRATCH_BYTES) {
     pkv_set_error("pkv_retrieve_noalloc: this shape needs %zu bytes of scratch, the fixed array holds %zu "
                   "(rows=%d n_keys=%lld n_cand=%lld k=%lld); use pkv_retrieve with a workspace of the caller's",
@@ -339,7 +347,7 @@ extern "C" int pkv_retrieve_noalloc(const pkv_retrieve_args *a, void *stream) {
   void *ws = nullptr;
   const int rc = scratch_for_current_device(&ws);
   if (rc) return rc;
-  return retrieve_impl(a, ws, (size_t)PKV_NOALLOC_SCRATCH_BYTES, stream);
+  return retrieve_impl(a, ws, (size_t)PKV_NOALLOC_SCRATCH_BYTES, stream, nullptr, least_chunk);
 }
 
 extern "C" int pkv_decode_step(const pkv_retrieve_args *retrieve, void *ws, size_t ws_bytes,

@@ -183,3 +183,17 @@ def test_prefill_store_has_room_for_the_longest_rows():
         a.n_encode = n
         assert L.pkv_prefill_store(a, None) == _lib.EINVAL
         assert (b"token counts" not in L.pkv_last_error()) == ok, (n, L.pkv_last_error())
+
+
+def test_noalloc_scratch_takes_the_shapes_of_the_largest_chunks():
+    """Rows scanned in chunks below 2048 keys need more room for histograms: near the end of the fixed scratch array such a shape
+    is scanned in larger chunks instead of being refused.  (Shapes that the check lets through end at the null pointers.)"""
+    from pariskv_amd import _lib
+
+    L = _lib.lib()
+    room = L.pkv_retrieve_noalloc_max_bytes()
+    for rows, n, c, ok in ((75, 13065, 13065, True), (58, 17168, 16996, True), (31, 32217, 32217, True), (8, 4096, 2048, True),
+                           (76, 13165, 13165, False), (31, 33217, 33217, False)):
+        a = _lib.RetrieveArgs()
+        a.dtype, a.bs, a.n_kv_heads, a.group, a.n_keys, a.n_cand, a.k, a.cap, a.out_ids = _lib.DTYPE_BF16, 1, rows, 1, n, c, c, n, 256
+        assert (L.pkv_retrieve_noalloc(a, None) != _lib.ENOMEM) == ok, (rows, n, c, L.pkv_retrieve_ws_bytes(rows, n, c, c), room)

@@ -98,3 +98,26 @@ def test_noalloc_rejects_what_it_cannot_hold():
     assert lib.pkv_retrieve_noalloc(C.byref(a), stream) == 0
     torch.cuda.synchronize()
     assert np.array_equal(ids[0, 0].cpu().numpy(), W.oracle_stages(w, 0)["final"])
+
+
+def test_noalloc_scans_in_larger_chunks_where_the_scratch_is_nearly_full():
+    """A shape whose small chunks' histograms would not fit the fixed array: same ids and scores as with a workspace."""
+    from pariskv_amd import _lib, ops
+
+    bs, H, G, N, C, K = 2, 29, 2, 17168, 16996, 16996
+    print(f"no-alloc: {bs * H} rows x {N} keys, {C} candidates", flush=True)
+    assert _lib.lib().pkv_retrieve_ws_bytes(bs * H, N, C, K) > _lib.lib().pkv_retrieve_noalloc_max_bytes()
+    g = torch.Generator(device=DEV).manual_seed(1)
+    codes_km, nib_km, w_km, cb, k4, kw = ops.alloc_keymajor(bs, H, N, DEV)
+    cc = torch.zeros(bs, H, 16, 256, dtype=torch.int32, device=DEV)
+    signs, centers = ops.srht_signs(DEV), ops.mag_centers(DEV)
+    ops.encode_append(torch.randn(bs, H, N, 128, generator=g, device=DEV).to(torch.bfloat16), signs, cb, k4, kw, cc)
+    q = torch.randn(bs, 1, H * G, 128, generator=g, device=DEV).to(torch.bfloat16)
+    args = (q, signs, centers, cc, codes_km, nib_km, w_km, 0, N, O.tier_counts(N, 0.3), C, K)
+    out = []
+    plan = ops.RetrievePlan(bs, H, G, N, DEV, N, C, K)
+    for run in (plan.run, ops.retrieve_noalloc):
+        ids, scores = torch.empty(bs, H, K, dtype=torch.int64, device=DEV), torch.empty(bs, H, K, device=DEV)
+        run(*args, ids, out_scores=scores)
+        out.append((ids, scores))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
