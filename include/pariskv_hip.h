@@ -186,6 +186,11 @@ int pkv_collision_scan(const uint8_t *codes, int64_t cs_b, int64_t cs_h, int64_t
                        uint8_t *cnt_u8, int32_t *cnt_i32, uint32_t *row_suf, uint16_t *chunk_suf,
                        int chunk_keys, void *stream);
 
+/* Keys per chunk that pkv_retrieve scans rows of n_keys keys in (a power of two of
+ * 256 .. 32768), for callers that scan on their own.
+ * No counterpart in the reference. */
+int pkv_scan_chunk_keys(int rows, int64_t n_keys);
+
 /* pkv_collision_scan (u8 counts, row stride cnt_u8_stride) as ONE launch whose
  * own begin/end timestamps are returned in *kernel_us: the call blocks until
  * the kernel has finished.  Measurement aid for the benchmark's roofline line;

@@ -304,6 +304,8 @@ int pkv_launch_scan_i32_codes(const int32_t *codebook, int rows, int64_t n_keys,
   return PKV_OK;
 }
 
+extern "C" int pkv_scan_chunk_keys(int rows, int64_t n_keys) { return pkv_pick_chunk_keys(rows, n_keys); }
+
 extern "C" int pkv_collision_scan(const uint8_t *codes, int64_t cs_b, int64_t cs_h, int64_t cs_key, int64_t cs_sub,
                                   int bs, int n_kv_heads, int64_t n_keys, const uint8_t *lut, uint8_t *cnt_u8,
                                   int32_t *cnt_i32, uint32_t *row_suf, uint16_t *chunk_suf, int chunk_keys,

@@ -308,12 +308,8 @@ def update_cache_cnt_legacy(sorted_cluster_ids: torch.Tensor, topk_cluster_cnt: 
 
 
 def pick_chunk_keys(rows: int, n_keys: int) -> int:
-    chunk = 2048
-    while chunk < 16384 and rows * ((n_keys + chunk - 1) // chunk) > 1024:
-        chunk *= 2
-    while chunk < 32768 and (n_keys + chunk - 1) // chunk > 512:
-        chunk *= 2
-    return chunk
+    """Keys per chunk that the retrieval scans such rows in (pkv_scan_chunk_keys)."""
+    return _lib.lib().pkv_scan_chunk_keys(rows, n_keys)
 
 
 def collision_scan(codebook: torch.Tensor, lut: torch.Tensor, out_dtype=torch.int32, want_hist: bool = False):

@@ -197,3 +197,19 @@ def test_noalloc_scratch_takes_the_shapes_of_the_largest_chunks():
         a = _lib.RetrieveArgs()
         a.dtype, a.bs, a.n_kv_heads, a.group, a.n_keys, a.n_cand, a.k, a.cap, a.out_ids = _lib.DTYPE_BF16, 1, rows, 1, n, c, min(c, 8192), n, 256
         assert (L.pkv_retrieve_noalloc(a, None) != _lib.ENOMEM) == ok, (rows, n, c, L.pkv_retrieve_ws_bytes(rows, n, c, min(c, 8192)), room)
+
+
+def test_one_chunk_rule():
+    """ops.pick_chunk_keys (stand-alone scans) is the rule the retrieval lays its workspace out by: a row's histogram table
+    there holds one entry a chunk, or four where chunks of 8192 keys and more are scanned in pieces."""
+    from pariskv_amd import _lib, ops
+
+    L = _lib.lib()
+    for rows in (1, 2, 3, 8, 12, 64, 200, 1500):
+        for n in (1, 255, 256, 257, 4000, 8192, 8193, 16385, 33000, 131072, 1000003, 1 << 24):
+            chunk = ops.pick_chunk_keys(rows, n)
+            n_chunks = -(-n // chunk)
+            ptr, nbytes = ctypes.c_void_p(), ctypes.c_size_t()
+            _lib.check(L.pkv_retrieve_ws_view(256, rows, n, n, 1, b"chunk_suffix_hist", ctypes.byref(ptr), ctypes.byref(nbytes)))
+            pieces = 4 if chunk >= 8192 and 4 * n_chunks <= 512 else 1
+            assert nbytes.value == rows * n_chunks * pieces * 256, (rows, n, chunk)
