@@ -33,6 +33,9 @@ USE_RABITQ_RERANK = True
 # Offloading layers attend to every token while the sequence is below the dense-attention threshold; up to this threshold
 # the rows such a step needs also stay in HBM (see polar_cache._short_rows)
 SHORT_ROWS_MAX = 4096
+# ... and all layers' such rows together take at most this share of the card's memory (1/32 of 288 GB = 9 GB: 36 layers x 8 KV
+# heads at the default threshold for 43 sequences), so that a cache sized for the card without them still fits
+SHORT_ROWS_SHARE = 32
 DEFAULT_SRHT_ROUNDS = 1
 
 
@@ -160,6 +163,7 @@ class polar_cache(KV_Cache):
             "host_layers": n_host, "hbm_layers": layer_num - n_host,
             "host_pinned_bytes": n_host * layer_host_bytes,
             "hbm_kv_bytes": sum(2 * bs * H * r * D * esz for r in self._gpu_rows),
+            "hbm_short_rows_bytes": 0,  # held at present by the zone rows of short sequences, see _short_rows
             "host_kv_budget_bytes": host_kv_budget_bytes,
         }
 
@@ -264,20 +268,30 @@ class polar_cache(KV_Cache):
         """Where the prefill of samples b0..b1-1 puts the retrieval-zone rows of a prompt that is still below the
         dense-attention threshold: K/V [b1-b0,H,rows,D] in HBM, beside the host store.  Every step of such a sequence
         attends to all of its tokens; read from the host they cost a wait for the copy stream and two strided copies over
-        PCIe per layer and token (235 us for 924 rows x 8 heads), from HBM 7 us.  At most SHORT_ROWS_MAX rows a head;
-        given back by the first step that retrieves; every stream that works on them is told to the allocator (a decode on
-        another stream than the prefill's may still have attention over them queued then).  None for longer prompts or a threshold too high for that."""
+        PCIe per layer and token (235 us for 924 rows x 8 heads), from HBM 7 us.  At most SHORT_ROWS_MAX rows a head and a
+        share of the card for all layers (kv_placement reports what is held); given back by the first step that retrieves.
+        Every stream that works on them is told to the allocator: a decode on another stream than the prefill's may still
+        have attention over them queued then.  None for longer prompts and beyond those bounds: such a step reads the host."""
         rows = self._min_total() - self.sink_size - self.local_size
         self._dense_bound[layer_idx] = None
         if n_tok >= self._min_total() or rows > SHORT_ROWS_MAX:
-            self._short_kv[layer_idx] = None
+            self._drop_short_rows(layer_idx)
             return None
         kv = self._short_kv[layer_idx]
         if kv is None or kv[0].shape[2] < rows:
+            self._drop_short_rows(layer_idx)
             shape = (self.batch_size, self.kv_head, rows, self.head_dim)
-            kv = (torch.empty(shape, dtype=self.dtype, device=self.device),
-                  torch.empty(shape, dtype=self.dtype, device=self.device), [False] * self.batch_size)
+            more = 2 * math.prod(shape) * torch.empty((), dtype=self.dtype).element_size()
+            most = torch.cuda.get_device_properties(self.device).total_memory // SHORT_ROWS_SHARE
+            if self.kv_placement["hbm_short_rows_bytes"] + more > most:
+                return None
+            try:
+                kv = (torch.empty(shape, dtype=self.dtype, device=self.device),
+                      torch.empty(shape, dtype=self.dtype, device=self.device), [False] * self.batch_size)
+            except torch.cuda.OutOfMemoryError:
+                return None
             self._short_kv[layer_idx] = kv
+            self.kv_placement["hbm_short_rows_bytes"] += more
         self._record_short_rows(kv)
         kv[2][b0:b1] = [True] * (b1 - b0)   # samples whose rows are here: prompts may arrive one by one
         return kv[0][b0:b1], kv[1][b0:b1]
@@ -290,6 +304,9 @@ class polar_cache(KV_Cache):
     def _drop_short_rows(self, layer_idx: int) -> None:
         """The sequence has outgrown the dense branch: its retrieval-zone rows in HBM go back to the allocator, and with them
         the argument block that holds them."""
+        kv = self._short_kv[layer_idx]
+        if kv is not None:
+            self.kv_placement["hbm_short_rows_bytes"] -= 2 * kv[0].numel() * kv[0].element_size()
         self._short_kv[layer_idx] = self._dense_bound[layer_idx] = None
 
     def release_prefill_staging(self) -> None:

@@ -1200,3 +1200,36 @@ def test_outgrown_adaptive_scratch_outlives_the_stream_that_uses_it():
                 pytest.skip("the decode stream was done before the check")
             assert not {o[0] for o in gone} & {t.data_ptr() for t in taken}
         torch.cuda.synchronize()
+
+
+def test_short_rows_are_reported_and_bounded(monkeypatch):
+    """HBM taken by the zone rows of short sequences shows in kv_placement while it is held, and stays below a share of the
+    card's memory; a cache beyond that reads such rows from the host, with the same results."""
+    from pariskv_amd.cache_hub import polar_cache as module
+
+    bs, H, group, layers, S, thr, steps = 2, 2, 4, 2, 250, 260, 16
+    sink, local = 4, 64
+    caches = [_cache_of("fixed", True, bs, H, group, S, steps, sink, local, 16, 50, thr, layers=layers) for _ in range(2)]
+    held = 2 * bs * H * (thr - sink - local) * 128 * 2
+    gen = torch.Generator().manual_seed(6)
+    assert caches[0].kv_placement["hbm_short_rows_bytes"] == 0
+    share = module.SHORT_ROWS_SHARE
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    for l in range(layers):
+        k, v = (t.to(DEV) for t in _synth_kv(gen, bs, S, H))
+        caches[0].prefill_update_kv_cache(None, k, v, l, 0)
+        assert caches[0].kv_placement["hbm_short_rows_bytes"] == held * (l + 1)
+        monkeypatch.setattr(module, "SHORT_ROWS_SHARE", total // (held + 1))   # room for one layer, not for two
+        caches[1].prefill_update_kv_cache(None, k, v, l, 0)
+        monkeypatch.setattr(module, "SHORT_ROWS_SHARE", share)
+        assert caches[1].kv_placement["hbm_short_rows_bytes"] == held
+    for step in range(steps):
+        for l in range(layers):
+            k1, v1 = (t.to(DEV) for t in _synth_kv(gen, bs, 1, H))
+            q = torch.randn(bs, 1, H * group, 128, generator=gen).to(torch.bfloat16).to(DEV)
+            out = []
+            for c in caches:
+                c.decode_update_kv_cache(k1, v1, l)
+                out.append(c.compute(q, l))
+            assert torch.equal(out[0], out[1])
+    assert [c.kv_placement["hbm_short_rows_bytes"] for c in caches] == [0, 0]
