@@ -326,7 +326,7 @@ class polar_cache(KV_Cache):
         if any(t.stride(3) != 1 or t.data_ptr() % 16 or any(x % vec for x in t.stride()[:3]) for t in (k, v)):
             # a clone, as contiguous() hands a tensor that is contiguous but misaligned back as it is
             k, v = (t.clone(memory_format=torch.contiguous_format) for t in (k, v))
-        index = zone_norms = None
+        index = None
         if n_encode > 0:
             sl = slice(abs0, abs0 + n_encode)
             index = (self.codebook_gpu[layer_idx][b0:b1, :, :, sl], self.key_4bit_packed_gpu[layer_idx][b0:b1, :, :, sl],
@@ -459,14 +459,12 @@ class polar_cache(KV_Cache):
         """Where the launch that stores rows leaves their value norms (keyword arguments of ``ops.prefill_store``)."""
         return {}
 
-    def _append(self, layer_idx, slot, key_states, value_states):
+    def _append(self, layer_idx, slot, key_states, value_states, vnorm=None):
         bound = self._append_bound[layer_idx]
         if bound is None:
-            bound = self._append_bound[layer_idx] = self._bind_append(layer_idx)
+            bound = ops.BoundAppend(self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx], vnorm)
+            self._append_bound[layer_idx] = bound
         bound.launch(key_states, value_states, slot)
-
-    def _bind_append(self, layer_idx):
-        return ops.BoundAppend(self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx])
 
     def _on_refresh(self, layer_idx, r):
         pass

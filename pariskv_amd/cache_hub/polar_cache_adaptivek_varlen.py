@@ -105,11 +105,7 @@ class polar_cache(_polar_cache_base):
 
     def _append(self, layer_idx, slot, key_states, value_states):
         """K/V rows and the value norm of the new token (:1179) in one launch."""
-        super()._append(layer_idx, slot, key_states, value_states)
-
-    def _bind_append(self, layer_idx):
-        return ops.BoundAppend(self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx],
-                               vnorm=self._sl_vnorm_cache[layer_idx])
+        super()._append(layer_idx, slot, key_states, value_states, vnorm=self._sl_vnorm_cache[layer_idx])
 
     def _on_refresh(self, layer_idx, r):
         S0, n, L = self.sink_size, r.n_new, self.local_size
