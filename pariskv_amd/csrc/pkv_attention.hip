@@ -550,9 +550,11 @@ __global__ void pkv_attn_merge_kernel(const float *__restrict__ ws, int n_splits
     ((float *)out)[oi] = os;
 }
 
+// rows: times the workgroups that a KV head's query heads take (two for five to eight heads).
 int pick_splits(int rows, int64_t total) {
-  // One round of workgroups: with four query heads the kernel holds 3 workgroups per CU (768 on the chip);
-  // a few more would run as a second round and double the launch's duration.
+  // One round of workgroups: with four query heads the kernel holds 3 workgroups per CU (768 on the chip); more would run as
+  // a second round.  us with the second four heads' workgroups left out of this count / with them, 8 heads:
+  // 32 rows x 1600 keys 31.7 / 26.6, 64 x 800 30.8 / 26.6, 256 x 800 80.8 / 75.2, 24 x 1600 22.5 / 22.4, 8 x 6000 27.7 / 25.6.
   int64_t s = 768 / rows;
   const int64_t max_by_len = (total + 63) / 64;  // at least 64 keys per split
   if (s > max_by_len) s = max_by_len;
@@ -645,7 +647,9 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
   PKV_REQUIRE(total < ((int64_t)1 << 23), "pkv_decode_attention: at most 2^23 - 1 keys (got %lld)", (long long)total);
   const int rows = bs * n_kv_heads;
   const bool bf = dtype == PKV_DTYPE_BF16;
-  const int n_splits = bf ? pick_splits_mfma(rows, total) : pick_splits(rows, total);
+  const int heads_per_wg = group == 1 ? 1 : group == 2 ? 2 : 4;  // fp32 kernel
+  const int head_wgs = (group + heads_per_wg - 1) / heads_per_wg;
+  const int n_splits = bf ? pick_splits_mfma(rows, total) : pick_splits(rows * head_wgs, total);
   const size_t need = (size_t)rows * n_splits * group * kPartStride * sizeof(float);
   if (ws_bytes < need || !pkv_aligned(ws, 16)) {
     pkv_set_error("pkv_decode_attention: workspace of %zu bytes required, got %zu", need, ws_bytes);
@@ -673,15 +677,14 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
   } else {
     // The KV head's other query heads in workgroups beside the first four's, in one launch: 12 rows x 865 keys, seven
     // heads, 2 x 8.0 us as two launches one after the other; the decode step around it (9001 keys) 48.3 -> 43 us.
-    const int per_wg = group == 1 ? 1 : group == 2 ? 2 : 4;
-    grid.z = (unsigned)((group + per_wg - 1) / per_wg);
+    grid.z = (unsigned)head_wgs;
 #define PKV_ATT(GG, IDX, S)                                                                                               \
   hipLaunchKernelGGL((pkv_attn_partial_kernel<false, GG, IDX, decltype(S)>), grid, dim3(kAttThreads), 0, s, q, n_kv_heads, group, \
                      S, total, row_keys, uniform, per_split, scale_log2e, (float *)ws)
 #define PKV_ATT_G(IDX, S)                     \
   do {                                        \
-    if (per_wg == 1) PKV_ATT(1, IDX, S);      \
-    else if (per_wg == 2) PKV_ATT(2, IDX, S); \
+    if (heads_per_wg == 1) PKV_ATT(1, IDX, S);      \
+    else if (heads_per_wg == 2) PKV_ATT(2, IDX, S); \
     else PKV_ATT(4, IDX, S);                  \
   } while (0)
     if (is_one) {
