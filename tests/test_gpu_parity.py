@@ -1900,3 +1900,60 @@ def test_bound_append_refuses_a_slot_behind_the_norms(ops):
             bound.launch(k, v, slot)
     torch.cuda.synchronize()
     assert torch.all(dk[:, :, [4, 7]] == 1) and torch.all(dk[:, :, [0, 1, 2, 3, 5, 6]] == 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("layout", ["subspace", "packed", "records"])
+@pytest.mark.parametrize("norms", [False, True])
+@pytest.mark.parametrize("n_enc", [1, 255, 257, 1033])
+def test_prefill_store_index_layouts(ops, dtype, layout, norms, n_enc):
+    """The index layouts that pkv_prefill_store takes beside whole key records with their norms: subspace-major and packed
+    tensors with norms in a tensor of their own (or none), records with none or with norms elsewhere.  Index, rows and norms
+    equal pkv_encode_append's and the records form's; what lies behind the encoded keys stays as it was."""
+    bs, H, n_sink, n_tail, cap = 2, 3, 3, 66, n_enc + 5
+    _say(f"prefill_store {dtype} {layout} norms={norms} {n_enc}")
+    gen = torch.Generator().manual_seed(n_enc)
+    k, v = (torch.randn(bs, n_sink + n_enc + n_tail, H, 128, generator=gen).to(dtype).to(DEV).permute(0, 2, 1, 3) for _ in range(2))
+    signs = ops.srht_signs(DEV)
+
+    def index(form):
+        if form == "records":
+            _, nib, w, cb, k4, kw = ops.alloc_keymajor(bs, H, cap, DEV)
+            return cb, k4, kw
+        if form == "subspace":
+            return (torch.zeros(bs, H, 16, cap, dtype=torch.uint8, device=DEV), torch.zeros(bs, H, 16, cap, 4, dtype=torch.uint8, device=DEV),
+                    torch.zeros(bs, H, 16, cap, dtype=torch.bfloat16, device=DEV))
+        return (torch.zeros(bs, H, cap, 16, dtype=torch.uint8, device=DEV).permute(0, 1, 3, 2),
+                torch.zeros(bs, H, cap, 16, 4, dtype=torch.uint8, device=DEV).permute(0, 1, 3, 2, 4),
+                torch.zeros(bs, H, cap, 16, dtype=torch.bfloat16, device=DEV).permute(0, 1, 3, 2))
+
+    def store(form, **kw_norms):
+        cb, k4, kw = index(form)
+        cc = torch.ones(bs, H, 16, 256, dtype=torch.int32, device=DEV)
+        dk, zk = (torch.full((bs, H, n, 128), 7.0, dtype=dtype, device=DEV) for n in (n_sink + n_tail + 2, cap))
+        dv, zv = dk.clone(), zk.clone()
+        ops.prefill_store(k, v, n_sink, n_enc, signs, (dk, dv), n_sink, (zk, zv),
+                          (cb[..., :n_enc], k4[:, :, :, :n_enc], kw[..., :n_enc], cc), **kw_norms)
+        return cb, k4, kw.contiguous().view(torch.int16), cc, dk, dv, zk, zv
+
+    # the form the caches use, for rows and norms
+    _, nib, _, cb, k4, kw = ops.alloc_keymajor(bs, H, cap, DEV)
+    want_n = ops.record_value_norm_view(nib)
+    dn = torch.zeros(bs, H, n_sink + n_tail, device=DEV)
+    rows = [torch.full((bs, H, n, 128), 7.0, dtype=dtype, device=DEV) for n in (n_sink + n_tail + 2, cap) for _ in range(2)]
+    ops.prefill_store(k, v, n_sink, n_enc, signs, rows[:2], n_sink, rows[2:],
+                      (cb[..., :n_enc], k4[:, :, :, :n_enc], kw[..., :n_enc], torch.zeros(bs, H, 16, 256, dtype=torch.int32, device=DEV)),
+                      dense_vnorm=dn, zone_vnorm=want_n[..., :n_enc])
+    cb2, k42, kw2 = index(layout)
+    cc2 = torch.ones(bs, H, 16, 256, dtype=torch.int32, device=DEV)
+    ops.encode_append(k[:, :, n_sink:n_sink + n_enc], signs, cb2[..., :n_enc], k42[:, :, :, :n_enc], kw2[..., :n_enc], cc2)
+    extra, zn = {}, torch.full((bs, H, cap, 3), 7.0, device=DEV)   # every third word: any key stride
+    if norms:
+        extra = dict(zone_vnorm=zn[:, :, :n_enc, 1])
+    got = store(layout, **extra)
+    for a, b in zip(got, (cb2, k42, kw2.contiguous().view(torch.int16), cc2, *rows)):
+        assert torch.equal(a, b)
+    want = torch.full_like(zn, 7.0)
+    if norms:
+        want[:, :, :n_enc, 1] = want_n[..., :n_enc]
+    assert torch.equal(zn, want)
