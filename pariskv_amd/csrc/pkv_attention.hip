@@ -446,6 +446,7 @@ __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_k
     mx = fmaxf(mx, __shfl_xor(mx, 16, PKV_WAVE));
     mx = fmaxf(mx, __shfl_xor(mx, 32, PKV_WAVE));
     const float m_new = fmaxf(m_run, mx);
+    // the hardware's exp2: exp2f but for results below 2^-126, which are zero; nothing beside the largest weight, which is 1
     const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
     m_run = m_new;
     float p[8], psum = 0.f;

@@ -59,6 +59,9 @@ struct PkvTiers {
 // the histograms of the chunks before it.  us per decode step with chunks of 256 / 512 / 1024 / 2048 keys:
 //   8 rows x 3.5K 32.2 / 34.1 / - / 39.5,  8 x 7.6K 32.8 / 33.1 / - / 38.0,  8 x 16K 34.8 / 33.9 / - / 37.5,
 //   8 x 32K - / 37.2 / 36.5 / 38.0,  32 x 11K - / 35.8 / 37.0 / 37.9,  32 x 32K - / - / 40.0 / 40.8.
+// One to three rows, where the 128 workgroups decide: us per retrieval (no attention) with up to 32 chunks to a row / up to 128
+// workgroups: 1 x 16K 18.6 / 18.8, 1 x 32K 19.1 / 20.1, 1 x 33K 20.2 / 18.8, 1 x 65K 22.9 / 21.3, 2 x 20K 20.8 / 19.1,
+// 2 x 33K 21.3 / 19.2, 2 x 65K 23.5 / 21.1, 3 x 33K 21.8 / 19.2.
 // Always a power of two of 256 .. 32768 (a chunk's histogram bins are uint16).
 // least: the smallest chunk to consider (a power of two of 256 .. 2048).
 static inline int pkv_pick_chunk_keys(int rows, int64_t n_keys, int least = 256) {

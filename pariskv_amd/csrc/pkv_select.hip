@@ -2181,7 +2181,7 @@ int pkv_launch_select(const uint8_t *cnt_u8, int64_t cnt_stride, const uint32_t 
 #define PKV_SEL(KPT)                                                                                                       \
   hipLaunchKernelGGL(pkv_select_kernel<KPT>, grid, dim3(kSelThreads), 0, s, cnt_u8, cnt_stride, row_suf, chunk_suf, chunk_keys, \
                      n_keys, k, out)
-  if (chunk_keys <= 256) PKV_SEL(1);  // one pass per chunk, as in pkv_launch_select_rerank
+  if (chunk_keys <= 256) PKV_SEL(1);  // as in pkv_launch_select_rerank
   else if (chunk_keys <= 1024) PKV_SEL(4);
   else if (chunk_keys <= 2048) PKV_SEL(8);
   else PKV_SEL(16);
@@ -2223,7 +2223,8 @@ int pkv_launch_select_rerank(const uint8_t *cnt_u8, int64_t cnt_stride, const ui
     PKV_LAUNCH_CHECK("pkv_select_rerank_pieces_kernel");
     return PKV_OK;
   }
-  // as many counts per thread as make one pass of the chunk (chunks are powers of two from 256 keys on)
+  // 1, 4, 8 and 16 counts per thread: one pass of a chunk of 256, 1024, 2048 and 4096 keys (chunks are powers of two from 256 keys
+  // on).  Chunks of 512 keys take the form with 4, in which half of the threads have none.
 #define PKV_SR(KPT)                                                                                                           \
   hipLaunchKernelGGL(pkv_select_rerank_kernel<KPT>, grid, dim3(kSelThreads), 0, s, cnt_u8, cnt_stride, row_suf, chunk_suf,    \
                      chunk_keys, n_kv_heads, n_keys, k, nib, ns_b, ns_h, (int)ns_key, weight, ws_b, ws_h, (int)ws_key, qhat,  \
