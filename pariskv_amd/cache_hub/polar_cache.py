@@ -363,6 +363,10 @@ class polar_cache(KV_Cache):
         kg, vg = self.unified_keys_gpu[layer_idx], self.unified_values_gpu[layer_idx]
         last = (layer_idx == self.layer_num - 1) and (b1 == self.batch_size)
         dense = kg[b0:b1], vg[b0:b1]
+        # nothing of an earlier prompt in this cache counts: prefill assigns, refresh accumulates (:493, :775)
+        self.cluster_key_counts_gpu[layer_idx][b0:b1].zero_()
+        if self._layer_offload[layer_idx]:
+            self.cpu_valid_end[layer_idx] = retrieval
         if retrieval == 0:  # short prompt: everything stays dense on the GPU (:430-440)
             n = min(n_tok, self._gpu_rows[layer_idx])
             self._store_rows(layer_idx, k[:, :, :n], v[:, :, :n], b0, b1, n, 0, dense, 0, None, 0)
@@ -370,7 +374,6 @@ class polar_cache(KV_Cache):
                 self.context += n
             return key_states[:, vs:], value_states[:, vs:]
         S0, r_end = self.sink_size, self.sink_size + retrieval
-        self.cluster_key_counts_gpu[layer_idx][b0:b1].zero_()  # prefill assigns, refresh accumulates (:493, :775)
         if self._layer_offload[layer_idx]:
             self._wait_offload(layer_idx)
             short = self._short_rows(layer_idx, b0, b1, n_tok)
@@ -382,7 +385,6 @@ class polar_cache(KV_Cache):
             event = self._offload_rows(layer_idx, b0, b1, stage_k, stage_v, 0)
             if short is None:
                 self._prefill_stage_event[slot] = event
-            self.cpu_valid_end[layer_idx] = retrieval
         else:
             self._store_rows(layer_idx, k, v, b0, b1, S0, retrieval, dense, r_end, (dense[0][:, :, S0:], dense[1][:, :, S0:]), S0)
         if last:

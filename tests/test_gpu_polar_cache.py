@@ -1233,3 +1233,26 @@ def test_short_rows_are_reported_and_bounded(monkeypatch):
                 out.append(c.compute(q, l))
             assert torch.equal(out[0], out[1])
     assert [c.kv_placement["hbm_short_rows_bytes"] for c in caches] == [0, 0]
+
+
+@pytest.mark.parametrize("form,offload", [("fixed", True), ("fixed", False), ("varlen", True), ("dense", False)])
+def test_short_prompt_after_a_long_one_equals_a_fresh_cache(form, offload):
+    """A prompt without a retrieval zone in a cache that held a longer one before: every step, from the dense branch over the
+    first refreshes to retrieval, equals that of a cache that never held another prompt."""
+    bs, H, group, steps = 2, 2, 4, 330
+    caches = [_cache_of(form, offload, bs, H, group, 700, steps + 4, 4, 64, 100, 20, 100) for _ in range(2)]
+    gen = torch.Generator().manual_seed(12)
+    caches[0].prefill_update_kv_cache(None, *(t.to(DEV) for t in _synth_kv(gen, bs, 700, H)), 0, 0)
+    caches[0].compute(torch.randn(bs, 1, H * group, 128, generator=gen).to(torch.bfloat16).to(DEV), 0)
+    k, v = (t.to(DEV) for t in _synth_kv(gen, bs, 50, H))
+    for c in caches:
+        c.context = 0
+        c.prefill_update_kv_cache(None, k, v, 0, 0)
+    for step in range(steps):
+        k1, v1 = (t.to(DEV) for t in _synth_kv(gen, bs, 1, H))
+        q = torch.randn(bs, 1, H * group, 128, generator=gen).to(torch.bfloat16).to(DEV)
+        out = []
+        for c in caches:
+            c.decode_update_kv_cache(k1, v1, 0)
+            out.append(c.compute(q, 0))
+        assert torch.equal(out[0], out[1]), step
