@@ -54,12 +54,11 @@ def _cuda(*ts):
             _need(t.is_cuda, "tensor must be on the GPU")
 
 
-def _one_device(*ts):
-    first = None
-    for t in ts:
-        if t is not None:
-            first = t if first is None else first
-            _need(t.device == first.device, f"tensors of one launch are on {first.device} and {t.device}")
+def _one_device(first, *others):
+    at = first.get_device()
+    for t in others:
+        if t is not None and t.get_device() != at:
+            raise RuntimeError(f"tensors of one launch are on {first.device} and {t.device}")
 
 
 def _philox4x32_10(ctr, key):
@@ -166,12 +165,12 @@ def prefill_store(k: torch.Tensor, v: torch.Tensor, n_sink: int, n_encode: int, 
     row, ``zone_vnorm`` / ``zone_vnorm2`` [bs,H,n_encode]."""
     bs, H, S, D = k.shape
     n_tail = S - n_sink - n_encode
-    _cuda(k, v)
+    _cuda(k)
+    _one_device(k, v, signs if n_encode else None, *(dense or ()), *(zone or ()), *(index or ()), dense_vnorm, zone_vnorm,
+                zone_vnorm2)
     _need(D == HEAD_DIM and v.shape == k.shape and v.dtype == k.dtype and n_sink >= 0 and n_encode >= 0 and n_tail >= 0,
           "k, v: [bs,H,S,128] of one dtype, n_sink + n_encode <= S")
     _need(k.stride(3) == 1 and v.stride(3) == 1, "k, v: contiguous rows")
-    _one_device(k, v, signs if n_encode else None, *(dense or ()), *(zone or ()), *(index or ()), dense_vnorm, zone_vnorm,
-                zone_vnorm2)
     a = _lib.PrefillArgs()
     a.k, a.v, a.dtype, a.bs, a.n_kv_heads = k.data_ptr(), v.data_ptr(), _dt(k.dtype), bs, H
     a.k_stride_b, a.k_stride_h, a.k_stride_key = k.stride()[:3]
@@ -180,14 +179,12 @@ def prefill_store(k: torch.Tensor, v: torch.Tensor, n_sink: int, n_encode: int, 
 
     def rows_of(pair, need):
         dk, dv = pair
-        _cuda(dk, dv)
         _need(dk.dtype == k.dtype and dv.dtype == k.dtype and dk.shape == dv.shape and dk.stride() == dv.stride() and
               tuple(dk.shape[:2]) == (bs, H) and dk.shape[3] == D and dk.stride(3) == 1 and dk.stride(2) == D and
               dk.shape[2] >= need, f"destination: [bs,H,>={need},128] of the source dtype with contiguous rows")
         return dk.data_ptr(), dv.data_ptr(), dk.stride(0), dk.stride(1)
 
     def norms_of(t, need, unit):
-        _cuda(t)
         _need(t.dtype == torch.float32 and tuple(t.shape[:2]) == (bs, H) and t.shape[2] >= need and
               (not unit or t.stride(2) == 1), f"value norms: fp32 [bs,H,>={need}]")
         return t.data_ptr(), t.stride(0), t.stride(1)
@@ -200,8 +197,7 @@ def prefill_store(k: torch.Tensor, v: torch.Tensor, n_sink: int, n_encode: int, 
     if n_encode > 0:
         a.zone_k, a.zone_v, a.zone_stride_b, a.zone_stride_h = rows_of(zone, n_encode)
         cb, k4, kw, cc = index
-        _cuda(cb, k4, kw, cc)
-        _need(signs.is_cuda and signs.dtype == torch.float32 and signs.numel() == HEAD_DIM and signs.is_contiguous(), "signs: float32[128]")
+        _need(signs.dtype == torch.float32 and signs.numel() == HEAD_DIM and signs.is_contiguous(), "signs: float32[128]")
         _need(cb.dtype == torch.uint8 and tuple(cb.shape) == (bs, H, B_SUB, n_encode), "codebook must be u8 [bs,H,16,n_encode]")
         _need(k4.dtype == torch.uint8 and tuple(k4.shape) == (bs, H, B_SUB, n_encode, 4) and k4.stride(4) == 1,
               "key_4bit must be u8 [bs,H,16,n_encode,4] with a contiguous last dim")

@@ -153,6 +153,9 @@ def test_prefill_store_refuses_operands_of_several_devices():
         def __init__(self, device, t):
             self._t, self.device, self.is_cuda = t, torch.device(device), True
 
+        def get_device(self):
+            return self.device.index
+
         def __getattr__(self, name):
             return getattr(self._t, name)
 
