@@ -120,7 +120,7 @@ class polar_cache(KV_Cache):
         self.unified_values_cpu = [None] * layer_num if enable_offload else None
         self.cpu_valid_end = [0] * layer_num if enable_offload else None
         self._layer_offload = [False] * layer_num
-        self._short_kv = [None] * layer_num  # (k, v, samples present), see _short_rows
+        self._short_kv = [None] * layer_num  # (k, v, samples present, streams told), see _short_rows
         self._offload_keys_buffer = [None] * layer_num
         self._offload_values_buffer = [None] * layer_num
         if enable_offload:
@@ -287,7 +287,7 @@ class polar_cache(KV_Cache):
                 return None
             try:
                 kv = (torch.empty(shape, dtype=self.dtype, device=self.device),
-                      torch.empty(shape, dtype=self.dtype, device=self.device), [False] * self.batch_size)
+                      torch.empty(shape, dtype=self.dtype, device=self.device), [False] * self.batch_size, set())
             except torch.cuda.OutOfMemoryError:
                 return None
             self._short_kv[layer_idx] = kv
@@ -298,8 +298,10 @@ class polar_cache(KV_Cache):
 
     def _record_short_rows(self, kv) -> None:
         stream = torch.cuda.current_stream(self.device)
-        for t in kv[:2]:
-            t.record_stream(stream)
+        if stream.cuda_stream not in kv[3]:
+            for t in kv[:2]:
+                t.record_stream(stream)
+            kv[3].add(stream.cuda_stream)
 
     def _drop_short_rows(self, layer_idx: int) -> None:
         """The sequence has outgrown the dense branch: its retrieval-zone rows in HBM go back to the allocator, and with them
@@ -562,7 +564,8 @@ class polar_cache(KV_Cache):
         n_keys = self.cpu_valid_end[layer_idx] if offload else z.encoded
         if total < self._min_total() or n_keys <= 0:
             return self._attend_all(queries if queries.is_contiguous() else queries.contiguous(), layer_idx, z)
-        self._drop_short_rows(layer_idx)
+        if self._dense_bound[layer_idx] is not None or self._short_kv[layer_idx] is not None:
+            self._drop_short_rows(layer_idx)
         q = queries if queries.is_contiguous() else queries.contiguous()
         step = self._bound[layer_idx]
         if step is None or step[0] != n_keys:

@@ -157,7 +157,8 @@ class polar_cache(_polar_cache_base):
         n_keys = self.cpu_valid_end[layer_idx]
         if total < self._min_total() or n_keys <= 0:
             return super().compute(queries, layer_idx)  # dense branch
-        self._drop_short_rows(layer_idx)
+        if self._dense_bound[layer_idx] is not None or self._short_kv[layer_idx] is not None:
+            self._drop_short_rows(layer_idx)
         q = queries if queries.is_contiguous() else queries.contiguous()
         step = self._adaptive_bound[layer_idx]
         if step is None or step[0] != n_keys:

@@ -554,8 +554,8 @@ class BoundAppend:
         ks, vs, es = k.stride(), v.stride(), self._es
         _need(k.shape == self._shape and v.shape == self._shape and ks[3] == 1 and vs[3] == 1 and k.is_cuda and v.is_cuda,
               "key_states, value_states: [bs,1,Hkv,D] on the GPU with contiguous rows")
-        _need(k.dtype == self._dtype and v.dtype == self._dtype, "append: dtypes differ")
-        _need(0 <= slot < self._slots, "append: the slot lies outside the K/V rows or the value norms")
+        _need(k.dtype == self._dtype and v.dtype == self._dtype and 0 <= slot < self._slots,
+              "append: dtypes differ, or the slot lies outside the K/V rows or the value norms")
         rc = self._fn(self._ra, k.data_ptr(), ks[0] * es, ks[2] * es, v.data_ptr(), vs[0] * es, vs[2] * es, slot,
                       torch.cuda.current_stream(self._device).cuda_stream)
         if rc != 0:
@@ -821,9 +821,9 @@ def gather_cpu(src: torch.Tensor, index: torch.Tensor, out: torch.Tensor, n_thre
 class BoundAttention:
     """The argument block of one layer's pkv_decode_attention, validated once; the caller patches ``segs[i].n_rows``.
     ``lent``: tensors of the segments that the caller may let go while a launch is queued; every stream that launches is
-    told to the allocator once, so that their memory waits for it."""
+    told to the allocator, so that their memory waits for it."""
 
-    __slots__ = ("aa", "segs", "keep", "_raa", "_dims", "_fn", "_numel", "_dtype", "_lent", "_streams")
+    __slots__ = ("aa", "segs", "keep", "_raa", "_dims", "_fn", "_numel", "_dtype", "_lent", "_told")
 
     def __init__(self, att, q, segments, lent=()):
         self.aa, _ = att.c_args(q, segments, out=q)  # out is patched at every launch
@@ -831,7 +831,7 @@ class BoundAttention:
         self._dims = (_dt(q.dtype), att.bs, att.H, att.G)
         self._fn = _lib.lib().pkv_decode_attention_run
         self._numel, self._dtype = q.numel(), q.dtype
-        self._lent, self._streams = lent, set()
+        self._lent, self._told = lent, None
 
     def launch(self, q: torch.Tensor) -> torch.Tensor:
         """q: contiguous [bs,1,Hq,128] of the bound dtype.  Returns the attention output, shaped like q."""
@@ -841,10 +841,10 @@ class BoundAttention:
         self.aa.out = out.data_ptr()
         stream = torch.cuda.current_stream(q.device)
         handle = stream.cuda_stream
-        if self._lent and handle not in self._streams:
+        if handle != self._told:
             for t in self._lent:
                 t.record_stream(stream)
-            self._streams.add(handle)
+            self._told = handle
         rc = self._fn(q.data_ptr(), *self._dims, self._raa, handle)
         if rc != 0:
             _lib.check(rc)
