@@ -18,7 +18,7 @@
 // fp32, probabilities rounded to bf16 before P.V as flash-attn does), exp2 with the scale
 // folded in; the output is rounded to the input dtype.  Not bit-reproducible against another summation order -
 // the tolerance of this row is 2e-2 absolute in bf16.
-#include "pkv_common.h"
+#include "pkv_attn.h"
 
 // Fused multiply-add is welcome here (the rest of the library forbids it because integer results are
 // derived from its float steps; this kernel's only contract is the 2e-2 tolerance).
@@ -26,343 +26,16 @@
 
 namespace {
 
-constexpr int kAttThreads = 256;
-constexpr int kAttKeysPerIter = kAttThreads / 16;  // 16 keys per workgroup step
-constexpr int kAttUnroll = 2;                      // keys per 16-lane group per step
-constexpr float kNegBig = -1.0e30f;
-
-struct AttSegs {
-  const void *k[PKV_ATTN_MAX_SEGMENTS];
-  const void *v[PKV_ATTN_MAX_SEGMENTS];
-  int64_t stride_b[PKV_ATTN_MAX_SEGMENTS], stride_h[PKV_ATTN_MAX_SEGMENTS];
-  int64_t row0[PKV_ATTN_MAX_SEGMENTS];
-  int64_t end[PKV_ATTN_MAX_SEGMENTS];  // exclusive end of the segment in the concatenated key order
-  const int64_t *idx[PKV_ATTN_MAX_SEGMENTS];  // per segment: selected rows (relative to row0) or nullptr
-  int64_t idx_stride[PKV_ATTN_MAX_SEGMENTS], idx_limit[PKV_ATTN_MAX_SEGMENTS];
-  int n;
-};
-
-// Row (inside the (b, h) slab of its segment, row0 included) and segment of concatenated key jj, packed as
-// row | segment << 29.  Indexed segments cost one dependent 8-byte load.
-__device__ __forceinline__ uint32_t att_resolve_row(const AttSegs &segs, int row, uint32_t jj) {
-  int s = 0;
-  uint32_t first = 0;
-#pragma unroll
-  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
-    if (t < segs.n && jj >= (uint32_t)segs.end[t - 1]) s = t, first = (uint32_t)segs.end[t - 1];
-  const int64_t *ip = segs.idx[0];
-  int64_t stride = segs.idx_stride[0], limit = segs.idx_limit[0], row0 = segs.row0[0];
-#pragma unroll
-  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
-    if (s == t) ip = segs.idx[t], stride = segs.idx_stride[t], limit = segs.idx_limit[t], row0 = segs.row0[t];
-  int64_t r = jj - first;
-  if (ip) {
-    r = ip[(int64_t)row * stride + r];
-    r = r < 0 ? 0 : (r >= limit ? limit - 1 : r);
-  }
-  return (uint32_t)(r + row0) | ((uint32_t)s << 29);
-}
-
-// Eight consecutive elements as loaded (16 B of bf16, or 32 B of fp32) and their fp32 values.  Kept
-// apart so that a load can be issued a whole step before its data is touched.
-template <bool BF16>
-struct Raw8 {
-  pkv_u32x4 a;
-  pkv_u32x4 b[BF16 ? 0 : 1];
-};
-
-// Plain loads: two instructions share every 128-byte line of an fp32 row, and a streaming load gives the line up after the first.
-// Decode step, streaming / plain: 12 rows x 865 attended keys, 7 heads (2 layers) 68.6 / 64.8 us.
-template <bool BF16>
-__device__ __forceinline__ void load_raw8(const void *base, int64_t elem_off, Raw8<BF16> &r) {
-  if (BF16) {
-    r.a = *(const pkv_u32x4 *)((const uint16_t *)base + elem_off);
-  } else {
-    r.a = *(const pkv_u32x4 *)((const float *)base + elem_off);
-    r.b[BF16 ? -1 : 0] = *(const pkv_u32x4 *)((const float *)base + elem_off + 4);
-  }
-}
-
-template <bool BF16>
-__device__ __forceinline__ void expand8(const Raw8<BF16> &r, float (&x)[8]) {
-  const uint32_t ww[4] = {r.a.x, r.a.y, r.a.z, r.a.w};
-  if (BF16) {
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      x[2 * p] = __uint_as_float(ww[p] << 16);
-      x[2 * p + 1] = __uint_as_float(ww[p] & 0xffff0000u);
-    }
-  } else {
-    const pkv_u32x4 hi = r.b[BF16 ? -1 : 0];
-    x[0] = __uint_as_float(ww[0]), x[1] = __uint_as_float(ww[1]), x[2] = __uint_as_float(ww[2]);
-    x[3] = __uint_as_float(ww[3]), x[4] = __uint_as_float(hi.x), x[5] = __uint_as_float(hi.y);
-    x[6] = __uint_as_float(hi.z), x[7] = __uint_as_float(hi.w);
-  }
-}
-
-template <bool BF16>
-__device__ __forceinline__ void load8(const void *base, int64_t elem_off, float (&x)[8]) {
-  Raw8<BF16> r;
-  load_raw8<BF16>(base, elem_off, r);
-  expand8<BF16>(r, x);
-}
-
-// Keys row `row` attends to: all `total`, its own row_keys[row], or with uniform > 0 the largest of row_keys[0 .. uniform)
-// (the dense form of the adaptive-k step, where a launch of its own for the maximum took 4.5 us at 24 rows).
-__device__ __forceinline__ int64_t att_row_total(int64_t total, const int32_t *__restrict__ row_keys, int row, int uniform) {
-  if (!row_keys) return total;
-  int64_t rk;
-  if (uniform > 0) {
-    int m = 0;
-    for (int r = pkv_lane(); r < uniform; r += PKV_WAVE) m = max(m, row_keys[r]);
-#define PKV_ATT_MAX(M) { const int o = (int)pkv_lane_xor<M>((uint32_t)m); m = max(m, o); }
-    PKV_ATT_MAX(1) PKV_ATT_MAX(2) PKV_ATT_MAX(4) PKV_ATT_MAX(8) PKV_ATT_MAX(16) PKV_ATT_MAX(32)
-#undef PKV_ATT_MAX
-    rk = __builtin_amdgcn_readfirstlane(m);
-  } else {
-    rk = row_keys[row];
-  }
-  return rk < total ? (rk > 0 ? rk : 1) : total;
-}
-
-// Segments that share one K and one V tensor (the cache's rows in HBM: sink, selected rows, local window), at most one of
-// them indexed: a key is a 32-bit byte offset into the (b, h) slab.  Half of a launch over a few hundred keys used to go
-// into finding addresses (1.2 us to pick a 64-bit pointer out of four for each of a lane's ten rows, after 1 us for a
-// 300-byte argument block); here that is one lane exchange per row.
-struct AttOne {
-  const char *k, *v;
-  int64_t stride_b, stride_h;           // bytes
-  uint32_t end[PKV_ATTN_MAX_SEGMENTS];  // exclusive ends in the concatenated key order; unused: 2^32 - 1
-  int32_t delta[PKV_ATTN_MAX_SEGMENTS]; // row - concatenated key
-  const int64_t *idx;                   // of the indexed segment, keys [idx_lo, idx_hi)
-  int64_t idx_stride, idx_limit;
-  uint32_t idx_lo, idx_hi, idx_row0;
-};
-
-// One key's place: a byte offset into the slab (AttOne), or the addresses of its K and V rows.
-template <bool ONE>
-struct AttPlace {
-  uint32_t off;
-  __device__ __forceinline__ AttPlace from(int lane) const { return {(uint32_t)__shfl((int)off, lane, PKV_WAVE)}; }
-};
-template <>
-struct AttPlace<false> {
-  uint64_t k, v;
-  __device__ __forceinline__ const char *k_from(int lane) const { return (const char *)pull(k, lane); }
-  __device__ __forceinline__ const char *v_from(int lane) const { return (const char *)pull(v, lane); }
-  static __device__ __forceinline__ uint64_t pull(uint64_t x, int lane) {
-    return ((uint64_t)(uint32_t)__shfl((int)(x >> 32), lane, PKV_WAVE) << 32) | (uint32_t)__shfl((int)(uint32_t)x, lane, PKV_WAVE);
-  }
-};
-
-// ROW: bytes of a row.
-template <bool INDEXED, uint32_t ROW>
-__device__ __forceinline__ AttPlace<true> att_place(const AttOne &a, int row, int, int, uint32_t jj) {
-  int32_t d = a.delta[0];
-#pragma unroll
-  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t) d = jj >= a.end[t - 1] ? a.delta[t] : d;
-  uint32_t r = jj + (uint32_t)d;
-  if (INDEXED && jj >= a.idx_lo && jj < a.idx_hi) {
-    const int64_t x = a.idx[(int64_t)row * a.idx_stride + (jj - a.idx_lo)];
-    r = a.idx_row0 + (uint32_t)(x < 0 ? 0 : (x >= a.idx_limit ? a.idx_limit - 1 : x));
-  }
-  return {r * ROW};
-}
-
-template <bool INDEXED, uint32_t ROW>
-__device__ __forceinline__ AttPlace<false> att_place(const AttSegs &a, int row, int b, int h, uint32_t jj) {
-  int s = 0;
-  uint32_t first = 0;
-#pragma unroll
-  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
-    if (t < a.n && jj >= (uint32_t)a.end[t - 1]) s = t, first = (uint32_t)a.end[t - 1];
-  const char *k = (const char *)a.k[0], *v = (const char *)a.v[0];
-  int64_t sb = a.stride_b[0], sh = a.stride_h[0], row0 = a.row0[0];
-#pragma unroll
-  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
-    if (s == t) k = (const char *)a.k[t], v = (const char *)a.v[t], sb = a.stride_b[t], sh = a.stride_h[t], row0 = a.row0[t];
-  const int64_t r = INDEXED ? (int64_t)(att_resolve_row(a, row, jj) & 0x1fffffffu) : row0 + (int64_t)(jj - first);
-  const int64_t off = ((int64_t)b * sb + (int64_t)h * sh) * (ROW / 128) + r * ROW;
-  return {(uint64_t)(k + off), (uint64_t)(v + off)};
-}
-
-// Partial results layout: ws[((row * n_splits + split) * G + g) * 130 + {0: max, 1: sum, 2..129: output}].
-constexpr int kPartStride = 130;
-
-// Splits are of 64 keys while the key set allows: a launch is one chain of dependent loads with some 1000 instructions behind
-// it, not bandwidth.  Places of keys as in the bf16 kernel below.  Decode step, us, with a 64-bit pointer picked out of four for
-// each row / with places: 12 rows x 865 attended keys, 7 heads (2 layers) 74.6 / 70.0, 8 rows x 696 (2 layers) 66.5 / 61.0,
-// 32 rows x 896 48.6 / 45.2.
+// grid (splits, rows, query heads by G)
 template <bool BF16, int G, bool INDEXED, typename SEGS>
 __global__ __launch_bounds__(kAttThreads) void pkv_attn_partial_kernel(const void *__restrict__ q, int n_kv_heads,
                                                                        int group, SEGS segs, int64_t total,
                                                                        const int32_t *__restrict__ row_keys, int uniform,
                                                                        int64_t per_split, float scale_log2e,
                                                                        float *__restrict__ ws) {
-  // blockIdx.z: query heads g0 .. g0 + g_count - 1 of the KV head (more than four would not fit the registers)
-  const int g0 = blockIdx.z * G, g_count = group - g0 < G ? group - g0 : G;
-  const int split = blockIdx.x, row = blockIdx.y;
-  const int b = row / n_kv_heads, h = row % n_kv_heads;
-  const int tid = threadIdx.x;
-  const int lane16 = tid & 15;        // owns dims 8*lane16 .. +7
-  const int grp = tid >> 4;           // 16 key slots per workgroup step
-
-  total = att_row_total(total, row_keys, row, uniform);  // ragged rows
-  const int64_t j0 = (int64_t)split * per_split;
-  const int64_t j1 = (j0 + per_split < total) ? j0 + per_split : total;
-  constexpr bool ONE = __is_same(SEGS, AttOne);
-  constexpr uint32_t kRow = BF16 ? 256 : 512;
-  const int lane = tid & (PKV_WAVE - 1), wave = tid / PKV_WAVE;
-  const char *kbase = nullptr, *vbase = nullptr;
-  if constexpr (ONE) {
-    const int64_t slab = (int64_t)b * segs.stride_b + (int64_t)h * segs.stride_h;
-    kbase = segs.k + slab, vbase = segs.v + slab;
-  }
-  // K/V rows of the step after the current one are requested before the current one is consumed
-  float kx[kAttUnroll][8], vx[kAttUnroll][8];
-  Raw8<BF16> kn[kAttUnroll], vn[kAttUnroll];
-  AttPlace<ONE> mine;
-  auto fetch = [&](int64_t jb, Raw8<BF16> (&kd)[kAttUnroll], Raw8<BF16> (&vd)[kAttUnroll]) {
-    // four turns (64 keys) at a time: lane 4 t + i (mod 16) finds the place of the key that the wave's lanes 16 i .. 16 i + 15
-    // read in turn t
-    static_assert(4 % kAttUnroll == 0 && kAttKeysPerIter == 16, "a wave reads four keys in a turn");
-    const int turn = ((int)(jb - j0) / kAttKeysPerIter) & 3;
-    if (turn == 0) {
-      const int64_t key = jb + ((lane >> 2) & 3) * kAttKeysPerIter + 4 * wave + (lane & 3);
-      mine = att_place<INDEXED, kRow>(segs, row, b, h, (uint32_t)(key < j1 ? key : j1 - 1));  // fewer than 2^24 keys
-    }
-#pragma unroll
-    for (int u = 0; u < kAttUnroll; ++u) {
-      const int at = 4 * (turn + u) + (lane >> 4);
-      const char *kp, *vp;
-      if constexpr (ONE) {
-        const uint64_t off = mine.from(at).off + (kRow / 16) * (uint32_t)lane16;
-        kp = kbase + off, vp = vbase + off;
-      } else {
-        kp = mine.k_from(at) + (kRow / 16) * lane16, vp = mine.v_from(at) + (kRow / 16) * lane16;
-      }
-      load_raw8<BF16>(kp, 0, kd[u]);
-      load_raw8<BF16>(vp, 0, vd[u]);
-    }
-  };
-  if (j0 < j1) fetch(j0, kn, vn);  // before the queries: nothing here waits for them
-
-  float qv[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {  // surplus slots idle
-    load8<BF16>(q, ((int64_t)row * group + g0 + (g < g_count ? g : 0)) * 128 + 8 * lane16, qv[g]);
-#pragma unroll
-    for (int d = 0; d < 8; ++d) qv[g][d] *= scale_log2e;  // scores come out in units of log2(e)
-  }
-  float m[G], l[G], o[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = kNegBig, l[g] = 0.f;
-#pragma unroll
-    for (int d = 0; d < 8; ++d) o[g][d] = 0.f;
-  }
-
-  for (int64_t jb = j0; jb < j1; jb += kAttKeysPerIter * kAttUnroll) {
-    bool valid[kAttUnroll];
-#pragma unroll
-    for (int u = 0; u < kAttUnroll; ++u) {
-      valid[u] = jb + u * kAttKeysPerIter + grp < j1;
-      expand8<BF16>(kn[u], kx[u]);
-      expand8<BF16>(vn[u], vx[u]);
-    }
-    if (jb + kAttKeysPerIter * kAttUnroll < j1) fetch(jb + kAttKeysPerIter * kAttUnroll, kn, vn);
-    float s[G][kAttUnroll];
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-#pragma unroll
-      for (int u = 0; u < kAttUnroll; ++u) {
-        float acc = qv[g][0] * kx[u][0];
-#pragma unroll
-        for (int d = 1; d < 8; ++d) acc += qv[g][d] * kx[u][d];
-        acc += pkv_lane_xor_f<1>(acc);
-        acc += pkv_lane_xor_f<2>(acc);
-        acc += pkv_lane_xor_f<4>(acc);
-        acc += pkv_lane_xor_f<8>(acc);
-        s[g][u] = valid[u] ? acc : kNegBig;
-      }
-    }
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-      float mn = m[g];
-#pragma unroll
-      for (int u = 0; u < kAttUnroll; ++u) mn = fmaxf(mn, s[g][u]);
-      const float corr = exp2f(m[g] - mn);
-      m[g] = mn;
-      float p[kAttUnroll], psum = 0.f;
-#pragma unroll
-      for (int u = 0; u < kAttUnroll; ++u) {
-        p[u] = valid[u] ? exp2f(s[g][u] - mn) : 0.f;
-        psum += p[u];
-      }
-      l[g] = l[g] * corr + psum;
-#pragma unroll
-      for (int d = 0; d < 8; ++d) {
-        float acc = o[g][d] * corr;
-#pragma unroll
-        for (int u = 0; u < kAttUnroll; ++u) acc += p[u] * vx[u][d];
-        o[g][d] = acc;
-      }
-    }
-  }
-
-  // merge the 16 key slots of the workgroup through LDS
-  __shared__ float s_m[16][G], s_l[16][G], s_o[16][G][128 + 4];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    if (lane16 == 0) s_m[grp][g] = m[g], s_l[grp][g] = l[g];
-    *(float4 *)&s_o[grp][g][8 * lane16] = float4{o[g][0], o[g][1], o[g][2], o[g][3]};
-    *(float4 *)&s_o[grp][g][8 * lane16 + 4] = float4{o[g][4], o[g][5], o[g][6], o[g][7]};
-  }
-  __syncthreads();
-  float *part = ws + (((int64_t)row * gridDim.x + split) * group + g0) * kPartStride;
-  for (int e = tid; e < g_count * 128; e += kAttThreads) {
-    const int g = e >> 7, d = e & 127;
-    float mn = s_m[0][g];
-#pragma unroll
-    for (int w = 1; w < 16; ++w) mn = fmaxf(mn, s_m[w][g]);
-    float ls = 0.f, os = 0.f;
-#pragma unroll
-    for (int w = 0; w < 16; ++w) {
-      const float c = exp2f(s_m[w][g] - mn);
-      ls += s_l[w][g] * c;
-      os += s_o[w][g][d] * c;
-    }
-    part[g * kPartStride + 2 + d] = os;
-    if (d == 0) part[g * kPartStride] = mn, part[g * kPartStride + 1] = ls;
-  }
+  att_partial_vector<BF16, G, INDEXED>(q, n_kv_heads, group, segs, total, row_keys, uniform, per_split, scale_log2e, ws,
+                                       (int)gridDim.x, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
 }
-
-// ---- bf16 inputs: the same partial step on the matrix cores ----
-//
-// Each wave: 32 keys per step, v_mfma_f32_16x16x32_bf16 throughout.
-//   scores:  S^T[key][head] = K[key][dim] . Q^T[dim][head]: A = 16 keys x 32 dims (lane (r, j) holds dims
-//            32c + 8j .. +7 of key r: one 128-bit load), B = the query heads (zero columns past `group`),
-//            4 instructions per 16 keys.  Lane (n, j) receives the scores of head n for keys 4j .. 4j+3 of the
-//            tile - which is exactly where the next product wants the probabilities, so nothing is moved.
-//   output:  O[head][dim] += P[head][key] . V[key][dim] over the 32 keys of two tiles: lane (n, j) supplies its
-//            8 probabilities as A; for B it loads dims 8n .. 8n+7 of its 8 keys (rows read whole, 16 lanes per
-//            row) and regroups them with byte permutes so that instruction m covers the dims 8n + m.
-// The running maximum of head n lives in the lanes n, n+16, n+32, n+48; the output rows of head h live in lanes
-// with j == h / 4.  group <= 16, all heads of the KV head in one pass.
-typedef __bf16 pkv_bf16x8 __attribute__((ext_vector_type(8)));
-typedef float pkv_f32x4 __attribute__((ext_vector_type(4)));
-constexpr int kMfmaStepKeys = 32;
-
-__device__ __forceinline__ pkv_f32x4 mfma_bf16(pkv_u32x4 a, pkv_u32x4 b, pkv_f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(pkv_bf16x8, a), __builtin_bit_cast(pkv_bf16x8, b), c,
-                                                 0, 0, 0);
-}
-
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-  return (uint32_t)pkv_f32_to_bf16_bits(lo) | ((uint32_t)pkv_f32_to_bf16_bits(hi) << 16);
-}
-
-constexpr int kMfmaWaves = 4;  // waves per workgroup: each takes a quarter of the split, merged through LDS
 
 // grid (splits, KV heads, batch).  Decode step, us, with four-way pointer selection per row / with places by lane exchange:
 // 8 rows x 693 attended keys 30.2 / 27.7, 8 x 1188 (4 layers) 136.5 / 124.2, 64 x 887 (2 layers) 133.4 / 122.8.
@@ -370,148 +43,9 @@ template <bool INDEXED, typename SEGS>
 __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_kernel(
     const void *__restrict__ q, int group, SEGS segs, int64_t total, const int32_t *__restrict__ row_keys, int uniform,
     int64_t per_split, float scale_log2e, float *__restrict__ ws) {
-  constexpr bool ONE = __is_same(SEGS, AttOne);
-  const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int row = b * (int)gridDim.y + h;
-  const int lane = threadIdx.x & (PKV_WAVE - 1), wave = threadIdx.x / PKV_WAVE;
-  const int n = lane & 15, j = lane >> 4;
-  total = att_row_total(total, row_keys, row, uniform);
-  const int64_t per_wave = per_split / kMfmaWaves;  // a multiple of the 32 keys of one step
-  const int64_t j0 = (int64_t)split * per_split + (int64_t)wave * per_wave;
-  const int64_t j1 = (j0 + per_wave < total) ? j0 + per_wave : total;  // j1 <= j0: nothing left for this wave
-
-  // Lane l holds the place of key blk0 + l of the current block of 64 keys (two steps; keys past j1 repeat the last one);
-  // the lanes that read a row get it from there, so that a place is found once per key and wave.
-  AttPlace<ONE> mine;
-  const char *kbase = nullptr, *vbase = nullptr;
-  if constexpr (ONE) {
-    const int64_t slab = (int64_t)b * segs.stride_b + (int64_t)h * segs.stride_h;
-    kbase = segs.k + slab, vbase = segs.v + slab;
-  }
-  auto place_block = [&](int64_t jb) {
-    const int64_t key = jb + lane;
-    mine = att_place<INDEXED, 256>(segs, row, b, h, (uint32_t)(key < j1 ? key : j1 - 1));
-  };
-  if (j0 < j1) place_block(j0);  // before the queries: the indices' latency is the longer one
-
-  const pkv_u32x4 zero4 = {0u, 0u, 0u, 0u};
-  pkv_u32x4 qb[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c)
-    qb[c] = n < group ? *(const pkv_u32x4 *)((const uint16_t *)q + ((int64_t)row * group + n) * 128 + 32 * c + 8 * j) : zero4;
-
-  float m_run = kNegBig, l_part = 0.f;
-  pkv_f32x4 o[8];
-#pragma unroll
-  for (int m = 0; m < 8; ++m) o[m] = pkv_f32x4{0.f, 0.f, 0.f, 0.f};
-
-  for (int64_t jb = j0; jb < j1; jb += kMfmaStepKeys) {
-    const int in_block = (int)(jb - j0) & (PKV_WAVE - 1);
-    if (in_block == 0 && jb != j0) place_block(jb);
-    // K: two tiles of 16 keys, lane (n, j) reads dims 32c + 8j .. +7 of key jb + 16t + n.  Two instructions share a 128-byte line:
-    // plain loads, as a streaming load gives it up after the first (decode step, streaming / plain: 8 rows x 1188 attended
-    // keys (4 layers) 115.0 / 112.8 us, 24 x 1900 (2) 92.6 / 91.7; at 64 x 887 (2) 117.2 / 118.6).  V rows are read whole.
-    pkv_u32x4 ka[2][4], vr[8];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const char *kp;
-      if constexpr (ONE) kp = kbase + (uint64_t)(mine.from(in_block + 16 * t + n).off + 16u * (uint32_t)j);
-      else kp = mine.k_from(in_block + 16 * t + n) + 16 * j;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) ka[t][c] = *(const pkv_u32x4 *)(kp + 64 * c);
-    }
-    // V: dims 8n .. 8n+7 of the 8 keys whose probabilities this lane will hold
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int at = in_block + 16 * (e >> 2) + 4 * j + (e & 3);
-      const char *vp;
-      if constexpr (ONE) vp = vbase + (uint64_t)(mine.from(at).off + 16u * (uint32_t)n);
-      else vp = mine.v_from(at) + 16 * n;
-      vr[e] = __builtin_nontemporal_load((const pkv_u32x4 *)vp);
-    }
-
-    pkv_f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      s0 = mfma_bf16(ka[0][c], qb[c], s0);
-      s1 = mfma_bf16(ka[1][c], qb[c], s1);
-    }
-    float sc[8];
-    bool valid[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      valid[e] = jb + 16 * (e >> 2) + 4 * j + (e & 3) < j1;
-      const float raw = (e < 4) ? s0[e & 3] : s1[e & 3];
-      sc[e] = valid[e] ? raw * scale_log2e : kNegBig;
-    }
-    float mx = sc[0];
-#pragma unroll
-    for (int e = 1; e < 8; ++e) mx = fmaxf(mx, sc[e]);
-    mx = fmaxf(mx, __shfl_xor(mx, 16, PKV_WAVE));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, PKV_WAVE));
-    const float m_new = fmaxf(m_run, mx);
-    // the hardware's exp2: exp2f but for results below 2^-126, which are zero; nothing beside the largest weight, which is 1
-    const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
-    m_run = m_new;
-    float p[8], psum = 0.f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      p[e] = valid[e] ? __builtin_amdgcn_exp2f(sc[e] - m_new) : 0.f;
-      psum += p[e];
-    }
-    l_part = l_part * corr + psum;
-    const pkv_u32x4 pa = {pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
-                          pack_bf16x2(p[6], p[7])};
-    // the output rows of this lane belong to heads 4j .. 4j+3: fetch their correction factors
-    float cr[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) cr[i] = __shfl(corr, 4 * j + i, PKV_WAVE);
-#pragma unroll
-    for (int m = 0; m < 8; ++m) {
-      // element m of each of the eight V vectors: dword m/2, half m%2
-      const uint32_t sel = (m & 1) ? 0x07060302u : 0x05040100u;
-      pkv_u32x4 bm;
-      bm.x = __builtin_amdgcn_perm(vr[1][m >> 1], vr[0][m >> 1], sel);
-      bm.y = __builtin_amdgcn_perm(vr[3][m >> 1], vr[2][m >> 1], sel);
-      bm.z = __builtin_amdgcn_perm(vr[5][m >> 1], vr[4][m >> 1], sel);
-      bm.w = __builtin_amdgcn_perm(vr[7][m >> 1], vr[6][m >> 1], sel);
-      pkv_f32x4 acc = o[m];
-      acc.x *= cr[0], acc.y *= cr[1], acc.z *= cr[2], acc.w *= cr[3];
-      o[m] = mfma_bf16(pa, bm, acc);
-    }
-  }
-
-  l_part += __shfl_xor(l_part, 16, PKV_WAVE);
-  l_part += __shfl_xor(l_part, 32, PKV_WAVE);
-  // merge the waves of the workgroup: every wave leaves (max, sum, output) of its keys in LDS, then the
-  // workgroup's 256 threads combine them, one (head, dim) pair at a time.  group <= 8.
-  __shared__ float s_m[kMfmaWaves][8], s_l[kMfmaWaves][8], s_o[kMfmaWaves][8][128 + 4];
-  if (j == 0 && n < group) s_m[wave][n] = m_run, s_l[wave][n] = l_part;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int head = 4 * j + i;
-    if (head < group) {
-      *(float4 *)&s_o[wave][head][8 * n] = float4{o[0][i], o[1][i], o[2][i], o[3][i]};
-      *(float4 *)&s_o[wave][head][8 * n + 4] = float4{o[4][i], o[5][i], o[6][i], o[7][i]};
-    }
-  }
-  __syncthreads();
-  float *part = ws + ((int64_t)row * gridDim.x + split) * group * kPartStride;
-  for (int e = threadIdx.x; e < group * 128; e += kMfmaWaves * PKV_WAVE) {
-    const int g = e >> 7, d = e & 127;
-    float mn = s_m[0][g];
-#pragma unroll
-    for (int w = 1; w < kMfmaWaves; ++w) mn = fmaxf(mn, s_m[w][g]);
-    float ls = 0.f, os = 0.f;
-#pragma unroll
-    for (int w = 0; w < kMfmaWaves; ++w) {
-      const float c = exp2f(s_m[w][g] - mn);
-      ls += s_l[w][g] * c;
-      os += s_o[w][g][d] * c;
-    }
-    part[g * kPartStride + 2 + d] = os;
-    if (d == 0) part[g * kPartStride] = mn, part[g * kPartStride + 1] = ls;
-  }
+  const int h = blockIdx.y, b = blockIdx.z;
+  att_partial_mfma<INDEXED>(q, group, segs, total, row_keys, uniform, per_split, scale_log2e, ws, (int)gridDim.x,
+                            (int)blockIdx.x, b * (int)gridDim.y + h, b, h);
 }
 
 // grid R, G*128 threads: merge the splits (at most 64) and normalise.
@@ -606,27 +140,28 @@ bool as_one_tensor(const AttSegs &sg, int es, AttOne &one) {
 
 }  // namespace
 
+PKV_INTERNAL bool pkv_topk_selects(int64_t len, int64_t k);
+
+// One CU fetches scattered rows at 35 to 40 GB/s, 2.7 us for 200 of them and as much as the merge's launch: up to eight blocks of 32
+// are one workgroup's, which then merges; more go to a workgroup per split of 128, each selecting anew, or per two or three where
+// that would be more workgroups than CUs.  Decode step, us, attention after the top-k / in two parts: 8 rows x 4096 keys, top 100,
+// 28.2 / 23.9, top 256 28.6 / 26.0; 8 x 32768, top 512, 30.0 / 27.1; 32 x 16000, 8 heads, top 100 34.5 / 31.0, top 512 36.9 / 33.4;
+// 64 x 40000, top 256 48.9 / 44.7, top 512 52.4 / 46.9; 64 x 65536, top 100, 56.3 / 52.2; 256 x 8000, top 100, 73.1 / 59.8.
+constexpr int kSplitWorkgroups = 256;
+constexpr int64_t kSplitMaxSelected = 1024;
+
 extern "C" size_t pkv_decode_attention_ws_bytes(int bs, int n_kv_heads, int group, int64_t total_keys) {
   if (bs <= 0 || n_kv_heads <= 0 || group <= 0 || total_keys <= 0) return 256;
   // room for the largest split count either path uses (64), whatever the key count and dtype
   return pkv_align_up((size_t)bs * n_kv_heads * 64 * group * kPartStride * sizeof(float), 256);
 }
 
-static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_segment *segments,
-                            int n_segments, const int32_t *row_keys, int uniform, float scale, void *out, void *ws,
-                            size_t ws_bytes, void *stream) {
-  PKV_REQUIRE(q && segments && out && ws, "pkv_decode_attention: null pointer");
-  PKV_REQUIRE(dtype == PKV_DTYPE_F32 || dtype == PKV_DTYPE_BF16, "unknown dtype %d", dtype);
-  PKV_REQUIRE(bs > 0 && n_kv_heads > 0 && (int64_t)bs * n_kv_heads <= 65535, "bad shape bs=%d kv_heads=%d", bs,
-              n_kv_heads);
-  PKV_REQUIRE(group >= 1 && group <= 8, "GQA group must be in [1, 8] (got %d)", group);
-  PKV_REQUIRE(n_segments >= 1 && n_segments <= PKV_ATTN_MAX_SEGMENTS, "1..%d key segments", PKV_ATTN_MAX_SEGMENTS);
-  PKV_REQUIRE(pkv_aligned(q, 16) && pkv_aligned(out, 4), "q must be 16-byte aligned");
+// The segments that have rows, checked, one behind the other.
+static int collect_segments(int dtype, const pkv_attn_segment *segments, int n_segments, AttSegs &sg, int64_t &total, bool &indexed) {
   const int64_t vec = dtype == PKV_DTYPE_BF16 ? 8 : 4;
-  AttSegs sg;
   memset(&sg, 0, sizeof sg);
-  int64_t total = 0;
-  bool indexed = false;
+  total = 0;
+  indexed = false;
   for (int i = 0; i < n_segments; ++i) {
     const pkv_attn_segment &s = segments[i];
     PKV_REQUIRE(s.n_rows >= 0 && s.row0 >= 0, "segment %d: negative extent", i);
@@ -648,6 +183,24 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
     sg.end[sg.n] = total;
     ++sg.n;
   }
+  return PKV_OK;
+}
+
+static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_segment *segments,
+                            int n_segments, const int32_t *row_keys, int uniform, float scale, void *out, void *ws,
+                            size_t ws_bytes, void *stream) {
+  PKV_REQUIRE(q && segments && out && ws, "pkv_decode_attention: null pointer");
+  PKV_REQUIRE(dtype == PKV_DTYPE_F32 || dtype == PKV_DTYPE_BF16, "unknown dtype %d", dtype);
+  PKV_REQUIRE(bs > 0 && n_kv_heads > 0 && (int64_t)bs * n_kv_heads <= 65535, "bad shape bs=%d kv_heads=%d", bs,
+              n_kv_heads);
+  PKV_REQUIRE(group >= 1 && group <= 8, "GQA group must be in [1, 8] (got %d)", group);
+  PKV_REQUIRE(n_segments >= 1 && n_segments <= PKV_ATTN_MAX_SEGMENTS, "1..%d key segments", PKV_ATTN_MAX_SEGMENTS);
+  PKV_REQUIRE(pkv_aligned(q, 16) && pkv_aligned(out, 4), "q must be 16-byte aligned");
+  AttSegs sg;
+  int64_t total;
+  bool indexed;
+  const int rc = collect_segments(dtype, segments, n_segments, sg, total, indexed);
+  if (rc) return rc;
   PKV_REQUIRE(total > 0, "pkv_decode_attention: no keys");
   PKV_REQUIRE(total < ((int64_t)1 << 23), "pkv_decode_attention: at most 2^23 - 1 keys (got %lld)", (long long)total);
   const int rows = bs * n_kv_heads;
@@ -722,4 +275,75 @@ extern "C" int pkv_decode_attention_run(const void *q, int dtype, int bs, int n_
   PKV_REQUIRE(a != nullptr, "pkv_decode_attention: null args");
   return decode_attention(q, dtype, bs, n_kv_heads, group, a->segments, a->n_segments, a->row_keys,
                           a->row_keys_uniform ? bs * n_kv_heads : 0, a->scale, a->out, a->ws, a->ws_bytes, stream);
+}
+
+bool pkv_plan_split_attention(const pkv_retrieve_args *r, const pkv_attn_args *at, PkvSplitAttn *out) {
+  // What the general path would refuse is left to it.
+  if (r->dtype != PKV_DTYPE_BF16 || !r->q || !pkv_aligned(r->q, 16) || !at->out || !pkv_aligned(at->out, 4) || !at->ws ||
+      !pkv_aligned(at->ws, 16) || r->bs <= 0 || r->n_kv_heads <= 0 || (int64_t)r->bs * r->n_kv_heads > 65535 || r->group < 1 ||
+      r->group > 8 || at->n_segments < 1 || at->n_segments > PKV_ATTN_MAX_SEGMENTS)
+    return false;
+  // The query side: a launch of this call's own, for the dense part to run beside.
+  if (r->launch_plan != PKV_PLAN_SEPARATE || r->table_ready) return false;
+  // The selection: in any order, of one workgroup a row, into the list that the attention reads, nothing gathered.
+  if (!r->out_ids || !r->any_order || r->src_k || r->n_cand == r->n_keys || at->row_keys || r->k > kSplitMaxSelected ||
+      !pkv_topk_selects(r->n_cand, r->k))
+    return false;
+  for (int i = 0; i < at->n_segments; ++i) {
+    const pkv_attn_segment &s = at->segments[i];
+    if (s.n_rows < 0 || s.row0 < 0) return false;
+    if (s.n_rows == 0) continue;
+    if (!s.k || !s.v || !pkv_aligned(s.k, 16) || !pkv_aligned(s.v, 16) || s.stride_b % 8 || s.stride_h % 8) return false;
+    if (s.idx && (s.idx != r->out_ids || s.idx_stride != r->k || s.n_rows != r->k || s.idx_limit <= 0 ||
+                  s.row0 + s.idx_limit >= ((int64_t)1 << 29)))
+      return false;
+  }
+  AttSegs sg;
+  int64_t total;
+  bool indexed;
+  if (collect_segments(r->dtype, at->segments, at->n_segments, sg, total, indexed) || !indexed || total >= ((int64_t)1 << 23)) return false;
+  memset(out, 0, sizeof *out);
+  if (!as_one_tensor(sg, 2, out->segs)) return false;  // also: one indexed segment at most
+  const int rows = r->bs * r->n_kv_heads;
+  out->n_splits = pick_splits_mfma(rows, total);
+  constexpr int kSplitKeys = kMfmaWaves * kMfmaStepKeys;
+  if (total > (int64_t)out->n_splits * kSplitKeys) return false;  // a wave would take several blocks
+  out->total = (uint32_t)total;
+  out->blk_lo = (int)(out->segs.idx_lo / kMfmaStepKeys), out->blk_hi = (int)((out->segs.idx_hi - 1) / kMfmaStepKeys);
+  const int lo = out->blk_lo / kMfmaWaves, hi = out->blk_hi / kMfmaWaves, n_sel = hi - lo + 1;  // splits with selected keys
+  if (out->blk_hi - out->blk_lo < kSelBlocks && out->n_splits < kSelSplits) {
+    out->sel_wgs = 1;
+    // the splits between the first and the last one's own blocks have nothing else to do
+    const int last_block = (int)((total - 1) / kMfmaStepKeys);
+    out->dense_a = (out->blk_lo + kMfmaWaves - 1) / kMfmaWaves;
+    const int from = out->blk_hi == last_block ? out->n_splits : (out->blk_hi + 1) / kMfmaWaves;
+    out->dense_skip = from > out->dense_a ? from - out->dense_a : 0;
+    for (int i = 0; i <= last_block; ++i) {
+      const bool mixed = i / kMfmaWaves >= lo && i / kMfmaWaves <= hi;
+      if (i < out->blk_lo || i > out->blk_hi) out->slots |= 1u << (mixed ? att_block_slot(*out, i) : i / kMfmaWaves);
+    }
+    if ((int64_t)rows * 20 * r->group * 128 >= ((int64_t)1 << 31)) return false;
+    out->ws_ml = (float *)at->ws + (int64_t)rows * 20 * r->group * 128;
+  } else {
+    do {
+      out->sel_wgs = (n_sel + ++out->splits_per_wg - 1) / out->splits_per_wg;
+    } while (out->splits_per_wg < kSelSplits / 4 && (int64_t)rows * out->sel_wgs > kSplitWorkgroups);
+    if (out->sel_wgs == 1) return false;  // few selected keys among very many others
+    out->dense_a = lo, out->dense_skip = n_sel;
+  }
+  out->n_dense = out->n_splits - out->dense_skip;
+  const size_t row_floats = out->sel_wgs == 1 ? (size_t)20 * r->group * 128 + (size_t)r->group * kSelSlots * 2
+                                              : (size_t)out->n_splits * r->group * kPartStride;
+  if (at->ws_bytes < (size_t)rows * row_floats * sizeof(float)) return false;
+  out->n_kv_heads = r->n_kv_heads, out->group = r->group, out->q = r->q;
+  out->scale_log2e = at->scale * 1.4426950408889634f;
+  out->ws = (float *)at->ws, out->out = at->out;
+  return true;
+}
+
+int pkv_launch_attn_merge(const PkvSplitAttn &a, int rows, hipStream_t s) {
+  hipLaunchKernelGGL(pkv_attn_merge_kernel<true>, dim3((unsigned)rows), dim3(a.group * 128), 0, s, (const float *)a.ws, a.n_splits, a.group,
+                     a.out);
+  PKV_LAUNCH_CHECK("pkv_attn_merge_kernel");
+  return PKV_OK;
 }

@@ -1,0 +1,768 @@
+// Device side of the decode attention: key segments, places of keys, one workgroup's partial result over a run of keys (fp32
+// vector units, bf16 matrix cores).  Shared by the attention's own kernels, by the launch that runs the partial results of the
+// keys every step attends to beside the retrieval's query side, and by the top-k that goes on to attend to what it selected.
+#pragma once
+
+#include "pkv_common.h"
+
+#if defined(__HIPCC__)
+
+// Fused multiply-add is welcome in every function here (the rest of the library forbids it because integer results are
+// derived from its float steps; the attention's only contract is its tolerance).
+#define PKV_ATT_CONTRACT _Pragma("clang fp contract(fast)")
+
+
+constexpr int kAttThreads = 256;
+constexpr int kAttKeysPerIter = kAttThreads / 16;  // 16 keys per workgroup step
+constexpr int kAttUnroll = 2;                      // keys per 16-lane group per step
+constexpr float kNegBig = -1.0e30f;
+
+struct AttSegs {
+  const void *k[PKV_ATTN_MAX_SEGMENTS];
+  const void *v[PKV_ATTN_MAX_SEGMENTS];
+  int64_t stride_b[PKV_ATTN_MAX_SEGMENTS], stride_h[PKV_ATTN_MAX_SEGMENTS];
+  int64_t row0[PKV_ATTN_MAX_SEGMENTS];
+  int64_t end[PKV_ATTN_MAX_SEGMENTS];  // exclusive end of the segment in the concatenated key order
+  const int64_t *idx[PKV_ATTN_MAX_SEGMENTS];  // per segment: selected rows (relative to row0) or nullptr
+  int64_t idx_stride[PKV_ATTN_MAX_SEGMENTS], idx_limit[PKV_ATTN_MAX_SEGMENTS];
+  int n;
+};
+
+// Row (inside the (b, h) slab of its segment, row0 included) and segment of concatenated key jj, packed as
+// row | segment << 29.  Indexed segments cost one dependent 8-byte load.
+__device__ __forceinline__ uint32_t att_resolve_row(const AttSegs &segs, int row, uint32_t jj) {
+  int s = 0;
+  uint32_t first = 0;
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (t < segs.n && jj >= (uint32_t)segs.end[t - 1]) s = t, first = (uint32_t)segs.end[t - 1];
+  const int64_t *ip = segs.idx[0];
+  int64_t stride = segs.idx_stride[0], limit = segs.idx_limit[0], row0 = segs.row0[0];
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (s == t) ip = segs.idx[t], stride = segs.idx_stride[t], limit = segs.idx_limit[t], row0 = segs.row0[t];
+  int64_t r = jj - first;
+  if (ip) {
+    r = ip[(int64_t)row * stride + r];
+    r = r < 0 ? 0 : (r >= limit ? limit - 1 : r);
+  }
+  return (uint32_t)(r + row0) | ((uint32_t)s << 29);
+}
+
+// Eight consecutive elements as loaded (16 B of bf16, or 32 B of fp32) and their fp32 values.  Kept
+// apart so that a load can be issued a whole step before its data is touched.
+template <bool BF16>
+struct Raw8 {
+  pkv_u32x4 a;
+  pkv_u32x4 b[BF16 ? 0 : 1];
+};
+
+// Plain loads: two instructions share every 128-byte line of an fp32 row, and a streaming load gives the line up after the first.
+// Decode step, streaming / plain: 12 rows x 865 attended keys, 7 heads (2 layers) 68.6 / 64.8 us.
+template <bool BF16>
+__device__ __forceinline__ void load_raw8(const void *base, int64_t elem_off, Raw8<BF16> &r) {
+  if (BF16) {
+    r.a = *(const pkv_u32x4 *)((const uint16_t *)base + elem_off);
+  } else {
+    r.a = *(const pkv_u32x4 *)((const float *)base + elem_off);
+    r.b[BF16 ? -1 : 0] = *(const pkv_u32x4 *)((const float *)base + elem_off + 4);
+  }
+}
+
+template <bool BF16>
+__device__ __forceinline__ void expand8(const Raw8<BF16> &r, float (&x)[8]) {
+  const uint32_t ww[4] = {r.a.x, r.a.y, r.a.z, r.a.w};
+  if (BF16) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      x[2 * p] = __uint_as_float(ww[p] << 16);
+      x[2 * p + 1] = __uint_as_float(ww[p] & 0xffff0000u);
+    }
+  } else {
+    const pkv_u32x4 hi = r.b[BF16 ? -1 : 0];
+    x[0] = __uint_as_float(ww[0]), x[1] = __uint_as_float(ww[1]), x[2] = __uint_as_float(ww[2]);
+    x[3] = __uint_as_float(ww[3]), x[4] = __uint_as_float(hi.x), x[5] = __uint_as_float(hi.y);
+    x[6] = __uint_as_float(hi.z), x[7] = __uint_as_float(hi.w);
+  }
+}
+
+template <bool BF16>
+__device__ __forceinline__ void load8(const void *base, int64_t elem_off, float (&x)[8]) {
+  Raw8<BF16> r;
+  load_raw8<BF16>(base, elem_off, r);
+  expand8<BF16>(r, x);
+}
+
+// Keys row `row` attends to: all `total`, its own row_keys[row], or with uniform > 0 the largest of row_keys[0 .. uniform)
+// (the dense form of the adaptive-k step, where a launch of its own for the maximum took 4.5 us at 24 rows).
+__device__ __forceinline__ int64_t att_row_total(int64_t total, const int32_t *__restrict__ row_keys, int row, int uniform) {
+  if (!row_keys) return total;
+  int64_t rk;
+  if (uniform > 0) {
+    int m = 0;
+    for (int r = pkv_lane(); r < uniform; r += PKV_WAVE) m = max(m, row_keys[r]);
+#define PKV_ATT_MAX(M) { const int o = (int)pkv_lane_xor<M>((uint32_t)m); m = max(m, o); }
+    PKV_ATT_MAX(1) PKV_ATT_MAX(2) PKV_ATT_MAX(4) PKV_ATT_MAX(8) PKV_ATT_MAX(16) PKV_ATT_MAX(32)
+#undef PKV_ATT_MAX
+    rk = __builtin_amdgcn_readfirstlane(m);
+  } else {
+    rk = row_keys[row];
+  }
+  return rk < total ? (rk > 0 ? rk : 1) : total;
+}
+
+// Segments that share one K and one V tensor (the cache's rows in HBM: sink, selected rows, local window), at most one of
+// them indexed: a key is a 32-bit byte offset into the (b, h) slab.  Half of a launch over a few hundred keys used to go
+// into finding addresses (1.2 us to pick a 64-bit pointer out of four for each of a lane's ten rows, after 1 us for a
+// 300-byte argument block); here that is one lane exchange per row.
+struct AttOne {
+  const char *k, *v;
+  int64_t stride_b, stride_h;           // bytes
+  uint32_t end[PKV_ATTN_MAX_SEGMENTS];  // exclusive ends in the concatenated key order; unused: 2^32 - 1
+  int32_t delta[PKV_ATTN_MAX_SEGMENTS]; // row - concatenated key
+  const int64_t *idx;                   // of the indexed segment, keys [idx_lo, idx_hi)
+  int64_t idx_stride, idx_limit;
+  uint32_t idx_lo, idx_hi, idx_row0;
+};
+
+// One key's place: a byte offset into the slab (AttOne), or the addresses of its K and V rows.
+template <bool ONE>
+struct AttPlace {
+  uint32_t off;
+  __device__ __forceinline__ AttPlace from(int lane) const { return {(uint32_t)__shfl((int)off, lane, PKV_WAVE)}; }
+};
+template <>
+struct AttPlace<false> {
+  uint64_t k, v;
+  __device__ __forceinline__ const char *k_from(int lane) const { return (const char *)pull(k, lane); }
+  __device__ __forceinline__ const char *v_from(int lane) const { return (const char *)pull(v, lane); }
+  static __device__ __forceinline__ uint64_t pull(uint64_t x, int lane) {
+    return ((uint64_t)(uint32_t)__shfl((int)(x >> 32), lane, PKV_WAVE) << 32) | (uint32_t)__shfl((int)(uint32_t)x, lane, PKV_WAVE);
+  }
+};
+
+// ROW: bytes of a row.
+template <bool INDEXED, uint32_t ROW>
+__device__ __forceinline__ AttPlace<true> att_place(const AttOne &a, int row, int, int, uint32_t jj) {
+  int32_t d = a.delta[0];
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t) d = jj >= a.end[t - 1] ? a.delta[t] : d;
+  uint32_t r = jj + (uint32_t)d;
+  if (INDEXED && jj >= a.idx_lo && jj < a.idx_hi) {
+    const int64_t x = a.idx[(int64_t)row * a.idx_stride + (jj - a.idx_lo)];
+    r = a.idx_row0 + (uint32_t)(x < 0 ? 0 : (x >= a.idx_limit ? a.idx_limit - 1 : x));
+  }
+  return {r * ROW};
+}
+
+template <bool INDEXED, uint32_t ROW>
+__device__ __forceinline__ AttPlace<false> att_place(const AttSegs &a, int row, int b, int h, uint32_t jj) {
+  int s = 0;
+  uint32_t first = 0;
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (t < a.n && jj >= (uint32_t)a.end[t - 1]) s = t, first = (uint32_t)a.end[t - 1];
+  const char *k = (const char *)a.k[0], *v = (const char *)a.v[0];
+  int64_t sb = a.stride_b[0], sh = a.stride_h[0], row0 = a.row0[0];
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (s == t) k = (const char *)a.k[t], v = (const char *)a.v[t], sb = a.stride_b[t], sh = a.stride_h[t], row0 = a.row0[t];
+  const int64_t r = INDEXED ? (int64_t)(att_resolve_row(a, row, jj) & 0x1fffffffu) : row0 + (int64_t)(jj - first);
+  const int64_t off = ((int64_t)b * sb + (int64_t)h * sh) * (ROW / 128) + r * ROW;
+  return {(uint64_t)(k + off), (uint64_t)(v + off)};
+}
+
+// Partial results layout: ws[((row * n_splits + split) * G + g) * 130 + {0: max, 1: sum, 2..129: output}].
+constexpr int kPartStride = 130;
+// Splits are of 64 keys while the key set allows: a launch is one chain of dependent loads with some 1000 instructions behind
+// it, not bandwidth.  Places of keys as in the bf16 kernel below.  Decode step, us, with a 64-bit pointer picked out of four for
+// each row / with places: 12 rows x 865 attended keys, 7 heads (2 layers) 74.6 / 70.0, 8 rows x 696 (2 layers) 66.5 / 61.0,
+// 32 rows x 896 48.6 / 45.2.
+template <bool BF16, int G, bool INDEXED, typename SEGS>
+__device__ __forceinline__ void att_partial_vector(const void *__restrict__ q, int n_kv_heads, int group, const SEGS &segs,
+                                                   int64_t total, const int32_t *__restrict__ row_keys, int uniform,
+                                                   int64_t per_split, float scale_log2e, float *__restrict__ ws, int n_splits,
+                                                   int split, int row, int head_wg) {
+  PKV_ATT_CONTRACT
+  // head_wg: query heads g0 .. g0 + g_count - 1 of the KV head (more than four would not fit the registers)
+  const int g0 = head_wg * G, g_count = group - g0 < G ? group - g0 : G;
+  const int b = row / n_kv_heads, h = row % n_kv_heads;
+  const int tid = threadIdx.x;
+  const int lane16 = tid & 15;        // owns dims 8*lane16 .. +7
+  const int grp = tid >> 4;           // 16 key slots per workgroup step
+
+  total = att_row_total(total, row_keys, row, uniform);  // ragged rows
+  const int64_t j0 = (int64_t)split * per_split;
+  const int64_t j1 = (j0 + per_split < total) ? j0 + per_split : total;
+  constexpr bool ONE = __is_same(SEGS, AttOne);
+  constexpr uint32_t kRow = BF16 ? 256 : 512;
+  const int lane = tid & (PKV_WAVE - 1), wave = tid / PKV_WAVE;
+  const char *kbase = nullptr, *vbase = nullptr;
+  if constexpr (ONE) {
+    const int64_t slab = (int64_t)b * segs.stride_b + (int64_t)h * segs.stride_h;
+    kbase = segs.k + slab, vbase = segs.v + slab;
+  }
+  // K/V rows of the step after the current one are requested before the current one is consumed
+  float kx[kAttUnroll][8], vx[kAttUnroll][8];
+  Raw8<BF16> kn[kAttUnroll], vn[kAttUnroll];
+  AttPlace<ONE> mine;
+  auto fetch = [&](int64_t jb, Raw8<BF16> (&kd)[kAttUnroll], Raw8<BF16> (&vd)[kAttUnroll]) {
+    // four turns (64 keys) at a time: lane 4 t + i (mod 16) finds the place of the key that the wave's lanes 16 i .. 16 i + 15
+    // read in turn t
+    static_assert(4 % kAttUnroll == 0 && kAttKeysPerIter == 16, "a wave reads four keys in a turn");
+    const int turn = ((int)(jb - j0) / kAttKeysPerIter) & 3;
+    if (turn == 0) {
+      const int64_t key = jb + ((lane >> 2) & 3) * kAttKeysPerIter + 4 * wave + (lane & 3);
+      mine = att_place<INDEXED, kRow>(segs, row, b, h, (uint32_t)(key < j1 ? key : j1 - 1));  // fewer than 2^24 keys
+    }
+#pragma unroll
+    for (int u = 0; u < kAttUnroll; ++u) {
+      const int at = 4 * (turn + u) + (lane >> 4);
+      const char *kp, *vp;
+      if constexpr (ONE) {
+        const uint64_t off = mine.from(at).off + (kRow / 16) * (uint32_t)lane16;
+        kp = kbase + off, vp = vbase + off;
+      } else {
+        kp = mine.k_from(at) + (kRow / 16) * lane16, vp = mine.v_from(at) + (kRow / 16) * lane16;
+      }
+      load_raw8<BF16>(kp, 0, kd[u]);
+      load_raw8<BF16>(vp, 0, vd[u]);
+    }
+  };
+  if (j0 < j1) fetch(j0, kn, vn);  // before the queries: nothing here waits for them
+
+  float qv[G][8];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {  // surplus slots idle
+    load8<BF16>(q, ((int64_t)row * group + g0 + (g < g_count ? g : 0)) * 128 + 8 * lane16, qv[g]);
+#pragma unroll
+    for (int d = 0; d < 8; ++d) qv[g][d] *= scale_log2e;  // scores come out in units of log2(e)
+  }
+  float m[G], l[G], o[G][8];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    m[g] = kNegBig, l[g] = 0.f;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) o[g][d] = 0.f;
+  }
+
+  for (int64_t jb = j0; jb < j1; jb += kAttKeysPerIter * kAttUnroll) {
+    bool valid[kAttUnroll];
+#pragma unroll
+    for (int u = 0; u < kAttUnroll; ++u) {
+      valid[u] = jb + u * kAttKeysPerIter + grp < j1;
+      expand8<BF16>(kn[u], kx[u]);
+      expand8<BF16>(vn[u], vx[u]);
+    }
+    if (jb + kAttKeysPerIter * kAttUnroll < j1) fetch(jb + kAttKeysPerIter * kAttUnroll, kn, vn);
+    float s[G][kAttUnroll];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+#pragma unroll
+      for (int u = 0; u < kAttUnroll; ++u) {
+        float acc = qv[g][0] * kx[u][0];
+#pragma unroll
+        for (int d = 1; d < 8; ++d) acc += qv[g][d] * kx[u][d];
+        acc += pkv_lane_xor_f<1>(acc);
+        acc += pkv_lane_xor_f<2>(acc);
+        acc += pkv_lane_xor_f<4>(acc);
+        acc += pkv_lane_xor_f<8>(acc);
+        s[g][u] = valid[u] ? acc : kNegBig;
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float mn = m[g];
+#pragma unroll
+      for (int u = 0; u < kAttUnroll; ++u) mn = fmaxf(mn, s[g][u]);
+      const float corr = exp2f(m[g] - mn);
+      m[g] = mn;
+      float p[kAttUnroll], psum = 0.f;
+#pragma unroll
+      for (int u = 0; u < kAttUnroll; ++u) {
+        p[u] = valid[u] ? exp2f(s[g][u] - mn) : 0.f;
+        psum += p[u];
+      }
+      l[g] = l[g] * corr + psum;
+#pragma unroll
+      for (int d = 0; d < 8; ++d) {
+        float acc = o[g][d] * corr;
+#pragma unroll
+        for (int u = 0; u < kAttUnroll; ++u) acc += p[u] * vx[u][d];
+        o[g][d] = acc;
+      }
+    }
+  }
+
+  // merge the 16 key slots of the workgroup through LDS
+  __shared__ float s_m[16][G], s_l[16][G], s_o[16][G][128 + 4];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    if (lane16 == 0) s_m[grp][g] = m[g], s_l[grp][g] = l[g];
+    *(float4 *)&s_o[grp][g][8 * lane16] = float4{o[g][0], o[g][1], o[g][2], o[g][3]};
+    *(float4 *)&s_o[grp][g][8 * lane16 + 4] = float4{o[g][4], o[g][5], o[g][6], o[g][7]};
+  }
+  __syncthreads();
+  float *part = ws + (((int64_t)row * n_splits + split) * group + g0) * kPartStride;
+  for (int e = tid; e < g_count * 128; e += kAttThreads) {
+    const int g = e >> 7, d = e & 127;
+    float mn = s_m[0][g];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) mn = fmaxf(mn, s_m[w][g]);
+    float ls = 0.f, os = 0.f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      const float c = exp2f(s_m[w][g] - mn);
+      ls += s_l[w][g] * c;
+      os += s_o[w][g][d] * c;
+    }
+    part[g * kPartStride + 2 + d] = os;
+    if (d == 0) part[g * kPartStride] = mn, part[g * kPartStride + 1] = ls;
+  }
+}
+
+// ---- bf16 inputs: the same partial step on the matrix cores ----
+//
+// Each wave: 32 keys per step, v_mfma_f32_16x16x32_bf16 throughout.
+//   scores:  S^T[key][head] = K[key][dim] . Q^T[dim][head]: A = 16 keys x 32 dims (lane (r, j) holds dims
+//            32c + 8j .. +7 of key r: one 128-bit load), B = the query heads (zero columns past `group`),
+//            4 instructions per 16 keys.  Lane (n, j) receives the scores of head n for keys 4j .. 4j+3 of the
+//            tile - which is exactly where the next product wants the probabilities, so nothing is moved.
+//   output:  O[head][dim] += P[head][key] . V[key][dim] over the 32 keys of two tiles: lane (n, j) supplies its
+//            8 probabilities as A; for B it loads dims 8n .. 8n+7 of its 8 keys (rows read whole, 16 lanes per
+//            row) and regroups them with byte permutes so that instruction m covers the dims 8n + m.
+// The running maximum of head n lives in the lanes n, n+16, n+32, n+48; the output rows of head h live in lanes
+// with j == h / 4.  group <= 16, all heads of the KV head in one pass.
+typedef __bf16 pkv_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float pkv_f32x4 __attribute__((ext_vector_type(4)));
+constexpr int kMfmaStepKeys = 32;
+
+__device__ __forceinline__ pkv_f32x4 mfma_bf16(pkv_u32x4 a, pkv_u32x4 b, pkv_f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(pkv_bf16x8, a), __builtin_bit_cast(pkv_bf16x8, b), c,
+                                                 0, 0, 0);
+}
+
+// A score is rounded before the maximum is taken from it, whatever the compiler could fuse around a call.
+__device__ __forceinline__ float att_scaled(float score, float scale) {
+#pragma clang fp contract(off)
+  return score * scale;
+}
+
+__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
+  return (uint32_t)pkv_f32_to_bf16_bits(lo) | ((uint32_t)pkv_f32_to_bf16_bits(hi) << 16);
+}
+
+constexpr int kMfmaWaves = 4;  // waves per workgroup: each takes a quarter of the split, merged through LDS
+
+// Keys jb .. jb + 31 (of them those below j1) into the running maximum, the lane's share of the sum and the output of a wave.
+// Lane in_block + i of `mine` holds the place of key jb + i.  FIRST: nothing has run yet.
+template <bool ONE, bool FIRST>
+__device__ __forceinline__ void att_step_mfma(const char *kbase, const char *vbase, const AttPlace<ONE> &mine, int in_block, int64_t jb,
+                                              int64_t j1, const pkv_u32x4 (&qb)[4], float scale_log2e, float &m_run, float &l_part,
+                                              pkv_f32x4 (&o)[8]) {
+  PKV_ATT_CONTRACT
+  const int lane = threadIdx.x & (PKV_WAVE - 1), n = lane & 15, j = lane >> 4;
+  // K: two tiles of 16 keys, lane (n, j) reads dims 32c + 8j .. +7 of key jb + 16t + n.  Two instructions share a 128-byte line:
+  // plain loads, as a streaming load gives it up after the first (decode step, streaming / plain: 8 rows x 1188 attended
+  // keys (4 layers) 115.0 / 112.8 us, 24 x 1900 (2) 92.6 / 91.7; at 64 x 887 (2) 117.2 / 118.6).  V rows are read whole.
+  pkv_u32x4 ka[2][4], vr[8];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const char *kp;
+    if constexpr (ONE) kp = kbase + (uint64_t)(mine.from(in_block + 16 * t + n).off + 16u * (uint32_t)j);
+    else kp = mine.k_from(in_block + 16 * t + n) + 16 * j;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) ka[t][c] = *(const pkv_u32x4 *)(kp + 64 * c);
+  }
+  // V: dims 8n .. 8n+7 of the 8 keys whose probabilities this lane will hold
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const int at = in_block + 16 * (e >> 2) + 4 * j + (e & 3);
+    const char *vp;
+    if constexpr (ONE) vp = vbase + (uint64_t)(mine.from(at).off + 16u * (uint32_t)n);
+    else vp = mine.v_from(at) + 16 * n;
+    vr[e] = __builtin_nontemporal_load((const pkv_u32x4 *)vp);
+  }
+
+  pkv_f32x4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    s0 = mfma_bf16(ka[0][c], qb[c], s0);
+    s1 = mfma_bf16(ka[1][c], qb[c], s1);
+  }
+  float sc[8];
+  bool valid[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    valid[e] = jb + 16 * (e >> 2) + 4 * j + (e & 3) < j1;
+    const float raw = (e < 4) ? s0[e & 3] : s1[e & 3];
+    sc[e] = valid[e] ? att_scaled(raw, scale_log2e) : kNegBig;
+  }
+  float mx = sc[0];
+#pragma unroll
+  for (int e = 1; e < 8; ++e) mx = fmaxf(mx, sc[e]);
+  mx = fmaxf(mx, __shfl_xor(mx, 16, PKV_WAVE));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, PKV_WAVE));
+  const float m_new = fmaxf(m_run, mx);
+  // the hardware's exp2: exp2f but for results below 2^-126, which are zero; nothing beside the largest weight, which is 1
+  const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
+  m_run = m_new;
+  float p[8], psum = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    p[e] = valid[e] ? __builtin_amdgcn_exp2f(sc[e] - m_new) : 0.f;
+    psum += p[e];
+  }
+  l_part = l_part * corr + psum;
+  const pkv_u32x4 pa = {pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
+                        pack_bf16x2(p[6], p[7])};
+  // the output rows of this lane belong to heads 4j .. 4j+3: fetch their correction factors
+  float cr[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) cr[i] = __shfl(corr, 4 * j + i, PKV_WAVE);
+#pragma unroll
+  for (int m = 0; m < 8; ++m) {
+    // element m of each of the eight V vectors: dword m/2, half m%2
+    const uint32_t sel = (m & 1) ? 0x07060302u : 0x05040100u;
+    pkv_u32x4 bm;
+    bm.x = __builtin_amdgcn_perm(vr[1][m >> 1], vr[0][m >> 1], sel);
+    bm.y = __builtin_amdgcn_perm(vr[3][m >> 1], vr[2][m >> 1], sel);
+    bm.z = __builtin_amdgcn_perm(vr[5][m >> 1], vr[4][m >> 1], sel);
+    bm.w = __builtin_amdgcn_perm(vr[7][m >> 1], vr[6][m >> 1], sel);
+    pkv_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    if (!FIRST) acc = o[m], acc.x *= cr[0], acc.y *= cr[1], acc.z *= cr[2], acc.w *= cr[3];
+    o[m] = mfma_bf16(pa, bm, acc);
+  }
+}
+
+// Merge of the waves of a workgroup: every wave leaves (max, sum, output) of its keys in LDS, then the workgroup's 256 threads
+// combine them, one (head, dim) pair at a time.  group <= 8.
+// ml / out: of head 0; the next head's lie ml_stride / out_stride floats on.
+__device__ __forceinline__ void att_merge_waves(int group, float m_run, float l_part, const pkv_f32x4 (&o)[8], float *ml, int ml_stride,
+                                                float *out, int out_stride) {
+  PKV_ATT_CONTRACT
+  const int lane = threadIdx.x & (PKV_WAVE - 1), wave = threadIdx.x / PKV_WAVE, n = lane & 15, j = lane >> 4;
+  __shared__ float s_m[kMfmaWaves][8], s_l[kMfmaWaves][8], s_o[kMfmaWaves][8][128 + 4];
+  if (j == 0 && n < group) s_m[wave][n] = m_run, s_l[wave][n] = l_part;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int head = 4 * j + i;
+    if (head < group) {
+      *(float4 *)&s_o[wave][head][8 * n] = float4{o[0][i], o[1][i], o[2][i], o[3][i]};
+      *(float4 *)&s_o[wave][head][8 * n + 4] = float4{o[4][i], o[5][i], o[6][i], o[7][i]};
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < group * 128; e += kMfmaWaves * PKV_WAVE) {
+    const int g = e >> 7, d = e & 127;
+    float mn = s_m[0][g];
+#pragma unroll
+    for (int w = 1; w < kMfmaWaves; ++w) mn = fmaxf(mn, s_m[w][g]);
+    float ls = 0.f, os = 0.f;
+#pragma unroll
+    for (int w = 0; w < kMfmaWaves; ++w) {
+      const float c = exp2f(s_m[w][g] - mn);
+      ls += s_l[w][g] * c;
+      os += s_o[w][g][d] * c;
+    }
+    out[g * out_stride + d] = os;
+    if (d == 0) ml[g * ml_stride] = mn, ml[g * ml_stride + 1] = ls;
+  }
+}
+
+template <bool INDEXED, typename SEGS>
+__device__ __forceinline__ void att_partial_mfma(const void *__restrict__ q, int group, const SEGS &segs, int64_t total,
+                                                 const int32_t *__restrict__ row_keys, int uniform, int64_t per_split,
+                                                 float scale_log2e, float *__restrict__ ws, int n_splits, int split, int row,
+                                                 int b, int h) {
+  PKV_ATT_CONTRACT
+  constexpr bool ONE = __is_same(SEGS, AttOne);
+  const int lane = threadIdx.x & (PKV_WAVE - 1), wave = threadIdx.x / PKV_WAVE;
+  const int n = lane & 15, j = lane >> 4;
+  total = att_row_total(total, row_keys, row, uniform);
+  const int64_t per_wave = per_split / kMfmaWaves;  // a multiple of the 32 keys of one step
+  const int64_t j0 = (int64_t)split * per_split + (int64_t)wave * per_wave;
+  const int64_t j1 = (j0 + per_wave < total) ? j0 + per_wave : total;  // j1 <= j0: nothing left for this wave
+
+  // Lane l holds the place of key blk0 + l of the current block of 64 keys (two steps; keys past j1 repeat the last one);
+  // the lanes that read a row get it from there, so that a place is found once per key and wave.
+  AttPlace<ONE> mine;
+  const char *kbase = nullptr, *vbase = nullptr;
+  if constexpr (ONE) {
+    const int64_t slab = (int64_t)b * segs.stride_b + (int64_t)h * segs.stride_h;
+    kbase = segs.k + slab, vbase = segs.v + slab;
+  }
+  auto place_block = [&](int64_t jb) {
+    const int64_t key = jb + lane;
+    mine = att_place<INDEXED, 256>(segs, row, b, h, (uint32_t)(key < j1 ? key : j1 - 1));
+  };
+  if (j0 < j1) place_block(j0);  // before the queries: the indices' latency is the longer one
+
+  const pkv_u32x4 zero4 = {0u, 0u, 0u, 0u};
+  pkv_u32x4 qb[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    qb[c] = n < group ? *(const pkv_u32x4 *)((const uint16_t *)q + ((int64_t)row * group + n) * 128 + 32 * c + 8 * j) : zero4;
+
+  float m_run = kNegBig, l_part = 0.f;
+  pkv_f32x4 o[8];
+#pragma unroll
+  for (int m = 0; m < 8; ++m) o[m] = pkv_f32x4{0.f, 0.f, 0.f, 0.f};
+
+  if (j0 < j1) att_step_mfma<ONE, true>(kbase, vbase, mine, 0, j0, j1, qb, scale_log2e, m_run, l_part, o);
+  for (int64_t jb = j0 + kMfmaStepKeys; jb < j1; jb += kMfmaStepKeys) {
+    const int in_block = (int)(jb - j0) & (PKV_WAVE - 1);
+    if (in_block == 0) place_block(jb);
+    att_step_mfma<ONE, false>(kbase, vbase, mine, in_block, jb, j1, qb, scale_log2e, m_run, l_part, o);
+  }
+
+  l_part += __shfl_xor(l_part, 16, PKV_WAVE);
+  l_part += __shfl_xor(l_part, 32, PKV_WAVE);
+  float *part = ws + ((int64_t)row * n_splits + split) * group * kPartStride;
+  att_merge_waves(group, m_run, l_part, o, part, kPartStride, part + 2, kPartStride);
+}
+
+// ---- a decode step's attention in two parts ----
+//
+// The sink and local rows are known before the retrieval starts, and a third of a short step went into the two launches behind
+// its top-k (4.9 + 2.7 of 26.5 us at 8 rows x 4096 keys), so: workgroups beside the query side of the retrieval, on an otherwise
+// idle chip, take the keys that are not selected, and the top-k's workgroups go on with those that are.  The sums are those of the
+// one-piece attention, bit for bit: the same blocks of 32 keys (a wave's), merged by fours into splits and the splits into the
+// output in the same order.
+constexpr int kSelBlocks = 8;   // most blocks of a selecting workgroup
+constexpr int kSelSplits = 12;  // one more than a row's splits may be where the selecting workgroup merges
+constexpr int kSelSlots = 32;   // partial results of a row there: splits in 0 .. 11, single blocks in 12 .. 19
+
+struct PkvSplitAttn {
+  AttOne segs;
+  uint32_t total;
+  int n_splits;               // of 128 keys
+  int blk_lo, blk_hi;         // blocks of 32 keys that hold a selected one; the top-k's workgroups take these ...
+  int sel_wgs, splits_per_wg; // ... sel_wgs == 1: one workgroup a row, which also merges; else whole splits, so many to a workgroup
+  uint32_t slots;             // sel_wgs == 1: the partial results that the first launch leaves
+  int n_dense, dense_a, dense_skip;  // workgroups of the first launch: splits 0 .. dense_a - 1, then from dense_a + dense_skip on
+  int n_kv_heads, group;
+  const void *q;
+  float scale_log2e;
+  float *ws;                  // sel_wgs == 1: outputs [row][20][group][128], then at ws_ml (max, sum) [row][group][kSelSlots]; else
+  float *ws_ml;               // partial results of the splits as the one-piece attention leaves them
+  void *out;
+};
+
+// sel_wgs == 1: a split with selected keys in some of its blocks leaves its other blocks one by one: the first such split in slots
+// 12 .. 15, another (the last) in 16 .. 19.
+__host__ __device__ __forceinline__ int att_block_slot(const PkvSplitAttn &a, int block) {
+  return kSelSplits + (block & 3) + (block / 4 == a.blk_lo / 4 ? 0 : 4);
+}
+__device__ __forceinline__ float *att_slot_o(const PkvSplitAttn &a, int row, int slot, int head) {
+  return a.ws + (uint32_t)(((row * 20 + slot) * a.group + head) * 128);
+}
+__device__ __forceinline__ float *att_slot_ml(const PkvSplitAttn &a, int row, int slot, int head) {
+  return a.ws_ml + (uint32_t)(((row * a.group + head) * kSelSlots + slot) * 2);
+}
+
+__device__ __forceinline__ void att_load_q(const PkvSplitAttn &a, int row, pkv_u32x4 (&qb)[4]) {
+  const int lane = pkv_lane(), n = lane & 15, j = lane >> 4;
+  const pkv_u32x4 zero4 = {0u, 0u, 0u, 0u};
+  const pkv_u32x4 *qp = (const pkv_u32x4 *)((const uint16_t *)a.q + ((int64_t)row * a.group + (n < a.group ? n : 0)) * 128 + 8 * j);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) qb[c] = qp[4 * c];
+  if (n >= a.group) qb[0] = qb[1] = qb[2] = qb[3] = zero4;
+}
+
+// Workgroup x of a row's n_dense: 256 threads.
+__device__ __forceinline__ void att_dense_part(const PkvSplitAttn &a, int x, int row) {
+  const int split = x < a.dense_a ? x : x + a.dense_skip;
+  const int lane = pkv_lane(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PKV_WAVE), n = lane & 15, j = lane >> 4;
+  const int b = row / a.n_kv_heads, h = row % a.n_kv_heads, block = 4 * split + wave;
+  const bool mixed = 4 * split + 3 >= a.blk_lo && 4 * split <= a.blk_hi;
+  const uint32_t j0 = 32u * (uint32_t)block, j1 = j0 + 32u < a.total ? j0 + 32u : a.total;
+  const bool has = j0 < a.total && !(block >= a.blk_lo && block <= a.blk_hi);
+  float m_run = kNegBig, l_part = 0.f;
+  pkv_f32x4 o[8];
+#pragma unroll
+  for (int m = 0; m < 8; ++m) o[m] = pkv_f32x4{0.f, 0.f, 0.f, 0.f};
+  if (has) {
+    const int64_t slab = (int64_t)b * a.segs.stride_b + (int64_t)h * a.segs.stride_h;
+    const uint32_t key = j0 + (uint32_t)(lane & 31);
+    const AttPlace<true> mine = att_place<false, 256>(a.segs, row, b, h, key < j1 ? key : j1 - 1);
+    pkv_u32x4 qb[4];
+    att_load_q(a, row, qb);
+    att_step_mfma<true, true>(a.segs.k + slab, a.segs.v + slab, mine, 0, j0, j1, qb, a.scale_log2e, m_run, l_part, o);
+  }
+  l_part += pkv_lane_xor_f<16>(l_part);
+  l_part += pkv_lane_xor_f<32>(l_part);
+  if (!mixed) {
+    if (a.sel_wgs == 1) {
+      att_merge_waves(a.group, m_run, l_part, o, att_slot_ml(a, row, split, 0), 2 * kSelSlots, att_slot_o(a, row, split, 0), 128);
+    } else {
+      float *part = a.ws + ((int64_t)row * a.n_splits + split) * a.group * kPartStride;
+      att_merge_waves(a.group, m_run, l_part, o, part, kPartStride, part + 2, kPartStride);
+    }
+  } else if (has) {
+    const int slot = att_block_slot(a, block);
+    if (lane < a.group) *(float2 *)att_slot_ml(a, row, slot, n) = float2{m_run, l_part};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int head = 4 * j + i;
+      if (head < a.group) {
+        float *dst = att_slot_o(a, row, slot, head) + 8 * n;
+        *(float4 *)dst = float4{o[0][i], o[1][i], o[2][i], o[3][i]};
+        *(float4 *)(dst + 4) = float4{o[4][i], o[5][i], o[6][i], o[7][i]};
+      }
+    }
+  }
+}
+
+constexpr int kSelThreadsAtt = 1024;  // threads of the selecting workgroup
+constexpr int kSelWaves = kSelThreadsAtt / PKV_WAVE;
+
+// What a merging workgroup needs beside its own keys, as requested.  The last waves merge (two to a head, the first head's the
+// last), the first ones take blocks: lane s of a merging wave the maximum and sum in slot s, its thread the outputs at its dim.
+struct AttSelRequests {
+  float2 ml;
+  float o[kSelSplits + 8];
+};
+
+__device__ __forceinline__ void att_request(const PkvSplitAttn &a, int row, AttSelRequests &p) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PKV_WAVE), g = (kSelWaves - 1 - wave) >> 1, lane = pkv_lane();
+  p.ml = float2{kNegBig, 0.f};
+#pragma unroll
+  for (int s = 0; s < kSelSplits + 8; ++s) p.o[s] = 0.f;
+  if (g >= a.group) return;
+  if (lane < kSelSlots && ((a.slots >> (lane & 31)) & 1u)) p.ml = *(const float2 *)(att_slot_ml(a, row, 0, g) + 2 * lane);
+  const float *base = att_slot_o(a, row, 0, g);
+  const uint32_t d = threadIdx.x & 127;
+#pragma unroll
+  for (int s = 0; s < kSelSplits + 8; ++s)
+    if ((a.slots >> s) & 1u) p.o[s] = (base + (uint32_t)(s * a.group * 128))[d];
+}
+
+__device__ __forceinline__ float att_lane(float x, int lane) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(x), lane));
+}
+
+// LDS of the selecting workgroups: the blocks of the splits that hold selected keys, the first of these splits first.
+struct AttSelSmem {
+  float m[8][16], l[8][16], o[kSelSplits][8][128 + 4];
+};
+
+// Clears (max, sum) of the blocks; a barrier lies between this and att_selected.
+__device__ __forceinline__ void att_clear(AttSelSmem &sm) {
+  if (threadIdx.x < 128) (&sm.m[0][0])[threadIdx.x] = kNegBig, (&sm.l[0][0])[threadIdx.x] = 0.f;
+}
+
+// The attention over the blocks with selected keys: ids s_sel[0 .. k) of row `row`, in LDS, made visible by the caller.  All 1024
+// threads, a block to a wave.  MERGE: all of them, merged with what the first launch left, into the output; else splits
+// wg * splits_per_wg .. of those with selected keys, each merged into a partial result of its own.  Bound by the instructions of
+// the waves on the one CU (each costs 16 cycles where all 16 waves run it) and one round trip to memory.
+template <bool MERGE>
+__device__ __forceinline__ void att_selected(const PkvSplitAttn &a, int row, const uint32_t *s_sel, int wg, AttSelSmem &sm,
+                                             const AttSelRequests &req) {
+  PKV_ATT_CONTRACT
+  const int tid = threadIdx.x, lane = tid & (PKV_WAVE - 1), wave = __builtin_amdgcn_readfirstlane(tid / PKV_WAVE);
+  const int split0 = a.blk_lo / 4 + (MERGE ? 0 : wg * a.splits_per_wg), splits = MERGE ? a.blk_hi / 4 - split0 + 1 : a.splits_per_wg;
+  const int block = MERGE ? a.blk_lo + wave : 4 * split0 + wave, local = block - 4 * split0;
+  const uint32_t j0 = 32u * (uint32_t)block, j1 = j0 + 32u < a.total ? j0 + 32u : a.total;
+  if ((MERGE ? block <= a.blk_hi : local < 4 * splits && block / 4 <= a.blk_hi / 4) && j0 < a.total) {
+    const int n = lane & 15, j = lane >> 4, b = row / a.n_kv_heads, h = row % a.n_kv_heads;
+    const int64_t slab = (int64_t)b * a.segs.stride_b + (int64_t)h * a.segs.stride_h;
+    uint32_t key = j0 + (uint32_t)(lane & 31);
+    key = key < j1 ? key : j1 - 1;
+    AttPlace<true> mine = att_place<false, 256>(a.segs, row, b, h, key);
+    if (key >= a.segs.idx_lo && key < a.segs.idx_hi) {
+      const uint32_t id = s_sel[key - a.segs.idx_lo], limit = (uint32_t)a.segs.idx_limit;
+      mine.off = (a.segs.idx_row0 + (id < limit ? id : limit - 1)) * 256u;
+    }
+    pkv_u32x4 qb[4];
+    att_load_q(a, row, qb);
+    float m_run = kNegBig, l_part = 0.f;
+    pkv_f32x4 o[8];
+    att_step_mfma<true, true>(a.segs.k + slab, a.segs.v + slab, mine, 0, j0, j1, qb, a.scale_log2e, m_run, l_part, o);
+    l_part += pkv_lane_xor_f<16>(l_part);
+    l_part += pkv_lane_xor_f<32>(l_part);
+    if (lane < a.group) sm.m[n][local] = m_run, sm.l[n][local] = l_part;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int head = 4 * j + i;
+      if (head < a.group) {
+        *(float4 *)&sm.o[local][head][8 * n] = float4{o[0][i], o[1][i], o[2][i], o[3][i]};
+        *(float4 *)&sm.o[local][head][8 * n + 4] = float4{o[4][i], o[5][i], o[6][i], o[7][i]};
+      }
+    }
+  }
+  const int g = (kSelWaves - 1 - wave) >> 1, d = tid & 127;
+  if (MERGE && g < a.group) {  // the other blocks of these splits
+    const int slot = lane - kSelSplits;
+    if (slot >= 0 && slot < 8 && ((a.slots >> lane) & 1u) && (tid & 64)) {
+      const int at = slot < 4 ? slot : 4 * (splits - 1) + slot - 4;
+      sm.m[g][at] = req.ml.x, sm.l[g][at] = req.ml.y;
+    }
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      if ((a.slots >> (kSelSplits + t)) & 1u) sm.o[t < 4 ? t : 4 * (splits - 1) + t - 4][g][d] = req.o[kSelSplits + t];
+  }
+  __syncthreads();
+  if constexpr (!MERGE) {
+    for (int e = tid; e < splits * a.group * 128; e += kSelThreadsAtt) {
+      const int sub = (e >> 7) / a.group, gg = (e >> 7) % a.group, dd = e & 127, w0 = 4 * sub, split = split0 + sub;
+      if (split > a.blk_hi / 4) break;
+      float mn = sm.m[gg][w0];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) mn = fmaxf(mn, sm.m[gg][w0 + w]);
+      float ls = 0.f, os = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        const float c = exp2f(sm.m[gg][w0 + w] - mn);
+        ls = fmaf(sm.l[gg][w0 + w], c, ls);
+        if (32u * (uint32_t)(4 * split + w) < a.total) os = fmaf(sm.o[w0 + w][gg][dd], c, os);
+      }
+      float *part = a.ws + (((int64_t)row * a.n_splits + split) * a.group + gg) * kPartStride;
+      part[2 + dd] = os;
+      if (dd == 0) part[0] = mn, part[1] = ls;
+    }
+  } else {
+    if (g >= a.group) return;
+    // lane = split: its maximum and sum; cw: the weights of the blocks of a split that holds selected keys
+    const bool own = lane >= split0 && lane < split0 + splits;
+    const float4 mw = *(const float4 *)&sm.m[g][own ? 4 * (lane - split0) : 0], lw = *(const float4 *)&sm.l[g][own ? 4 * (lane - split0) : 0];
+    const float mx = fmaxf(fmaxf(mw.x, mw.y), fmaxf(mw.z, mw.w));
+    const float cw[4] = {exp2f(mw.x - mx), exp2f(mw.y - mx), exp2f(mw.z - mx), exp2f(mw.w - mx)};
+    // in the order of the one-piece merge, which the compiler may otherwise turn round (a b + c d has two fused forms)
+    const float ls = fmaf(lw.w, cw[3], fmaf(lw.z, cw[2], fmaf(lw.y, cw[1], lw.x * cw[0])));
+    const bool split_lane = lane < kSelSplits;  // the lanes behind hold single blocks
+    const float mi = own ? mx : split_lane ? req.ml.x : kNegBig, li = own ? ls : split_lane ? req.ml.y : 0.f;
+    float mn = mi;
+#define PKV_ATT_MAX(M) mn = fmaxf(mn, pkv_lane_xor_f<M>(mn));
+    PKV_ATT_MAX(1) PKV_ATT_MAX(2) PKV_ATT_MAX(4) PKV_ATT_MAX(8) PKV_ATT_MAX(16) PKV_ATT_MAX(32)
+#undef PKV_ATT_MAX
+    const float c = exp2f(mi - mn);
+    float tot = fmaf(li, c, pkv_lane_xor_f<1>(li * c));
+#define PKV_ATT_ADD(M) tot += pkv_lane_xor_f<M>(tot);
+    PKV_ATT_ADD(2) PKV_ATT_ADD(4) PKV_ATT_ADD(8) PKV_ATT_ADD(16) PKV_ATT_ADD(32)
+#undef PKV_ATT_ADD
+    const float weight = c / tot;
+    float os = 0.f;
+#pragma unroll
+    for (int s = 0; s < kSelSplits; ++s) {
+      if (s < a.n_splits) {  // the same in the whole workgroup, as the next
+        float x = req.o[s];
+        if (s >= split0 && s < split0 + splits) {
+          x = 0.f;
+#pragma unroll
+          for (int w = 0; w < 4; ++w)
+            if (32u * (uint32_t)(4 * s + w) < a.total) x = fmaf(sm.o[4 * (s - split0) + w][g][d], att_lane(cw[w], s), x);
+        }
+        os = fmaf(x, att_lane(weight, s), os);
+      }
+    }
+    ((uint16_t *)a.out)[((int64_t)row * a.group + g) * 128 + d] = pkv_f32_to_bf16_bits(os);
+  }
+}
+
+// The merge of a row's splits (where sel_wgs > 1).
+PKV_INTERNAL int pkv_launch_attn_merge(const PkvSplitAttn &a, int rows, hipStream_t s);
+// Whether pkv_decode_step's attention over `attn` can be taken in two parts around a top-k of k ids into out_ids; fills `out`.
+PKV_INTERNAL bool pkv_plan_split_attention(const pkv_retrieve_args *r, const pkv_attn_args *attn, PkvSplitAttn *out);
+
+#endif  // __HIPCC__

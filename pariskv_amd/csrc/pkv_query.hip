@@ -7,7 +7,7 @@
 // nested tier bitsets of the reference collapse into one weight per centroid:
 // weight = number of tiers whose key budget is not yet exhausted at the
 // centroid's rank.
-#include "pkv_common.h"
+#include "pkv_attn.h"
 #include "pkv_lut.h"
 
 namespace {
@@ -48,6 +48,28 @@ __global__ __launch_bounds__(256) void pkv_query_prep_lut_kernel(
                          tiers, sub, sm, lut + ((int64_t)row * 16 + sub) * 256,
                          sub == 0 ? qhat + (int64_t)row * 128 : nullptr, sub == 0 ? qnorm + row : nullptr,
                          sorted_ids ? sorted_ids + ((int64_t)row * 16 + sub) * 256 : nullptr);
+}
+
+// The same beside the part of the step's attention that waits for nothing: workgroups 16 and up of a row (see PkvSplitAttn).
+// us: 8 rows x 4096 keys 4.6 -> 5.1 with five such workgroups a row, 32 rows x 16000, 8 heads, 7.1 with six.  The
+// bound keeps the compiler from accumulation registers: 76 registers instead of 62 and 64 of those, six waves a SIMD instead of
+// four; decode step of 64 rows x 65536 keys, 2 layers, 117.7 / 112.8.
+__global__ __launch_bounds__(256, 4) void pkv_query_prep_attend_kernel(
+    const void *__restrict__ q, int n_kv_heads, int group, const float *__restrict__ signs, const int32_t *__restrict__ cc,
+    float *__restrict__ qhat, float *__restrict__ qnorm, int64_t cc_b, int64_t cc_h, PkvTiers tiers, uint8_t *__restrict__ lut,
+    uint32_t *__restrict__ row_suf_to_zero, PkvSplitAttn attn) {
+  const int sub = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
+  if (sub >= 16) {
+    att_dense_part(attn, sub - 16, row);
+    return;
+  }
+  const int b = row / n_kv_heads, h = row % n_kv_heads;
+  if (row_suf_to_zero && sub == 1 && tid < 128) row_suf_to_zero[(int64_t)row * 128 + tid] = 0u;
+  __shared__ PkvLutSmem sm;
+  pkv_lut_build_subspace(q, PKV_DTYPE_BF16, b, h, n_kv_heads, group, signs,
+                         cc + (int64_t)b * cc_b + (int64_t)h * cc_h + sub * 256, tiers, sub, sm,
+                         lut + ((int64_t)row * 16 + sub) * 256, sub == 0 ? qhat + (int64_t)row * 128 : nullptr,
+                         sub == 0 ? qnorm + row : nullptr, nullptr);
 }
 
 // Ranking supplied by the caller (reference-shaped API).  grid (16, R), 256 threads.
@@ -94,6 +116,17 @@ int pkv_launch_query_prep_lut(const void *q, int dtype, int bs, int n_kv_heads, 
                        tiers, qhat, qnorm, lut, sorted_ids, row_suf_to_zero, zero_ptr, zero_ptr ? zero_words : 0, PkvDenseLogits());
   }
   PKV_LAUNCH_CHECK("pkv_query_prep_lut_kernel");
+  return PKV_OK;
+}
+
+// The query side of the retrieval with the dense part of the attention beside it; nothing to clear for the top-k (a top-k that
+// attends has no control area).
+int pkv_launch_query_prep_attend(const pkv_retrieve_args *a, const PkvTiers &tiers, float *qhat, float *qnorm, uint8_t *lut,
+                                 uint32_t *row_suf_to_zero, const PkvSplitAttn &attn, hipStream_t s) {
+  hipLaunchKernelGGL(pkv_query_prep_attend_kernel, dim3((unsigned)(16 + attn.n_dense), (unsigned)(a->bs * a->n_kv_heads)), dim3(256),
+                     0, s, a->q, a->n_kv_heads, a->group, a->signs, a->cluster_counts, qhat, qnorm, (int64_t)a->n_kv_heads * 4096,
+                     (int64_t)4096, tiers, lut, row_suf_to_zero, attn);
+  PKV_LAUNCH_CHECK("pkv_query_prep_attend_kernel");
   return PKV_OK;
 }
 

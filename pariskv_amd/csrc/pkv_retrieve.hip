@@ -6,7 +6,7 @@
 //
 // Reference: cache_hub/polar_cache.py:1126-1162 (collision_based_topk_batch),
 // :1207-1231, :1244-1304 and the gather at :1075-1095.
-#include "pkv_common.h"
+#include "pkv_attn.h"
 
 #include <mutex>
 
@@ -16,6 +16,10 @@ PKV_INTERNAL int pkv_launch_qk_norm_rope_table(const void *qkv, int64_t stride_b
                                   const void *sin_row, void *q_out, void *k_out, const float *signs, const int32_t *cc,
                                   const PkvTiers &tiers, float *qhat, float *qnorm, uint8_t *lut, uint32_t *row_suf,
                                   uint32_t *zero_ptr, int64_t zero_words, const pkv_kv_append *append, hipStream_t s);
+PKV_INTERNAL int pkv_launch_query_prep_attend(const pkv_retrieve_args *a, const PkvTiers &tiers, float *qhat, float *qnorm, uint8_t *lut,
+                                              uint32_t *row_suf_to_zero, const PkvSplitAttn &attn, hipStream_t s);
+PKV_INTERNAL int pkv_launch_topk_attend(const float *x, int64_t x_stride, const int64_t *ids, int64_t ids_stride, int rows, int64_t len,
+                                        int64_t k, int64_t *out_ids, float *out_vals, const PkvSplitAttn &attn, hipStream_t s);
 PKV_INTERNAL size_t pkv_fused_sync_bytes(int rows, int64_t n_chunks);
 PKV_INTERNAL bool pkv_fused_usable(int rows, int64_t n_keys, int chunk_keys, hipStream_t s);
 PKV_INTERNAL int pkv_launch_fused_retrieve(const void *q, int dtype, int bs, int n_kv_heads, int group, const float *signs,
@@ -119,8 +123,9 @@ extern "C" int pkv_retrieve_ws_view(void *ws, int rows, int64_t n_keys, int64_t 
 }
 
 // dense (or null): the adaptive-k step's dense tokens, whose logits ride with the query prep where that is a launch of its own
+// attn (or null): the step's attention in two parts, the first of which rides there as well and the second with the top-k
 static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, void *stream, const PkvDenseLogits *dense = nullptr,
-                         int least_chunk = 256) {
+                         int least_chunk = 256, const PkvSplitAttn *attn = nullptr) {
   PKV_REQUIRE(a != nullptr, "pkv_retrieve: null args");
   PKV_REQUIRE(a->q && a->signs && a->centers && a->cluster_counts && a->codes && a->nib && a->weight,
               "pkv_retrieve: null pointer");
@@ -190,8 +195,9 @@ static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, 
   } else {
     // table_ready: pkv_qk_norm_rope_table already left the rotated query, its norm and the vote table of these
     // queries in the workspace and cleared what this launch would clear
-    rc = a->table_ready ? PKV_OK
-                        : pkv_launch_query_prep_lut(a->q, a->dtype, a->bs, H, a->group, a->signs, a->cluster_counts,
+    rc = a->table_ready           ? PKV_OK
+         : attn && attn->n_dense ? pkv_launch_query_prep_attend(a, t, qhat, qnorm, lut, rowsuf, *attn, s)
+                                  : pkv_launch_query_prep_lut(a->q, a->dtype, a->bs, H, a->group, a->signs, a->cluster_counts,
                                                     (int64_t)H * 4096, 4096, t, qhat, qnorm, lut, nullptr, rowsuf, s, topk_ctl,
                                                     ctl_words, dense);
     if (rc) return rc;
@@ -219,6 +225,8 @@ static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, 
     if (rc) return rc;
   }
   if (!a->out_ids) return PKV_OK;  // candidates only: the caller reads them out of the workspace
+  if (attn)
+    return pkv_launch_topk_attend(scores, a->n_cand, cand, a->n_cand, rows, a->n_cand, a->k, a->out_ids, a->out_scores, *attn, s);
   rc = pkv_launch_topk_f32(scores, a->n_cand, cand, a->n_cand, rows, a->n_cand, a->k, a->out_ids, a->out_scores,
                            (char *)ws + w.topk, w.topk_bytes, s, a->any_order != 0, topk_ctl != nullptr);
   if (rc) return rc;
@@ -353,6 +361,8 @@ extern "C" int pkv_retrieve_noalloc(const pkv_retrieve_args *a, void *stream) {
 extern "C" int pkv_decode_step(const pkv_retrieve_args *retrieve, void *ws, size_t ws_bytes,
                                const pkv_attn_args *attention, void *stream) {
   PKV_REQUIRE(retrieve && attention, "pkv_decode_step: null args");
+  PkvSplitAttn split;
+  if (pkv_plan_split_attention(retrieve, attention, &split)) return retrieve_impl(retrieve, ws, ws_bytes, stream, nullptr, 256, &split);
   int rc = pkv_retrieve(retrieve, ws, ws_bytes, stream);
   if (rc) return rc;
   return pkv_decode_attention_run(retrieve->q, retrieve->dtype, retrieve->bs, retrieve->n_kv_heads, retrieve->group, attention,

@@ -12,7 +12,7 @@
 // workgroup the global threshold and its own output offsets, so the candidate
 // list is produced in one pass, in a fixed order: indices above the threshold
 // ascending, then indices at the threshold ascending.
-#include "pkv_common.h"
+#include "pkv_attn.h"
 #include "pkv_selcore.h"
 
 namespace {
@@ -1065,10 +1065,12 @@ __device__ __forceinline__ void collect_winners_streamed(KeyFn key_of, int64_t l
 // SORTED = false leaves the sort out: the winners come out in a fixed order of their positions in the row (by the
 // wave that loaded them, then by element index, then by lane: a function of the inputs only), for callers that use
 // them as a set (gather + attention).
-template <int EIN, bool SORTED>
-__global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_sort_kernel(
-    const float *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ ids, int64_t ids_stride, int len, int P,
-    int64_t k, int64_t *__restrict__ out_ids, float *__restrict__ out_vals) {
+// s_sel (or null; any order only): the ids in LDS as well, for the caller to go on with after a barrier; out_ids may be null then.
+// more(): called once the row's own loads are requested.
+template <int EIN, bool SORTED, typename Requests>
+__device__ __forceinline__ void topk_select_sort(const float *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ ids,
+                                                 int64_t ids_stride, int len, int P, int64_t k, int64_t *__restrict__ out_ids,
+                                                 float *__restrict__ out_vals, uint32_t *s_sel, Requests more) {
   extern __shared__ uint64_t s_keys[];
   __shared__ uint32_t s_hist[2 * kLinBins];
   __shared__ uint32_t s_cnt[kLinBins];
@@ -1094,6 +1096,7 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_sort_kernel(
     const int i = tid + e * kTopkThreads;
     id[e] = ir ? (uint32_t)ir[i < len ? i : len - 1] : (uint32_t)i;
   }
+  more();
 #pragma unroll
   for (int e = 0; e < EIN; ++e)
     v[e] = tid + e * kTopkThreads < len ? ((uint64_t)pkv_ordered_u32(__uint_as_float(score[e])) << 32) | 1ull : 0ull;
@@ -1107,8 +1110,8 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_sort_kernel(
 #pragma unroll
   for (int e = 0; e < EIN; ++e)  // the whole keys
     if (v[e] != 0ull) v[e] = (v[e] & 0xffffffff00000000ull) | (uint64_t)(uint32_t)~id[e];
-  int64_t *oi = out_ids + (int64_t)row * k;
-  float *ov = out_vals ? out_vals + (int64_t)row * k : nullptr;
+  int64_t *oi = out_ids ? out_ids + (int64_t)row * k : nullptr;
+  float *ov = out_ids && out_vals ? out_vals + (int64_t)row * k : nullptr;
   if (SORTED && lin && L.max_winners <= kLinRankMax) {
     // counting sort: a key of a bin above b* takes a slot of [off[b], off[b] + count[b]) and the keys of b* go to
     // a list of their own; then every key counts the larger keys of its own bin, which is its place inside the
@@ -1167,14 +1170,16 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_sort_kernel(
     for (int e = 0; e < EIN; ++e) {
       const uint32_t mine = slot + (uint32_t)__popcll(ballot[e] & below);
       if (((ballot[e] >> pkv_lane()) & 1ull) && mine < n_above) {
-        oi[mine] = (int64_t)(uint32_t)(~(uint32_t)v[e]);
+        if (oi) oi[mine] = (int64_t)(uint32_t)(~(uint32_t)v[e]);
+        if (s_sel) s_sel[mine] = ~(uint32_t)v[e];
         if (ov) ov[mine] = pkv_from_ordered_u32((uint32_t)(v[e] >> 32));
       }
       slot += (uint32_t)__popcll(ballot[e]);
     }
     rank_bucket_desc(s_bucket, L.in_bstar, [&](uint64_t key, uint32_t r) {
       if (r < L.need) {
-        oi[n_above + r] = (int64_t)(uint32_t)(~(uint32_t)key);
+        if (oi) oi[n_above + r] = (int64_t)(uint32_t)(~(uint32_t)key);
+        if (s_sel) s_sel[n_above + r] = ~(uint32_t)key;
         if (ov) ov[n_above + r] = pkv_from_ordered_u32((uint32_t)(key >> 32));
       }
     });
@@ -1213,7 +1218,8 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_sort_kernel(
     for (int e = 0; e < EIN; ++e) {
       const uint32_t mine = slot + (uint32_t)__popcll(ballot[e] & below);
       if (win[e] && mine < (uint32_t)k) {
-        oi[mine] = (int64_t)(uint32_t)(~(uint32_t)v[e]);
+        if (oi) oi[mine] = (int64_t)(uint32_t)(~(uint32_t)v[e]);
+        if (s_sel) s_sel[mine] = ~(uint32_t)v[e];
         if (ov) ov[mine] = pkv_from_ordered_u32((uint32_t)(v[e] >> 32));
       }
       slot += (uint32_t)__popcll(ballot[e]);
@@ -1229,6 +1235,31 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_sort_kernel(
 #define PKV_SORT_K(NT, E) sort_lds_keys_and_emit<NT, E>(s_keys, k, oi, ov, nullptr)
   PKV_DISPATCH_E(P, PKV_SORT_K);
 #undef PKV_SORT_K
+}
+
+template <int EIN, bool SORTED>
+__global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_sort_kernel(
+    const float *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ ids, int64_t ids_stride, int len, int P,
+    int64_t k, int64_t *__restrict__ out_ids, float *__restrict__ out_vals) {
+  topk_select_sort<EIN, SORTED>(x, x_stride, ids, ids_stride, len, P, k, out_ids, out_vals, nullptr, [] {});
+}
+
+// The selection in any order, and the attention over what it selected: see att_selected.  grid (rows, sel_wgs): with several
+// every workgroup selects for itself (the same ids in the same order) and attends to its share.  Dynamic LDS: k words.
+template <int EIN, bool MERGE>
+__global__ __launch_bounds__(kTopkThreads) void pkv_topk_attend_kernel(
+    const float *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ ids, int64_t ids_stride, int len, int64_t k,
+    int64_t *__restrict__ out_ids, float *__restrict__ out_vals, PkvSplitAttn attn) {
+  extern __shared__ uint32_t s_sel[];
+  __shared__ AttSelSmem sm;
+  static_assert(kTopkThreads == kSelThreadsAtt, "one workgroup does both");
+  const int row = blockIdx.x, wg = MERGE ? 0 : blockIdx.y;
+  AttSelRequests req;
+  att_clear(sm);
+  topk_select_sort<EIN, false>(x, x_stride, ids, ids_stride, len, 0, k, wg ? nullptr : out_ids, out_vals, s_sel,
+                               [&] { if (MERGE) att_request(attn, row, req); });
+  __syncthreads();
+  att_selected<MERGE>(attn, row, s_sel, wg, sm, req);
 }
 
 // ------------------------------------------------- rows wider than one workgroup
@@ -2331,6 +2362,30 @@ extern "C" size_t pkv_topk_f32_ws_bytes(int rows, int64_t len, int64_t k) {
   return pkv_topk_ws_bytes_impl(rows, len, k);
 }
 
+// Rows that one workgroup selects from, well short of all their keys (anything else sorts the row or spreads it).
+bool pkv_topk_selects(int64_t len, int64_t k) {
+  return len <= kTopkMaxSort && pow2_ceil(k) * 2 <= pow2_ceil(len) && pow2_ceil(len) >= 2048;
+}
+
+int pkv_launch_topk_attend(const float *x, int64_t x_stride, const int64_t *ids, int64_t ids_stride, int rows, int64_t len,
+                           int64_t k, int64_t *out_ids, float *out_vals, const PkvSplitAttn &attn, hipStream_t s) {
+  const int ein = pow2_ceil(len) / kTopkThreads;
+#define PKV_SEL_ATT(EIN, MERGE)                                                                                              \
+  hipLaunchKernelGGL((pkv_topk_attend_kernel<EIN, MERGE>), dim3((unsigned)rows, (unsigned)attn.sel_wgs), dim3(kTopkThreads), \
+                     (size_t)k * 4, s, x, x_stride, ids, ids_stride, (int)len, k, out_ids, out_vals, attn)
+#define PKV_SEL_ATT_E(MERGE)                \
+  do {                                      \
+    if (ein <= 2) PKV_SEL_ATT(2, MERGE);      \
+    else if (ein == 4) PKV_SEL_ATT(4, MERGE); \
+    else PKV_SEL_ATT(8, MERGE);               \
+  } while (0)
+  if (attn.sel_wgs == 1) PKV_SEL_ATT_E(true); else PKV_SEL_ATT_E(false);
+#undef PKV_SEL_ATT_E
+#undef PKV_SEL_ATT
+  PKV_LAUNCH_CHECK("pkv_topk_attend_kernel");
+  return attn.sel_wgs == 1 ? PKV_OK : pkv_launch_attn_merge(attn, rows, s);
+}
+
 int pkv_launch_topk_f32(const float *x, int64_t x_stride, const int64_t *ids, int64_t ids_stride, int rows,
                         int64_t len, int64_t k, int64_t *out_ids, float *out_vals, void *ws, size_t ws_bytes,
                         hipStream_t s, bool any_order, bool ctl_ready) {
@@ -2338,7 +2393,7 @@ int pkv_launch_topk_f32(const float *x, int64_t x_stride, const int64_t *ids, in
   PKV_REQUIRE(k > 0, "k must be positive");
   PKV_REQUIRE(k <= len, "k cannot exceed sequence length");
   PKV_REQUIRE(rows > 0 && rows <= 65535 && len < ((int64_t)1 << 31), "bad shape rows=%d len=%lld", rows, (long long)len);
-  if (len <= kTopkMaxSort && pow2_ceil(k) * 2 <= pow2_ceil(len) && pow2_ceil(len) >= 2048) {
+  if (pkv_topk_selects(len, k)) {
     const int P = pow2_ceil(k);
     const int ein = pow2_ceil(len) / kTopkThreads;
 #define PKV_SEL(EIN, SORTED)                                                                                      \

@@ -1957,3 +1957,36 @@ def test_prefill_store_index_layouts(ops, dtype, layout, norms, n_enc):
     if norms:
         want[:, :, :n_enc, 1] = want_n[..., :n_enc]
     assert torch.equal(zn, want)
+
+
+@pytest.mark.parametrize("group,k,sink,tail", [
+    (4, 100, 64, 529), (1, 1, 0, 1), (3, 15, 3, 0), (5, 16, 64, 64), (8, 17, 64, 1100), (2, 33, 95, 30), (6, 256, 1, 130), (4, 256, 64, 700),
+    (7, 257, 0, 0), (4, 512, 64, 700), (8, 100, 64, 1300), (6, 1024, 64, 1300), (4, 64, 31, 1), (2, 31, 129, 65)])
+def test_decode_step_in_place_attends_in_two_parts(ops, group, k, sink, tail):
+    """The step whose attention reads selected rows where they lie: the other rows beside the query side, selected rows in the
+    top-k's workgroups.  The same ids and the same sums, bit for bit, as the top-k and the attention called one by one; and the
+    attention against 64 bits: probabilities and output are rounded to 8 bits, 2^-9 of the largest value each."""
+    _say(f"two-part attention group {group} k {k} sink {sink} tail {tail}")
+    w = W.make_workload("two_parts", 2, 2, group, 3000, 1500, k, O.BF16, 0.5, seed0=11)
+    d = W.to_device(w, DEV, torch)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    rows = sink + w.N + tail
+    kk, vv = (torch.randn(w.bs, w.H, rows, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    plan = ops.RetrievePlan(w.bs, w.H, w.G, w.N, DEV, w.N, w.C, w.K)
+    att = ops.DecodeAttention(w.bs, w.H, w.G, rows, DEV)
+    args = (d["queries"], d["signs"], d["centers"], d["cluster_counts"], d["codes_km"], d["nib_km"], d["w_km"], 0, w.N, w.tiers, w.C, w.K)
+    want_ids = plan.run(*args, any_order=True)
+    ids = torch.zeros_like(want_ids)
+    segs = [s for s in [(kk, vv, 0, sink), (kk, vv, sink, k, ids), (kk, vv, sink + w.N, tail)] if s[3]]
+    plan.run(*args, out_ids=ids, attention=(att, segs, None), any_order=True)
+    torch.cuda.synchronize()
+    got = plan.attn_out.clone()
+    assert torch.equal(ids, want_ids)
+    assert torch.equal(got, att.run(d["queries"], segs))
+    sel = torch.cat([torch.arange(sink, device=DEV).expand(w.bs, w.H, -1), sink + ids,
+                     torch.arange(sink + w.N, rows, device=DEV).expand(w.bs, w.H, -1)], dim=2)[..., None].expand(-1, -1, -1, 128)
+    ks, vs = (t.gather(2, sel).double().cpu() for t in (kk, vv))
+    q = d["queries"].view(w.bs, w.H, group, 128).double().cpu()
+    want = torch.softmax(q @ ks.transpose(2, 3) / 128 ** 0.5, dim=-1) @ vs
+    err = (got.view(w.bs, w.H, group, 128).double().cpu() - want).abs().max().item()
+    assert err <= vv.abs().max().item() * 2.0 ** -8, err
