@@ -140,15 +140,17 @@ bool as_one_tensor(const AttSegs &sg, int es, AttOne &one) {
 
 }  // namespace
 
-PKV_INTERNAL bool pkv_topk_selects(int64_t len, int64_t k);
-
-// One CU fetches scattered rows at 35 to 40 GB/s, 2.7 us for 200 of them and as much as the merge's launch: up to eight blocks of 32
+// One CU fetches scattered rows at 35 to 40 GB/s, 2.7 us for 200 of them and as much as the merge's launch: up to five blocks of 32
 // are one workgroup's, which then merges; more go to a workgroup per split of 128, each selecting anew, or per two or three where
-// that would be more workgroups than CUs.  Decode step, us, attention after the top-k / in two parts: 8 rows x 4096 keys, top 100,
-// 28.2 / 23.9, top 256 28.6 / 26.0; 8 x 32768, top 512, 30.0 / 27.1; 32 x 16000, 8 heads, top 100 34.5 / 31.0, top 512 36.9 / 33.4;
-// 64 x 40000, top 256 48.9 / 44.7, top 512 52.4 / 46.9; 64 x 65536, top 100, 56.3 / 52.2; 256 x 8000, top 100, 73.1 / 59.8.
-constexpr int kSplitWorkgroups = 256;
-constexpr int64_t kSplitMaxSelected = 1024;
+// that would be more workgroups than CUs; there up to eight blocks are one workgroup's as well.  Where the selection takes several
+// launches (more than 8192 candidates), only the first form: its last launch is too long to be run by several workgroups a row.
+// Decode step, us, attention after the top-k / in two parts: 8 rows x 4096 keys, top 100, 28.2 / 23.9, top 256 25.5 / 23.7 (25.5 by
+// one workgroup a row); 8 x 32768, top 512, 30.0 / 27.1; 32 x 16000, 8 heads, top 100 34.5 / 31.0, top 512 36.9 / 33.4; 64 x 40000,
+// top 256 46.5 / 44.7, top 512 52.4 / 46.9; 64 x 65536, top 100, 56.3 / 52.2; 256 x 8000, top 100, 73.1 / 59.8, top 256 77.1 / 67.7
+// (76.7 by several a row).  More than 8192 candidates: 8 x 100000, top 100, 45.7 / 42.9, 64 x 100000 88.8 / 87.9; by several
+// workgroups a row 16 x 131072, top 200, 52.0 / 52.5.
+constexpr int kSplitWorkgroups = 256, kMergeBlocks = 5;
+constexpr int64_t kSplitMaxSelected = 1024, kSplitMaxCand = 8192;
 
 extern "C" size_t pkv_decode_attention_ws_bytes(int bs, int n_kv_heads, int group, int64_t total_keys) {
   if (bs <= 0 || n_kv_heads <= 0 || group <= 0 || total_keys <= 0) return 256;
@@ -287,7 +289,7 @@ bool pkv_plan_split_attention(const pkv_retrieve_args *r, const pkv_attn_args *a
   if (r->launch_plan != PKV_PLAN_SEPARATE || r->table_ready) return false;
   // The selection: in any order, of one workgroup a row, into the list that the attention reads, nothing gathered.
   if (!r->out_ids || !r->any_order || r->src_k || r->n_cand == r->n_keys || at->row_keys || r->k > kSplitMaxSelected ||
-      !pkv_topk_selects(r->n_cand, r->k))
+      !pkv_topk_attends(r->n_cand, r->k))
     return false;
   for (int i = 0; i < at->n_segments; ++i) {
     const pkv_attn_segment &s = at->segments[i];
@@ -311,7 +313,8 @@ bool pkv_plan_split_attention(const pkv_retrieve_args *r, const pkv_attn_args *a
   out->total = (uint32_t)total;
   out->blk_lo = (int)(out->segs.idx_lo / kMfmaStepKeys), out->blk_hi = (int)((out->segs.idx_hi - 1) / kMfmaStepKeys);
   const int lo = out->blk_lo / kMfmaWaves, hi = out->blk_hi / kMfmaWaves, n_sel = hi - lo + 1;  // splits with selected keys
-  if (out->blk_hi - out->blk_lo < kSelBlocks && out->n_splits < kSelSplits) {
+  const int blocks = out->blk_hi - out->blk_lo + 1;
+  if (out->n_splits < kSelSplits && (blocks <= kMergeBlocks || (blocks <= kSelBlocks && (int64_t)rows * n_sel > kSplitWorkgroups))) {
     out->sel_wgs = 1;
     // the splits between the first and the last one's own blocks have nothing else to do
     const int last_block = (int)((total - 1) / kMfmaStepKeys);
@@ -324,6 +327,8 @@ bool pkv_plan_split_attention(const pkv_retrieve_args *r, const pkv_attn_args *a
     }
     if ((int64_t)rows * 20 * r->group * 128 >= ((int64_t)1 << 31)) return false;
     out->ws_ml = (float *)at->ws + (int64_t)rows * 20 * r->group * 128;
+  } else if (r->n_cand > kSplitMaxCand) {
+    return false;
   } else {
     do {
       out->sel_wgs = (n_sel + ++out->splits_per_wg - 1) / out->splits_per_wg;

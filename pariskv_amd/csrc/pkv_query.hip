@@ -57,13 +57,14 @@ __global__ __launch_bounds__(256) void pkv_query_prep_lut_kernel(
 __global__ __launch_bounds__(256, 4) void pkv_query_prep_attend_kernel(
     const void *__restrict__ q, int n_kv_heads, int group, const float *__restrict__ signs, const int32_t *__restrict__ cc,
     float *__restrict__ qhat, float *__restrict__ qnorm, int64_t cc_b, int64_t cc_h, PkvTiers tiers, uint8_t *__restrict__ lut,
-    uint32_t *__restrict__ row_suf_to_zero, PkvSplitAttn attn) {
+    uint32_t *__restrict__ row_suf_to_zero, uint32_t *__restrict__ zero_ptr, int64_t zero_words, PkvSplitAttn attn) {
   const int sub = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
   if (sub >= 16) {
     att_dense_part(attn, sub - 16, row);
     return;
   }
   const int b = row / n_kv_heads, h = row % n_kv_heads;
+  for (int64_t i = ((int64_t)row * 16 + sub) * 256 + tid; i < zero_words; i += (int64_t)16 * gridDim.y * 256) zero_ptr[i] = 0u;
   if (row_suf_to_zero && sub == 1 && tid < 128) row_suf_to_zero[(int64_t)row * 128 + tid] = 0u;
   __shared__ PkvLutSmem sm;
   pkv_lut_build_subspace(q, PKV_DTYPE_BF16, b, h, n_kv_heads, group, signs,
@@ -119,13 +120,14 @@ int pkv_launch_query_prep_lut(const void *q, int dtype, int bs, int n_kv_heads, 
   return PKV_OK;
 }
 
-// The query side of the retrieval with the dense part of the attention beside it; nothing to clear for the top-k (a top-k that
-// attends has no control area).
+// The query side of the retrieval with the first part of the attention beside it.
 int pkv_launch_query_prep_attend(const pkv_retrieve_args *a, const PkvTiers &tiers, float *qhat, float *qnorm, uint8_t *lut,
-                                 uint32_t *row_suf_to_zero, const PkvSplitAttn &attn, hipStream_t s) {
+                                 uint32_t *row_suf_to_zero, uint32_t *zero_ptr, int64_t zero_words, const PkvSplitAttn &attn,
+                                 hipStream_t s) {
   hipLaunchKernelGGL(pkv_query_prep_attend_kernel, dim3((unsigned)(16 + attn.n_dense), (unsigned)(a->bs * a->n_kv_heads)), dim3(256),
                      0, s, a->q, a->n_kv_heads, a->group, a->signs, a->cluster_counts, qhat, qnorm, (int64_t)a->n_kv_heads * 4096,
-                     (int64_t)4096, tiers, lut, row_suf_to_zero, attn);
+                     (int64_t)4096, tiers, lut, row_suf_to_zero, zero_ptr,
+                     zero_ptr ? zero_words : 0, attn);
   PKV_LAUNCH_CHECK("pkv_query_prep_attend_kernel");
   return PKV_OK;
 }

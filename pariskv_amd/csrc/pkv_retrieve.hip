@@ -17,9 +17,8 @@ PKV_INTERNAL int pkv_launch_qk_norm_rope_table(const void *qkv, int64_t stride_b
                                   const PkvTiers &tiers, float *qhat, float *qnorm, uint8_t *lut, uint32_t *row_suf,
                                   uint32_t *zero_ptr, int64_t zero_words, const pkv_kv_append *append, hipStream_t s);
 PKV_INTERNAL int pkv_launch_query_prep_attend(const pkv_retrieve_args *a, const PkvTiers &tiers, float *qhat, float *qnorm, uint8_t *lut,
-                                              uint32_t *row_suf_to_zero, const PkvSplitAttn &attn, hipStream_t s);
-PKV_INTERNAL int pkv_launch_topk_attend(const float *x, int64_t x_stride, const int64_t *ids, int64_t ids_stride, int rows, int64_t len,
-                                        int64_t k, int64_t *out_ids, float *out_vals, const PkvSplitAttn &attn, hipStream_t s);
+                                              uint32_t *row_suf_to_zero, uint32_t *zero_ptr, int64_t zero_words,
+                                              const PkvSplitAttn &attn, hipStream_t s);
 PKV_INTERNAL size_t pkv_fused_sync_bytes(int rows, int64_t n_chunks);
 PKV_INTERNAL bool pkv_fused_usable(int rows, int64_t n_keys, int chunk_keys, hipStream_t s);
 PKV_INTERNAL int pkv_launch_fused_retrieve(const void *q, int dtype, int bs, int n_kv_heads, int group, const float *signs,
@@ -196,7 +195,7 @@ static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, 
     // table_ready: pkv_qk_norm_rope_table already left the rotated query, its norm and the vote table of these
     // queries in the workspace and cleared what this launch would clear
     rc = a->table_ready           ? PKV_OK
-         : attn && attn->n_dense ? pkv_launch_query_prep_attend(a, t, qhat, qnorm, lut, rowsuf, *attn, s)
+         : attn && attn->n_dense ? pkv_launch_query_prep_attend(a, t, qhat, qnorm, lut, rowsuf, topk_ctl, ctl_words, *attn, s)
                                   : pkv_launch_query_prep_lut(a->q, a->dtype, a->bs, H, a->group, a->signs, a->cluster_counts,
                                                     (int64_t)H * 4096, 4096, t, qhat, qnorm, lut, nullptr, rowsuf, s, topk_ctl,
                                                     ctl_words, dense);
@@ -225,10 +224,8 @@ static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, 
     if (rc) return rc;
   }
   if (!a->out_ids) return PKV_OK;  // candidates only: the caller reads them out of the workspace
-  if (attn)
-    return pkv_launch_topk_attend(scores, a->n_cand, cand, a->n_cand, rows, a->n_cand, a->k, a->out_ids, a->out_scores, *attn, s);
   rc = pkv_launch_topk_f32(scores, a->n_cand, cand, a->n_cand, rows, a->n_cand, a->k, a->out_ids, a->out_scores,
-                           (char *)ws + w.topk, w.topk_bytes, s, a->any_order != 0, topk_ctl != nullptr);
+                           (char *)ws + w.topk, w.topk_bytes, s, a->any_order != 0, topk_ctl != nullptr, attn);
   if (rc) return rc;
   if (a->src_k) {
     PKV_REQUIRE(a->src_v && a->dst_k && a->dst_v, "pkv_retrieve: gather needs src_v, dst_k, dst_v");

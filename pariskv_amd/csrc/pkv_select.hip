@@ -1583,27 +1583,53 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_wide_compact_kernel(
 }
 
 // grid rows; dynamic LDS lds_bytes_sort(P): the winners, and as many keys again for the counting sort when they fit.
-__global__ __launch_bounds__(kTopkThreads) void pkv_topk_wide_finish_kernel(
-    int64_t len, int P, int64_t k, const uint32_t *__restrict__ ctl, const uint64_t *__restrict__ list_a,
-    const uint64_t *__restrict__ list_b, int64_t *__restrict__ out_ids, float *__restrict__ out_vals) {
-  extern __shared__ uint64_t s_keys[];
-  __shared__ SelSmem sm;
+// s_keys: max(P, 1024) keys, and a second copy behind them where P <= kCountingSortMaxP.  out_ids may be null.
+__device__ __forceinline__ void wide_finish(int row, int64_t len, int P, int64_t k, const uint32_t *__restrict__ ctl,
+                                            const uint64_t *__restrict__ list_a, const uint64_t *__restrict__ list_b,
+                                            int64_t *__restrict__ out_ids, float *__restrict__ out_vals, uint64_t *s_keys,
+                                            SelSmem &sm) {
   uint64_t *s_tmp = P <= kCountingSortMaxP ? s_keys + (P < 1024 ? 1024 : P) : nullptr;
-  const int row = blockIdx.x;
   const bool sorted = wide_finish_keys((uint32_t)k, P, ctl + (int64_t)row * kWideRowWords, list_a + (int64_t)row * k,
                                        list_b + (int64_t)row * len, len, s_keys, s_tmp, sm);
-  int64_t *oi = out_ids + (int64_t)row * k;
-  float *ov = out_vals ? out_vals + (int64_t)row * k : nullptr;
   if (!sorted) {
 #define PKV_SORT_K(NT, E) sort_lds_keys_desc<NT, E>(s_keys, (uint32_t)k, s_tmp, sm)
     PKV_DISPATCH_E(P, PKV_SORT_K);
 #undef PKV_SORT_K
   }
+  if (!out_ids) return;
+  int64_t *oi = out_ids + (int64_t)row * k;
+  float *ov = out_vals ? out_vals + (int64_t)row * k : nullptr;
   for (int64_t i = threadIdx.x; i < k; i += kTopkThreads) {
     const uint64_t key = s_keys[i];
     oi[i] = (int64_t)(uint32_t)(~(uint32_t)key);
     if (ov) ov[i] = pkv_from_ordered_u32((uint32_t)(key >> 32));
   }
+}
+
+__global__ __launch_bounds__(kTopkThreads) void pkv_topk_wide_finish_kernel(
+    int64_t len, int P, int64_t k, const uint32_t *__restrict__ ctl, const uint64_t *__restrict__ list_a,
+    const uint64_t *__restrict__ list_b, int64_t *__restrict__ out_ids, float *__restrict__ out_vals) {
+  extern __shared__ uint64_t s_keys[];
+  __shared__ SelSmem sm;
+  wide_finish(blockIdx.x, len, P, k, ctl, list_a, list_b, out_ids, out_vals, s_keys, sm);
+}
+
+// ... and the attention over the winners, merged: see pkv_topk_attend_kernel.  P <= kCountingSortMaxP.
+__global__ __launch_bounds__(kTopkThreads) void pkv_topk_wide_finish_attend_kernel(
+    int64_t len, int P, int64_t k, const uint32_t *__restrict__ ctl, const uint64_t *__restrict__ list_a,
+    const uint64_t *__restrict__ list_b, int64_t *__restrict__ out_ids, float *__restrict__ out_vals, PkvSplitAttn attn) {
+  extern __shared__ uint64_t s_keys[];
+  __shared__ SelSmem sm;
+  __shared__ AttSelSmem sa;
+  const int row = blockIdx.x;
+  AttSelRequests req;
+  att_clear(sa);
+  att_request(attn, row, req);
+  wide_finish(row, len, P, k, ctl, list_a, list_b, out_ids, out_vals, s_keys, sm);
+  uint32_t *s_sel = (uint32_t *)(s_keys + (P < 1024 ? 1024 : P));  // the second copy has done its work
+  for (int i = threadIdx.x; i < (int)k; i += kTopkThreads) s_sel[i] = ~(uint32_t)s_keys[i];
+  __syncthreads();
+  att_selected<true>(attn, row, s_sel, 0, sa, req);
 }
 
 // ------------------------------------------------------------------ adaptive-k
@@ -2367,8 +2393,10 @@ bool pkv_topk_selects(int64_t len, int64_t k) {
   return len <= kTopkMaxSort && pow2_ceil(k) * 2 <= pow2_ceil(len) && pow2_ceil(len) >= 2048;
 }
 
-int pkv_launch_topk_attend(const float *x, int64_t x_stride, const int64_t *ids, int64_t ids_stride, int rows, int64_t len,
-                           int64_t k, int64_t *out_ids, float *out_vals, const PkvSplitAttn &attn, hipStream_t s) {
+bool pkv_topk_attends(int64_t len, int64_t k) { return pkv_topk_selects(len, k) || (len > kTopkMaxSort && pow2_ceil(k) <= kCountingSortMaxP); }
+
+static int launch_topk_attend(const float *x, int64_t x_stride, const int64_t *ids, int64_t ids_stride, int rows, int64_t len,
+                              int64_t k, int64_t *out_ids, float *out_vals, const PkvSplitAttn &attn, hipStream_t s) {
   const int ein = pow2_ceil(len) / kTopkThreads;
 #define PKV_SEL_ATT(EIN, MERGE)                                                                                              \
   hipLaunchKernelGGL((pkv_topk_attend_kernel<EIN, MERGE>), dim3((unsigned)rows, (unsigned)attn.sel_wgs), dim3(kTopkThreads), \
@@ -2388,11 +2416,16 @@ int pkv_launch_topk_attend(const float *x, int64_t x_stride, const int64_t *ids,
 
 int pkv_launch_topk_f32(const float *x, int64_t x_stride, const int64_t *ids, int64_t ids_stride, int rows,
                         int64_t len, int64_t k, int64_t *out_ids, float *out_vals, void *ws, size_t ws_bytes,
-                        hipStream_t s, bool any_order, bool ctl_ready) {
+                        hipStream_t s, bool any_order, bool ctl_ready, const PkvSplitAttn *attn) {
   PKV_REQUIRE(x && out_ids, "pkv_topk_f32: null pointer");
   PKV_REQUIRE(k > 0, "k must be positive");
   PKV_REQUIRE(k <= len, "k cannot exceed sequence length");
   PKV_REQUIRE(rows > 0 && rows <= 65535 && len < ((int64_t)1 << 31), "bad shape rows=%d len=%lld", rows, (long long)len);
+  PKV_REQUIRE(!attn || (pkv_topk_attends(len, k) && (len <= kTopkMaxSort || attn->sel_wgs == 1)),
+              "no attention goes with a top-k of %lld out of %lld", (long long)k, (long long)len);
+  if (attn && pkv_topk_selects(len, k)) {
+    return launch_topk_attend(x, x_stride, ids, ids_stride, rows, len, k, out_ids, out_vals, *attn, s);
+  }
   if (pkv_topk_selects(len, k)) {
     const int P = pow2_ceil(k);
     const int ein = pow2_ceil(len) / kTopkThreads;
@@ -2448,8 +2481,12 @@ int pkv_launch_topk_f32(const float *x, int64_t x_stride, const int64_t *ids, in
     hipLaunchKernelGGL(pkv_topk_wide_compact_kernel, grid, dim3(kTopkThreads), 0, s, x, x_stride, ids, ids_stride, len, k,
                        ctl, list_a, list_b, n_range_slots);
     PKV_LAUNCH_CHECK("pkv_topk_wide_compact_kernel");
-    hipLaunchKernelGGL(pkv_topk_wide_finish_kernel, dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes_sort(P), s, len, P, k,
-                       ctl, list_a, list_b, out_ids, out_vals);
+    if (attn)
+      hipLaunchKernelGGL(pkv_topk_wide_finish_attend_kernel, dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes_sort(P), s, len, P, k,
+                         ctl, list_a, list_b, out_ids, out_vals, *attn);
+    else
+      hipLaunchKernelGGL(pkv_topk_wide_finish_kernel, dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes_sort(P), s, len, P, k,
+                         ctl, list_a, list_b, out_ids, out_vals);
     PKV_LAUNCH_CHECK("pkv_topk_wide_finish_kernel");
   }
   return PKV_OK;

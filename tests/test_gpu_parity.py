@@ -1959,15 +1959,16 @@ def test_prefill_store_index_layouts(ops, dtype, layout, norms, n_enc):
     assert torch.equal(zn, want)
 
 
-@pytest.mark.parametrize("group,k,sink,tail", [
+@pytest.mark.parametrize("group,k,sink,tail,keys,cand", [(*c, 3000, 1500) for c in (
     (4, 100, 64, 529), (1, 1, 0, 1), (3, 15, 3, 0), (5, 16, 64, 64), (8, 17, 64, 1100), (2, 33, 95, 30), (6, 256, 1, 130), (4, 256, 64, 700),
-    (7, 257, 0, 0), (4, 512, 64, 700), (8, 100, 64, 1300), (6, 1024, 64, 1300), (4, 64, 31, 1), (2, 31, 129, 65)])
-def test_decode_step_in_place_attends_in_two_parts(ops, group, k, sink, tail):
+    (7, 257, 0, 0), (4, 512, 64, 700), (8, 100, 64, 1300), (6, 1024, 64, 1300), (4, 64, 31, 1), (2, 31, 129, 65))] + [
+    (4, 100, 64, 529, 20000, 8193), (3, 129, 31, 65, 20000, 9001), (2, 200, 64, 1, 20000, 9001)])
+def test_decode_step_in_place_attends_in_two_parts(ops, group, k, sink, tail, keys, cand):
     """The step whose attention reads selected rows where they lie: the other rows beside the query side, selected rows in the
     top-k's workgroups.  The same ids and the same sums, bit for bit, as the top-k and the attention called one by one; and the
     attention against 64 bits: probabilities and output are rounded to 8 bits, 2^-9 of the largest value each."""
-    _say(f"two-part attention group {group} k {k} sink {sink} tail {tail}")
-    w = W.make_workload("two_parts", 2, 2, group, 3000, 1500, k, O.BF16, 0.5, seed0=11)
+    _say(f"two-part attention group {group} k {k} sink {sink} tail {tail} candidates {cand} of {keys}")
+    w = W.make_workload("two_parts", 2, 2, group, keys, cand, k, O.BF16, 0.5, seed0=11, with_values=False)
     d = W.to_device(w, DEV, torch)
     g = torch.Generator(device=DEV).manual_seed(5)
     rows = sink + w.N + tail
@@ -1975,7 +1976,7 @@ def test_decode_step_in_place_attends_in_two_parts(ops, group, k, sink, tail):
     plan = ops.RetrievePlan(w.bs, w.H, w.G, w.N, DEV, w.N, w.C, w.K)
     att = ops.DecodeAttention(w.bs, w.H, w.G, rows, DEV)
     args = (d["queries"], d["signs"], d["centers"], d["cluster_counts"], d["codes_km"], d["nib_km"], d["w_km"], 0, w.N, w.tiers, w.C, w.K)
-    want_ids = plan.run(*args, any_order=True)
+    want_ids = plan.run(*args, any_order=True)  # more than 8192 candidates come out sorted all the same
     ids = torch.zeros_like(want_ids)
     segs = [s for s in [(kk, vv, 0, sink), (kk, vv, sink, k, ids), (kk, vv, sink + w.N, tail)] if s[3]]
     plan.run(*args, out_ids=ids, attention=(att, segs, None), any_order=True)
