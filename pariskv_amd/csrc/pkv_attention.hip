@@ -67,13 +67,9 @@ __global__ void pkv_attn_merge_kernel(const float *__restrict__ ws, int n_splits
     const bool live = d < n_splits;
     const float *p = rowp + ((int64_t)(live ? d : 0) * G + g) * kPartStride;
     const float mi = live ? p[0] : kNegBig, li = live ? p[1] : 0.f;
-    float mn = mi;
-#pragma unroll
-    for (int x = 1; x < PKV_WAVE; x <<= 1) mn = fmaxf(mn, __shfl_xor(mn, x, PKV_WAVE));
-    const float c = exp2f(mi - mn);
-    float tot = li * c;
-#pragma unroll
-    for (int x = 1; x < PKV_WAVE; x <<= 1) tot += __shfl_xor(tot, x, PKV_WAVE);
+    const float c = exp2f(mi - pkv_wave_max(mi));
+    const float two = fmaf(li, c, pkv_lane_xor_f<1>(li * c));
+    const float tot = pkv_pair_add<32>(pkv_pair_add<16>(pkv_pair_add<8>(pkv_pair_add<4>(pkv_pair_add<2>(two)))));
     s_w[g][d] = c / tot;
   }
   __syncthreads();

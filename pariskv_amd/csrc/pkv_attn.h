@@ -401,8 +401,7 @@ __device__ __forceinline__ void att_step_mfma(const char *kbase, const char *vba
   float mx = sc[0];
 #pragma unroll
   for (int e = 1; e < 8; ++e) mx = fmaxf(mx, sc[e]);
-  mx = fmaxf(mx, __shfl_xor(mx, 16, PKV_WAVE));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, PKV_WAVE));
+  mx = pkv_pair_max<32>(pkv_pair_max<16>(mx));
   const float m_new = fmaxf(m_run, mx);
   // the hardware's exp2: exp2f but for results below 2^-126, which are zero; nothing beside the largest weight, which is 1
   const float corr = __builtin_amdgcn_exp2f(m_run - m_new);
@@ -516,8 +515,7 @@ __device__ __forceinline__ void att_partial_mfma(const void *__restrict__ q, int
     att_step_mfma<ONE, false>(kbase, vbase, mine, in_block, jb, j1, qb, scale_log2e, m_run, l_part, o);
   }
 
-  l_part += __shfl_xor(l_part, 16, PKV_WAVE);
-  l_part += __shfl_xor(l_part, 32, PKV_WAVE);
+  l_part = pkv_pair_add<32>(pkv_pair_add<16>(l_part));
   float *part = ws + ((int64_t)row * n_splits + split) * group * kPartStride;
   att_merge_waves(group, m_run, l_part, o, part, kPartStride, part + 2, kPartStride);
 }
@@ -590,8 +588,7 @@ __device__ __forceinline__ void att_dense_part(const PkvSplitAttn &a, int x, int
     att_load_q(a, row, qb);
     att_step_mfma<true, true>(a.segs.k + slab, a.segs.v + slab, mine, 0, j0, j1, qb, a.scale_log2e, m_run, l_part, o);
   }
-  l_part += pkv_lane_xor_f<16>(l_part);
-  l_part += pkv_lane_xor_f<32>(l_part);
+  l_part = pkv_pair_add<32>(pkv_pair_add<16>(l_part));
   if (!mixed) {
     if (a.sel_wgs == 1) {
       att_merge_waves(a.group, m_run, l_part, o, att_slot_ml(a, row, split, 0), 2 * kSelSlots, att_slot_o(a, row, split, 0), 128);
@@ -679,8 +676,7 @@ __device__ __forceinline__ void att_selected(const PkvSplitAttn &a, int row, con
     float m_run = kNegBig, l_part = 0.f;
     pkv_f32x4 o[8];
     att_step_mfma<true, true>(a.segs.k + slab, a.segs.v + slab, mine, 0, j0, j1, qb, a.scale_log2e, m_run, l_part, o);
-    l_part += pkv_lane_xor_f<16>(l_part);
-    l_part += pkv_lane_xor_f<32>(l_part);
+    l_part = pkv_pair_add<32>(pkv_pair_add<16>(l_part));
     if (lane < a.group) sm.m[n][local] = m_run, sm.l[n][local] = l_part;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -732,15 +728,9 @@ __device__ __forceinline__ void att_selected(const PkvSplitAttn &a, int row, con
     const float ls = fmaf(lw.w, cw[3], fmaf(lw.z, cw[2], fmaf(lw.y, cw[1], lw.x * cw[0])));
     const bool split_lane = lane < kSelSplits;  // the lanes behind hold single blocks
     const float mi = own ? mx : split_lane ? req.ml.x : kNegBig, li = own ? ls : split_lane ? req.ml.y : 0.f;
-    float mn = mi;
-#define PKV_ATT_MAX(M) mn = fmaxf(mn, pkv_lane_xor_f<M>(mn));
-    PKV_ATT_MAX(1) PKV_ATT_MAX(2) PKV_ATT_MAX(4) PKV_ATT_MAX(8) PKV_ATT_MAX(16) PKV_ATT_MAX(32)
-#undef PKV_ATT_MAX
-    const float c = exp2f(mi - mn);
-    float tot = fmaf(li, c, pkv_lane_xor_f<1>(li * c));
-#define PKV_ATT_ADD(M) tot += pkv_lane_xor_f<M>(tot);
-    PKV_ATT_ADD(2) PKV_ATT_ADD(4) PKV_ATT_ADD(8) PKV_ATT_ADD(16) PKV_ATT_ADD(32)
-#undef PKV_ATT_ADD
+    const float c = exp2f(mi - pkv_wave_max(mi));
+    const float two = fmaf(li, c, pkv_lane_xor_f<1>(li * c));  // the order, and the fused first step, of the merge kernel
+    const float tot = pkv_pair_add<32>(pkv_pair_add<16>(pkv_pair_add<8>(pkv_pair_add<4>(pkv_pair_add<2>(two)))));
     const float weight = c / tot;
     float os = 0.f;
 #pragma unroll

@@ -213,6 +213,48 @@ __device__ __forceinline__ uint64_t pkv_lane_xor64(uint64_t v) {
   return ((uint64_t)pkv_lane_xor<M>((uint32_t)(v >> 32)) << 32) | pkv_lane_xor<M>((uint32_t)v);
 }
 
+// The values of lane i and lane i ^ M, for an operation that does not mind their order: M = 16 and 32 by the instructions that
+// swap rows between two registers, without the LDS crossbar of a shuffle (some 60 cycles, six in a chain to reduce a wave).
+// All 64 lanes must be active.  Steps reduced with shuffles / like this, us: adaptive k, 24 rows x 41003 keys (2 layers) 93.2 / 91.3,
+// 8 x 1M keys 156.9 / 155.5; 8 x 9000 keys, top 100, 25.1 / 24.4.
+template <int M>
+__device__ __forceinline__ void pkv_lane_pair(uint32_t v, uint32_t &a, uint32_t &b) {
+  if constexpr (M == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    a = r[0], b = r[1];
+  } else if constexpr (M == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    a = r[0], b = r[1];
+  } else {
+    a = v, b = pkv_lane_xor<M>(v);
+  }
+}
+template <int M>
+__device__ __forceinline__ float pkv_pair_add(float v) {
+  uint32_t a, b;
+  pkv_lane_pair<M>(__float_as_uint(v), a, b);
+  return __uint_as_float(a) + __uint_as_float(b);
+}
+template <int M>
+__device__ __forceinline__ float pkv_pair_max(float v) {
+  uint32_t a, b;
+  pkv_lane_pair<M>(__float_as_uint(v), a, b);
+  return fmaxf(__uint_as_float(a), __uint_as_float(b));
+}
+template <int M>
+__device__ __forceinline__ uint32_t pkv_pair_max(uint32_t v) {
+  uint32_t a, b;
+  pkv_lane_pair<M>(v, a, b);
+  return a > b ? a : b;
+}
+// Over each 16 lanes, then over the wave, in the order of the butterfly with distances 1, 2, 4, ...
+__device__ __forceinline__ float pkv_row_sum(float v) { return pkv_pair_add<8>(pkv_pair_add<4>(pkv_pair_add<2>(pkv_pair_add<1>(v)))); }
+__device__ __forceinline__ float pkv_wave_sum(float v) { return pkv_pair_add<32>(pkv_pair_add<16>(pkv_row_sum(v))); }
+template <typename T>
+__device__ __forceinline__ T pkv_row_max(T v) { return pkv_pair_max<8>(pkv_pair_max<4>(pkv_pair_max<2>(pkv_pair_max<1>(v)))); }
+template <typename T>
+__device__ __forceinline__ T pkv_wave_max(T v) { return pkv_pair_max<32>(pkv_pair_max<16>(pkv_row_max(v))); }
+
 // Inclusive scan over the 64 lanes of a wave: four row_shr steps inside each row of 16 lanes, then the
 // row totals travel with row_bcast:15 (rows 1, 3) and row_bcast:31 (rows 2, 3).
 __device__ __forceinline__ int pkv_wave_incl_scan(int v) {

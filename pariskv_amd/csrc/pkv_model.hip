@@ -15,8 +15,7 @@ __device__ __forceinline__ void qk_norm_rope_head(float x1, float x2, const uint
                                                   float s, float &y1, float &y2) {
   const int lane = pkv_lane();
   float ss = x1 * x1 + x2 * x2;
-#pragma unroll
-  for (int m = 1; m < PKV_WAVE; m <<= 1) ss += __shfl_xor(ss, m, PKV_WAVE);
+  ss = pkv_wave_sum(ss);
   const float inv = 1.0f / sqrtf(ss * (1.0f / 128.0f) + eps);
   if (w) {
     x1 = x1 * inv * pkv_bf16_bits_to_f32(w[lane]);
@@ -176,8 +175,7 @@ __global__ __launch_bounds__(256) void pkv_add_rmsnorm_kernel(const uint16_t *__
       if (out_sum) *(pkv_u32x4 *)(out_sum + (int64_t)row * width + vec * 8) = pkv_u32x4{ow[0], ow[1], ow[2], ow[3]};
     }
   }
-#pragma unroll
-  for (int m = 1; m < PKV_WAVE; m <<= 1) ss += __shfl_xor(ss, m, PKV_WAVE);
+  ss = pkv_wave_sum(ss);
   if (pkv_lane() == 0) s_part[tid / PKV_WAVE] = ss;
   __syncthreads();
   const float inv = 1.0f / sqrtf((s_part[0] + s_part[1] + s_part[2] + s_part[3]) / (float)width + eps);

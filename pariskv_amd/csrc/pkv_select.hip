@@ -212,12 +212,7 @@ __global__ __launch_bounds__(kSelThreads) void pkv_select_rerank_kernel(
   // slots with atomicMax from zero (one address per row would serialise the atomics of hundreds of workgroups:
   // measured +15 us at 8 rows x 256 chunks; a slot per workgroup costs the readers 3 us of loads)
   if (range_slots) {
-#pragma unroll
-    for (int x = 1; x < PKV_WAVE; x <<= 1) {
-      const uint32_t a = (uint32_t)__shfl_xor((int)smax, x, PKV_WAVE), c = (uint32_t)__shfl_xor((int)smin, x, PKV_WAVE);
-      smax = a > smax ? a : smax;
-      smin = c < smin ? c : smin;
-    }
+    smax = pkv_wave_max(smax), smin = ~pkv_wave_max(~smin);
     if (pkv_lane() == 0) s_scan[0][tid / PKV_WAVE] = (int)smax, s_scan[1][tid / PKV_WAVE] = (int)smin;
     __syncthreads();
     if (tid == 0) {
@@ -383,12 +378,7 @@ __global__ __launch_bounds__(kSelThreads) void pkv_select_rerank_pieces_kernel(
     __syncthreads();  // the list is rewritten by the next pass
   }
   if (range_slots) {
-#pragma unroll
-    for (int x = 1; x < PKV_WAVE; x <<= 1) {
-      const uint32_t a = (uint32_t)__shfl_xor((int)smax, x, PKV_WAVE), c = (uint32_t)__shfl_xor((int)smin, x, PKV_WAVE);
-      smax = a > smax ? a : smax;
-      smin = c < smin ? c : smin;
-    }
+    smax = pkv_wave_max(smax), smin = ~pkv_wave_max(~smin);
     if (pkv_lane() == 0) s_scan[0][tid / PKV_WAVE] = (int)smax, s_scan[1][tid / PKV_WAVE] = (int)smin;
     __syncthreads();
     if (tid == 0) {
@@ -780,14 +770,7 @@ __device__ __forceinline__ bool linear_bins(const uint64_t (&v)[EIN], uint32_t k
       mn = hi < mn ? hi : mn;
     }
   }
-#define PKV_LIN_RED(M)                              \
-  {                                                 \
-    const uint32_t a = pkv_lane_xor<M>(mx), c = pkv_lane_xor<M>(mn); \
-    mx = a > mx ? a : mx;                           \
-    mn = c < mn ? c : mn;                           \
-  }
-  PKV_LIN_RED(1) PKV_LIN_RED(2) PKV_LIN_RED(4) PKV_LIN_RED(8) PKV_LIN_RED(16) PKV_LIN_RED(32)
-#undef PKV_LIN_RED
+  mx = pkv_wave_max(mx), mn = ~pkv_wave_max(~mn);
   if (lane == 0) {
     atomicMax(&s_bcast[0], mx);
     atomicMin(&s_bcast[1], mn);
@@ -1317,12 +1300,7 @@ __device__ __forceinline__ WideBinning wide_binning(const uint32_t *__restrict__
       mx = sl.x > mx ? sl.x : mx;
       mi = sl.y > mi ? sl.y : mi;
     }
-#pragma unroll
-    for (int x = 1; x < PKV_WAVE; x <<= 1) {
-      const uint32_t a = (uint32_t)__shfl_xor((int)mx, x, PKV_WAVE), c = (uint32_t)__shfl_xor((int)mi, x, PKV_WAVE);
-      mx = a > mx ? a : mx;
-      mi = c > mi ? c : mi;
-    }
+    mx = pkv_wave_max(mx), mi = pkv_wave_max(mi);
   }
   const uint32_t mn = ~mi;
   const float hi = pkv_from_ordered_u32(mx), lo = pkv_from_ordered_u32(mn);
@@ -1504,12 +1482,7 @@ __device__ __forceinline__ bool wide_finish_keys(uint32_t k, int P, const uint32
 // range slot, written plainly, no matter what it held.  s_red: 32 words.  All threads of the workgroup.
 __device__ __forceinline__ void wide_range_out(uint32_t mx, uint32_t mn, uint32_t *__restrict__ rctl, int slot,
                                                uint32_t *s_red) {
-#pragma unroll
-  for (int x = 1; x < PKV_WAVE; x <<= 1) {
-    const uint32_t a = (uint32_t)__shfl_xor((int)mx, x, PKV_WAVE), c = (uint32_t)__shfl_xor((int)mn, x, PKV_WAVE);
-    mx = a > mx ? a : mx;
-    mn = c < mn ? c : mn;
-  }
+  mx = pkv_wave_max(mx), mn = ~pkv_wave_max(~mn);
   const int wave = threadIdx.x / PKV_WAVE, n_waves = (blockDim.x + PKV_WAVE - 1) / PKV_WAVE;
   if (pkv_lane() == 0) s_red[wave] = mx, s_red[16 + wave] = mn;
   __syncthreads();
@@ -1662,31 +1635,19 @@ __device__ __forceinline__ float pkv_expf(float x) {
 // Sum over the workgroup's 1024 lanes as a pairwise tree (stride 1, 2, 4, ...): xor butterflies
 // inside each wave, then the 16 wave sums.  Every thread returns the same value.
 __device__ __forceinline__ float block_tree_sum_1024(float v, float *s_part) {
-#pragma unroll
-  for (int m = 1; m < PKV_WAVE; m <<= 1) v = v + __shfl_xor(v, m, PKV_WAVE);
+  v = pkv_wave_sum(v);
   __syncthreads();
   if (pkv_lane() == 0) s_part[threadIdx.x / PKV_WAVE] = v;
   __syncthreads();
-  float w[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) w[i] = s_part[i];
-#pragma unroll
-  for (int h = 1; h < 16; h <<= 1)
-#pragma unroll
-    for (int i = 0; i < 16; i += 2 * h) w[i] = w[i] + w[i + h];
-  return w[0];
+  return pkv_row_sum(s_part[threadIdx.x & 15]);  // the wave sums, one to a lane
 }
 
 __device__ __forceinline__ float block_max_1024(float v, float *s_part) {
-#pragma unroll
-  for (int m = 1; m < PKV_WAVE; m <<= 1) v = fmaxf(v, __shfl_xor(v, m, PKV_WAVE));
+  v = pkv_wave_max(v);
   __syncthreads();
   if (pkv_lane() == 0) s_part[threadIdx.x / PKV_WAVE] = v;
   __syncthreads();
-  float r = s_part[0];
-#pragma unroll
-  for (int i = 1; i < 16; ++i) r = fmaxf(r, s_part[i]);
-  return r;
+  return pkv_row_max(s_part[threadIdx.x & 15]);
 }
 
 // Two sums, each in the order of block_tree_sum_1024, and the largest / smallest of two unsigned words, all in one
@@ -1696,34 +1657,16 @@ struct AdkReduced {
   uint32_t mx, mn;
 };
 __device__ __forceinline__ AdkReduced block_reduce_adk_1024(float a, float b, uint32_t mx, uint32_t mn, uint32_t *s_red) {
-#pragma unroll
-  for (int m = 1; m < PKV_WAVE; m <<= 1) {
-    const float oa = __shfl_xor(a, m, PKV_WAVE), ob = __shfl_xor(b, m, PKV_WAVE);
-    const uint32_t ox = (uint32_t)__shfl_xor((int)mx, m, PKV_WAVE), on = (uint32_t)__shfl_xor((int)mn, m, PKV_WAVE);
-    a = a + oa, b = b + ob;
-    mx = ox > mx ? ox : mx, mn = on < mn ? on : mn;
-  }
+  a = pkv_wave_sum(a), b = pkv_wave_sum(b), mx = pkv_wave_max(mx), mn = ~pkv_wave_max(~mn);
   __syncthreads();
   if (pkv_lane() == 0) {
     const int w = threadIdx.x / PKV_WAVE;
     s_red[w] = __float_as_uint(a), s_red[16 + w] = __float_as_uint(b), s_red[32 + w] = mx, s_red[48 + w] = mn;
   }
   __syncthreads();
-  float wa[16], wb[16];
-  AdkReduced r;
-  r.mx = 0u, r.mn = 0xffffffffu;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    wa[i] = __uint_as_float(s_red[i]), wb[i] = __uint_as_float(s_red[16 + i]);
-    r.mx = s_red[32 + i] > r.mx ? s_red[32 + i] : r.mx;
-    r.mn = s_red[48 + i] < r.mn ? s_red[48 + i] : r.mn;
-  }
-#pragma unroll
-  for (int h = 1; h < 16; h <<= 1)
-#pragma unroll
-    for (int i = 0; i < 16; i += 2 * h) wa[i] = wa[i] + wa[i + h], wb[i] = wb[i] + wb[i + h];
-  r.sum_a = wa[0], r.sum_b = wb[0];
-  return r;
+  const int w = threadIdx.x & 15;
+  return {pkv_row_sum(__uint_as_float(s_red[w])), pkv_row_sum(__uint_as_float(s_red[16 + w])), pkv_row_max(s_red[32 + w]),
+          ~pkv_row_max(~s_red[48 + w])};
 }
 
 __device__ __forceinline__ float cand_logit(const void *__restrict__ scores, int dtype, float scale, int64_t i) {
@@ -2085,8 +2028,7 @@ __global__ __launch_bounds__(kAdkPartThreads) void pkv_adk_max_gather_kernel(
     for (int64_t i = tid; i < sl; i += kAdkPartThreads) m = fmaxf(m, sll[i]);
     for (int i = tid; i < kWideRowWords; i += kAdkPartThreads) ctl[(int64_t)row * kWideRowWords + i] = 0;
   }
-#pragma unroll
-  for (int x = 1; x < PKV_WAVE; x <<= 1) m = fmaxf(m, __shfl_xor(m, x, PKV_WAVE));
+  m = pkv_wave_max(m);
   if (pkv_lane() == 0) s_part[tid / PKV_WAVE] = m;
   __syncthreads();
   if (tid == 0) {
@@ -2112,8 +2054,7 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_adk_benefit_kernel(
   float *ben = ws_ben + (int64_t)row * n_cand;
   float g = -__uint_as_float(0x7f800000u);
   for (int w = tid & (PKV_WAVE - 1); w < n_parts; w += PKV_WAVE) g = fmaxf(g, ws_max[(int64_t)row * n_parts + w]);
-#pragma unroll
-  for (int x = 1; x < PKV_WAVE; x <<= 1) g = fmaxf(g, __shfl_xor(g, x, PKV_WAVE));
+  g = pkv_wave_max(g);
   if (slice == n_slices) {  // the row's last workgroup: the dense tokens' benefit, kept after the slice sums
     const float d = dense_benefit_sum(sl_logits + (int64_t)row * sl_stride, sl_vnorm + (int64_t)row * slv_stride, sl, g,
                                       s_part);
