@@ -631,7 +631,11 @@ int pkv_retrieve_noalloc(const pkv_retrieve_args *args, void *stream);
  * gather) followed by pkv_decode_attention over the attended set, on the same
  * stream - polar_cache.compute (cache_hub/polar_cache.py:1002-1107) after the
  * dense-fallback test.  Queries, dtype and head counts are taken from
- * `retrieve`; the segments normally include the rows the gather just wrote. */
+ * `retrieve`; the segments normally include the rows the gather just wrote.
+ * Where a bf16 step gathers nothing and one segment reads the selected rows
+ * through `retrieve`'s out_ids (any_order, PKV_PLAN_SEPARATE, no table_ready),
+ * the attention may ride in the query-prep and top-k launches: the same
+ * results, bit for bit, and other contents of `ws`. */
 typedef struct pkv_attn_args {
   pkv_attn_segment segments[PKV_ATTN_MAX_SEGMENTS];
   int n_segments;

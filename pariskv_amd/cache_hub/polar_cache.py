@@ -7,7 +7,7 @@ under ``attn_hub/polar_attn.py``.  What differs inside:
 
 * metadata is stored key-major (``ops.alloc_keymajor``); ``codebook_gpu``,
   ``key_4bit_packed_gpu`` and ``key_block_weight_gpu`` are reference-shaped views of it;
-* one decode step's retrieval is a single ``pkv_retrieve`` call (6 launches) that
+* one decode step's retrieval is a single ``pkv_retrieve`` call that
   also gathers the selected K/V rows straight behind the dense prefix, so no
   ``torch.cat`` / ``torch.gather`` of K/V happens per step;
 * zone counters are per layer (see ``zones.py``);

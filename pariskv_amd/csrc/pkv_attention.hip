@@ -10,7 +10,7 @@
 // all G query heads.  Split over the key axis (flash-decoding): grid (n_splits, R);
 // every split keeps a running (max, sum, output) per query head and the partial
 // results are merged by a second small launch.
-//   bf16: four waves per split on the matrix cores (v_mfma_f32_16x16x32_bf16), merged through LDS, see below.
+//   bf16: four waves per split on the matrix cores (v_mfma_f32_16x16x32_bf16), merged through LDS, see pkv_attn.h.
 //   fp32: 256 threads per split, every 16 lanes own one key at a time (a wave
 //         instruction moves four whole rows), fp32 FMA and lane-exchange reductions.
 //

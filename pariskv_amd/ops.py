@@ -854,7 +854,7 @@ class BoundAttention:
 class BoundStep:
     """The argument blocks of one layer's pkv_decode_step, validated once.  A launch patches only what moves with
     every token: the query and output pointers and, through ``a`` / ``segs``, the caller's row counts.  Filling and
-    checking the blocks costs more host time than the seven launches themselves, which matters when the K/V live in
+    checking the blocks costs more host time than the launches themselves, which matters when the K/V live in
     HBM and the GPU side of a step is a few tens of microseconds."""
 
     __slots__ = ("a", "aa", "segs", "keep", "_ra", "_raa", "_ws", "_ws_bytes", "_fn", "_numel", "_dtype")
