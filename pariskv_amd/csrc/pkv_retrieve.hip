@@ -3,7 +3,8 @@
 // histograms) -> candidate select fused with the 4-bit rerank -> exact top-k ->
 // optional gather of the selected K/V rows (5 launches).  With the attention
 // of the whole step in the same call its parts may ride in the first and the
-// top-k's launch (pkv_attn.h).  The adaptive-k step replaces the exact top-k by the dense logits and the adaptive selection.
+// top-k's launch (pkv_attn.h).  The adaptive-k step replaces the exact top-k by
+// the dense logits and the adaptive selection.
 //
 // Reference: cache_hub/polar_cache.py:1126-1162 (collision_based_topk_batch),
 // :1207-1231, :1244-1304 and the gather at :1075-1095.
