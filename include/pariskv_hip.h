@@ -635,7 +635,9 @@ int pkv_retrieve_noalloc(const pkv_retrieve_args *args, void *stream);
  * Where a bf16 step gathers nothing and one segment reads the selected rows
  * through `retrieve`'s out_ids (any_order, PKV_PLAN_SEPARATE, no table_ready),
  * the attention may ride in the query-prep and top-k launches: the same
- * results, bit for bit, and other contents of `ws`. */
+ * results, bit for bit, and other contents of `ws`.  Buffers may be shared as
+ * the order of the two calls allows (attention->ws inside `ws`, an output over
+ * the queries or the workspace): the attention then waits for the retrieval. */
 typedef struct pkv_attn_args {
   pkv_attn_segment segments[PKV_ATTN_MAX_SEGMENTS];
   int n_segments;
@@ -653,6 +655,11 @@ int pkv_decode_attention_run(const void *q, int dtype, int bs, int n_kv_heads, i
 
 int pkv_decode_step(const pkv_retrieve_args *retrieve, void *ws, size_t ws_bytes,
                     const pkv_attn_args *attention, void *stream);
+
+/* How pkv_decode_step takes these arguments (host code, nothing is launched; no counterpart in the reference): 0 = the
+ * retrieval, then the attention; 1 = the attention in two parts, the second by the top-k's one workgroup a row; 2 = by
+ * several workgroups a row and a merge launch. */
+int pkv_decode_step_form(const pkv_retrieve_args *retrieve, const void *ws, const pkv_attn_args *attention);
 
 /* The adaptive-k decode step of one layer from one host call
  * (cache_hub/polar_cache_adaptivek_varlen.py:1391-1677 after the dense-fallback

@@ -166,6 +166,7 @@ PROTOTYPES = {
     "pkv_retrieve_noalloc_prepare": (_i, []),
     "pkv_retrieve_noalloc": (_i, [C.POINTER(RetrieveArgs), _vp]),
     "pkv_decode_step": (_i, [C.POINTER(RetrieveArgs), _vp, _sz, C.POINTER(AttnArgs), _vp]),
+    "pkv_decode_step_form": (_i, [C.POINTER(RetrieveArgs), _vp, C.POINTER(AttnArgs)]),
     "pkv_adaptive_decode_step": (_i, [C.POINTER(RetrieveArgs), _vp, _sz, C.POINTER(AdaptiveArgs), C.POINTER(AttnArgs), _vp]),
     "pkv_retrieve_ws_view": (_i, [_vp, _i, _i64, _i64, _i64, C.c_char_p, C.POINTER(_vp), C.POINTER(_sz)]),
 }

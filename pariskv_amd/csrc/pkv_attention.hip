@@ -275,7 +275,11 @@ extern "C" int pkv_decode_attention_run(const void *q, int dtype, int bs, int n_
                           a->row_keys_uniform ? bs * n_kv_heads : 0, a->scale, a->out, a->ws, a->ws_bytes, stream);
 }
 
-bool pkv_plan_split_attention(const pkv_retrieve_args *r, const pkv_attn_args *at, PkvSplitAttn *out) {
+static bool meets(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+  return a && b && (uintptr_t)a < (uintptr_t)b + b_bytes && (uintptr_t)b < (uintptr_t)a + a_bytes;
+}
+
+bool pkv_plan_split_attention(const pkv_retrieve_args *r, const void *ws, const pkv_attn_args *at, PkvSplitAttn *out) {
   // What the general path would refuse is left to it.
   if (r->dtype != PKV_DTYPE_BF16 || !r->q || !pkv_aligned(r->q, 16) || !at->out || !pkv_aligned(at->out, 4) || !at->ws ||
       !pkv_aligned(at->ws, 16) || r->bs <= 0 || r->n_kv_heads <= 0 || (int64_t)r->bs * r->n_kv_heads > 65535 || r->group < 1 ||
@@ -335,7 +339,18 @@ bool pkv_plan_split_attention(const pkv_retrieve_args *r, const pkv_attn_args *a
   out->n_dense = out->n_splits - out->dense_skip;
   const size_t row_floats = out->sel_wgs == 1 ? (size_t)20 * r->group * 128 + (size_t)r->group * kSelSlots * 2
                                               : (size_t)out->n_splits * r->group * kPartStride;
-  if (at->ws_bytes < (size_t)rows * row_floats * sizeof(float)) return false;
+  const size_t at_bytes = (size_t)rows * row_floats * sizeof(float), out_bytes = (size_t)rows * r->group * 256;
+  if (at->ws_bytes < at_bytes) return false;
+  // Partial results and output are written while the retrieval still works, not after it: where they would lie in its workspace,
+  // queries or results, the attention waits.  (An output in place of the queries is fine: a row's are read before it is written.)
+  const size_t r_bytes = pkv_retrieve_ws_bytes(rows, r->n_keys, r->n_cand, r->k);
+  const struct {
+    const void *p;
+    size_t n;
+  } busy[] = {{ws, r_bytes}, {r->out_ids, (size_t)rows * r->k * 8}, {r->out_scores, (size_t)rows * r->k * 4}, {r->q, out_bytes}};
+  for (const auto &u : busy)
+    if (meets(at->ws, at_bytes, u.p, u.n) || (meets(at->out, out_bytes, u.p, u.n) && !(u.p == r->q && at->out == r->q))) return false;
+  if (meets(at->out, out_bytes, at->ws, at_bytes)) return false;
   out->n_kv_heads = r->n_kv_heads, out->group = r->group, out->q = r->q;
   out->scale_log2e = at->scale * 1.4426950408889634f;
   out->ws = (float *)at->ws, out->out = at->out;

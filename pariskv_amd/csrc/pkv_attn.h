@@ -752,7 +752,8 @@ __device__ __forceinline__ void att_selected(const PkvSplitAttn &a, int row, con
 
 // The merge of a row's splits (where sel_wgs > 1).
 PKV_INTERNAL int pkv_launch_attn_merge(const PkvSplitAttn &a, int rows, hipStream_t s);
-// Whether pkv_decode_step's attention over `attn` can be taken in two parts around a top-k of k ids into out_ids; fills `out`.
-PKV_INTERNAL bool pkv_plan_split_attention(const pkv_retrieve_args *r, const pkv_attn_args *attn, PkvSplitAttn *out);
+// Whether pkv_decode_step's attention over `attn` can be taken in two parts around a top-k of k ids into out_ids, the retrieval
+// working in `ws`; fills `out`.
+PKV_INTERNAL bool pkv_plan_split_attention(const pkv_retrieve_args *r, const void *ws, const pkv_attn_args *attn, PkvSplitAttn *out);
 
 #endif  // __HIPCC__

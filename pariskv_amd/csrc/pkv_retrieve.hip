@@ -361,11 +361,17 @@ extern "C" int pkv_decode_step(const pkv_retrieve_args *retrieve, void *ws, size
                                const pkv_attn_args *attention, void *stream) {
   PKV_REQUIRE(retrieve && attention, "pkv_decode_step: null args");
   PkvSplitAttn split;
-  if (pkv_plan_split_attention(retrieve, attention, &split)) return retrieve_impl(retrieve, ws, ws_bytes, stream, nullptr, 256, &split);
+  if (pkv_plan_split_attention(retrieve, ws, attention, &split)) return retrieve_impl(retrieve, ws, ws_bytes, stream, nullptr, 256, &split);
   int rc = pkv_retrieve(retrieve, ws, ws_bytes, stream);
   if (rc) return rc;
   return pkv_decode_attention_run(retrieve->q, retrieve->dtype, retrieve->bs, retrieve->n_kv_heads, retrieve->group, attention,
                                   stream);
+}
+
+extern "C" int pkv_decode_step_form(const pkv_retrieve_args *retrieve, const void *ws, const pkv_attn_args *attention) {
+  PKV_REQUIRE(retrieve && attention, "pkv_decode_step_form: null args");
+  PkvSplitAttn split;
+  return pkv_plan_split_attention(retrieve, ws, attention, &split) ? (split.sel_wgs == 1 ? 1 : 2) : 0;
 }
 
 extern "C" int pkv_adaptive_decode_step(const pkv_retrieve_args *retrieve, void *ws, size_t ws_bytes,

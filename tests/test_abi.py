@@ -216,3 +216,57 @@ def test_one_chunk_rule():
             _lib.check(L.pkv_retrieve_ws_view(256, rows, n, n, 1, b"chunk_suffix_hist", ctypes.byref(ptr), ctypes.byref(nbytes)))
             pieces = 4 if chunk >= 8192 and 4 * n_chunks <= 512 else 1
             assert nbytes.value == rows * n_chunks * pieces * 256, (rows, n, chunk)
+
+
+def _in_place_step(bs=1, H=8, group=4, n_keys=4096, n_cand=1500, k=100, sink=64, tail=529):
+    """Argument blocks of a bf16 decode step that attends to the selected rows in place, with buffers side by side at made-up
+    addresses: (retrieve, retrieval workspace and its bytes, attention)."""
+    from pariskv_amd import _lib
+
+    L = _lib.lib()
+    a, aa, at = _lib.RetrieveArgs(), _lib.AttnArgs(), 1 << 32
+
+    def take(nbytes):
+        nonlocal at
+        p, at = at, at + (nbytes + 255) // 256 * 256
+        return p
+
+    rows = bs * H
+    a.dtype, a.bs, a.n_kv_heads, a.group, a.cap, a.n_keys, a.n_cand, a.k = _lib.DTYPE_BF16, bs, H, group, n_keys, n_keys, n_cand, k
+    a.any_order, a.n_tiers = 1, 6
+    a.q, a.out_ids, a.out_scores = take(rows * group * 256), take(rows * k * 8), take(rows * k * 4)
+    ws_bytes = L.pkv_retrieve_ws_bytes(rows, n_keys, n_cand, k)
+    ws = take(ws_bytes)
+    total = sink + n_keys + tail
+    K, V = take(rows * total * 256), take(rows * total * 256)
+    for i, (row0, n, idx) in enumerate([(0, sink, 0), (sink, k, a.out_ids), (sink + n_keys, tail, 0)]):
+        aa.segments[i] = _lib.AttnSegment(K, V, H * total * 128, total * 128, row0, n, idx or None, k if idx else 0, n_keys if idx else 0)
+    aa.n_segments, aa.scale, aa.out = 3, 0.1, take(rows * group * 256)
+    aa.ws_bytes = L.pkv_decode_attention_ws_bytes(bs, H, group, sink + k + tail)
+    aa.ws = take(aa.ws_bytes)
+    return a, ws, ws_bytes, aa
+
+
+def test_decode_step_waits_where_buffers_are_shared():
+    """pkv_decode_step is the retrieval followed by the attention: scratch memory, queries and results may be shared as that order
+    allows.  The attention in two parts writes while the retrieval still works, so it is not taken there."""
+    from pariskv_amd import _lib
+
+    form = _lib.lib().pkv_decode_step_form
+    for shape in ({}, dict(k=512), dict(n_keys=100000, n_cand=10000)):
+        a, ws, ws_bytes, aa = _in_place_step(**shape)
+        apart, at_ws, out = form(a, ws, aa), aa.ws, aa.out
+        assert apart == (2 if shape.get("k") == 512 else 1)
+        for p in (ws, ws + 256, ws + ws_bytes - 256, ws - 256, a.out_ids, a.out_scores, a.q):
+            aa.ws = p
+            assert form(a, ws, aa) == 0, (shape, p)
+        aa.ws = at_ws
+        for p in (ws, ws + ws_bytes - 256, a.out_ids, a.out_scores, a.q + 256, at_ws):
+            aa.out = p
+            assert form(a, ws, aa) == 0, (shape, p)
+        aa.out = a.q  # in place of the queries: row by row
+        assert form(a, ws, aa) == apart
+        aa.out = out
+        aa.ws = ws + ws_bytes  # right behind it
+        assert form(a, ws, aa) == apart
+        assert form(a, at_ws + aa.ws_bytes, aa) == apart

@@ -1991,3 +1991,33 @@ def test_decode_step_in_place_attends_in_two_parts(ops, group, k, sink, tail, ke
     want = torch.softmax(q @ ks.transpose(2, 3) / 128 ** 0.5, dim=-1) @ vs
     err = (got.view(w.bs, w.H, group, 128).double().cpu() - want).abs().max().item()
     assert err <= vv.abs().max().item() * 2.0 ** -8, err
+
+
+@pytest.mark.parametrize("k,keys,cand", [(100, 3000, 1500), (512, 3000, 1500), (100, 20000, 9001)])
+def test_decode_step_with_one_scratch_buffer(ops, k, keys, cand):
+    """Retrieval and attention with the same scratch memory, and with the output over the queries: as with buffers of their own."""
+    _say(f"decode step in one scratch buffer, k {k} candidates {cand} of {keys}")
+    w = W.make_workload("one_scratch", 2, 2, 4, keys, cand, k, O.BF16, 0.5, seed0=12, with_values=False)
+    d = W.to_device(w, DEV, torch)
+    g = torch.Generator(device=DEV).manual_seed(6)
+    rows = 64 + w.N + 529
+    kk, vv = (torch.randn(w.bs, w.H, rows, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    plan = ops.RetrievePlan(w.bs, w.H, w.G, w.N, DEV, w.N, w.C, w.K)
+    att = ops.DecodeAttention(w.bs, w.H, w.G, rows, DEV)
+
+    def step(q, out=None):
+        ids = torch.zeros(w.bs, w.H, k, dtype=torch.int64, device=DEV)
+        segs = [(kk, vv, 0, 64), (kk, vv, 64, k, ids), (kk, vv, 64 + w.N, 529)]
+        plan.run(q, d["signs"], d["centers"], d["cluster_counts"], d["codes_km"], d["nib_km"], d["w_km"], 0, w.N, w.tiers, w.C, w.K,
+                 out_ids=ids, attention=(att, segs, out), any_order=True)
+        torch.cuda.synchronize()
+        return ids, plan.attn_out.clone()
+
+    want_ids, want = step(d["queries"])
+    q = d["queries"].clone()
+    ids, got = step(q, q)
+    assert torch.equal(ids, want_ids) and torch.equal(got, want)
+    plan.ws = att.ws = torch.empty(plan.ws.numel() + att.ws.numel(), dtype=torch.uint8, device=DEV)
+    for _ in range(3):
+        ids, got = step(d["queries"])
+        assert torch.equal(ids, want_ids) and torch.equal(got, want)
