@@ -334,6 +334,13 @@ bool pkv_plan_split_attention(const pkv_retrieve_args *r, const void *ws, const 
       out->sel_wgs = (n_sel + ++out->splits_per_wg - 1) / out->splits_per_wg;
     } while (out->splits_per_wg < kSelSplits / 4 && (int64_t)rows * out->sel_wgs > kSplitWorkgroups);
     if (out->sel_wgs == 1) return false;  // few selected keys among very many others
+    // A second round of workgroups selects once more for every row: never with eight candidates to a thread, and with fewer where
+    // the last round is less than 3/8 full.  Decode step, us, attention after the top-k / by several workgroups a row: 128 rows,
+    // 8192 candidates, top 1024 (384 workgroups) 94.3 / 102.5, 192 rows, 5000, top 512 (384) 105.9 / 110.4; 4096 candidates: 96 rows,
+    // top 1024 (288) 59.9 / 61.6, 136, top 700 (272) 72.2 / 74.0, 192, top 1024 (576) 101.3 / 105.0; 176, top 512 (352) 85.7 / 83.5,
+    // 160, top 1024 (480) 90.1 / 86.8, 256, top 512 (512) 113.3 / 106.2.
+    const int64_t all = (int64_t)rows * out->sel_wgs, last = all % kSplitWorkgroups;
+    if (all > kSplitWorkgroups && (r->n_cand > kSplitMaxCand / 2 || (last && last < kSplitWorkgroups * 3 / 8))) return false;
     out->dense_a = lo, out->dense_skip = n_sel;
   }
   out->n_dense = out->n_splits - out->dense_skip;

@@ -270,3 +270,15 @@ def test_decode_step_waits_where_buffers_are_shared():
         aa.ws = ws + ws_bytes  # right behind it
         assert form(a, ws, aa) == apart
         assert form(a, at_ws + aa.ws_bytes, aa) == apart
+
+
+def test_decode_step_selects_several_times_a_row_only_in_one_round():
+    """Several workgroups a row select the same keys each: where they are more than the chip takes at once, only if the rounds fill."""
+    from pariskv_amd import _lib
+
+    form = _lib.lib().pkv_decode_step_form
+    for rows, cand, k, want in ((64, 8192, 1024, 2), (85, 8192, 1024, 2), (86, 8192, 1024, 0), (128, 8192, 700, 2), (129, 8192, 700, 0),
+                                (192, 4097, 512, 0), (192, 4096, 512, 2), (96, 3000, 1024, 0), (96, 3000, 700, 2), (136, 1500, 700, 0),
+                                (160, 3000, 1024, 2), (192, 3000, 1024, 0), (256, 4096, 512, 2), (256, 8192, 250, 1), (512, 1500, 200, 1)):
+        a, ws, _, aa = _in_place_step(bs=rows, H=1, n_keys=20000, n_cand=cand, k=k)
+        assert form(a, ws, aa) == want, (rows, cand, k)
