@@ -136,16 +136,19 @@ bool as_one_tensor(const AttSegs &sg, int es, AttOne &one) {
 
 }  // namespace
 
-// One CU fetches scattered rows at 35 to 40 GB/s, 2.7 us for 200 of them and as much as the merge's launch: up to five blocks of 32
+// One CU fetches scattered rows at 35 to 40 GB/s, 2.7 us for 200 of them and as much as the merge's launch: up to six blocks of 32
 // are one workgroup's, which then merges; more go to a workgroup per split of 128, each selecting anew, or per two or three where
 // that would be more workgroups than CUs; there up to eight blocks are one workgroup's as well.  Where the selection takes several
-// launches (more than 8192 candidates), only the first form: its last launch is too long to be run by several workgroups a row.
-// Decode step, us, attention after the top-k / in two parts: 8 rows x 4096 keys, top 100, 28.2 / 23.9, top 256 25.5 / 23.7 (25.5 by
-// one workgroup a row); 8 x 32768, top 512, 30.0 / 27.1; 32 x 16000, 8 heads, top 100 34.5 / 31.0, top 512 36.9 / 33.4; 64 x 40000,
-// top 256 46.5 / 44.7, top 512 52.4 / 46.9; 64 x 65536, top 100, 56.3 / 52.2; 256 x 8000, top 100, 73.1 / 59.8, top 256 77.1 / 67.7
-// (76.7 by several a row).  More than 8192 candidates: 8 x 100000, top 100, 45.7 / 42.9, 64 x 100000 88.8 / 87.9; by several
-// workgroups a row 16 x 131072, top 200, 52.0 / 52.5.
-constexpr int kSplitWorkgroups = 256, kMergeBlocks = 5;
+// launches (more than 8192 candidates), only the first form: its last launch is too long to be run by several workgroups a row
+// (16 rows x 131072, top 200, 52.0 / 52.5).
+// Decode step, us, attention after the top-k / in two parts, by one workgroup a row: 8 rows x 4096 keys, top 100, 25.5 / 23.5;
+// 32 x 16000, 8 heads, top 100, 31.6 / 30.8; 64 x 65536, top 100, 60.0 / 56.8; 256 x 8000, top 100, 74.0 / 66.0, top 256 80.3 / 70.8;
+// more than 8192 candidates: 8 x 100000, top 100, 47.2 / 45.7, 64 x 100000 96.7 / 94.2.  By several: 8 x 32768, top 512, 28.6 / 28.4;
+// 32 x 16000, 8 heads, top 512, 33.6 / 32.8; 64 x 40000, top 512, 52.6 / 51.4, top 1024 57.0 / 55.2.
+// After the top-k / by one / by several, 40000 keys, 4000 candidates: six blocks, 8 rows 31.3 / 29.7 / 30.9, 32 rows 38.0 / 36.5 / 38.0,
+// 64 rows 51.4 / 49.0 / 49.8; eight, 16 rows 33.5 / 34.4 / 33.8, 64 rows 51.9 / 50.3 / 50.2.  After the top-k / by one, 100000 keys,
+// 9000 candidates: six blocks, 8 rows 47.2 / 45.9, 64 rows 94.6 / 93.0; eight, 16 rows 52.6 / 53.7.
+constexpr int kSplitWorkgroups = 256, kMergeBlocks = 6;
 constexpr int64_t kSplitMaxSelected = 1024, kSplitMaxCand = 8192;
 
 extern "C" size_t pkv_decode_attention_ws_bytes(int bs, int n_kv_heads, int group, int64_t total_keys) {

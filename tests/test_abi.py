@@ -282,3 +282,15 @@ def test_decode_step_selects_several_times_a_row_only_in_one_round():
                                 (160, 3000, 1024, 2), (192, 3000, 1024, 0), (256, 4096, 512, 2), (256, 8192, 250, 1), (512, 1500, 200, 1)):
         a, ws, _, aa = _in_place_step(bs=rows, H=1, n_keys=20000, n_cand=cand, k=k)
         assert form(a, ws, aa) == want, (rows, cand, k)
+
+
+def test_decode_step_merges_up_to_six_blocks_in_one_workgroup():
+    """Selected keys in up to six blocks of 32 are one workgroup's; beyond, several workgroups' where they fit one round and the
+    selection is one launch."""
+    from pariskv_amd import _lib
+
+    form = _lib.lib().pkv_decode_step_form
+    for rows, cand, k, want in ((8, 4000, 160, 1), (8, 4000, 192, 1), (8, 4000, 193, 2), (64, 4000, 192, 1), (8, 9000, 192, 1),
+                                (8, 9000, 193, 0), (8, 9000, 512, 0), (128, 9000, 250, 1), (128, 9000, 257, 0), (8, 4000, 1024, 2), (8, 4000, 1025, 0)):
+        a, ws, _, aa = _in_place_step(bs=rows, H=1, n_keys=20000, n_cand=cand, k=k)  # 64 rows before the selected ones: two whole blocks
+        assert form(a, ws, aa) == want, (rows, cand, k)

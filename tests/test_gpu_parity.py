@@ -1961,8 +1961,8 @@ def test_prefill_store_index_layouts(ops, dtype, layout, norms, n_enc):
 
 @pytest.mark.parametrize("group,k,sink,tail,keys,cand", [(*c, 3000, 1500) for c in (
     (4, 100, 64, 529), (1, 1, 0, 1), (3, 15, 3, 0), (5, 16, 64, 64), (8, 17, 64, 1100), (2, 33, 95, 30), (6, 256, 1, 130), (4, 256, 64, 700),
-    (7, 257, 0, 0), (4, 512, 64, 700), (8, 100, 64, 1300), (6, 1024, 64, 1300), (4, 64, 31, 1), (2, 31, 129, 65))] + [
-    (4, 100, 64, 529, 20000, 8193), (3, 129, 31, 65, 20000, 9001), (2, 200, 64, 1, 20000, 9001)])
+    (7, 257, 0, 0), (4, 512, 64, 700), (8, 100, 64, 1300), (6, 1024, 64, 1300), (4, 64, 31, 1), (2, 31, 129, 65), (4, 192, 64, 700), (8, 162, 33, 0))] + [
+    (4, 100, 64, 529, 20000, 8193), (3, 129, 31, 65, 20000, 9001), (2, 200, 64, 1, 20000, 9001), (4, 192, 64, 529, 20000, 9001)])
 def test_decode_step_in_place_attends_in_two_parts(ops, group, k, sink, tail, keys, cand):
     """The step whose attention reads selected rows where they lie: the other rows beside the query side, selected rows in the
     top-k's workgroups.  The same ids and the same sums, bit for bit, as the top-k and the attention called one by one; and the
