@@ -75,9 +75,9 @@ __global__ void pkv_attn_merge_kernel(const float *__restrict__ ws, int n_splits
   __syncthreads();
   float os = 0.f;
 #pragma unroll
-  for (int s = 0; s < kEarly; ++s) os += early[s] * (s < n_splits ? s_w[g][s] : 0.f);
+  for (int s = 0; s < kEarly; ++s) os = fmaf(early[s], s < n_splits ? s_w[g][s] : 0.f, os);
 #pragma unroll 8
-  for (int s = kEarly; s < n_splits; ++s) os += po[(int64_t)s * G * kPartStride] * s_w[g][s];
+  for (int s = kEarly; s < n_splits; ++s) os = fmaf(po[(int64_t)s * G * kPartStride], s_w[g][s], os);
   const int64_t oi = ((int64_t)row * G + g) * 128 + d;
   if (BF16)
     ((uint16_t *)out)[oi] = pkv_f32_to_bf16_bits(os);

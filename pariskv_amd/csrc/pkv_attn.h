@@ -412,7 +412,7 @@ __device__ __forceinline__ void att_step_mfma(const char *kbase, const char *vba
     p[e] = valid[e] ? __builtin_amdgcn_exp2f(sc[e] - m_new) : 0.f;
     psum += p[e];
   }
-  l_part = l_part * corr + psum;
+  l_part = fmaf(l_part, corr, psum);
   const pkv_u32x4 pa = {pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]),
                         pack_bf16x2(p[6], p[7])};
   // the output rows of this lane belong to heads 4j .. 4j+3: fetch their correction factors
@@ -461,8 +461,8 @@ __device__ __forceinline__ void att_merge_waves(int group, float m_run, float l_
 #pragma unroll
     for (int w = 0; w < kMfmaWaves; ++w) {
       const float c = exp2f(s_m[w][g] - mn);
-      ls += s_l[w][g] * c;
-      os += s_o[w][g][d] * c;
+      ls = fmaf(s_l[w][g], c, ls);
+      os = fmaf(s_o[w][g][d], c, os);
     }
     out[g * out_stride + d] = os;
     if (d == 0) ml[g * ml_stride] = mn, ml[g * ml_stride + 1] = ls;
@@ -526,7 +526,7 @@ __device__ __forceinline__ void att_partial_mfma(const void *__restrict__ q, int
 // its top-k (4.9 + 2.7 of 26.5 us at 8 rows x 4096 keys), so: workgroups beside the query side of the retrieval, on an otherwise
 // idle chip, take the keys that are not selected, and the top-k's workgroups go on with those that are.  The sums are those of the
 // one-piece attention, bit for bit: the same blocks of 32 keys (a wave's), merged by fours into splits and the splits into the
-// output in the same order.
+// output in the same order, with the fused form of each a * b + c written out on both sides.
 constexpr int kSelBlocks = 8;   // most blocks of a selecting workgroup
 constexpr int kSelSplits = 12;  // one more than a row's splits may be where the selecting workgroup merges
 constexpr int kSelSlots = 32;   // partial results of a row there: splits in 0 .. 11, single blocks in 12 .. 19
