@@ -295,7 +295,8 @@ __device__ __forceinline__ void att_partial_vector(const void *__restrict__ q, i
   }
 
   // merge the 16 key slots of the workgroup through LDS
-  __shared__ float s_m[16][G], s_l[16][G], s_o[16][G][128 + 4];
+  __shared__ float s_m[16][G], s_l[16][G];
+  __shared__ alignas(16) float s_o[16][G][128 + 4];  // written by 128 bits
 #pragma unroll
   for (int g = 0; g < G; ++g) {
     if (lane16 == 0) s_m[grp][g] = m[g], s_l[grp][g] = l[g];
@@ -441,7 +442,8 @@ __device__ __forceinline__ void att_merge_waves(int group, float m_run, float l_
                                                 float *out, int out_stride) {
   PKV_ATT_CONTRACT
   const int lane = threadIdx.x & (PKV_WAVE - 1), wave = threadIdx.x / PKV_WAVE, n = lane & 15, j = lane >> 4;
-  __shared__ float s_m[kMfmaWaves][8], s_l[kMfmaWaves][8], s_o[kMfmaWaves][8][128 + 4];
+  __shared__ float s_m[kMfmaWaves][8], s_l[kMfmaWaves][8];
+  __shared__ alignas(16) float s_o[kMfmaWaves][8][128 + 4];  // written by 128 bits
   if (j == 0 && n < group) s_m[wave][n] = m_run, s_l[wave][n] = l_part;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -640,9 +642,10 @@ __device__ __forceinline__ float att_lane(float x, int lane) {
 }
 
 // LDS of the selecting workgroups: the blocks of the splits that hold selected keys, the first of these splits first.
-struct AttSelSmem {
+struct alignas(16) AttSelSmem {  // read and written by 128 bits
   float m[8][16], l[8][16], o[kSelSplits][8][128 + 4];
 };
+static_assert(offsetof(AttSelSmem, l) % 16 == 0 && offsetof(AttSelSmem, o) % 16 == 0 && (128 + 4) * sizeof(float) % 16 == 0, "128-bit rows");
 
 // Clears (max, sum) of the blocks; a barrier lies between this and att_selected.
 __device__ __forceinline__ void att_clear(AttSelSmem &sm) {
