@@ -26,15 +26,247 @@
 
 namespace {
 
+constexpr int kAttThreads = 256;
+constexpr int kAttKeysPerIter = kAttThreads / 16;  // 16 keys per workgroup step
+constexpr int kAttUnroll = 2;                      // keys per 16-lane group per step
+
+struct AttSegs {
+  const void *k[PKV_ATTN_MAX_SEGMENTS];
+  const void *v[PKV_ATTN_MAX_SEGMENTS];
+  int64_t stride_b[PKV_ATTN_MAX_SEGMENTS], stride_h[PKV_ATTN_MAX_SEGMENTS];
+  int64_t row0[PKV_ATTN_MAX_SEGMENTS];
+  int64_t end[PKV_ATTN_MAX_SEGMENTS];  // exclusive end of the segment in the concatenated key order
+  const int64_t *idx[PKV_ATTN_MAX_SEGMENTS];  // per segment: selected rows (relative to row0) or nullptr
+  int64_t idx_stride[PKV_ATTN_MAX_SEGMENTS], idx_limit[PKV_ATTN_MAX_SEGMENTS];
+  int n;
+};
+
+// Row (inside the (b, h) slab of its segment, row0 included) and segment of concatenated key jj, packed as
+// row | segment << 29.  Indexed segments cost one dependent 8-byte load.
+__device__ __forceinline__ uint32_t att_resolve_row(const AttSegs &segs, int row, uint32_t jj) {
+  int s = 0;
+  uint32_t first = 0;
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (t < segs.n && jj >= (uint32_t)segs.end[t - 1]) s = t, first = (uint32_t)segs.end[t - 1];
+  const int64_t *ip = segs.idx[0];
+  int64_t stride = segs.idx_stride[0], limit = segs.idx_limit[0], row0 = segs.row0[0];
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (s == t) ip = segs.idx[t], stride = segs.idx_stride[t], limit = segs.idx_limit[t], row0 = segs.row0[t];
+  int64_t r = jj - first;
+  if (ip) {
+    r = ip[(int64_t)row * stride + r];
+    r = r < 0 ? 0 : (r >= limit ? limit - 1 : r);
+  }
+  return (uint32_t)(r + row0) | ((uint32_t)s << 29);
+}
+// Keys row `row` attends to: all `total`, its own row_keys[row], or with uniform > 0 the largest of row_keys[0 .. uniform)
+// (the dense form of the adaptive-k step, where a launch of its own for the maximum took 4.5 us at 24 rows).
+__device__ __forceinline__ int64_t att_row_total(int64_t total, const int32_t *__restrict__ row_keys, int row, int uniform) {
+  if (!row_keys) return total;
+  int64_t rk;
+  if (uniform > 0) {
+    int m = 0;
+    for (int r = pkv_lane(); r < uniform; r += PKV_WAVE) m = max(m, row_keys[r]);
+#define PKV_ATT_MAX(M) { const int o = (int)pkv_lane_xor<M>((uint32_t)m); m = max(m, o); }
+    PKV_ATT_MAX(1) PKV_ATT_MAX(2) PKV_ATT_MAX(4) PKV_ATT_MAX(8) PKV_ATT_MAX(16) PKV_ATT_MAX(32)
+#undef PKV_ATT_MAX
+    rk = __builtin_amdgcn_readfirstlane(m);
+  } else {
+    rk = row_keys[row];
+  }
+  return rk < total ? (rk > 0 ? rk : 1) : total;
+}
+template <bool INDEXED, uint32_t ROW>
+__device__ __forceinline__ AttPlace<false> att_place(const AttSegs &a, int row, int b, int h, uint32_t jj) {
+  int s = 0;
+  uint32_t first = 0;
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (t < a.n && jj >= (uint32_t)a.end[t - 1]) s = t, first = (uint32_t)a.end[t - 1];
+  const char *k = (const char *)a.k[0], *v = (const char *)a.v[0];
+  int64_t sb = a.stride_b[0], sh = a.stride_h[0], row0 = a.row0[0];
+#pragma unroll
+  for (int t = 1; t < PKV_ATTN_MAX_SEGMENTS; ++t)
+    if (s == t) k = (const char *)a.k[t], v = (const char *)a.v[t], sb = a.stride_b[t], sh = a.stride_h[t], row0 = a.row0[t];
+  const int64_t r = INDEXED ? (int64_t)(att_resolve_row(a, row, jj) & 0x1fffffffu) : row0 + (int64_t)(jj - first);
+  const int64_t off = ((int64_t)b * sb + (int64_t)h * sh) * (ROW / 128) + r * ROW;
+  return {(uint64_t)(k + off), (uint64_t)(v + off)};
+}
+
+// Eight consecutive elements as loaded.  Kept apart from their use so that a load can be issued a whole step before its data is
+// touched.
+struct Raw8 {
+  pkv_u32x4 a, b;
+};
+
+// Plain loads: two instructions share every 128-byte line of a row, and a streaming load gives the line up after the first.
+// Decode step, streaming / plain: 12 rows x 865 attended keys, 7 heads (2 layers) 68.6 / 64.8 us.
+__device__ __forceinline__ void load_raw8(const void *base, int64_t elem_off, Raw8 &r) {
+  r.a = *(const pkv_u32x4 *)((const float *)base + elem_off);
+  r.b = *(const pkv_u32x4 *)((const float *)base + elem_off + 4);
+}
+
+__device__ __forceinline__ void expand8(const Raw8 &r, float (&x)[8]) {
+  x[0] = __uint_as_float(r.a.x), x[1] = __uint_as_float(r.a.y), x[2] = __uint_as_float(r.a.z), x[3] = __uint_as_float(r.a.w);
+  x[4] = __uint_as_float(r.b.x), x[5] = __uint_as_float(r.b.y), x[6] = __uint_as_float(r.b.z), x[7] = __uint_as_float(r.b.w);
+}
+
+__device__ __forceinline__ void load8(const void *base, int64_t elem_off, float (&x)[8]) {
+  Raw8 r;
+  load_raw8(base, elem_off, r);
+  expand8(r, x);
+}
+
+// Splits are of 64 keys while the key set allows: a launch is one chain of dependent loads with some 1000 instructions behind
+// it, not bandwidth.  Places of keys as in the bf16 kernel below.  Decode step, us, with a 64-bit pointer picked out of four for
+// each row / with places: 12 rows x 865 attended keys, 7 heads (2 layers) 74.6 / 70.0, 8 rows x 696 (2 layers) 66.5 / 61.0,
+// 32 rows x 896 48.6 / 45.2.
 // grid (splits, rows, query heads by G)
-template <bool BF16, int G, bool INDEXED, typename SEGS>
+template <int G, bool INDEXED, typename SEGS>
 __global__ __launch_bounds__(kAttThreads) void pkv_attn_partial_kernel(const void *__restrict__ q, int n_kv_heads,
                                                                        int group, SEGS segs, int64_t total,
                                                                        const int32_t *__restrict__ row_keys, int uniform,
                                                                        int64_t per_split, float scale_log2e,
                                                                        float *__restrict__ ws) {
-  att_partial_vector<BF16, G, INDEXED>(q, n_kv_heads, group, segs, total, row_keys, uniform, per_split, scale_log2e, ws,
-                                       (int)gridDim.x, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
+  // blockIdx.z: query heads g0 .. g0 + g_count - 1 of the KV head (more than four would not fit the registers)
+  const int g0 = blockIdx.z * G, g_count = group - g0 < G ? group - g0 : G;
+  const int split = blockIdx.x, row = blockIdx.y;
+  const int b = row / n_kv_heads, h = row % n_kv_heads;
+  const int tid = threadIdx.x;
+  const int lane16 = tid & 15;        // owns dims 8*lane16 .. +7
+  const int grp = tid >> 4;           // 16 key slots per workgroup step
+
+  total = att_row_total(total, row_keys, row, uniform);  // ragged rows
+  const int64_t j0 = (int64_t)split * per_split;
+  const int64_t j1 = (j0 + per_split < total) ? j0 + per_split : total;
+  constexpr bool ONE = __is_same(SEGS, AttOne);
+  constexpr uint32_t kRow = 512;
+  const int lane = tid & (PKV_WAVE - 1), wave = tid / PKV_WAVE;
+  const char *kbase = nullptr, *vbase = nullptr;
+  if constexpr (ONE) {
+    const int64_t slab = (int64_t)b * segs.stride_b + (int64_t)h * segs.stride_h;
+    kbase = segs.k + slab, vbase = segs.v + slab;
+  }
+  // K/V rows of the step after the current one are requested before the current one is consumed
+  float kx[kAttUnroll][8], vx[kAttUnroll][8];
+  Raw8 kn[kAttUnroll], vn[kAttUnroll];
+  AttPlace<ONE> mine;
+  auto fetch = [&](int64_t jb, Raw8 (&kd)[kAttUnroll], Raw8 (&vd)[kAttUnroll]) {
+    // four turns (64 keys) at a time: lane 4 t + i (mod 16) finds the place of the key that the wave's lanes 16 i .. 16 i + 15
+    // read in turn t
+    static_assert(4 % kAttUnroll == 0 && kAttKeysPerIter == 16, "a wave reads four keys in a turn");
+    const int turn = ((int)(jb - j0) / kAttKeysPerIter) & 3;
+    if (turn == 0) {
+      const int64_t key = jb + ((lane >> 2) & 3) * kAttKeysPerIter + 4 * wave + (lane & 3);
+      mine = att_place<INDEXED, kRow>(segs, row, b, h, (uint32_t)(key < j1 ? key : j1 - 1));  // fewer than 2^24 keys
+    }
+#pragma unroll
+    for (int u = 0; u < kAttUnroll; ++u) {
+      const int at = 4 * (turn + u) + (lane >> 4);
+      const char *kp, *vp;
+      if constexpr (ONE) {
+        const uint64_t off = mine.from(at).off + (kRow / 16) * (uint32_t)lane16;
+        kp = kbase + off, vp = vbase + off;
+      } else {
+        kp = mine.k_from(at) + (kRow / 16) * lane16, vp = mine.v_from(at) + (kRow / 16) * lane16;
+      }
+      load_raw8(kp, 0, kd[u]);
+      load_raw8(vp, 0, vd[u]);
+    }
+  };
+  if (j0 < j1) fetch(j0, kn, vn);  // before the queries: nothing here waits for them
+
+  float qv[G][8];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {  // surplus slots idle
+    load8(q, ((int64_t)row * group + g0 + (g < g_count ? g : 0)) * 128 + 8 * lane16, qv[g]);
+#pragma unroll
+    for (int d = 0; d < 8; ++d) qv[g][d] *= scale_log2e;  // scores come out in units of log2(e)
+  }
+  float m[G], l[G], o[G][8];
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    m[g] = kNegBig, l[g] = 0.f;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) o[g][d] = 0.f;
+  }
+
+  for (int64_t jb = j0; jb < j1; jb += kAttKeysPerIter * kAttUnroll) {
+    bool valid[kAttUnroll];
+#pragma unroll
+    for (int u = 0; u < kAttUnroll; ++u) {
+      valid[u] = jb + u * kAttKeysPerIter + grp < j1;
+      expand8(kn[u], kx[u]);
+      expand8(vn[u], vx[u]);
+    }
+    if (jb + kAttKeysPerIter * kAttUnroll < j1) fetch(jb + kAttKeysPerIter * kAttUnroll, kn, vn);
+    float s[G][kAttUnroll];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+#pragma unroll
+      for (int u = 0; u < kAttUnroll; ++u) {
+        float acc = qv[g][0] * kx[u][0];
+#pragma unroll
+        for (int d = 1; d < 8; ++d) acc += qv[g][d] * kx[u][d];
+        acc += pkv_lane_xor_f<1>(acc);
+        acc += pkv_lane_xor_f<2>(acc);
+        acc += pkv_lane_xor_f<4>(acc);
+        acc += pkv_lane_xor_f<8>(acc);
+        s[g][u] = valid[u] ? acc : kNegBig;
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      float mn = m[g];
+#pragma unroll
+      for (int u = 0; u < kAttUnroll; ++u) mn = fmaxf(mn, s[g][u]);
+      const float corr = exp2f(m[g] - mn);
+      m[g] = mn;
+      float p[kAttUnroll], psum = 0.f;
+#pragma unroll
+      for (int u = 0; u < kAttUnroll; ++u) {
+        p[u] = valid[u] ? exp2f(s[g][u] - mn) : 0.f;
+        psum += p[u];
+      }
+      l[g] = l[g] * corr + psum;
+#pragma unroll
+      for (int d = 0; d < 8; ++d) {
+        float acc = o[g][d] * corr;
+#pragma unroll
+        for (int u = 0; u < kAttUnroll; ++u) acc += p[u] * vx[u][d];
+        o[g][d] = acc;
+      }
+    }
+  }
+
+  // merge the 16 key slots of the workgroup through LDS
+  __shared__ float s_m[16][G], s_l[16][G];
+  __shared__ alignas(16) float s_o[16][G][128 + 4];  // written by 128 bits
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    if (lane16 == 0) s_m[grp][g] = m[g], s_l[grp][g] = l[g];
+    *(float4 *)&s_o[grp][g][8 * lane16] = float4{o[g][0], o[g][1], o[g][2], o[g][3]};
+    *(float4 *)&s_o[grp][g][8 * lane16 + 4] = float4{o[g][4], o[g][5], o[g][6], o[g][7]};
+  }
+  __syncthreads();
+  float *part = ws + (((int64_t)row * gridDim.x + split) * group + g0) * kPartStride;
+  for (int e = tid; e < g_count * 128; e += kAttThreads) {
+    const int g = e >> 7, d = e & 127;
+    float mn = s_m[0][g];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) mn = fmaxf(mn, s_m[w][g]);
+    float ls = 0.f, os = 0.f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      const float c = exp2f(s_m[w][g] - mn);
+      ls += s_l[w][g] * c;
+      os += s_o[w][g][d] * c;
+    }
+    part[g * kPartStride + 2 + d] = os;
+    if (d == 0) part[g * kPartStride] = mn, part[g * kPartStride + 1] = ls;
+  }
 }
 
 // grid (splits, KV heads, batch).  Decode step, us, with four-way pointer selection per row / with places by lane exchange:
@@ -43,9 +275,50 @@ template <bool INDEXED, typename SEGS>
 __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_kernel(
     const void *__restrict__ q, int group, SEGS segs, int64_t total, const int32_t *__restrict__ row_keys, int uniform,
     int64_t per_split, float scale_log2e, float *__restrict__ ws) {
-  const int h = blockIdx.y, b = blockIdx.z;
-  att_partial_mfma<INDEXED>(q, group, segs, total, row_keys, uniform, per_split, scale_log2e, ws, (int)gridDim.x,
-                            (int)blockIdx.x, b * (int)gridDim.y + h, b, h);
+  const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z, row = b * (int)gridDim.y + h;
+  constexpr bool ONE = __is_same(SEGS, AttOne);
+  const int lane = threadIdx.x & (PKV_WAVE - 1), wave = threadIdx.x / PKV_WAVE;
+  const int n = lane & 15, j = lane >> 4;
+  total = att_row_total(total, row_keys, row, uniform);
+  const int64_t per_wave = per_split / kMfmaWaves;  // a multiple of the 32 keys of one step
+  const int64_t j0 = (int64_t)split * per_split + (int64_t)wave * per_wave;
+  const int64_t j1 = (j0 + per_wave < total) ? j0 + per_wave : total;  // j1 <= j0: nothing left for this wave
+
+  // Lane l holds the place of key blk0 + l of the current block of 64 keys (two steps; keys past j1 repeat the last one);
+  // the lanes that read a row get it from there, so that a place is found once per key and wave.
+  AttPlace<ONE> mine;
+  const char *kbase = nullptr, *vbase = nullptr;
+  if constexpr (ONE) {
+    const int64_t slab = (int64_t)b * segs.stride_b + (int64_t)h * segs.stride_h;
+    kbase = segs.k + slab, vbase = segs.v + slab;
+  }
+  auto place_block = [&](int64_t jb) {
+    const int64_t key = jb + lane;
+    mine = att_place<INDEXED, 256>(segs, row, b, h, (uint32_t)(key < j1 ? key : j1 - 1));
+  };
+  if (j0 < j1) place_block(j0);  // before the queries: the indices' latency is the longer one
+
+  const pkv_u32x4 zero4 = {0u, 0u, 0u, 0u};
+  pkv_u32x4 qb[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    qb[c] = n < group ? *(const pkv_u32x4 *)((const uint16_t *)q + ((int64_t)row * group + n) * 128 + 32 * c + 8 * j) : zero4;
+
+  float m_run = kNegBig, l_part = 0.f;
+  pkv_f32x4 o[8];
+#pragma unroll
+  for (int m = 0; m < 8; ++m) o[m] = pkv_f32x4{0.f, 0.f, 0.f, 0.f};
+
+  if (j0 < j1) att_step_mfma<ONE, true>(kbase, vbase, mine, 0, j0, j1, qb, scale_log2e, m_run, l_part, o);
+  for (int64_t jb = j0 + kMfmaStepKeys; jb < j1; jb += kMfmaStepKeys) {
+    const int in_block = (int)(jb - j0) & (PKV_WAVE - 1);
+    if (in_block == 0) place_block(jb);
+    att_step_mfma<ONE, false>(kbase, vbase, mine, in_block, jb, j1, qb, scale_log2e, m_run, l_part, o);
+  }
+
+  l_part = pkv_pair_add<32>(pkv_pair_add<16>(l_part));
+  float *part = ws + ((int64_t)row * gridDim.x + split) * group * kPartStride;
+  att_merge_waves(group, m_run, l_part, o, part, kPartStride, part + 2, kPartStride);
 }
 
 // grid R, G*128 threads: merge the splits (at most 64) and normalise.
@@ -238,7 +511,7 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
     // heads, 2 x 8.0 us as two launches one after the other; the decode step around it (9001 keys) 48.3 -> 43 us.
     grid.z = (unsigned)head_wgs;
 #define PKV_ATT(GG, IDX, S)                                                                                               \
-  hipLaunchKernelGGL((pkv_attn_partial_kernel<false, GG, IDX, decltype(S)>), grid, dim3(kAttThreads), 0, s, q, n_kv_heads, group, \
+  hipLaunchKernelGGL((pkv_attn_partial_kernel<GG, IDX, decltype(S)>), grid, dim3(kAttThreads), 0, s, q, n_kv_heads, group, \
                      S, total, row_keys, uniform, per_split, scale_log2e, (float *)ws)
 #define PKV_ATT_G(IDX, S)                     \
   do {                                        \
