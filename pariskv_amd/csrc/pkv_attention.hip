@@ -422,7 +422,7 @@ bool as_one_tensor(const AttSegs &sg, int es, AttOne &one) {
 // 64 rows 51.4 / 49.0 / 49.8; eight, 16 rows 33.5 / 34.4 / 33.8, 64 rows 51.9 / 50.3 / 50.2.  After the top-k / by one, 100000 keys,
 // 9000 candidates: six blocks, 8 rows 47.2 / 45.9, 64 rows 94.6 / 93.0; eight, 16 rows 52.6 / 53.7.
 constexpr int kSplitWorkgroups = 256, kMergeBlocks = 6;
-constexpr int64_t kSplitMaxSelected = 1024, kSplitMaxCand = 8192;
+constexpr int64_t kSplitMaxSelected = 1024;
 
 extern "C" size_t pkv_decode_attention_ws_bytes(int bs, int n_kv_heads, int group, int64_t total_keys) {
   if (bs <= 0 || n_kv_heads <= 0 || group <= 0 || total_keys <= 0) return 256;
@@ -603,7 +603,7 @@ bool pkv_plan_split_attention(const pkv_retrieve_args *r, const void *ws, const 
     }
     if ((int64_t)rows * 20 * r->group * 128 >= ((int64_t)1 << 31)) return false;
     out->ws_ml = (float *)at->ws + (int64_t)rows * 20 * r->group * 128;
-  } else if (r->n_cand > kSplitMaxCand) {
+  } else if (r->n_cand > kTopkMaxSort) {
     return false;
   } else {
     do {
@@ -616,7 +616,7 @@ bool pkv_plan_split_attention(const pkv_retrieve_args *r, const void *ws, const 
     // top 1024 (288) 59.9 / 61.6, 136, top 700 (272) 72.2 / 74.0, 192, top 1024 (576) 101.3 / 105.0; 176, top 512 (352) 85.7 / 83.5,
     // 160, top 1024 (480) 90.1 / 86.8, 256, top 512 (512) 113.3 / 106.2.
     const int64_t all = (int64_t)rows * out->sel_wgs, last = all % kSplitWorkgroups;
-    if (all > kSplitWorkgroups && (r->n_cand > kSplitMaxCand / 2 || (last && last < kSplitWorkgroups * 3 / 8))) return false;
+    if (all > kSplitWorkgroups && (r->n_cand > kTopkMaxSort / 2 || (last && last < kSplitWorkgroups * 3 / 8))) return false;
     out->dense_a = lo, out->dense_skip = n_sel;
   }
   out->n_dense = out->n_splits - out->dense_skip;

@@ -442,7 +442,6 @@ __global__ void pkv_zero_u32_kernel(uint32_t *__restrict__ p, int64_t n) {
 // ------------------------------------------------------------ exact fp32 top-k
 
 constexpr int kTopkThreads = 1024;
-constexpr int kTopkMaxSort = 8192;  // 64 KB of 64-bit keys in LDS
 
 __device__ __forceinline__ uint64_t make_key(const float *__restrict__ x, const int64_t *__restrict__ ids,
                                              int64_t i) {
@@ -1556,7 +1555,7 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_wide_compact_kernel(
 }
 
 // grid rows; dynamic LDS lds_bytes_sort(P): the winners, and as many keys again for the counting sort when they fit.
-// s_keys: max(P, 1024) keys, and a second copy behind them where P <= kCountingSortMaxP.  out_ids may be null.
+// s_keys: max(P, 1024) keys, and a second copy behind them where P <= kCountingSortMaxP.
 __device__ __forceinline__ void wide_finish(int row, int64_t len, int P, int64_t k, const uint32_t *__restrict__ ctl,
                                             const uint64_t *__restrict__ list_a, const uint64_t *__restrict__ list_b,
                                             int64_t *__restrict__ out_ids, float *__restrict__ out_vals, uint64_t *s_keys,
@@ -1569,7 +1568,6 @@ __device__ __forceinline__ void wide_finish(int row, int64_t len, int P, int64_t
     PKV_DISPATCH_E(P, PKV_SORT_K);
 #undef PKV_SORT_K
   }
-  if (!out_ids) return;
   int64_t *oi = out_ids + (int64_t)row * k;
   float *ov = out_vals ? out_vals + (int64_t)row * k : nullptr;
   for (int64_t i = threadIdx.x; i < k; i += kTopkThreads) {
