@@ -1979,18 +1979,100 @@ def test_decode_step_in_place_attends_in_two_parts(ops, group, k, sink, tail, ke
     want_ids = plan.run(*args, any_order=True)  # more than 8192 candidates come out sorted all the same
     ids = torch.zeros_like(want_ids)
     segs = [s for s in [(kk, vv, 0, sink), (kk, vv, sink, k, ids), (kk, vv, sink + w.N, tail)] if s[3]]
+    blocks = (sink + k - 1) // 32 - sink // 32 + 1
+    assert _step_form(ops, plan, att, d["queries"], args, segs) == (
+        1 if blocks <= 6 and sink + k + tail <= 11 * 128 else 2 if cand <= 8192 else 0)
     plan.run(*args, out_ids=ids, attention=(att, segs, None), any_order=True)
     torch.cuda.synchronize()
     got = plan.attn_out.clone()
     assert torch.equal(ids, want_ids)
     assert torch.equal(got, att.run(d["queries"], segs))
-    sel = torch.cat([torch.arange(sink, device=DEV).expand(w.bs, w.H, -1), sink + ids,
-                     torch.arange(sink + w.N, rows, device=DEV).expand(w.bs, w.H, -1)], dim=2)[..., None].expand(-1, -1, -1, 128)
-    ks, vs = (t.gather(2, sel).double().cpu() for t in (kk, vv))
-    q = d["queries"].view(w.bs, w.H, group, 128).double().cpu()
-    want = torch.softmax(q @ ks.transpose(2, 3) / 128 ** 0.5, dim=-1) @ vs
-    err = (got.view(w.bs, w.H, group, 128).double().cpu() - want).abs().max().item()
+    want = _near_attention_in_64_bits(got, d["queries"], kk, vv, sink, w.N, ids)
+    err = (got.view(w.bs, w.H, group, 128).double() - want).abs().max().item()
     assert err <= vv.abs().max().item() * 2.0 ** -8, err
+
+
+def _step_form(ops, plan, att, q, args, segs):
+    """How pkv_decode_step takes plan.run(*args, out_ids=segs' ids, attention=(att, segs, None), any_order=True)."""
+    import ctypes
+
+    ids = next(s[4] for s in segs if len(s) > 4)
+    a = plan._fill(*args, ids, None, None, False, any_order=True)
+    aa, out = att.c_args(q, segs)
+    return ops._lib.lib().pkv_decode_step_form(ctypes.byref(a), plan.ws.data_ptr(), ctypes.byref(aa))
+
+
+def _near_attention_in_64_bits(got, queries, kk, vv, sink, n, ids):
+    """The attention over rows 0 .. sink, sink + ids and sink + n .. in 64 bits, close to `got`: probabilities are rounded to bf16
+    before they meet the values and the output is, 2^-8 relative each; scores and sums are fp32 (1e-5)."""
+    bs, H, rows, _ = kk.shape
+    group = queries.numel() // (bs * H * 128)
+    sel = torch.cat([torch.arange(sink, device=DEV).expand(bs, H, -1), sink + ids,
+                     torch.arange(sink + n, rows, device=DEV).expand(bs, H, -1)], dim=2)[..., None].expand(-1, -1, -1, 128)
+    ks, vs = (t.gather(2, sel).double() for t in (kk, vv))
+    p = torch.softmax(queries.view(bs, H, group, 128).double() @ ks.transpose(2, 3).contiguous() / 128 ** 0.5, dim=-1)
+    want, weight = p @ vs, p @ vs.abs()
+    err = (got.view(bs, H, group, 128).double() - want).abs()
+    assert (err <= (weight + want.abs()) * 2.0 ** -8 + 1e-5 * weight).all(), (err / weight).max().item()
+    return want
+
+
+@pytest.mark.parametrize("bs,H,group,k,sink,tail,keys,cand,form", [
+    # candidates per thread: 2, 4, 8; one workgroup a row and several
+    (2, 2, 4, 100, 64, 529, 5000, 3000, 1), (2, 2, 4, 100, 64, 529, 9000, 8192, 1), (2, 2, 4, 512, 64, 529, 5000, 4096, 2),
+    (2, 2, 8, 1024, 64, 529, 9000, 8192, 2), (1, 3, 5, 300, 1, 40, 9000, 5001, 2),
+    # two and three splits to a workgroup, the last workgroup's not all there
+    (8, 8, 4, 512, 64, 300, 3000, 1500, 2), (8, 8, 4, 1024, 64, 300, 5000, 2500, 2), (9, 8, 4, 800, 64, 300, 5000, 2500, 2),
+    (9, 8, 3, 800, 50, 0, 9000, 8000, 2), (64, 4, 8, 512, 64, 129, 3000, 1500, 2), (40, 4, 1, 1024, 64, 1, 5000, 4096, 2),
+    # six to eight blocks by one workgroup a row: over two splits, over three, with a split that is selected whole
+    (16, 8, 4, 200, 64, 300, 3000, 1500, 1), (16, 8, 4, 250, 64, 300, 5000, 3000, 1), (17, 8, 4, 225, 127, 300, 3000, 1500, 1),
+    (17, 8, 8, 256, 0, 70, 3000, 1500, 1), (16, 8, 2, 230, 40, 900, 9000, 8192, 1), (16, 8, 4, 225, 127, 529, 20000, 9001, 1),
+    # refused: a second round of workgroups that select again
+    (12, 8, 4, 1024, 64, 300, 5000, 2500, 0)])
+def test_decode_step_in_two_parts_by_number_of_rows(ops, bs, H, group, k, sink, tail, keys, cand, form):
+    """The forms that depend on the rows and the candidates: as the top-k and the attention called one by one, bit for bit."""
+    _say(f"two-part attention {bs}x{H} rows group {group} k {k} sink {sink} tail {tail} candidates {cand} of {keys}")
+    _two_parts(ops, bs, H, group, k, sink, tail, keys, cand, form)
+
+
+@pytest.mark.parametrize("scores", ["equal", "few", "infinite"])
+@pytest.mark.parametrize("bs,k,keys,cand,form", [(2, 100, 3000, 1500, 1), (2, 512, 5000, 3000, 2), (32, 512, 5000, 5000 - 1, 2),
+                                                 (2, 100, 20000, 9001, 1)])
+def test_decode_step_in_two_parts_where_scores_tie(ops, scores, bs, k, keys, cand, form):
+    """Selections that no bins of the scores' range separate (all scores equal, a few values, infinite ones): the ids that the
+    attention goes on with are those of the top-k."""
+    _say(f"two-part attention, scores {scores}, {bs * 2} rows k {k} candidates {cand} of {keys}")
+    _two_parts(ops, bs, 2, 4, k, 64, 100, keys, cand, form, scores)
+
+
+def _two_parts(ops, bs, H, group, k, sink, tail, keys, cand, form, scores=None):
+    g = torch.Generator(device=DEV).manual_seed(7)
+    rows = sink + keys + tail
+    kk, vv = (torch.randn(bs, H, rows, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    zone = kk[:, :, sink:sink + keys]
+    if scores in ("equal", "few"):  # one key, or four, again and again in the index (the attended rows stay apart)
+        zone = zone[:, :, :1 if scores == "equal" else 4].repeat(1, 1, keys, 1)[:, :, :keys].contiguous()
+    signs, centers = torch.from_numpy(O.srht_signs(42)).to(DEV), torch.from_numpy(O.mag_constants()[1]).to(DEV)
+    codes, nib, wt, cb, k4, kw = ops.alloc_keymajor(bs, H, keys, DEV)
+    cc = torch.zeros(bs, H, 16, 256, dtype=torch.int32, device=DEV)
+    ops.encode_append(zone, signs, cb, k4, kw, cc)
+    if scores == "infinite":
+        wt[:, :, ::7] = float("inf")
+    q = torch.randn(bs, 1, H * group, 128, generator=g, device=DEV).to(torch.bfloat16)
+    plan = ops.RetrievePlan(bs, H, group, keys, DEV, keys, cand, k)
+    att = ops.DecodeAttention(bs, H, group, rows, DEV)
+    args = (q, signs, centers, cc, codes, nib, wt, 0, keys, O.tier_counts(keys, 0.5), cand, k)
+    want_ids = plan.run(*args, any_order=True)
+    ids = torch.zeros_like(want_ids)
+    segs = [s for s in [(kk, vv, 0, sink), (kk, vv, sink, k, ids), (kk, vv, sink + keys, tail)] if s[3]]
+    assert _step_form(ops, plan, att, q, args, segs) == form
+    plan.run(*args, out_ids=ids, attention=(att, segs, None), any_order=True)
+    torch.cuda.synchronize()
+    got = plan.attn_out.clone()
+    assert torch.equal(ids, want_ids)
+    assert (ids.sort(dim=2).values.diff(dim=2) > 0).all() and int(ids.min()) >= 0 and int(ids.max()) < keys
+    assert torch.equal(got, att.run(q, segs))
+    _near_attention_in_64_bits(got, q, kk, vv, sink, keys, ids)
 
 
 @pytest.mark.parametrize("k,keys,cand", [(100, 3000, 1500), (512, 3000, 1500), (100, 20000, 9001)])
