@@ -333,6 +333,7 @@ void pkv_o_attention(const float *q, int g_heads, const float *k, const float *v
 
 /* --------------------------------------------------------------- adaptive-k */
 
+/* Range reduction and polynomial of expf in S. L. Moshier's Cephes library. */
 float pkv_o_expf(float x) {
   if (!(x >= -87.0f)) return (x != x) ? x : 0.0f;
   if (x > 88.0f) return INFINITY;

@@ -101,8 +101,10 @@ struct Raw8 {
   pkv_u32x4 a, b;
 };
 
-// Plain loads: two instructions share every 128-byte line of a row, and a streaming load gives the line up after the first.
-// Decode step, streaming / plain: 12 rows x 865 attended keys, 7 heads (2 layers) 68.6 / 64.8 us.
+// Queries and K and V rows.  Plain loads: two instructions share every 128-byte line of a row, and a streaming load gives the line up
+// after the first.  Attention, us, streaming / plain: 12 rows x 865 keys, 7 heads, 13.0 / 11.6, by index 13.4 / 11.8; 64 x 2000
+// 35.9 / 33.3, by index 39.8 / 32.3; 256 x 900 52.4 / 51.4, by index 57.1 / 52.3; 768 x 900 140.7 / 136.3.  Slower only
+// where 512 or 1024 KV heads' keys are read in order: 512 x 900 91.0 / 93.2 (by index 96.4 / 93.0), 1024 x 900 183.0 / 188.9.
 __device__ __forceinline__ void load_raw8(const void *base, int64_t elem_off, Raw8 &r) {
   r.a = *(const pkv_u32x4 *)((const float *)base + elem_off);
   r.b = *(const pkv_u32x4 *)((const float *)base + elem_off + 4);

@@ -102,8 +102,9 @@ __device__ __forceinline__ void att_step_mfma(const char *kbase, const char *vba
   PKV_ATT_CONTRACT
   const int lane = threadIdx.x & (PKV_WAVE - 1), n = lane & 15, j = lane >> 4;
   // K: two tiles of 16 keys, lane (n, j) reads dims 32c + 8j .. +7 of key jb + 16t + n.  Two instructions share a 128-byte line:
-  // plain loads, as a streaming load gives it up after the first (decode step, streaming / plain: 8 rows x 1188 attended
-  // keys (4 layers) 115.0 / 112.8 us, 24 x 1900 (2) 92.6 / 91.7; at 64 x 887 (2) 117.2 / 118.6).  V rows are read whole.
+  // plain loads, as a streaming load gives it up after the first.  V rows are read whole.  Attention, us, K streaming / plain:
+  // 8 rows x 700 keys 7.4 / 7.1, 64 x 887 11.4 / 10.6, by index 12.3 / 11.6, 64 x 2000 18.7 / 18.1, by index 21.5 / 19.0,
+  // 512 x 900 52.2 / 49.2, by index 61.1 / 49.7, 1024 x 2000 207.7 / 188.1.
   pkv_u32x4 ka[2][4], vr[8];
 #pragma unroll
   for (int t = 0; t < 2; ++t) {

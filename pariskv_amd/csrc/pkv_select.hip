@@ -1612,6 +1612,7 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_wide_finish_attend_kern
 // resolved by candidate position and the result is reproducible; sums run in a
 // fixed lane/tree order; exp() is a fixed fp32 sequence shared with the CPU checker.
 
+// Range reduction and polynomial of expf in S. L. Moshier's Cephes library.
 __device__ __forceinline__ float pkv_expf(float x) {
   if (!(x >= -87.0f)) return (x != x) ? x : 0.0f;
   if (x > 88.0f) return __uint_as_float(0x7f800000u);

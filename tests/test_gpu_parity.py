@@ -2045,7 +2045,14 @@ def test_decode_step_in_two_parts_where_scores_tie(ops, scores, bs, k, keys, can
     _two_parts(ops, bs, 2, 4, k, 64, 100, keys, cand, form, scores)
 
 
-def _two_parts(ops, bs, H, group, k, sink, tail, keys, cand, form, scores=None):
+@pytest.mark.parametrize("k,keys,cand,form", [(100, 4000, 1500, 1), (512, 5000, 3000, 2), (100, 20000, 9001, 1)])
+def test_decode_step_in_two_parts_replays_from_a_captured_graph(ops, k, keys, cand, form):
+    """Captured once, replayed with other queries and eager work in between: each replay as the eager step."""
+    _say(f"two-part attention captured, k {k} candidates {cand} of {keys}")
+    _two_parts(ops, 2, 2, 4, k, 64, 100, keys, cand, form, replays=4)
+
+
+def _two_parts(ops, bs, H, group, k, sink, tail, keys, cand, form, scores=None, replays=0):
     g = torch.Generator(device=DEV).manual_seed(7)
     rows = sink + keys + tail
     kk, vv = (torch.randn(bs, H, rows, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
@@ -2073,6 +2080,21 @@ def _two_parts(ops, bs, H, group, k, sink, tail, keys, cand, form, scores=None):
     assert (ids.sort(dim=2).values.diff(dim=2) > 0).all() and int(ids.min()) >= 0 and int(ids.max()) < keys
     assert torch.equal(got, att.run(q, segs))
     _near_attention_in_64_bits(got, q, kk, vv, sink, keys, ids)
+    if not replays:
+        return
+    out = torch.zeros_like(q)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        plan.run(*args, out_ids=ids, attention=(att, segs, out), any_order=True)
+    for _ in range(replays):
+        q.copy_(torch.randn(q.shape, generator=g, device=DEV))
+        ids.zero_(), out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        got_ids, got = ids.clone(), out.clone()
+        torch.randn(1 << 20, device=DEV).sum().item()  # unrelated eager work between replays
+        assert torch.equal(got_ids, plan.run(*args, any_order=True))
+        assert torch.equal(got, att.run(q, segs))
 
 
 @pytest.mark.parametrize("k,keys,cand", [(100, 3000, 1500), (512, 3000, 1500), (100, 20000, 9001)])
