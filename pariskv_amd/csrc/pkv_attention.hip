@@ -61,6 +61,7 @@ __device__ __forceinline__ uint32_t att_resolve_row(const AttSegs &segs, int row
   }
   return (uint32_t)(r + row0) | ((uint32_t)s << 29);
 }
+
 // Keys row `row` attends to: all `total`, its own row_keys[row], or with uniform > 0 the largest of row_keys[0 .. uniform)
 // (the dense form of the adaptive-k step, where a launch of its own for the maximum took 4.5 us at 24 rows).
 __device__ __forceinline__ int64_t att_row_total(int64_t total, const int32_t *__restrict__ row_keys, int row, int uniform) {
@@ -78,6 +79,8 @@ __device__ __forceinline__ int64_t att_row_total(int64_t total, const int32_t *_
   }
   return rk < total ? (rk > 0 ? rk : 1) : total;
 }
+
+// The addresses of key jj's K and V rows; ROW: bytes of a row.
 template <bool INDEXED, uint32_t ROW>
 __device__ __forceinline__ AttPlace<false> att_place(const AttSegs &a, int row, int b, int h, uint32_t jj) {
   int s = 0;
@@ -125,6 +128,7 @@ __device__ __forceinline__ void load8(const void *base, int64_t elem_off, float 
 // it, not bandwidth.  Places of keys as in the bf16 kernel below.  Decode step, us, with a 64-bit pointer picked out of four for
 // each row / with places: 12 rows x 865 attended keys, 7 heads (2 layers) 74.6 / 70.0, 8 rows x 696 (2 layers) 66.5 / 61.0,
 // 32 rows x 896 48.6 / 45.2.
+//
 // grid (splits, rows, query heads by G)
 template <int G, bool INDEXED, typename SEGS>
 __global__ __launch_bounds__(kAttThreads) void pkv_attn_partial_kernel(const void *__restrict__ q, int n_kv_heads,
