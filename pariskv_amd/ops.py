@@ -31,7 +31,14 @@ def _p(t: Optional[torch.Tensor]):
     return t.data_ptr() if t is not None else None
 
 
+# The handle of a device's current stream, as the streams of torch.cuda hold it: 0.1 us a call, where current_stream builds a
+# Stream object in 1.9 us, a sixth of the host's part of a decode step.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor):
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
@@ -532,7 +539,7 @@ def gather_hbm(src_k, src_v, idx, dst_k, dst_v, idx_offset: int = 0, dst_row0: i
 class BoundAppend:
     """The destination of one layer's :func:`append_kv`, validated once: a token costs the checks of its own rows."""
 
-    __slots__ = ("_a", "_ra", "keep", "_shape", "_dtype", "_es", "_fn", "_device", "_slots")
+    __slots__ = ("_a", "_ra", "keep", "_shape", "_dtype", "_es", "_fn", "_slots")
 
     def __init__(self, dst_k, dst_v, vnorm: Optional[torch.Tensor] = None):
         bs, H, rows, D = dst_k.shape
@@ -545,7 +552,7 @@ class BoundAppend:
         self._a = _lib.AppendArgs(dst_k.data_ptr(), dst_v.data_ptr(), dst_k.stride(0) * es, dst_k.stride(1) * es, rows, bs, H,
                                   D * es, _p(vnorm), *(vnorm.stride()[:2] if vnorm is not None else (0, 0)))
         self._ra, self.keep = C.byref(self._a), (dst_k, dst_v, vnorm)
-        self._shape, self._dtype, self._es, self._device = (bs, 1, H, D), dst_k.dtype, es, dst_k.device
+        self._shape, self._dtype, self._es = (bs, 1, H, D), dst_k.dtype, es
         self._fn = _lib.lib().pkv_append_kv_run
         self._slots = rows if vnorm is None else min(rows, vnorm.shape[2])  # the kernel checks nothing: rows and norms have these
 
@@ -557,7 +564,7 @@ class BoundAppend:
         _need(k.dtype == self._dtype and v.dtype == self._dtype and 0 <= slot < self._slots,
               "append: dtypes differ, or the slot lies outside the K/V rows or the value norms")
         rc = self._fn(self._ra, k.data_ptr(), ks[0] * es, ks[2] * es, v.data_ptr(), vs[0] * es, vs[2] * es, slot,
-                      torch.cuda.current_stream(self._device).cuda_stream)
+                      _stream(self.keep[0]))
         if rc != 0:
             _lib.check(rc)
 
@@ -839,9 +846,9 @@ class BoundAttention:
               "queries must be contiguous [bs,1,Hq,128] of the cache dtype")
         out = torch.empty_like(q)
         self.aa.out = out.data_ptr()
-        stream = torch.cuda.current_stream(q.device)
-        handle = stream.cuda_stream
+        handle = _stream(q)
         if handle != self._told:
+            stream = torch.cuda.current_stream(q.device)
             for t in self._lent:
                 t.record_stream(stream)
             self._told = handle
@@ -872,7 +879,7 @@ class BoundStep:
               "queries must be contiguous [bs,1,Hq,128] of the cache dtype")
         out = torch.empty_like(q)
         self.a.q, self.aa.out = q.data_ptr(), out.data_ptr()
-        rc = self._fn(self._ra, self._ws, self._ws_bytes, self._raa, torch.cuda.current_stream(q.device).cuda_stream)
+        rc = self._fn(self._ra, self._ws, self._ws_bytes, self._raa, _stream(q))
         self.a.table_ready = 0  # a table left by qk_norm_rope(table_for=self) serves one launch
         if rc != 0:
             _lib.check(rc)
@@ -899,7 +906,7 @@ class BoundAdaptiveStep:
         out = torch.empty_like(q)
         self.a.q, self.aa.out = q.data_ptr(), out.data_ptr()
         rc = self._fn(self._ra, self._ws, self._ws_bytes, self._rad, self._raa,
-                      torch.cuda.current_stream(q.device).cuda_stream)
+                      _stream(q))
         self.a.table_ready = 0  # a table left by qk_norm_rope(table_for=self) serves one launch
         if rc != 0:
             _lib.check(rc)
