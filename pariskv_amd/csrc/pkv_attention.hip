@@ -417,16 +417,16 @@ bool as_one_tensor(const AttSegs &sg, int es, AttOne &one) {
 
 // One CU fetches scattered rows at 35 to 40 GB/s, 2.7 us for 200 of them and as much as the merge's launch: up to six blocks of 32
 // are one workgroup's, which then merges; more go to a workgroup per split of 128, each selecting anew, or per two or three where
-// that would be more workgroups than CUs; there up to eight blocks are one workgroup's as well.  Where the selection takes several
-// launches (more than 8192 candidates), only the first form: its last launch is too long to be run by several workgroups a row
-// (16 rows x 131072, top 200, 52.0 / 52.5).
+// that would be more workgroups than CUs; there up to eight blocks are one workgroup's as well.  More than 8192 candidates
+// take longer to select from: only the first form (several workgroups a row gain 0.6 of 43.5 us at 16 rows x 131072, top 1024, and
+// 1.7 of 55.4 at 200000: not built).
 // Decode step, us, attention after the top-k / in two parts, by one workgroup a row: 8 rows x 4096 keys, top 100, 25.5 / 23.5;
 // 32 x 16000, 8 heads, top 100, 31.6 / 30.8; 64 x 65536, top 100, 60.0 / 56.8; 256 x 8000, top 100, 74.0 / 66.0, top 256 80.3 / 70.8;
-// more than 8192 candidates: 8 x 100000, top 100, 47.2 / 45.7, 64 x 100000 96.7 / 94.2.  By several: 8 x 32768, top 512, 28.6 / 28.4;
-// 32 x 16000, 8 heads, top 512, 33.6 / 32.8; 64 x 40000, top 512, 52.6 / 51.4, top 1024 57.0 / 55.2.
+// more than 8192 candidates, where their selection took three launches: 8 x 100000, top 100, 47.2 / 45.7, 64 x 100000 96.7 / 94.2.
+// By several: 8 x 32768, top 512, 28.6 / 28.4; 32 x 16000, 8 heads, top 512, 33.6 / 32.8; 64 x 40000, top 512, 52.6 / 51.4, top 1024 57.0 / 55.2.
 // After the top-k / by one / by several, 40000 keys, 4000 candidates: six blocks, 8 rows 31.3 / 29.7 / 30.9, 32 rows 38.0 / 36.5 / 38.0,
 // 64 rows 51.4 / 49.0 / 49.8; eight, 16 rows 33.5 / 34.4 / 33.8, 64 rows 51.9 / 50.3 / 50.2.  After the top-k / by one, 100000 keys,
-// 9000 candidates: six blocks, 8 rows 47.2 / 45.9, 64 rows 94.6 / 93.0; eight, 16 rows 52.6 / 53.7.
+// 9000 candidates (selected in three launches): six blocks, 8 rows 47.2 / 45.9, 64 rows 94.6 / 93.0; eight, 16 rows 52.6 / 53.7.
 constexpr int kSplitWorkgroups = 256, kMergeBlocks = 6;
 constexpr int64_t kSplitMaxSelected = 1024;
 

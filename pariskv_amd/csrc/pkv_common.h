@@ -129,9 +129,10 @@ PKV_INTERNAL int pkv_launch_rerank(const int64_t *cand, int bs, int n_kv_heads, 
                                    int64_t ws_sub, const float *qhat, const float *qnorm, const float *centers,
                                    float *scores, uint16_t *v4b, hipStream_t s);
 PKV_INTERNAL size_t pkv_topk_ws_bytes_impl(int rows, int64_t len, int64_t k);
-PKV_INTERNAL int64_t pkv_topk_ctl_words(int rows, int64_t len);
+PKV_INTERNAL int64_t pkv_topk_ctl_words(int rows, int64_t len, int64_t k);
 PKV_INTERNAL uint32_t *pkv_topk_range_slots(uint32_t *ctl, int64_t len, int64_t *row_stride);
-constexpr int kTopkMaxSort = 8192;  // longest row that one workgroup selects from or sorts: 64 KB of 64-bit keys in LDS
+constexpr int kTopkMaxSort = 8192;  // longest row that one workgroup sorts, or selects from with whole keys in registers: 64 KB of 64-bit keys in LDS
+constexpr int kTopkMaxSelect = 32768;  // longest row that one workgroup selects from: scores and bins of 32 keys a thread in registers
 struct PkvSplitAttn;
 // attn (or null): the launch that ends the selection goes on with the attention over it (pkv_topk_attends(len, k))
 PKV_INTERNAL int pkv_launch_topk_f32(const float *x, int64_t x_stride, const int64_t *ids, int64_t ids_stride,

@@ -66,7 +66,7 @@ WsLayout layout(int rows, int64_t n_keys, int64_t n_cand, int64_t k, int least_c
   w.cand_extra = take((size_t)rows * (size_t)n_cand * sizeof(float));  // record word passed through per candidate
   // the top-k's control area (range slots; for wide rows the control blocks and lists of the multi-workgroup form)
   w.topk_bytes = pkv_topk_ws_bytes_impl(rows, n_cand, k);
-  const size_t ctl_bytes = pkv_align_up((size_t)pkv_topk_ctl_words(rows, n_cand) * 4, 256);
+  const size_t ctl_bytes = pkv_align_up((size_t)pkv_topk_ctl_words(rows, n_cand, k) * 4, 256);
   if (w.topk_bytes < ctl_bytes) w.topk_bytes = ctl_bytes;
   w.topk = take(w.topk_bytes);
   // flags and status word of the one-launch form of the first three stages
@@ -171,10 +171,10 @@ static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, 
   PKV_REQUIRE(nk >= 64 && nk % 16 == 0 && wk >= 16 && wk % 8 == 0,
               "key strides of %lld / %lld bytes: nibbles need >= 64, weights >= 32, multiples of 16",
               (long long)a->nib_key_stride, (long long)a->weight_key_stride);
-  // the top-k takes the rows' score ranges from its control area (and a multi-workgroup top-k, more than 8192
-  // candidates, wants its control blocks cleared): the first launch of the step clears, the select + rerank launch
+  // the top-k takes the rows' score ranges from its control area (and a multi-workgroup top-k, see
+  // pkv_launch_topk_f32, wants its control blocks cleared): the first launch of the step clears, the select + rerank launch
   // leaves the ranges
-  const int64_t ctl_words = a->out_ids && a->n_cand != a->n_keys ? pkv_topk_ctl_words(rows, a->n_cand) : 0;
+  const int64_t ctl_words = a->out_ids && a->n_cand != a->n_keys ? pkv_topk_ctl_words(rows, a->n_cand, a->k) : 0;
   uint32_t *topk_ctl = ctl_words ? (uint32_t *)(base + w.topk) : nullptr;
   int64_t range_stride = 0;
   uint32_t *range_slots = topk_ctl ? pkv_topk_range_slots(topk_ctl, a->n_cand, &range_stride) : nullptr;
@@ -269,7 +269,7 @@ extern "C" int pkv_qk_norm_rope_table(const void *qkv, int64_t stride_b, int n_q
   memset(&t, 0, sizeof t);
   t.n = a->n_tiers;
   for (int i = 0; i < a->n_tiers; ++i) t.t[i] = a->tier_counts[i];
-  const int64_t ctl_words = a->out_ids && a->n_cand != a->n_keys ? pkv_topk_ctl_words(rows, a->n_cand) : 0;
+  const int64_t ctl_words = a->out_ids && a->n_cand != a->n_keys ? pkv_topk_ctl_words(rows, a->n_cand, a->k) : 0;
   return pkv_launch_qk_norm_rope_table(qkv, stride_b, a->bs, n_q_heads, a->n_kv_heads, q_weight, k_weight, eps, cos_row,
                                        sin_row, q_out, k_out, a->signs, a->cluster_counts, t, (float *)(base + w.qhat),
                                        (float *)(base + w.qnorm), (uint8_t *)(base + w.lut), (uint32_t *)(base + w.rowsuf),

@@ -737,46 +737,32 @@ __device__ __forceinline__ uint32_t lin_bin(uint64_t key, const LinSel &L) {
   return b > (uint32_t)(kLinBins - 1) ? (uint32_t)(kLinBins - 1) : b;
 }
 
-// Bins of the thread's keys and the threshold bin.  On return s_hist[0,kLinBins) = keys per bin, s_hist[kLinBins,2*kLinBins) =
-// off[b] = keys in the bins above b, s_cnt[b] = off[b] (a running output slot for the counting sort), s_bcast[6] = 0.
-// s_hist: 2*kLinBins words, s_cnt: kLinBins words, s_bcast: 8 words.  All 1024 threads call it; false = not applicable.
-// BITS: bins of the ordered key bits instead of the values, for rows of one sign whose values span many binades
-// (e.g. the winners of a selection, about to be sorted): kLinBins equal steps of the bit pattern between the row's
-// smallest and largest key, i.e. equal steps of the logarithm up to the mantissa's linear pieces.
-// range: null, or the largest and the smallest ordered score of the nonzero keys (range[0] < range[1]: no key at
-// all) where the caller knows them already, which saves the reduction that finds them.
-template <int EIN, bool BITS = false>
-__device__ __forceinline__ bool linear_bins(const uint64_t (&v)[EIN], uint32_t k, uint32_t *s_hist, uint32_t *s_cnt,
-                                            uint32_t *s_bcast, uint32_t (&bin)[EIN], LinSel &L,
-                                            const uint32_t *range = nullptr) {
-  const int tid = threadIdx.x, lane = pkv_lane();
+// The steps of the binning.  s_hist: 2*kLinBins words, s_cnt: kLinBins words, s_bcast: 8 words; all 1024 threads call each.
+// Clear; a barrier follows.
+__device__ __forceinline__ void lin_clear(uint32_t *s_hist, uint32_t *s_bcast) {
+  const int tid = threadIdx.x;
   for (int i = tid; i < 2 * kLinBins; i += kTopkThreads) s_hist[i] = 0;
   // [2..4]: threshold bin, keys needed from it, keys in it.  They are set below only if some bin reaches k; a row
   // with fewer than k keys leaves "keys in the threshold bin" at its all-ones start and the caller falls back.
   if (tid == 0)
     s_bcast[0] = 0u, s_bcast[1] = 0xffffffffu, s_bcast[2] = 0u, s_bcast[3] = 0u, s_bcast[4] = 0xffffffffu, s_bcast[5] = 0u,
     s_bcast[6] = 0u;
-  __syncthreads();
-  uint32_t mx = 0u, mn = 0xffffffffu;
-  if (range) {
-    mx = range[0], mn = range[1];
-  } else {
-#pragma unroll
-  for (int e = 0; e < EIN; ++e) {
-    if (v[e] != 0ull) {
-      const uint32_t hi = (uint32_t)(v[e] >> 32);
-      mx = hi > mx ? hi : mx;
-      mn = hi < mn ? hi : mn;
-    }
-  }
+}
+
+// Largest and smallest ordered score of the workgroup from the threads' own.  One barrier.
+__device__ __forceinline__ void lin_range(uint32_t &mx, uint32_t &mn, uint32_t *s_bcast) {
   mx = pkv_wave_max(mx), mn = ~pkv_wave_max(~mn);
-  if (lane == 0) {
+  if (pkv_lane() == 0) {
     atomicMax(&s_bcast[0], mx);
     atomicMin(&s_bcast[1], mn);
   }
   __syncthreads();
   mx = s_bcast[0], mn = s_bcast[1];
-  }
+}
+
+// The bins of that range; false = not applicable.
+template <bool BITS>
+__device__ __forceinline__ bool lin_steps(uint32_t mx, uint32_t mn, LinSel &L) {
   L.lo = 0.f, L.scale = 0.f, L.lo_bits = mn, L.shift = -1;
   if (BITS) {
     if (mx <= mn) return false;  // one value (or no key at all)
@@ -790,15 +776,12 @@ __device__ __forceinline__ bool linear_bins(const uint64_t (&v)[EIN], uint32_t k
     if (!(mx < 0xff800000u && mn > 0x007fffffu && range > 0.f && range < inf && scale < inf)) return false;
     L.lo = lo, L.scale = scale;
   }
-#pragma unroll
-  for (int e = 0; e < EIN; ++e) {
-    bin[e] = 0;
-    if (v[e] != 0ull) {
-      bin[e] = lin_bin(v[e], L);
-      atomicAdd(&s_hist[bin[e]], 1u);
-    }
-  }
-  __syncthreads();
+  return true;
+}
+
+// Threshold bin and output slots from the histogram (a barrier lies before this).  One barrier.
+__device__ __forceinline__ bool lin_decide(uint32_t k, uint32_t *s_hist, uint32_t *s_cnt, uint32_t *s_bcast, LinSel &L) {
+  const int tid = threadIdx.x;
   if (tid < PKV_WAVE) {  // lane l owns the kPer bins below kLinBins - kPer * l: an inclusive scan over lanes is the suffix sum over bins
     constexpr int kPer = kLinBins / PKV_WAVE;
     uint32_t h[kPer];
@@ -837,6 +820,47 @@ __device__ __forceinline__ bool linear_bins(const uint64_t (&v)[EIN], uint32_t k
   L.bstar = s_bcast[2], L.need = s_bcast[3], L.in_bstar = s_bcast[4], L.max_winners = s_bcast[5];
   L.T = 0ull;
   return L.in_bstar <= kLinBucketMax;
+}
+
+// Bins of the thread's keys and the threshold bin.  On return s_hist[0,kLinBins) = keys per bin, s_hist[kLinBins,2*kLinBins) =
+// off[b] = keys in the bins above b, s_cnt[b] = off[b] (a running output slot for the counting sort), s_bcast[6] = 0.
+// All 1024 threads call it; false = not applicable.
+// BITS: bins of the ordered key bits instead of the values, for rows of one sign whose values span many binades
+// (e.g. the winners of a selection, about to be sorted): kLinBins equal steps of the bit pattern between the row's
+// smallest and largest key, i.e. equal steps of the logarithm up to the mantissa's linear pieces.
+// range: null, or the largest and the smallest ordered score of the nonzero keys (range[0] < range[1]: no key at
+// all) where the caller knows them already, which saves the reduction that finds them.
+template <int EIN, bool BITS = false>
+__device__ __forceinline__ bool linear_bins(const uint64_t (&v)[EIN], uint32_t k, uint32_t *s_hist, uint32_t *s_cnt,
+                                            uint32_t *s_bcast, uint32_t (&bin)[EIN], LinSel &L,
+                                            const uint32_t *range = nullptr) {
+  lin_clear(s_hist, s_bcast);
+  __syncthreads();
+  uint32_t mx = 0u, mn = 0xffffffffu;
+  if (range) {
+    mx = range[0], mn = range[1];
+  } else {
+#pragma unroll
+    for (int e = 0; e < EIN; ++e) {
+      if (v[e] != 0ull) {
+        const uint32_t hi = (uint32_t)(v[e] >> 32);
+        mx = hi > mx ? hi : mx;
+        mn = hi < mn ? hi : mn;
+      }
+    }
+    lin_range(mx, mn, s_bcast);
+  }
+  if (!lin_steps<BITS>(mx, mn, L)) return false;
+#pragma unroll
+  for (int e = 0; e < EIN; ++e) {
+    bin[e] = 0;
+    if (v[e] != 0ull) {
+      bin[e] = lin_bin(v[e], L);
+      atomicAdd(&s_hist[bin[e]], 1u);
+    }
+  }
+  __syncthreads();
+  return lin_decide(k, s_hist, s_cnt, s_bcast, L);
 }
 
 // Threshold key of bin b*: the need-th largest of its keys, found by counting with 16 lanes per key.
@@ -1219,6 +1243,149 @@ __device__ __forceinline__ void topk_select_sort(const float *__restrict__ x, in
 #undef PKV_SORT_K
 }
 
+// The same for rows of 8193 to 32768 keys and k <= 2048, sorted, EIN = 16 or 32 keys a thread.  The registers hold the scores and
+// their bins, two to a word; ids are read for the winners and the threshold bin alone, in one round trip with what the caller
+// requests.  One CU reads its row's scores at some 130 GB/s, 0.8 us for 26000, and runs eight steps between barriers; the three
+// launches of the wide form read scores and ids twice and take 5 to 7 us each.  Where the bins do not apply, the radix select and
+// the sort of that form.  Dynamic LDS: max(P, 1024) keys; s_sel lies elsewhere.  more(): the caller's own requests.
+template <int EIN, typename Requests>
+__device__ __forceinline__ void topk_select_long(const float *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ ids,
+                                                 int64_t ids_stride, int len, int P, int64_t k, int64_t *__restrict__ out_ids,
+                                                 float *__restrict__ out_vals, uint32_t *s_sel, Requests more) {
+  extern __shared__ uint64_t s_keys[];
+  __shared__ SelSmem sm;
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const float *xr = x + (int64_t)row * x_stride;
+  const int64_t *ir = ids ? ids + (int64_t)row * ids_stride : nullptr;
+  int64_t *oi = out_ids + (int64_t)row * k;
+  float *ov = out_vals ? out_vals + (int64_t)row * k : nullptr;
+  uint32_t ord[EIN], bins[EIN / 2];
+#pragma unroll
+  for (int e = 0; e < EIN; ++e) {
+    const int i = tid + e * kTopkThreads;
+    ord[e] = __float_as_uint(xr[i < len ? i : len - 1]);
+  }
+  // 16 keys a thread leave registers for the caller's requests at once, 32 only when scores and bins are done with: 8 rows x
+  // 131072 keys, top 100, 33.8 / 33.2 us a step late / at once; 262144 keys 47.1 / 48.4
+  constexpr bool kEarly = EIN <= 16;
+  if (kEarly) more();
+  const int n_mine = (len - tid + kTopkThreads - 1) / kTopkThreads;  // of the thread's keys; the others repeat the row's last
+  lin_clear(sm.hist, sm.bcast);
+  __syncthreads();
+  uint32_t mx = 0u, mn = 0xffffffffu;
+#pragma unroll
+  for (int e = 0; e < EIN; ++e) {
+    ord[e] = pkv_ordered_u32(__uint_as_float(ord[e]));
+    mx = ord[e] > mx ? ord[e] : mx;
+    mn = ord[e] < mn ? ord[e] : mn;
+  }
+  lin_range(mx, mn, sm.bcast);
+  LinSel L;
+  bool lin = lin_steps<false>(mx, mn, L);  // uniform over the workgroup
+  if (lin) {
+#pragma unroll
+    for (int e = 0; e < EIN; e += 2) {
+      const uint32_t b0 = lin_bin((uint64_t)ord[e] << 32, L), b1 = lin_bin((uint64_t)ord[e + 1] << 32, L);
+      bins[e / 2] = b0 | b1 << 16;
+      if (e < n_mine) atomicAdd(&sm.hist[b0], 1u);
+      if (e + 1 < n_mine) atomicAdd(&sm.hist[b1], 1u);
+    }
+    __syncthreads();
+    lin = lin_decide((uint32_t)k, sm.hist, sm.cnt, sm.bcast, L) && L.max_winners <= kLinRankMax;
+  }
+  if (!lin) {
+    if (!kEarly) more();
+    auto key_of = [&](int64_t i) { return make_key(xr, ir, i); };
+    uint64_t prefix;
+    int shift;
+    __syncthreads();
+    radix_select_streamed(key_of, len, (uint32_t)k, sm.hist, sm.bcast, prefix, shift);
+    for (int i = tid; i < (P < 1024 ? 1024 : P); i += kTopkThreads) s_keys[i] = 0ull;
+    if (tid == 0) sm.counter = 0;
+    __syncthreads();
+    collect_winners_streamed(key_of, len, (uint32_t)k, prefix, shift, &sm.counter, s_keys);
+    __syncthreads();
+    if (P <= 1024) sort_lds_keys_and_emit<1024, 1>(s_keys, k, oi, ov, s_sel ? s_keys : nullptr);
+    else sort_lds_keys_and_emit<1024, 2>(s_keys, k, oi, ov, s_sel ? s_keys : nullptr);
+    if (s_sel)
+      for (int i = tid; i < (int)k; i += kTopkThreads) s_sel[i] = ~(uint32_t)s_keys[i];
+    return;
+  }
+  // counting sort as in topk_select_sort, the keys with their positions in the row first
+  const uint32_t n_above = (uint32_t)k - L.need;
+#pragma unroll
+  for (int e = 0; e < EIN; ++e) {
+    const uint32_t bin = (e & 1) ? bins[e / 2] >> 16 : bins[e / 2] & 0xffffu;
+    if (e < n_mine && bin >= L.bstar) {
+      const uint64_t key = (uint64_t)ord[e] << 32 | (uint32_t)(tid + e * kTopkThreads);
+      if (bin > L.bstar) s_keys[atomicAdd(&sm.cnt[bin], 1u)] = key;
+      else sm.bucket[atomicAdd(&sm.bcast[6], 1u)] = key;
+    }
+  }
+  __syncthreads();
+  if (!kEarly) more();
+  {  // ... then with their ids
+    constexpr int kOut = kCountingSortMaxP / kTopkThreads;
+    uint64_t key[kOut + 1];
+    uint32_t id[kOut + 1];
+#pragma unroll
+    for (int u = 0; u <= kOut; ++u) {
+      const uint32_t p = (uint32_t)(tid + (u < kOut ? u : 0) * kTopkThreads);
+      key[u] = u < kOut ? (p < n_above ? s_keys[p] : 0ull) : (p < L.in_bstar ? sm.bucket[p] : 0ull);
+      id[u] = ir ? (uint32_t)ir[(uint32_t)key[u]] : (uint32_t)key[u];
+    }
+#pragma unroll
+    for (int u = 0; u <= kOut; ++u) {
+      const uint32_t p = (uint32_t)(tid + (u < kOut ? u : 0) * kTopkThreads);
+      const uint64_t whole = (key[u] & 0xffffffff00000000ull) | (uint64_t)(uint32_t)~id[u];
+      if (u < kOut && p < n_above) s_keys[p] = whole;
+      if (u == kOut && p < L.in_bstar) sm.bucket[p] = whole;
+    }
+  }
+  __syncthreads();
+  auto emit = [&](uint32_t at, uint64_t key) {
+    oi[at] = (int64_t)(uint32_t)(~(uint32_t)key);
+    if (s_sel) s_sel[at] = ~(uint32_t)key;
+    if (ov) ov[at] = pkv_from_ordered_u32((uint32_t)(key >> 32));
+  };
+  const uint32_t *s_off = sm.hist + kLinBins;
+  for (uint32_t p = tid; p < n_above; p += kTopkThreads) {
+    const uint64_t key = s_keys[p];
+    const uint32_t b = lin_bin(key, L);
+    const uint32_t start = s_off[b], cnt = sm.cnt[b] - start;
+    uint32_t r = 0;
+#pragma unroll 4
+    for (uint32_t j = 0; j < cnt; ++j) r += s_keys[start + j] > key ? 1u : 0u;
+    emit(start + r, key);
+  }
+  rank_bucket_desc(sm.bucket, L.in_bstar, [&](uint64_t key, uint32_t r) {
+    if (r < L.need) emit(n_above + r, key);
+  });
+}
+
+template <int EIN>
+__global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_long_kernel(
+    const float *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ ids, int64_t ids_stride, int len, int P,
+    int64_t k, int64_t *__restrict__ out_ids, float *__restrict__ out_vals) {
+  topk_select_long<EIN>(x, x_stride, ids, ids_stride, len, P, k, out_ids, out_vals, nullptr, [] {});
+}
+
+// ... and the attention over the winners, merged: see pkv_topk_attend_kernel.  Dynamic LDS: max(P, 1024) keys, then k words.
+template <int EIN>
+__global__ __launch_bounds__(kTopkThreads) void pkv_topk_long_attend_kernel(
+    const float *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ ids, int64_t ids_stride, int len, int P, int64_t k,
+    int64_t *__restrict__ out_ids, float *__restrict__ out_vals, PkvSplitAttn attn) {
+  extern __shared__ uint64_t s_keys[];
+  __shared__ AttSelSmem sm;
+  const int row = blockIdx.x;
+  uint32_t *s_sel = (uint32_t *)(s_keys + (P < 1024 ? 1024 : P));
+  AttSelRequests req;
+  att_clear(sm);
+  topk_select_long<EIN>(x, x_stride, ids, ids_stride, len, P, k, out_ids, out_vals, s_sel, [&] { att_request(attn, row, req); });
+  __syncthreads();
+  att_selected<true>(attn, row, s_sel, 0, sm, req);
+}
+
 template <int EIN, bool SORTED>
 __global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_sort_kernel(
     const float *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ ids, int64_t ids_stride, int len, int P,
@@ -1246,7 +1413,7 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_attend_kernel(
 
 // ------------------------------------------------- rows wider than one workgroup
 //
-// More than 8192 keys in a row: the row is cut into slices of 8192 keys, one workgroup (8 keys per
+// More than 8192 keys in a row (and more than topk_selects_long takes): the row is cut into slices of 8192 keys, one workgroup (8 keys per
 // thread) each, and the k winners are found in three steps.
 //   histogram  every slice adds bits [BINSHIFT, BINSHIFT+11) of its 64-bit keys to a 2048-bin
 //              histogram of the row: in LDS first, then one global atomic per non-empty bin;
@@ -2308,10 +2475,26 @@ static WideWs wide_ws_layout(int rows, int64_t len, int64_t k, size_t off) {
   return w;
 }
 
+// Rows that one workgroup selects from, well short of all their keys (anything else sorts the row or spreads it).
+static bool topk_selects(int64_t len, int64_t k) {
+  return len <= kTopkMaxSort && pow2_ceil(k) * 2 <= pow2_ceil(len) && pow2_ceil(len) >= 2048;
+}
+
+// ... and the longer ones it selects from with fewer registers a key.  k <= 2048: two winners a thread, and the sort's list in 16 KB
+// of LDS.  Decode step, us, by the wide form / by one workgroup a row: 8 rows x 131072 keys (13050 candidates), top 100, 43.2 / 31.7,
+// 40 x 90000 (8943), top 100, 61.6 / 49.5, 64 x 90000, top 1024, 88.0 / 76.9, 16 x 131072, top 1024, 53.9 / 43.5, K/V on the host
+// 214.1 / 203.4; 17 to 32 keys a thread: 16 x 200000 (19942) 62.1 / 55.4, 8 x 262144 (26157), top 100, 51.0 / 42.6, fp32, top 1024,
+// 58.2 / 52.8.  With whole keys and ids in registers 16 a thread gave 34.7 at the first shape and 32 spilled (71.7 at 262144).
+static bool topk_selects_long(int64_t len, int64_t k) {
+  return len > kTopkMaxSort && len <= kTopkMaxSelect && pow2_ceil(k) <= kCountingSortMaxP;
+}
+
 // Words at the start of pkv_topk_f32's workspace that must be zero when its first launch starts (0: none).
 // (Handing the range to the one-workgroup kernel as well was measured: its min/max pass is cheaper than the
 // producer's extra epilogue, +0.6 us on the step at 32 rows x 4096 candidates.)
-int64_t pkv_topk_ctl_words(int rows, int64_t len) { return len > kTopkMaxSort ? (int64_t)rows * kWideRowWords : 0; }
+int64_t pkv_topk_ctl_words(int rows, int64_t len, int64_t k) {
+  return len > kTopkMaxSort && !topk_selects_long(len, k) ? (int64_t)rows * kWideRowWords : 0;
+}
 // Where a producer's workgroups leave their (max, ~min) in that area, and the distance between rows in words.
 uint32_t *pkv_topk_range_slots(uint32_t *ctl, int64_t len, int64_t *row_stride) {
   (void)len;
@@ -2328,12 +2511,7 @@ extern "C" size_t pkv_topk_f32_ws_bytes(int rows, int64_t len, int64_t k) {
   return pkv_topk_ws_bytes_impl(rows, len, k);
 }
 
-// Rows that one workgroup selects from, well short of all their keys (anything else sorts the row or spreads it).
-bool pkv_topk_selects(int64_t len, int64_t k) {
-  return len <= kTopkMaxSort && pow2_ceil(k) * 2 <= pow2_ceil(len) && pow2_ceil(len) >= 2048;
-}
-
-bool pkv_topk_attends(int64_t len, int64_t k) { return pkv_topk_selects(len, k) || (len > kTopkMaxSort && pow2_ceil(k) <= kCountingSortMaxP); }
+bool pkv_topk_attends(int64_t len, int64_t k) { return topk_selects(len, k) || (len > kTopkMaxSort && pow2_ceil(k) <= kCountingSortMaxP); }
 
 static int launch_topk_attend(const float *x, int64_t x_stride, const int64_t *ids, int64_t ids_stride, int rows, int64_t len,
                               int64_t k, int64_t *out_ids, float *out_vals, const PkvSplitAttn &attn, hipStream_t s) {
@@ -2363,10 +2541,10 @@ int pkv_launch_topk_f32(const float *x, int64_t x_stride, const int64_t *ids, in
   PKV_REQUIRE(rows > 0 && rows <= 65535 && len < ((int64_t)1 << 31), "bad shape rows=%d len=%lld", rows, (long long)len);
   PKV_REQUIRE(!attn || (pkv_topk_attends(len, k) && (len <= kTopkMaxSort || attn->sel_wgs == 1)),
               "no attention goes with a top-k of %lld out of %lld", (long long)k, (long long)len);
-  if (attn && pkv_topk_selects(len, k)) {
+  if (attn && topk_selects(len, k)) {
     return launch_topk_attend(x, x_stride, ids, ids_stride, rows, len, k, out_ids, out_vals, *attn, s);
   }
-  if (pkv_topk_selects(len, k)) {
+  if (topk_selects(len, k)) {
     const int P = pow2_ceil(k);
     const int ein = pow2_ceil(len) / kTopkThreads;
 #define PKV_SEL(EIN, SORTED)                                                                                      \
@@ -2395,6 +2573,22 @@ int pkv_launch_topk_f32(const float *x, int64_t x_stride, const int64_t *ids, in
       pkv_set_error("pkv_topk_f32: rows of more than %d keys need a workspace of %zu bytes (256-aligned), got %zu",
                     kTopkMaxSort, need, ws_bytes);
       return PKV_ENOMEM;
+    }
+    if (topk_selects_long(len, k)) {
+      const int P = pow2_ceil(k);
+#define PKV_SEL(EIN)                                                                                                            \
+  do {                                                                                                                          \
+    if (attn)                                                                                                                   \
+      hipLaunchKernelGGL(pkv_topk_long_attend_kernel<EIN>, dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes(P) + (size_t)k * 4, \
+                         s, x, x_stride, ids, ids_stride, (int)len, P, k, out_ids, out_vals, *attn);                            \
+    else                                                                                                                        \
+      hipLaunchKernelGGL(pkv_topk_select_long_kernel<EIN>, dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes(P), s, x, x_stride, \
+                         ids, ids_stride, (int)len, P, k, out_ids, out_vals);                                                   \
+  } while (0)
+      if (len <= 2 * kTopkMaxSort) PKV_SEL(16); else PKV_SEL(32);
+#undef PKV_SEL
+      PKV_LAUNCH_CHECK("pkv_topk_select_long_kernel");
+      return PKV_OK;
     }
     const WideWs w = wide_ws_layout(rows, len, k, 0);
     uint32_t *ctl = (uint32_t *)((char *)ws + w.ctl);

@@ -2125,3 +2125,47 @@ def test_decode_step_with_one_scratch_buffer(ops, k, keys, cand):
     for _ in range(3):
         ids, got = step(d["queries"])
         assert torch.equal(ids, want_ids) and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rows,L,k", [(3, 8193, 1), (2, 8193, 2048), (2, 16384, 2048), (2, 16385, 100), (2, 24577, 1025), (2, 32767, 1024),
+                                      (2, 32768, 2048), (2, 32769, 100), (300, 9000, 64)])
+@pytest.mark.parametrize("kind", ["spread", "ties", "few values", "crowded bin", "constant", "infinite", "nan", "lowest"])
+def test_topk_f32_of_long_rows(ops, rows, L, k, kind):
+    """Rows of 8193 to 32768 scores, which one workgroup selects from: both ends of its two forms, a last thread without all its keys,
+    and scores that the bins of their range do not separate.  Ids and scores exactly as the oracle's, ties by id."""
+    _say(f"topk_f32 long {rows}x{L} k={k} {kind}")
+    rng = np.random.default_rng(L + k)
+    x = (rng.standard_normal((rows, L)) * 10 + 3).astype(np.float32)
+    if kind == "ties":
+        x = np.round(x * 8).astype(np.float32) / 8
+    elif kind == "few values":
+        x = rng.integers(0, 4, (rows, L)).astype(np.float32)
+    elif kind == "crowded bin":
+        x[:, 50:50 + 400] = np.float32(90.0)
+        x[:, 9:L:3] = np.float32(12.0)
+    elif kind == "constant":
+        x[:] = np.float32(-2.5)
+    elif kind == "infinite":
+        x[:, ::1000], x[0, 7] = np.inf, -np.inf
+    elif kind == "nan":
+        x[:, 11::2000] = np.nan
+    elif kind == "lowest":
+        x[:, L // 2:] = np.finfo(np.float32).min
+    some = sorted({0, rows // 2, rows - 1})
+    ids = np.stack([rng.permutation(2 * L)[:L] for _ in range(rows)]).astype(np.int64)
+    out, vals = ops.topk_f32(torch.from_numpy(x).to(DEV), k, torch.from_numpy(ids).to(DEV), want_values=True)
+    pos = ops.topk_f32(torch.from_numpy(x).to(DEV), k)
+    torch.cuda.synchronize()
+    for r in some:
+        ref_ids, ref_pos = O.topk_f32(x[r], ids[r], k)
+        assert np.array_equal(out[r].cpu().numpy(), ref_ids)
+        assert np.array_equal(vals[r].cpu().numpy().view(np.uint32), x[r][ref_pos].view(np.uint32))
+        assert np.array_equal(pos[r].cpu().numpy(), O.topk_f32(x[r], None, k)[1])
+
+
+@pytest.mark.parametrize("scores", [None, "equal", "infinite"])
+@pytest.mark.parametrize("bs,group,k,keys,cand", [(2, 4, 100, 40000, 16384), (1, 8, 192, 40000, 16385), (2, 3, 1, 60000, 32768)])
+def test_decode_step_merges_after_the_selection_from_a_long_row(ops, bs, group, k, keys, cand, scores):
+    """The attention behind that selection, in the selecting workgroup: as top-k and attention called one by one, bit for bit."""
+    _say(f"two-part attention behind a long row, {bs} x 2 rows group {group} k {k} candidates {cand} of {keys} scores {scores}")
+    _two_parts(ops, bs, 2, group, k, 64, 300, keys, cand, 1, scores, replays=3 if scores is None else 0)
