@@ -599,60 +599,57 @@ __device__ __forceinline__ void pkv_build_prod_table(float *s_prod, const float 
 
 typedef const __attribute__((address_space(3))) float *pkv_lds_cfloat_ptr;
 
-__device__ __forceinline__ float pkv_block_dot(const float *__restrict__ s_prod, int blk, uint32_t word) {
-  // the table always lives in LDS: say so, or the 128 reads become flat loads with 64-bit addresses
-  const pkv_lds_cfloat_ptr lp = (pkv_lds_cfloat_ptr)s_prod;
-  float t = 0.f;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const float prod = lp[(8 * blk + j) * 16 + ((word >> (4 * j)) & 15u)];
-    t = (j == 0) ? prod : t + prod;
-  }
-  return t;
-}
-
-// Score of one key stored key-major: 64 B of nibbles at np, 16 bf16 weights at wp (both 16-byte aligned; in the
-// cache's layout the two sit in one 128-byte record, so a candidate costs one HBM line).
-// Order: dims 0..7 inside a block, blocks 0..15, then * ||q||; multiply and add rounded separately.
-// The four 16-byte groups are walked by a rolled loop that rotates the data registers, so that only one
-// group's 32 table reads are in flight at a time (fully unrolled, the scheduler hoists all 128 reads and
-// the kernel needs ~170 registers).
-// LDS byte address base + 4 * (nibble of `word` at bit `shift`): a bit-field extract and a shift-and-add.  Written
-// out because the compiler turns the same expression into shift, mask and add (three instructions, 128 times per key).
-__device__ __forceinline__ uint32_t pkv_nibble_lds_addr(uint32_t word, int shift, uint32_t base) {
-  uint32_t a;
-  asm("v_bfe_u32 %0, %1, %2, 4\n\tv_lshl_add_u32 %0, %0, 2, %3" : "=&v"(a) : "v"(word), "s"(shift), "s"(base));
-  return a;
-}
-
-__device__ __forceinline__ float pkv_rerank_keymajor(const float *__restrict__ s_prod, const pkv_u32x4 *__restrict__ np,
-                                                     const pkv_u32x4 *__restrict__ wp, float qnorm) {
-  pkv_u32x4 n0 = np[0], n1 = np[1], n2 = np[2], n3 = np[3];
-  pkv_u32x4 w0 = wp[0], w1 = wp[1];
+// Score of one key before the query's norm: words[blk] the nibbles of block blk, weight(blk) its weight.  Order: dims 0..7 inside a
+// block, blocks 0..15; multiply and add rounded separately.
+// Bound by vector issue where candidates are many: two instructions a dimension, the table's byte offset 4 * nibble (even and odd
+// nibbles of a word are masked apart once, then each is one bit-field extract that takes two cleared bits along; the place of the
+// dimension's row is the read's immediate offset) and the addition.  With a third, an addition for the row's place, a step of 64
+// rows x 65536 keys took 52.4 us (51.6), 64 x 9000 34.2 (33.7).  Four groups of four blocks, one group's 32 table reads in flight
+// at a time (all 128, as the scheduler would have them, take 180 registers; the next group's reads before this one's additions 123:
+// no gain there, and 5 us lost at 8 rows x 1 M keys).
+template <typename Weight>
+__device__ __forceinline__ float pkv_rerank_words(const float *__restrict__ s_prod, uint32_t (&words)[16], Weight weight) {
+  // the table always lives in LDS: say so, or the reads become flat loads with 64-bit addresses
   const pkv_lds_cfloat_ptr lp = (pkv_lds_cfloat_ptr)s_prod;
   float s = 0.f;
-#pragma unroll 1
+#pragma unroll
   for (int u = 0; u < 4; ++u) {
-    const uint32_t words[4] = {n0.x, n0.y, n0.z, n0.w};
-    const uint32_t wpair[2] = {w0.x, w0.y};
-    const uint32_t group_base = (uint32_t)(uintptr_t)(lp + 512 * u);  // LDS byte address of this group's 32 table rows
+    // this group's addresses wait for the last one's sum
+    if (u > 0) asm("" : "+v"(words[4 * u]), "+v"(words[4 * u + 1]), "+v"(words[4 * u + 2]), "+v"(words[4 * u + 3]) : "v"(s));
+    float prod[4][8];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      float t = 0.f;
+      uint32_t even = words[4 * u + i] & 0x0f0f0f0fu, odd = words[4 * u + i] & 0xf0f0f0f0u;
+      asm("" : "+v"(even), "+v"(odd));  // as masked: else every extract becomes a shift and a mask again
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float prod = ((pkv_lds_cfloat_ptr)(uintptr_t)pkv_nibble_lds_addr(words[i], 4 * j, group_base))[(8 * i + j) * 16];
-        t = (j == 0) ? prod : t + prod;
+        const uint32_t at = j == 0 ? (even << 2) & 0x3cu : __builtin_amdgcn_ubfe(j & 1 ? odd : even, 4 * j - 2, 6);
+        prod[i][j] = *(pkv_lds_cfloat_ptr)((const __attribute__((address_space(3))) char *)(lp + (32 * u + 8 * i + j) * 16) + at);
       }
-      const uint32_t wb = (i & 1) ? (wpair[i >> 1] >> 16) : (wpair[i >> 1] & 0xffffu);
-      const float tw = t * pkv_bf16_bits_to_f32(wb);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float t = prod[i][0];
+#pragma unroll
+      for (int j = 1; j < 8; ++j) t = t + prod[i][j];
+      const float tw = t * weight(4 * u + i);
       s = (u == 0 && i == 0) ? tw : s + tw;
     }
-    n0 = n1, n1 = n2, n2 = n3;
-    w0 = pkv_u32x4{w0.z, w0.w, w1.x, w1.y};
-    w1 = pkv_u32x4{w1.z, w1.w, 0u, 0u};
   }
-  return s * qnorm;
+  return s;
+}
+
+// ... of a key stored key-major, with the norm: 64 B of nibbles at np, 16 bf16 weights at wp (both 16-byte aligned; in the
+// cache's layout the two sit in one 128-byte record, so a candidate costs one HBM line).
+__device__ __forceinline__ float pkv_rerank_keymajor(const float *__restrict__ s_prod, const pkv_u32x4 *__restrict__ np,
+                                                     const pkv_u32x4 *__restrict__ wp, float qnorm) {
+  const pkv_u32x4 n0 = np[0], n1 = np[1], n2 = np[2], n3 = np[3], w0 = wp[0], w1 = wp[1];
+  uint32_t words[16] = {n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, n1.z, n1.w, n2.x, n2.y, n2.z, n2.w, n3.x, n3.y, n3.z, n3.w};
+  const uint32_t wpair[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+  return pkv_rerank_words(s_prod, words, [&](int blk) {
+           return __uint_as_float(blk & 1 ? wpair[blk >> 1] & 0xffff0000u : wpair[blk >> 1] << 16);
+         }) * qnorm;
 }
 
 // Turn a 128-bin histogram in LDS (s_hist) into its suffix sums suf[t] = sum_{t' >= t} hist[t'],

@@ -59,41 +59,34 @@ __global__ __launch_bounds__(kRerankThreads) void pkv_rerank_kernel(
   }
   const uint8_t *nrow = nib + (int64_t)b * ns_b + (int64_t)h * ns_h;
   const uint16_t *wrow = weight + (int64_t)b * ws_b + (int64_t)h * ws_h;
-  float s = 0.f;
+  uint32_t words[16], wbits[16];
   if (KEYMAJOR) {
     const pkv_u32x4 *np = (const pkv_u32x4 *)(nrow + key * ns_key);
     const pkv_u32x4 *wp = (const pkv_u32x4 *)(wrow + key * ws_key);
-    pkv_u32x4 nv[4], wv[2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) nv[u] = np[u];
-    wv[0] = wp[0];
-    wv[1] = wp[1];
-    const uint32_t words[16] = {nv[0].x, nv[0].y, nv[0].z, nv[0].w, nv[1].x, nv[1].y, nv[1].z, nv[1].w,
-                                nv[2].x, nv[2].y, nv[2].z, nv[2].w, nv[3].x, nv[3].y, nv[3].z, nv[3].w};
-    const uint32_t wpair[8] = {wv[0].x, wv[0].y, wv[0].z, wv[0].w, wv[1].x, wv[1].y, wv[1].z, wv[1].w};
+    for (int u = 0; u < 4; ++u) {
+      const pkv_u32x4 n = np[u];
+      words[4 * u] = n.x, words[4 * u + 1] = n.y, words[4 * u + 2] = n.z, words[4 * u + 3] = n.w;
+    }
 #pragma unroll
-    for (int blk = 0; blk < 16; ++blk) {
-      const float t = pkv_block_dot(s_prod, blk, words[blk]);
-      const uint32_t wb = (blk & 1) ? (wpair[blk >> 1] >> 16) : (wpair[blk >> 1] & 0xffffu);
-      const float tw = t * pkv_bf16_bits_to_f32(wb);
-      s = (blk == 0) ? tw : s + tw;
-      if (V4B) store_v4b(v4b, row, n_cand, i, blk, s_val, words[blk]);
+    for (int u = 0; u < 2; ++u) {
+      const pkv_u32x4 w = wp[u];
+      const uint32_t pair[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+      for (int i = 0; i < 8; ++i) wbits[8 * u + i] = (i & 1) ? pair[i >> 1] >> 16 : pair[i >> 1] & 0xffffu;
     }
   } else {
     // all 32 loads in flight before the first product: 16 rows x 4003 of 20011 keys 16.0 -> 14.3 us; bound by the lines it
     // touches (every line of the index at one key in five) and the unpacked values, 47 MB
-    uint32_t words[16], wbits[16];
 #pragma unroll
     for (int blk = 0; blk < 16; ++blk) words[blk] = *(const uint32_t *)(nrow + key * ns_key + (int64_t)blk * ns_sub);
 #pragma unroll
     for (int blk = 0; blk < 16; ++blk) wbits[blk] = wrow[key * ws_key + (int64_t)blk * ws_sub];
+  }
+  const float s = pkv_rerank_words(s_prod, words, [&](int blk) { return pkv_bf16_bits_to_f32(wbits[blk]); });
+  if (V4B) {
 #pragma unroll
-    for (int blk = 0; blk < 16; ++blk) {
-      const float t = pkv_block_dot(s_prod, blk, words[blk]);
-      const float tw = t * pkv_bf16_bits_to_f32(wbits[blk]);
-      s = (blk == 0) ? tw : s + tw;
-      if (V4B) store_v4b(v4b, row, n_cand, i, blk, s_val, words[blk]);
-    }
+    for (int blk = 0; blk < 16; ++blk) store_v4b(v4b, row, n_cand, i, blk, s_val, words[blk]);
   }
   *out = s * qnorm[row];
 }
