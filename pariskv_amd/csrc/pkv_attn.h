@@ -248,6 +248,14 @@ __device__ __forceinline__ float *att_slot_ml(const PkvSplitAttn &a, int row, in
   return a.ws_ml + (uint32_t)(((row * a.group + head) * kSelSlots + slot) * 2);
 }
 
+// The arguments arrive in 64-byte lines when first read.  Read here, behind the caller's own loads, they are there when the attention
+// starts instead of after a trip to memory of its own.
+__device__ __forceinline__ void att_arguments(const PkvSplitAttn &a) {
+  const uint64_t k = (uint64_t)a.segs.k, idx = (uint64_t)a.segs.idx_limit, q = (uint64_t)a.q;
+  const int blk = a.blk_lo;
+  asm volatile("" ::"s"(k), "s"(idx), "s"(q), "s"(blk));
+}
+
 __device__ __forceinline__ void att_load_q(const PkvSplitAttn &a, int row, pkv_u32x4 (&qb)[4]) {
   const int lane = pkv_lane(), n = lane & 15, j = lane >> 4;
   const pkv_u32x4 zero4 = {0u, 0u, 0u, 0u};

@@ -741,7 +741,7 @@ __device__ __forceinline__ uint32_t lin_bin(uint64_t key, const LinSel &L) {
 // Clear; a barrier follows.
 __device__ __forceinline__ void lin_clear(uint32_t *s_hist, uint32_t *s_bcast) {
   const int tid = threadIdx.x;
-  for (int i = tid; i < 2 * kLinBins; i += kTopkThreads) s_hist[i] = 0;
+  if (tid < kLinBins) s_hist[tid] = 0;  // the slots behind them are written before they are read
   // [2..4]: threshold bin, keys needed from it, keys in it.  They are set below only if some bin reaches k; a row
   // with fewer than k keys leaves "keys in the threshold bin" at its all-ones start and the caller falls back.
   if (tid == 0)
@@ -779,42 +779,43 @@ __device__ __forceinline__ bool lin_steps(uint32_t mx, uint32_t mn, LinSel &L) {
   return true;
 }
 
-// Threshold bin and output slots from the histogram (a barrier lies before this).  One barrier.
+// Threshold bin, and with OFFS every bin's output slot and the most winners of a bin, from the histogram (a barrier lies before
+// this).  One barrier.  One wave works and 15 wait, so no branches and 128-bit accesses, 0.4 us (with eight branches 0.9; decode
+// step, 8 rows x 32768 keys, 4 layers, 108.0 -> 106.4, 12 x 9001 fp32, 2 layers, 63.1 -> 62.3).
+template <bool OFFS>
 __device__ __forceinline__ bool lin_decide(uint32_t k, uint32_t *s_hist, uint32_t *s_cnt, uint32_t *s_bcast, LinSel &L) {
   const int tid = threadIdx.x;
   if (tid < PKV_WAVE) {  // lane l owns the kPer bins below kLinBins - kPer * l: an inclusive scan over lanes is the suffix sum over bins
     constexpr int kPer = kLinBins / PKV_WAVE;
-    uint32_t h[kPer];
+    static_assert(kPer == 8, "two 128-bit words a lane");
+    const int first = kLinBins - kPer * (tid + 1);  // lowest of the lane's bins
+    const pkv_u32x4 lo = *(const pkv_u32x4 *)(s_hist + first), hi = *(const pkv_u32x4 *)(s_hist + first + 4);
+    const uint32_t h[kPer] = {hi.w, hi.z, hi.y, hi.x, lo.w, lo.z, lo.y, lo.x};  // highest bin first
     uint32_t mine = 0;
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      h[j] = s_hist[kLinBins - 1 - kPer * tid - j];
-      mine += h[j];
-    }
+    for (int j = 0; j < kPer; ++j) mine += h[j];
     uint32_t above = (uint32_t)pkv_wave_incl_scan((int)mine) - mine;
-    uint32_t most = 0;
+    const bool here = above < k && above + mine >= k;  // the threshold bin is one of this lane's
+    uint32_t off[kPer], bstar = 0, need = 0, in_bstar = 0, most = 0;
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
-      const int b = kLinBins - 1 - kPer * tid - j;
-      s_hist[kLinBins + b] = above;
-      s_cnt[b] = above;
-      if (above < k) {
-        const uint32_t take = above + h[j] >= k ? k - above : h[j];
-        most = take > most ? take : most;
-        if (above + h[j] >= k) s_bcast[2] = (uint32_t)b, s_bcast[3] = take, s_bcast[4] = h[j];
-      }
+      const uint32_t room = above < k ? k - above : 0u, take = h[j] < room ? h[j] : room;
+      const bool last = room != 0u && h[j] >= room;
+      bstar = last ? (uint32_t)(first + kPer - 1 - j) : bstar;
+      need = last ? take : need;
+      in_bstar = last ? h[j] : in_bstar;
+      most = take > most ? take : most;
+      off[j] = above;
       above += h[j];
     }
-    // every lane exchange is evaluated once, by all lanes: inside a conditional expression the compiler may run it
-    // under a partial execution mask, and a lane-crossing read of an inactive lane returns nothing
-#define PKV_MAX_XOR(M)                               \
-  {                                                  \
-    const uint32_t o = pkv_lane_xor<M>(most);        \
-    most = o > most ? o : most;                      \
-  }
-    PKV_MAX_XOR(1) PKV_MAX_XOR(2) PKV_MAX_XOR(4) PKV_MAX_XOR(8)
-#undef PKV_MAX_XOR
-    if ((tid & 15) == 0) atomicMax(&s_bcast[5], most);
+    if (here) s_bcast[2] = bstar, s_bcast[3] = need, s_bcast[4] = in_bstar;
+    if (OFFS) {
+      const pkv_u32x4 olo = {off[7], off[6], off[5], off[4]}, ohi = {off[3], off[2], off[1], off[0]};
+      *(pkv_u32x4 *)(s_hist + kLinBins + first) = olo, *(pkv_u32x4 *)(s_hist + kLinBins + first + 4) = ohi;
+      *(pkv_u32x4 *)(s_cnt + first) = olo, *(pkv_u32x4 *)(s_cnt + first + 4) = ohi;
+      most = pkv_wave_max(most);
+      if (tid == 0) s_bcast[5] = most;
+    }
   }
   __syncthreads();
   L.bstar = s_bcast[2], L.need = s_bcast[3], L.in_bstar = s_bcast[4], L.max_winners = s_bcast[5];
@@ -822,24 +823,26 @@ __device__ __forceinline__ bool lin_decide(uint32_t k, uint32_t *s_hist, uint32_
   return L.in_bstar <= kLinBucketMax;
 }
 
-// Bins of the thread's keys and the threshold bin.  On return s_hist[0,kLinBins) = keys per bin, s_hist[kLinBins,2*kLinBins) =
-// off[b] = keys in the bins above b, s_cnt[b] = off[b] (a running output slot for the counting sort), s_bcast[6] = 0.
+// Bins of the thread's keys and the threshold bin.  On return s_hist[0,kLinBins) = keys per bin, s_bcast[6] = 0, and with OFFS
+// s_hist[kLinBins,2*kLinBins) = off[b] = keys in the bins above b, s_cnt[b] = off[b] (a running output slot for the counting sort)
+// and L.max_winners.
 // All 1024 threads call it; false = not applicable.
 // BITS: bins of the ordered key bits instead of the values, for rows of one sign whose values span many binades
 // (e.g. the winners of a selection, about to be sorted): kLinBins equal steps of the bit pattern between the row's
 // smallest and largest key, i.e. equal steps of the logarithm up to the mantissa's linear pieces.
 // range: null, or the largest and the smallest ordered score of the nonzero keys (range[0] < range[1]: no key at
-// all) where the caller knows them already, which saves the reduction that finds them.
-template <int EIN, bool BITS = false>
+// all) where the caller knows them already, which saves the reduction that finds them; the caller has called lin_clear as
+// well then, with a barrier behind it.
+template <int EIN, bool BITS = false, bool OFFS = true>
 __device__ __forceinline__ bool linear_bins(const uint64_t (&v)[EIN], uint32_t k, uint32_t *s_hist, uint32_t *s_cnt,
                                             uint32_t *s_bcast, uint32_t (&bin)[EIN], LinSel &L,
                                             const uint32_t *range = nullptr) {
-  lin_clear(s_hist, s_bcast);
-  __syncthreads();
   uint32_t mx = 0u, mn = 0xffffffffu;
   if (range) {
     mx = range[0], mn = range[1];
   } else {
+    lin_clear(s_hist, s_bcast);
+    __syncthreads();
 #pragma unroll
     for (int e = 0; e < EIN; ++e) {
       if (v[e] != 0ull) {
@@ -853,14 +856,14 @@ __device__ __forceinline__ bool linear_bins(const uint64_t (&v)[EIN], uint32_t k
   if (!lin_steps<BITS>(mx, mn, L)) return false;
 #pragma unroll
   for (int e = 0; e < EIN; ++e) {
-    bin[e] = 0;
+    bin[e] = 0xffffffffu;  // no key: below every bin as a signed number, none of them as either
     if (v[e] != 0ull) {
       bin[e] = lin_bin(v[e], L);
       atomicAdd(&s_hist[bin[e]], 1u);
     }
   }
   __syncthreads();
-  return lin_decide(k, s_hist, s_cnt, s_bcast, L);
+  return lin_decide<OFFS>(k, s_hist, s_cnt, s_bcast, L);
 }
 
 // Threshold key of bin b*: the need-th largest of its keys, found by counting with 16 lanes per key.
@@ -890,8 +893,8 @@ __device__ __forceinline__ void linear_threshold(const uint64_t (&v)[EIN], const
 }
 
 // LDS scratch of a selection / sort over one workgroup's keys.
-struct SelSmem {
-  uint32_t hist[2 * kLinBins];
+struct alignas(16) SelSmem {
+  uint32_t hist[2 * kLinBins];  // these two by 128 bits
   uint32_t cnt[kLinBins];
   uint32_t bcast[8];
   uint32_t counter;
@@ -1067,6 +1070,17 @@ __device__ __forceinline__ void collect_winners_streamed(KeyFn key_of, int64_t l
   }
 }
 
+// Sum of the first `wave` of 16 words in LDS, one to a lane.
+__device__ __forceinline__ uint32_t waves_before(const uint32_t *s_words, int wave) {
+  const int at = threadIdx.x & 15;
+  int x = at < wave ? (int)s_words[at] : 0;
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+  return (uint32_t)__builtin_amdgcn_readlane(x, 15);
+}
+
 // len <= 8192 and k well below len: select the k winners exactly, then sort only those.
 // SORTED = false leaves the sort out: the winners come out in a fixed order of their positions in the row (by the
 // wave that loaded them, then by element index, then by lane: a function of the inputs only), for callers that use
@@ -1078,8 +1092,8 @@ __device__ __forceinline__ void topk_select_sort(const float *__restrict__ x, in
                                                  int64_t ids_stride, int len, int P, int64_t k, int64_t *__restrict__ out_ids,
                                                  float *__restrict__ out_vals, uint32_t *s_sel, Requests more) {
   extern __shared__ uint64_t s_keys[];
-  __shared__ uint32_t s_hist[2 * kLinBins];
-  __shared__ uint32_t s_cnt[kLinBins];
+  __shared__ alignas(16) uint32_t s_hist[2 * kLinBins];
+  __shared__ alignas(16) uint32_t s_cnt[kLinBins];
   __shared__ uint32_t s_bcast[8];
   __shared__ uint32_t s_counter;
   __shared__ uint64_t s_bucket[kLinBucketMax];
@@ -1112,7 +1126,7 @@ __device__ __forceinline__ void topk_select_sort(const float *__restrict__ x, in
   bool win[EIN];
   uint32_t bin[EIN];
   LinSel L;
-  const bool lin = linear_bins<EIN>(v, (uint32_t)k, s_hist, s_cnt, s_bcast, bin, L);  // uniform over the workgroup
+  const bool lin = linear_bins<EIN, false, SORTED>(v, (uint32_t)k, s_hist, s_cnt, s_bcast, bin, L);  // uniform over the workgroup
 #pragma unroll
   for (int e = 0; e < EIN; ++e)  // the whole keys
     if (v[e] != 0ull) v[e] = (v[e] & 0xffffffff00000000ull) | (uint64_t)(uint32_t)~id[e];
@@ -1151,6 +1165,8 @@ __device__ __forceinline__ void topk_select_sort(const float *__restrict__ x, in
     return;
   }
   if (!SORTED && lin) {
+    // (every instruction here is run by 16 waves on one CU, 16 cycles each: tests for no key, a loop over the waves' totals and
+    // slots of elements without a winner took 1 us more; decode step, 64 rows x 65536 keys, 2 layers, 103.0 -> 101.0)
     // any order, without the threshold key: the keys of the bins above b* all win and take the first k - need slots
     // (slot = winners of the lower waves + winners of the own wave at lower e + those at the same e in lower lanes:
     // one ballot per e and one exchange of the 16 wave totals); the keys of b* are ranked among themselves and the
@@ -1159,23 +1175,20 @@ __device__ __forceinline__ void topk_select_sort(const float *__restrict__ x, in
     uint32_t wave_total = 0;
 #pragma unroll
     for (int e = 0; e < EIN; ++e) {
-      const bool nz = v[e] != 0ull;
-      if (nz && bin[e] == L.bstar) s_bucket[atomicAdd(&s_bcast[6], 1u)] = v[e];
-      ballot[e] = __ballot(nz && bin[e] > L.bstar);
+      if (bin[e] == L.bstar) s_bucket[atomicAdd(&s_bcast[6], 1u)] = v[e];
+      ballot[e] = __ballot((int)bin[e] > (int)L.bstar);
       wave_total += (uint32_t)__popcll(ballot[e]);
     }
-    const int wave = tid / PKV_WAVE;
-    if (pkv_lane() == 0) s_hist[wave] = wave_total;  // the histograms have been read by everyone
+    const int wave = __builtin_amdgcn_readfirstlane(tid / PKV_WAVE), lane = pkv_lane();
+    if (lane == 0) s_hist[wave] = wave_total;  // the histograms have been read by everyone
     __syncthreads();
-    uint32_t slot = 0;
-#pragma unroll
-    for (int w = 0; w < kTopkThreads / PKV_WAVE; ++w) slot += w < wave ? s_hist[w] : 0u;
-    const uint64_t below = ((uint64_t)1 << pkv_lane()) - 1;
+    uint32_t slot = waves_before(s_hist, wave);
     const uint32_t n_above = (uint32_t)k - L.need;
 #pragma unroll
     for (int e = 0; e < EIN; ++e) {
-      const uint32_t mine = slot + (uint32_t)__popcll(ballot[e] & below);
-      if (((ballot[e] >> pkv_lane()) & 1ull) && mine < n_above) {
+      if (ballot[e] == 0ull) continue;  // the whole wave
+      const uint32_t mine = slot + __builtin_amdgcn_mbcnt_hi((uint32_t)(ballot[e] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ballot[e], 0u));
+      if (((ballot[e] >> lane) & 1ull) && mine < n_above) {
         if (oi) oi[mine] = (int64_t)(uint32_t)(~(uint32_t)v[e]);
         if (s_sel) s_sel[mine] = ~(uint32_t)v[e];
         if (ov) ov[mine] = pkv_from_ordered_u32((uint32_t)(v[e] >> 32));
@@ -1291,7 +1304,7 @@ __device__ __forceinline__ void topk_select_long(const float *__restrict__ x, in
       if (e + 1 < n_mine) atomicAdd(&sm.hist[b1], 1u);
     }
     __syncthreads();
-    lin = lin_decide((uint32_t)k, sm.hist, sm.cnt, sm.bcast, L) && L.max_winners <= kLinRankMax;
+    lin = lin_decide<true>((uint32_t)k, sm.hist, sm.cnt, sm.bcast, L) && L.max_winners <= kLinRankMax;
   }
   if (!lin) {
     if (!kEarly) more();
@@ -1381,7 +1394,10 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_long_attend_kernel(
   uint32_t *s_sel = (uint32_t *)(s_keys + (P < 1024 ? 1024 : P));
   AttSelRequests req;
   att_clear(sm);
-  topk_select_long<EIN>(x, x_stride, ids, ids_stride, len, P, k, out_ids, out_vals, s_sel, [&] { att_request(attn, row, req); });
+  topk_select_long<EIN>(x, x_stride, ids, ids_stride, len, P, k, out_ids, out_vals, s_sel, [&] {
+    att_arguments(attn);
+    att_request(attn, row, req);
+  });
   __syncthreads();
   att_selected<true>(attn, row, s_sel, 0, sm, req);
 }
@@ -1406,7 +1422,10 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_attend_kernel(
   AttSelRequests req;
   att_clear(sm);
   topk_select_sort<EIN, false>(x, x_stride, ids, ids_stride, len, 0, k, wg ? nullptr : out_ids, out_vals, s_sel,
-                               [&] { if (MERGE) att_request(attn, row, req); });
+                               [&] {
+                                 att_arguments(attn);
+                                 if (MERGE) att_request(attn, row, req);
+                               });
   __syncthreads();
   att_selected<MERGE>(attn, row, s_sel, wg, sm, req);
 }
@@ -1881,64 +1900,54 @@ __device__ __forceinline__ float wave_running_sum(float val, float carry) {
   return acc;
 }
 
-// Smallest k <= k_out with sl_benefit + prefix_{k-1} >= tgt over the sorted keys in s_keys (k_out if the
+// Place of sorted benefit i in s_ben: a word of padding behind every 64, so that lanes that walk a block each meet no bank conflict.
+__device__ __forceinline__ uint32_t ben_at(uint32_t i) { return i + i / PKV_WAVE; }
+
+// Smallest k <= k_out with sl_benefit + prefix_{k-1} >= tgt over the sorted benefits in s_ben (k_out if the
 // target is never reached).  prefix is the cumulative sum of the reference (adaptive_topk.py:300-303) in
 // a fixed two-level order: blocks of 64 consecutive benefits are summed left to right, the block totals
 // are summed left to right, prefix_i = (total of the earlier blocks) + (running sum inside the block).
 // Benefits are not negative, so the prefixes never decrease: the first block whose last prefix reaches the
-// target holds the answer.  Every wave runs the short second level for itself (no barrier for its result);
-// the wave that owns that block finds the element.  All 1024 threads call it; k_out <= 8192.
-// s_f: 128 floats, s_k: one word.
-__device__ __forceinline__ int64_t first_k_reaching(const uint64_t *s_keys, int64_t k_out, float sl_benefit, float tgt,
-                                                    float *s_f, uint32_t *s_k) {
-  const int lane = pkv_lane(), wave = threadIdx.x / PKV_WAVE;
-  const int n_blocks = (int)((k_out + PKV_WAVE - 1) / PKV_WAVE);  // <= 128; wave w owns blocks w, w+16, ...
-  float *s_tot = s_f;
-  float run[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int c = wave + 16 * j;
-    run[j] = 0.f;
-    if (c < n_blocks) {
-      const int64_t i = (int64_t)c * PKV_WAVE + lane;
-      run[j] = wave_running_sum(i < k_out ? pkv_from_ordered_u32((uint32_t)(s_keys[i] >> 32)) : 0.f, 0.f);
-      if (lane == PKV_WAVE - 1) s_tot[c] = run[j];
-    }
-  }
-  if (threadIdx.x == 0) *s_k = (uint32_t)k_out;
-  __syncthreads();
-  // second level: lane l of pass p holds block 64p + l; the chain of adds needs as many steps as there are blocks
-  int cstar = -1;
-  float before_star = 0.f, carry = 0.f;
-  for (int base = 0; base < n_blocks && cstar < 0; base += PKV_WAVE) {
+// target holds the answer.  One wave, while the others are done: where all 16 ran the same serial chains an instruction cost 16
+// cycles, and the blocks and their totals took 2.9 us (adaptive step, 24 rows x 41003 keys, 2 layers, 89.4 -> 87.0).
+// s_ben: k_out benefits at ben_at(i), zeros behind them up to a whole block.  k_out <= 8192.
+__device__ __forceinline__ int64_t first_k_reaching(const float *s_ben, int64_t k_out, float sl_benefit, float tgt) {
+  const int lane = pkv_lane();
+  const int n_blocks = (int)((k_out + PKV_WAVE - 1) / PKV_WAVE);  // <= 128
+  float carry = 0.f;
+  for (int base = 0; base < n_blocks; base += PKV_WAVE) {  // lane l: block base + l
     const int c = base + lane, live = n_blocks - base < PKV_WAVE ? n_blocks - base : PKV_WAVE;
-    const float val = c < n_blocks ? s_tot[c] : 0.f;
+    float val = 0.f;
+    if (c < n_blocks) {
+      const float *blk = s_ben + ben_at((uint32_t)(c * PKV_WAVE));
+#pragma unroll 16
+      for (int j = 0; j < PKV_WAVE; ++j) val = val + blk[j];
+    }
+    // the chain of adds over the totals needs as many steps as there are blocks; more change nothing (16 in a row, as a loop of
+    // four takes four times as long a step)
     float acc = val;
-    for (int st = 0; st < live; ++st) {
-      const float below =
-          __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(carry), __float_as_int(acc), 0x138, 0xf, 0xf, false));
-      acc = below + val;
+    for (int st = 0; st < live; st += 16) {
+#pragma unroll
+      for (int u = 0; u < 16; ++u) {
+        const float below =
+            __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(carry), __float_as_int(acc), 0x138, 0xf, 0xf, false));
+        acc = below + val;
+      }
     }
     const float before =
         __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(carry), __float_as_int(acc), 0x138, 0xf, 0xf, false));
     const uint64_t hit = __ballot(c < n_blocks && sl_benefit + acc >= tgt);
     if (hit) {
-      const int l = __ffsll((long long)hit) - 1;
-      cstar = base + l;
-      before_star = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(before), l));
+      const int l = __ffsll((long long)hit) - 1, cstar = base + l;
+      const float before_star = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(before), l));
+      const float mine = wave_running_sum(s_ben[ben_at((uint32_t)(cstar * PKV_WAVE)) + lane], 0.f);
+      const int64_t i = (int64_t)cstar * PKV_WAVE + lane;
+      const uint64_t at = __ballot(i < k_out && sl_benefit + (before_star + mine) >= tgt);
+      return at ? (int64_t)(cstar * PKV_WAVE + __ffsll((long long)at)) : k_out;
     }
     carry = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc), live - 1));
   }
-  if (cstar >= 0 && (cstar & 15) == wave) {
-    float mine = run[0];
-#pragma unroll
-    for (int j = 1; j < 8; ++j) mine = (cstar >> 4) == j ? run[j] : mine;
-    const int64_t i = (int64_t)cstar * PKV_WAVE + lane;
-    const uint64_t hit = __ballot(i < k_out && sl_benefit + (before_star + mine) >= tgt);
-    if (lane == 0 && hit) *s_k = (uint32_t)(cstar * PKV_WAVE + __ffsll((long long)hit));
-  }
-  __syncthreads();
-  return (int64_t)*s_k;
+  return k_out;
 }
 
 // Sum of the per-slice sums of a row in slice order, starting from the first.  `first` is ssum[lane] (0 beyond
@@ -1978,25 +1987,32 @@ __device__ __forceinline__ void adaptive_tail(uint64_t *s_keys, int P, int64_t k
     PKV_DISPATCH_E(P, PKV_SORT_K);
 #undef PKV_SORT_K
   }
-  float *s_f = (float *)sm.hist;
-  uint32_t *s_k = &sm.counter;
-  // the winners' ids do not depend on k: they are requested now and stored after the search for k
+  // the benefits once more, padded, where the sort's second copy of the keys was
+  float *s_ben = (float *)(s_keys + (P < 1024 ? 1024 : P));
+  // the winners' ids do not depend on k
   int64_t id[kTopkMaxSort / kTopkThreads];
 #pragma unroll
   for (int e = 0; e < kTopkMaxSort / kTopkThreads; ++e) {
     const int64_t i = threadIdx.x + e * kTopkThreads;
     id[e] = 0;
     if (i < k_out) {
-      const uint32_t pos = ~(uint32_t)s_keys[i];
+      const uint64_t key = s_keys[i];
+      const uint32_t pos = ~(uint32_t)key;
+      s_ben[ben_at((uint32_t)i)] = pkv_from_ordered_u32((uint32_t)(key >> 32));
       if (pos < (uint64_t)n_cand) id[e] = ci[pos];
+    } else if (i < (k_out + PKV_WAVE - 1) / PKV_WAVE * PKV_WAVE) {
+      s_ben[ben_at((uint32_t)i)] = 0.f;
     }
   }
-  int64_t k = 1;  // total <= 0: adaptive_topk.py:304-306
-  if (total > 0.f) k = first_k_reaching(s_keys, k_out, sl_benefit, threshold * total, s_f, s_k);
-  if (threadIdx.x == 0) {
-    if (cl.k_max > 0) k = k < cl.k_min ? cl.k_min : (k > cl.k_max ? cl.k_max : k);
-    *adaptive_k_row = k;
-    if (cl.row_keys) cl.row_keys[row] = (int32_t)(cl.row_keys_base + k);
+  __syncthreads();
+  if (threadIdx.x < PKV_WAVE) {
+    int64_t k = 1;  // total <= 0: adaptive_topk.py:304-306
+    if (total > 0.f) k = first_k_reaching(s_ben, k_out, sl_benefit, threshold * total);
+    if (threadIdx.x == 0) {
+      if (cl.k_max > 0) k = k < cl.k_min ? cl.k_min : (k > cl.k_max ? cl.k_max : k);
+      *adaptive_k_row = k;
+      if (cl.row_keys) cl.row_keys[row] = (int32_t)(cl.row_keys_base + k);
+    }
   }
 #pragma unroll
   for (int e = 0; e < kTopkMaxSort / kTopkThreads; ++e) {
@@ -2031,8 +2047,8 @@ __device__ __forceinline__ AdkRow adk_row(int row, const float *sl_logits, int64
   return r;
 }
 
-// n_cand <= 1024*EIN <= 8192: one workgroup per row, everything in registers.  Dynamic LDS P*8 bytes
-// (P = pow2 >= k_out, at least 1024 keys).
+// n_cand <= 1024*EIN <= 8192: one workgroup per row, everything in registers.  Dynamic LDS: lds_bytes_adk(P)
+// (P = pow2 >= k_out).
 template <int EIN>
 __global__ __launch_bounds__(kTopkThreads) void pkv_adaptive_topk_kernel(
     const float *__restrict__ sl_logits, int64_t sl_stride, const float *__restrict__ sl_vnorm, int64_t slv_stride,
@@ -2046,6 +2062,7 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_adaptive_topk_kernel(
   __shared__ SelSmem sm;
   const int row = blockIdx.x;
   const int tid = threadIdx.x;
+  lin_clear(sm.hist, sm.bcast);  // for select_sort_desc; several barriers lie between
   const AdkRow r = adk_row(row, sl_logits, sl_stride, sl_vnorm, slv_stride, cand_scores, cand_dtype, cand_vnorm,
                            value_norm, vn_stride, cand_ids, n_cand);
   // candidate logits and value norms: element i = tid + e*1024, so a lane adds its elements in increasing i
@@ -2116,10 +2133,11 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_adaptive_topk_kernel(
   // binades: bins of the key bits), else selected first and sorted afterwards
   if (tid == 0) sm.counter = 0;
   const int Pz = P < 1024 ? 1024 : P;
-  for (int i = tid; i < Pz; i += kTopkThreads) s_keys[i] = 0ull;
   const bool sorted = P <= kCountingSortMaxP &&
                       select_sort_desc<EIN>(v, (uint32_t)k_out, s_keys + Pz, s_keys, sm, key_range);  // k_out <= n_cand
   if (!sorted) {
+    __syncthreads();
+    for (int i = tid; i < Pz; i += kTopkThreads) s_keys[i] = 0ull;
     bool win[EIN];
     if (k_out < n_cand) {
       select_topk_flags<EIN, true>(v, (uint32_t)k_out, sm, win);
@@ -2265,7 +2283,7 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_adk_compact_kernel(const flo
                          list_b + (int64_t)row * n_cand, s_tmp);
 }
 
-// grid rows; dynamic LDS: lds_bytes_sort(P).
+// grid rows; dynamic LDS: lds_bytes_adk(P).
 __global__ __launch_bounds__(kTopkThreads) void pkv_adk_finish_kernel(
     const int64_t *__restrict__ cand_ids, int64_t n_cand, int n_slices, float threshold, int64_t k_out, int P,
     const float *__restrict__ ws_sum, const uint32_t *__restrict__ ctl, const uint64_t *__restrict__ list_a,
@@ -2324,6 +2342,11 @@ __global__ __launch_bounds__(kDenseLogitThreads) void pkv_dense_logits_kernel(co
 static size_t lds_bytes(int P) { return (size_t)(P < 1024 ? 1024 : P) * 8; }
 // with room for the counting sort's second copy of the winners where the kernels use it
 static size_t lds_bytes_sort(int P) { return lds_bytes(P) * (P <= kCountingSortMaxP ? 2 : 1); }
+
+// ... and the adaptive-k kernels' padded benefits in its place (they fit where it is there)
+static size_t lds_bytes_adk(int P) {
+  return P <= kCountingSortMaxP ? lds_bytes_sort(P) : lds_bytes(P) + (size_t)(P + P / PKV_WAVE) * sizeof(float);
+}
 
 static int pow2_ceil(int64_t v) {
   int p = 1;
@@ -2685,7 +2708,7 @@ extern "C" int pkv_adaptive_topk(const float *sl_logits, int64_t sl_stride, cons
   if (n_cand <= kTopkMaxSort) {  // one workgroup per row, no workspace
     const int ein = pow2_ceil(n_cand) / kTopkThreads;
 #define PKV_ADK(EIN)                                                                                                  \
-  hipLaunchKernelGGL((pkv_adaptive_topk_kernel<EIN>), dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes_sort(P), s,      \
+  hipLaunchKernelGGL((pkv_adaptive_topk_kernel<EIN>), dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes_adk(P), s,       \
                      sl_logits, sl_stride, sl_vnorm, slv_stride, sl, cand_scores, cand_dtype, cand_scale, cand_vnorm, \
                      value_norm, vn_stride, vn_offset, vn_pos_stride, cand_ids, (int)n_cand, threshold, k_out, P,     \
                      adaptive_k, topk_ids, cl)
@@ -2717,7 +2740,7 @@ extern "C" int pkv_adaptive_topk(const float *sl_logits, int64_t sl_stride, cons
   PKV_LAUNCH_CHECK("pkv_adk_benefit_kernel");
   hipLaunchKernelGGL(pkv_adk_compact_kernel, grid, dim3(kTopkThreads), 0, s, ben, n_cand, k_out, ctl, list_a, list_b);
   PKV_LAUNCH_CHECK("pkv_adk_compact_kernel");
-  hipLaunchKernelGGL(pkv_adk_finish_kernel, dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes_sort(P), s, cand_ids,
+  hipLaunchKernelGGL(pkv_adk_finish_kernel, dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes_adk(P), s, cand_ids,
                      n_cand, n_slices, threshold, k_out, P, ssum, ctl, list_a, list_b, adaptive_k, topk_ids, cl);
   PKV_LAUNCH_CHECK("pkv_adk_finish_kernel");
   return PKV_OK;
