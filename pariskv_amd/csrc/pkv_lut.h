@@ -16,7 +16,6 @@ struct PkvLutSmem {
   __attribute__((aligned(16))) uint32_t key[256];
   int id[256];
   int cc[256];
-  int part[128];
   int wave_tot[4];
 };
 
@@ -72,77 +71,48 @@ __device__ __forceinline__ void pkv_lut_rank_subspace(int dtype, const int32_t *
   const int tid = threadIdx.x;
   if (cc_sub) sm.cc[tid] = cc_sub[tid];  // read again only after the barriers below
 
-  // score of centroid c = tid: sum_j (+-) qhat_sub[j], sequential j
-  {
-    float acc = 0.f;
+  // rank = number of centroids ahead of this one under (score desc, id asc).  The sign codebook is antipodal (score[255-c] ==
+  // -score[c] exactly), hence rank[255-c] = 255 - rank[c], and of each such pair the member whose score is not negative (of two
+  // zeros the smaller id) is ahead of every member that is not of its kind: its rank is the number of pairs whose own such member
+  // is ahead of it, by magnitude and then id.  Threads 2c and 2c + 1 count for pair c over every other group of four pairs, 64
+  // comparisons each and no exchange through LDS (128 comparisons each, against all 256 centroids: 64 rows x 65536 keys, 2 layers,
+  // 101.3 / 99.9 us a step, adaptive 24 x 41003, 2 layers, 87.8 / 86.0).
+  const int c = tid >> 1, half = tid & 1;
+  float acc = 0.f;  // score of centroid c: sum_j (+-) qhat_sub[j], sequential j
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float v = sm.y[8 * sub + j];
-      const float t = ((tid >> j) & 1) ? v : -v;
-      acc = (j == 0) ? t : acc + t;
-    }
-    acc = pkv_rdt(acc + 0.0f, dtype);
-    uint32_t key = pkv_ordered_u32(acc);
-    // bf16 scores occupy the top 16 bits: fold the tie rule (smaller id first) into one 32-bit key
-    if (dtype == PKV_DTYPE_BF16) key = ((key >> 16) << 8) | (uint32_t)(255 - tid);
-    sm.key[tid] = key;
+  for (int j = 0; j < 8; ++j) {
+    const float v = sm.y[8 * sub + j];
+    const float t = ((c >> j) & 1) ? v : -v;
+    acc = (j == 0) ? t : acc + t;
   }
-  __syncthreads();
-  // rank = number of centroids ahead of this one under (score desc, id asc).  The sign codebook is
-  // antipodal (score[255-c] == -score[c] exactly), hence rank[255-c] = 255 - rank[c]: thread t counts,
-  // for centroid c = t & 127, over half (t >> 7) of the keys; the two partial counts are added.
-  {
-    const int c = tid & 127, half = tid >> 7;
-    const uint32_t mine = sm.key[c];
-    int part = 0, part1 = 0, part2 = 0, part3 = 0;  // four chains of dependent adds (one: +0.3 us per launch)
-    const pkv_u32x4 *k4 = (const pkv_u32x4 *)sm.key + half * 32;
-    if (dtype == PKV_DTYPE_BF16) {
-#pragma unroll 8
-      for (int c4 = 0; c4 < 32; ++c4) {
-        const pkv_u32x4 k = k4[c4];
-        part += (k.x > mine), part1 += (k.y > mine), part2 += (k.z > mine), part3 += (k.w > mine);
-      }
-    } else {
-      // "ahead" is k > mine, and from smaller ids also k == mine.  A wave's 64 centroids lie in one block of 64 ids, so of
-      // the two blocks a thread counts over, only the wave's own needs the ids compared key by key (all of them: +0.6 us a launch
-      // at 12 rows, 7.7 against 7.1).
-      const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), c0 = (wave & 1) * 64, o_half = (wave >> 1) * 128;
-      for (int o0 = o_half; o0 < o_half + 128; o0 += 64) {
-        const pkv_u32x4 *kb = (const pkv_u32x4 *)sm.key + o0 / 4;
-        if (o0 > c0) {
-#pragma unroll
-          for (int c4 = 0; c4 < 16; ++c4) {
-            const pkv_u32x4 k = kb[c4];
-            part += (k.x > mine), part1 += (k.y > mine), part2 += (k.z > mine), part3 += (k.w > mine);
-          }
-        } else if (o0 < c0) {
-#pragma unroll
-          for (int c4 = 0; c4 < 16; ++c4) {
-            const pkv_u32x4 k = kb[c4];
-            part += (k.x >= mine), part1 += (k.y >= mine), part2 += (k.z >= mine), part3 += (k.w >= mine);
-          }
-        } else {
-#pragma unroll 8
-          for (int c4 = 0; c4 < 16; ++c4) {
-            const pkv_u32x4 k = kb[c4];
-            const int o = o0 + 4 * c4;
-            part += (k.x > mine || (k.x == mine && o + 0 < c)) ? 1 : 0;
-            part1 += (k.y > mine || (k.y == mine && o + 1 < c)) ? 1 : 0;
-            part2 += (k.z > mine || (k.z == mine && o + 2 < c)) ? 1 : 0;
-            part3 += (k.w > mine || (k.w == mine && o + 3 < c)) ? 1 : 0;
-          }
-        }
-      }
-    }
-    part += part1 + part2 + part3;
-    if (half) sm.part[c] = part;
+  const uint32_t bits = __float_as_uint(pkv_rdt(acc + 0.0f, dtype)), magnitude = bits & 0x7fffffffu;
+  const int front = (bits >> 31) ? 255 - c : c;
+  int ahead = 0, ahead1 = 0, ahead2 = 0, ahead3 = 0;  // four chains of dependent adds (one: +0.3 us per launch)
+  if (dtype == PKV_DTYPE_BF16) {
+    // bf16 magnitudes occupy 15 bits: fold the tie rule (smaller id first) into one 32-bit key
+    const uint32_t mine = ((magnitude >> 16) << 8) | (uint32_t)(255 - front);
+    if (!half) sm.key[c] = mine;
     __syncthreads();
-    if (!half) {
-      const int rank = part + sm.part[c];
-      sm.id[rank] = c;
-      sm.id[255 - rank] = 255 - c;
+    const pkv_u32x4 *k4 = (const pkv_u32x4 *)sm.key + half;
+#pragma unroll 8
+    for (int i = 0; i < 16; ++i) {
+      const pkv_u32x4 k = k4[2 * i];
+      ahead += (k.x > mine), ahead1 += (k.y > mine), ahead2 += (k.z > mine), ahead3 += (k.w > mine);
+    }
+  } else {
+    uint64_t *s_key = (uint64_t *)sm.key;
+    const uint64_t mine = ((uint64_t)magnitude << 8) | (uint64_t)(255 - front);
+    if (!half) s_key[c] = mine;
+    __syncthreads();
+    const uint64_t *k = s_key + 2 * half;
+#pragma unroll 8
+    for (int i = 0; i < 32; i += 2) {
+      ahead += (k[4 * i] > mine), ahead1 += (k[4 * i + 1] > mine), ahead2 += (k[4 * i + 4] > mine), ahead3 += (k[4 * i + 5] > mine);
     }
   }
+  ahead += ahead1 + ahead2 + ahead3;
+  ahead += (int)pkv_lane_xor<1>((uint32_t)ahead);
+  sm.id[half ? 255 - ahead : ahead] = half ? 255 - front : front;
   __syncthreads();
   const int id = sm.id[tid];
   const int w = pkv_tier_weight_from_rank(sm.cc[id], tiers, sm.wave_tot);

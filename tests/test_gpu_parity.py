@@ -2169,3 +2169,38 @@ def test_decode_step_merges_after_the_selection_from_a_long_row(ops, bs, group, 
     """The attention behind that selection, in the selecting workgroup: as top-k and attention called one by one, bit for bit."""
     _say(f"two-part attention behind a long row, {bs} x 2 rows group {group} k {k} candidates {cand} of {keys} scores {scores}")
     _two_parts(ops, bs, 2, group, k, 64, 300, keys, cand, 1, scores, replays=3 if scores is None else 0)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["spread", "ties", "one dim", "zero subspaces", "tiny"])
+def test_query_prep_ranks_equal_and_zero_scores_by_id(ops, dtype, kind):
+    """The ranking by pairs of antipodal centroids where scores tie, vanish or differ in sign alone: as the oracle's, ids and votes."""
+    _say(f"query prep ranking {dtype} {kind}")
+    bs, H, group = 2, 3, 4
+    g = torch.Generator().manual_seed(5)
+    q = torch.randn(bs, 1, H * group, 128, generator=g)
+    if kind == "ties":
+        q = torch.where(q > 0, 1.0, -1.0)
+    elif kind == "one dim":
+        q[..., 1:] = 0
+    elif kind == "zero subspaces":   # the rotation undone: the rotated query has zeros in whole subspaces
+        had = torch.ones(1, 1)
+        for _ in range(7):
+            had = torch.cat([torch.cat([had, had], 1), torch.cat([had, -had], 1)], 0)
+        want = torch.zeros(128)
+        want[:24] = torch.tensor([1.0, 2.0, -1.0, 0.5, 0.0, -2.0, 1.0, 1.0]).repeat(3)
+        q = ((want @ had) * torch.from_numpy(O.srht_signs(42)) / 128).expand(bs, 1, H * group, 128).clone()
+    elif kind == "tiny":
+        q = q * 1e-20
+    q = q.to(dtype)
+    signs = torch.from_numpy(O.srht_signs(42))
+    cc = torch.randint(0, 40, (bs, H, 16, 256), generator=g, dtype=torch.int32)
+    tiers = [200, 400, 800, 1200, 2000, 3000]
+    qhat, _, lut, ids = ops.query_prep_lut(q.to(DEV), H, signs.to(DEV), cc.to(DEV), tiers, want_sorted_ids=True)
+    torch.cuda.synchronize()
+    od = O.BF16 if dtype == torch.bfloat16 else O.F32
+    for b in range(bs):
+        for h in range(H):
+            want_ids = O.rank_centroids(qhat[b, h].cpu().numpy(), od)
+            assert np.array_equal(ids[b, h].cpu().numpy(), want_ids), (b, h)
+            assert np.array_equal(lut[b, h].cpu().numpy(), O.tier_lut(want_ids, cc[b, h].numpy(), tiers)), (b, h)
