@@ -46,9 +46,13 @@ constexpr int kEncThreads = 256;
 constexpr int kEncWavesPerSimd = 4;
 constexpr int kEncKeysPerIter = kEncThreads / 16;
 constexpr int kEncKeysPerWg = 16 * kEncKeysPerIter;
-// iterations whose keys a wave has in flight (bf16 keys, 1 / 2 / 4: 132 / 127 / 125 us per 1M key-heads); an fp32
+// a workgroup's keys are runs of this many neighbours, side by side or (SPREAD) set apart
+constexpr int kEncRun = 128;
+constexpr int kEncRuns = kEncKeysPerWg / kEncRun;
+// iterations whose keys a wave has in flight (bf16 keys, 1 / 2 / 4: 132 / 127 / 125 us per 1M key-heads; SPREAD, 2 / 4:
+// 457 / 459 us per 2M with their rows); an fp32
 // key takes two 16-byte words per lane, so half as many iterations hold the same bytes in as many registers
-constexpr int kEncAheadBf16 = 4, kEncAheadF32 = 2;
+constexpr int kEncAheadBf16 = 4, kEncAheadBf16Spread = 2, kEncAheadF32 = 2;
 
 #define PKV_ENC_THRESHOLDS 0.08447265625f, 0.169921875f, 0.2578125f, 0.349609375f, 0.44921875f, 0.55859375f, 0.69140625f
 #define PKV_ENC_CENTERS 0.0419921875f, 0.126953125f, 0.212890625f, 0.302734375f, 0.396484375f, 0.5f, 0.6171875f, 0.76171875f
@@ -461,10 +465,22 @@ __device__ __forceinline__ bool enc_key_fast_f32(const float (&xr)[8], const flo
 // A STORE launch, grid (blocks, kv heads, batch): an encode workgroup first copies the value rows of its keys to their
 // place in the zone (taking their norms), then encodes the keys and writes each key row from the registers it is
 // encoded from (no second read of K); behind the encode workgroups of a head, dense workgroups copy K and V rows of 64
-// sink or local-window tokens each.  Bound by HBM: 1136 bytes per key in bf16, in 478 us for 4 x 8 heads x 65536 keys =
-// 5.0 TB/s, what a plain copy reaches (762 us as two copies and the encoder alone).  Value rows by workgroups of their
-// own between the encoding ones: 555 us with the records' tails left out, 485 us with whole records; heads instead of
-// blocks fastest over the grid 595 us; 128 / 512 keys per workgroup 479 / 504 us.
+// sink or local-window tokens each.  Bound by HBM: 1136 bytes per key in bf16, in 458 us for 4 x 8 heads x 65536 keys =
+// 5.2 TB/s (762 us as two copies and the encoder alone); without the encoding's arithmetic, which is hidden, 449 us.  A copy
+// of rows alone reaches 6.0 TB/s.  Value rows by workgroups of their own between the encoding ones: 555 us with the records'
+// tails left out, 485 us with whole records; heads instead of blocks fastest over the grid 595 us; 128 / 512 keys per
+// workgroup 476 / 483 us; value rows moved one per key inside the loop 479 us; a workgroup that goes on to the next 512
+// keys instead of ending (fewer histogram flushes) 509 us; 5 waves a SIMD instead of 4 462 us.
+//
+// SPREAD, for prompts of more than kEncSpreadBytes moved, more than twice what the memory-side cache holds: a workgroup's
+// two runs of kEncRun keys lie as many runs apart as the head has workgroups, so that the workgroups that run side by side
+// read and write one narrow window of the prompt and of the zone; value rows are loaded past the caches; codes and records,
+// whose 128-byte lines are shared by two waves or two stores, stay in the L2 until both halves are there; and two
+// iterations' keys instead of four in flight are enough.  Against the same launch without these (4 x 8 x 65536 bf16
+// 479 -> 458 us, 16 heads x 65536 250 -> 238, 8 x 100000 200 -> 186, 8 x 65536 131 -> 119, 8 x 80000 fp32 315 -> 309).
+// Smaller prompts partly stay in the memory-side cache, and there the plain stores and spread windows gain or lose by where
+// things happen to lie (8 x 55000 100 -> 103 us, 8 x 32768 62 -> 66, 4 x 100000 96 -> 99): they keep the other form.
+constexpr int64_t kEncSpreadBytes = 576ll << 20;
 enum EncStoreMode {
   kEncNoStore = 0,
   kEncStoreRows = 1,
@@ -491,28 +507,31 @@ struct EncStore {
 };
 constexpr int kEncDenseRows = 64;
 
-// n_rows rows of 128 elements from src (src_step bytes apart) to consecutive rows at dst, by one workgroup; norm /
+// n_rows rows of 128 elements from src (src_step bytes apart) to consecutive rows at dst, by one workgroup; SPREAD: with
+// streaming loads, and after every kEncRun rows source, destination, norm and norm2 (not s_norm) skip gap rows; norm /
 // norm2 / s_norm (may be null): the rows' 2-norms in the rows' type: four consecutive squares left to right, then a
 // pairwise tree over the row's 32 groups, which is the order of torch.linalg.vector_norm over the last dimension (its fp32
 // bits; an order of one's own moves about one norm in a million to the neighbouring bf16 value).
-template <bool BF16>
+template <bool BF16, bool SPREAD = false>
 __device__ __forceinline__ void enc_copy_rows(const char *src, int64_t src_step, char *dst, int n_rows, float *norm,
-                                              int64_t norm_step, float *norm2, float *s_norm = nullptr) {
+                                              int64_t norm_step, float *norm2, float *s_norm = nullptr, int64_t gap = 0) {
   constexpr int kVec = BF16 ? 16 : 32;             // 16-byte words per row
   constexpr int kRowsPerStep = kEncThreads / kVec;
   constexpr int kAhead = 8;                        // loads of a thread in flight
   const int lane = threadIdx.x % kVec, r0 = threadIdx.x / kVec;
+  auto place = [&](int row) { return SPREAD ? row + row / kEncRun * gap : (int64_t)row; };
   for (int base = 0; base < n_rows; base += kAhead * kRowsPerStep) {
     pkv_u32x4 val[kAhead];
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
       const int row = base + u * kRowsPerStep + r0;
-      val[u] = *(const pkv_u32x4 *)(src + (int64_t)(row < n_rows ? row : n_rows - 1) * src_step + 16 * lane);
+      const pkv_u32x4 *p = (const pkv_u32x4 *)(src + place(row < n_rows ? row : n_rows - 1) * src_step + 16 * lane);
+      val[u] = SPREAD ? __builtin_nontemporal_load(p) : *p;
     }
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
       const int row = base + u * kRowsPerStep + r0;
-      if (row < n_rows) __builtin_nontemporal_store(val[u], (pkv_u32x4 *)(dst + (int64_t)row * (16 * kVec) + 16 * lane));
+      if (row < n_rows) __builtin_nontemporal_store(val[u], (pkv_u32x4 *)(dst + place(row) * (16 * kVec) + 16 * lane));
     }
     if (norm || norm2 || s_norm) {  // uniform
 #pragma unroll
@@ -541,8 +560,8 @@ __device__ __forceinline__ void enc_copy_rows(const char *src, int64_t src_step,
         if (!BF16) acc = acc + pkv_lane_xor_f<16>(acc);
         if (lane == 0 && row < n_rows) {
           const float n = BF16 ? pkv_bf16_round(sqrtf(acc)) : sqrtf(acc);
-          if (norm) norm[(int64_t)row * norm_step] = n;
-          if (norm2) norm2[row] = n;
+          if (norm) norm[place(row) * norm_step] = n;
+          if (norm2) norm2[place(row)] = n;
           if (s_norm) s_norm[row] = n;
         }
       }
@@ -565,18 +584,24 @@ __device__ __forceinline__ void enc_store_dense(const EncStore &st, int b, int h
                       st.dn ? st.dn + b * st.dn_b + h * st.dn_h + dst0 : nullptr);
 }
 
+template <bool PLAIN, typename T>
+__device__ __forceinline__ void enc_put(T v, T *p) {
+  if (PLAIN) *p = v;
+  else __builtin_nontemporal_store(v, p);
+}
+
 // ALL: codes, 4-bit records, weights and cluster sizes are all written (the caller's pointers are all set), so the
 // loop body has no branch around a store.  Loads and stores retire through one in-order counter; with a store that
 // may or may not have been issued after the load of the next key, the only safe wait for that key is "everything
 // outstanding", stores included.  Without the branches the wait names the exact count and the stores stay in flight.
 // STORE (with ALL): the launch also stores the prompt's rows, see EncStore.
-template <bool BF16, bool ALL, int STORE>
+template <bool BF16, bool ALL, int STORE, bool SPREAD = false>
 __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEncWavesPerSimd, kEncWavesPerSimd))) void pkv_encode_kernel(
     const void *__restrict__ keys, int n_kv_heads, int64_t n_keys, int64_t k_stride_b, int64_t k_stride_h,
     int64_t k_stride_key, const float *__restrict__ signs, uint8_t *__restrict__ codes, int64_t cs_b, int64_t cs_h,
     int64_t cs_key, int64_t cs_sub, uint8_t *__restrict__ nib, int64_t ns_b, int64_t ns_h, int64_t ns_key,
     int64_t ns_sub, uint16_t *__restrict__ weight, int64_t ws_b, int64_t ws_h, int64_t ws_key, int64_t ws_sub,
-    int32_t *__restrict__ cluster_counts, int64_t cc_b, int64_t cc_h, int keys_per_wg, EncStore st) {
+    int32_t *__restrict__ cluster_counts, int64_t cc_b, int64_t cc_h, EncStore st) {
   const bool has_nib = ALL || nib, has_weight = ALL || weight, has_hist = ALL || cluster_counts;
   const int b = STORE ? (int)blockIdx.z : (int)blockIdx.y / n_kv_heads, h = STORE ? (int)blockIdx.y : (int)blockIdx.y % n_kv_heads;
   if (STORE && (int)blockIdx.x >= st.n_blocks) {
@@ -604,14 +629,21 @@ __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEn
   }
   if (has_hist)
     for (int i = tid; i < 16 * 256; i += kEncThreads) s_hist[i] = 0;
+  // the workgroup's runs are run0, run0 + run_step, ...; its key i is key i % kEncRun of its run i / kEncRun, and last is the
+  // i of its last key.  Only the head's last run may be ragged, and whoever has it has it last.
+  const int64_t run0 = SPREAD ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * kEncRuns, run_step = SPREAD ? st.n_blocks : 1;
+  const int64_t n_runs = (n_keys + kEncRun - 1) / kEncRun;
+  int64_t mine = (n_runs - run0 + run_step - 1) / run_step;
+  mine = mine < kEncRuns ? mine : kEncRuns;  // >= 1 by the grid's construction
+  const int64_t end_run = run0 + (mine - 1) * run_step;
+  const int last = (int)((mine - 1) * kEncRun + (end_run == n_runs - 1 ? n_keys - end_run * kEncRun : kEncRun)) - 1;
   if (STORE) {
     constexpr int row_bytes = BF16 ? 256 : 512;
-    const int64_t i0 = (int64_t)blockIdx.x * keys_per_wg;
-    enc_copy_rows<BF16>(st.v + b * st.v_b + h * st.v_h + i0 * st.v_key, st.v_key, st.zv + b * st.z_b + h * st.z_h + i0 * row_bytes,
-                        (int)(n_keys - i0 < keys_per_wg ? n_keys - i0 : keys_per_wg),
-                        st.zn ? st.zn + b * st.zn_b + h * st.zn_h + i0 * st.zn_key : nullptr, st.zn_key,
+    const int64_t i0 = run0 * kEncRun;
+    enc_copy_rows<BF16, SPREAD>(st.v + b * st.v_b + h * st.v_h + i0 * st.v_key, st.v_key, st.zv + b * st.z_b + h * st.z_h + i0 * row_bytes,
+                                last + 1, st.zn ? st.zn + b * st.zn_b + h * st.zn_h + i0 * st.zn_key : nullptr, st.zn_key,
                         st.zn2 ? st.zn2 + b * st.zn2_b + h * st.zn2_h + i0 : nullptr,
-                        STORE == kEncStoreRecords && st.record_norm ? s_norm : nullptr);
+                        STORE == kEncStoreRecords && st.record_norm ? s_norm : nullptr, (run_step - 1) * kEncRun);
   }
   __syncthreads();
 
@@ -626,38 +658,38 @@ __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEn
   const float scale = (__builtin_popcount((unsigned)s) & 1) ? -PKV_HADAMARD_SCALE : PKV_HADAMARD_SCALE;
   const bool rerank = ALL || nib || weight;
 
-  // Addresses are a wave-uniform base, which advances by one iteration's 16 keys through scalar adds, plus a
+  // Addresses are a wave-uniform base, that of the iteration's first key, plus a
   // 32-bit lane offset that never changes (the launcher checks that the offsets fit).  Lanes past the end of a
   // ragged last block load its last key (all lanes take part in the lane-crossing steps); they store nothing, or,
   // in the ALL form, that key's results once more.
-  const int64_t key_begin = (int64_t)blockIdx.x * keys_per_wg;  // < n_keys by the grid's construction
-  const int last = (int)((n_keys - key_begin < keys_per_wg) ? n_keys - key_begin : keys_per_wg) - 1;
+  constexpr int kRunIters = kEncRun / kEncKeysPerIter;
+  auto key_at = [&](int it) {  // first key of an iteration; uniform
+    return (run0 + (int64_t)(it / kRunIters) * run_step) * kEncRun + it % kRunIters * kEncKeysPerIter;
+  };
   constexpr int esize = BF16 ? 2 : 4;
-  const char *k_base = (const char *)keys + ((int64_t)b * k_stride_b + (int64_t)h * k_stride_h + key_begin * k_stride_key) * esize;
-  uint8_t *c_base = codes + (int64_t)b * cs_b + (int64_t)h * cs_h + key_begin * cs_key;
-  uint8_t *n_base = has_nib ? nib + (int64_t)b * ns_b + (int64_t)h * ns_h + key_begin * ns_key : nullptr;
-  char *w_base = has_weight ? (char *)(weight + (int64_t)b * ws_b + (int64_t)h * ws_h + key_begin * ws_key) : nullptr;
+  const char *k_base = (const char *)keys + ((int64_t)b * k_stride_b + (int64_t)h * k_stride_h) * esize;
+  uint8_t *c_base = codes + (int64_t)b * cs_b + (int64_t)h * cs_h;
+  uint8_t *n_base = has_nib ? nib + (int64_t)b * ns_b + (int64_t)h * ns_h : nullptr;
+  char *w_base = has_weight ? (char *)(weight + (int64_t)b * ws_b + (int64_t)h * ws_h) : nullptr;
   const uint32_t key_bytes = (uint32_t)(k_stride_key * esize), blk_off = (uint32_t)(8 * s * esize);
   const uint32_t k_lane = (uint32_t)kq * key_bytes + blk_off;
   const uint32_t c_lane = (uint32_t)(kq * cs_key + s * cs_sub), n_lane = (uint32_t)(kq * ns_key + s * ns_sub),
                  w_blk = STORE == kEncStoreRecords ? (uint32_t)(4 * (s >> 1) + (s & 1) * 32) : (uint32_t)(2 * s * ws_sub),
                  w_lane = (uint32_t)(2 * kq * ws_key) + w_blk;
-  char *z_base = STORE ? st.zk + b * st.z_b + h * st.z_h + key_begin * (128 * esize) : nullptr;
+  char *z_base = STORE ? st.zk + b * st.z_b + h * st.z_h : nullptr;
   const uint32_t z_lane = (uint32_t)kq * (128 * esize) + blk_off;
-  const int64_t k_step = (int64_t)kEncKeysPerIter * k_stride_key * esize, c_step = (int64_t)kEncKeysPerIter * cs_key,
-                n_step = (int64_t)kEncKeysPerIter * ns_key, w_step = (int64_t)kEncKeysPerIter * ws_key * 2;
   // A wave keeps the keys of its next kEncAhead iterations in flight, each in a register set of its own: set j holds
   // iterations j, j + kEncAhead, ... and is refilled as soon as its key has been copied out.  (A ring whose sets are
   // copied into each other waits for the newest load at every copy and hides one iteration of latency whatever its
   // depth.)  Loads are never skipped - past the block's end they fetch its last iteration again - because a load that
   // may or may not have been issued makes every later wait of the in-order counter a wait for everything.
   constexpr int kW = BF16 ? 1 : 2;  // 16-byte words per lane and key
-  constexpr int kEncAhead = BF16 ? kEncAheadBf16 : kEncAheadF32;
+  constexpr int kEncAhead = !BF16 ? kEncAheadF32 : SPREAD ? kEncAheadBf16Spread : kEncAheadBf16;
   const int n_iter = last / kEncKeysPerIter + 1;
   pkv_u32x4 raw[kEncAhead][kW];
   auto load_iter = [&](int it, pkv_u32x4 (&reg)[kW]) {
     const int it_c = it < n_iter ? it : n_iter - 1;  // uniform
-    const char *base = k_base + (int64_t)it_c * k_step;
+    const char *base = k_base + key_at(it_c) * key_bytes;
     const int lim = last - it_c * kEncKeysPerIter;  // the iteration holds the block's keys 16 it_c .. 16 it_c + lim
     uint32_t off = k_lane;
     if (lim < kEncKeysPerIter - 1) off = kq <= lim ? k_lane : (uint32_t)lim * key_bytes + blk_off;  // uniform: it is ragged
@@ -672,7 +704,7 @@ __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEn
     for (int q = 0; q < kW; ++q) cur[q] = reg[q];
     load_iter(it + kEncAhead, reg);
     if (STORE) {  // lanes past a ragged end hold the block's last key and store that row once more
-      char *zb = z_base + (int64_t)it * (kEncKeysPerIter * 128 * esize);
+      char *zb = z_base + key_at(it) * (128 * esize);
       uint32_t z_off = z_lane;
       if (last - first < kEncKeysPerIter - 1) z_off = (uint32_t)(kq < last - first ? kq : last - first) * (128 * esize) + blk_off;
       asm volatile("" : "+v"(z_off));
@@ -710,8 +742,9 @@ __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEn
 
     // the empty statement keeps the lane offsets apart from the bases, so that the stores address
     // scalar base + lane offset instead of three 64-bit lane pointers that would each need an add per iteration
-    uint8_t *cb = c_base + (int64_t)it * c_step, *nb = n_base + (int64_t)it * n_step;
-    char *wb = w_base + (int64_t)it * w_step;
+    const int64_t key0 = key_at(it);
+    uint8_t *cb = c_base + key0 * cs_key, *nb = n_base + key0 * ns_key;
+    char *wb = w_base + key0 * ws_key * 2;
     uint32_t c_off = c_lane, n_off = n_lane, w_off = w_lane;
     if (ALL) {
       // No branch around the stores (see above): a lane past the end of a ragged block holds the block's last key
@@ -724,16 +757,16 @@ __global__ __launch_bounds__(kEncThreads) __attribute__((amdgpu_waves_per_eu(kEn
       }
       asm volatile("" : "+v"(c_off), "+v"(n_off), "+v"(w_off));
       // written once and not read again by this launch: streaming stores (5 - 8 % on two of three shapes)
-      __builtin_nontemporal_store((uint8_t)o.code, cb + c_off);
-      __builtin_nontemporal_store(o.packed, (uint32_t *)(nb + n_off));
+      enc_put<SPREAD>((uint8_t)o.code, cb + c_off);
+      enc_put<SPREAD>(o.packed, (uint32_t *)(nb + n_off));
       if (STORE == kEncStoreRecords) {
         // the second half of the record as sixteen words: even blocks hold two weights, block 1 the value norm
         const uint32_t pair = o.wbits | (pkv_lane_xor<1>(o.wbits) << 16);
         const float norm = st.record_norm ? s_norm[first + (kq < last - first ? kq : last - first)] : 0.f;
         const uint32_t word = (s & 1) ? (s == 1 ? __float_as_uint(norm) : 0u) : pair;
-        __builtin_nontemporal_store(word, (uint32_t *)(wb + w_off));
+        enc_put<SPREAD>(word, (uint32_t *)(wb + w_off));
       } else {
-        __builtin_nontemporal_store((uint16_t)o.wbits, (uint16_t *)(wb + w_off));
+        enc_put<SPREAD>((uint16_t)o.wbits, (uint16_t *)(wb + w_off));
       }
       if (active) atomicAdd(&s_hist[s * 256 + o.code], 1u);
     } else if (active) {
@@ -817,7 +850,7 @@ extern "C" int pkv_encode_append(const void *keys, int dtype, int bs, int n_kv_h
 #define PKV_ENC(BF, ALL)                                                                                               \
   hipLaunchKernelGGL((pkv_encode_kernel<BF, ALL, kEncNoStore>), grid, dim3(kEncThreads), 0, (hipStream_t)stream, keys, n_kv_heads,  \
                      n_keys, k_stride_b, k_stride_h, k_stride_key, signs, codes, cs_b, cs_h, cs_key, cs_sub, nib, ns_b, \
-                     ns_h, ns_key, ns_sub, weight, ws_b, ws_h, ws_key, ws_sub, cluster_counts, cc_b, cc_h, (int)per_wg, EncStore())
+                     ns_h, ns_key, ns_sub, weight, ws_b, ws_h, ws_key, ws_sub, cluster_counts, cc_b, cc_h, EncStore())
   const bool all = nib && weight && cluster_counts;
   if (dtype == PKV_DTYPE_BF16) {
     if (all) PKV_ENC(true, true); else PKV_ENC(true, false);
@@ -891,17 +924,19 @@ extern "C" int pkv_prefill_store(const pkv_prefill_args *a, void *stream) {
   if (records && norm_in_record) st.record_norm = 1, st.zn = nullptr;
   const int dense_blocks = (st.n_sink + kEncDenseRows - 1) / kEncDenseRows + (st.n_tail + kEncDenseRows - 1) / kEncDenseRows;
   const dim3 grid((unsigned)(st.n_blocks + dense_blocks), (unsigned)a->n_kv_heads, (unsigned)a->bs);
-#define PKV_ENC_ST(BF, MODE)                                                                                           \
-  hipLaunchKernelGGL((pkv_encode_kernel<BF, true, MODE>), grid, dim3(kEncThreads), 0, (hipStream_t)stream,              \
+  const bool spread = (a->n_encode * a->n_kv_heads) * a->bs * (4 * 128 * es + 144) > kEncSpreadBytes;
+#define PKV_ENC_ST(BF, MODE, SPREAD)                                                                                   \
+  hipLaunchKernelGGL((pkv_encode_kernel<BF, true, MODE, SPREAD>), grid, dim3(kEncThreads), 0, (hipStream_t)stream,      \
                      k + a->n_sink * st.k_key, a->n_kv_heads, a->n_encode, a->k_stride_b, a->k_stride_h, a->k_stride_key, \
                      a->signs, a->codes, a->cs_b, a->cs_h, a->cs_key, a->cs_sub, a->nib, a->ns_b, a->ns_h, a->ns_key,   \
-                     a->ns_sub, a->weight, a->ws_b, a->ws_h, a->ws_key, a->ws_sub, a->cluster_counts, a->cc_b, a->cc_h, \
-                     kEncKeysPerWg, st)
+                     a->ns_sub, a->weight, a->ws_b, a->ws_h, a->ws_key, a->ws_sub, a->cluster_counts, a->cc_b, a->cc_h, st)
+#define PKV_ENC_ST2(BF, MODE) if (spread) PKV_ENC_ST(BF, MODE, true); else PKV_ENC_ST(BF, MODE, false)
   if (bf) {
-    if (records) PKV_ENC_ST(true, kEncStoreRecords); else PKV_ENC_ST(true, kEncStoreRows);
+    if (records) { PKV_ENC_ST2(true, kEncStoreRecords); } else { PKV_ENC_ST2(true, kEncStoreRows); }
   } else {
-    if (records) PKV_ENC_ST(false, kEncStoreRecords); else PKV_ENC_ST(false, kEncStoreRows);
+    if (records) { PKV_ENC_ST2(false, kEncStoreRecords); } else { PKV_ENC_ST2(false, kEncStoreRows); }
   }
+#undef PKV_ENC_ST2
 #undef PKV_ENC_ST
   PKV_LAUNCH_CHECK("pkv_encode_kernel");
   return PKV_OK;

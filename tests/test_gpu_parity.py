@@ -2204,3 +2204,39 @@ def test_query_prep_ranks_equal_and_zero_scores_by_id(ops, dtype, kind):
             want_ids = O.rank_centroids(qhat[b, h].cpu().numpy(), od)
             assert np.array_equal(ids[b, h].cpu().numpy(), want_ids), (b, h)
             assert np.array_equal(lut[b, h].cpu().numpy(), O.tier_lut(want_ids, cc[b, h].numpy(), tiers)), (b, h)
+
+
+@pytest.mark.parametrize("dtype,rows", [(torch.bfloat16, 8), (torch.float32, 5)])
+@pytest.mark.parametrize("n_enc", [129, 300, 513])
+@pytest.mark.parametrize("layout", ["records", "subspace"])
+def test_prefill_store_of_many_keys(ops, dtype, rows, n_enc, layout):
+    """A call that moves more than 576 MiB spreads a workgroup's keys over its head; rows, index, cluster sizes and norms are
+    those of calls for a few samples each, which keep them together.  One run and a remainder of keys per head up to three
+    workgroups of two runs."""
+    es, cap = (2, n_enc + 3) if dtype == torch.bfloat16 else (4, n_enc + 3)
+    bs = (576 << 20) // ((512 * es + 144) * rows * n_enc) + 1
+    _say(f"prefill_store of many keys {dtype} bs={bs} heads={rows} {n_enc} {layout}")
+    gen = torch.Generator(device=DEV).manual_seed(n_enc)
+    k, v = (torch.randn(bs, 2 + n_enc + 1, rows, 128, generator=gen, device=DEV).to(dtype).permute(0, 2, 1, 3) for _ in range(2))
+    signs = ops.srht_signs(DEV)
+
+    def store(step):
+        zk, zv = (torch.full((bs, rows, cap, 128), 7.0, dtype=dtype, device=DEV) for _ in range(2))
+        dk, dv = (torch.full((bs, rows, 3, 128), 7.0, dtype=dtype, device=DEV) for _ in range(2))
+        cc = torch.zeros(bs, rows, 16, 256, dtype=torch.int32, device=DEV)
+        if layout == "records":
+            _, nib, _, cb, k4, kw = ops.alloc_keymajor(bs, rows, cap, DEV)
+            zn = ops.record_value_norm_view(nib)
+        else:
+            cb, k4 = (torch.zeros(bs, rows, 16, cap, *e, dtype=torch.uint8, device=DEV) for e in ((), (4,)))
+            kw, zn = torch.zeros(bs, rows, 16, cap, dtype=torch.bfloat16, device=DEV), torch.zeros(bs, rows, cap, device=DEV)
+        zn2 = torch.zeros(bs, rows, cap, device=DEV)
+        for b in range(0, bs, step):
+            s = slice(b, b + step)
+            ops.prefill_store(k[s], v[s], 2, n_enc, signs, (dk[s], dv[s]), 2, (zk[s], zv[s]),
+                              (cb[s, ..., :n_enc], k4[s, :, :, :n_enc], kw[s, ..., :n_enc], cc[s]),
+                              zone_vnorm=zn[s, :, :n_enc], zone_vnorm2=zn2[s, :, :n_enc])
+        return zk, zv, dk, dv, cc, cb, k4, kw.view(torch.int16), zn, zn2
+
+    for a, b in zip(store(bs), store(bs // 3 + 1)):
+        assert torch.equal(a, b)
