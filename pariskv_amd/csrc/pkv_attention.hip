@@ -28,6 +28,13 @@ namespace {
 
 constexpr int kAttThreads = 256;
 constexpr int kAttKeysPerIter = kAttThreads / 16;  // 16 keys per workgroup step
+// A call whose caller keeps counters takes one launch, the last workgroup of a row merging, up to this many splits a row and
+// workgroups in all.  A decode step over a short context waits for its launches' host time (3.4 us each), not for the GPU: 8 rows x
+// 1500 keys, append and attention, 14.1 us a step where two launches for the attention took 16.7.  Back to back and with nothing else
+// to launch, us, one / two launches: 8 rows x 300 keys 7.0 / 9.7, 1600 8.0 / 9.9, 16 rows x 1600 9.0 / 9.6, 32 x 1600 10.1 / 9.3,
+// 8 x 2500 9.7 / 9.7, 4000 11.0 / 9.9; the GPU alone, without the host, 6.7 / 6.2, 7.7 / 6.5, 8.9 / 6.8, 10.2 / 8.5, 9.6 / 7.7, 11.0 / 7.7.
+// fp32 loses there as well (12 rows x 865 keys, 7 heads, 11.5 / 10.7) and keeps its two launches.
+constexpr int kWholeSplits = 16, kWholeWorkgroups = 256;
 constexpr int kAttUnroll = 2;                      // keys per 16-lane group per step
 
 struct AttSegs {
@@ -122,6 +129,61 @@ __device__ __forceinline__ void load8(const void *base, int64_t elem_off, float 
   Raw8 r;
   load_raw8(base, elem_off, r);
   expand8(r, x);
+}
+
+// WHOLE launches: the splits of a row are merged, as pkv_attn_merge_kernel merges them and to the same bits, by the workgroup
+// that stores its partial result last.  gridDim.x workgroups of a row come here with their partial results stored for other
+// dies (att_put); *arrived is zero before the first of them and after the last.  Nobody waits: a workgroup that is not the last
+// one ends.  One chain of store acknowledgement, count and dependent loads, so every load is requested before the weights are
+// known; see kWholeSplits for what it costs and saves.
+__device__ __forceinline__ void att_last_merges(const float *ws, int row, int group, uint32_t *arrived, uint16_t *out) {
+  constexpr int kThreads = kMfmaWaves * PKV_WAVE;
+  const int tid = threadIdx.x, n_splits = gridDim.x, lane = tid & (PKV_WAVE - 1);
+  __shared__ uint32_t s_before;
+  __shared__ float s_w[8][PKV_WAVE];  // weight of split s for head g, already divided by the total
+  pkv_wait_vmem();
+  __syncthreads();
+  if (tid == 0) s_before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (s_before != (uint32_t)n_splits - 1) return;  // uniform
+  if (tid == 0) __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const float *rowp = ws + (int64_t)row * n_splits * group * kPartStride;
+  const int next = group * kPartStride;
+  auto get = [](const float *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+  // a thread's (head, dim) pairs, two at a time: four heads take one turn
+  for (int base = 0; base < group * 128; base += 2 * kThreads) {
+    float part[2][kWholeSplits];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int e = base + u * kThreads + tid < group * 128 ? base + u * kThreads + tid : tid & 127;
+      const float *po = rowp + (e >> 7) * kPartStride + 2 + (e & 127);
+#pragma unroll
+      for (int s = 0; s < kWholeSplits; ++s) part[u][s] = get(po + (s < n_splits ? s : 0) * next);
+    }
+    if (base == 0) {
+      for (int g = tid / PKV_WAVE; g < group; g += kMfmaWaves) {  // one wave per head: lane = split
+        const bool live = lane < n_splits;
+        const float *p = rowp + (live ? lane : 0) * next + g * kPartStride;
+        const float m0 = get(p), l0 = get(p + 1);
+        const float mi = live ? m0 : kNegBig, li = live ? l0 : 0.f;
+        const float c = exp2f(mi - pkv_wave_max(mi));
+        const float two = fmaf(li, c, pkv_lane_xor_f<1>(li * c));
+        const float tot = pkv_pair_add<32>(pkv_pair_add<16>(pkv_pair_add<8>(pkv_pair_add<4>(pkv_pair_add<2>(two)))));
+        s_w[g][lane] = c / tot;
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int e = base + u * kThreads + tid;
+      if (e >= group * 128) break;
+      const int g = e >> 7, d = e & 127;
+      float os = 0.f;
+#pragma unroll
+      for (int s = 0; s < kWholeSplits; ++s) os = fmaf(part[u][s], s < n_splits ? s_w[g][s] : 0.f, os);
+      out[((int64_t)row * group + g) * 128 + d] = pkv_f32_to_bf16_bits(os);
+    }
+  }
 }
 
 // Splits are of 64 keys while the key set allows: a launch is one chain of dependent loads with some 1000 instructions behind
@@ -277,10 +339,10 @@ __global__ __launch_bounds__(kAttThreads) void pkv_attn_partial_kernel(const voi
 
 // grid (splits, KV heads, batch).  Decode step, us, with four-way pointer selection per row / with places by lane exchange:
 // 8 rows x 693 attended keys 30.2 / 27.7, 8 x 1188 (4 layers) 136.5 / 124.2, 64 x 887 (2 layers) 133.4 / 122.8.
-template <bool INDEXED, typename SEGS>
+template <bool INDEXED, typename SEGS, bool WHOLE>
 __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_kernel(
     const void *__restrict__ q, int group, SEGS segs, int64_t total, const int32_t *__restrict__ row_keys, int uniform,
-    int64_t per_split, float scale_log2e, float *__restrict__ ws) {
+    int64_t per_split, float scale_log2e, float *__restrict__ ws, uint32_t *arrivals, void *out) {
   const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z, row = b * (int)gridDim.y + h;
   constexpr bool ONE = __is_same(SEGS, AttOne);
   const int lane = threadIdx.x & (PKV_WAVE - 1), wave = threadIdx.x / PKV_WAVE;
@@ -324,7 +386,8 @@ __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_k
 
   l_part = pkv_pair_add<32>(pkv_pair_add<16>(l_part));
   float *part = ws + ((int64_t)row * gridDim.x + split) * group * kPartStride;
-  att_merge_waves(group, m_run, l_part, o, part, kPartStride, part + 2, kPartStride);
+  att_merge_waves<WHOLE>(group, m_run, l_part, o, part, kPartStride, part + 2, kPartStride);
+  if (WHOLE) att_last_merges(ws, row, group, arrivals + row, (uint16_t *)out);
 }
 
 // grid R, G*128 threads: merge the splits (at most 64) and normalise.
@@ -468,7 +531,7 @@ static int collect_segments(int dtype, const pkv_attn_segment *segments, int n_s
 
 static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_segment *segments,
                             int n_segments, const int32_t *row_keys, int uniform, float scale, void *out, void *ws,
-                            size_t ws_bytes, void *stream) {
+                            size_t ws_bytes, uint32_t *arrivals, void *stream) {
   PKV_REQUIRE(q && segments && out && ws, "pkv_decode_attention: null pointer");
   PKV_REQUIRE(dtype == PKV_DTYPE_F32 || dtype == PKV_DTYPE_BF16, "unknown dtype %d", dtype);
   PKV_REQUIRE(bs > 0 && n_kv_heads > 0 && (int64_t)bs * n_kv_heads <= 65535, "bad shape bs=%d kv_heads=%d", bs,
@@ -501,17 +564,23 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
   dim3 grid((unsigned)n_splits, (unsigned)rows);
   AttOne one;
   const bool is_one = as_one_tensor(sg, bf ? 2 : 4, one);
+  const bool whole = arrivals && bf && n_splits <= kWholeSplits && rows * n_splits <= kWholeWorkgroups;
   if (bf) {
     const dim3 grid3((unsigned)n_splits, (unsigned)n_kv_heads, (unsigned)bs);
-#define PKV_ATT_MFMA(IDX, S)                                                                                                    \
-  hipLaunchKernelGGL((pkv_attn_partial_mfma_kernel<IDX, decltype(S)>), grid3, dim3(kMfmaWaves * PKV_WAVE), 0, s, q, group, S, total, \
-                     row_keys, uniform, per_split, scale_log2e, (float *)ws)
+#define PKV_ATT_MFMA_W(IDX, S, WHOLE)                                                                                           \
+  hipLaunchKernelGGL((pkv_attn_partial_mfma_kernel<IDX, decltype(S), WHOLE>), grid3, dim3(kMfmaWaves * PKV_WAVE), 0, s, q, group, S, \
+                     total, row_keys, uniform, per_split, scale_log2e, (float *)ws, arrivals, out)
+#define PKV_ATT_MFMA(IDX, S)                                                         \
+  do {                                                                               \
+    if (whole) PKV_ATT_MFMA_W(IDX, S, true); else PKV_ATT_MFMA_W(IDX, S, false);     \
+  } while (0)
     if (is_one) {
       if (indexed) PKV_ATT_MFMA(true, one); else PKV_ATT_MFMA(false, one);
     } else {
       if (indexed) PKV_ATT_MFMA(true, sg); else PKV_ATT_MFMA(false, sg);
     }
 #undef PKV_ATT_MFMA
+#undef PKV_ATT_MFMA_W
   } else {
     // The KV head's other query heads in workgroups beside the first four's, in one launch: 12 rows x 865 keys, seven
     // heads, 2 x 8.0 us as two launches one after the other; the decode step around it (9001 keys) 48.3 -> 43 us.
@@ -534,6 +603,7 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
 #undef PKV_ATT
   }
   PKV_LAUNCH_CHECK("pkv_attn_partial_kernel");
+  if (whole) return PKV_OK;
   if (bf)
     hipLaunchKernelGGL(pkv_attn_merge_kernel<true>, dim3((unsigned)rows), dim3(group * 128), 0, s, (const float *)ws,
                        n_splits, group, out);
@@ -547,14 +617,22 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
 extern "C" int pkv_decode_attention(const void *q, int dtype, int bs, int n_kv_heads, int group,
                                     const pkv_attn_segment *segments, int n_segments, const int32_t *row_keys,
                                     float scale, void *out, void *ws, size_t ws_bytes, void *stream) {
-  return decode_attention(q, dtype, bs, n_kv_heads, group, segments, n_segments, row_keys, 0, scale, out, ws, ws_bytes, stream);
+  return decode_attention(q, dtype, bs, n_kv_heads, group, segments, n_segments, row_keys, 0, scale, out, ws, ws_bytes, nullptr, stream);
 }
 
 extern "C" int pkv_decode_attention_run(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_args *a,
                                         void *stream) {
   PKV_REQUIRE(a != nullptr, "pkv_decode_attention: null args");
   return decode_attention(q, dtype, bs, n_kv_heads, group, a->segments, a->n_segments, a->row_keys,
-                          a->row_keys_uniform ? bs * n_kv_heads : 0, a->scale, a->out, a->ws, a->ws_bytes, stream);
+                          a->row_keys_uniform ? bs * n_kv_heads : 0, a->scale, a->out, a->ws, a->ws_bytes, nullptr, stream);
+}
+
+extern "C" int pkv_decode_attention_counted(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_args *a,
+                                            uint32_t *arrivals, void *stream) {
+  PKV_REQUIRE(a != nullptr && arrivals != nullptr, "pkv_decode_attention_counted: null pointer");
+  PKV_REQUIRE(pkv_aligned(arrivals, 4), "arrivals must be 4-byte aligned");
+  return decode_attention(q, dtype, bs, n_kv_heads, group, a->segments, a->n_segments, a->row_keys,
+                          a->row_keys_uniform ? bs * n_kv_heads : 0, a->scale, a->out, a->ws, a->ws_bytes, arrivals, stream);
 }
 
 static bool meets(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {

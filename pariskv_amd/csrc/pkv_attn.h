@@ -174,9 +174,17 @@ __device__ __forceinline__ void att_step_mfma(const char *kbase, const char *vba
   }
 }
 
+// a value for a later launch, or (HANDED) for another workgroup of this one, whatever die that runs on
+template <bool HANDED>
+__device__ __forceinline__ void att_put(float *p, float v) {
+  if (HANDED) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else *p = v;
+}
+
 // Merge of the waves of a workgroup: every wave leaves (max, sum, output) of its keys in LDS, then the workgroup's 256 threads
 // combine them, one (head, dim) pair at a time.  group <= 8.
-// ml / out: of head 0; the next head's lie ml_stride / out_stride floats on.
+// ml / out: of head 0; the next head's lie ml_stride / out_stride floats on.  HANDED: another workgroup of the launch reads them.
+template <bool HANDED = false>
 __device__ __forceinline__ void att_merge_waves(int group, float m_run, float l_part, const pkv_f32x4 (&o)[8], float *ml, int ml_stride,
                                                 float *out, int out_stride) {
   PKV_ATT_CONTRACT
@@ -205,8 +213,8 @@ __device__ __forceinline__ void att_merge_waves(int group, float m_run, float l_
       ls = fmaf(s_l[w][g], c, ls);
       os = fmaf(s_o[w][g][d], c, os);
     }
-    out[g * out_stride + d] = os;
-    if (d == 0) ml[g * ml_stride] = mn, ml[g * ml_stride + 1] = ls;
+    att_put<HANDED>(out + g * out_stride + d, os);
+    if (d == 0) att_put<HANDED>(ml + g * ml_stride, mn), att_put<HANDED>(ml + g * ml_stride + 1, ls);
   }
 }
 // ---- a decode step's attention in two parts ----

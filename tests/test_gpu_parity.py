@@ -2240,3 +2240,36 @@ def test_prefill_store_of_many_keys(ops, dtype, rows, n_enc, layout):
 
     for a, b in zip(store(bs), store(bs // 3 + 1)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype,group", [(torch.bfloat16, 4), (torch.bfloat16, 8), (torch.bfloat16, 1), (torch.float32, 2), (torch.float32, 7)])
+@pytest.mark.parametrize("n", [1, 127, 129, 2048, 2049, 6000])
+def test_bound_attention_merges_in_its_own_launch(ops, dtype, group, n):
+    """The kept dense attention (the last workgroup of a row merges, while the splits are few) and the two launches of
+    DecodeAttention.run: the same bits, launch after launch and in a replayed graph, and the counters are zero again."""
+    _say(f"bound attention {dtype} group={group} {n}")
+    bs, H = 2, 3
+    g = torch.Generator(device=DEV).manual_seed(n + group)
+    k, v = (torch.randn(bs, H, n + 9, 128, generator=g, device=DEV).to(dtype) for _ in range(2))
+    att = ops.DecodeAttention(bs, H, group, n + 9, DEV)
+    qs = [torch.randn(bs, 1, H * group, 128, generator=g, device=DEV).to(dtype) for _ in range(3)]
+    bound = ops.BoundAttention(att, qs[0], [(k, v, 2, n)])
+    for q, m in zip(qs, (n, max(1, n - 60), n)):
+        bound.segs[0].n_rows = m
+        got = bound.launch(q)
+        assert torch.equal(got, att.run(q, [(k, v, 2, m)]))
+        assert not torch.any(att.arrivals)
+    graph, q = torch.cuda.CUDAGraph(), qs[0].clone()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        bound.launch(q)
+    torch.cuda.current_stream().wait_stream(side)
+    with torch.cuda.graph(graph):
+        out = bound.launch(q)
+    for other in qs:
+        q.copy_(other)
+        graph.replay()
+        want = att.run(other, [(k, v, 2, n)])
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and not torch.any(att.arrivals)
