@@ -434,6 +434,107 @@ __global__ __launch_bounds__(256) void pkv_counts_to_u8_kernel(const int32_t *__
                         chunk_suf + ((int64_t)row * gridDim.x + chunk) * 128);
 }
 
+// Both steps of the bucket top-k for a row of up to 4096 NB values, by one workgroup: a thread holds four neighbouring values of
+// each block of 4096 as clamped bytes, so nothing is read twice and neither counts nor histograms go through memory.
+// grid (rows).  Bound by what one CU's 16 waves issue, 1.1 us a block of 4096 behind 1.9 for the launch and the chain of phases:
+// hence a histogram copy per lane (16 copies: 8.8 instead of 6.6 us for 20011 values) and byte-parallel comparisons.
+constexpr int kBucketThreads = 1024, kBucketBlock = 4 * kBucketThreads;
+template <int NB>
+__global__ __launch_bounds__(kBucketThreads) void pkv_bucket_row_kernel(const int32_t *__restrict__ x, int64_t x_stride, int len,
+                                                                        int k, int64_t *__restrict__ out) {
+  constexpr int kWaves = kBucketThreads / PKV_WAVE;
+  constexpr uint32_t kTops = 0x80808080u, kOnes = 0x01010101u;
+  const int tid = threadIdx.x, lane = pkv_lane(), wave = tid / PKV_WAVE;
+  const int32_t *xr = x + (int64_t)blockIdx.x * x_stride;
+  __shared__ __align__(16) uint32_t s_hist[128 * PKV_WAVE];  // a copy per lane: no two lanes on one bank
+  __shared__ uint32_t s_suf[129], s_theta;
+  __shared__ uint32_t s_tot[NB * kWaves];
+  int v[NB][4];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int at = i * kBucketBlock + 4 * tid;
+    if (at + 4 <= len) {
+      __builtin_memcpy(v[i], xr + at, 16);  // rows of odd length: any 4-byte alignment
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[i][e] = at + e < len ? xr[at + e] : 0;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 128 * PKV_WAVE / 4 / kBucketThreads; ++i) ((pkv_u32x4 *)s_hist)[tid + i * kBucketThreads] = pkv_u32x4{0, 0, 0, 0};
+  __syncthreads();
+  uint32_t w[NB];  // four clamped values
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int left = len - (i * kBucketBlock + 4 * tid);
+    int c[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c[e] = v[i][e] < 0 ? 0 : (v[i][e] > 127 ? 127 : v[i][e]);
+    w[i] = (uint32_t)(c[0] | c[1] << 8 | c[2] << 16 | c[3] << 24);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (i + 1 < NB || e < left) atomicAdd(&s_hist[c[e] * PKV_WAVE + lane], 1u);  // only the last block is ragged
+  }
+  __syncthreads();
+  {  // eight threads add up a value's copies
+    const pkv_u32x4 *h = (const pkv_u32x4 *)s_hist + tid * 2;
+    const pkv_u32x4 p = h[0], q = h[1];
+    uint32_t sum = p.x + p.y + p.z + p.w + q.x + q.y + q.z + q.w;
+    sum += pkv_lane_xor<1>(sum);
+    sum += pkv_lane_xor<2>(sum);
+    sum += pkv_lane_xor<4>(sum);
+    if ((tid & 7) == 0) s_suf[tid >> 3] = sum;
+    if (tid == 0) s_suf[128] = 0;
+  }
+  __syncthreads();
+  uint32_t incl = 0;
+  if (tid < 128) {  // suffix sums: thread t owns value 127 - t
+    incl = (uint32_t)pkv_wave_incl_scan((int)s_suf[127 - tid]);
+    if (tid == PKV_WAVE - 1) s_theta = incl;
+  }
+  __syncthreads();
+  if (tid < 128) s_suf[127 - tid] = incl + (tid >= PKV_WAVE ? s_theta : 0u);
+  __syncthreads();
+  if (tid < 128 && (int)s_suf[tid] >= k && (int)s_suf[tid + 1] < k) s_theta = (uint32_t)tid | s_suf[tid + 1] << 8;
+  __syncthreads();
+  const uint32_t theta = s_theta & 127u, n_gt = s_theta >> 8;
+  // per thread and block: top bits of the bytes above / at the threshold; their ranks in the two halves of a word
+  uint32_t gt[NB], eq[NB], excl[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int left = len - (i * kBucketBlock + 4 * tid);
+    const uint32_t live = i + 1 < NB || left >= 4 ? kTops : left <= 0 ? 0u : kTops >> (8 * (4 - left));
+    const uint32_t up = w[i] | kTops, ge = (up - theta * kOnes) & live;
+    gt[i] = (up - (theta + 1) * kOnes) & live;
+    eq[i] = ge & ~gt[i];
+    const uint32_t mine = (uint32_t)__popc(gt[i]) | (uint32_t)__popc(eq[i]) << 16;
+    const uint32_t wave_incl = (uint32_t)pkv_wave_incl_scan((int)mine);
+    if (lane == PKV_WAVE - 1) s_tot[i * kWaves + wave] = wave_incl;
+    excl[i] = wave_incl - mine;
+  }
+  __syncthreads();
+  if (wave == 0) {  // exclusive sums over blocks and waves, two entries a lane
+    const bool has = 2 * lane < NB * kWaves;
+    const uint32_t a = has ? s_tot[2 * lane] : 0u, b = has ? s_tot[2 * lane + 1] : 0u;
+    const uint32_t before = (uint32_t)pkv_wave_incl_scan((int)(a + b)) - (a + b);
+    if (has) s_tot[2 * lane] = before, s_tot[2 * lane + 1] = before + a;
+  }
+  __syncthreads();
+  int64_t *orow = out + (int64_t)blockIdx.x * k;
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const uint32_t base = s_tot[i * kWaves + wave] + excl[i];
+    uint32_t pg = base & 0xffffu, pe = n_gt + (base >> 16);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t g = gt[i] >> (8 * e + 7) & 1u, q = eq[i] >> (8 * e + 7) & 1u;
+      const uint32_t pos = g ? pg : pe;
+      if ((g | q) && pos < (uint32_t)k) orow[pos] = i * kBucketBlock + 4 * tid + e;
+      pg += g, pe += q;
+    }
+  }
+}
+
 __global__ void pkv_zero_u32_kernel(uint32_t *__restrict__ p, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0u;
@@ -2443,6 +2544,11 @@ static void bucket_ws_layout(int rows, int64_t len, int &chunk_keys, int64_t &cn
   total = off_row + pkv_align_up((size_t)rows * 128 * sizeof(uint32_t), 256);
 }
 
+// One launch instead of two where a row's workgroup is as fast as the chunks', or nearly.  us on the GPU, two launches / one: 16 rows
+// x 4096 5.5 / 3.2, x 9001 6.4 / 4.7, x 20011 7.4 / 6.6, x 32768 6.8 / 9.0; 64 rows x 32768 9.2 / 9.3, 256 rows 25.2 / 12.6.  A call by
+// itself, host included: 13.5 / 8.3, 16 rows x 32768 13.6 / 8.9.
+constexpr int kBucketMaxBlocks = 8, kBucketFewRowsBlocks = 6, kBucketManyRows = 64;
+
 extern "C" size_t pkv_bucket_topk_ws_bytes(int rows, int64_t len) {
   if (rows <= 0 || len <= 0) return 256;
   int ck;
@@ -2469,11 +2575,29 @@ extern "C" int pkv_bucket_topk(const int32_t *x, int64_t x_stride, int rows, int
     pkv_set_error("pkv_bucket_topk: workspace of %zu bytes (256-aligned) required, got %zu", tot, ws_bytes);
     return PKV_ENOMEM;
   }
+  const int blocks = (int)((len + kBucketBlock - 1) / kBucketBlock);
+  if (blocks <= (rows < kBucketManyRows ? kBucketFewRowsBlocks : kBucketMaxBlocks)) {
+#define PKV_BUCKET(NB)                                                                                                  \
+  hipLaunchKernelGGL(pkv_bucket_row_kernel<NB>, dim3((unsigned)rows), dim3(kBucketThreads), 0, s, x, x_stride, (int)len, (int)k, out)
+    switch (blocks) {
+      case 1: PKV_BUCKET(1); break;
+      case 2: PKV_BUCKET(2); break;
+      case 3: PKV_BUCKET(3); break;
+      case 4: PKV_BUCKET(4); break;
+      case 5: PKV_BUCKET(5); break;
+      case 6: PKV_BUCKET(6); break;
+      case 7: PKV_BUCKET(7); break;
+      default: PKV_BUCKET(8); break;
+    }
+#undef PKV_BUCKET
+    PKV_LAUNCH_CHECK("pkv_bucket_row_kernel");
+    return PKV_OK;
+  }
   uint8_t *cnt = (uint8_t *)ws;
   uint16_t *hist = (uint16_t *)((char *)ws + oh);
   uint32_t *row_suf = (uint32_t *)((char *)ws + orow);
   const int64_t n_chunks = (len + ck - 1) / ck;
-  // two launches: counts -> clamped bytes + chunk suffix histograms, then the select, which adds the chunks'
+  // longer rows, two launches: counts -> clamped bytes + chunk suffix histograms, then the select, which adds the chunks'
   // histograms up for the row totals itself (no atomics, so nothing has to be cleared first)
   (void)row_suf;
   hipLaunchKernelGGL(pkv_counts_to_u8_kernel, dim3((unsigned)n_chunks, (unsigned)rows), dim3(256), 0, s, x, x_stride,

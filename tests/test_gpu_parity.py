@@ -2273,3 +2273,20 @@ def test_bound_attention_merges_in_its_own_launch(ops, dtype, group, n):
         want = att.run(other, [(k, v, 2, n)])
         torch.cuda.synchronize()
         assert torch.equal(out, want) and not torch.any(att.arrivals)
+
+
+@pytest.mark.parametrize("rows,L", [(3, 1), (2, 3), (3, 64), (2, 4095), (2, 4096), (3, 4097), (1, 12287), (2, 20480), (5, 24573), (2, 24577),
+                                    (64, 24577), (65, 28673), (64, 32768), (64, 32769)])
+def test_bucket_topk_of_rows_of_every_length(ops, rows, L):
+    """One workgroup a row up to 24576 values (32768 from 64 rows on) and two launches beyond: the oracle's indices, in order, for
+    rows at any alignment, values outside [0, 127], few distinct values and every kind of k."""
+    _say(f"bucket_topk rows={rows} L={L}")
+    g = torch.Generator().manual_seed(rows * L)
+    wide = torch.randint(-40, 200, (rows, L + 3), generator=g, dtype=torch.int32)
+    for x in (wide[:, :L], torch.randint(3, 6, (rows, L), generator=g, dtype=torch.int32), torch.full((rows, L), 127, dtype=torch.int32)):
+        clamped = x.clamp(0, 127).numpy()
+        dev = wide.to(DEV)[:, 1:L + 1].copy_(x.to(DEV))   # rows an odd number of words apart, one word in
+        for k in sorted({1, (L + 1) // 2, max(1, L - 1), max(1, L // 7)}):
+            out = ops.bucket_topk(dev, k).cpu().numpy()
+            for r in {0, rows - 1}:
+                assert np.array_equal(out[r], np.arange(L) if k == L else O.select_candidates(clamped[r], k)[0])
