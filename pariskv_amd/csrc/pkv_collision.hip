@@ -35,6 +35,54 @@ __device__ __forceinline__ void load_lut(uint32_t *s_lut, const uint8_t *__restr
   ((pkv_u32x4 *)s_lut)[threadIdx.x] = g[threadIdx.x];
 }
 
+// The row's vote table from a ranking that the caller supplies, built by each workgroup of the row for itself: one wave takes four
+// subspaces, a lane four ranks of each.  s_max: 16 x 256 words.  Contains barriers, the last one behind the table's last word.
+struct ScanRanking {
+  const int64_t *ids;
+  int64_t si_b, si_h, si_sub;
+  const int32_t *cc;
+  int64_t cc_b, cc_h, cc_sub;
+  PkvTiers tiers;
+};
+__device__ __forceinline__ void lut_from_ranking(const ScanRanking &r, int b, int h, uint32_t *s_max, uint32_t *s_lut) {
+  const int tid = threadIdx.x, lane = pkv_lane(), sub0 = 4 * (tid / PKV_WAVE);
+  const int64_t *ids = r.ids + (int64_t)b * r.si_b + (int64_t)h * r.si_h + (int64_t)sub0 * r.si_sub + 4 * lane;
+  const int32_t *cc = r.cc + (int64_t)b * r.cc_b + (int64_t)h * r.cc_h + (int64_t)sub0 * r.cc_sub;
+  int id[4][4], n[4][4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) id[s][e] = (int)ids[s * r.si_sub + e] & 255;
+  for (int i = tid; i < 1024; i += kScanThreads) ((pkv_u32x4 *)s_max)[i] = pkv_u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) n[s][e] = cc[s * r.cc_sub + id[s][e]];
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int mine = n[s][0] + n[s][1] + n[s][2] + n[s][3];
+    int before = pkv_wave_incl_scan(mine) - mine;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      uint32_t votes = 0;
+#pragma unroll
+      for (int t = 0; t < PKV_MAX_TIERS; ++t) votes += t < r.tiers.n && (uint32_t)before < r.tiers.t[t] ? 1u : 0u;
+      if (votes) atomicMax(&s_max[(sub0 + s) * 256 + id[s][e]], votes);  // an id named twice keeps its best rank
+      before += n[s][e];
+    }
+  }
+  __syncthreads();
+  pkv_u32x4 packed;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const pkv_u32x4 v = ((const pkv_u32x4 *)s_max)[4 * tid + d];
+    packed[d] = v.x | v.y << 8 | v.z << 16 | v.w << 24;
+  }
+  ((pkv_u32x4 *)s_lut)[tid] = packed;
+  __syncthreads();
+}
+
 // KPT * 256 whole keys from key k0 on, in the form the retrieval runs (one-byte counts out, histogram kept): every
 // load of the thread is issued before the first table lookup, and nothing in between is conditional, so the waits
 // of the in-order memory counter name exact counts and the lookups of one key run while the codes of the others are
@@ -166,22 +214,29 @@ __global__ __launch_bounds__(kScanThreads) void pkv_scan_keymajor_kernel(
 // tensor): a thread takes four keys, sixteen 4-byte loads in flight, at any alignment (rows of odd length).  Bound by the
 // latency of that one round trip at the sizes such a call has: 16 rows x 20011 keys 4.4 us; 6.9 us with one key and sixteen
 // byte loads per thread and pass.
-template <bool RUNS>
+// RANKED: from a caller's ranking, counts only; the table is built here instead of by a launch before this one.
+template <bool RUNS, bool RANKED>
 __global__ __launch_bounds__(kScanThreads) void pkv_scan_strided_kernel(
     const uint8_t *__restrict__ codes, int64_t cs_b, int64_t cs_h, int64_t cs_key, int64_t cs_sub, int n_kv_heads,
     int64_t n_keys, const uint8_t *__restrict__ lut, uint8_t *__restrict__ cnt_u8, int64_t cnt_u8_stride,
-    int32_t *__restrict__ cnt_i32, uint32_t *__restrict__ row_suf, uint16_t *__restrict__ chunk_suf, int chunk_keys) {
+    int32_t *__restrict__ cnt_i32, uint32_t *__restrict__ row_suf, uint16_t *__restrict__ chunk_suf, int chunk_keys,
+    ScanRanking ranking) {
   const int row = blockIdx.y;
   const int chunk = blockIdx.x;
   const int b = row / n_kv_heads, h = row % n_kv_heads;
   const int tid = threadIdx.x;
 
   __shared__ __attribute__((aligned(16))) uint32_t s_lut[1024];
-  __shared__ uint32_t s_hist[128 * kHistCopies];  // also reused for the compacted histogram
-  load_lut(s_lut, lut, row);
-  if (chunk_suf)
-    for (int i = tid; i < 128 * kHistCopies; i += kScanThreads) s_hist[i] = 0;
-  __syncthreads();
+  __shared__ __attribute__((aligned(16))) uint32_t s_hist[RANKED ? 4096 : 128 * kHistCopies];  // also reused for the compacted histogram
+  if (RANKED) {
+    lut_from_ranking(ranking, b, h, s_hist, s_lut);
+    chunk_suf = nullptr;
+  } else {
+    load_lut(s_lut, lut, row);
+    if (chunk_suf)
+      for (int i = tid; i < 128 * kHistCopies; i += kScanThreads) s_hist[i] = 0;
+    __syncthreads();
+  }
   const uint8_t *l8 = (const uint8_t *)s_lut;
   const int copy = tid & (kHistCopies - 1);
 
@@ -279,9 +334,9 @@ static int launch_scan_impl(const uint8_t *codes, int64_t cs_b, int64_t cs_h, in
     PKV_LAUNCH_CHECK("pkv_scan_keymajor_kernel");
   } else {
 #define PKV_SCAN_STRIDED(RUNS)                                                                                           \
-  hipExtLaunchKernelGGL(pkv_scan_strided_kernel<RUNS>, grid, dim3(kScanThreads), 0, s, ev_start, ev_stop, 0, codes, cs_b, \
+  hipExtLaunchKernelGGL((pkv_scan_strided_kernel<RUNS, false>), grid, dim3(kScanThreads), 0, s, ev_start, ev_stop, 0, codes, cs_b, \
                         cs_h, cs_key, cs_sub, n_kv_heads, n_keys, lut, cnt_u8, cnt_u8_stride, cnt_i32, row_suf,          \
-                        chunk_suf, chunk_keys)
+                        chunk_suf, chunk_keys, ScanRanking())
     if (cs_key == 1) PKV_SCAN_STRIDED(true); else PKV_SCAN_STRIDED(false);
 #undef PKV_SCAN_STRIDED
     PKV_LAUNCH_CHECK("pkv_scan_strided_kernel");
@@ -294,6 +349,26 @@ int pkv_launch_scan(const uint8_t *codes, int64_t cs_b, int64_t cs_h, int64_t cs
                     int32_t *cnt_i32, uint32_t *row_suf, uint16_t *chunk_suf, int chunk_keys, hipStream_t s, int sub_blocks) {
   return launch_scan_impl(codes, cs_b, cs_h, cs_key, cs_sub, bs, n_kv_heads, n_keys, lut, cnt_u8, cnt_u8_stride, cnt_i32,
                           row_suf, chunk_suf, chunk_keys, s, nullptr, nullptr, sub_blocks);
+}
+
+// Votes of subspace-major codes from a caller's ranking in one launch.  Every workgroup builds its row's table, 0.6 to 1.4 us more
+// than the launch before the scan took on the GPU; a call waits for the host time of its launches, 3.4 us each, while its keys are
+// few.  us, GPU alone and call by itself, two launches / one: 8 rows x 3000 4.7, 15.6 / 5.4, 11.7; 16 x 20011 5.8, 15.4 / 7.0, 11.8;
+// 8 x 80001 6.8, 15.7 / 8.3, 11.7; not taken: 24 x 80001 10.3, 15.6 / 13.1, 12.7; 64 x 80000 21.4, 20.9 / 23.6, 23.3.  Codes requested
+// before the table is built: 16 x 20011 7.7.
+constexpr int64_t kRankedKeys = 1 << 20;
+bool pkv_scan_takes_ranking(int64_t cs_key, int rows, int64_t n_keys) { return cs_key == 1 && rows * n_keys <= kRankedKeys; }
+
+int pkv_launch_scan_ranked(const uint8_t *codes, int64_t cs_b, int64_t cs_h, int64_t cs_sub, int bs, int n_kv_heads, int64_t n_keys,
+                           const int64_t *ids, int64_t si_b, int64_t si_h, int64_t si_sub, const int32_t *cc, int64_t cc_b,
+                           int64_t cc_h, int64_t cc_sub, const PkvTiers &tiers, int32_t *cnt, hipStream_t s) {
+  const int chunk_keys = pkv_pick_chunk_keys(bs * n_kv_heads, n_keys);
+  const dim3 grid((unsigned)((n_keys + chunk_keys - 1) / chunk_keys), (unsigned)(bs * n_kv_heads));
+  hipLaunchKernelGGL((pkv_scan_strided_kernel<true, true>), grid, dim3(kScanThreads), 0, s, codes, cs_b, cs_h, (int64_t)1, cs_sub,
+                     n_kv_heads, n_keys, (const uint8_t *)nullptr, (uint8_t *)nullptr, (int64_t)0, cnt, (uint32_t *)nullptr,
+                     (uint16_t *)nullptr, chunk_keys, ScanRanking{ids, si_b, si_h, si_sub, cc, cc_b, cc_h, cc_sub, tiers});
+  PKV_LAUNCH_CHECK("pkv_scan_strided_kernel");
+  return PKV_OK;
 }
 
 int pkv_launch_scan_i32_codes(const int32_t *codebook, int rows, int64_t n_keys, const uint8_t *lut, int32_t *cnt,

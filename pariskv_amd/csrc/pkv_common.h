@@ -106,6 +106,11 @@ PKV_INTERNAL int pkv_launch_scan(const uint8_t *codes, int64_t cs_b, int64_t cs_
                                  int bs, int n_kv_heads, int64_t n_keys, const uint8_t *lut, uint8_t *cnt_u8,
                                  int64_t cnt_u8_stride, int32_t *cnt_i32, uint32_t *row_suf, uint16_t *chunk_suf,
                                  int chunk_keys, hipStream_t s, int sub_blocks = 1);
+PKV_INTERNAL bool pkv_scan_takes_ranking(int64_t cs_key, int rows, int64_t n_keys);
+PKV_INTERNAL int pkv_launch_scan_ranked(const uint8_t *codes, int64_t cs_b, int64_t cs_h, int64_t cs_sub, int bs, int n_kv_heads,
+                                        int64_t n_keys, const int64_t *ids, int64_t si_b, int64_t si_h, int64_t si_sub,
+                                        const int32_t *cc, int64_t cc_b, int64_t cc_h, int64_t cc_sub, const PkvTiers &tiers,
+                                        int32_t *cnt, hipStream_t s);
 // Pieces per chunk for the scan -> select + rerank pair of a retrieval: chunks of 8192 keys and more are cut into four
 // pieces spread over the row (where the row's piece tables stay within what the select keeps in LDS), smaller
 // chunks stay whole.

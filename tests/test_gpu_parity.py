@@ -2290,3 +2290,19 @@ def test_bucket_topk_of_rows_of_every_length(ops, rows, L):
             out = ops.bucket_topk(dev, k).cpu().numpy()
             for r in {0, rows - 1}:
                 assert np.array_equal(out[r], np.arange(L) if k == L else O.select_candidates(clamped[r], k)[0])
+
+
+@pytest.mark.parametrize("bs,H,N,n_tiers", [(1, 1, 1, 6), (1, 3, 5, 1), (2, 3, 1027, 6), (1, 5, 20011, 3), (1, 1, 1 << 20, 6), (1, 1, (1 << 20) + 3, 6)])
+def test_votes_of_a_ranking_with_repeats_in_any_layout(ops, bs, H, N, n_tiers):
+    """Subspace-major codes (one launch while rows x keys <= 2^20, each workgroup building the table) and key-major ones (the table
+    first): the same votes from rankings that name a centroid twice, from slices of wider tensors."""
+    _say(f"votes of a ranking {bs} x {H} x {N}, {n_tiers} tiers")
+    g = torch.Generator(device=DEV).manual_seed(N)
+    ids = torch.randint(0, 256, (bs, H + 1, 18, 256), generator=g, device=DEV)[:, 1:, 1:17]
+    counts = torch.randint(0, N // 100 + 2, (bs, H, 17, 256), generator=g, device=DEV, dtype=torch.int32)[:, :, 1:]
+    code = torch.randint(0, 256, (bs, H, 16, N + 2), generator=g, device=DEV).to(torch.uint8)[..., 1:N + 1]
+    tiers = [max(1, N * (t + 1) // (2 * n_tiers)) for t in range(n_tiers)]
+    got = ops.update_cache_cnt(ids, counts, code, tiers)
+    want = ops.update_cache_cnt(ids, counts, code.permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2), tiers)
+    assert torch.equal(got, want)
+    assert N < 100 or got.max() > 0   # the few keys of a short row may all have unranked codes
