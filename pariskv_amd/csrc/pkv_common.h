@@ -135,6 +135,16 @@ PKV_INTERNAL int pkv_launch_rerank(const int64_t *cand, int bs, int n_kv_heads, 
                                    float *scores, uint16_t *v4b, hipStream_t s);
 PKV_INTERNAL size_t pkv_topk_ws_bytes_impl(int rows, int64_t len, int64_t k);
 PKV_INTERNAL int64_t pkv_topk_ctl_words(int rows, int64_t len, int64_t k);
+// pkv_adaptive_topk; ranged: its control block (below) was cleared and then given the rows' score ranges, and cand_vnorm is set.
+PKV_INTERNAL int pkv_launch_adaptive_topk(const float *sl_logits, int64_t sl_stride, const float *sl_vnorm, int64_t slv_stride,
+                                          int64_t sl, const void *cand_scores, int cand_dtype, float cand_scale,
+                                          const float *cand_vnorm, const float *value_norm, int64_t vn_stride, int64_t vn_offset,
+                                          int64_t vn_pos_stride, const int64_t *cand_ids, int64_t n_cand, float threshold,
+                                          int64_t k_out, int rows, int64_t *adaptive_k, int64_t *topk_ids, int64_t k_min,
+                                          int64_t k_max, int32_t *row_keys, int64_t row_keys_base, void *ws, size_t ws_bytes,
+                                          bool ranged, void *stream);
+// The control block in its workspace (null: this call has none, or the workspace would be refused); words: its length.
+PKV_INTERNAL uint32_t *pkv_adaptive_topk_ctl(void *ws, size_t ws_bytes, int rows, int64_t n_cand, int64_t k_out, int64_t *words);
 PKV_INTERNAL uint32_t *pkv_topk_range_slots(uint32_t *ctl, int64_t len, int64_t *row_stride);
 constexpr int kTopkMaxSort = 8192;  // longest row that one workgroup sorts, or selects from with whole keys in registers: 64 KB of 64-bit keys in LDS
 constexpr int kTopkMaxSelect = 32768;  // longest row that one workgroup selects from: scores and bins of 32 keys a thread in registers

@@ -125,8 +125,11 @@ extern "C" int pkv_retrieve_ws_view(void *ws, int rows, int64_t n_keys, int64_t 
 
 // dense (or null): the adaptive-k step's dense tokens, whose logits ride with the query prep where that is a launch of its own
 // attn (or null): the step's attention in two parts, the first of which rides there as well and the second with the top-k
+// adk_ctl (or null; candidates only, launches of their own): a control block of adk_words words for the adaptive-k stage, cleared by
+// the query prep and given the rows' score ranges by the select + rerank
 static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, void *stream, const PkvDenseLogits *dense = nullptr,
-                         int least_chunk = 256, const PkvSplitAttn *attn = nullptr) {
+                         int least_chunk = 256, const PkvSplitAttn *attn = nullptr, uint32_t *adk_ctl = nullptr,
+                         int64_t adk_words = 0) {
   PKV_REQUIRE(a != nullptr, "pkv_retrieve: null args");
   PKV_REQUIRE(a->q && a->signs && a->centers && a->cluster_counts && a->codes && a->nib && a->weight,
               "pkv_retrieve: null pointer");
@@ -174,8 +177,8 @@ static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, 
   // the top-k takes the rows' score ranges from its control area (and a multi-workgroup top-k, see
   // pkv_launch_topk_f32, wants its control blocks cleared): the first launch of the step clears, the select + rerank launch
   // leaves the ranges
-  const int64_t ctl_words = a->out_ids && a->n_cand != a->n_keys ? pkv_topk_ctl_words(rows, a->n_cand, a->k) : 0;
-  uint32_t *topk_ctl = ctl_words ? (uint32_t *)(base + w.topk) : nullptr;
+  const int64_t ctl_words = adk_ctl ? adk_words : a->out_ids && a->n_cand != a->n_keys ? pkv_topk_ctl_words(rows, a->n_cand, a->k) : 0;
+  uint32_t *topk_ctl = adk_ctl ? adk_ctl : ctl_words ? (uint32_t *)(base + w.topk) : nullptr;
   int64_t range_stride = 0;
   uint32_t *range_slots = topk_ctl ? pkv_topk_range_slots(topk_ctl, a->n_cand, &range_stride) : nullptr;
   const uint8_t *codes = a->codes + a->key0 * 16;
@@ -397,9 +400,21 @@ extern "C" int pkv_adaptive_decode_step(const pkv_retrieve_args *retrieve, void 
                              two_runs ? ad->dense_split : ad->dense_rows, two_runs ? ad->dense_row1 - ad->dense_split : 0, ad->scale,
                              ad->dense_logits, ad->dense_logits_stride, ad->dense_vnorm, ad->dense_vnorm_stride,
                              two_runs ? ad->dense_vnorm_run : nullptr};
-  int rc = retrieve_impl(retrieve, ws, ws_bytes, stream, &dense);
-  if (rc) return rc;
   const int rows = retrieve->bs * retrieve->n_kv_heads;
+  // Norms from the key records and more candidates than one workgroup takes: the adaptive stage has the rows' score ranges from the
+  // select + rerank instead of a launch of its own for the maximum (8 rows x 1M keys, 52429 candidates: 154.8 -> 151.8 us a step),
+  // unless its control block lies where the retrieval works or someone else has run the query prep.
+  int64_t adk_words = 0;
+  uint32_t *adk_ctl = nullptr;
+  if (retrieve->record_word_offset > 0 && retrieve->n_cand < retrieve->n_keys && !retrieve->table_ready &&
+      retrieve->launch_plan != PKV_PLAN_ONE_LAUNCH && ad->scale > 0.f && retrieve->bs > 0 && retrieve->n_kv_heads > 0 &&
+      ad->k_out > 0 && ad->k_out <= kTopkMaxSort) {
+    adk_ctl = pkv_adaptive_topk_ctl(ad->ws, ad->ws_bytes, rows, retrieve->n_cand, ad->k_out, &adk_words);
+    const char *c = (const char *)adk_ctl;
+    if (c && c < (const char *)ws + ws_bytes && c + 4 * adk_words > (const char *)ws) adk_ctl = nullptr;
+  }
+  int rc = retrieve_impl(retrieve, ws, ws_bytes, stream, &dense, 256, nullptr, adk_ctl, adk_words);
+  if (rc) return rc;
   const WsLayout w = layout(rows, retrieve->n_keys, retrieve->n_cand, retrieve->k);
   const int64_t *cand = (const int64_t *)((char *)ws + w.cand);
   const float *scores = (const float *)((char *)ws + w.scores);
@@ -407,11 +422,11 @@ extern "C" int pkv_adaptive_decode_step(const pkv_retrieve_args *retrieve, void 
   // records (not on the all-keys-are-candidates path, which reranks without the fused kernel)
   const bool norms_emitted = retrieve->record_word_offset > 0 && retrieve->n_cand != retrieve->n_keys;
   const float *cand_vnorm = norms_emitted ? (const float *)((char *)ws + w.cand_extra) : nullptr;
-  rc = pkv_adaptive_topk(ad->dense_logits, ad->dense_logits_stride, two_runs ? ad->dense_vnorm_run : ad->dense_vnorm,
+  rc = pkv_launch_adaptive_topk(ad->dense_logits, ad->dense_logits_stride, two_runs ? ad->dense_vnorm_run : ad->dense_vnorm,
                          two_runs ? ad->dense_logits_stride : ad->dense_vnorm_stride,
                          ad->dense_rows, scores, PKV_DTYPE_F32, ad->scale, cand_vnorm, ad->value_norm, ad->vn_stride,
                          ad->vn_offset, ad->vn_pos_stride, cand, retrieve->n_cand, ad->threshold, ad->k_out, rows, ad->adaptive_k,
-                         ad->topk_ids, ad->k_min, ad->k_max, ad->row_keys, ad->row_keys_base, ad->ws, ad->ws_bytes, stream);
+                         ad->topk_ids, ad->k_min, ad->k_max, ad->row_keys, ad->row_keys_base, ad->ws, ad->ws_bytes, adk_ctl != nullptr, stream);
   if (rc) return rc;
   if (ad->uniform_k) {
     rc = pkv_uniform_k(ad->adaptive_k, rows, ad->uniform_k, ad->row_keys, ad->row_keys_base, stream);

@@ -2323,35 +2323,57 @@ __global__ __launch_bounds__(kAdkPartThreads) void pkv_adk_max_gather_kernel(
   }
 }
 
+// Joint maximum of a row's logits where no launch left partial maxima: the candidates' from the score ranges that the select +
+// rerank launch left in the row's control block, the dense tokens' from the logits themselves.  All 1024 threads.
+__device__ __forceinline__ float adk_max_from_ranges(const uint32_t *__restrict__ rctl, const float *__restrict__ sll, int64_t sl,
+                                                     const void *__restrict__ cs, int cand_dtype, float cand_scale, int64_t n_cand,
+                                                     float *s_max) {
+  const int lane = pkv_lane();
+  const uint32_t slot = lane < kWideRangeSlots ? rctl[kWideCtlSlots + 2 * lane] : 0u;
+  float m = -__uint_as_float(0x7f800000u);
+  for (int64_t i = threadIdx.x; i < sl; i += kTopkThreads) m = fmaxf(m, sll[i]);
+  const float top = pkv_from_ordered_u32(pkv_wave_max(slot)) * cand_scale;  // rounding is monotone: the largest logit
+  if (top == top) m = fmaxf(m, top);
+  else  // a score that is not a number: the maximum of the others
+    for (int64_t i = threadIdx.x; i < n_cand; i += kTopkThreads) m = fmaxf(m, cand_logit(cs, cand_dtype, cand_scale, i));
+  return block_max_1024(m, s_max);
+}
+
 // grid (slices + 1, rows) x 1024: benefits of the slice into ws_ben, their sum (lane order, then the 1024-lane tree)
 // into ws_sum, and their top key bits into the row histogram; one more workgroup per row sums the benefits of the
-// dense tokens meanwhile.
+// dense tokens meanwhile.  n_parts = 0: the maximum comes from the row's score ranges, which saves the launch before this one.
 __global__ __launch_bounds__(kTopkThreads) void pkv_adk_benefit_kernel(
     const float *__restrict__ sl_logits, int64_t sl_stride, const float *__restrict__ sl_vnorm, int64_t slv_stride,
     int64_t sl, const void *__restrict__ cand_scores, int cand_dtype, float cand_scale,
     const float *__restrict__ cand_vnorm, int64_t n_cand, const float *__restrict__ ws_max, int n_parts,
     float *__restrict__ ws_ben, float *__restrict__ ws_sum, uint32_t *__restrict__ ctl) {
-  __shared__ float s_part[16];
+  __shared__ float s_part[16], s_max[16];
   __shared__ uint32_t s_bins[kWideBins];
   const int row = blockIdx.y, slice = blockIdx.x, tid = threadIdx.x, n_slices = gridDim.x - 1;
   const char *cs = (const char *)cand_scores + (int64_t)row * n_cand * (cand_dtype == PKV_DTYPE_BF16 ? 2 : 4);
   const float *cv = cand_vnorm + (int64_t)row * n_cand;  // the caller's, or the ones gathered by the first launch
   float *ben = ws_ben + (int64_t)row * n_cand;
+  const float *sll = sl_logits + (int64_t)row * sl_stride;
+  float lg[kWideE], vv[kWideE];
+  if (slice < n_slices) {
+#pragma unroll
+    for (int e = 0; e < kWideE; ++e) {
+      const int64_t i = (int64_t)slice * kWideSlice + e * kTopkThreads + tid, ii = i < n_cand ? i : n_cand - 1;
+      lg[e] = cand_logit(cs, cand_dtype, cand_scale, ii);
+      vv[e] = cv[ii];
+    }
+  }
   float g = -__uint_as_float(0x7f800000u);
-  for (int w = tid & (PKV_WAVE - 1); w < n_parts; w += PKV_WAVE) g = fmaxf(g, ws_max[(int64_t)row * n_parts + w]);
-  g = pkv_wave_max(g);
+  if (n_parts == 0) {  // uniform
+    g = adk_max_from_ranges(ctl + (int64_t)row * kWideRowWords, sll, sl, cs, cand_dtype, cand_scale, n_cand, s_max);
+  } else {
+    for (int w = tid & (PKV_WAVE - 1); w < n_parts; w += PKV_WAVE) g = fmaxf(g, ws_max[(int64_t)row * n_parts + w]);
+    g = pkv_wave_max(g);
+  }
   if (slice == n_slices) {  // the row's last workgroup: the dense tokens' benefit, kept after the slice sums
-    const float d = dense_benefit_sum(sl_logits + (int64_t)row * sl_stride, sl_vnorm + (int64_t)row * slv_stride, sl, g,
-                                      s_part);
+    const float d = dense_benefit_sum(sll, sl_vnorm + (int64_t)row * slv_stride, sl, g, s_part);
     if (tid == 0) ws_sum[(int64_t)row * (n_slices + 1) + n_slices] = d;
     return;
-  }
-  float lg[kWideE], vv[kWideE];
-#pragma unroll
-  for (int e = 0; e < kWideE; ++e) {
-    const int64_t i = (int64_t)slice * kWideSlice + e * kTopkThreads + tid, ii = i < n_cand ? i : n_cand - 1;
-    lg[e] = cand_logit(cs, cand_dtype, cand_scale, ii);
-    vv[e] = cv[ii];
   }
   float acc = 0.f;
   uint64_t keys[kWideE];
@@ -2807,6 +2829,14 @@ extern "C" size_t pkv_adaptive_topk_ws_bytes(int rows, int64_t n_cand, int64_t k
   return adk_ws_layout(rows, n_cand, k_out).total;
 }
 
+uint32_t *pkv_adaptive_topk_ctl(void *ws, size_t ws_bytes, int rows, int64_t n_cand, int64_t k_out, int64_t *words) {
+  if (!ws || !pkv_aligned(ws, 256) || rows <= 0 || n_cand <= kTopkMaxSort || k_out <= 0 || k_out > n_cand) return nullptr;
+  const AdkWs w = adk_ws_layout(rows, n_cand, k_out);
+  if (ws_bytes < w.total) return nullptr;
+  *words = (int64_t)rows * kWideRowWords;
+  return (uint32_t *)((char *)ws + w.wide.ctl);
+}
+
 extern "C" int pkv_adaptive_topk(const float *sl_logits, int64_t sl_stride, const float *sl_vnorm, int64_t slv_stride,
                                  int64_t sl, const void *cand_scores, int cand_dtype, float cand_scale,
                                  const float *cand_vnorm, const float *value_norm, int64_t vn_stride, int64_t vn_offset,
@@ -2814,6 +2844,18 @@ extern "C" int pkv_adaptive_topk(const float *sl_logits, int64_t sl_stride, cons
                                  int64_t k_out, int rows,
                                  int64_t *adaptive_k, int64_t *topk_ids, int64_t k_min, int64_t k_max,
                                  int32_t *row_keys, int64_t row_keys_base, void *ws, size_t ws_bytes, void *stream) {
+  return pkv_launch_adaptive_topk(sl_logits, sl_stride, sl_vnorm, slv_stride, sl, cand_scores, cand_dtype, cand_scale, cand_vnorm,
+                                  value_norm, vn_stride, vn_offset, vn_pos_stride, cand_ids, n_cand, threshold, k_out, rows,
+                                  adaptive_k, topk_ids, k_min, k_max, row_keys, row_keys_base, ws, ws_bytes, false, stream);
+}
+
+int pkv_launch_adaptive_topk(const float *sl_logits, int64_t sl_stride, const float *sl_vnorm, int64_t slv_stride,
+                                 int64_t sl, const void *cand_scores, int cand_dtype, float cand_scale,
+                                 const float *cand_vnorm, const float *value_norm, int64_t vn_stride, int64_t vn_offset,
+                                 int64_t vn_pos_stride, const int64_t *cand_ids, int64_t n_cand, float threshold,
+                                 int64_t k_out, int rows,
+                                 int64_t *adaptive_k, int64_t *topk_ids, int64_t k_min, int64_t k_max,
+                                 int32_t *row_keys, int64_t row_keys_base, void *ws, size_t ws_bytes, bool ranged, void *stream) {
   PKV_REQUIRE(k_max <= 0 || (k_min >= 0 && k_min <= k_max), "pkv_adaptive_topk: clamp [%lld, %lld] is empty",
               (long long)k_min, (long long)k_max);
   const AdkClamp cl{k_min, k_max, row_keys, row_keys_base};
@@ -2852,12 +2894,14 @@ extern "C" int pkv_adaptive_topk(const float *sl_logits, int64_t sl_stride, cons
   uint64_t *list_a = (uint64_t *)(base + w.wide.list_a), *list_b = (uint64_t *)(base + w.wide.list_b);
   float *gathered = (float *)(base + w.vn);
   const int n_slices = (int)((n_cand + kWideSlice - 1) / kWideSlice);
-  const int n_parts = (int)((n_cand + kAdkPart - 1) / kAdkPart);
+  const int n_parts = ranged ? 0 : (int)((n_cand + kAdkPart - 1) / kAdkPart);
   const dim3 grid((unsigned)n_slices, (unsigned)rows);
-  hipLaunchKernelGGL(pkv_adk_max_gather_kernel, dim3((unsigned)n_parts, (unsigned)rows), dim3(kAdkPartThreads), 0, s,
-                     sl_logits, sl_stride, sl, cand_scores, cand_dtype, cand_scale, cand_vnorm ? nullptr : value_norm,
-                     vn_stride, vn_offset, vn_pos_stride, cand_ids, n_cand, smax, gathered, ctl);
-  PKV_LAUNCH_CHECK("pkv_adk_max_gather_kernel");
+  if (!ranged) {
+    hipLaunchKernelGGL(pkv_adk_max_gather_kernel, dim3((unsigned)n_parts, (unsigned)rows), dim3(kAdkPartThreads), 0, s,
+                       sl_logits, sl_stride, sl, cand_scores, cand_dtype, cand_scale, cand_vnorm ? nullptr : value_norm,
+                       vn_stride, vn_offset, vn_pos_stride, cand_ids, n_cand, smax, gathered, ctl);
+    PKV_LAUNCH_CHECK("pkv_adk_max_gather_kernel");
+  }
   hipLaunchKernelGGL(pkv_adk_benefit_kernel, dim3((unsigned)n_slices + 1, (unsigned)rows), dim3(kTopkThreads), 0, s,
                      sl_logits, sl_stride, sl_vnorm, slv_stride, sl, cand_scores, cand_dtype, cand_scale,
                      cand_vnorm ? cand_vnorm : gathered, n_cand, smax, n_parts, ben, ssum, ctl);

@@ -1256,3 +1256,43 @@ def test_short_prompt_after_a_long_one_equals_a_fresh_cache(form, offload):
             c.decode_update_kv_cache(k1, v1, 0)
             out.append(c.compute(q, 0))
         assert torch.equal(out[0], out[1]), step
+
+
+def test_adaptive_step_takes_the_maximum_from_the_score_ranges():
+    """More candidates than one workgroup holds: the step has the rows' largest score from the select + rerank launch.  k and ids equal
+    the stand-alone operator's, which looks for it, step after step: ordinary rows, weights that make scores infinite or not a
+    number, and a row of equal scores."""
+    from pariskv_amd import ops
+
+    bs, H, group, S, sink, local, steps = 1, 6, 4, 172_000, 4, 64, 3
+    cache = _cache_of("dense", False, bs, H, group, S, 40, sink, local, 16, 50, 100, adaptive_topk_max_k=300)
+    g = torch.Generator(device=DEV).manual_seed(5)
+
+    def rows(n):
+        return torch.randn(bs, n, H, 128, generator=g, device=DEV).to(torch.bfloat16)
+
+    cache.prefill_update_kv_cache(None, rows(S), rows(S), 0, 0)
+    w = cache._w_km[0]
+    w[0, 1, 1000:150_000:7] = float("nan")
+    w[0, 2, 1000:150_000:7, 3] = float("inf")   # one block of sixteen: infinite, not undefined
+    w[0, 3, 1000:150_000:7, 3] = float("-inf")
+    w[0, 4] = float("nan")
+    w[0, 5] = 0.0
+    for step in range(steps):
+        q = torch.randn(bs, 1, H * group, 128, generator=g, device=DEV).to(torch.bfloat16)
+        cache.compute(q, 0)
+        k_got, z = cache.last_adaptive_k.clone(), cache._zones[0]
+        n_keys, n_cand, _, tiers = cache.retrieval_shape(0)
+        assert n_cand > 8192
+        cap = cache._caps(n_cand)[0]
+        ids_got = cache._topk_ids[:bs * H * cap].view(bs, H, cap).clone()
+        pos = torch.cat([torch.arange(sink), torch.arange(z.local_start, z.seq_len)]).to(DEV)
+        cand, scores = cache._plan.run_candidates(q, cache._srht_signs, cache._mag_centers, cache.cluster_key_counts_gpu[0],
+                                                  cache._codes_km[0], cache._nib_km[0], cache._w_km[0], sink, n_keys, tiers, n_cand)
+        k_ref, ids_ref = ops.adaptive_topk(cache._dense_logits[:, :, :len(pos)].contiguous(),
+                                           cache._sl_vnorm_cache[0][:, :, pos].contiguous(), scores, cache._attn_scale, cand,
+                                           cache.adaptive_topk_threshold, cap, value_norm=cache.value_norm_gpu[0],
+                                           vn_offset=sink, k_min=1, k_max=cap)
+        assert torch.equal(k_got, k_ref) and torch.equal(ids_got, ids_ref), step
+        assert torch.isnan(scores[0, 1]).any() and torch.isinf(scores[0, 2]).any()
+        cache.decode_update_kv_cache(rows(1), rows(1), 0)
