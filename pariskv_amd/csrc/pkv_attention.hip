@@ -645,8 +645,8 @@ bool pkv_plan_split_attention(const pkv_retrieve_args *r, const void *ws, const 
       !pkv_aligned(at->ws, 16) || r->bs <= 0 || r->n_kv_heads <= 0 || (int64_t)r->bs * r->n_kv_heads > 65535 || r->group < 1 ||
       r->group > 8 || at->n_segments < 1 || at->n_segments > PKV_ATTN_MAX_SEGMENTS)
     return false;
-  // The query side: a launch of this call's own, for the dense part to run beside.
-  if (r->launch_plan != PKV_PLAN_SEPARATE || r->table_ready) return false;
+  // Launches of this call's own, for the dense part to run beside: the query side's, or the scan's where that is already done.
+  if (r->launch_plan != PKV_PLAN_SEPARATE) return false;
   // The selection: in any order, of one workgroup a row, into the list that the attention reads, nothing gathered.
   if (!r->out_ids || !r->any_order || r->src_k || r->n_cand == r->n_keys || at->row_keys || r->k > kSplitMaxSelected ||
       !pkv_topk_attends(r->n_cand, r->k))

@@ -18,6 +18,9 @@ PKV_INTERNAL int pkv_launch_qk_norm_rope_table(const void *qkv, int64_t stride_b
                                   const void *sin_row, void *q_out, void *k_out, const float *signs, const int32_t *cc,
                                   const PkvTiers &tiers, float *qhat, float *qnorm, uint8_t *lut, uint32_t *row_suf,
                                   uint32_t *zero_ptr, int64_t zero_words, const pkv_kv_append *append, hipStream_t s);
+PKV_INTERNAL int pkv_launch_scan_attend(const uint8_t *codes, int64_t cs_b, int64_t cs_h, int bs, int n_kv_heads, int64_t n_keys,
+                                        const uint8_t *lut, uint8_t *cnt_u8, int64_t cnt_u8_stride, uint32_t *row_suf,
+                                        uint16_t *chunk_suf, int chunk_keys, int sub_blocks, const PkvSplitAttn &attn, hipStream_t s);
 PKV_INTERNAL int pkv_launch_query_prep_attend(const pkv_retrieve_args *a, const PkvTiers &tiers, float *qhat, float *qnorm, uint8_t *lut,
                                               uint32_t *row_suf_to_zero, uint32_t *zero_ptr, int64_t zero_words,
                                               const PkvSplitAttn &attn, hipStream_t s);
@@ -213,8 +216,12 @@ static int retrieve_impl(const pkv_retrieve_args *a, void *ws, size_t ws_bytes, 
                              weight, (int64_t)H * a->cap * wk, a->cap * wk, wk, 1, qhat, qnorm, a->centers, scores,
                              nullptr, s);
     } else {
-      rc = pkv_launch_scan(codes, (int64_t)H * a->cap * 16, a->cap * 16, 16, 1, a->bs, H, a->n_keys, lut, cnt,
-                           w.cnt_stride, nullptr, rowsuf, hist, w.chunk_keys, s, w.sub_blocks);
+      if (a->table_ready && attn && attn->n_dense)
+        rc = pkv_launch_scan_attend(codes, (int64_t)H * a->cap * 16, a->cap * 16, a->bs, H, a->n_keys, lut, cnt, w.cnt_stride, rowsuf,
+                                    hist, w.chunk_keys, w.sub_blocks, *attn, s);
+      else
+        rc = pkv_launch_scan(codes, (int64_t)H * a->cap * 16, a->cap * 16, 16, 1, a->bs, H, a->n_keys, lut, cnt,
+                             w.cnt_stride, nullptr, rowsuf, hist, w.chunk_keys, s, w.sub_blocks);
       if (rc) return rc;
       rc = pkv_launch_select_rerank(cnt, w.cnt_stride, rowsuf, hist, w.chunk_keys, a->bs, H, a->n_keys, a->n_cand, nib,
                                     (int64_t)H * a->cap * nk, a->cap * nk, nk, weight, (int64_t)H * a->cap * wk, a->cap * wk,

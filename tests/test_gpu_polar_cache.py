@@ -1296,3 +1296,38 @@ def test_adaptive_step_takes_the_maximum_from_the_score_ranges():
         assert torch.equal(k_got, k_ref) and torch.equal(ids_got, ids_ref), step
         assert torch.isnan(scores[0, 1]).any() and torch.isinf(scores[0, 2]).any()
         cache.decode_update_kv_cache(rows(1), rows(1), 0)
+
+
+@pytest.mark.parametrize("bs,Hq,Hkv,S,topk,form", [(1, 4, 4, 1500, 1, 0), (2, 16, 2, 3001, 100, 1), (1, 8, 2, 20000, 100, 1), (2, 8, 2, 9000, 512, 2),
+                                                   (1, 12, 4, 20003, 700, 2), (3, 8, 2, 1300, 600, 0)])
+def test_attention_in_two_parts_behind_a_table_from_the_rope_launch(bs, Hq, Hkv, S, topk, form):
+    """Steps whose query side another kernel has done: the part of the attention that waits for nothing rides with the scan.  Output
+    and ids are those of the same step with its own query prep, in every form of the step and from an empty buffer to a full one."""
+    import ctypes
+
+    from pariskv_amd import _lib, ops
+
+    D, interval = 128, 16
+    g = torch.Generator(device=DEV).manual_seed(S)
+    cache = _make_cache(False, bs, Hkv, Hq, 1, S, 64, 4, 64, interval, topk)
+    k, v = _synth_kv(torch.Generator().manual_seed(2), bs, S, Hkv)
+    cache.prefill_update_kv_cache(None, k.to(DEV), v.to(DEV), 0, 0)
+    cos, sin = torch.ones(D // 2, dtype=torch.bfloat16, device=DEV), torch.zeros(D // 2, dtype=torch.bfloat16, device=DEV)
+    used = 0
+    for step in range(interval + 3):
+        qkv = torch.randn(bs, 1, (Hq + 2 * Hkv) * D, generator=g, device=DEV).to(torch.bfloat16)
+        target = cache.query_table_target(0)
+        q, kk = ops.qk_norm_rope(qkv, Hq, Hkv, None, None, 1e-6, cos, sin, table_for=target)
+        cache.decode_update_kv_cache(kk, qkv[..., (Hq + Hkv) * D:].reshape(bs, 1, Hkv, D), 0)
+        if target is not None:
+            used += 1
+            assert target.a.table_ready == 1
+        out1, ids1 = cache.compute(q, 0).clone(), cache.last_topk_indices.clone()
+        out0 = cache.compute(q, 0)
+        if target is not None:
+            target.a.table_ready = 1
+            got = _lib.lib().pkv_decode_step_form(ctypes.byref(target.a), target._ws, ctypes.byref(target.aa))
+            target.a.table_ready = 0
+            assert got == form, (got, step)
+        assert torch.equal(out0, out1) and torch.equal(ids1, cache.last_topk_indices), step
+    assert used >= interval
