@@ -633,8 +633,8 @@ int pkv_retrieve_noalloc(const pkv_retrieve_args *args, void *stream);
  * dense-fallback test.  Queries, dtype and head counts are taken from
  * `retrieve`; the segments normally include the rows the gather just wrote.
  * Where a bf16 step gathers nothing and one segment reads the selected rows
- * through `retrieve`'s out_ids (any_order, PKV_PLAN_SEPARATE, no table_ready),
- * the attention may ride in the query-prep and top-k launches: the same
+ * through `retrieve`'s out_ids (any_order, PKV_PLAN_SEPARATE), the attention
+ * may ride in the query-prep (table_ready: scan) and top-k launches: the same
  * results, bit for bit, and other contents of `ws`.  Buffers may be shared as
  * the order of the two calls allows (attention->ws inside `ws`, an output over
  * the queries or the workspace): the attention then waits for the retrieval. */
