@@ -654,10 +654,11 @@ int pkv_decode_attention_run(const void *q, int dtype, int bs, int n_kv_heads, i
                              void *stream);
 
 /* The same with counters (no counterpart in the reference): arrivals [2 * bs * n_kv_heads] words belong to args->ws, are zero before the first launch and left
- * zero by every launch.  Same results; a short set of keys then takes one launch instead of two.  Launches that share ws and
- * arrivals follow one another on the GPU, as for ws alone. */
+ * zero by every launch; turn, 0 or 1, says which half this launch counts in, and launches that take turns clear what launches
+ * that overlapped have left.  Same results; a short set of keys then takes one launch instead of two.  Launches that share ws
+ * and arrivals follow one another on the GPU, as for ws alone. */
 int pkv_decode_attention_counted(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_args *args,
-                                 uint32_t *arrivals, void *stream);
+                                 uint32_t *arrivals, int turn, void *stream);
 
 int pkv_decode_step(const pkv_retrieve_args *retrieve, void *ws, size_t ws_bytes,
                     const pkv_attn_args *attention, void *stream);

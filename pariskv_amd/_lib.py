@@ -153,7 +153,7 @@ PROTOTYPES = {
     "pkv_dense_logits": (_i, [_vp, _i, _i, _i, _i, _vp, _i64, _i64, _i64, C.c_float, _vp, _i64, _vp]),
     "pkv_decode_attention_ws_bytes": (_sz, [_i, _i, _i, _i64]),
     "pkv_decode_attention_run": (_i, [_vp, _i, _i, _i, _i, C.POINTER(AttnArgs), _vp]),
-    "pkv_decode_attention_counted": (_i, [_vp, _i, _i, _i, _i, C.POINTER(AttnArgs), _vp, _vp]),
+    "pkv_decode_attention_counted": (_i, [_vp, _i, _i, _i, _i, C.POINTER(AttnArgs), _vp, _i, _vp]),
     "pkv_append_kv_run": (_i, [C.POINTER(AppendArgs), _vp, _i64, _i64, _vp, _i64, _i64, _i64, _vp]),
     "pkv_decode_attention": (_i, [_vp, _i, _i, _i, _i, C.POINTER(AttnSegment), _i, _vp, C.c_float, _vp, _vp, _sz, _vp]),
     "pkv_qk_norm_rope": (_i, [_vp, _i64, _i, _i, _i, _vp, _vp, C.c_float, _vp, _vp, _vp, _vp, _vp]),

@@ -149,13 +149,15 @@ __device__ __forceinline__ void load8(const void *base, int64_t elem_off, float 
 // WHOLE launches: the splits of a row are merged, as pkv_attn_merge_kernel merges them and to the same bits, by the workgroup
 // that stores its partial result last.  gridDim.x workgroups of a row come here with their partial results stored for other
 // dies (att_put); *arrived is zero before the first of them and after the last.  Nobody waits: a workgroup that is not the last
-// one ends.  One chain of store acknowledgement, count and dependent loads, so every load is requested before the weights are
+// one ends.  *spare, the next launch's counter, is zero as well unless launches that share the workspace ran at once, which spoils
+// their results: it is cleared here, so that it spoils no later ones.  One chain of store acknowledgement, count and dependent loads, so every load is requested before the weights are
 // known; see kWholeSplits for what it costs and saves.
-__device__ __forceinline__ void att_last_merges(const float *ws, int row, int group, uint32_t *arrived, uint16_t *out) {
+__device__ __forceinline__ void att_last_merges(const float *ws, int row, int group, uint32_t *arrived, uint32_t *spare, uint16_t *out) {
   constexpr int kThreads = kMfmaWaves * PKV_WAVE;
   const int tid = threadIdx.x, n_splits = gridDim.x, lane = tid & (PKV_WAVE - 1);
   __shared__ uint32_t s_before;
   __shared__ float s_w[8][PKV_WAVE];  // weight of split s for head g, already divided by the total
+  if (blockIdx.x == 0 && tid == 0) __hip_atomic_store(spare, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   pkv_wait_vmem();
   __syncthreads();
   if (tid == 0) s_before = __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -357,7 +359,7 @@ __global__ __launch_bounds__(kAttThreads) void pkv_attn_partial_kernel(const voi
 template <bool INDEXED, typename SEGS, bool WHOLE>
 __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_kernel(
     const void *__restrict__ q, int group, SEGS segs, int64_t total, const int32_t *__restrict__ row_keys, int uniform,
-    int64_t per_split, float scale_log2e, float *__restrict__ ws, uint32_t *arrivals, void *out) {
+    int64_t per_split, float scale_log2e, float *__restrict__ ws, uint32_t *arrivals, uint32_t *spares, void *out) {
   const int split = blockIdx.x, h = blockIdx.y, b = blockIdx.z, row = b * (int)gridDim.y + h;
   constexpr bool ONE = __is_same(SEGS, AttOne);
   const int lane = threadIdx.x & (PKV_WAVE - 1), wave = threadIdx.x / PKV_WAVE;
@@ -402,7 +404,7 @@ __global__ __launch_bounds__(kMfmaWaves * PKV_WAVE) void pkv_attn_partial_mfma_k
   l_part = pkv_pair_add<32>(pkv_pair_add<16>(l_part));
   float *part = ws + ((int64_t)row * gridDim.x + split) * group * kPartStride;
   att_merge_waves<WHOLE>(group, m_run, l_part, o, part, kPartStride, part + 2, kPartStride);
-  if (WHOLE) att_last_merges(ws, row, group, arrivals + row, (uint16_t *)out);
+  if (WHOLE) att_last_merges(ws, row, group, arrivals + row, spares + row, (uint16_t *)out);
 }
 
 // grid R, G*128 threads: merge the splits (at most 64) and normalise.
@@ -546,7 +548,7 @@ static int collect_segments(int dtype, const pkv_attn_segment *segments, int n_s
 
 static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_segment *segments,
                             int n_segments, const int32_t *row_keys, int uniform, float scale, void *out, void *ws,
-                            size_t ws_bytes, uint32_t *arrivals, void *stream) {
+                            size_t ws_bytes, uint32_t *arrivals, uint32_t *spares, void *stream) {
   PKV_REQUIRE(q && segments && out && ws, "pkv_decode_attention: null pointer");
   PKV_REQUIRE(dtype == PKV_DTYPE_F32 || dtype == PKV_DTYPE_BF16, "unknown dtype %d", dtype);
   PKV_REQUIRE(bs > 0 && n_kv_heads > 0 && (int64_t)bs * n_kv_heads <= 65535, "bad shape bs=%d kv_heads=%d", bs,
@@ -584,7 +586,7 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
     const dim3 grid3((unsigned)n_splits, (unsigned)n_kv_heads, (unsigned)bs);
 #define PKV_ATT_MFMA_W(IDX, S, WHOLE)                                                                                           \
   hipLaunchKernelGGL((pkv_attn_partial_mfma_kernel<IDX, decltype(S), WHOLE>), grid3, dim3(kMfmaWaves * PKV_WAVE), 0, s, q, group, S, \
-                     total, row_keys, uniform, per_split, scale_log2e, (float *)ws, arrivals, out)
+                     total, row_keys, uniform, per_split, scale_log2e, (float *)ws, arrivals, spares, out)
 #define PKV_ATT_MFMA(IDX, S)                                                         \
   do {                                                                               \
     if (whole) PKV_ATT_MFMA_W(IDX, S, true); else PKV_ATT_MFMA_W(IDX, S, false);     \
@@ -632,22 +634,24 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
 extern "C" int pkv_decode_attention(const void *q, int dtype, int bs, int n_kv_heads, int group,
                                     const pkv_attn_segment *segments, int n_segments, const int32_t *row_keys,
                                     float scale, void *out, void *ws, size_t ws_bytes, void *stream) {
-  return decode_attention(q, dtype, bs, n_kv_heads, group, segments, n_segments, row_keys, 0, scale, out, ws, ws_bytes, nullptr, stream);
+  return decode_attention(q, dtype, bs, n_kv_heads, group, segments, n_segments, row_keys, 0, scale, out, ws, ws_bytes, nullptr, nullptr, stream);
 }
 
 extern "C" int pkv_decode_attention_run(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_args *a,
                                         void *stream) {
   PKV_REQUIRE(a != nullptr, "pkv_decode_attention: null args");
   return decode_attention(q, dtype, bs, n_kv_heads, group, a->segments, a->n_segments, a->row_keys,
-                          a->row_keys_uniform ? bs * n_kv_heads : 0, a->scale, a->out, a->ws, a->ws_bytes, nullptr, stream);
+                          a->row_keys_uniform ? bs * n_kv_heads : 0, a->scale, a->out, a->ws, a->ws_bytes, nullptr, nullptr, stream);
 }
 
 extern "C" int pkv_decode_attention_counted(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_args *a,
-                                            uint32_t *arrivals, void *stream) {
+                                            uint32_t *arrivals, int turn, void *stream) {
   PKV_REQUIRE(a != nullptr && arrivals != nullptr, "pkv_decode_attention_counted: null pointer");
-  PKV_REQUIRE(pkv_aligned(arrivals, 4), "arrivals must be 4-byte aligned");
+  PKV_REQUIRE(pkv_aligned(arrivals, 4) && (turn == 0 || turn == 1), "arrivals must be 4-byte aligned, turn 0 or 1");
+  const int64_t rows = (int64_t)bs * n_kv_heads;  // checked before they are used
   return decode_attention(q, dtype, bs, n_kv_heads, group, a->segments, a->n_segments, a->row_keys,
-                          a->row_keys_uniform ? bs * n_kv_heads : 0, a->scale, a->out, a->ws, a->ws_bytes, arrivals, stream);
+                          a->row_keys_uniform ? bs * n_kv_heads : 0, a->scale, a->out, a->ws, a->ws_bytes, arrivals + turn * rows,
+                          arrivals + (1 - turn) * rows, stream);
 }
 
 static bool meets(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {

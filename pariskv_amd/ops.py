@@ -653,6 +653,7 @@ class DecodeAttention:
         nbytes = _lib.lib().pkv_decode_attention_ws_bytes(bs, n_kv_heads, group, max(1, max_keys))
         self.ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
         self.arrivals = torch.zeros(2 * bs * n_kv_heads, dtype=torch.int32, device=device)  # every launch leaves them zero
+        self.turn = 0  # the half of them that the next launch counts in
         self._segs = (_lib.AttnSegment * 4)()  # reused between calls: filling it is most of the host time
 
     def run(self, queries: torch.Tensor, segments, scale: float = None, out: torch.Tensor = None,
@@ -831,13 +832,13 @@ class BoundAttention:
     ``lent``: tensors of the segments that the caller may let go while a launch is queued; every stream that launches is
     told to the allocator, so that their memory waits for it."""
 
-    __slots__ = ("aa", "segs", "keep", "_raa", "_dims", "_arrivals", "_fn", "_numel", "_dtype", "_lent", "_told")
+    __slots__ = ("aa", "segs", "keep", "_raa", "_dims", "_arrivals", "_att", "_fn", "_numel", "_dtype", "_lent", "_told")
 
     def __init__(self, att, q, segments, lent=()):
         self.aa, _ = att.c_args(q, segments, out=q)  # out is patched at every launch
         self.segs, self._raa, self.keep = self.aa.segments, C.byref(self.aa), (att, segments)
         self._dims = (_dt(q.dtype), att.bs, att.H, att.G)
-        self._arrivals = att.arrivals.data_ptr()
+        self._arrivals, self._att = att.arrivals.data_ptr(), att
         self._fn = _lib.lib().pkv_decode_attention_counted
         self._numel, self._dtype = q.numel(), q.dtype
         self._lent, self._told = lent, None
@@ -854,7 +855,8 @@ class BoundAttention:
             for t in self._lent:
                 t.record_stream(stream)
             self._told = handle
-        rc = self._fn(q.data_ptr(), *self._dims, self._raa, self._arrivals, handle)
+        self._att.turn ^= 1
+        rc = self._fn(q.data_ptr(), *self._dims, self._raa, self._arrivals, self._att.turn, handle)
         if rc != 0:
             _lib.check(rc)
         return out
