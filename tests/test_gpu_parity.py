@@ -2313,3 +2313,26 @@ def test_votes_of_a_ranking_with_repeats_in_any_layout(ops, bs, H, N, n_tiers):
     want = ops.update_cache_cnt(ids, counts, code.permute(0, 1, 3, 2).contiguous().permute(0, 1, 3, 2), tiers)
     assert torch.equal(got, want)
     assert N < 100 or got.max() > 0   # the few keys of a short row may all have unranked codes
+
+
+@pytest.mark.parametrize("group", [1, 4, 7, 8])
+@pytest.mark.parametrize("n", [130, 700, 1280, 2048])
+def test_bound_attention_of_infinite_values(ops, group, n):
+    """The merge in the attention's own launch, 2 to 16 splits: an infinite value makes its dimension infinite, with its sign, and no
+    other one, as the merge by a launch of its own has it, in whatever split it lies."""
+    _say(f"bound attention, infinite values, group={group} {n}")
+    bs, H = 1, 3
+    g = torch.Generator(device=DEV).manual_seed(n)
+    k, v = (torch.randn(bs, H, n, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    at = {3: (0, float("inf")), 40: (127, float("-inf")), 64: (128, float("inf")), 90: (n // 2, float("-inf")), 127: (n - 2, float("inf"))}
+    for d, (key, x) in at.items():
+        v[:, :, key, d] = x
+    att = ops.DecodeAttention(bs, H, group, n, DEV)
+    q = torch.randn(bs, 1, H * group, 128, generator=g, device=DEV).to(torch.bfloat16)
+    got = ops.BoundAttention(att, q, [(k, v, 0, n)]).launch(q)
+    for d in range(128):
+        if d in at:
+            assert (got[..., d] == at[d][1]).all(), d
+        else:
+            assert torch.isfinite(got[..., d]).all(), d
+    assert torch.equal(got, att.run(q, [(k, v, 0, n)]))
