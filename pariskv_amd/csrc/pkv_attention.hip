@@ -175,9 +175,7 @@ __device__ __forceinline__ void att_last_merges(const float *ws, int row, int gr
       const int e = base + u * kThreads + tid < group * 128 ? base + u * kThreads + tid : tid & 127;
       const float *po = rowp + (e >> 7) * kPartStride + 2 + (e & 127);
 #pragma unroll
-      for (int s = 0; s < kWholeSplits; ++s) part[u][s] = get(po + (s < n_splits ? s : 0) * next);
-#pragma unroll
-      for (int s = 1; s < kWholeSplits; ++s) part[u][s] = s < n_splits ? part[u][s] : 0.f;  // split 0's may be infinite
+      for (int s = 0; s < kWholeSplits; ++s) part[u][s] = s < n_splits ? get(po + s * next) : 0.f;  // uniform
     }
     if (base == 0) {
       for (int g = tid / PKV_WAVE; g < group; g += kMfmaWaves) {  // one wave per head: lane = split
