@@ -827,14 +827,14 @@ struct LinSel {
   uint64_t T;             // threshold key inside bin b* (0: the whole bin wins); set by linear_threshold
 };
 
+__device__ __forceinline__ uint32_t lin_value_bin(float x, const LinSel &L) {
+  const uint32_t b = (uint32_t)((x - L.lo) * L.scale);
+  return b > (uint32_t)(kLinBins - 1) ? (uint32_t)(kLinBins - 1) : b;
+}
+
 __device__ __forceinline__ uint32_t lin_bin(uint64_t key, const LinSel &L) {
-  uint32_t b;
-  if (L.shift >= 0) {
-    b = ((uint32_t)(key >> 32) - L.lo_bits) >> L.shift;
-  } else {
-    const float t = (pkv_from_ordered_u32((uint32_t)(key >> 32)) - L.lo) * L.scale;
-    b = (uint32_t)t;
-  }
+  if (L.shift < 0) return lin_value_bin(pkv_from_ordered_u32((uint32_t)(key >> 32)), L);
+  const uint32_t b = ((uint32_t)(key >> 32) - L.lo_bits) >> L.shift;
   return b > (uint32_t)(kLinBins - 1) ? (uint32_t)(kLinBins - 1) : b;
 }
 
@@ -1360,7 +1360,9 @@ __device__ __forceinline__ void topk_select_sort(const float *__restrict__ x, in
 // The same for rows of 8193 to 32768 keys and k <= 2048, sorted, EIN = 16 or 32 keys a thread.  The registers hold the scores and
 // their bins, two to a word; ids are read for the winners and the threshold bin alone, in one round trip with what the caller
 // requests.  One CU reads its row's scores at some 130 GB/s, 0.8 us for 26000, and runs eight steps between barriers; the three
-// launches of the wide form read scores and ids twice and take 5 to 7 us each.  Where the bins do not apply, the radix select and
+// launches of the wide form read scores and ids twice and take 5 to 7 us each.  What the compiler would keep beside them (ordered
+// bits, places, unpacked bins) is computed again: with 32 to 64 bytes a lane in scratch instead, 8 rows x 32768 scores 10.3 (9.7), a step of
+// 8 rows x 262144 keys, top 100, 43.7 (40.7).  Where the bins do not apply, the radix select and
 // the sort of that form.  Dynamic LDS: max(P, 1024) keys; s_sel lies elsewhere.  more(): the caller's own requests.
 template <int EIN, typename Requests>
 __device__ __forceinline__ void topk_select_long(const float *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ ids,
@@ -1373,11 +1375,12 @@ __device__ __forceinline__ void topk_select_long(const float *__restrict__ x, in
   const int64_t *ir = ids ? ids + (int64_t)row * ids_stride : nullptr;
   int64_t *oi = out_ids + (int64_t)row * k;
   float *ov = out_vals ? out_vals + (int64_t)row * k : nullptr;
-  uint32_t ord[EIN], bins[EIN / 2];
+  float val[EIN];
+  uint32_t bins[EIN / 2];
 #pragma unroll
   for (int e = 0; e < EIN; ++e) {
-    const int i = tid + e * kTopkThreads;
-    ord[e] = __float_as_uint(xr[i < len ? i : len - 1]);
+    const uint32_t i = (uint32_t)(tid + e * kTopkThreads), last = (uint32_t)len - 1;
+    val[e] = *(const float *)((const char *)xr + 4u * (i < last ? i : last));
   }
   // 16 keys a thread leave registers for the caller's requests at once, 32 only when scores and bins are done with: 8 rows x
   // 131072 keys, top 100, 33.8 / 33.2 us a step late / at once; 262144 keys 47.1 / 48.4
@@ -1389,9 +1392,10 @@ __device__ __forceinline__ void topk_select_long(const float *__restrict__ x, in
   uint32_t mx = 0u, mn = 0xffffffffu;
 #pragma unroll
   for (int e = 0; e < EIN; ++e) {
-    ord[e] = pkv_ordered_u32(__uint_as_float(ord[e]));
-    mx = ord[e] > mx ? ord[e] : mx;
-    mn = ord[e] < mn ? ord[e] : mn;
+    const uint32_t ord = pkv_ordered_u32(val[e]);
+    asm("" : "+v"(val[e]));  // its ordered bits are computed again: kept as well, they are a register more
+    mx = ord > mx ? ord : mx;
+    mn = ord < mn ? ord : mn;
   }
   lin_range(mx, mn, sm.bcast);
   LinSel L;
@@ -1399,8 +1403,9 @@ __device__ __forceinline__ void topk_select_long(const float *__restrict__ x, in
   if (lin) {
 #pragma unroll
     for (int e = 0; e < EIN; e += 2) {
-      const uint32_t b0 = lin_bin((uint64_t)ord[e] << 32, L), b1 = lin_bin((uint64_t)ord[e + 1] << 32, L);
+      const uint32_t b0 = lin_value_bin(val[e], L), b1 = lin_value_bin(val[e + 1], L);
       bins[e / 2] = b0 | b1 << 16;
+      asm("" : "+v"(bins[e / 2]));  // one register, not the two that the compiler would rather keep
       if (e < n_mine) atomicAdd(&sm.hist[b0], 1u);
       if (e + 1 < n_mine) atomicAdd(&sm.hist[b1], 1u);
     }
@@ -1427,11 +1432,13 @@ __device__ __forceinline__ void topk_select_long(const float *__restrict__ x, in
   }
   // counting sort as in topk_select_sort, the keys with their positions in the row first
   const uint32_t n_above = (uint32_t)k - L.need;
+  uint32_t first = (uint32_t)tid;
+  if (EIN > 16) asm("" : "+v"(first));  // places computed again: kept since the loads, they are a register each
 #pragma unroll
   for (int e = 0; e < EIN; ++e) {
     const uint32_t bin = (e & 1) ? bins[e / 2] >> 16 : bins[e / 2] & 0xffffu;
     if (e < n_mine && bin >= L.bstar) {
-      const uint64_t key = (uint64_t)ord[e] << 32 | (uint32_t)(tid + e * kTopkThreads);
+      const uint64_t key = (uint64_t)pkv_ordered_u32(val[e]) << 32 | (first + (uint32_t)(e * kTopkThreads));
       if (bin > L.bstar) s_keys[atomicAdd(&sm.cnt[bin], 1u)] = key;
       else sm.bucket[atomicAdd(&sm.bcast[6], 1u)] = key;
     }

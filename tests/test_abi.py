@@ -3,6 +3,8 @@ include/pariskv_hip.h declares, and the Python binding has a prototype for each.
 import ctypes
 import os
 import re
+import shutil
+import subprocess
 
 import pytest
 
@@ -294,3 +296,25 @@ def test_decode_step_merges_up_to_six_blocks_in_one_workgroup():
                                 (8, 9000, 193, 0), (8, 9000, 512, 0), (128, 9000, 250, 1), (128, 9000, 257, 0), (8, 4000, 1024, 2), (8, 4000, 1025, 0)):
         a, ws, _, aa = _in_place_step(bs=rows, H=1, n_keys=20000, n_cand=cand, k=k)  # 64 rows before the selected ones: two whole blocks
         assert form(a, ws, aa) == want, (rows, cand, k)
+
+
+def test_topk_kernels_have_no_scratch(tmp_path):
+    """The selections hold up to 32 scores a thread in the 128 registers that 16 waves a CU leave: a spilled one is a trip to memory."""
+    from pariskv_amd import _lib
+
+    llvm = "/opt/rocm/llvm/bin/"
+    if not (os.path.exists(llvm + "llvm-objdump") and os.path.exists(llvm + "llvm-readelf")):
+        pytest.skip("no tools to read the library")
+    if not os.path.exists(_lib.SO_PATH):
+        _lib.build()
+    shutil.copy(_lib.SO_PATH, tmp_path / "lib.so")   # the parts are written beside it
+    subprocess.run([llvm + "llvm-objdump", "--offloading", "lib.so"], cwd=tmp_path, check=True, capture_output=True)
+    sizes = {}
+    for part in tmp_path.glob("lib.so.*gfx950"):
+        notes = subprocess.run([llvm + "llvm-readelf", "--notes", str(part)], check=True, capture_output=True, text=True).stdout
+        for kernel in re.split(r"(?m)^  - ", notes):
+            name, size = re.search(r"(?m)^    \.name: +(\S+)", kernel), re.search(r"\.private_segment_fixed_size: +(\d+)", kernel)
+            if name and size:
+                sizes[name.group(1)] = int(size.group(1))
+    topk = {n: s for n, s in sizes.items() if "pkv_topk" in n}
+    assert sum("long" in n for n in topk) == 4 and not any(topk.values()), topk
