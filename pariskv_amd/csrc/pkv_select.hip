@@ -578,6 +578,16 @@ __device__ __forceinline__ void wave_hist_add(uint32_t *hist, uint32_t d, bool a
   if (active) atomicAdd(&hist[d], 1u);
 }
 
+// Lanes that meet in a bin are counted one after the other.  A wave that sees many do so, in one of its values or of every eight, adds
+// up the largest such group of every value first (wave_hist_add, one round); spread scores put at most 1 in 100 in one bin.
+constexpr int kCrowdedLanes = 16;
+__device__ __forceinline__ bool wave_crowded(uint32_t bin, bool active) {
+  const uint64_t act = __ballot(active);
+  if (act == 0) return false;
+  const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)bin, __ffsll((long long)act) - 1);
+  return __popcll(__ballot(active && bin == b)) >= kCrowdedLanes;
+}
+
 // Slot for every lane with `take` set, out of a workgroup-wide counter: one atomic per wave.
 __device__ __forceinline__ uint32_t wave_take_slots(uint32_t *counter, bool take) {
   const uint64_t m = __ballot(take);
@@ -859,6 +869,14 @@ __device__ __forceinline__ void lin_range(uint32_t &mx, uint32_t &mn, uint32_t *
   }
   __syncthreads();
   mx = s_bcast[0], mn = s_bcast[1];
+}
+
+// ... once more, of other values.
+__device__ __forceinline__ void lin_range_again(uint32_t &mx, uint32_t &mn, uint32_t *s_bcast) {
+  __syncthreads();
+  if (threadIdx.x == 0) s_bcast[0] = 0u, s_bcast[1] = 0xffffffffu;
+  __syncthreads();
+  lin_range(mx, mn, s_bcast);
 }
 
 // The bins of that range; false = not applicable.
@@ -1357,13 +1375,73 @@ __device__ __forceinline__ void topk_select_sort(const float *__restrict__ x, in
 #undef PKV_SORT_K
 }
 
+// Of a thread's EIN values, those whose bit is set in `edge`, n_edge of them in the workgroup and all between mn and mx, the `need` largest
+// win: bins of their bits, then of those in the bin that holds the last winner, until that one is small or taken whole.  Winners
+// go from edge to win.  On return n_edge <= kLinBucketMax, or n_edge == need, or all that are left are equal.  A round narrows the
+// range 512-fold, so four are the most.  val(e) is read again in every pass, eight in flight, from the L2: kept in registers across
+// the rounds they spill.  All 1024 threads call it.
+template <int EIN, typename Val>
+__device__ __forceinline__ void narrow_edge(Val val, uint32_t &win, uint32_t &edge, uint32_t &need, uint32_t &n_edge, uint32_t mx,
+                                            uint32_t mn, SelSmem &sm) {
+  LinSel L;
+  while (n_edge > (uint32_t)kLinBucketMax && n_edge != need && lin_steps<true>(mx, mn, L)) {  // uniform
+    __syncthreads();  // what the last round left has been read
+    lin_clear(sm.hist, sm.bcast);
+    __syncthreads();
+#pragma unroll 1
+    for (int e0 = 0; e0 < EIN; e0 += 8) {
+      uint32_t v[8];
+      const uint32_t some = edge >> e0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = (val(e0 + u) - L.lo_bits) >> L.shift;
+      if (wave_crowded(v[0], some & 1u) || wave_crowded(v[4], some & 16u)) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) wave_hist_add(sm.hist, v[u], (some >> u) & 1u, 1);
+      } else {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if ((some >> u) & 1u) atomicAdd(&sm.hist[v[u]], 1u);
+      }
+    }
+    __syncthreads();
+    lin_decide<false>(need, sm.hist, sm.cnt, sm.bcast, L);
+    uint32_t above = 0u, in = 0u;
+    mx = 0u, mn = 0xffffffffu;
+#pragma unroll 1
+    for (int e0 = 0; e0 < EIN; e0 += 8) {
+      uint32_t v[8], a = 0u, d = 0u;
+      const uint32_t some = edge >> e0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = val(e0 + u);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const uint32_t b = (v[u] - L.lo_bits) >> L.shift;
+        a |= b > L.bstar ? some & (1u << u) : 0u;
+        if ((some & (1u << u)) && b == L.bstar) {
+          d |= 1u << u;
+          mx = v[u] > mx ? v[u] : mx;
+          mn = v[u] < mn ? v[u] : mn;
+        }
+      }
+      above |= a << e0, in |= d << e0;
+    }
+    win |= above, edge = in, need = L.need, n_edge = L.in_bstar;
+    lin_range(mx, mn, sm.bcast);  // its two words are as lin_clear left them
+  }
+}
+
 // The same for rows of 8193 to 32768 keys and k <= 2048, sorted, EIN = 16 or 32 keys a thread.  The registers hold the scores and
 // their bins, two to a word; ids are read for the winners and the threshold bin alone, in one round trip with what the caller
 // requests.  One CU reads its row's scores at some 130 GB/s, 0.8 us for 26000, and runs eight steps between barriers; the three
 // launches of the wide form read scores and ids twice and take 5 to 7 us each.  What the compiler would keep beside them (ordered
 // bits, places, unpacked bins) is computed again: with 32 to 64 bytes a lane in scratch instead, 8 rows x 32768 scores 10.3 (9.7), a step of
-// 8 rows x 262144 keys, top 100, 43.7 (40.7).  Where the bins do not apply, the radix select and
-// the sort of that form.  Dynamic LDS: max(P, 1024) keys; s_sel lies elsewhere.  more(): the caller's own requests.
+// 8 rows x 262144 keys, top 100, 43.7 (40.7).
+// Infinities and NaN stay out of the bins' range.  Where the bins leave too many keys at the threshold (outliers, many equal scores),
+// narrow_edge over the scores, then over the ids of those that tie.  Top-k of 8 rows x 32768, top 100, us, three launches / a radix select
+// of eight passes over scores and ids from memory / this: spread scores 20.8 / 9.7 / 9.9, infinities 22.1 / 65.4 / 18.4, log-normal 20.8 /
+// 35.9 / 16.5, one outlier 76 / 94 / 54, four values 67 / 121 / 55, one value 185 / 184 / 37; 8 x 9000 infinities 21.9 / 25.1 / 10.4, log-normal
+// 21.0 / 28.4 / 22.9.
+// Dynamic LDS: 2 max(P, 1024) keys; s_sel lies elsewhere.  more(): the caller's own requests.
 template <int EIN, typename Requests>
 __device__ __forceinline__ void topk_select_long(const float *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ ids,
                                                  int64_t ids_stride, int len, int P, int64_t k, int64_t *__restrict__ out_ids,
@@ -1399,35 +1477,165 @@ __device__ __forceinline__ void topk_select_long(const float *__restrict__ x, in
   }
   lin_range(mx, mn, sm.bcast);
   LinSel L;
-  bool lin = lin_steps<false>(mx, mn, L);  // uniform over the workgroup
-  if (lin) {
+  // uniform over the workgroup: infinities or NaN.  The bins are of the others' range; what is above or below them all goes to the
+  // highest and the lowest bin
+  const uint32_t kInf = 0xff800000u, kMinusInf = 0x007fffffu;
+  const bool infinite = mx >= kInf || mn <= kMinusInf;
+  if (infinite) {
+    mx = 0u, mn = 0xffffffffu;
 #pragma unroll
-    for (int e = 0; e < EIN; e += 2) {
-      const uint32_t b0 = lin_value_bin(val[e], L), b1 = lin_value_bin(val[e + 1], L);
-      bins[e / 2] = b0 | b1 << 16;
-      asm("" : "+v"(bins[e / 2]));  // one register, not the two that the compiler would rather keep
-      if (e < n_mine) atomicAdd(&sm.hist[b0], 1u);
-      if (e + 1 < n_mine) atomicAdd(&sm.hist[b1], 1u);
+    for (int e = 0; e < EIN; ++e) {
+      const uint32_t ord = pkv_ordered_u32(val[e]);
+      asm("" : "+v"(val[e]));
+      mx = ord < kInf && ord > mx ? ord : mx;
+      mn = ord > kMinusInf && ord < mn ? ord : mn;
+    }
+    lin_range_again(mx, mn, sm.bcast);
+  }
+  const bool binned = lin_steps<false>(mx, mn, L);
+  auto bin_of = [&](float x) {
+    const uint32_t ord = pkv_ordered_u32(x);
+    if (infinite && ord >= kInf) return (uint32_t)kLinBins - 1;
+    if (infinite && ord <= kMinusInf) return 0u;
+    return lin_value_bin(x, L);
+  };
+  bool lin = false;
+  if (binned) {
+    // (a pair of bins in one register, not in the two that the compiler would rather keep)
+    if (infinite || wave_crowded(lin_value_bin(val[0], L), true)) {
+#pragma unroll
+      for (int e = 0; e < EIN; e += 2) {
+        const uint32_t b0 = bin_of(val[e]), b1 = bin_of(val[e + 1]);
+        bins[e / 2] = b0 | b1 << 16;
+        asm("" : "+v"(bins[e / 2]));
+        wave_hist_add(sm.hist, b0, e < n_mine, 1);
+        wave_hist_add(sm.hist, b1, e + 1 < n_mine, 1);
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < EIN; e += 2) {
+        const uint32_t b0 = lin_value_bin(val[e], L), b1 = lin_value_bin(val[e + 1], L);
+        bins[e / 2] = b0 | b1 << 16;
+        asm("" : "+v"(bins[e / 2]));
+        if (e < n_mine) atomicAdd(&sm.hist[b0], 1u);
+        if (e + 1 < n_mine) atomicAdd(&sm.hist[b1], 1u);
+      }
     }
     __syncthreads();
     lin = lin_decide<true>((uint32_t)k, sm.hist, sm.cnt, sm.bcast, L) && L.max_winners <= kLinRankMax;
   }
+  // positions in the row become ids: the first n_keys of s_keys and the first n_bucket of the threshold bin, in one round trip
+  auto name_keys = [&](uint32_t n_keys, uint32_t n_bucket) {
+    constexpr int kOut = kCountingSortMaxP / kTopkThreads;
+    uint64_t key[kOut + 1];
+    uint32_t id[kOut + 1];
+#pragma unroll
+    for (int u = 0; u <= kOut; ++u) {
+      const uint32_t p = (uint32_t)(tid + (u < kOut ? u : 0) * kTopkThreads);
+      key[u] = u < kOut ? (p < n_keys ? s_keys[p] : 0ull) : (p < n_bucket ? sm.bucket[p] : 0ull);
+      id[u] = ir ? (uint32_t)ir[(uint32_t)key[u]] : (uint32_t)key[u];
+    }
+#pragma unroll
+    for (int u = 0; u <= kOut; ++u) {
+      const uint32_t p = (uint32_t)(tid + (u < kOut ? u : 0) * kTopkThreads);
+      const uint64_t whole = (key[u] & 0xffffffff00000000ull) | (uint64_t)(uint32_t)~id[u];
+      if (u < kOut && p < n_keys) s_keys[p] = whole;
+      if (u == kOut && p < n_bucket) sm.bucket[p] = whole;
+    }
+    __syncthreads();
+  };
+  auto emit = [&](uint32_t at, uint64_t key) {
+    oi[at] = (int64_t)(uint32_t)(~(uint32_t)key);
+    if (s_sel) s_sel[at] = ~(uint32_t)key;
+    if (ov) ov[at] = pkv_from_ordered_u32((uint32_t)(key >> 32));
+  };
   if (!lin) {
-    if (!kEarly) more();
-    auto key_of = [&](int64_t i) { return make_key(xr, ir, i); };
-    uint64_t prefix;
-    int shift;
+    // scores and ids are read again, from the L2
+    uint32_t first = (uint32_t)tid;
+    asm("" : "+v"(first));  // and their places computed again
+    auto place = [&](int e) { const uint32_t i = first + (uint32_t)(e * kTopkThreads); return i < (uint32_t)len ? i : (uint32_t)len - 1; };
+    auto score = [&](int e) { return pkv_ordered_u32(*(const float *)((const char *)xr + 4u * place(e))); };
+    auto name = [&](int e) { return ~(ir ? *(const uint32_t *)((const char *)ir + 8u * place(e)) : place(e)); };
+    uint32_t win = 0u, edge = n_mine >= 32 ? 0xffffffffu : (1u << n_mine) - 1u, need = (uint32_t)k, n_edge = (uint32_t)len;
+    if (binned) {  // as far as the bins above got
+      uint32_t above = 0u, in = 0u;
+      mx = 0u, mn = 0xffffffffu;
+#pragma unroll 1
+      for (int e0 = 0; e0 < EIN; e0 += 8) {
+        uint32_t v[8], a = 0u, d = 0u;
+        const uint32_t some = edge >> e0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = score(e0 + u);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const uint32_t b = bin_of(pkv_from_ordered_u32(v[u]));
+          a |= b > L.bstar ? some & (1u << u) : 0u;
+          if ((some & (1u << u)) && b == L.bstar) {
+            d |= 1u << u;
+            mx = v[u] > mx ? v[u] : mx;
+            mn = v[u] < mn ? v[u] : mn;
+          }
+        }
+        above |= a << e0, in |= d << e0;
+      }
+      win = above, edge = in, need = L.need, n_edge = L.in_bstar;
+      lin_range_again(mx, mn, sm.bcast);
+    } else if (infinite) {
+      mx = 0xffffffffu, mn = 0u;
+    }
+    narrow_edge<EIN>(score, win, edge, need, n_edge, mx, mn, sm);
+    if (n_edge > (uint32_t)kLinBucketMax && n_edge != need) {  // more equal scores than win: the smallest ids do
+      mx = 0u, mn = 0xffffffffu;
+#pragma unroll 1
+      for (int e0 = 0; e0 < EIN; e0 += 8) {
+        uint32_t v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = name(e0 + u);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          if ((edge >> e0) & (1u << u)) {
+            mx = v[u] > mx ? v[u] : mx;
+            mn = v[u] < mn ? v[u] : mn;
+          }
+        }
+      }
+      lin_range_again(mx, mn, sm.bcast);
+      narrow_edge<EIN>(name, win, edge, need, n_edge, mx, mn, sm);
+    }
+    const uint32_t n_above = (uint32_t)k - need;
+    const bool in_bucket = n_edge <= (uint32_t)kLinBucketMax;  // if not, all of the edge win, or any of its equal keys
     __syncthreads();
-    radix_select_streamed(key_of, len, (uint32_t)k, sm.hist, sm.bcast, prefix, shift);
     for (int i = tid; i < (P < 1024 ? 1024 : P); i += kTopkThreads) s_keys[i] = 0ull;
-    if (tid == 0) sm.counter = 0;
+    if (tid < 2) sm.cnt[tid] = 0u;
     __syncthreads();
-    collect_winners_streamed(key_of, len, (uint32_t)k, prefix, shift, &sm.counter, s_keys);
+#pragma unroll 1
+    for (int e0 = 0; e0 < EIN; e0 += 8) {
+      uint32_t v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = score(e0 + u);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const uint64_t key = (uint64_t)v[u] << 32 | place(e0 + u);
+        const bool w = (win >> (e0 + u)) & 1u, d = (edge >> (e0 + u)) & 1u;
+        const uint32_t slot = wave_take_slots(&sm.cnt[0], w), slot_d = wave_take_slots(&sm.cnt[1], d);
+        if (w && slot < n_above) s_keys[slot] = key;
+        if (d && in_bucket) sm.bucket[slot_d] = key;
+        if (d && !in_bucket && slot_d < need) s_keys[n_above + slot_d] = key;
+      }
+    }
     __syncthreads();
-    if (P <= 1024) sort_lds_keys_and_emit<1024, 1>(s_keys, k, oi, ov, s_sel ? s_keys : nullptr);
-    else sort_lds_keys_and_emit<1024, 2>(s_keys, k, oi, ov, s_sel ? s_keys : nullptr);
-    if (s_sel)
-      for (int i = tid; i < (int)k; i += kTopkThreads) s_sel[i] = ~(uint32_t)s_keys[i];
+    name_keys(in_bucket ? n_above : (uint32_t)k, in_bucket ? n_edge : 0u);
+    if (in_bucket) {  // uniform
+      rank_bucket_desc(sm.bucket, n_edge, [&](uint64_t key, uint32_t r) {
+        if (r < need) s_keys[n_above + r] = key;
+      });
+      __syncthreads();
+    }
+    uint64_t *s_tmp = s_keys + (P < 1024 ? 1024 : P);
+    if (P <= 1024) sort_lds_keys_desc<1024, 1>(s_keys, (uint32_t)k, s_tmp, sm);
+    else sort_lds_keys_desc<1024, 2>(s_keys, (uint32_t)k, s_tmp, sm);
+    for (int i = tid; i < (int)k; i += kTopkThreads) emit((uint32_t)i, s_keys[i]);
+    if (!kEarly) more();
     return;
   }
   // counting sort as in topk_select_sort, the keys with their positions in the row first
@@ -1445,34 +1653,11 @@ __device__ __forceinline__ void topk_select_long(const float *__restrict__ x, in
   }
   __syncthreads();
   if (!kEarly) more();
-  {  // ... then with their ids
-    constexpr int kOut = kCountingSortMaxP / kTopkThreads;
-    uint64_t key[kOut + 1];
-    uint32_t id[kOut + 1];
-#pragma unroll
-    for (int u = 0; u <= kOut; ++u) {
-      const uint32_t p = (uint32_t)(tid + (u < kOut ? u : 0) * kTopkThreads);
-      key[u] = u < kOut ? (p < n_above ? s_keys[p] : 0ull) : (p < L.in_bstar ? sm.bucket[p] : 0ull);
-      id[u] = ir ? (uint32_t)ir[(uint32_t)key[u]] : (uint32_t)key[u];
-    }
-#pragma unroll
-    for (int u = 0; u <= kOut; ++u) {
-      const uint32_t p = (uint32_t)(tid + (u < kOut ? u : 0) * kTopkThreads);
-      const uint64_t whole = (key[u] & 0xffffffff00000000ull) | (uint64_t)(uint32_t)~id[u];
-      if (u < kOut && p < n_above) s_keys[p] = whole;
-      if (u == kOut && p < L.in_bstar) sm.bucket[p] = whole;
-    }
-  }
-  __syncthreads();
-  auto emit = [&](uint32_t at, uint64_t key) {
-    oi[at] = (int64_t)(uint32_t)(~(uint32_t)key);
-    if (s_sel) s_sel[at] = ~(uint32_t)key;
-    if (ov) ov[at] = pkv_from_ordered_u32((uint32_t)(key >> 32));
-  };
+  name_keys(n_above, L.in_bstar);
   const uint32_t *s_off = sm.hist + kLinBins;
   for (uint32_t p = tid; p < n_above; p += kTopkThreads) {
     const uint64_t key = s_keys[p];
-    const uint32_t b = lin_bin(key, L);
+    const uint32_t b = bin_of(pkv_from_ordered_u32((uint32_t)(key >> 32)));
     const uint32_t start = s_off[b], cnt = sm.cnt[b] - start;
     uint32_t r = 0;
 #pragma unroll 4
@@ -1491,7 +1676,7 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_select_long_kernel(
   topk_select_long<EIN>(x, x_stride, ids, ids_stride, len, P, k, out_ids, out_vals, nullptr, [] {});
 }
 
-// ... and the attention over the winners, merged: see pkv_topk_attend_kernel.  Dynamic LDS: max(P, 1024) keys, then k words.
+// ... and the attention over the winners, merged: see pkv_topk_attend_kernel.  Dynamic LDS: 2 max(P, 1024) keys, then k words.
 template <int EIN>
 __global__ __launch_bounds__(kTopkThreads) void pkv_topk_long_attend_kernel(
     const float *__restrict__ x, int64_t x_stride, const int64_t *__restrict__ ids, int64_t ids_stride, int len, int P, int64_t k,
@@ -1499,7 +1684,7 @@ __global__ __launch_bounds__(kTopkThreads) void pkv_topk_long_attend_kernel(
   extern __shared__ uint64_t s_keys[];
   __shared__ AttSelSmem sm;
   const int row = blockIdx.x;
-  uint32_t *s_sel = (uint32_t *)(s_keys + (P < 1024 ? 1024 : P));
+  uint32_t *s_sel = (uint32_t *)(s_keys + 2 * (P < 1024 ? 1024 : P));
   AttSelRequests req;
   att_clear(sm);
   topk_select_long<EIN>(x, x_stride, ids, ids_stride, len, P, k, out_ids, out_vals, s_sel, [&] {
@@ -2755,10 +2940,10 @@ int pkv_launch_topk_f32(const float *x, int64_t x_stride, const int64_t *ids, in
 #define PKV_SEL(EIN)                                                                                                            \
   do {                                                                                                                          \
     if (attn)                                                                                                                   \
-      hipLaunchKernelGGL(pkv_topk_long_attend_kernel<EIN>, dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes(P) + (size_t)k * 4, \
+      hipLaunchKernelGGL(pkv_topk_long_attend_kernel<EIN>, dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes_sort(P) + (size_t)k * 4, \
                          s, x, x_stride, ids, ids_stride, (int)len, P, k, out_ids, out_vals, *attn);                            \
     else                                                                                                                        \
-      hipLaunchKernelGGL(pkv_topk_select_long_kernel<EIN>, dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes(P), s, x, x_stride, \
+      hipLaunchKernelGGL(pkv_topk_select_long_kernel<EIN>, dim3((unsigned)rows), dim3(kTopkThreads), lds_bytes_sort(P), s, x, x_stride, \
                          ids, ids_stride, (int)len, P, k, out_ids, out_vals);                                                   \
   } while (0)
       if (len <= 2 * kTopkMaxSort) PKV_SEL(16); else PKV_SEL(32);

@@ -2163,6 +2163,89 @@ def test_topk_f32_of_long_rows(ops, rows, L, k, kind):
         assert np.array_equal(pos[r].cpu().numpy(), O.topk_f32(x[r], None, k)[1])
 
 
+@pytest.mark.parametrize("L,k", [(8193, 1), (8193, 2048), (16384, 256), (16385, 257), (26000, 1024), (32768, 2048)])
+@pytest.mark.parametrize("kind", ["log-normal", "outlier", "two outliers", "lowest outlier", "half zero", "many infinite", "infinite only", "few finite",
+                                  "nan of both signs", "tie 256", "tie 257", "tie taken whole", "equal ids", "neighbours"])
+def test_topk_f32_of_long_rows_narrows_the_edge(ops, L, k, kind):
+    """Scores that the bins of a long row's range leave together: binned again, by their bits and then by the ids of those that tie, up to
+    the most keys that are ranked one by one (256) and beyond.  Ids and scores exactly as the oracle's."""
+    _say(f"topk_f32 long, edge {L} k={k} {kind}")
+    rng = np.random.default_rng(L * 31 + k)
+    x = rng.standard_normal((2, L)).astype(np.float32)
+    ids = np.stack([rng.permutation(2 * L)[:L] for _ in range(2)]).astype(np.int64)
+    if kind == "log-normal":
+        x = np.exp(4 * x)
+    elif kind == "outlier":
+        x[:, L // 3] = 1e30
+    elif kind == "two outliers":
+        x[:, L // 3], x[:, L - 1] = 1e30, 1e9
+    elif kind == "lowest outlier":
+        x[:, 5] = np.finfo(np.float32).min
+    elif kind == "half zero":
+        x = np.maximum(x, np.float32(0))
+        x[:, ::3] = -0.0
+    elif kind == "many infinite":
+        x[0, ::5], x[1, ::7] = np.inf, -np.inf
+    elif kind == "infinite only":
+        x[0], x[1] = np.where(x[0] > 0, np.inf, -np.inf), np.inf
+    elif kind == "few finite":
+        x[:, 300:] = -np.inf
+    elif kind == "nan of both signs":
+        x[:, 3::40] = np.nan
+        x.view(np.uint32)[:, 4::50] = 0xffc00001
+        x[:, 6::60] = -np.inf
+    elif kind.startswith("tie"):   # k - 1 scores above the tied ones, or (taken whole) as many above as leave all of them winners
+        n = {"tie 256": 256, "tie 257": 257, "tie taken whole": 300}[kind]
+        above = max(0, k - (n if n == 300 else 1))
+        for r in range(2):
+            order = rng.permutation(L)
+            x[r] = -np.abs(x[r]) - 1
+            x[r, order[:above]] = 100 + rng.random(above).astype(np.float32)
+            x[r, order[above:above + n]] = 50
+    elif kind == "equal ids":
+        x[:] = np.where(x > 1, 2.0, 0.5)
+        ids[:] = 7
+    elif kind == "neighbours":   # one part in 2^23 apart, beside one far away
+        x = (np.float32(1.0).view(np.uint32) + rng.integers(0, 900, (2, L)).astype(np.uint32)).view(np.float32)
+        x[:, 0] = -1e5
+    out, vals = ops.topk_f32(torch.from_numpy(x).to(DEV), k, torch.from_numpy(ids).to(DEV), want_values=True)
+    pos = ops.topk_f32(torch.from_numpy(x).to(DEV), k)
+    torch.cuda.synchronize()
+    for r in range(2):
+        ref_ids, ref_pos = O.topk_f32(x[r], ids[r], k)
+        assert np.array_equal(out[r].cpu().numpy(), ref_ids)
+        assert np.array_equal(vals[r].cpu().numpy().view(np.uint32), x[r][ref_pos].view(np.uint32))
+        assert np.array_equal(pos[r].cpu().numpy(), O.topk_f32(x[r], None, k)[1])
+
+
+def test_topk_f32_of_long_rows_with_infinities_is_no_cliff(ops):
+    """A few infinities among the scores of a long row cost no more than three times a row without (1.9; a selection that reads scores and ids
+    from memory in each of eight passes, 6.3).  The best of several replays of a graph."""
+    _say("topk_f32 long, time of infinities")
+    x = torch.randn(8, 32768, generator=torch.Generator(device=DEV).manual_seed(0), device=DEV)
+    y, ids = x.clone(), torch.arange(32768, device=DEV).repeat(8, 1)
+    y[:, ::1000] = float("inf")
+    took = []
+    for s in (x, y):
+        ops.topk_f32(s, 100, ids)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                ops.topk_f32(s, 100, ids)
+        graph.replay()
+        best = float("inf")
+        for _ in range(10):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            graph.replay()
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b))
+        took.append(best)
+    assert took[1] <= 3 * took[0], took
+
+
 @pytest.mark.parametrize("scores", [None, "equal", "infinite"])
 @pytest.mark.parametrize("bs,group,k,keys,cand", [(2, 4, 100, 40000, 16384), (1, 8, 192, 40000, 16385), (2, 3, 1, 60000, 32768)])
 def test_decode_step_merges_after_the_selection_from_a_long_row(ops, bs, group, k, keys, cand, scores):
