@@ -653,10 +653,11 @@ typedef struct pkv_attn_args {
 int pkv_decode_attention_run(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_args *args,
                              void *stream);
 
-/* The same with counters (no counterpart in the reference): arrivals [2 * bs * n_kv_heads] words belong to args->ws, are zero before the first launch and left
- * zero by every launch; turn, 0 or 1, says which half this launch counts in, and launches that take turns clear what launches
- * that overlapped have left.  Same results; a short set of keys then takes one launch instead of two.  Launches that share ws
- * and arrivals follow one another on the GPU, as for ws alone. */
+/* The same with counters (no counterpart in the reference): arrivals [2 * bs * n_kv_heads] words belong to args->ws, are
+ * zero before the first launch and left zero by every launch; turn, 0 or 1, says which half this launch counts in, and
+ * launches that take turns clear what launches that overlapped have left.  Same results; a short set of keys then takes one
+ * launch instead of two, except under capture, where nothing is counted.  Launches that share ws and arrivals follow one
+ * another on the GPU, as for ws alone. */
 int pkv_decode_attention_counted(const void *q, int dtype, int bs, int n_kv_heads, int group, const pkv_attn_args *args,
                                  uint32_t *arrivals, int turn, void *stream);
 

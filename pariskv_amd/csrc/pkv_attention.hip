@@ -29,10 +29,13 @@ namespace {
 constexpr int kAttThreads = 256;
 constexpr int kAttKeysPerIter = kAttThreads / 16;  // 16 keys per workgroup step
 // A call whose caller keeps counters takes one launch, the last workgroup of a row merging, up to this many splits a row and
-// workgroups in all.  A decode step over a short context waits for its launches' host time (3.4 us each), not for the GPU: 8 rows x
+// workgroups in all, unless it is captured: a replayed graph has no host time to save, and would count in one half of the counters for
+// good.  A decode step over a short context waits for its launches' host time (3.4 us each), not for the GPU: 8 rows x
 // 1500 keys, append and attention, 14.1 us a step where two launches for the attention took 16.7.  Back to back and with nothing else
 // to launch, us, one / two launches: 8 rows x 300 keys 7.0 / 9.7, 1600 8.0 / 9.9, 16 rows x 1600 9.0 / 9.6, 32 x 1600 10.1 / 9.3,
 // 8 x 2500 9.7 / 9.7, 4000 11.0 / 9.9; the GPU alone, without the host, 6.7 / 6.2, 7.7 / 6.5, 8.9 / 6.8, 10.2 / 8.5, 9.6 / 7.7, 11.0 / 7.7.
+// In a replayed graph 8 x 300 6.8 / 6.5, 8 x 1500 7.8 / 6.9 (eight heads 10.0 / 7.8), 16 x 1600 9.0 / 7.2, 32 x 1000 8.3 / 7.2; a call whose host
+// runs ahead of the GPU loses as much, and cannot be told from one that waits for its host.
 // fp32 loses there as well (12 rows x 865 keys, 7 heads, 11.5 / 10.7) and keeps its two launches.
 constexpr int kWholeSplits = 16, kWholeWorkgroups = 256;
 constexpr int kAttUnroll = 2;                      // keys per 16-lane group per step
@@ -581,7 +584,7 @@ static int decode_attention(const void *q, int dtype, int bs, int n_kv_heads, in
   dim3 grid((unsigned)n_splits, (unsigned)rows);
   AttOne one;
   const bool is_one = as_one_tensor(sg, bf ? 2 : 4, one);
-  const bool whole = arrivals && bf && n_splits <= kWholeSplits && rows * n_splits <= kWholeWorkgroups;
+  const bool whole = arrivals && bf && n_splits <= kWholeSplits && rows * n_splits <= kWholeWorkgroups && !pkv_capturing(s);
   if (bf) {
     const dim3 grid3((unsigned)n_splits, (unsigned)n_kv_heads, (unsigned)bs);
 #define PKV_ATT_MFMA_W(IDX, S, WHOLE)                                                                                           \

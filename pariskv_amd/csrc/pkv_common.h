@@ -45,6 +45,14 @@ void pkv_set_error(const char *fmt, ...);
 static inline size_t pkv_align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 static inline bool pkv_aligned(const void *p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
+// A stream under capture, or one whose state cannot be read.
+static inline bool pkv_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 struct PkvTiers {
   uint32_t t[PKV_MAX_TIERS];
   int n;

@@ -352,12 +352,7 @@ bool pkv_fused_usable(int rows, int64_t n_keys, int chunk_keys, hipStream_t s) {
   // at most 1024 workgroups: with four of them per compute unit the whole launch is resident at once on the
   // 256 compute units, so no wait depends on the order in which workgroups are dispatched
   if (chunk_keys > kFusedMaxChunkKeys || n_chunks > 256 || (int64_t)rows * n_chunks > 1024) return false;
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
-    return false;
-  }
-  return true;
+  return !pkv_capturing(s);
 }
 
 int pkv_launch_fused_retrieve(const void *q, int dtype, int bs, int n_kv_heads, int group, const float *signs,

@@ -2363,6 +2363,13 @@ def test_bound_attention_merges_in_its_own_launch(ops, dtype, group, n):
         want = att.run(other, [(k, v, 2, n)])
         torch.cuda.synchronize()
         assert torch.equal(out, want) and not torch.any(att.arrivals)
+    # nor does a graph, which would count in the same half for good, depend on what they hold
+    att.arrivals.fill_(1)
+    for other in qs:
+        q.copy_(other)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, att.run(other, [(k, v, 2, n)])) and torch.all(att.arrivals == 1)
 
 
 @pytest.mark.parametrize("rows,L", [(3, 1), (2, 3), (3, 64), (2, 4095), (2, 4096), (3, 4097), (1, 12287), (2, 20480), (5, 24573), (2, 24577),
