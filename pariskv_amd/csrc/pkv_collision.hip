@@ -391,9 +391,11 @@ int pkv_launch_scan_attend(const uint8_t *codes, int64_t cs_b, int64_t cs_h, int
 // than the launch before the scan took on the GPU; a call waits for the host time of its launches, 3.4 us each, while its keys are
 // few.  us, GPU alone and call by itself, two launches / one: 8 rows x 3000 4.7, 15.6 / 5.4, 11.7; 16 x 20011 5.8, 15.4 / 7.0, 11.8;
 // 8 x 80001 6.8, 15.7 / 8.3, 11.7; not taken: 24 x 80001 10.3, 15.6 / 13.1, 12.7; 64 x 80000 21.4, 20.9 / 23.6, 23.3.  Codes requested
-// before the table is built: 16 x 20011 7.7.
+// before the table is built: 16 x 20011 7.7.  A captured call has no host time to save (in a graph, 8 x 3000 5.2 / 5.7, 64 x 3000 6.3 / 8.8).
 constexpr int64_t kRankedKeys = 1 << 20;
-bool pkv_scan_takes_ranking(int64_t cs_key, int rows, int64_t n_keys) { return cs_key == 1 && rows * n_keys <= kRankedKeys; }
+bool pkv_scan_takes_ranking(int64_t cs_key, int rows, int64_t n_keys, hipStream_t s) {
+  return cs_key == 1 && rows * n_keys <= kRankedKeys && !pkv_capturing(s);
+}
 
 int pkv_launch_scan_ranked(const uint8_t *codes, int64_t cs_b, int64_t cs_h, int64_t cs_sub, int bs, int n_kv_heads, int64_t n_keys,
                            const int64_t *ids, int64_t si_b, int64_t si_h, int64_t si_sub, const int32_t *cc, int64_t cc_b,

@@ -45,8 +45,9 @@ void pkv_set_error(const char *fmt, ...);
 static inline size_t pkv_align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 static inline bool pkv_aligned(const void *p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
-// A stream under capture, or one whose state cannot be read.
+// A stream under capture, or one whose state cannot be read.  The null stream cannot be captured.
 static inline bool pkv_capturing(hipStream_t s) {
+  if (s == nullptr) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
   (void)hipGetLastError();
@@ -114,7 +115,7 @@ PKV_INTERNAL int pkv_launch_scan(const uint8_t *codes, int64_t cs_b, int64_t cs_
                                  int bs, int n_kv_heads, int64_t n_keys, const uint8_t *lut, uint8_t *cnt_u8,
                                  int64_t cnt_u8_stride, int32_t *cnt_i32, uint32_t *row_suf, uint16_t *chunk_suf,
                                  int chunk_keys, hipStream_t s, int sub_blocks = 1);
-PKV_INTERNAL bool pkv_scan_takes_ranking(int64_t cs_key, int rows, int64_t n_keys);
+PKV_INTERNAL bool pkv_scan_takes_ranking(int64_t cs_key, int rows, int64_t n_keys, hipStream_t s);
 PKV_INTERNAL int pkv_launch_scan_ranked(const uint8_t *codes, int64_t cs_b, int64_t cs_h, int64_t cs_sub, int bs, int n_kv_heads,
                                         int64_t n_keys, const int64_t *ids, int64_t si_b, int64_t si_h, int64_t si_sub,
                                         const int32_t *cc, int64_t cc_b, int64_t cc_h, int64_t cc_sub, const PkvTiers &tiers,

@@ -171,7 +171,7 @@ extern "C" int pkv_update_cache_cnt(const int64_t *sorted_ids, int64_t si_b, int
   int rc = make_tiers(tier_counts, n_tiers, t);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  if (pkv_scan_takes_ranking(cs_key, bs * n_kv_heads, n_keys))
+  if (pkv_scan_takes_ranking(cs_key, bs * n_kv_heads, n_keys, s))
     return pkv_launch_scan_ranked(codes, cs_b, cs_h, cs_sub, bs, n_kv_heads, n_keys, sorted_ids, si_b, si_h, si_sub, cluster_counts,
                                   cc_b, cc_h, cc_sub, t, cnt, s);
   dim3 grid(16, (unsigned)(bs * n_kv_heads));

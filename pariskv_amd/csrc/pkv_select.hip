@@ -2761,7 +2761,12 @@ static void bucket_ws_layout(int rows, int64_t len, int &chunk_keys, int64_t &cn
 // One launch instead of two where a row's workgroup is as fast as the chunks', or nearly.  us on the GPU, two launches / one: 16 rows
 // x 4096 5.5 / 3.2, x 9001 6.4 / 4.7, x 20011 7.4 / 6.6, x 32768 6.8 / 9.0; 64 rows x 32768 9.2 / 9.3, 256 rows 25.2 / 12.6.  A call by
 // itself, host included: 13.5 / 8.3, 16 rows x 32768 13.6 / 8.9.
-constexpr int kBucketMaxBlocks = 8, kBucketFewRowsBlocks = 6, kBucketManyRows = 64;
+// A captured call has no host time to save: 16 rows x 20480 7.4 / 6.7, x 24576 6.7 / 7.6, 32 x 24576 7.4 / 7.7, 63 x 24576 9.0 / 7.8,
+// 64 x 28672 10.1 / 8.6, x 32768 9.0 / 9.4, 96 x 32768 10.4 / 9.7.
+static int bucket_row_blocks(int rows, bool captured) {
+  if (captured) return rows < 48 ? 5 : rows < 96 ? 7 : 8;
+  return rows < 64 ? 6 : 8;
+}
 
 extern "C" size_t pkv_bucket_topk_ws_bytes(int rows, int64_t len) {
   if (rows <= 0 || len <= 0) return 256;
@@ -2790,7 +2795,7 @@ extern "C" int pkv_bucket_topk(const int32_t *x, int64_t x_stride, int rows, int
     return PKV_ENOMEM;
   }
   const int blocks = (int)((len + kBucketBlock - 1) / kBucketBlock);
-  if (blocks <= (rows < kBucketManyRows ? kBucketFewRowsBlocks : kBucketMaxBlocks)) {
+  if (blocks <= 5 || (blocks <= 8 && blocks <= bucket_row_blocks(rows, pkv_capturing(s)))) {
 #define PKV_BUCKET(NB)                                                                                                  \
   hipLaunchKernelGGL(pkv_bucket_row_kernel<NB>, dim3((unsigned)rows), dim3(kBucketThreads), 0, s, x, x_stride, (int)len, (int)k, out)
     switch (blocks) {

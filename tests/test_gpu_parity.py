@@ -2426,3 +2426,58 @@ def test_bound_attention_of_infinite_values(ops, group, n):
         else:
             assert torch.isfinite(got[..., d]).all(), d
     assert torch.equal(got, att.run(q, [(k, v, 0, n)]))
+
+
+@pytest.mark.parametrize("what", ["votes", "bucket"])
+def test_captured_operators_take_their_faster_launches(ops, what):
+    """Votes from a ranking and the bucket top-k of a row that one launch is as long as two for: replayed, the same results as eagerly, in
+    the two launches that are faster where no host waits (one launch writes nothing into the table's workspace or the counts')."""
+    from pariskv_amd import _lib
+
+    _say(f"captured {what}")
+    g = torch.Generator(device=DEV).manual_seed(3)
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    if what == "votes":
+        bs, H, N = 2, 3, 3001
+        ids = torch.randint(0, 256, (bs, H, 16, 256), generator=g, device=DEV)
+        counts = torch.randint(0, 40, (bs, H, 16, 256), generator=g, device=DEV, dtype=torch.int32)
+        code = torch.randint(0, 256, (bs, H, 16, N), generator=g, device=DEV).to(torch.uint8)
+        ws, out = torch.zeros(bs * H * 4096, dtype=torch.uint8, device=DEV), torch.zeros(bs, H, N, dtype=torch.int32, device=DEV)
+        tiers, nt = ops._tiers([300, 700, 1500])
+
+        def call():
+            _lib.check(_lib.lib().pkv_update_cache_cnt(
+                ids.data_ptr(), *ids.stride()[:3], counts.data_ptr(), *counts.stride()[:3], code.data_ptr(), code.stride(0), code.stride(1),
+                code.stride(3), code.stride(2), bs, H, N, tiers, nt, ws.data_ptr(), out.data_ptr(), torch.cuda.current_stream().cuda_stream))
+
+        def want():
+            return ops.update_cache_cnt(ids, counts, code, [300, 700, 1500])
+
+        change = ids
+    else:
+        rows, L, k = 3, 24000, 2000
+        x = torch.randint(0, 90, (rows, L), generator=g, device=DEV, dtype=torch.int32)
+        n = _lib.lib().pkv_bucket_topk_ws_bytes(rows, L)
+        ws, out = torch.zeros(n, dtype=torch.uint8, device=DEV), torch.zeros(rows, k, dtype=torch.int64, device=DEV)
+
+        def call():
+            _lib.check(_lib.lib().pkv_bucket_topk(x.data_ptr(), L, rows, L, k, out.data_ptr(), ws.data_ptr(), n,
+                                                  torch.cuda.current_stream().cuda_stream))
+
+        def want():
+            return ops.bucket_topk(x, k)
+
+        change = x
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(out, want()) and not ws.any()
+    with torch.cuda.graph(graph):
+        call()
+    for _ in range(3):
+        change.copy_(change.flip(-1))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want()) and ws.any()
