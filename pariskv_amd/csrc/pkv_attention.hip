@@ -657,10 +657,6 @@ extern "C" int pkv_decode_attention_counted(const void *q, int dtype, int bs, in
                           arrivals + (1 - turn) * rows, stream);
 }
 
-static bool meets(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
-  return a && b && (uintptr_t)a < (uintptr_t)b + b_bytes && (uintptr_t)b < (uintptr_t)a + a_bytes;
-}
-
 bool pkv_plan_split_attention(const pkv_retrieve_args *r, const void *ws, const pkv_attn_args *at, PkvSplitAttn *out) {
   // What the general path would refuse is left to it.
   if (r->dtype != PKV_DTYPE_BF16 || !r->q || !pkv_aligned(r->q, 16) || !at->out || !pkv_aligned(at->out, 4) || !at->ws ||
@@ -738,8 +734,8 @@ bool pkv_plan_split_attention(const pkv_retrieve_args *r, const void *ws, const 
     size_t n;
   } busy[] = {{ws, r_bytes}, {r->out_ids, (size_t)rows * r->k * 8}, {r->out_scores, (size_t)rows * r->k * 4}, {r->q, out_bytes}};
   for (const auto &u : busy)
-    if (meets(at->ws, at_bytes, u.p, u.n) || (meets(at->out, out_bytes, u.p, u.n) && !(u.p == r->q && at->out == r->q))) return false;
-  if (meets(at->out, out_bytes, at->ws, at_bytes)) return false;
+    if (pkv_meets(at->ws, at_bytes, u.p, u.n) || (pkv_meets(at->out, out_bytes, u.p, u.n) && !(u.p == r->q && at->out == r->q))) return false;
+  if (pkv_meets(at->out, out_bytes, at->ws, at_bytes)) return false;
   out->n_kv_heads = r->n_kv_heads, out->group = r->group, out->q = r->q;
   out->scale_log2e = at->scale * 1.4426950408889634f;
   out->ws = (float *)at->ws, out->out = at->out;

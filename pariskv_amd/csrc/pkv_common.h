@@ -45,6 +45,15 @@ void pkv_set_error(const char *fmt, ...);
 static inline size_t pkv_align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 static inline bool pkv_aligned(const void *p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
+static inline bool pkv_meets(const void *a, size_t a_bytes, const void *b, size_t b_bytes) {
+  return a && b && (uintptr_t)a < (uintptr_t)b + b_bytes && (uintptr_t)b < (uintptr_t)a + a_bytes;
+}
+// ... where a is `rows` rows of row_bytes, a_step (of either sign) apart.
+static inline bool pkv_rows_meet(const void *a, int64_t rows, int64_t a_step, size_t row_bytes, const void *b, size_t b_bytes) {
+  const int64_t last = (rows - 1) * a_step;
+  return a && pkv_meets((const char *)a + (last < 0 ? last : 0), (size_t)(last < 0 ? -last : last) + row_bytes, b, b_bytes);
+}
+
 // A stream under capture, or one whose state cannot be read.  The null stream cannot be captured.
 static inline bool pkv_capturing(hipStream_t s) {
   if (s == nullptr) return false;

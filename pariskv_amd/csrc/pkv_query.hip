@@ -171,7 +171,15 @@ extern "C" int pkv_update_cache_cnt(const int64_t *sorted_ids, int64_t si_b, int
   int rc = make_tiers(tier_counts, n_tiers, t);
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
-  if (pkv_scan_takes_ranking(cs_key, bs * n_kv_heads, n_keys, s))
+  // every workgroup of that scan reads the ranking while others write votes: not where these go over it
+  const size_t cnt_bytes = (size_t)bs * n_kv_heads * (size_t)n_keys * 4;
+  auto over = [&](const void *in, int64_t step_b, int64_t step_h, int64_t step_sub, size_t es) {
+    int64_t lo = 0, hi = 256;
+    for (const int64_t last : {(bs - 1) * step_b, (n_kv_heads - 1) * step_h, 15 * step_sub}) (last < 0 ? lo : hi) += last;
+    return pkv_meets((const char *)in + lo * (int64_t)es, (size_t)(hi - lo) * es, cnt, cnt_bytes);
+  };
+  if (pkv_scan_takes_ranking(cs_key, bs * n_kv_heads, n_keys, s) && !over(sorted_ids, si_b, si_h, si_sub, 8) &&
+      !over(cluster_counts, cc_b, cc_h, cc_sub, 4))
     return pkv_launch_scan_ranked(codes, cs_b, cs_h, cs_sub, bs, n_kv_heads, n_keys, sorted_ids, si_b, si_h, si_sub, cluster_counts,
                                   cc_b, cc_h, cc_sub, t, cnt, s);
   dim3 grid(16, (unsigned)(bs * n_kv_heads));

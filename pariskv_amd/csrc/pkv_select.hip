@@ -2795,7 +2795,9 @@ extern "C" int pkv_bucket_topk(const int32_t *x, int64_t x_stride, int rows, int
     return PKV_ENOMEM;
   }
   const int blocks = (int)((len + kBucketBlock - 1) / kBucketBlock);
-  if (blocks <= 5 || (blocks <= 8 && blocks <= bucket_row_blocks(rows, pkv_capturing(s)))) {
+  // a row's workgroup writes while others read: not where the indices go over the values
+  if ((blocks <= 5 || (blocks <= 8 && blocks <= bucket_row_blocks(rows, pkv_capturing(s)))) &&
+      !pkv_rows_meet(x, rows, x_stride * 4, (size_t)len * 4, out, (size_t)rows * (size_t)k * 8)) {
 #define PKV_BUCKET(NB)                                                                                                  \
   hipLaunchKernelGGL(pkv_bucket_row_kernel<NB>, dim3((unsigned)rows), dim3(kBucketThreads), 0, s, x, x_stride, (int)len, (int)k, out)
     switch (blocks) {
@@ -2940,7 +2942,13 @@ int pkv_launch_topk_f32(const float *x, int64_t x_stride, const int64_t *ids, in
                     kTopkMaxSort, need, ws_bytes);
       return PKV_ENOMEM;
     }
-    if (topk_selects_long(len, k)) {
+    // a row's workgroup writes while others read: results over the scores or the ids take the launches that read them all first
+    const size_t out_n = (size_t)rows * (size_t)k;
+    auto over = [&](const void *in, int64_t step, size_t es) {
+      return pkv_rows_meet(in, rows, step * (int64_t)es, (size_t)len * es, out_ids, out_n * 8) ||
+             pkv_rows_meet(in, rows, step * (int64_t)es, (size_t)len * es, out_vals, out_n * 4);
+    };
+    if (topk_selects_long(len, k) && (attn || (!over(x, x_stride, 4) && !over(ids, ids_stride, 8)))) {
       const int P = pow2_ceil(k);
 #define PKV_SEL(EIN)                                                                                                            \
   do {                                                                                                                          \

@@ -2481,3 +2481,63 @@ def test_captured_operators_take_their_faster_launches(ops, what):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want()) and ws.any()
+
+
+@pytest.mark.parametrize("what", ["topk values", "topk ids", "bucket", "votes over the ranking", "votes over the counts"])
+def test_results_over_the_inputs(ops, what):
+    """Results written over the operator's own inputs, the first rows' over the last ones', with more rows than run at once: the results of
+    separate buffers.  The forms in which a row's workgroup writes while others still read stay out of such calls."""
+    from pariskv_amd import _lib
+
+    _say(f"results over the inputs, {what}")
+    lib, s = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=DEV).manual_seed(11)
+
+    def at_end(n_bytes, tail):   # `tail` bytes at the end of a buffer of n_bytes, as its address
+        buf = torch.empty(n_bytes, dtype=torch.uint8, device=DEV)
+        return buf, buf.data_ptr() + n_bytes - tail
+
+    if what.startswith("topk") or what == "bucket":
+        rows, L, k = (3000, 8200, 512) if what != "bucket" else (3000, 5000, 512)
+        if what == "bucket":
+            x = torch.randint(0, 100, (rows, L), generator=g, device=DEV, dtype=torch.int32)
+            want = ops.bucket_topk(x, k)
+            n = lib.pkv_bucket_topk_ws_bytes(rows, L)
+            ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+            buf, out = at_end(rows * L * 4, rows * k * 8)
+            buf.view(torch.int32).view(rows, L).copy_(x)
+            _lib.check(lib.pkv_bucket_topk(buf.data_ptr(), L, rows, L, k, out, ws.data_ptr(), n, s))
+            assert torch.equal(buf[-rows * k * 8:].view(torch.int64).view(rows, k), want)
+            return
+        x = torch.randn(rows, L, generator=g, device=DEV)
+        ids = torch.arange(L, device=DEV).repeat(rows, 1).flip(1).contiguous()
+        want_ids, want = ops.topk_f32(x, k, ids, want_values=True)
+        n = lib.pkv_topk_f32_ws_bytes(rows, L, k)
+        ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+        ids_out, vals = torch.empty(rows, k, dtype=torch.int64, device=DEV), torch.empty(rows, k, device=DEV)
+        if what == "topk values":
+            buf, out = at_end(rows * L * 4, rows * k * 4)
+            buf.view(torch.float32).view(rows, L).copy_(x)
+            _lib.check(lib.pkv_topk_f32(buf.data_ptr(), L, ids.data_ptr(), L, rows, L, k, ids_out.data_ptr(), out, ws.data_ptr(), n, s))
+            vals = buf[-rows * k * 4:].view(torch.float32).view(rows, k)
+        else:
+            buf, out = at_end(rows * L * 8, rows * k * 8)
+            buf.view(torch.int64).view(rows, L).copy_(ids)
+            _lib.check(lib.pkv_topk_f32(x.data_ptr(), L, buf.data_ptr(), L, rows, L, k, out, vals.data_ptr(), ws.data_ptr(), n, s))
+            ids_out = buf[-rows * k * 8:].view(torch.int64).view(rows, k)
+        assert torch.equal(ids_out, want_ids) and torch.equal(vals, want)
+        return
+    bs, H, N = 187, 8, 700
+    ids = torch.stack([torch.randperm(256, generator=g, device=DEV) for _ in range(64)]).repeat(bs * H * 16 // 64, 1).view(bs, H, 16, 256)
+    counts = torch.randint(0, 40, (bs, H, 16, 256), generator=g, device=DEV, dtype=torch.int32)
+    code = torch.randint(0, 256, (bs, H, 16, N), generator=g, device=DEV).to(torch.uint8)
+    want = ops.update_cache_cnt(ids, counts, code, [300, 700, 1500])
+    tiers, nt = ops._tiers([300, 700, 1500])
+    lut = torch.empty(bs * H * 4096, dtype=torch.uint8, device=DEV)
+    src = ids if what.endswith("ranking") else counts
+    buf, out = at_end(src.numel() * src.element_size(), bs * H * N * 4)
+    buf.view(src.dtype).view(src.shape).copy_(src)
+    i, c = (buf.data_ptr(), counts.data_ptr()) if src is ids else (ids.data_ptr(), buf.data_ptr())
+    _lib.check(lib.pkv_update_cache_cnt(i, *ids.stride()[:3], c, *counts.stride()[:3], code.data_ptr(), code.stride(0), code.stride(1), 1,
+                                        code.stride(2), bs, H, N, tiers, nt, lut.data_ptr(), out, s))
+    assert torch.equal(buf[-bs * H * N * 4:].view(torch.int32).view(bs, H, N), want)
