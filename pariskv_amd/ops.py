@@ -653,6 +653,8 @@ class DecodeAttention:
         nbytes = _lib.lib().pkv_decode_attention_ws_bytes(bs, n_kv_heads, group, max(1, max_keys))
         self.ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
         self.arrivals = torch.zeros(2 * bs * n_kv_heads, dtype=torch.int32, device=device)  # every launch leaves them zero
+        if self.arrivals.is_cuda and not torch.cuda.is_current_stream_capturing():
+            torch.cuda.current_stream(self.arrivals.device).synchronize()  # zero for launches on any stream
         self.turn = 0  # the half of them that the next launch counts in
         self._segs = (_lib.AttnSegment * 4)()  # reused between calls: filling it is most of the host time
 

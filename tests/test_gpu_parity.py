@@ -2541,3 +2541,27 @@ def test_results_over_the_inputs(ops, what):
     _lib.check(lib.pkv_update_cache_cnt(i, *ids.stride()[:3], c, *counts.stride()[:3], code.data_ptr(), code.stride(0), code.stride(1), 1,
                                         code.stride(2), bs, H, N, tiers, nt, lut.data_ptr(), out, s))
     assert torch.equal(buf[-bs * H * N * 4:].view(torch.int32).view(bs, H, N), want)
+
+
+def test_bound_attention_on_another_stream_than_its_counters(ops):
+    """Counters made behind a long queue of one stream are zero for a launch on another one, which shares no data with it and does not wait."""
+    _say("bound attention, counters of another stream")
+    bs, H, group, n = 1, 4, 4, 700
+    g = torch.Generator(device=DEV).manual_seed(1)
+    k, v = (torch.randn(bs, H, n, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    q = torch.randn(bs, 1, H * group, 128, generator=g, device=DEV).to(torch.bfloat16)
+    want = ops.DecodeAttention(bs, H, group, n, DEV).run(q, [(k, v, 0, n)])
+    a = torch.randn(8192, 8192, generator=g, device=DEV).to(torch.bfloat16)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    used = [torch.full((2 * bs * H,), 5, dtype=torch.int32, device=DEV) for _ in range(64)]   # what the counters' memory held before
+    del used
+    torch.cuda.synchronize()
+    for _ in range(10):
+        a @ a
+    att = ops.DecodeAttention(bs, H, group, n, DEV)
+    with torch.cuda.stream(side):
+        got = ops.BoundAttention(att, q, [(k, v, 0, n)]).launch(q)
+    side.synchronize()
+    assert torch.equal(got, want)
+    torch.cuda.synchronize()
