@@ -2565,3 +2565,23 @@ def test_bound_attention_on_another_stream_than_its_counters(ops):
     side.synchronize()
     assert torch.equal(got, want)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("bs,H,group,lens,base", [(2, 3, 4, (700, 300), 9), (1, 5, 5, (1, 1300), 0), (3, 2, 7, (513, 512, 30), 4), (2, 2, 6, (64, 1, 900), 1),
+                                                  (4, 4, 4, (1000, 1048), 3), (4, 4, 4, (1000, 1049), 3), (16, 4, 4, (500, 12), 0), (16, 4, 4, (501, 12), 0),
+                                                  (17, 4, 3, (200, 200), 2), (1, 1, 8, (2048,), 0)])
+def test_bound_attention_of_several_tensors(ops, bs, H, group, lens, base):
+    """The merge in the attention's own launch where the keys lie in tensors of different strides, for query heads that fill a turn of its
+    loop in part, and on both sides of its limits (16 splits a row, 256 workgroups): the two launches' bits."""
+    _say(f"bound attention, several tensors, {bs} x {H} group {group} {lens}")
+    g = torch.Generator(device=DEV).manual_seed(sum(lens) + group)
+    segs = []
+    for i, n in enumerate(lens):
+        k, v = (torch.randn(bs, H, n + base + 5 * i, 128, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+        segs.append((k, v, base, n))
+    att = ops.DecodeAttention(bs, H, group, sum(lens), DEV)
+    q = torch.randn(bs, 1, H * group, 128, generator=g, device=DEV).to(torch.bfloat16)
+    bound = ops.BoundAttention(att, q, segs)
+    for _ in range(3):
+        q.normal_(generator=g)
+        assert torch.equal(bound.launch(q), att.run(q, segs)) and not torch.any(att.arrivals)

@@ -1299,10 +1299,11 @@ def test_adaptive_step_takes_the_maximum_from_the_score_ranges():
 
 
 @pytest.mark.parametrize("bs,Hq,Hkv,S,topk,form", [(1, 4, 4, 1500, 1, 0), (2, 16, 2, 3001, 100, 1), (1, 8, 2, 20000, 100, 1), (2, 8, 2, 9000, 512, 2),
-                                                   (1, 12, 4, 20003, 700, 2), (3, 8, 2, 1300, 600, 0)])
+                                                   (1, 12, 4, 20003, 700, 2), (3, 8, 2, 1300, 600, 0), (8, 16, 8, 66500, 100, 1)])
 def test_attention_in_two_parts_behind_a_table_from_the_rope_launch(bs, Hq, Hkv, S, topk, form):
     """Steps whose query side another kernel has done: the part of the attention that waits for nothing rides with the scan.  Output
-    and ids are those of the same step with its own query prep, in every form of the step and from an empty buffer to a full one."""
+    and ids are those of the same step with its own query prep, in every form of the step and from an empty buffer to a full one; the
+    longest with chunks of 8192 keys, which the scan works through in four pieces."""
     import ctypes
 
     from pariskv_amd import _lib, ops
@@ -1310,7 +1311,11 @@ def test_attention_in_two_parts_behind_a_table_from_the_rope_launch(bs, Hq, Hkv,
     D, interval = 128, 16
     g = torch.Generator(device=DEV).manual_seed(S)
     cache = _make_cache(False, bs, Hkv, Hq, 1, S, 64, 4, 64, interval, topk)
-    k, v = _synth_kv(torch.Generator().manual_seed(2), bs, S, Hkv)
+    if S > 60000:
+        k, v = (torch.randn(bs, S, Hkv, D, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+        assert ops.pick_chunk_keys(bs * Hkv, S - 68) == 8192
+    else:
+        k, v = _synth_kv(torch.Generator().manual_seed(2), bs, S, Hkv)
     cache.prefill_update_kv_cache(None, k.to(DEV), v.to(DEV), 0, 0)
     cos, sin = torch.ones(D // 2, dtype=torch.bfloat16, device=DEV), torch.zeros(D // 2, dtype=torch.bfloat16, device=DEV)
     used = 0
