@@ -436,7 +436,7 @@ __global__ __launch_bounds__(256) void pkv_counts_to_u8_kernel(const int32_t *__
 
 // Both steps of the bucket top-k for a row of up to 4096 NB values, by one workgroup: a thread holds four neighbouring values of
 // each block of 4096 as clamped bytes, so nothing is read twice and neither counts nor histograms go through memory.
-// grid (rows).  Bound by what one CU's 16 waves issue, 1.1 us a block of 4096 behind 1.9 for the launch and the chain of phases:
+// grid (rows).  Bound by what one CU's 16 waves issue, 0.8 us a block of 4096 behind 2.6 for the launch and the chain of phases:
 // hence a histogram copy per lane (16 copies: 8.8 instead of 6.6 us for 20011 values) and byte-parallel comparisons.
 constexpr int kBucketThreads = 1024, kBucketBlock = 4 * kBucketThreads;
 template <int NB>
@@ -819,8 +819,8 @@ __device__ __forceinline__ void radix_select_regs(const uint64_t (&v)[EIN], uint
 // of bin b occupy the output slots [off[b], off[b] + count[b]), and the slot inside the bin is again found by
 // counting, which replaces the bitonic sort (and T: the first `need` of b* by that count are its winners).
 // Rows this does not suit take the older steps: non-finite scores, a zero or subnormal range or more than
-// kLinBucketMax keys in b* the radix select; more than kLinRankMax winners in one bin the bitonic sort.  The
-// result is the same set in the same order either way.
+// kLinBucketMax keys in b* the radix select; more than kLinRankMax winners in one bin the bitonic sort (rows of more than
+// kTopkMaxSort keys: see topk_select_long).  The result is the same set in the same order either way.
 constexpr int kLinBins = 512;   // a multiple of 64: wave 0 owns kLinBins / 64 bins per lane
 constexpr int kLinBinBits = 9;
 constexpr int kLinBucketMax = 256;
@@ -1434,8 +1434,8 @@ __device__ __forceinline__ void narrow_edge(Val val, uint32_t &win, uint32_t &ed
 // their bins, two to a word; ids are read for the winners and the threshold bin alone, in one round trip with what the caller
 // requests.  One CU reads its row's scores at some 130 GB/s, 0.8 us for 26000, and runs eight steps between barriers; the three
 // launches of the wide form read scores and ids twice and take 5 to 7 us each.  What the compiler would keep beside them (ordered
-// bits, places, unpacked bins) is computed again: with 32 to 64 bytes a lane in scratch instead, 8 rows x 32768 scores 10.3 (9.7), a step of
-// 8 rows x 262144 keys, top 100, 43.7 (40.7).
+// bits, places, unpacked bins) is computed again: with 32 to 64 bytes a lane in scratch instead, 8 rows x 32768 scores 10.3 (9.9), a step of
+// 8 rows x 262144 keys, top 100, 43.7 (41.0).
 // Infinities and NaN stay out of the bins' range.  Where the bins leave too many keys at the threshold (outliers, many equal scores),
 // narrow_edge over the scores, then over the ids of those that tie.  Top-k of 8 rows x 32768, top 100, us, three launches / a radix select
 // of eight passes over scores and ids from memory / this: spread scores 20.8 / 9.7 / 9.9, infinities 22.1 / 65.4 / 18.4, log-normal 20.8 /
@@ -1461,7 +1461,7 @@ __device__ __forceinline__ void topk_select_long(const float *__restrict__ x, in
     val[e] = *(const float *)((const char *)xr + 4u * (i < last ? i : last));
   }
   // 16 keys a thread leave registers for the caller's requests at once, 32 only when scores and bins are done with: 8 rows x
-  // 131072 keys, top 100, 33.8 / 33.2 us a step late / at once; 262144 keys 47.1 / 48.4
+  // 131072 keys, top 100, 30.2 / 29.8 us a step late / at once; 262144 keys 40.9 / 41.5
   constexpr bool kEarly = EIN <= 16;
   if (kEarly) more();
   const int n_mine = (len - tid + kTopkThreads - 1) / kTopkThreads;  // of the thread's keys; the others repeat the row's last
@@ -2848,11 +2848,11 @@ static bool topk_selects(int64_t len, int64_t k) {
   return len <= kTopkMaxSort && pow2_ceil(k) * 2 <= pow2_ceil(len) && pow2_ceil(len) >= 2048;
 }
 
-// ... and the longer ones it selects from with fewer registers a key.  k <= 2048: two winners a thread, and the sort's list in 16 KB
+// ... and the longer ones it selects from with fewer registers a key.  k <= 2048: two winners a thread, and the sort's two lists in 32 KB
 // of LDS.  Decode step, us, by the wide form / by one workgroup a row: 8 rows x 131072 keys (13050 candidates), top 100, 43.2 / 31.7,
 // 40 x 90000 (8943), top 100, 61.6 / 49.5, 64 x 90000, top 1024, 88.0 / 76.9, 16 x 131072, top 1024, 53.9 / 43.5, K/V on the host
-// 214.1 / 203.4; 17 to 32 keys a thread: 16 x 200000 (19942) 62.1 / 55.4, 8 x 262144 (26157), top 100, 51.0 / 42.6, fp32, top 1024,
-// 58.2 / 52.8.  With whole keys and ids in registers 16 a thread gave 34.7 at the first shape and 32 spilled (71.7 at 262144).
+// 214.1 / 203.4; 17 to 32 keys a thread: 16 x 200000 (19942) 61.0 / 52.4, 8 x 262144 (26157), top 100, 50.6 / 41.0, top 1024 54.0 / 46.3.
+// With whole keys and ids in registers 16 a thread gave 34.7 at the first shape and 32 spilled (71.7 at 262144).
 static bool topk_selects_long(int64_t len, int64_t k) {
   return len > kTopkMaxSort && len <= kTopkMaxSelect && pow2_ceil(k) <= kCountingSortMaxP;
 }
