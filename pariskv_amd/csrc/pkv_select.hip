@@ -2764,7 +2764,7 @@ static void bucket_ws_layout(int rows, int64_t len, int &chunk_keys, int64_t &cn
 // A captured call has no host time to save: 16 rows x 20480 7.4 / 6.7, x 24576 6.7 / 7.6, 32 x 24576 7.4 / 7.7, 63 x 24576 9.0 / 7.8,
 // 64 x 28672 10.1 / 8.6, x 32768 9.0 / 9.4, 96 x 32768 10.4 / 9.7.
 static int bucket_row_blocks(int rows, bool captured) {
-  if (captured) return rows < 48 ? 5 : rows < 96 ? 7 : 8;
+  if (captured) return rows < 48 ? 5 : rows < 64 ? 6 : rows < 96 ? 7 : 8;
   return rows < 64 ? 6 : 8;
 }
 
