@@ -164,6 +164,7 @@ extern "C" int pkv_update_cache_cnt(const int64_t *sorted_ids, int64_t si_b, int
                                     const uint32_t *tier_counts, int n_tiers, uint8_t *lut_ws, int32_t *cnt,
                                     void *stream) {
   PKV_REQUIRE(sorted_ids && cluster_counts && codes && lut_ws && cnt, "pkv_update_cache_cnt: null pointer");
+  PKV_REQUIRE(pkv_aligned(lut_ws, 4), "lut must be 4-byte aligned");
   PKV_REQUIRE(bs > 0 && n_kv_heads > 0 && (int64_t)bs * n_kv_heads <= 65535 && n_keys > 0 &&
                   n_keys <= PKV_MAX_KEYS_PER_ROW,
               "bad shape bs=%d kv_heads=%d n_keys=%lld", bs, n_kv_heads, (long long)n_keys);

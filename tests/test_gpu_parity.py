@@ -2585,3 +2585,21 @@ def test_bound_attention_of_several_tensors(ops, bs, H, group, lens, base):
     for _ in range(3):
         q.normal_(generator=g)
         assert torch.equal(bound.launch(q), att.run(q, segs)) and not torch.any(att.arrivals)
+
+
+def test_votes_of_a_ranking_refuse_an_unaligned_table(ops):
+    """Whether the scan builds the table itself or not."""
+    from pariskv_amd import _lib
+
+    _say("votes of a ranking, unaligned table")
+    ids = torch.arange(256, device=DEV).repeat(1, 1, 16, 1)
+    counts = torch.ones(1, 1, 16, 256, dtype=torch.int32, device=DEV)
+    ws, tiers = torch.zeros(4096 + 4, dtype=torch.uint8, device=DEV), ops._tiers([10])
+    for code in (torch.zeros(1, 1, 16, 100, dtype=torch.uint8, device=DEV), torch.zeros(1, 1, 100, 16, dtype=torch.uint8, device=DEV).transpose(2, 3)):
+        out = torch.full((1, 1, 100), -1, dtype=torch.int32, device=DEV)
+        rc = _lib.lib().pkv_update_cache_cnt(
+            ids.data_ptr(), *ids.stride()[:3], counts.data_ptr(), *counts.stride()[:3], code.data_ptr(), code.stride(0), code.stride(1),
+            code.stride(3), code.stride(2), 1, 1, 100, *tiers, ws.data_ptr() + 1, out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        with pytest.raises(RuntimeError, match="aligned"):
+            _lib.check(rc)
+        assert torch.all(out == -1)
